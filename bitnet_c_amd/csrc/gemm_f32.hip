@@ -1,0 +1,335 @@
+// C[M, N] = A[M, K] . W[N, K]^T in true float32 on the float32 matrix instruction (v_mfma_f32_16x16x4_f32: float32
+// products and float32 sums, no reduced-precision mode), the matrix product of the float32 path.  W is row-major
+// [out, in] as the reference keeps it (src/model.c:157-158); out[row] = sum_col W[row, col] x[col]
+// (src/quant/f32_scalar.c:4-32).
+//
+// One order of summation, a function of K alone, whatever M, N, the kernel and its tiles are, so that a row's result does
+// not depend on what else is in the batch: K is cut in chunks of 128; a chunk is summed from nothing by 32 instructions, the
+// one of (block j of 16 columns, e) taking columns 16 j + 4 g + e (g = 0..3, the instruction's four); the chunks' sums are
+// added in order.  The cut is what lets a product of few rows spread one output's K over the waves of a workgroup (and it
+// keeps the rounding error at that of a sum of 128 and of K / 128 terms).
+//
+// gemm_f32_stream_kernel, up to 64 rows: bound by the bytes of W.  A workgroup of 8 waves owns up to 16 columns and all of
+// K; a wave takes every eighth chunk, asks for its whole 8 KB of W (and the rows' 128 columns of A) at once and leaves
+// 16 x 16 sums in shared memory; then a thread an output adds them up in order.  us at one row, cold weights, and at 6.5
+// TB/s: 11,264 x 2,048 22 (14), 2,048 x 5,632 20 (7), 32,000 x 2,048 53 (40), 28,672 x 4,096 96 (72); the vector kernel that
+// walked K in one chain (gemm_tiled.hip) took 325 on the average of a layer's products, whatever the rows up to 16.
+// gemm_f32_tile_kernel, more rows: bound by the instruction (157 TFLOP/s on this chip, 32 cycles each on a SIMD).  5,136 x
+// 11,264 x 2,048 2.02 ms (117 TFLOP/s), 2,048 x 2,048 x 5,632 0.40 ms; the matrix unit is busy four fifths of a round, the
+// rest is the last round's empty CUs.  The vector kernel did 27 TFLOP/s.
+#include "common.h"
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+#define GF_CHUNK 128                 // columns of K whose products are summed from nothing
+#define GF_BLOCKS (GF_CHUNK / 16)
+#define GF_WAVES 8                   // waves of a workgroup of the streaming kernel
+#define GF_SUMS_KB 64                // shared memory for a round of chunk sums
+
+struct GfArgs {
+    const float* x;
+    const float* w;
+    float* y;
+    int M, N, K;                     // N: rows of W
+    int ldx, ldw, ldy;
+    int cols;                        // columns a workgroup of the streaming kernel owns (<= 16)
+    int glu;                         // rows of W are gate and up rows in turns of 8; y[M, N / 2] = act(gate) * up
+    int act;
+};
+
+struct gf_true { static constexpr bool value = true; };
+struct gf_false { static constexpr bool value = false; };
+
+__device__ __forceinline__ f32x4 gf_load(const float* p, bool ok) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (ok) v = *reinterpret_cast<const f32x4*>(p);
+    return v;
+}
+
+// MT row tiles of 16 share a wave's registers of W
+template <int MT>
+__global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArgs a) {
+    constexpr int ROUND = GF_SUMS_KB / MT;                       // chunks whose sums shared memory holds at a time
+    constexpr int THREADS = 64 * GF_WAVES;
+    __shared__ float sums[ROUND * MT * 256];                     // [chunk][row tile][row][column]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * a.cols;
+    // lanes without a column or a row read their neighbour's (no other bytes, and no load under a branch); what they form is
+    // not stored
+    const float* wp = a.w + (size_t)min(n0 + min(r, a.cols - 1), a.N - 1) * a.ldw + 4 * g;
+    const float* xp[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) xp[t] = a.x + (size_t)min(16 * t + r, a.M - 1) * a.ldx + 4 * g;
+    const int n_chunks = (a.K + GF_CHUNK - 1) / GF_CHUNK;
+    // the outputs that this thread adds up
+    constexpr int OWN = (MT * 256 + THREADS - 1) / THREADS;
+    float tot[OWN];
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) tot[o] = 0.f;
+
+    for (int c0 = 0; c0 < n_chunks; c0 += ROUND) {
+        const int c1 = min(n_chunks, c0 + ROUND);
+        auto chunk = [&](int c, auto whole) {
+            const int k0 = c * GF_CHUNK;
+            auto fetch = [&](const float* p, f32x4 (&v)[GF_BLOCKS]) {
+#pragma unroll
+                for (int j = 0; j < GF_BLOCKS; ++j)
+                    v[j] = gf_load(p + k0 + 16 * j, decltype(whole)::value || k0 + 16 * j + 4 * g < a.K);
+            };
+            f32x4 wv[GF_BLOCKS];
+            fetch(wp, wv);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                f32x4 xv[GF_BLOCKS], acc = {0.f, 0.f, 0.f, 0.f};
+                fetch(xp[t], xv);
+#pragma unroll
+                for (int j = 0; j < GF_BLOCKS; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j][e], xv[j][e], acc, 0, 0, 0);
+                // lane: columns 4 g .. 4 g + 3 of row r
+                *reinterpret_cast<f32x4*>(&sums[((c - c0) * MT + t) * 256 + 16 * r + 4 * g]) = acc;
+            }
+        };
+        for (int c = c0 + wave; c < c1; c += GF_WAVES) {
+            if ((c + 1) * GF_CHUNK <= a.K) chunk(c, gf_true());
+            else chunk(c, gf_false());
+        }
+        __syncthreads();
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) {
+            const int idx = tid + o * THREADS;
+            if (idx < MT * 256)
+                for (int c = 0; c < c1 - c0; ++c) tot[o] += sums[c * MT * 256 + idx];
+        }
+        if (c1 < n_chunks) __syncthreads();
+    }
+    if (a.glu) __syncthreads();
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+        const int idx = tid + o * THREADS;
+        if (idx >= MT * 256) continue;
+        const int m = idx >> 4, c = idx & 15;
+        if (a.glu) sums[idx] = tot[o];
+        else if (m < a.M && c < a.cols && n0 + c < a.N) a.y[(size_t)m * a.ldy + n0 + c] = tot[o];
+    }
+    if (!a.glu) return;
+    __syncthreads();
+    for (int idx = tid; idx < MT * 128; idx += THREADS) {
+        const int m = idx >> 3, n = idx & 7;
+        if (m < a.M) a.y[(size_t)m * a.ldy + n0 / 2 + n] = bn_gate_act(sums[m * 16 + n], a.act) * sums[m * 16 + 8 + n];
+    }
+}
+
+#define GF_BK 32
+#define GF_STRIDE (GF_BK + 4)        // of a staged row: 16-byte reads of the lanes' rows fall on different banks
+
+// orders shared memory alone: loads from memory stay in flight across it
+__device__ __forceinline__ void gf_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// A workgroup of 4 waves (2 x 2) owns BM rows of A and BN rows of W; a wave (BM / 2) x (BN / 2).
+template <int BM, int BN>
+__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(GfArgs a, int m_tiles, int n_tiles) {
+    constexpr int MT = BM / 32, NT = BN / 32;                    // 16 x 16 tiles of a wave
+    constexpr int XL = BM * GF_BK / 4 / 256, WL = BN * GF_BK / 4 / 256;      // 16-byte loads a thread and step
+    __shared__ float xs[2][BM * GF_STRIDE];
+    __shared__ float ws[2][BN * GF_STRIDE];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    // consecutive workgroups go to consecutive XCDs: give each XCD a run of tiles, and walk a run in bands of 8 row tiles, so
+    // that what runs on an XCD together shares its operands in that L2
+    int id = blockIdx.x;
+    const int total = m_tiles * n_tiles;
+    {
+        const int per = total / 8, rest = total % 8, xcd = id % 8, at = id / 8;
+        id = xcd * per + min(xcd, rest) + at;
+    }
+    const int band = id / (8 * n_tiles), in_band = id - band * 8 * n_tiles;
+    const int band_rows = min(8, m_tiles - band * 8);
+    const int m0 = (band * 8 + in_band % band_rows) * BM, n0 = (in_band / band_rows) * BN;
+    const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
+
+    f32x4 acc[NT][MT], tot[NT][MT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) { acc[i][j] = 0.f; tot[i][j] = 0.f; }
+
+    // staging: thread -> (row tid / 8 + 32 i, 16-byte group tid % 8); rows past the matrix read its last row and are not stored.
+    // Offsets are 32 bits wide against the tile's own (uniform) address.
+    const int sr = tid >> 3, sc = 4 * (tid & 7);
+    const float* xbase = a.x + (size_t)m0 * a.ldx;
+    const float* wbase = a.w + (size_t)n0 * a.ldw;
+    uint32_t xo[XL], wo[WL];
+#pragma unroll
+    for (int i = 0; i < XL; ++i) xo[i] = (uint32_t)min(sr + 32 * i, a.M - 1 - m0) * (uint32_t)a.ldx;
+#pragma unroll
+    for (int i = 0; i < WL; ++i) wo[i] = (uint32_t)min(sr + 32 * i, a.N - 1 - n0) * (uint32_t)a.ldw;
+    f32x4 xr[XL], wr[WL];
+    // loads are in straight line (one under a branch would be waited for at once); groups past K read the row's last one
+    // and become zeros when they are stored
+    auto load = [&](int k0) {
+        const uint32_t k = min(k0 + sc, a.K - 4);
+#pragma unroll
+        for (int i = 0; i < XL; ++i) xr[i] = *reinterpret_cast<const f32x4*>(xbase + (xo[i] + k));
+#pragma unroll
+        for (int i = 0; i < WL; ++i) wr[i] = *reinterpret_cast<const f32x4*>(wbase + (wo[i] + k));
+    };
+    auto store = [&](int b, int k0) {
+        if (k0 + GF_BK > a.K && k0 + sc >= a.K) {
+#pragma unroll
+            for (int i = 0; i < XL; ++i) xr[i] = 0.f;
+#pragma unroll
+            for (int i = 0; i < WL; ++i) wr[i] = 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < XL; ++i) *reinterpret_cast<f32x4*>(&xs[b][(sr + 32 * i) * GF_STRIDE + sc]) = xr[i];
+#pragma unroll
+        for (int i = 0; i < WL; ++i) *reinterpret_cast<f32x4*>(&ws[b][(sr + 32 * i) * GF_STRIDE + sc]) = wr[i];
+    };
+    f32x4 wv[2][NT], xv[2][MT];                                  // operands of the two blocks of a step
+    auto read = [&](int b, int blk) {
+#pragma unroll
+        for (int i = 0; i < NT; ++i) wv[blk][i] = *reinterpret_cast<const f32x4*>(&ws[b][(wn + 16 * i + r) * GF_STRIDE + 16 * blk + 4 * g]);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) xv[blk][j] = *reinterpret_cast<const f32x4*>(&xs[b][(wm + 16 * j + r) * GF_STRIDE + 16 * blk + 4 * g]);
+    };
+    auto multiply = [&](int blk, int from, int to) {
+#pragma unroll
+        for (int e = from; e < to; ++e)
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int j = 0; j < MT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[blk][i][e], xv[blk][j][e], acc[i][j], 0, 0, 0);
+    };
+    // A step multiplies two blocks of 16; every read of shared memory is asked for a block ahead of its products, a tile's
+    // stores stand in front of products that do not need them, and its loads a step earlier.  The one barrier of a step lies
+    // between its blocks: in front of it every wave has read all of buffer b and stored its part of the other.
+    const int steps = (a.K + GF_BK - 1) / GF_BK;
+    load(0);
+    store(0, 0);
+    load(GF_BK);
+    gf_barrier();
+    read(0, 0);
+    for (int s = 0; s < steps; ++s) {
+        const int b = s & 1;
+        multiply(0, 0, 1);       // first, so that the compiler's wait for block 0's operands meets no younger access
+        __builtin_amdgcn_sched_barrier(0);
+        read(b, 1);
+        store(b ^ 1, (s + 1) * GF_BK);
+        load((s + 2) * GF_BK);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(0, 1, 4);
+        __builtin_amdgcn_sched_barrier(0);
+        gf_barrier();
+        read(b ^ 1, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(1, 0, 4);
+        if ((s + 1) % (GF_CHUNK / GF_BK) == 0 || s + 1 == steps) {           // a chunk of K ends
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int j = 0; j < MT; ++j) { tot[i][j] += acc[i][j]; acc[i][j] = 0.f; }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        const int n = n0 + wn + 16 * i + 4 * g;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const int m = m0 + wm + 16 * j + r;
+            if (a.glu) {                                         // lanes with g < 2 hold gates, the lane 32 further their ups
+                f32x4 up;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) up[e] = __shfl_xor(tot[i][j][e], 32, BN_WAVE);
+                if (g < 2 && m < a.M && n < a.N) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        a.y[(size_t)m * a.ldy + (n0 + wn + 16 * i) / 2 + 4 * g + e] = bn_gate_act(tot[i][j][e], a.act) * up[e];
+                }
+            } else if (m < a.M) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < a.N) a.y[(size_t)m * a.ldy + n + e] = tot[i][j][e];
+            }
+        }
+    }
+}
+
+template <int MT>
+static int gf_launch_stream(const GfArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL((gemm_f32_stream_kernel<MT>), dim3((a.N + a.cols - 1) / a.cols), dim3(64 * GF_WAVES), 0, s, a);
+    return bn_launch_status();
+}
+
+template <int BM, int BN>
+static int gf_launch_tile(const GfArgs& a, hipStream_t s) {
+    const int mt = (a.M + BM - 1) / BM, nt = (a.N + BN - 1) / BN;
+    hipLaunchKernelGGL((gemm_f32_tile_kernel<BM, BN>), dim3(mt * nt), dim3(256), 0, s, a, mt, nt);
+    return bn_launch_status();
+}
+
+#define GF_CUS 256
+
+// Columns a workgroup of the streaming kernel owns: 16, or fewer where the busiest CU then has at least an eighth fewer
+// (us at one row: 3,072 x 2,048 in 16 / 12 9.8 / 9.3, 6,144 x 4,096 28.2 / 24.4, 2,048 x 5,632 in 16 / 8 18.6 / 17.1; where
+// the even split gains nothing fewer columns only read the rows more often: 11,264 x 2,048 in 16 / 12 22.6 / 24.5).
+static int gf_stream_cols(int N) {
+    int best = 16, cost = 1 << 30;
+    for (int c : {16, 12, 8}) {
+        const long long tiles = (N + c - 1) / c, busiest = (tiles + GF_CUS - 1) / GF_CUS * c;
+        if (busiest * 8 <= (long long)cost * 7) { best = c; cost = (int)busiest; }
+    }
+    return best;
+}
+
+// The tile kernel's form with the least time for the busiest CU, which is the longer of one tile's own chain of steps and of
+// all its tiles' instructions.  ns a step of 32 columns of K, measured at 2,048 columns with one tile a CU and with many: 128 x
+// 128 2,400 and 2,090 a tile, 64 x 128 1,360 and 1,060, 64 x 64 790 and 520, 32 x 64 520 and 290.
+static int gf_tile_form(int M, int N) {
+    static const int bm[4] = {128, 64, 64, 32}, bn[4] = {128, 128, 64, 64}, alone[4] = {2400, 1360, 790, 520}, many[4] = {2090, 1060, 520, 290};
+    int best = 0;
+    long long cost = -1;
+    for (int i = 0; i < 4; ++i) {
+        const long long tiles = (long long)((M + bm[i] - 1) / bm[i]) * ((N + bn[i] - 1) / bn[i]);
+        const long long per_cu = (tiles + GF_CUS - 1) / GF_CUS, t = per_cu * many[i];
+        const long long c = t > alone[i] ? t : alone[i];
+        if (cost < 0 || c < cost) { best = i; cost = c; }
+    }
+    return 2 + best;
+}
+
+// what the kernels need of the operands: rows of whole 16-byte groups at 16-byte addresses; offsets inside a tile's rows are
+// 32 bits wide
+extern "C" int bn_gemm_f32_supports(int N, int K, int ldw, const void* w) {
+    return N > 0 && K > 0 && K % 4 == 0 && ldw % 4 == 0 && ldw >= K && ldw <= (1 << 22) && ((uintptr_t)w & 15) == 0;
+}
+
+// form 0: by the sizes; 1: streaming; 2 .. 5: tiles of 128 x 128, 64 x 128, 64 x 64, 32 x 64 (every form gives the same bits).
+// Streaming up to 16 rows; up to 64 while the rows' 16-row tiles times the column tiles of a CU stay few, since every
+// workgroup of it reads all rows (us at 64 rows, streaming against tiles: 2,048 x 5,632 54 / 82, 4,096 x 14,336 139 / 202,
+// 11,264 x 2,048 60 / 54, 28,672 x 4,096 255 / 164; at 20 rows 6,144 x 4,096 43 / 61, 32,000 x 2,048 86 / 54).
+extern "C" int bn_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K, int ldx, int ldw, int ldy, int glu, int act,
+                           int form, hipStream_t s) {
+    if (M <= 0 || !bn_gemm_f32_supports(N, K, ldw, w) || ldx % 4 || ldx < K || ldx > (1 << 22) || ((uintptr_t)x & 15)) return BN_ERR_ARG;
+    if (ldy < (glu ? N / 2 : N) || (glu && N % 16) || act < 0 || act >= BN_ACT_KINDS) return BN_ERR_ARG;
+    if ((long long)((M + 31) / 32) * ((N + 63) / 64) > 0x7fffffffLL) return BN_ERR_ARG;
+    GfArgs a = {(const float*)x, (const float*)w, (float*)y, M, N, K, ldx, ldw, ldy, 16, glu ? 1 : 0, act};
+    const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+    if (form == 0)
+        form = M <= 16 || (M <= 64 && (long long)mt * N <= 6LL * 16 * GF_CUS) ? 1 : gf_tile_form(M, N);
+    switch (form) {
+        case 1:
+            if (M > 64) return BN_ERR_ARG;
+            a.cols = glu ? 16 : gf_stream_cols(N);
+            return mt == 1 ? gf_launch_stream<1>(a, s) : mt == 2 ? gf_launch_stream<2>(a, s) : gf_launch_stream<4>(a, s);
+        case 2: return gf_launch_tile<128, 128>(a, s);
+        case 3: return gf_launch_tile<64, 128>(a, s);
+        case 4: return gf_launch_tile<64, 64>(a, s);
+        case 5: return gf_launch_tile<32, 64>(a, s);
+    }
+    return BN_ERR_ARG;
+}

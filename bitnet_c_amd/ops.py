@@ -160,6 +160,10 @@ _SIGNATURES = {
                          c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p,
                          c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p],
     },
+    "gemm_f32": {
+        "bn_gemm_f32_supports": [c_int, c_int, c_int, c_void_p],
+        "bn_gemm_f32": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    },
     "gemm_tiled": {
         "bn_gemm_tiled": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                           c_void_p],
@@ -442,6 +446,25 @@ def _tiled(x, w, out_dtype):
     return y
 
 
+def _f32_product(x, w, glu: bool = False, activation: str = "silu", form: int = 0):
+    """x . w^T in float32 on the float32 matrix instruction (gemm_f32.hip), or with glu act(gate) * up for w = gate and up
+    rows interleaved in blocks of 8; None for weights that the kernels do not take (rows that are not whole 16-byte groups).
+    Whether they do depends on the weights alone, and every form of the kernels has one order of summation, so a row's bits do
+    not depend on the step it comes in.  form: 0, by the sizes; the others are bn_gemm_f32's, for tests."""
+    M, K = x.shape
+    N, ldw = w.shape[0], _rows(w, "w")
+    if not _fn("gemm_f32", "bn_gemm_f32_supports")(N, K, ldw, w.data_ptr()):
+        return None
+    ldx = _rows(x, "x")
+    if ldx % 4 or ldx > 1 << 22 or x.data_ptr() % 16:
+        x = x.clone(memory_format=torch.contiguous_format)
+        ldx = K
+    y = torch.empty((M, N // 2 if glu else N), dtype=torch.float32, device=x.device)
+    _check(_fn("gemm_f32", "bn_gemm_f32")(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, ldx, ldw, y.shape[1], int(glu),
+                                          _act(activation), int(form), _stream()), "gemm_f32")
+    return y
+
+
 def gemm_mfma(x: torch.Tensor, w: torch.Tensor, out_dtype=None, glu8: bool = False, activation: str = "silu",
               width: int = 0) -> torch.Tensor:
     """The library-free bf16 product for many rows: y[M, N] = x[M, K] . w[N, K]^T on the matrix cores,
@@ -571,7 +594,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, *, allow_library: O
            streamed: Optional[StreamedWeight] = None) -> torch.Tensor:
     """y[M, N] = x[M, K] . w[N, K]^T.  streamed: w's streamed copy, which the kernel of up to 16 rows reads instead.
 
-    float32: the tiled kernel (plain fmaf, a fixed order of summation).
+    float32: the float32 matrix instruction (gemm_f32.hip; float32 products and sums in one order whatever M is); rows that
+    are not whole 16-byte groups go to the tiled kernel (plain fmaf, a fixed order of summation).
     bf16: up to 16 rows (one MFMA tile of activations) the matrix-core kernel that streams
     the weights once; above that the library's matrix product, which from 32 rows on is about
     twice as fast as the streaming kernel, with a bf16 or a float32 result (logits).  Without the
@@ -594,7 +618,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, *, allow_library: O
     if x.dtype == torch.float32:
         if out_dtype != torch.float32:
             raise KernelError("linear: float32 inputs give float32 outputs")
-        return _tiled(x, w, torch.float32)
+        y = _f32_product(x, w)
+        return y if y is not None else _tiled(x, w, torch.float32)
     if x.dtype != torch.bfloat16:
         raise KernelError(f"linear: unsupported dtype {x.dtype}")
     aligned = (x.data_ptr() % 16 == 0) and (w.data_ptr() % 16 == 0)
@@ -704,8 +729,8 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, interleaved: bool = 
                   streamed: Optional[StreamedWeight] = None) -> torch.Tensor:
     """act(x.Wg^T) * (x.Wu^T) for w_gate_up = [Wg; Wu] ([2F, K]), or the two interleaved in
     blocks of 8 rows (interleave_gate_up); act is silu unless `activation` names another of
-    ACTIVATIONS.  The decode-sized bf16 case is one kernel, and so is the interleaved case without
-    the library; every other case is the product followed by the gated-unit kernel."""
+    ACTIVATIONS.  The decode-sized bf16 case is one kernel, and so are the interleaved case in float32 and
+    the one without the library; every other case is the product followed by the gated-unit kernel."""
     require_gpu()
     _dev(x, "x", dims=2)
     _dev(w_gate_up, "w_gate_up", x.dtype, 2)
@@ -720,6 +745,10 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, interleaved: bool = 
     if M == 0:
         return torch.empty((0, F), dtype=x.dtype, device=x.device)
     ldx, ldw = _rows(x, "x"), _rows(w_gate_up, "w_gate_up")
+    if x.dtype == torch.float32 and interleaved:
+        y = _f32_product(x, w_gate_up, True, activation)
+        if y is not None:
+            return y
     aligned = x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0
     if x.dtype == torch.bfloat16 and interleaved and aligned and _staged_swiglu_rows(M, allow_library, 2 * F, streamed):
         y = _staged_swiglu(x, w_gate_up, None, activation, streamed)

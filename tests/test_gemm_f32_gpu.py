@@ -1,0 +1,99 @@
+"""The float32 product on the float32 matrix instruction: every form of the kernel against 64 bits, and against each other
+bit for bit (the order of summation is a function of K alone)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _ops():
+    from bitnet_c_amd import ops
+    return ops
+
+
+def _data(M, N, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
+
+
+def _bound(x, w):
+    """What float32 sums of products can be off by at the most: a chunk is a chain of 32 instructions of four products, the
+    chunks' sums a chain of K / 128; every link rounds at 2^-24 of a partial sum, which the sum of magnitudes bounds."""
+    K = x.shape[1]
+    links = 4 * 32 + -(-K // 128) + 4
+    return links * 2.0 ** -24 * (x.abs().double() @ w.abs().double().t())
+
+
+# rows: the streaming kernel's tiles of 16 and their edges, the tile kernels' 32, 64, 128; columns: not a multiple of 8, 12 or
+# 16, one past a tile; K: one 16-byte group, the edges of a block of 16, a step of 32 and a chunk of 128, several chunks,
+# more chunks than one round of the streaming kernel's shared memory holds at 64 rows (16)
+@pytest.mark.parametrize("M,N,K", [(1, 1, 4), (1, 2048, 12), (2, 17, 16), (15, 3072, 36), (16, 70, 128), (17, 130, 132), (33, 64, 2052),
+                                   (64, 65, 2176), (64, 16, 8200)])
+def test_forms_agree_up_to_64_rows(M, N, K):
+    ops = _ops()
+    x, w = _data(M, N, K, 11 * M + N)
+    xd, wd = x.cuda(), w.cuda()
+    y = ops._f32_product(xd, wd)
+    assert torch.all((y.cpu().double() - x.double() @ w.double().t()).abs() <= _bound(x, w))
+    for form in (1, 2, 3, 4, 5):
+        assert torch.equal(ops._f32_product(xd, wd, form=form), y), form
+    assert torch.equal(ops.linear(xd, wd), y)
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 31, 64), (127, 129, 100), (129, 257, 1000), (300, 2048, 512)])
+def test_forms_agree_beyond_64_rows(M, N, K):
+    ops = _ops()
+    x, w = _data(M, N, K, M)
+    xd, wd = x.cuda(), w.cuda()
+    y = ops._f32_product(xd, wd)
+    assert torch.all((y.cpu().double() - x.double() @ w.double().t()).abs() <= _bound(x, w))
+    for form in (2, 3, 4, 5):
+        assert torch.equal(ops._f32_product(xd, wd, form=form), y), form
+    for m in (1, 17, 64):                                  # a row alone and among others
+        assert torch.equal(ops._f32_product(xd[:m].contiguous(), wd), y[:m]), m
+    with pytest.raises(ops.KernelError):
+        ops._f32_product(xd, wd, form=1)                   # the streaming form ends at 64 rows
+
+
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh", "relu2"])
+@pytest.mark.parametrize("M,F,K", [(1, 8, 16), (7, 88, 132), (40, 64, 260), (130, 200, 64)])
+def test_gated_epilogue(M, F, K, activation):
+    ops = _ops()
+    x, w = _data(M, 2 * F, K, F)
+    xd, wi = x.cuda(), ops.interleave_gate_up(w[:F], w[F:]).cuda()
+    want = ops.swiglu(ops._f32_product(xd, wi), True, activation)
+    for form in (0, 1, 2, 3, 4, 5) if M <= 64 else (0, 2, 3, 4, 5):
+        assert torch.equal(ops._f32_product(xd, wi, True, activation, form), want), form
+    assert torch.equal(ops.linear_swiglu(xd, wi, True, activation=activation), want)
+
+
+def test_operands_that_are_not_aligned():
+    """Activations at any address and stride give the same bits; weights whose rows are not whole 16-byte groups go to the
+    tiled kernel, at every row count."""
+    ops = _ops()
+    x, w = _data(5, 40, 64, 3)
+    y = ops.linear(x.cuda(), w.cuda())
+    wide = torch.zeros(5, 71).cuda()
+    wide[:, 3:67] = x.cuda()
+    assert torch.equal(ops.linear(wide[:, 3:67], w.cuda()), y)
+    padded = torch.zeros(40, 68).cuda()
+    padded[:, :64] = w.cuda()
+    assert torch.equal(ops.linear(x.cuda(), padded[:, :64]), y)
+    shifted = torch.zeros(40 * 64 + 1).cuda()[1:].view(40, 64)
+    shifted.copy_(w)
+    assert ops._f32_product(x.cuda(), shifted) is None
+    for m in (1, 5):
+        got = ops.linear(x[:m].cuda(), shifted)
+        assert torch.all((got.cpu().double() - x[:m].double() @ w.double().t()).abs() <= 64 * 2.0 ** -24 * (x[:m].abs().double() @ w.abs().double().t()))
+
+
+def test_infinities_and_nan_stay_in_their_rows_and_columns():
+    ops = _ops()
+    x, w = _data(20, 48, 100, 9)
+    x[3, 7], x[4, 99], w[5, 0] = float("inf"), float("nan"), float("-inf")
+    for form in (1, 2, 3, 4, 5):
+        y = ops._f32_product(x.cuda(), w.cuda(), form=form).cpu()
+        fine = torch.isfinite(y)
+        assert not fine[3].any() and not fine[4].any() and not fine[:, 5].any()
+        fine[3], fine[4], fine[:, 5] = True, True, True
+        assert fine.all()
