@@ -160,6 +160,12 @@ _SIGNATURES = {
                          c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p,
                          c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p],
     },
+    "attn_f32": {
+        "bn_attn_f32_supports": [c_int],
+        "bn_attn_f32_run_keys": [],
+        "bn_attn_f32": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int,
+                        c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p, c_void_p],
+    },
     "gemm_f32": {
         "bn_gemm_f32_supports": [c_int, c_int, c_int, c_void_p],
         "bn_gemm_f32": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
@@ -1197,13 +1203,22 @@ def mfma_attention(dtype, hs: int) -> bool:
     return dtype == torch.bfloat16 and int(hs) in MFMA_HEAD_DIMS
 
 
-def attention_row_shape(H: int, Hkv: int, decode: bool, dtype=None, hs: int = 0):
+def f32_attention(dtype, hs: int) -> bool:
+    """Whether the plain float32 attention (attn_f32.hip: pages with a row per position, no window, bias or sink) takes this
+    head size; everything else in float32 is the vector kernel's."""
+    return dtype == torch.float32 and bool(_fn("attn_f32", "bn_attn_f32_supports")(int(hs)))
+
+
+def attention_row_shape(H: int, Hkv: int, decode: bool, dtype=None, hs: int = 0, plain_f32: bool = False):
     """(RT, GT, QT): what one workgroup covers: QT query tokens x GT heads of one kv group
-    (RT = QT * GT rows for the vector kernel)."""
+    (RT = QT * GT rows for the vector kernel).  plain_f32: the caller's attention is the plain one over a float32 cache
+    (f32_attention), whose workgroups take tiles of up to four times the vector kernel's tokens."""
     G = H // Hkv
     GT = min(_pow2_at_least(G), 16)
     if decode:
         return GT, GT, 1
+    if plain_f32 and f32_attention(dtype, hs):
+        return 64, GT, 64 // GT
     if dtype is not None and mfma_attention(dtype, hs):
         qt = _fn("attn_mfma", "bn_attn_mfma_prompt_tokens")(int(hs), GT)
         return qt * GT, GT, qt
@@ -1390,6 +1405,8 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
     if not use_mfma and mfma_attention(qkv.dtype, hs) and not force_vector:
         force_vector = True          # pages in another order than the matrix-core kernels': the vector kernel reads them
     RT, GT, QT = attention_row_shape(H, Hkv, decode, qkv.dtype if use_mfma else None, hs)
+    f32_plain = (layout == "rows" and not extras and distance_bias is None and window == 0 and not force_vector
+                 and f32_attention(qkv.dtype, hs))
     if decode:
         _dev(seq_lens, "seq_lens", torch.int32, 1)
         if seq_lens.numel() != T or block_table.shape[0] < T or not seq_lens.is_contiguous():
@@ -1397,7 +1414,7 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
         n_tiles = T
     else:
         _dev(tiles, "tiles", torch.int32, 2)
-        if tiles.shape[1] != 4 or not tiles.is_contiguous() or qt != QT:
+        if tiles.shape[1] != 4 or not tiles.is_contiguous() or (qt != QT and not (f32_plain and qt == 4 * QT)):
             raise KernelError(f"attention(prompt): tiles must be [n, 4] built for qt={QT}, got qt={qt}")
         n_tiles = tiles.shape[0]
         n_splits, chunk = 1, 0
@@ -1425,8 +1442,12 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
                               f"{block_table.shape[1]} pages of the block table")
         if n_splits > (1024 if fold else 64):
             raise KernelError("attention: at most 64 splits (1,024 runs of a float32 cache)")
-        part_o = torch.empty((T * H * n_splits, vd), dtype=torch.float32, device=qkv.device)
-        part_ml = torch.empty((T * H * n_splits, 2), dtype=torch.float32, device=qkv.device)
+    parts = n_splits
+    if f32_plain:                     # however the caller cuts them, the keys are summed page by page and run by run
+        parts = -(-block_table.shape[1] * PAGE // _fn("attn_f32", "bn_attn_f32_run_keys")()) if decode else 1
+    if parts > 1:
+        part_o = torch.empty((T * H * parts, vd), dtype=torch.float32, device=qkv.device)
+        part_ml = torch.empty((T * H * parts, 2), dtype=torch.float32, device=qkv.device)
     po = part_o.data_ptr() if part_o is not None else None
     pm = part_ml.data_ptr() if part_ml is not None else None
     sl = seq_lens.data_ptr() if decode else None
@@ -1469,6 +1490,12 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
             int(bool(fused_write)), by_length.data_ptr() if by_length is not None else None,
             max_len_dev.data_ptr() if max_len_dev is not None else None, _stream()),
             "attention(mfma)")
+        return
+    if f32_plain:
+        _check(_fn("attn_f32", "bn_attn_f32")(
+            qkv.data_ptr(), _rows(qkv, "qkv"), out.data_ptr(), H * hs, k_pages.data_ptr(), v_pages.data_ptr(),
+            block_table.data_ptr(), block_table.shape[1], sl, tl, n_tiles, H, Hkv, hs, GT, float(scale), int(parts), po, pm,
+            _stream()), "attention(float32)")
         return
     _check(_fn("attn_rows", "bn_attn_rows")(
         _code(qkv.dtype), qkv.data_ptr(), _rows(qkv, "qkv"), out.data_ptr(), H * vd,

@@ -328,8 +328,9 @@ class Attention(Part):
                           by_length=ctx.by_length, max_len_dev=ctx.max_len_dev if n_splits > 1 else None,
                           v_transposed=vt, blocked=blocked)
         else:
-            # pages in another order than the matrix-core kernels' own: the vector kernel, with its tiles
-            _, _, qt = ops.attention_row_shape(H, Hkv, False, h.dtype if blocked else None, hs)
+            # pages in another order than the matrix-core kernels' own: the float32 kernel or the vector kernel, with their tiles
+            plain_f32 = h.dtype == torch.float32 and not blocked and not vt and not self.window
+            _, _, qt = ops.attention_row_shape(H, Hkv, False, h.dtype if blocked or plain_f32 else None, hs, plain_f32)
             ops.attention(qkv, out, kv.k_pages, kv.v_pages, kv.block_table, H, Hkv, hs, self.scale,
                           window=self.window, tiles=ctx.tiles(qt), qt=qt, v_transposed=vt, blocked=blocked)
         return last(out)
