@@ -131,10 +131,10 @@ _SIGNATURES = {
         "bn_wkv_state_floats": [c_int, c_int],
         "bn_wkv_scan": [c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p,
                         c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int,
-                        c_int, c_void_p],
+                        c_int, c_int, c_void_p, c_void_p, c_void_p],
         "bn_head_norm_gate": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_float, c_void_p],
         "bn_mingru_scan": [c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_int,
-                           c_void_p, c_void_p, c_int, c_void_p],
+                           c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p],
     },
     "rope_kv": {
         "bn_v_transposed_write": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int,
@@ -1942,12 +1942,37 @@ def wkv_state_floats(H: int, dk: int, dv: int) -> int:
     return H * p * WKV_ROWS_PER_THREAD * dv
 
 
-def wkv_scan(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, *, tiles=None, seq_lens=None) -> torch.Tensor:
+# Long prompt steps of few sequences are cut into pieces that are walked side by side instead of every sequence from its
+# first token to its last: twice the arithmetic on many times the workgroups.  us walked / in pieces, wkv with 32 heads of 64
+# and the min-GRU with 2,048 channels (32 workgroups a sequence either way): one sequence of 256 tokens 89 / 65 and 34 / 21, of
+# 2,048 617 / 203 and 235 / 44; four of 512 179 / 198 and 62 / 41; eight of 512 177 / 365 and 65 / 65.  So up to
+# SCAN_PIECES_GROUPS workgroups of the plain walk.
+SCAN_PIECES_GROUPS = 96
+SCAN_PIECES_MIN_ROWS = 256
+WKV_PIECE = _build.header_constant("WKV_PIECE", "state_mixers.hip")
+GRU_PIECE = _build.header_constant("GRU_TC", "state_mixers.hip")
+
+
+def _scan_pieces(pieces, tl, T: int, n_seqs: int, groups: int, piece: int, floats: int, device):
+    """(pieces that the step's sequences can have together or 0, scratch of a state a piece) of a prompt step; groups: the
+    workgroups of the plain walk; floats: of a sequence's state."""
+    most = -(-T // piece) + n_seqs                       # every sequence may end in a piece that is not full
+    if pieces is None:
+        pieces = T >= SCAN_PIECES_MIN_ROWS and groups <= SCAN_PIECES_GROUPS and n_seqs <= 32 and most * floats * 4 <= 2 << 30
+    if not pieces or tl is None or not T or not n_seqs:
+        return 0, None
+    return most, torch.empty((most, floats), dtype=torch.float32, device=device)
+
+
+def wkv_scan(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, *, tiles=None, seq_lens=None,
+             pieces: Optional[bool] = None) -> torch.Tensor:
     """The wkv recurrence over every sequence of a step; float32 [T, H dv].  r, k, d: [T, H dk] (rows contiguous, any row
     stride), v: [T, H dv], in the activations' type; w0, u: float32 [H dk] (the decay's offset, the current token's
     bonus); h [T, D]: the mixer's input.  state [slots, >= wkv_state_floats(H, dk, dv) + D] float32: the heads' matrices
     in the kernel's own order, then the last h, both updated in place.  Per head, in float32:
-        w_t = exp(-exp(d_t + w0));  o_t = (S + diag(u) k_t v_t^T)^T r_t;  S <- diag(w_t) S + k_t v_t^T."""
+        w_t = exp(-exp(d_t + w0));  o_t = (S + diag(u) k_t v_t^T)^T r_t;  S <- diag(w_t) S + k_t v_t^T.
+    pieces (prompt form): whether every sequence is cut into pieces of WKV_PIECE tokens that are walked side by side (the
+    results differ from the plain walk's by rounding alone); None: by the step's size (_scan_pieces)."""
     require_gpu()
     _dev(h, "h", dims=2)
     T, D = h.shape
@@ -1967,11 +1992,15 @@ def wkv_scan(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, *,
     _dev(slot_ids, "slot_ids", torch.int32, 1)
     tl, n_tiles, sl = _seq_args(tiles, seq_lens, "wkv_scan")
     o = torch.empty((T, H * dv), dtype=torch.float32, device=h.device)
+    floats = wkv_state_floats(H, dk, dv)
+    most, carry = _scan_pieces(pieces, tl, T, n_tiles, n_tiles * H, WKV_PIECE, floats, h.device)
+    fade = torch.empty((carry.shape[0], floats // dv), dtype=torch.float32, device=h.device) if most else None
     if T and n_tiles:
         _check(_fn("state_mixers", "bn_wkv_scan")(
             _code(h.dtype), r.data_ptr(), _rows(r, "r"), k.data_ptr(), _rows(k, "k"), v.data_ptr(), _rows(v, "v"),
             d.data_ptr(), _rows(d, "d"), w0.data_ptr(), u.data_ptr(), o.data_ptr(), h.data_ptr(), state.data_ptr(), stride,
-            tl, n_tiles, sl, slot_ids.data_ptr(), H, dk, dv, D, _stream()), "wkv_scan")
+            tl, n_tiles, sl, slot_ids.data_ptr(), H, dk, dv, D, most, carry.data_ptr() if most else None,
+            fade.data_ptr() if most else None, _stream()), "wkv_scan")
     return o
 
 
@@ -1996,11 +2025,12 @@ def head_norm_gate(o: torch.Tensor, gate: torch.Tensor, weight: Optional[torch.T
 
 
 def mingru_scan(zxg: torch.Tensor, bias_z, bias_x, state: torch.Tensor, slot_ids, W: int, *, tiles=None,
-                seq_lens=None) -> torch.Tensor:
+                seq_lens=None, pieces: Optional[bool] = None) -> torch.Tensor:
     """The min-GRU recurrence over every sequence of a step.  zxg [T, 3 W]: the projections of the update gate, the
     candidate and the output gate side by side, without biases (bias_z, bias_x: float32 [W] or None).  state
     [slots, >= W] float32, updated in place.  Per channel, in float32: z = sigmoid(a + bias_z); c = b + bias_x;
-    cand = c + 1/2 where c >= 0, sigmoid(c) below; S <- (1 - z) S + z cand; result S * silu(g), [T, W]."""
+    cand = c + 1/2 where c >= 0, sigmoid(c) below; S <- (1 - z) S + z cand; result S * silu(g), [T, W].
+    pieces: as wkv_scan's, of GRU_PIECE tokens."""
     require_gpu()
     _dev(zxg, "zxg", dims=2)
     T = zxg.shape[0]
@@ -2015,11 +2045,14 @@ def mingru_scan(zxg: torch.Tensor, bias_z, bias_x, state: torch.Tensor, slot_ids
     _dev(slot_ids, "slot_ids", torch.int32, 1)
     tl, n_tiles, sl = _seq_args(tiles, seq_lens, "mingru_scan")
     y = torch.empty((T, W), dtype=zxg.dtype, device=zxg.device)
+    most, carry = _scan_pieces(pieces, tl, T, n_tiles, n_tiles * -(-W // 64), GRU_PIECE, W, zxg.device)
+    fade = torch.empty_like(carry) if most else None
     if T and n_tiles:
         _check(_fn("state_mixers", "bn_mingru_scan")(
             _code(zxg.dtype), y.data_ptr(), zxg.data_ptr(), _rows(zxg, "zxg"),
             bias_z.data_ptr() if bias_z is not None else None, bias_x.data_ptr() if bias_x is not None else None,
-            state.data_ptr(), stride, tl, n_tiles, sl, slot_ids.data_ptr(), W, _stream()), "mingru_scan")
+            state.data_ptr(), stride, tl, n_tiles, sl, slot_ids.data_ptr(), W, most, carry.data_ptr() if most else None,
+            fade.data_ptr() if most else None, _stream()), "mingru_scan")
     return y
 
 
