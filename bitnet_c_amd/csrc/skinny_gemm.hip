@@ -40,21 +40,31 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast
 
 #define SK_XROW 528           // bytes between rows of a wave's staged X chunk (512 + 16: conflict-free 16-byte reads)
 
-template <int MT, bool DUAL, typename TO, bool GLU8 = false, bool XS = false, bool TILED = false>
-__global__ __launch_bounds__((DUAL && MT >= 3) ? 512 : 1024) void skinny_gemm_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W,
-                                                           TO* __restrict__ Y, int M, int N, int K, int ldx,
-                                                           int ldw, int ldy, int up_off, int act) {
+#define SK_ACT_UNARY 16       // act: this plus one of BN_UNARY_*: an activation of one argument on every result
+
+// The result of a product without a gate under its activation: none, a square of the positive part (the gate kind
+// BN_ACT_RELU2), or any activation of one argument (UNARY: kept out of the other instantiations, whose registers it would cost).
+template <bool UNARY> __device__ __forceinline__ float sk_result(float v, int act) {
+    if (UNARY) return act >= SK_ACT_UNARY ? bn_unary_act(v, act - SK_ACT_UNARY) : v;
+    const float p = fmaxf(v, 0.f);
+    return act == BN_ACT_RELU2 ? p * p : v;
+}
+
+// bx: the workgroup's number among those of its product
+template <int MT, bool DUAL, typename TO, bool GLU8, bool XS, bool TILED, bool UNARY>
+__device__ __forceinline__ void skinny_gemm_body(const bf16* __restrict__ X, const bf16* __restrict__ W, TO* __restrict__ Y, int M, int N,
+                                                 int K, int ldx, int ldw, int ldy, int up_off, int act, int bx) {
     constexpr int NA = DUAL ? 2 * MT : MT;            // accumulator tiles per wave
     extern __shared__ __align__(16) float red[];      // [n_waves][NA][64][4]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // a scalar
     const int n_waves = blockDim.x >> 6;
     const int i = lane & 15, g = lane >> 4;
     const int CW = TILED ? up_off : 16;               // columns a workgroup owns; TILED: up_off carries the copy's rows per tile
-    const int n0 = blockIdx.x * CW;
+    const int n0 = bx * CW;
     const int n = min(n0 + i, N - 1);                 // clamp: rows past N are computed and dropped
     const int TS = CW * BN_STREAM_TILE_COLS;          // elements of a tile
     // tiled: the row of tiles is the same for all lanes (a base in scalar registers), the lane adds its 16 bytes' place
-    const bf16* wrow = TILED ? W + (size_t)blockIdx.x * ldw * TS : W + (size_t)n * ldw;
+    const bf16* wrow = TILED ? W + (size_t)bx * ldw * TS : W + (size_t)n * ldw;
     const unsigned lane_at = (g * CW + i) * 8;
     const bf16* urow = DUAL ? W + (size_t)(up_off + n) * ldw : nullptr;
 
@@ -144,11 +154,36 @@ __global__ __launch_bounds__((DUAL && MT >= 3) ? 512 : 1024) void skinny_gemm_ke
             if ((l & 8) == 0 && m < M && nn < N)
                 Y[(size_t)m * ldy + (n0 >> 1) + (l & 7)] = from_f32<TO>(bn_gate_act(v, act) * up);
         } else if (m < M && nn < N) {
-            const float p = fmaxf(v, 0.f);
-            const float y = DUAL ? bn_gate_act(v, act) * u : (act == BN_ACT_RELU2 ? p * p : v);
+            const float y = DUAL ? bn_gate_act(v, act) * u : sk_result<UNARY>(v, act);
             Y[(size_t)m * ldy + nn] = from_f32<TO>(y);
         }
     }
+}
+
+template <int MT, bool DUAL, typename TO, bool GLU8 = false, bool XS = false, bool TILED = false, bool UNARY = false>
+__global__ __launch_bounds__((DUAL && MT >= 3) ? 512 : 1024) void skinny_gemm_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W,
+                                                           TO* __restrict__ Y, int M, int N, int K, int ldx,
+                                                           int ldw, int ldy, int up_off, int act) {
+    skinny_gemm_body<MT, DUAL, TO, GLU8, XS, TILED, UNARY>(X, W, Y, M, N, K, ldx, ldw, ldy, up_off, act, blockIdx.x);
+}
+
+// Several products of up to 16 rows over streamed copies that do not depend on each other, as one launch: a launch that waits
+// for the one before it costs some 4.5 us whatever it does, and five products of 2,048 x 2,048 take 4.5 to 6 each.  The
+// workgroups of product j are the numbers from first[j] on.
+#define SK_GROUP 6
+struct SkinnyGroup {
+    const bf16* x[SK_GROUP];
+    const bf16* w[SK_GROUP];
+    bf16* y[SK_GROUP];
+    int n[SK_GROUP], ldx[SK_GROUP], rows[SK_GROUP], act[SK_GROUP], first[SK_GROUP];      // rows: of a tile of the copy
+    int count;
+};
+
+__global__ __launch_bounds__(512) void skinny_group_kernel(SkinnyGroup p, int M, int K, int k_tiles) {
+    int j = 0;
+    while (j + 1 < p.count && (int)blockIdx.x >= p.first[j + 1]) ++j;
+    skinny_gemm_body<1, false, bf16, false, true, true, true>(p.x[j], p.w[j], p.y[j], M, p.n[j], K, p.ldx[j], k_tiles, p.n[j], p.rows[j],
+                                                              p.act[j], (int)blockIdx.x - p.first[j]);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -401,13 +436,13 @@ extern "C" int bn_skinny_gemm_fused(const void* X, const void* W, void* Y, int M
 #undef SK_FUSED
 }
 
-template <int MT, bool DUAL, typename TO, bool GLU8 = false, bool TILED = false>
+template <int MT, bool DUAL, typename TO, bool GLU8 = false, bool TILED = false, bool UNARY = false>
 static int launch(const void* X, const void* W, void* Y, int M, int N, int K, int ldx, int ldw, int ldy,
                   int up_off, int act, int n_waves, hipStream_t s) {
     constexpr int NA = DUAL ? 2 * MT : MT;
     constexpr bool XS = MT == 1 && !DUAL;          // the two-block form has no registers to spare for it
     const size_t smem = (size_t)n_waves * NA * 64 * 4 * sizeof(float) + (XS ? (size_t)n_waves * M * SK_XROW : 0);
-    auto kernel = skinny_gemm_kernel<MT, DUAL, TO, GLU8, XS, TILED>;
+    auto kernel = skinny_gemm_kernel<MT, DUAL, TO, GLU8, XS, TILED, UNARY>;
     if (smem > 64 * 1024) {                           // beyond the default limit of dynamic shared memory
         static bool raised = false;                   // per instantiation
         if (!raised) {
@@ -456,13 +491,15 @@ extern "C" int bn_skinny_gemm_supports(int M, int N, int K, int ldx, int ldw) {
 // the gate rows at [0, N) and the up rows at [up_off, up_off + N).  dual == 2: W has 2N rows, gate
 // and up interleaved in blocks of 8 (N a multiple of 8); the result has N columns.  act: the gate's activation
 // (BN_ACT_*) when dual != 0; with dual == 0 BN_ACT_RELU2 squares the positive part of every result (a feed-forward without
-// a gate) and any other value leaves the product as it is.
+// a gate), SK_ACT_UNARY + one of BN_UNARY_* puts every result under that activation (bf16 results of up to 16 rows) and any
+// other value leaves the product as it is.
 // tile_rows > 0: W is the streamed copy (common.h) with that many rows a tile and ldw its tiles along K; up to 16 rows,
 // dual == 0.
 extern "C" int bn_skinny_gemm(int out_dtype, const void* X, const void* W, void* Y, int M, int N, int K,
                               int ldx, int ldw, int ldy, int dual, int up_off, int act, int tile_rows, hipStream_t s) {
-    const bool tiled = tile_rows != 0;
-    if (!bn_skinny_gemm_supports(M, N, K, ldx, tiled ? 8 : ldw) || ldy < N || act < 0 || act >= BN_ACT_KINDS) return BN_ERR_ARG;
+    const bool tiled = tile_rows != 0, unary = act >= SK_ACT_UNARY;
+    if (!bn_skinny_gemm_supports(M, N, K, ldx, tiled ? 8 : ldw) || ldy < N || act < 0) return BN_ERR_ARG;
+    if (unary ? act >= SK_ACT_UNARY + BN_UNARY_KINDS || dual || M > 16 || out_dtype != BN_DT_BF16 : act >= BN_ACT_KINDS) return BN_ERR_ARG;
     if (((uintptr_t)X | (uintptr_t)W) & 15) return BN_ERR_ARG;
     if (tiled) {
         if (dual || M > 16 || !sk_tiled_ok(K, ldw) || tile_rows < 1 || tile_rows > BN_STREAM_TILE_ROWS) return BN_ERR_ARG;
@@ -470,6 +507,8 @@ extern "C" int bn_skinny_gemm(int out_dtype, const void* X, const void* W, void*
         const int k_chunks = (K + SK_CHUNK - 1) / SK_CHUNK;
         while (n_waves > 1 && n_waves / 2 >= k_chunks) n_waves >>= 1;
         // the kernel's up_off carries the rows per tile; its grid is one workgroup per row of tiles
+        if (unary)
+            return launch<1, false, bf16, false, true, true>(X, W, Y, M, N, K, ldx, ldw, ldy, tile_rows, act, n_waves, s);
         if (out_dtype == BN_DT_BF16)
             return launch<1, false, bf16, false, true>(X, W, Y, M, N, K, ldx, ldw, ldy, tile_rows, act, n_waves, s);
         if (out_dtype == BN_DT_F32)
@@ -491,6 +530,7 @@ extern "C" int bn_skinny_gemm(int out_dtype, const void* X, const void* W, void*
     while (n_waves > 1 && n_waves / 2 >= k_chunks) n_waves >>= 1;
     while (n_waves > 1 && n_waves * NA > 48) n_waves >>= 1;
     if (dual == 1 && MT >= 3 && n_waves > 8) n_waves = 8;      // that variant is built for 512 threads
+    if (unary) return launch<1, false, bf16, false, false, true>(X, W, Y, M, N, K, ldx, ldw, ldy, 0, act, n_waves, s);
     if (dual == 2) {
         if (out_dtype == BN_DT_BF16) return launch_glu8<bf16>(MT, X, W, Y, M, N, K, ldx, ldw, ldy, act, n_waves, s);
         if (out_dtype == BN_DT_F32) return launch_glu8<float>(MT, X, W, Y, M, N, K, ldx, ldw, ldy, act, n_waves, s);
@@ -503,4 +543,35 @@ extern "C" int bn_skinny_gemm(int out_dtype, const void* X, const void* W, void*
         return dual ? launch_mt<true, float>(MT, X, W, Y, M, N, K, ldx, ldw, ldy, up_off, act, n_waves, s)
                     : launch_mt<false, float>(MT, X, W, Y, M, N, K, ldx, ldw, ldy, up_off, act, n_waves, s);
     return BN_ERR_DTYPE;
+}
+
+// Up to SK_GROUP products of the same M <= 16 rows and K over streamed copies, bf16 results, in one launch.  Arrays of `count`:
+// X, W, Y addresses, N columns, ldx, the copies' rows per tile, and the activation of the results (a BN_UNARY_* or -1).  The
+// results are contiguous [M, N].
+extern "C" int bn_skinny_group(int count, const void* const* X, const void* const* W, void* const* Y, const int* N, const int* ldx,
+                               const int* tile_rows, const int* unary, int M, int K, int k_tiles, hipStream_t s) {
+    if (count < 1 || count > SK_GROUP || M < 1 || M > 16 || !sk_tiled_ok(K, k_tiles)) return BN_ERR_ARG;
+    SkinnyGroup p;
+    p.count = count;
+    int groups = 0;
+    for (int j = 0; j < count; ++j) {
+        if (!bn_skinny_gemm_supports(M, N[j], K, ldx[j], 8) || ldx[j] < K || tile_rows[j] < 1 || tile_rows[j] > BN_STREAM_TILE_ROWS ||
+            unary[j] < -1 || unary[j] >= BN_UNARY_KINDS || (((uintptr_t)X[j] | (uintptr_t)W[j]) & 15) || !Y[j])
+            return BN_ERR_ARG;
+        p.x[j] = (const bf16*)X[j]; p.w[j] = (const bf16*)W[j]; p.y[j] = (bf16*)Y[j];
+        p.n[j] = N[j]; p.ldx[j] = ldx[j]; p.rows[j] = tile_rows[j]; p.act[j] = unary[j] < 0 ? 0 : SK_ACT_UNARY + unary[j];
+        p.first[j] = groups;
+        groups += (N[j] + tile_rows[j] - 1) / tile_rows[j];
+    }
+    int n_waves = 8;
+    const int k_chunks = (K + SK_CHUNK - 1) / SK_CHUNK;
+    while (n_waves > 1 && n_waves / 2 >= k_chunks) n_waves >>= 1;
+    const size_t smem = (size_t)n_waves * 256 * sizeof(float) + (size_t)n_waves * M * SK_XROW;
+    if (smem > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(skinny_group_kernel),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return (int)e;
+    }
+    hipLaunchKernelGGL(skinny_group_kernel, dim3(groups), dim3(n_waves * 64), smem, s, p, M, K, k_tiles);
+    return bn_launch_status();
 }

@@ -582,6 +582,98 @@ extern "C" int bn_head_norm_gate(int dtype, void* y, const float* o, const void*
     return bn_launch_status();
 }
 
+// ---- a decode step of wkv with its norm and gate -------------------------------------------------------------------------
+// One token of every sequence: a workgroup owns a (sequence, head) whole, a thread the rows of a column that the walk gives it
+// (P neighbouring lanes a column), so the state's way in and out is one load and one store a number; the head's root mean
+// square, weight and gate follow on the sums that the lanes hold.  Bound by latency at few sequences (a trip to memory for the
+// state, three barriers): one sequence of 32 heads of 64 6.9 us, where the walk and
+// the norm's kernel took 7.8 + 5.0.
+template <typename T>
+__global__ __launch_bounds__(1024) void wkv_step_kernel(WkvArgs a, T* __restrict__ y, const T* __restrict__ gate, int ldg,
+                                                        const float* __restrict__ weight, float eps) {
+    __shared__ __align__(16) float r_s[WKV_MAX_DIM], k_s[WKV_MAX_DIM], w_s[WKV_MAX_DIM];
+    __shared__ float scratch[16];
+    const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
+    const int pos = a.seq_lens[seq] - 1;
+    if (pos < 0) return;
+    const int P = a.P, dk = a.dk, dv = a.dv, dkp = P * WKV_KR, p = tid % P, j = tid / P;
+    const bool owns = j < dv;
+    float* S_g = a.state + (size_t)a.slot_ids[seq] * a.state_stride + (size_t)head * dkp * dv;
+    float S[WKV_KR], ub[WKV_KR];
+    const int jc = owns ? j : 0;                          // loads in straight line; a thread without a column drops what it loads
+#pragma unroll
+    for (int ii = 0; ii < WKV_KR; ++ii) {
+        S[ii] = S_g[((size_t)ii * dv + jc) * P + p];
+        ub[ii] = a.u[(size_t)head * dk + min(p * WKV_KR + ii, dk - 1)];
+    }
+    const float vj = to_f32(reinterpret_cast<const T*>(a.v)[(size_t)seq * a.ldv + (size_t)head * dv + jc]);
+    const float gj = to_f32(gate[(size_t)seq * ldg + (size_t)head * dv + jc]), wj = weight ? weight[(size_t)head * dv + jc] : 1.0f;
+    for (int i = tid; i < dkp; i += blockDim.x) {
+        const size_t c = (size_t)head * dk + min(i, dk - 1);
+        const float r = to_f32(reinterpret_cast<const T*>(a.r)[(size_t)seq * a.ldr + c]);
+        const float k = to_f32(reinterpret_cast<const T*>(a.k)[(size_t)seq * a.ldk + c]);
+        const float d = to_f32(reinterpret_cast<const T*>(a.d)[(size_t)seq * a.ldd + c]) + a.w0[c];
+        r_s[i] = i < dk ? r : 0.f;
+        k_s[i] = i < dk ? k : 0.f;
+        w_s[i] = i < dk ? expf(-expf(d)) : 0.f;
+    }
+    if (head == 0) {                                      // the step's h, for the next step's shift
+        float* hp = a.state + (size_t)a.slot_ids[seq] * a.state_stride + (size_t)a.H * dkp * dv;
+        for (int e = tid; e < a.D; e += blockDim.x) hp[e] = to_f32(reinterpret_cast<const T*>(a.h)[(size_t)seq * a.D + e]);
+    }
+#pragma unroll
+    for (int ii = 0; ii < WKV_KR; ++ii) {
+        if (pos == 0 || !owns) S[ii] = 0.f;
+        if (p * WKV_KR + ii >= dk) ub[ii] = 0.f;
+    }
+    lds_barrier();
+    float4 rr[WKV_KR / 4], kk[WKV_KR / 4], ww[WKV_KR / 4];
+#pragma unroll
+    for (int q = 0; q < WKV_KR / 4; ++q) {
+        rr[q] = reinterpret_cast<const float4*>(r_s + p * WKV_KR)[q];
+        kk[q] = reinterpret_cast<const float4*>(k_s + p * WKV_KR)[q];
+        ww[q] = reinterpret_cast<const float4*>(w_s + p * WKV_KR)[q];
+    }
+    const float o = wkv_token(rr, kk, ww, vj, ub, S, P);
+    if (owns) {
+#pragma unroll
+        for (int ii = 0; ii < WKV_KR; ++ii) S_g[((size_t)ii * dv + j) * P + p] = S[ii];
+    }
+    const float ss = block_sum(owns && p == 0 ? o * o : 0.f, scratch);
+    const float f = 1.0f / sqrtf(ss / (float)dv + eps);
+    if (owns && p == 0) y[((size_t)seq * a.H + head) * dv + j] = from_f32<T>(o * f * wj * bn_unary_act(gj, BN_UNARY_SILU));
+}
+
+// 1 if a head of these sizes fits a workgroup of the kernel above
+extern "C" int bn_wkv_step_supports(int dk, int dv) {
+    int P, CB, TC, wk, th;
+    return wkv_shape(dk, dv, 1, P, CB, TC, wk, th) && P * dv <= 1024 ? 1 : 0;
+}
+
+extern "C" int bn_wkv_step(int dtype, const void* r, int ldr, const void* k, int ldk, const void* v, int ldv, const void* d, int ldd,
+                           const float* w0, const float* u, const void* h, float* state, long long state_stride,
+                           const int* seq_lens, const int* slot_ids, int n_seqs, int H, int dk, int dv, int D, void* y,
+                           const void* gate, int ldg, const float* weight, float eps, hipStream_t s) {
+    WkvArgs a = {};
+    int threads;
+    if (n_seqs <= 0 || H <= 0 || D <= 0 || !bn_wkv_step_supports(dk, dv) || !wkv_shape(dk, dv, 1, a.P, a.CB, a.TC, a.walkers, threads))
+        return BN_ERR_ARG;
+    if (!r || !k || !v || !d || !w0 || !u || !h || !state || !slot_ids || !seq_lens || !y || !gate || ldg < H * dv) return BN_ERR_ARG;
+    if (state_stride < (long long)H * a.P * WKV_KR * dv + D) return BN_ERR_ARG;
+    a.r = r; a.k = k; a.v = v; a.d = d; a.ldr = ldr; a.ldk = ldk; a.ldv = ldv; a.ldd = ldd;
+    a.w0 = w0; a.u = u; a.h = h; a.state = state; a.state_stride = (size_t)state_stride;
+    a.seq_lens = seq_lens; a.slot_ids = slot_ids;
+    a.H = H; a.dk = dk; a.dv = dv; a.D = D;
+    const dim3 grid(n_seqs, H), block((a.P * dv + BN_WAVE - 1) / BN_WAVE * BN_WAVE);
+    if (dtype == BN_DT_F32)
+        hipLaunchKernelGGL(wkv_step_kernel<float>, grid, block, 0, s, a, (float*)y, (const float*)gate, ldg, weight, eps);
+    else if (dtype == BN_DT_BF16)
+        hipLaunchKernelGGL(wkv_step_kernel<bf16>, grid, block, 0, s, a, (bf16*)y, (const bf16*)gate, ldg, weight, eps);
+    else
+        return BN_ERR_DTYPE;
+    return bn_launch_status();
+}
+
 // ---- min-GRU ------------------------------------------------------------------------------------------------------
 // zxg [T, ld]: the three projections side by side (update gate at 0, candidate at W, output gate at 2 W), without their
 // biases.  A workgroup owns GRU_CH channels of one sequence.  Its tokens come in stages of GRU_TC: all threads load a

@@ -132,6 +132,10 @@ _SIGNATURES = {
         "bn_wkv_scan": [c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p,
                         c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int,
                         c_int, c_int, c_void_p, c_void_p, c_void_p],
+        "bn_wkv_step_supports": [c_int, c_int],
+        "bn_wkv_step": [c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
+                        c_void_p, c_longlong, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int,
+                        c_void_p, c_float, c_void_p],
         "bn_head_norm_gate": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_float, c_void_p],
         "bn_mingru_scan": [c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_int,
                            c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p],
@@ -187,6 +191,8 @@ _SIGNATURES = {
                            c_int, c_int, c_int, c_void_p],
         "bn_skinny_gemm_fused_tile_cols": [c_int],
         "bn_skinny_gemm_fused_tiles": [c_int, c_int],
+        "bn_skinny_group": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
+                            c_void_p],
         "bn_skinny_gemm_fused": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                  c_void_p, c_int, c_int, c_float, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p,
                                  c_int, c_void_p],
@@ -646,23 +652,52 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, *, allow_library: O
     return _tiled(x, w, out_dtype)
 
 
+_ACT_UNARY = _build.header_constant("SK_ACT_UNARY", "skinny_gemm.hip")     # + a unary activation's number: the products' act
+
+
 def linear_unary(x: torch.Tensor, w: torch.Tensor, activation: str, streamed: Optional[StreamedWeight] = None) -> torch.Tensor:
     """activation(linear(x, w)) (one of UNARY_ACTIVATIONS): a feed-forward's first product without a gate.  bf16 steps of up
-    to 16 rows form relu2 in the product's own kernel; everything else is the product, then the activation's kernel."""
+    to 16 rows form it in the product's own kernel, on the float32 sums; everything else is the product, then the
+    activation's kernel."""
     require_gpu()
     _dev(x, "x", dims=2)
     _dev(w, "w", x.dtype, 2)
     M, K = x.shape
     N = w.shape[0]
-    if (activation == "relu2" and x.dtype == torch.bfloat16 and 1 <= M <= SKINNY_ROWS and w.shape[1] == K
+    if (x.dtype == torch.bfloat16 and 1 <= M <= SKINNY_ROWS and w.shape[1] == K
             and (x.data_ptr() | w.data_ptr()) % 16 == 0 and skinny_supported(M, N, K, _rows(x, "x"), _rows(w, "w"))):
         y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
         wp, wl, tiled = _weight_arg(w, streamed, "linear_unary")
+        act = _act("relu2") if activation == "relu2" else _ACT_UNARY + UNARY_ACTIVATIONS[activation]
         _check(_fn("skinny_gemm", "bn_skinny_gemm")(_code(torch.bfloat16), x.data_ptr(), wp, y.data_ptr(), M, N, K, _rows(x, "x"),
-                                                    wl, N, 0, 0, _act("relu2"), tiled, _stream()), "skinny_gemm(relu2)")
+                                                    wl, N, 0, 0, act, tiled, _stream()), "skinny_gemm(unary)")
         return y
     y = linear(x, w, streamed=streamed)
     return unary_act(y, activation, out=y)
+
+
+GROUP_PRODUCTS = _build.header_constant("SK_GROUP", "skinny_gemm.hip")
+
+
+def linear_group(items) -> list:
+    """[linear(x, w) or activation(linear(x, w))] for items (x, w, streamed copy of w or None, activation or None) whose
+    products do not depend on each other: one launch for bf16 steps of up to 16 rows over streamed copies of matrices with
+    equally many columns, else one after the other."""
+    items = list(items)
+    M, K = items[0][0].shape
+    if (len(items) > 1 and len(items) <= GROUP_PRODUCTS and 1 <= M <= SKINNY_ROWS
+            and all(x.dtype == w.dtype == torch.bfloat16 and tuple(x.shape) == (M, K) and w.shape[1] == K and sw is not None
+                    and x.data_ptr() % 16 == 0 and skinny_supported(M, w.shape[0], K, _rows(x, "x"), 8) for x, w, sw, _ in items)):
+        n = len(items)
+        ys = [torch.empty((M, w.shape[0]), dtype=torch.bfloat16, device=x.device) for x, w, _, _ in items]
+        args = [_weight_arg(w, sw, "linear_group") for _, w, sw, _ in items]
+        ptr, num = c_void_p * n, c_int * n
+        _check(_fn("skinny_gemm", "bn_skinny_group")(
+            n, ptr(*[x.data_ptr() for x, _, _, _ in items]), ptr(*[a[0] for a in args]), ptr(*[y.data_ptr() for y in ys]),
+            num(*[w.shape[0] for _, w, _, _ in items]), num(*[_rows(x, "x") for x, _, _, _ in items]), num(*[a[2] for a in args]),
+            num(*[-1 if act is None else UNARY_ACTIVATIONS[act] for _, _, _, act in items]), M, K, args[0][1], _stream()), "skinny_group")
+        return ys
+    return [linear(x, w, streamed=sw) if act is None else linear_unary(x, w, act, sw) for x, w, sw, act in items]
 
 
 def interleave_gate_up(w_gate: torch.Tensor, w_up: torch.Tensor) -> torch.Tensor:
@@ -1964,6 +1999,52 @@ def _scan_pieces(pieces, tl, T: int, n_seqs: int, groups: int, piece: int, float
     return most, torch.empty((most, floats), dtype=torch.float32, device=device)
 
 
+def _wkv_args(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, what: str):
+    _dev(h, "h", dims=2)
+    T, D = h.shape
+    if not wkv_supported(dk, dv):
+        raise KernelError(f"{what}: head sizes up to {WKV_MAX_DIM}, got {dk} x {dv}")
+    for t, nm, n in ((r, "r", H * dk), (k, "k", H * dk), (v, "v", H * dv), (d, "d", H * dk)):
+        _dev(t, nm, h.dtype, 2)
+        if t.shape != (T, n):
+            raise KernelError(f"{what}: {nm} must be [{T}, {n}], got {tuple(t.shape)}")
+    for t, nm in ((w0, "w0"), (u, "u")):
+        _dev(t, nm, torch.float32, 1)
+        if t.numel() != H * dk or not t.is_contiguous():
+            raise KernelError(f"{what}: {nm} must hold {H * dk} float32 values")
+    if not h.is_contiguous():
+        raise KernelError(f"{what}: h must be contiguous")
+    _dev(slot_ids, "slot_ids", torch.int32, 1)
+    return T, D, _state_rows(state, wkv_state_floats(H, dk, dv) + D, what)
+
+
+def wkv_step_supported(dk: int, dv: int) -> bool:
+    return bool(_fn("state_mixers", "bn_wkv_step_supports")(int(dk), int(dv)))
+
+
+def wkv_step(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, seq_lens, gate: torch.Tensor,
+             weight: Optional[torch.Tensor], eps: float) -> torch.Tensor:
+    """head_norm_gate(wkv_scan(...)) of a decode step in one kernel: [T, H dv] in h's type."""
+    require_gpu()
+    T, D, stride = _wkv_args(r, k, v, d, w0, u, h, state, slot_ids, H, dk, dv, "wkv_step")
+    _, n_seqs, sl = _seq_args(None, seq_lens, "wkv_step")
+    _dev(gate, "gate", h.dtype, 2)
+    if not wkv_step_supported(dk, dv) or n_seqs != T or tuple(gate.shape) != (T, H * dv):
+        raise KernelError(f"wkv_step: {n_seqs} sequences, h {tuple(h.shape)}, gate {tuple(gate.shape)}, heads of {dk} x {dv}")
+    if weight is not None:
+        _dev(weight, "weight", torch.float32, 1)
+        if weight.numel() != H * dv or not weight.is_contiguous():
+            raise KernelError(f"wkv_step: weight must hold {H * dv} float32 values")
+    y = torch.empty((T, H * dv), dtype=h.dtype, device=h.device)
+    if T:
+        _check(_fn("state_mixers", "bn_wkv_step")(
+            _code(h.dtype), r.data_ptr(), _rows(r, "r"), k.data_ptr(), _rows(k, "k"), v.data_ptr(), _rows(v, "v"), d.data_ptr(),
+            _rows(d, "d"), w0.data_ptr(), u.data_ptr(), h.data_ptr(), state.data_ptr(), stride, sl, slot_ids.data_ptr(), T, H, dk, dv,
+            D, y.data_ptr(), gate.data_ptr(), _rows(gate, "gate"), weight.data_ptr() if weight is not None else None, float(eps),
+            _stream()), "wkv_step")
+    return y
+
+
 def wkv_scan(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, *, tiles=None, seq_lens=None,
              pieces: Optional[bool] = None) -> torch.Tensor:
     """The wkv recurrence over every sequence of a step; float32 [T, H dv].  r, k, d: [T, H dk] (rows contiguous, any row
@@ -1974,22 +2055,7 @@ def wkv_scan(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, *,
     pieces (prompt form): whether every sequence is cut into pieces of WKV_PIECE tokens that are walked side by side (the
     results differ from the plain walk's by rounding alone); None: by the step's size (_scan_pieces)."""
     require_gpu()
-    _dev(h, "h", dims=2)
-    T, D = h.shape
-    if not wkv_supported(dk, dv):
-        raise KernelError(f"wkv_scan: head sizes up to {WKV_MAX_DIM}, got {dk} x {dv}")
-    for t, nm, n in ((r, "r", H * dk), (k, "k", H * dk), (v, "v", H * dv), (d, "d", H * dk)):
-        _dev(t, nm, h.dtype, 2)
-        if t.shape != (T, n):
-            raise KernelError(f"wkv_scan: {nm} must be [{T}, {n}], got {tuple(t.shape)}")
-    for t, nm in ((w0, "w0"), (u, "u")):
-        _dev(t, nm, torch.float32, 1)
-        if t.numel() != H * dk or not t.is_contiguous():
-            raise KernelError(f"wkv_scan: {nm} must hold {H * dk} float32 values")
-    if not h.is_contiguous():
-        raise KernelError("wkv_scan: h must be contiguous")
-    stride = _state_rows(state, wkv_state_floats(H, dk, dv) + D, "wkv_scan")
-    _dev(slot_ids, "slot_ids", torch.int32, 1)
+    T, D, stride = _wkv_args(r, k, v, d, w0, u, h, state, slot_ids, H, dk, dv, "wkv_scan")
     tl, n_tiles, sl = _seq_args(tiles, seq_lens, "wkv_scan")
     o = torch.empty((T, H * dv), dtype=torch.float32, device=h.device)
     floats = wkv_state_floats(H, dk, dv)

@@ -201,7 +201,13 @@ class Attention(Part):
         return bool(ctx.is_decode and fuse_ok and inv_freq is not None and not self.has_bias and ops.LIBRARY_PRODUCTS
                     and ops.can_fuse_decode(self.qkv.weight.dtype, self.H, self.Hkv, self.hs))
 
-    def _forward_general(self, h, ctx, kv, lazy_ok: bool = False):
+    @property
+    def ends(self):
+        """The products that a mixer beside this one may run together with its own (ops.linear_group); None where the first or
+        the last has a bias, or the form is not the general one."""
+        return (self.qkv, self.o) if self.general and self.qkv.bias is None and self.o.bias is None else None
+
+    def _forward_general(self, h, ctx, kv, lazy_ok: bool = False, projected=None):
         """Projections; biases, norms, rotation and temperature with the cache write (one kernel); attention with its window,
         distance bias, sink and output gate (prompt steps on the matrix cores where the sizes allow, else the vector kernel); the
         output projection."""
@@ -209,7 +215,9 @@ class Attention(Part):
         if isinstance(h, ops.DeferredNorm):
             h = h.materialize()
         width = H * hs + Hkv * (hs if self.value_is_key else hs + vd) + (H * vd if self.out_gate else 0)
-        if kv.writes or self.out_gate:
+        if projected is not None:             # the first product's result; the last is left to whoever gave it
+            qkv = projected
+        elif kv.writes or self.out_gate:
             qkv = self.qkv(h)
         else:
             qkv = torch.empty((h.shape[0], width), dtype=h.dtype, device=h.device)
@@ -268,6 +276,8 @@ class Attention(Part):
                           sink=self._sink(), **mask)
         if gate is not None and not on_matrix_cores:      # the matrix-core kernels multiply by it as they store
             ops.sigmoid_gate_(out, gate)
+        if projected is not None:
+            return out
         return self.o.lazy(out) if lazy_ok else self.o(out)
 
     def _sink(self):
@@ -279,9 +289,9 @@ class Attention(Part):
             self._empty_state = torch.zeros((1, 1), dtype=torch.float32, device=device)
         return self._empty_state
 
-    def forward(self, h, ctx, kv, lazy_ok: bool = False):
+    def forward(self, h, ctx, kv, lazy_ok: bool = False, projected=None):
         if self.general:
-            return self._forward_general(h, ctx, kv, lazy_ok)
+            return self._forward_general(h, ctx, kv, lazy_ok, projected)
         H, Hkv, hs = self.H, self.Hkv, self.hs
         last = self.o.lazy if lazy_ok else self.o
         fuse_ok, inv_freq = self.position.fusable(hs)

@@ -68,6 +68,13 @@ class ParallelMixer(Part):
         if self.state_split is not None:
             kv_a = dataclasses.replace(kv, state=kv.state[:, :self.state_split])
             kv_b = dataclasses.replace(kv, state=kv.state[:, self.state_split:])
-        a = self.left.forward(h, ctx, kv_a)
-        b = self.right.forward(h, ctx, kv_b)
+        ends = [getattr(m, "ends", None) for m in (self.left, self.right)]
+        if all(ends) and kv.writes and isinstance(h, torch.Tensor):
+            # both read h, and neither's last product waits for the other: two launches instead of four where steps are short
+            pa, pb = ops.linear_group([(h, first.weight, first.streamed, None) for first, _ in ends])
+            ya, yb = self.left.forward(h, ctx, kv_a, projected=pa), self.right.forward(h, ctx, kv_b, projected=pb)
+            a, b = ops.linear_group([(y, last.weight, last.streamed, None) for y, (_, last) in zip((ya, yb), ends)])
+        else:
+            a = self.left.forward(h, ctx, kv_a)
+            b = self.right.forward(h, ctx, kv_b)
         return ops.rmsnorm_mean(a, self.w_left, b, self.w_right, self.eps)

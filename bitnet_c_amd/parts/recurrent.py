@@ -84,7 +84,7 @@ class WKV(Part):
         self.norm = upload(tensors["norm"], device, torch.float32)
 
     def linears(self):
-        return [self.r, self.k, self.v, self.g, self.o]
+        return [self.r, self.k, self.v, self.g, self.w1, self.w2, self.o]
 
     def cache_need(self) -> CacheNeed:
         # per head a [head_dim, head_dim] matrix (in the kernel's own order and rounding of its rows), then the last input row
@@ -94,12 +94,14 @@ class WKV(Part):
         H, hs = self.H, self.hs
         state = kv.state
         mixes = ops.token_shift(h, self.mu, state[:, self.state_floats:], ctx.positions, ctx.seq_index, ctx.slot_ids)
-        r, k, v, g = self.r(mixes[0]), self.k(mixes[1]), self.v(mixes[2]), self.g(mixes[3])
-        low = self.w1(mixes[4])
-        ops.unary_act(low, "tanh", out=low)
+        r, k, v, g, low = ops.linear_group([(x, l.weight, l.streamed, None) for x, l in zip(mixes, (self.r, self.k, self.v, self.g))]
+                                           + [(mixes[4], self.w1.weight, self.w1.streamed, "tanh")])
         d = self.w2(low)
-        o = ops.wkv_scan(r, k, v, d, self.w0, self.u, h, state, ctx.slot_ids, H, hs, hs, **_sequences(ctx))
-        y = ops.head_norm_gate(o, g, self.norm, H, hs, self.eps)
+        if ctx.is_decode and ops.wkv_step_supported(hs, hs):
+            y = ops.wkv_step(r, k, v, d, self.w0, self.u, h, state, ctx.slot_ids, H, hs, hs, ctx.seq_lens, g, self.norm, self.eps)
+        else:
+            o = ops.wkv_scan(r, k, v, d, self.w0, self.u, h, state, ctx.slot_ids, H, hs, hs, **_sequences(ctx))
+            y = ops.head_norm_gate(o, g, self.norm, H, hs, self.eps)
         return self.o(y)
 
 
@@ -132,10 +134,16 @@ class MinGRU(Part):
     def cache_need(self) -> CacheNeed:
         return CacheNeed(state=StateNeed((self.W,), torch.float32, device_addressed=True))
 
-    def forward(self, h, ctx, kv):
-        zxg = self.zxg(h)
+    @property
+    def ends(self):
+        """The products that a mixer beside this one may run together with its own (ops.linear_group)."""
+        return self.zxg, self.o
+
+    def forward(self, h, ctx, kv, projected=None):
+        """projected: the first product's result; the last product is then left to whoever gave it."""
+        zxg = self.zxg(h) if projected is None else projected
         y = ops.mingru_scan(zxg, self.bz, self.bx, kv.state, ctx.slot_ids, self.W, **_sequences(ctx))
-        return self.o(y)
+        return self.o(y) if projected is None else y
 
 
 class DecayedSums(Part):

@@ -1,0 +1,89 @@
+"""Products that share a launch, activations in a product's own kernel, the decode step of wkv with its norm and gate, and the
+mean of two normed branches in 16-byte groups: each against the kernels that do the same one by one."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rand(shape, seed, dtype=torch.float32):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(shape, generator=g).to(dtype).cuda()
+
+
+# columns: less than a tile, not a multiple of one, several tile heights; K: under, at and over a wave's chunk of 256, more
+# chunks than waves
+@pytest.mark.parametrize("M", [1, 5, 16, 17])
+@pytest.mark.parametrize("K,Ns,rows", [(64, [16, 8, 33], [16, 8, 12]), (256, [2048, 64], [8, 16]), (264, [100] * 6, [10] * 6),
+                                       (2304, [48, 5, 640, 16], [16, 5, 12, 3])])
+def test_group_is_the_products_one_by_one(M, K, Ns, rows):
+    from bitnet_c_amd import ops
+    acts = ["tanh", None, "gelu_erf", None, "silu", "sigmoid"]
+    items, want = [], []
+    for j, (N, R) in enumerate(zip(Ns, rows)):
+        x, w = _rand((M, K), j, torch.bfloat16), _rand((N, K), 50 + j, torch.bfloat16)
+        sw = ops.stream_copy(w, R)
+        items.append((x, w, sw, acts[j]))
+        want.append(ops.linear(x, w, streamed=sw) if acts[j] is None else ops.linear_unary(x, w, acts[j], sw))
+    got = ops.linear_group(items)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    items[0] = items[0][:2] + (None,) + items[0][3:]                  # a matrix without a streamed copy: one by one
+    assert all(torch.equal(a, b) for a, b in zip(ops.linear_group(items), want))
+
+
+@pytest.mark.parametrize("activation", ["gelu_erf", "gelu_tanh", "silu", "relu2", "tanh", "sigmoid"])
+@pytest.mark.parametrize("M", [1, 16, 17])
+def test_activation_in_the_product(activation, M):
+    from bitnet_c_amd import ops
+    x, w = _rand((M, 320), 1, torch.bfloat16), _rand((72, 320), 2, torch.bfloat16) / 16
+    z = (x.double() @ w.double().t()).float()
+    want = ops.unary_act(z.clone(), activation).double()
+    for sw in (None, ops.stream_copy(w)):
+        y = ops.linear_unary(x, w, activation, sw).double()
+        # one rounding of the result (2^-9) up to 16 rows, and one of the product before the activation beyond (every activation
+        # here moves by at most 2 |z| of what its argument moves by)
+        tol = 2.0 ** -8 * want.abs() + 2.0 ** -16 * 320 ** 0.5 + (2.0 ** -8 * 2 * (1 + z.abs()).double() ** 2 if M > 16 else 0.0)
+        assert torch.all((y - want).abs() <= tol)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,d", [(2, 64), (3, 24), (1, 128), (5, 8)])
+@pytest.mark.parametrize("weighted", [True, False])
+def test_wkv_step(dtype, H, d, weighted):
+    """Sequences at position 0 and later, a padding row; state, last row and outputs as the scan and the norm leave them."""
+    from bitnet_c_amd import ops
+    if not ops.wkv_step_supported(d, d):
+        pytest.skip("a head of this size does not fit the kernel")
+    B, A, D = 4, H * d, 40
+    r, k, v, dd, g = (_rand((B, A), 10 + i, dtype) for i in range(5))
+    h, w0, u = _rand((B, D), 20, dtype), _rand((A,), 21) - 2.0, _rand((A,), 22)
+    weight = _rand((A,), 23) if weighted else None
+    n = ops.wkv_state_floats(H, d, d)
+    state = torch.zeros(6, n + D).cuda()
+    lens, slots = torch.tensor([1, 9, 0, 3], dtype=torch.int32).cuda(), torch.tensor([4, 0, 5, 2], dtype=torch.int32).cuda()
+    for i in range(3):                                    # a state that the kernels themselves have made
+        ops.wkv_scan(r * (i + 1), k, v, dd, w0, u, h, state, slots, H, d, d, seq_lens=torch.tensor([5, 5, 0, 5], dtype=torch.int32).cuda())
+    a, b = state.clone(), state.clone()
+    o = ops.wkv_scan(r, k, v, dd, w0, u, h, a, slots, H, d, d, seq_lens=lens)
+    want = ops.head_norm_gate(o, g, weight, H, d, 1e-6)
+    got = ops.wkv_step(r, k, v, dd, w0, u, h, b, slots, H, d, d, lens, g, weight, 1e-6)
+    assert torch.equal(a, b)
+    live = [0, 1, 3]
+    # the same sums but for the order of the squares': the factor moves by some roundings of 2^-24, a bf16 result by one of its own
+    tol = 2.0 ** -7 if dtype == torch.bfloat16 else 1e-6
+    assert torch.all((got[live] - want[live]).abs() <= tol * want[live].abs() + 1e-30)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim", [8, 2048, 2056, 4096, 8192, 2052, 37])
+@pytest.mark.parametrize("two", [True, False])
+def test_rmsnorm_mean(dtype, dim, two):
+    from bitnet_c_amd import ops
+    a, b = _rand((3, dim), 1, dtype), _rand((3, dim), 2, dtype) * 5
+    wa, wb = _rand((dim,), 3), _rand((dim,), 4)
+    unit = lambda t: t.double() / torch.sqrt((t.double() ** 2).mean(-1, keepdim=True) + 1e-5)
+    want = 0.5 * (unit(a) * wa.double() + unit(b) * wb.double()) if two else unit(a) * wa.double()
+    got = ops.rmsnorm_mean(a, wa, b, wb, 1e-5) if two else ops.rmsnorm_mean(a, wa, None, None, 1e-5)
+    # a float32 sum of dim squares and a few products, then the result's own rounding
+    tol = (2.0 ** -8 if dtype == torch.bfloat16 else 0.0) + 2.0 ** -24 * (dim ** 0.5 + 8)
+    assert float((got.double() - want).abs().max()) <= tol * float(want.abs().max())
