@@ -99,19 +99,25 @@ __global__ __launch_bounds__(LA_THREADS) void lightning_scan_kernel(LaArgs a) {
     const bool has = c < a.dv;
     float* sp = a.state + (size_t)a.slot_ids[sr.seq] * a.state_stride + (size_t)head * a.dk * a.dv + c;
     float S[RPT];
+    // unconditional loads from places that exist (one under a branch is waited for where it stands), used or not below
+    const float* sl = has ? sp : sp - c;
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) S[i] = (has && r0 + i < a.dk && sr.pos0 > 0) ? sp[(size_t)(r0 + i) * a.dv] : 0.f;
+    for (int i = 0; i < RPT; ++i) S[i] = sl[(size_t)min(r0 + i, a.dk - 1) * a.dv];
+#pragma unroll
+    for (int i = 0; i < RPT; ++i)
+        if (!has || r0 + i >= a.dk || sr.pos0 <= 0) S[i] = 0.f;
     const float decay = a.decay[head];
     const T* x = reinterpret_cast<const T*>(a.x) + (size_t)sr.row0 * a.ld;
     float* o = a.o + (size_t)sr.row0 * a.H * a.dv + (size_t)head * a.dv + c0;
     for (int t0 = 0; t0 < sr.n; t0 += LA_TC) {
         const int nt = min(LA_TC, sr.n - t0);
         const int rd = a.feed.rope_dims, half = rd / 2;
-        for (int idx = tid; idx < LA_TC * DKP; idx += LA_THREADS) {
+        // (places of tokens that the chunk does not hold are not read: a decode step stages its one token)
+        for (int idx = tid; idx < nt * DKP; idx += LA_THREADS) {
             const int tt = idx / DKP, r = idx - tt * DKP;
             if (r < rd) continue;                        // the rotated dimensions, pair by pair, below
             float qv = 0.f, kv = 0.f;
-            if (tt < nt && r < a.dk) {
+            if (r < a.dk) {
                 const T* row = x + (size_t)(t0 + tt) * a.ld + (size_t)head * a.dk + r;
                 qv = la_act(to_f32(row[a.q_col]), a.feed.silu);
                 kv = la_act(to_f32(row[a.k_col]), a.feed.silu) * a.feed.k_scale;
@@ -119,24 +125,21 @@ __global__ __launch_bounds__(LA_THREADS) void lightning_scan_kernel(LaArgs a) {
             q_s[idx] = qv;
             k_s[idx] = kv;
         }
-        for (int idx = tid; idx < LA_TC * half; idx += LA_THREADS) {
+        for (int idx = tid; idx < nt * half; idx += LA_THREADS) {
             const int tt = idx / half, r = idx - tt * half;
-            float q0 = 0.f, q1 = 0.f, k0 = 0.f, k1 = 0.f;
-            if (tt < nt) {
-                const T* row = x + (size_t)(t0 + tt) * a.ld + (size_t)head * a.dk + r;
-                float sn, cs;
-                sincosf((float)(sr.pos0 + t0 + tt) * a.feed.inv_freq[r], &sn, &cs);
-                q0 = la_act(to_f32(row[a.q_col]), a.feed.silu); q1 = la_act(to_f32(row[a.q_col + half]), a.feed.silu);
-                k0 = la_act(to_f32(row[a.k_col]), a.feed.silu); k1 = la_act(to_f32(row[a.k_col + half]), a.feed.silu);
-                la_turn(q0, q1, sn, cs);
-                la_turn(k0, k1, sn, cs);
-            }
+            const T* row = x + (size_t)(t0 + tt) * a.ld + (size_t)head * a.dk + r;
+            float sn, cs;
+            sincosf((float)(sr.pos0 + t0 + tt) * a.feed.inv_freq[r], &sn, &cs);
+            float q0 = la_act(to_f32(row[a.q_col]), a.feed.silu), q1 = la_act(to_f32(row[a.q_col + half]), a.feed.silu);
+            float k0 = la_act(to_f32(row[a.k_col]), a.feed.silu), k1 = la_act(to_f32(row[a.k_col + half]), a.feed.silu);
+            la_turn(q0, q1, sn, cs);
+            la_turn(k0, k1, sn, cs);
             q_s[tt * DKP + r] = q0; q_s[tt * DKP + half + r] = q1;
             k_s[tt * DKP + r] = k0 * a.feed.k_scale; k_s[tt * DKP + half + r] = k1 * a.feed.k_scale;
         }
-        for (int idx = tid; idx < LA_TC * LA_CB; idx += LA_THREADS) {
+        for (int idx = tid; idx < nt * LA_CB; idx += LA_THREADS) {
             const int tt = idx / LA_CB, cc = idx - tt * LA_CB;
-            v_s[idx] = (tt < nt && c0 + cc < a.dv)
+            v_s[idx] = (c0 + cc < a.dv)
                            ? la_act(to_f32(x[(size_t)(t0 + tt) * a.ld + a.v_col + (size_t)head * a.dv + c0 + cc]), a.feed.silu) : 0.f;
         }
         __syncthreads();
@@ -536,9 +539,66 @@ __global__ __launch_bounds__(256) void row_norm_gate_kernel(T* __restrict__ y, c
         y[(size_t)t * W + e] = from_f32<T>(ov[e] * f * weight[e] * bn_unary_act(to_f32(gate[(size_t)t * ldg + e]), act));
 }
 
+// The same with the row in registers, eight numbers a thread and group (W and the gate's rows in groups of eight, everything
+// 16-byte aligned): one trip to memory and one sum over the workgroup.  W 2,048, four rows: 5.1 us (9.2
+// with a number a thread in two passes over memory).
+template <typename T, int G>
+__global__ __launch_bounds__(256) void row_norm_gate_wide_kernel(T* __restrict__ y, const float* __restrict__ o, const T* __restrict__ gate,
+                                                                 int ldg, const float* __restrict__ weight, int W, float eps, int act) {
+    struct __align__(16) GateGroup { T e[8]; };
+    __shared__ float scratch[16];
+    const size_t t = blockIdx.x;
+    const int groups = W / 8;
+    float ov[G][8], wv[G][8], gv[G][8];
+    float ss = 0.f;
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+        const int at = min((int)threadIdx.x + 256 * q, groups - 1) * 8;
+        const GateGroup g = *reinterpret_cast<const GateGroup*>(gate + t * ldg + at);
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+            *reinterpret_cast<float4*>(&ov[q][e]) = *reinterpret_cast<const float4*>(o + t * W + at + e);
+            *reinterpret_cast<float4*>(&wv[q][e]) = *reinterpret_cast<const float4*>(weight + at + e);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) gv[q][e] = to_f32(g.e[e]);
+    }
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+        if ((int)threadIdx.x + 256 * q < groups)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss = fmaf(ov[q][e], ov[q][e], ss);
+    ss = block_sum(ss, scratch);
+    const float f = 1.0f / sqrtf(ss / (float)W + eps);
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+        const int at = ((int)threadIdx.x + 256 * q) * 8;
+        if (at >= W) continue;
+        GateGroup r;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r.e[e] = from_f32<T>(ov[q][e] * f * wv[q][e] * bn_unary_act(gv[q][e], act));
+        *reinterpret_cast<GateGroup*>(y + t * W + at) = r;
+    }
+}
+
+template <typename T>
+static bool launch_row_norm_gate_wide(T* y, const float* o, const T* gate, int ldg, const float* weight, int n_rows, int W, float eps,
+                                      int act, hipStream_t s) {
+    const int per = (W / 8 + 255) / 256;
+    if (W % 8 || ldg % 8 || per > 4 || (((uintptr_t)y | (uintptr_t)o | (uintptr_t)gate | (uintptr_t)weight) & 15)) return false;
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(n_rows), dim3(256), 0, s, y, o, gate, ldg, weight, W, eps, act); };
+    if (per == 1) go(row_norm_gate_wide_kernel<T, 1>);
+    else if (per == 2) go(row_norm_gate_wide_kernel<T, 2>);
+    else go(row_norm_gate_wide_kernel<T, 4>);
+    return true;
+}
+
 extern "C" int bn_row_norm_gate(int dtype, void* y, const float* o, const void* gate, int ldg, const float* weight, int n_rows,
                                 int W, float eps, int act, hipStream_t s) {
     if (n_rows <= 0 || W <= 0 || !y || !o || !gate || !weight || ldg < W || act < 0 || act >= BN_UNARY_KINDS) return BN_ERR_ARG;
+    if (dtype == BN_DT_F32 ? launch_row_norm_gate_wide((float*)y, o, (const float*)gate, ldg, weight, n_rows, W, eps, act, s)
+        : dtype == BN_DT_BF16 && launch_row_norm_gate_wide((bf16*)y, o, (const bf16*)gate, ldg, weight, n_rows, W, eps, act, s))
+        return bn_launch_status();
     if (dtype == BN_DT_F32)
         hipLaunchKernelGGL(row_norm_gate_kernel<float>, dim3(n_rows), dim3(256), 0, s, (float*)y, o, (const float*)gate, ldg, weight,
                            W, eps, act);

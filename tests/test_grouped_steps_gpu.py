@@ -87,3 +87,45 @@ def test_rmsnorm_mean(dtype, dim, two):
     # a float32 sum of dim squares and a few products, then the result's own rounding
     tol = (2.0 ** -8 if dtype == torch.bfloat16 else 0.0) + 2.0 ** -24 * (dim ** 0.5 + 8)
     assert float((got.double() - want).abs().max()) <= tol * float(want.abs().max())
+
+
+# widths: one group of eight, a workgroup's 256 groups and one past them, the most that registers hold (8,192) and beyond, not a
+# multiple of eight
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim", [8, 2048, 2056, 8192, 8200, 36])
+@pytest.mark.parametrize("parts", [0, 1, 3])
+@pytest.mark.parametrize("form", ["norm", "rows", "sum"])
+def test_add_normed_rmsnorm_widths(dtype, dim, parts, form):
+    from bitnet_c_amd import ops
+    T = 3
+    x, wb, w = _rand((T, dim), 1), _rand((dim,), 2), _rand((dim,), 3)
+    if parts:
+        delta = ops.PartialSums(_rand((parts, T, dim), 4))
+        d = delta.slabs.double().sum(0)
+    else:
+        delta = _rand((T, dim), 4, dtype)
+        d = delta.double()
+    new = x.double() + d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-6) * wb.double()
+    want = new / torch.sqrt((new * new).mean(-1, keepdim=True) + 1e-5) * w.double() if form == "norm" else new
+    kw = dict(weight=w, eps=1e-5, out_dtype=dtype) if form == "norm" else dict(out_dtype=dtype, rows_out=True) if form == "rows" else {}
+    out = ops.add_normed_rmsnorm(x, delta, wb, 1e-6, **kw)
+    # float32 sums of dim squares and a handful of products; the result's own rounding
+    tol = 2.0 ** -24 * (dim ** 0.5 + 16)
+    assert float((x.double() - new).abs().max()) <= tol * float(new.abs().max())
+    if form != "sum":
+        tol += 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+        assert float((out.double() - want).abs().max()) <= tol * float(want.abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("W", [8, 2048, 2056, 8192, 8200, 36])
+def test_row_norm_gate_widths(dtype, W):
+    from bitnet_c_amd import ops
+    T = 3
+    o, weight = _rand((T, W), 1), _rand((W,), 2)
+    gate = _rand((T, W + 24), 3, dtype)[:, 16:16 + W]
+    f = o.double() / torch.sqrt((o.double() ** 2).mean(-1, keepdim=True) + 1e-6)
+    want = f * weight.double() * torch.sigmoid(gate.double())
+    got = ops.row_norm_gate(o, gate, weight, 1e-6)
+    tol = (2.0 ** -8 if dtype == torch.bfloat16 else 0.0) + 2.0 ** -24 * (W ** 0.5 + 16)
+    assert float((got.double() - want).abs().max()) <= tol * float(want.abs().max())
