@@ -2,7 +2,8 @@
 // values of a width of their own (a multiple of 32), a logarithmic distance bias, a sink in the softmax, no rotation
 // (the queries and keys arrive encoded).  bf16, 16x16x32 MFMA.  Keys lie in pages with a row per position
 // ([page, kv head, BN_PAGE, hs]), values transposed ([page, kv head, vd, BN_PAGE]): both operands of both products are
-// then 16 consecutive bytes a lane, straight from the pages (no shared memory, no barrier: a wave is on its own).
+// then 16 consecutive bytes a lane.  The prompt form lays them out through shared memory, the decode form takes them straight
+// from the pages.
 //
 // A wave owns one tile of up to 16 query tokens of one head and walks the keys 0 .. last query in blocks of 32 (with a
 // window w > 0 a query at position i sees the keys i - w + 1 .. i only, and the walk begins at the block of the tile's
@@ -30,9 +31,9 @@
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(8))) float f32x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 
 #define AG_LOG2E 1.4426950408889634f
-#define AG_WAVES 4            // waves (heads) of a workgroup
 
 struct GenArgs {
     const bf16* q;            // [T, q_stride]: head h at h * hs, norms and temperature applied
@@ -55,6 +56,15 @@ struct GenArgs {
 
 __device__ __forceinline__ bf16x8 ag_ld16(const bf16* p) {
     return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
+}
+
+// the largest of a value over the lanes 16, 32 and 48 away (the four lane groups of a column): two half-wave swaps between registers
+__device__ __forceinline__ float ag_max_over_groups(float x) {
+    const unsigned b = __float_as_uint(x);
+    const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    const unsigned c = __float_as_uint(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+    const auto t = __builtin_amdgcn_permlane32_swap(c, c, false, false);
+    return fmaxf(__uint_as_float(t[0]), __uint_as_float(t[1]));
 }
 
 // a lane's eight scores (keys first .. first + 7) of the query at qpos: scaled, less the distance bias, in the exponent's
@@ -88,13 +98,24 @@ __device__ __forceinline__ void ag_store4(bf16* op, const bf16* gp, float x0, fl
     *reinterpret_cast<uint2*>(op) = w;
 }
 
-template <int DC, int DT>     // hs = 32 DC, vd = 16 DT
-__global__ __launch_bounds__(AG_WAVES * BN_WAVE) void attn_general_prompt_kernel(GenArgs a) {
-    constexpr int HS = 32 * DC, VD = 16 * DT;
+// A workgroup is 4, 2 or 1 heads of one kv head (a wave each); they stage a block of keys and values through shared memory, the
+// loads of a block under way while the one before is worked on.  What bounds it: first the address unit of the loads (an operand
+// straight from the pages is sixteen rows in each sixteen lanes, 64 cycles an instruction instead of 16: a block took 4 x 16 x 64
+// cycles a workgroup, whatever ran beside it), now the instructions of a wave's softmax, so a block that is seen whole is not masked,
+// sums are rescaled only when a maximum has moved, and two waves a SIMD are asked for where the registers reach, which keeps the sums
+// out of the accumulation registers (the vector unit has to copy them).  2,048 tokens, 16 heads 128 wide: with 4 kv heads 228 -> 74 us,
+// with 16 of them 229 -> 115; 64 wide, 32 heads on 8: 227 -> 72; 256 wide: 397 -> 189; 128 tokens behind 2,000: 118 -> 62.
+template <int DC, int DT, int WAVES>     // hs = 32 DC, vd = 16 DT, heads of a workgroup
+__global__ __launch_bounds__(WAVES * BN_WAVE, DC + DT <= (WAVES > 1 ? 16 : 14) ? 2 : 1) void attn_general_prompt_kernel(GenArgs a) {
+    constexpr int HS = 32 * DC, VD = 16 * DT, THREADS = WAVES * BN_WAVE;
+    constexpr int KEYS = 128 * DC, VALUES = 64 * DT;                     // 16-byte pieces of a block of 32 keys, and of its values
+    constexpr int KN = (KEYS + THREADS - 1) / THREADS, VN = (VALUES + THREADS - 1) / THREADS;       // a thread's share of them
+    constexpr int BUFFERS = WAVES > 1 ? 2 : 1;
+    __shared__ __align__(16) u32x4 staged[BUFFERS][KEYS + VALUES];
     const int* tl = a.tiles + 4 * blockIdx.x;
     const int seq = tl[0], row0 = tl[1], n = min(tl[2], 16), pos0 = tl[3];
-    const int head = blockIdx.y * AG_WAVES + (threadIdx.x >> 6);
-    if (n <= 0 || pos0 < 0 || head >= a.H) return;
+    const int head = blockIdx.y * WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (n <= 0 || pos0 < 0) return;                      // the whole workgroup
     const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
     const int kvh = head / (a.H / a.Hkv);
     const bool col_ok = i < n;                           // this lane's query column exists
@@ -116,56 +137,88 @@ __global__ __launch_bounds__(AG_WAVES * BN_WAVE) void attn_general_prompt_kernel
     for (int t = 0; t < DT; ++t) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;
     const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
-    const int krow = 8 * (i >> 2) + (i & 3);             // this lane's key row of tile 0 inside a block; tile 1: 4 further
 
-    // The keys of a block are asked for one block ahead (the last block asks for itself once more: a load without a
-    // branch around it), so that the first product finds its operand there; the values are asked for when the block
-    // begins and are used behind the weights.
-    bf16x8 kn0[DC], kn1[DC];
-    auto ask_keys = [&](int kb) {
-        const int page = a.block_table[(size_t)seq * a.bt_stride + kb / BN_PAGE];
-        const bf16* kbase = a.k_pages + (((size_t)page * a.Hkv + kvh) * BN_PAGE + kb % BN_PAGE + krow) * HS + 8 * g;
+    // A block's pieces as they lie in the pages (the keys one run, of the values 64 bytes a dimension), and where a piece goes:
+    // piece 64 (2 c + tile) + 16 g + (i ^ (4 g + c % 4)) is dimensions 32 c + 8 g .. + 7 of row i of key tile `tile`, piece
+    // KEYS + 64 t + 16 g + (i ^ 4 g) keys 8 g .. 8 g + 7 of value column 16 t + i.  A wave then reads an operand as 1 KB in a row, and
+    // the exclusive or keeps the pieces that a row's threads write in different banks.
+    const int* pages = a.block_table + (size_t)seq * a.bt_stride;
+    u32x4 kr[KN], vr[VN];
+    auto ask = [&](int kb, int page) {
+        const size_t at = (size_t)page * a.Hkv + kvh;
+        const u32x4* kp = reinterpret_cast<const u32x4*>(a.k_pages + (at * BN_PAGE + kb % BN_PAGE) * HS);
+        const bf16* vp = a.v_pages + at * VD * BN_PAGE + kb % BN_PAGE;
 #pragma unroll
-        for (int c = 0; c < DC; ++c) { kn0[c] = ag_ld16(kbase + 32 * c); kn1[c] = ag_ld16(kbase + 4 * HS + 32 * c); }
+        for (int u = 0; u < KN; ++u) {
+            const int piece = u * THREADS + threadIdx.x;
+            if (KEYS % THREADS == 0 || piece < KEYS) kr[u] = kp[piece];
+        }
+#pragma unroll
+        for (int u = 0; u < VN; ++u) {
+            const int piece = u * THREADS + threadIdx.x;
+            if (VALUES % THREADS == 0 || piece < VALUES) vr[u] = *reinterpret_cast<const u32x4*>(vp + (piece >> 2) * BN_PAGE + 8 * (piece & 3));
+        }
+    };
+    auto put = [&](u32x4* to) {
+#pragma unroll
+        for (int u = 0; u < KN; ++u) {
+            const int piece = u * THREADS + threadIdx.x, r = piece / (4 * DC), q = piece % (4 * DC);
+            const int pi = (r >> 3) << 2 | (r & 3), pg = q & 3, pc = q >> 2;
+            if (KEYS % THREADS == 0 || piece < KEYS) to[64 * (2 * pc + (r >> 2 & 1)) + 16 * pg + (pi ^ (4 * pg + (pc & 3)))] = kr[u];
+        }
+#pragma unroll
+        for (int u = 0; u < VN; ++u) {
+            const int piece = u * THREADS + threadIdx.x, pi = piece >> 2 & 15, pg = piece & 3;
+            if (VALUES % THREADS == 0 || piece < VALUES) to[KEYS + 64 * (piece >> 6) + 16 * pg + (pi ^ (4 * pg))] = vr[u];
+        }
     };
     const int k_lo = a.window > 0 ? max(0, pos0 - a.window + 1) & ~31 : 0;      // the block of the first key any row sees
     const int q_lo = a.window > 0 ? qpos - a.window : -1;                        // keys at or below this are out of sight
+    const int width = a.window > 0 ? a.window : pos0 + 32;                       // (no window: every block is above its edge)
     const int keep = a.window > 0 ? min(a.keep_first, k_hi) : 0;                 // keys below this stay in sight
     auto leap = [&](int kb) { return kb >= keep && kb < k_lo ? k_lo : kb; };     // past what no row of the tile sees
-    const int last_block = ((k_hi - 1) / 32) * 32;
-    ask_keys(leap(0));
-    for (int kb = leap(0); kb < k_hi; kb = leap(kb + 32)) {
-        const int page = a.block_table[(size_t)seq * a.bt_stride + kb / BN_PAGE];
-        const int off = kb % BN_PAGE;
-        const bf16* vbase = a.v_pages + (((size_t)page * a.Hkv + kvh) * VD + i) * BN_PAGE + off + 8 * g;
-        bf16x8 k0[DC], k1[DC];
-#pragma unroll
-        for (int c = 0; c < DC; ++c) { k0[c] = kn0[c]; k1[c] = kn1[c]; }
-        ask_keys(min(leap(kb + 32), last_block));
+    const int last_block = ((k_hi - 1) / 32) * 32;       // asked for again behind the end: a load without a branch around it
+    int kb = leap(0), next = leap(kb + 32), buffer = 0;
+    int page = pages[min(next, last_block) / BN_PAGE];   // the page of the block that is asked for next: itself asked for a block before
+    ask(kb, pages[kb / BN_PAGE]);
+    put(staged[0]);
+    ask(min(next, last_block), page);
+    page = pages[min(leap(next + 32), last_block) / BN_PAGE];
+    __syncthreads();
+    for (; kb < k_hi; kb = next, next = leap(next + 32)) {
+        const u32x4* block = staged[buffer];
+        if (BUFFERS == 2) {                              // the other buffer was read before the barrier behind the last block
+            buffer ^= 1;
+            put(staged[buffer]);
+            ask(min(leap(next + 32), last_block), page);
+            page = pages[min(leap(leap(next + 32) + 32), last_block) / BN_PAGE];
+        }
         f32x4 st0 = (f32x4){0.f, 0.f, 0.f, 0.f}, st1 = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
-            st0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0[c], qf[c], st0, 0, 0, 0);
-            st1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1[c], qf[c], st1, 0, 0, 0);
+            const u32x4* kt = block + 128 * c + 16 * g + (i ^ (4 * g + (c & 3)));
+            st0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kt[0]), qf[c], st0, 0, 0, 0);
+            st1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kt[64]), qf[c], st1, 0, 0, 0);
         }
-        // the values' tiles are asked for now and used behind the weights
-        bf16x8 va[DT];
-#pragma unroll
-        for (int t = 0; t < DT; ++t) va[t] = ag_ld16(vbase + (size_t)t * 16 * BN_PAGE);
         // this lane's eight scores: keys kb + 8 g + e, e = 4 h + r
         float s[8];
         ag_scores(s, st0, st1, scale2, bias, ba, bb, qpos, kb + 8 * g);
+        // a block that every row sees whole is not masked (a column without a query is never stored)
         float mx = -INFINITY;
+        if (kb + 31 <= pos0 && (kb + 31 < keep || kb > pos0 + n - 1 - width)) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int key = kb + 8 * g + e;
-            float v = s[e];
-            if (!col_ok || key > qpos || key >= k_hi || (key <= q_lo && key >= keep)) v = -INFINITY;
-            s[e] = v;
-            mx = fmaxf(mx, v);
+            for (int e = 0; e < 8; ++e) mx = fmaxf(mx, s[e]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int key = kb + 8 * g + e;
+                float v = s[e];
+                if (!col_ok || key > qpos || key >= k_hi || (key <= q_lo && key >= keep)) v = -INFINITY;
+                s[e] = v;
+                mx = fmaxf(mx, v);
+            }
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, BN_WAVE));     // the four lane groups of a column
-        mx = fmaxf(mx, __shfl_xor(mx, 32, BN_WAVE));
+        mx = ag_max_over_groups(mx);
         const float m_new = fmaxf(m, mx);
         float alpha = 1.f;
         if (m_new == -INFINITY) {
@@ -176,11 +229,15 @@ __global__ __launch_bounds__(AG_WAVES * BN_WAVE) void attn_general_prompt_kernel
             for (int e = 0; e < 8; ++e) s[e] = __builtin_amdgcn_exp2f(s[e] - m_new);
             alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
         }
+        const bool rescale = __any(alpha != 1.f);        // a factor of 1 for every column changes nothing
         m = m_new;
         const f32x8 pv = {s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7]};
         const bf16x8 pb = __builtin_convertvector(pv, bf16x8);
         const f32x4 lsum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
         l = fmaf(l, alpha, lsum[0]);
+        bf16x8 va[DT];
+#pragma unroll
+        for (int t = 0; t < DT; ++t) va[t] = __builtin_bit_cast(bf16x8, block[KEYS + 64 * t + 16 * g + (i ^ (4 * g))]);
         // keys past the tile's last position may hold anything in V^T (0 * NaN is NaN): cleared
         if (kb + 32 > k_hi) {
 #pragma unroll
@@ -198,10 +255,20 @@ __global__ __launch_bounds__(AG_WAVES * BN_WAVE) void attn_general_prompt_kernel
                 va[t] = __builtin_bit_cast(bf16x8, w);
             }
         }
+        if (rescale) {
+#pragma unroll
+            for (int t = 0; t < DT; ++t) acc[t] *= alpha;
+        }
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
-            acc[t] *= alpha;
             acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[t], pb, acc[t], 0, 0, 0);
+        }
+        __syncthreads();
+        if (BUFFERS == 1) {
+            put(staged[0]);
+            ask(min(leap(next + 32), last_block), page);
+            page = pages[min(leap(leap(next + 32) + 32), last_block) / BN_PAGE];
+            __syncthreads();
         }
     }
     // the sink: a term 2^(sv - m') with no value, m' = max(m, sv)
@@ -441,9 +508,19 @@ extern "C" int bn_attn_general_supports(int hs, int vd) {
     return ag_size(hs) && ag_size(vd) ? 1 : 0;
 }
 
+// Heads of a workgroup: as many as share a kv head, up to four, since they share the staged block: 2,048 tokens, 16 heads on 4 take
+// 74 us with four, 83 with two, 109 with one.
+static int ag_waves(int group) { return group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1; }
+
 template <int DC>
-static int ag_launch_dt(const GenArgs& a, int vd, dim3 grid, hipStream_t s) {
-#define AG_CASE(DT) hipLaunchKernelGGL((attn_general_prompt_kernel<DC, DT>), grid, dim3(AG_WAVES * BN_WAVE), 0, s, a); return bn_launch_status()
+static int ag_launch_dt(const GenArgs& a, int vd, int n_tiles, hipStream_t s) {
+    const int waves = ag_waves(a.H / a.Hkv);
+    const dim3 grid(n_tiles, a.H / waves), block(waves * BN_WAVE);
+#define AG_CASE(DT)                                                                                   \
+    if (waves == 4) hipLaunchKernelGGL((attn_general_prompt_kernel<DC, DT, 4>), grid, block, 0, s, a);       \
+    else if (waves == 2) hipLaunchKernelGGL((attn_general_prompt_kernel<DC, DT, 2>), grid, block, 0, s, a);  \
+    else hipLaunchKernelGGL((attn_general_prompt_kernel<DC, DT, 1>), grid, block, 0, s, a);                  \
+    return bn_launch_status()
     switch (vd / 16) {
         case 2: AG_CASE(2);
         case 4: AG_CASE(4);
@@ -472,15 +549,14 @@ extern "C" int bn_attn_general_prompt(const void* q, int q_stride, void* out, in
     a.block_table = block_table; a.tiles = tiles; a.dist_a = dist_a; a.dist_b = dist_b;
     a.q_stride = q_stride; a.out_stride = out_stride; a.bt_stride = bt_stride; a.H = H; a.Hkv = Hkv;
     a.scale = scale; a.sink = sink ? 1 : 0; a.sink_values = sink ? sink_values : nullptr; a.window = window;
-    const dim3 grid(n_tiles, (H + AG_WAVES - 1) / AG_WAVES);
     switch (hs / 32) {
-        case 1: return ag_launch_dt<1>(a, vd, grid, s);
-        case 2: return ag_launch_dt<2>(a, vd, grid, s);
-        case 3: return ag_launch_dt<3>(a, vd, grid, s);
-        case 4: return ag_launch_dt<4>(a, vd, grid, s);
-        case 5: return ag_launch_dt<5>(a, vd, grid, s);
-        case 6: return ag_launch_dt<6>(a, vd, grid, s);
-        case 8: return ag_launch_dt<8>(a, vd, grid, s);
+        case 1: return ag_launch_dt<1>(a, vd, n_tiles, s);
+        case 2: return ag_launch_dt<2>(a, vd, n_tiles, s);
+        case 3: return ag_launch_dt<3>(a, vd, n_tiles, s);
+        case 4: return ag_launch_dt<4>(a, vd, n_tiles, s);
+        case 5: return ag_launch_dt<5>(a, vd, n_tiles, s);
+        case 6: return ag_launch_dt<6>(a, vd, n_tiles, s);
+        case 8: return ag_launch_dt<8>(a, vd, n_tiles, s);
     }
     return BN_ERR_ARG;
 }
