@@ -11,20 +11,20 @@
 //
 // One order of summation, whoever computes a row: a page of 64 keys is summed by itself from nothing (its maximum, its
 // exponentials' sum, its values' sum); the pages of a run of 256 positions are folded in order from nothing; the runs are
-// folded in order.  The prompt form walks a row's pages and folds as it goes; the decode form gives every page of a run a
-// wave and every run a workgroup, and a small kernel folds the runs: the same bits (float32 logits do not depend on how a
-// sequence was cut into steps).
+// folded in order.  The prompt form walks a row's pages and folds as it goes; the decode form gives every page (or, for so many rows
+// that the pages' sums would not have the room, every run) a workgroup, and a small kernel folds them: the same bits (float32
+// logits do not depend on how a sequence was cut into steps).
 //
 // The prompt form is bound by the instruction (a page is 8,192 cycles of a SIMD for a wave of 16 rows x 128): a workgroup of 4
 // waves shares the staged page, two workgroups a CU stage and multiply in turn.  Eight prompts of 64 to 1,024 tokens, 16
-// heads of 128 over 4: 0.31 ms a layer (2.70 in attn_rows.hip).  The decode form is bound by latency: one page a wave, all its
-// 64 KB asked for at once; the same eight sequences 20 us and 4 for the fold (243), one sequence of 200 keys 18 (58).
+// heads of 128 over 4: 0.31 ms a layer (2.70 in attn_rows.hip).
 #include "common.h"
 #include <math.h>
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define AF_RUN_PAGES 4
+#define AF_PARTS_BYTES (64ll << 20)
 
 struct AfArgs {
     const float* q;           // [n_tokens, q_stride], head h at h * hs (already rotated)
@@ -34,12 +34,16 @@ struct AfArgs {
     const int* block_table;   // [n_seqs, bt_stride]
     const int* seq_lens;      // decode form: keys in the cache, the new one included
     const int* tiles;         // prompt form: [n, 4] = sequence, first token row, tokens, position of the first
-    float* part_o;            // [n_tokens * H, n_runs, hs] (n_runs > 1)
-    float* part_ml;           // [n_tokens * H, n_runs, 2]
+    float* part_o;            // [n_tokens * H, n_parts, hs] (n_parts > 1)
+    float* part_ml;           // [n_tokens * H, n_parts, 2]
     int q_stride, out_stride, bt_stride, H, Hkv;
     int GT;                   // heads of a kv group handled together (a power of two <= 16)
-    int n_runs;               // runs that the block table can hold
+    int n_parts, part_pages;  // decode form: parts that the block table can hold, and a part's pages (1 or AF_RUN_PAGES)
     float scale;
+    const float* inv_freq;    // decode form: not null: q and the new key are rotated here, angle position * inv_freq[i], pairs (i, i + hs / 2)
+    int write;                // decode form: the new key and value (behind q in its row) are stored at position seq_lens - 1
+    float* k_new;             // k_pages and v_pages, to write
+    float* v_new;
 };
 
 // The fold of (m, l, o) into (M, L, O), its operations written out (no contraction left to the compiler): the same parts give
@@ -213,131 +217,237 @@ __global__ __launch_bounds__(256, 2) void attn_f32_prompt_kernel(AfArgs a) {
             for (int j = 0; j < 4; ++j) o[16 * S::VW * h + S::VW * (4 * g + j) + i] = __fmul_rn(tot.o[h][i][j], inv);
 }
 
-template <int HS>
-__global__ __launch_bounds__(256, 1) void attn_f32_decode_kernel(AfArgs a) {
-    using S = AfShape<HS>;
-    __shared__ float so[AF_RUN_PAGES][16][HS + 1];
-    __shared__ float sm[AF_RUN_PAGES][16], sl[AF_RUN_PAGES][16];
+// PAGES pages are a workgroup of 4 waves each: wave t of a page multiplies the keys 16 t .. 16 t + 15 with the queries, then, with the
+// page's scores exchanged through shared memory, the weights with a quarter of the value's dimensions.  Everything is asked for at
+// once, keys as they lie (their operand comes through shared memory: sixteen rows in sixteen lanes of a load would cost four times the
+// cycles).  inv_freq: the query and the new key arrive unrotated; write: the workgroup that holds the new position stores the new key
+// and value into the pages, and reads them from the token's row itself.  The order of every sum is the prompt form's (af_page).
+// What bounds it is how fast a CU can draw its keys and values (some 25 bytes a nanosecond): one sequence of 200 keys, 16 heads
+// of 128 over 4, 8.9 us and 4.1 for the fold, rotation and store inside; with a workgroup a run of four pages 18.6 in all, with a wave a
+// page of such a run 18.2 and 5.3 for the rotation in front.  Eight sequences of 64 to 1,024 keys: 11.7 and 4.1 (20 + 4 + 4.5 before).
+template <int HS, int PAGES>
+__global__ __launch_bounds__(256 * PAGES) void attn_f32_decode_kernel(AfArgs a) {
+    constexpr int NB = HS / 16, STRIDE = HS + 4, HALF = HS / 2;
+    constexpr int VW = HS >= 64 ? HS / 64 : 1;    // tiles of the second product a wave: value dimensions 16 VW part + VW row + tile
+    constexpr int PARTS = HS / (16 * VW);         // waves of a page that have any
+    extern __shared__ __align__(16) float af_smem[];
+    float* ks = af_smem;                          // [4 PAGES][16][STRIDE] every wave's keys; later [PAGES][16][HS + 1], the pages' sums
+    float* so = af_smem;
+    float* sx = ks + 4 * PAGES * 16 * STRIDE;     // [PAGES][4][64][4] every page's scores, as the lanes hold them
+    float* qs = sx + PAGES * 4 * 64 * 4;          // [16][STRIDE]     the queries
+    float* kn = qs + 16 * STRIDE;                 // [HS]             the new key
+    float* sm = kn + HS;                          // [PAGES][16] each
+    float* sl = sm + PAGES * 16;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), pg = wave >> 2, t = wave & 3;
     const int GT = a.GT, G = a.H / a.Hkv;
     const int head_tiles = (G + GT - 1) / GT;
     const int kvh = blockIdx.y / head_tiles, ht = blockIdx.y - kvh * head_tiles;
     const int tok = blockIdx.x, len = a.seq_lens[tok];
     const int rows = min(GT, G - ht * GT);
-    const bool live = r < rows;
-    const float* qp = a.q + (size_t)tok * a.q_stride + (size_t)(kvh * G + ht * GT + (live ? r : 0)) * HS + 4 * g;
-    f32x4 q[S::NB];
-#pragma unroll
-    for (int b = 0; b < S::NB; ++b)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) q[b][e] = live ? qp[16 * b + e] : 0.f;
-    for (int run = blockIdx.z; run < a.n_runs && (run == 0 || run * AF_RUN_PAGES * BN_PAGE < len); run += gridDim.z) {
-        const int j0 = (run * AF_RUN_PAGES + wave) * BN_PAGE;
-        AfSums<HS> p;
-        p.m = -INFINITY; p.l = 0.f;
-        if (j0 < len) {
-            const int page = a.block_table[(size_t)tok * a.bt_stride + j0 / BN_PAGE];
-            const float* kg = a.k_pages + ((size_t)page * a.Hkv + kvh) * BN_PAGE * HS;
-            const float* vg = a.v_pages + ((size_t)page * a.Hkv + kvh) * BN_PAGE * HS;
-            const int last = min(len - 1 - j0, BN_PAGE - 1);
-            f32x4 kf[4][S::NB];
-            float vf[4][4][S::NH][S::VW];
-            if (last == BN_PAGE - 1) {            // a whole page: straight-line loads
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int b = 0; b < S::NB; ++b) kf[t][b] = *reinterpret_cast<const f32x4*>(kg + (16 * t + r) * HS + 16 * b + 4 * g);
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-#pragma unroll
-                        for (int h = 0; h < S::NH; ++h) af_values<S::VW>(vg + (16 * t + 4 * g + e) * HS + 16 * S::VW * h + S::VW * r, vf[t][e][h]);
-            } else {                              // rows behind the last key count as zeros
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int b = 0; b < S::NB; ++b) kf[t][b] = *reinterpret_cast<const f32x4*>(kg + min(16 * t + r, last) * HS + 16 * b + 4 * g);
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-#pragma unroll
-                        for (int h = 0; h < S::NH; ++h) {
-                            const int row = 16 * t + 4 * g + e;
-                            af_values<S::VW>(vg + min(row, last) * HS + 16 * S::VW * h + S::VW * r, vf[t][e][h]);
-#pragma unroll
-                            for (int i = 0; i < S::VW; ++i) vf[t][e][h][i] = row <= last ? vf[t][e][h][i] : 0.f;
-                        }
-            }
-            af_page<HS>(q, a.scale, last, last < BN_PAGE - 1, [&](int t, int b) { return kf[t][b]; },
-                        [&](int t, int e, int h, float (&v)[S::VW]) {
-#pragma unroll
-                            for (int i = 0; i < S::VW; ++i) v[i] = vf[t][e][h][i];
-                        },
-                        p);
-#pragma unroll
-            for (int h = 0; h < S::NH; ++h)
-#pragma unroll
-                for (int i = 0; i < S::VW; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) so[wave][r][16 * S::VW * h + S::VW * (4 * g + j) + i] = p.o[h][i][j];
+    const float* row = a.q + (size_t)tok * a.q_stride;
+    const float* new_v = row + (size_t)(a.H + a.Hkv + kvh) * HS;
+    // the queries (rows without a head as zeros) and the new key, a pair of dimensions a thread
+    for (int idx = tid; idx < 17 * HALF; idx += 256 * PAGES) {
+        const int h = idx / HALF, i = idx - h * HALF;
+        const bool is_key = h == 16;
+        if (is_key && !a.write) break;
+        const float* src = row + (size_t)(is_key ? a.H + kvh : kvh * G + ht * GT + min(h, rows - 1)) * HS + i;
+        float x0 = src[0], x1 = src[HALF];
+        if (a.inv_freq) {
+            float sn, c;
+            sincosf((float)(len - 1) * a.inv_freq[i], &sn, &c);
+            bn_rotate_pair(x0, x1, c, sn);
         }
-        if (g == 0) { sm[wave][r] = p.m; sl[wave][r] = p.l; }
+        if (!is_key && h >= rows) x0 = x1 = 0.f;
+        float* dst = is_key ? kn + i : qs + h * STRIDE + i;
+        dst[0] = x0;
+        dst[HALF] = x1;
+    }
+    for (int part = blockIdx.z; part < a.n_parts && (part == 0 || part * PAGES * BN_PAGE < len); part += gridDim.z) {
+        const int j0 = (part * PAGES + pg) * BN_PAGE;
+        const bool live = j0 < len;               // this wave's page holds keys
+        const int last = min(len - 1 - j0, BN_PAGE - 1);
+        const bool newest = a.write && live && len - 1 - j0 < BN_PAGE;       // the page holds the new position: its row `last`
+        f32x4 kr[NB];
+        float vf[4][4][VW], nv[VW];
+        size_t at = 0;
+        if (live) {
+            at = ((size_t)a.block_table[(size_t)tok * a.bt_stride + j0 / BN_PAGE] * a.Hkv + kvh) * BN_PAGE * HS;
+            const f32x4* kg = reinterpret_cast<const f32x4*>(a.k_pages + at + (size_t)16 * t * HS);
+#pragma unroll
+            for (int i = 0; i < NB; ++i) kr[i] = kg[lane + 64 * i];
+            const float* vbase = a.v_pages + at + (4 * g * HS + 16 * VW * t + VW * r);
+            if (t < PARTS) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) af_values<VW>(vbase + (16 * u + e) * HS, vf[u][e]);
+                if (newest) af_values<VW>(new_v + 16 * VW * t + VW * r, nv);
+            }
+        }
+        __syncthreads();                          // the queries and the new key are there; the sums of the part before have been read
+        float* mine = ks + wave * 16 * STRIDE;
+        if (live) {
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const int piece = lane + 64 * i, key = piece / (HS / 4), d = 4 * (piece % (HS / 4));
+                if (newest && 16 * t + key == last) kr[i] = *reinterpret_cast<const f32x4*>(kn + d);
+                *reinterpret_cast<f32x4*>(mine + key * STRIDE + d) = kr[i];
+            }
+        }
+        if (newest && ht == 0 && t == 0) {        // the new position's rows of the pages, by a wave
+            float* kd = a.k_new + at + (size_t)last * HS;
+            float* vd = a.v_new + at + (size_t)last * HS;
+            for (int d = lane; d < HS; d += 64) { kd[d] = kn[d]; vd[d] = new_v[d]; }
+        }
+        __builtin_amdgcn_wave_barrier();          // a wave's own keys: its shared-memory operations run in order
+        if (live) {
+            f32x4 s = 0.f;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const f32x4 kf = *reinterpret_cast<const f32x4*>(mine + r * STRIDE + 16 * b + 4 * g);
+                const f32x4 qf = *reinterpret_cast<const f32x4*>(qs + r * STRIDE + 16 * b + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[e], s, 0, 0, 0);
+            }
+            *reinterpret_cast<f32x4*>(sx + ((pg * 4 + t) * 64 + lane) * 4) = s;
+        }
         __syncthreads();
-        for (int idx = tid; idx < rows * HS; idx += 256) {
-            const int row = idx / HS, d = idx - row * HS;
+        if (live && t < PARTS) {
+            f32x4 s[4];
+            float m = -INFINITY, l = 0.f;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                s[u] = *reinterpret_cast<const f32x4*>(sx + ((pg * 4 + u) * 64 + lane) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    s[u][e] = 16 * u + 4 * g + e > last ? -INFINITY : __fmul_rn(s[u][e], a.scale);
+                    m = fmaxf(m, s[u][e]);
+                }
+            }
+            m = fmaxf(m, __shfl_xor(m, 16, BN_WAVE));
+            m = fmaxf(m, __shfl_xor(m, 32, BN_WAVE));
+            const float base = m == -INFINITY ? 0.f : m;
+            f32x4 o[VW];
+#pragma unroll
+            for (int i = 0; i < VW; ++i) o[i] = 0.f;
+            if (last < BN_PAGE - 1 || newest) {   // the new value comes from the token's row; rows behind the last key count as zeros
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int key = 16 * u + 4 * g + e;
+#pragma unroll
+                        for (int i = 0; i < VW; ++i) vf[u][e][i] = key > last ? 0.f : key == last && newest ? nv[i] : vf[u][e][i];
+                    }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { s[u][e] = expf(__fsub_rn(s[u][e], base)); l = __fadd_rn(l, s[u][e]); }
+            l = __fadd_rn(l, __shfl_xor(l, 16, BN_WAVE));
+            l = __fadd_rn(l, __shfl_xor(l, 32, BN_WAVE));
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int i = 0; i < VW; ++i) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][e][i], s[u][e], o[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < VW; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) so[(pg * 16 + r) * (HS + 1) + 16 * VW * t + VW * (4 * g + j) + i] = o[i][j];
+            if (t == 0 && g == 0) { sm[pg * 16 + r] = m; sl[pg * 16 + r] = l; }
+        } else if (!live && t == 0 && g == 0) {
+            sm[pg * 16 + r] = -INFINITY;
+            sl[pg * 16 + r] = 0.f;
+        }
+        __syncthreads();
+        for (int idx = tid; idx < rows * HS; idx += 256 * PAGES) {
+            const int h = idx / HS, d = idx - h * HS;
             float M = -INFINITY, L = 0.f, O = 0.f;
 #pragma unroll
-            for (int w = 0; w < AF_RUN_PAGES; ++w) {
-                const float m = sm[w][row];
+            for (int w = 0; w < PAGES; ++w) {
+                const float m = sm[w * 16 + h];
                 if (m == -INFINITY) continue;
                 float m2, fa, fb;
                 af_factors(M, m, m2, fa, fb);
-                L = af_fold(L, fa, sl[w][row], fb);
-                O = af_fold(O, fa, so[w][row][d], fb);
+                L = af_fold(L, fa, sl[w * 16 + h], fb);
+                O = af_fold(O, fa, so[(w * 16 + h) * (HS + 1) + d], fb);
                 M = m2;
             }
-            const int head = kvh * G + ht * GT + row;
-            if (a.n_runs == 1) {
+            const int head = kvh * G + ht * GT + h;
+            if (a.n_parts == 1) {
                 a.out[(size_t)tok * a.out_stride + (size_t)head * HS + d] = __fmul_rn(O, L > 0.f ? 1.0f / L : 0.f);
             } else {
-                const size_t at = ((size_t)tok * a.H + head) * a.n_runs + run;
+                const size_t at = ((size_t)tok * a.H + head) * a.n_parts + part;
                 a.part_o[at * HS + d] = O;
                 if (d == 0) { a.part_ml[2 * at] = M; a.part_ml[2 * at + 1] = L; }
             }
         }
-        __syncthreads();
+        // (the barrier behind the next part's loads stands before its keys are stored over the sums)
     }
 }
 
-// the runs of a row in order
-__global__ __launch_bounds__(128) void attn_f32_fold_kernel(AfArgs a, int hs) {
-    const int row = blockIdx.x, tok = row / a.H, head = row - tok * a.H, d = threadIdx.x;
-    if (d >= hs) return;
+// The parts of a row in order: the per_run parts of a run from nothing (a group of 128 threads a run), then the runs.
+__global__ __launch_bounds__(1024) void attn_f32_fold_kernel(AfArgs a, int hs, int per_run) {
+    __shared__ float ro[8][128], rm[8], rl[8];
+    const int row = blockIdx.x, tok = row / a.H, head = row - tok * a.H, d = threadIdx.x & 127;
+    const int group = threadIdx.x >> 7, groups = blockDim.x >> 7;
     const int len = a.seq_lens[tok], runs = (len + AF_RUN_PAGES * BN_PAGE - 1) / (AF_RUN_PAGES * BN_PAGE);
-    const float* ml = a.part_ml + (size_t)row * a.n_runs * 2;
-    const float* po = a.part_o + (size_t)row * a.n_runs * hs + d;
+    const int part_keys = AF_RUN_PAGES / per_run * BN_PAGE, parts = (len + part_keys - 1) / part_keys;
+    const float* ml = a.part_ml + (size_t)row * a.n_parts * 2;
+    const float* po = a.part_o + (size_t)row * a.n_parts * hs + min(d, hs - 1);
     float M = -INFINITY, L = 0.f, O = 0.f;
-    for (int s0 = 0; s0 < runs; s0 += 8) {        // eight runs' sums are asked for at once
-        float m[8], l[8], o[8];
+    for (int r0 = 0; r0 < runs; r0 += groups) {
+        if (r0 + group < runs) {
+            const int first = (r0 + group) * per_run;
+            float m[AF_RUN_PAGES], l[AF_RUN_PAGES], o[AF_RUN_PAGES], RM = -INFINITY, RL = 0.f, RO = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int s = min(s0 + i, runs - 1);
-            m[i] = ml[2 * s]; l[i] = ml[2 * s + 1]; o[i] = po[(size_t)s * hs];
+            for (int i = 0; i < AF_RUN_PAGES; ++i) {
+                const int at = min(first + i, parts - 1);
+                m[i] = ml[2 * at]; l[i] = ml[2 * at + 1]; o[i] = po[(size_t)at * hs];
+            }
+#pragma unroll
+            for (int i = 0; i < AF_RUN_PAGES; ++i) {
+                if (i >= per_run || first + i >= parts || m[i] == -INFINITY) continue;
+                float m2, fa, fb;
+                af_factors(RM, m[i], m2, fa, fb);
+                RL = af_fold(RL, fa, l[i], fb);
+                RO = af_fold(RO, fa, o[i], fb);
+                RM = m2;
+            }
+            ro[group][d] = RO;
+            if (d == 0) { rm[group] = RM; rl[group] = RL; }
         }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            if (s0 + i >= runs || m[i] == -INFINITY) continue;
+        __syncthreads();
+        for (int i = 0; i < min(groups, runs - r0); ++i) {
+            if (rm[i] == -INFINITY) continue;
             float m2, fa, fb;
-            af_factors(M, m[i], m2, fa, fb);
-            L = af_fold(L, fa, l[i], fb);
-            O = af_fold(O, fa, o[i], fb);
+            af_factors(M, rm[i], m2, fa, fb);
+            L = af_fold(L, fa, rl[i], fb);
+            O = af_fold(O, fa, ro[i][d], fb);
             M = m2;
         }
+        __syncthreads();
     }
-    a.out[(size_t)tok * a.out_stride + (size_t)head * hs + d] = __fmul_rn(O, L > 0.f ? 1.0f / L : 0.f);
+    if (group == 0 && d < hs) a.out[(size_t)tok * a.out_stride + (size_t)head * hs + d] = __fmul_rn(O, L > 0.f ? 1.0f / L : 0.f);
+}
+
+template <int HS, int PAGES>
+static int af_launch_decode(const AfArgs& a, int n_seqs, int heads, hipStream_t s) {
+    // a workgroup a part up to some 8,192 workgroups; a longer table's parts are taken in turn
+    int z = 8192 / (n_seqs * heads);
+    z = z < 1 ? 1 : z > a.n_parts ? a.n_parts : z;
+    const size_t smem = sizeof(float) * (4 * PAGES * 16 * (HS + 4) + PAGES * 4 * 64 * 4 + 16 * (HS + 4) + HS + 2 * PAGES * 16);
+    auto kernel = attn_f32_decode_kernel<HS, PAGES>;
+    if (smem > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return (int)e;
+    }
+    hipLaunchKernelGGL(kernel, dim3(n_seqs, heads, z), dim3(256 * PAGES), smem, s, a);
+    return bn_launch_status();
 }
 
 template <int HS>
@@ -347,28 +457,39 @@ static int af_launch(const AfArgs& a, int n_tiles, hipStream_t s) {
         hipLaunchKernelGGL(attn_f32_prompt_kernel<HS>, dim3(n_tiles, heads), dim3(256), 0, s, a);
         return bn_launch_status();
     }
-    // a workgroup a run up to some 2,048 workgroups; a longer table's runs are taken in turn
-    int z = 2048 / (n_tiles * heads);
-    z = z < 1 ? 1 : z > a.n_runs ? a.n_runs : z;
-    hipLaunchKernelGGL(attn_f32_decode_kernel<HS>, dim3(n_tiles, heads, z), dim3(256), 0, s, a);
-    if (int rc = bn_launch_status()) return rc;
-    if (a.n_runs > 1) hipLaunchKernelGGL(attn_f32_fold_kernel, dim3(n_tiles * a.H), dim3(128), 0, s, a, HS);
+    const int pages = a.part_pages;
+    const int rc = pages == 1 ? af_launch_decode<HS, 1>(a, n_tiles, heads, s) : af_launch_decode<HS, AF_RUN_PAGES>(a, n_tiles, heads, s);
+    if (rc || a.n_parts == 1) return rc;
+    const int per_run = AF_RUN_PAGES / pages, runs = (a.n_parts + per_run - 1) / per_run;
+    hipLaunchKernelGGL(attn_f32_fold_kernel, dim3(n_tiles * a.H), dim3(128 * (runs < 8 ? runs : 8)), 0, s, a, HS, per_run);
     return bn_launch_status();
 }
 
 extern "C" int bn_attn_f32_supports(int hs) { return hs == 16 || hs == 32 || hs == 64 || hs == 128; }
-extern "C" int bn_attn_f32_run_keys(void) { return AF_RUN_PAGES * BN_PAGE; }
+// Pages of a part of the decode form for a step of this many rows (n_seqs x heads) over tables of bt_stride pages: one, which spreads
+// a sequence's keys over the most CUs (one sequence of 200 keys 8.9 us and the fold, a run a workgroup 18.6), while the partial sums
+// stay under AF_PARTS_BYTES; then a run, whose sums take a quarter of the room.
+extern "C" int bn_attn_f32_part_pages(long long rows, int bt_stride, int hs) {
+    return rows * bt_stride * (hs + 2) * 4 <= AF_PARTS_BYTES ? 1 : AF_RUN_PAGES;
+}
 
-// tiles: the prompt form, tiles of up to 64 / GT tokens; null: the decode form, n_tiles sequences, with n_runs > 1 over
-// partial sums of n_runs runs a row (the runs that a block table of bt_stride pages can hold)
+// tiles: the prompt form, tiles of up to 64 / GT tokens; null: the decode form, n_tiles sequences in parts of
+// part_pages pages (1 or a run's), with partial sums of ceil(bt_stride / part_pages) parts a row if that is more than one.  Decode form only: inv_freq
+// [hs / 2], not null: q and the new key arrive unrotated; write: a row of q is [H + 2 Hkv heads], its new key and value are stored
+// into the pages at position seq_lens - 1 (a row of no keys stores nothing).
 extern "C" int bn_attn_f32(const void* q, int q_stride, void* out, int out_stride, const void* k_pages, const void* v_pages,
                            const int* block_table, int bt_stride, const int* seq_lens, const int* tiles, int n_tiles, int H, int Hkv,
-                           int hs, int GT, float scale, int n_runs, float* part_o, float* part_ml, hipStream_t s) {
+                           int hs, int GT, float scale, int part_pages, float* part_o, float* part_ml, const float* inv_freq, int write,
+                           hipStream_t s) {
     if (n_tiles <= 0 || n_tiles > 65535 * 128 || H <= 0 || Hkv <= 0 || H % Hkv || GT < 1 || GT > 16 || (GT & (GT - 1))) return BN_ERR_ARG;
-    if (Hkv * ((H / Hkv + GT - 1) / GT) > 65535 || bt_stride < 1 || n_runs < 1) return BN_ERR_ARG;
-    if (!tiles && (!seq_lens || (long long)n_runs * AF_RUN_PAGES < bt_stride || (n_runs > 1 && (!part_o || !part_ml)))) return BN_ERR_ARG;
+    if (Hkv * ((H / Hkv + GT - 1) / GT) > 65535 || bt_stride < 1) return BN_ERR_ARG;
+    if (tiles && (inv_freq || write)) return BN_ERR_ARG;
+    if (write && (q_stride < (H + 2 * Hkv) * hs || q_stride % 2 || ((uintptr_t)q & 7))) return BN_ERR_ARG;
+    if (!tiles && part_pages != 1 && part_pages != AF_RUN_PAGES) return BN_ERR_ARG;
+    const int n_parts = tiles ? 1 : (bt_stride + part_pages - 1) / part_pages;
+    if (!tiles && (!seq_lens || (n_parts > 1 && (!part_o || !part_ml)))) return BN_ERR_ARG;
     AfArgs a = {(const float*)q, (float*)out, (const float*)k_pages, (const float*)v_pages, block_table, seq_lens, tiles, part_o,
-                part_ml, q_stride, out_stride, bt_stride, H, Hkv, GT, n_runs, scale};
+                part_ml, q_stride, out_stride, bt_stride, H, Hkv, GT, n_parts, part_pages, scale, inv_freq, write, (float*)k_pages, (float*)v_pages};
     switch (hs) {
         case 16: return af_launch<16>(a, n_tiles, s);
         case 32: return af_launch<32>(a, n_tiles, s);

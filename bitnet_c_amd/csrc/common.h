@@ -10,7 +10,8 @@
 // Decode attention splits a sequence's keys over workgroups in runs of at least this many pages: shorter
 // runs cost more in merging than they gain in parallelism (measured at batch 1, 8 and 64 of an 8B shape).
 #define BN_SPLIT_MIN_PAGES 2
-// A float32 cache's keys are summed in runs of this many positions (whole pages, counted from position 0), each run by
+// A float32 cache's keys are summed by attn_rows.hip (what attn_f32.hip, with runs of its own, does not take) in runs of this
+// many positions (whole pages, counted from position 0), each run by
 // itself and the runs folded in order: a decode step then spreads a long sequence's runs over workgroups and still forms
 // every sum in the order in which a prompt step forms it, so that float32 logits do not depend on how a sequence was cut.
 #define BN_F32_FOLD_KEYS 2048
@@ -76,6 +77,12 @@ template <> __device__ __forceinline__ bf16 from_f32<bf16>(float v) { return __f
 // bf16 bits <-> float without going through the class type (for packed loads)
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) {
     return __uint_as_float(((uint32_t)b) << 16);
+}
+// A rotation of (x0, x1) by an angle, its operations written out: the same bits in every kernel that turns float32 heads.
+__device__ __forceinline__ void bn_rotate_pair(float& x0, float& x1, float c, float s) {
+    const float y0 = __fmaf_rn(x0, c, -__fmul_rn(x1, s));
+    x1 = __fmaf_rn(x0, s, __fmul_rn(x1, c));
+    x0 = y0;
 }
 __device__ __forceinline__ float bf16lo_to_f32(uint32_t two) { return __uint_as_float(two << 16); }
 __device__ __forceinline__ float bf16hi_to_f32(uint32_t two) { return __uint_as_float(two & 0xffff0000u); }

@@ -45,7 +45,13 @@ __global__ void rope_kv_write_kernel(T* __restrict__ qkv, int row_stride,
     for (int idx = threadIdx.x; idx < H * half; idx += blockDim.x) {
         const int h = idx / half, i = idx - h * half;
         T* hd = row + h * hs;
-        const float v0 = to_f32(hd[i]), v1 = to_f32(hd[i + half]);
+        float v0 = to_f32(hd[i]), v1 = to_f32(hd[i + half]);
+        if (sizeof(T) == 4) {                // as the decode form of float32 attention does it
+            bn_rotate_pair(v0, v1, cos_s[i], sin_s[i]);
+            hd[i] = from_f32<T>(v0);
+            hd[i + half] = from_f32<T>(v1);
+            continue;
+        }
         hd[i] = from_f32<T>(v0 * cos_s[i] - v1 * sin_s[i]);
         hd[i + half] = from_f32<T>(v0 * sin_s[i] + v1 * cos_s[i]);
     }
@@ -58,7 +64,12 @@ __global__ void rope_kv_write_kernel(T* __restrict__ qkv, int row_stride,
         const int kh = idx / hs, d = idx - kh * hs;
         const T* hd = krow + kh * hs;
         float o;
-        if (d < half) {
+        if (sizeof(T) == 4 && d < 2 * half) {
+            const int i = d < half ? d : d - half;
+            float v0 = to_f32(hd[i]), v1 = to_f32(hd[i + half]);
+            bn_rotate_pair(v0, v1, cos_s[i], sin_s[i]);
+            o = d < half ? v0 : v1;
+        } else if (d < half) {
             o = to_f32(hd[d]) * cos_s[d] - to_f32(hd[d + half]) * sin_s[d];
         } else if (d < 2 * half) {
             const int i = d - half;

@@ -166,9 +166,9 @@ _SIGNATURES = {
     },
     "attn_f32": {
         "bn_attn_f32_supports": [c_int],
-        "bn_attn_f32_run_keys": [],
+        "bn_attn_f32_part_pages": [c_longlong, c_int, c_int],
         "bn_attn_f32": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int,
-                        c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p, c_void_p],
+                        c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     },
     "gemm_f32": {
         "bn_gemm_f32_supports": [c_int, c_int, c_int, c_void_p],
@@ -1388,7 +1388,7 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
     bf16 with head size 64 or 128 over blocked pages runs on the matrix cores, everything else on the vector ALUs,
     which read rows and transposed values (force_vector: say so where the pages are not blocked and the head size
     would be the other kernel's; its qt then is that of attention_row_shape without dtype).
-    Decode on the matrix cores can do the work of rope_kv_write itself (can_fuse_decode):
+    Decode on the matrix cores can do the work of rope_kv_write itself (bf16: can_fuse_decode; float32: f32_attention):
     fused_rotate = inv_freq [hs/2]: qkv arrives unrotated, Q and the new K are rotated inside;
     fused_write: the new K, V of every row (from qkv) are stored at position seq_lens - 1 first.
     by_length (decode form, optional): [B] int32, a permutation of the rows, longest sequence
@@ -1479,7 +1479,8 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
             raise KernelError("attention: at most 64 splits (1,024 runs of a float32 cache)")
     parts = n_splits
     if f32_plain:                     # however the caller cuts them, the keys are summed page by page and run by run
-        parts = -(-block_table.shape[1] * PAGE // _fn("attn_f32", "bn_attn_f32_run_keys")()) if decode else 1
+        part_pages = _fn("attn_f32", "bn_attn_f32_part_pages")(T * H, block_table.shape[1], hs)
+        parts = -(-block_table.shape[1] // part_pages) if decode else 1
     if parts > 1:
         part_o = torch.empty((T * H * parts, vd), dtype=torch.float32, device=qkv.device)
         part_ml = torch.empty((T * H * parts, 2), dtype=torch.float32, device=qkv.device)
@@ -1492,7 +1493,7 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
         if not decode or by_length.numel() != T or not by_length.is_contiguous():
             raise KernelError("attention: by_length is one entry per row of the decode form")
     fused = fused_rotate is not None or fused_write
-    if fused and not (use_mfma and decode and can_fuse_decode(qkv.dtype, H, Hkv, hs)):
+    if fused and not (decode and (f32_plain or (use_mfma and can_fuse_decode(qkv.dtype, H, Hkv, hs)))):
         raise KernelError("attention: rotation / cache write inside the kernel needs the decode form on the "
                           "matrix cores with at most 16 heads per kv head")
     if fused_rotate is not None:
@@ -1529,8 +1530,8 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
     if f32_plain:
         _check(_fn("attn_f32", "bn_attn_f32")(
             qkv.data_ptr(), _rows(qkv, "qkv"), out.data_ptr(), H * hs, k_pages.data_ptr(), v_pages.data_ptr(),
-            block_table.data_ptr(), block_table.shape[1], sl, tl, n_tiles, H, Hkv, hs, GT, float(scale), int(parts), po, pm,
-            _stream()), "attention(float32)")
+            block_table.data_ptr(), block_table.shape[1], sl, tl, n_tiles, H, Hkv, hs, GT, float(scale), int(part_pages), po, pm,
+            fused_rotate.data_ptr() if fused_rotate is not None else None, int(bool(fused_write)), _stream()), "attention(float32)")
         return
     _check(_fn("attn_rows", "bn_attn_rows")(
         _code(qkv.dtype), qkv.data_ptr(), _rows(qkv, "qkv"), out.data_ptr(), H * vd,

@@ -296,8 +296,9 @@ class Attention(Part):
         last = self.o.lazy if lazy_ok else self.o
         fuse_ok, inv_freq = self.position.fusable(hs)
         vt, blocked = kv.v_transposed, bool(kv.blocked)
-        decode_fused = (ctx.is_decode and fuse_ok and ops.can_fuse_decode(self.qkv.weight.dtype, H, Hkv, hs)
-                        and blocked)                            # the matrix-core kernels read blocked pages
+        plain_f32 = not blocked and not vt and not self.window and ops.f32_attention(self.qkv.weight.dtype, hs)
+        decode_fused = (ctx.is_decode and fuse_ok               # the matrix-core kernels for bf16 read blocked pages
+                        and (plain_f32 or (blocked and ops.can_fuse_decode(self.qkv.weight.dtype, H, Hkv, hs))))
         row_scale = None
         if isinstance(h, ops.DeferredNorm) and h.shape[0] > ops.FUSED_ROWS:
             # More rows than the fused product takes.  When the decode kernel rotates by itself it can apply the norm's
@@ -339,7 +340,6 @@ class Attention(Part):
                           v_transposed=vt, blocked=blocked)
         else:
             # pages in another order than the matrix-core kernels' own: the float32 kernel or the vector kernel, with their tiles
-            plain_f32 = h.dtype == torch.float32 and not blocked and not vt and not self.window
             _, _, qt = ops.attention_row_shape(H, Hkv, False, h.dtype if blocked or plain_f32 else None, hs, plain_f32)
             ops.attention(qkv, out, kv.k_pages, kv.v_pages, kv.block_table, H, Hkv, hs, self.scale,
                           window=self.window, tiles=ctx.tiles(qt), qt=qt, v_transposed=vt, blocked=blocked)
