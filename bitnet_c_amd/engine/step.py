@@ -564,8 +564,10 @@ class Engine:
 
     def _prompt_bucket_ready(self, entries, n_new) -> bool:
         """Whether this prompt step is replayed from a graph: its bucket has been seen before (the first step of a
-        bucket runs eagerly: one-off prompts never pay for a capture)."""
-        if sum(n_new) > MAX_PROMPT_GRAPH_ROWS:
+        bucket runs eagerly: one-off prompts never pay for a capture).  No graph holds more sequences or wanted rows than
+        the largest bucket: such steps stay eager."""
+        if (sum(n_new) > MAX_PROMPT_GRAPH_ROWS
+                or max(len(entries), sum(len(e.want) for e in entries)) > DECODE_BUCKETS[-1]):
             return False
         key = self._prompt_key(entries, n_new)
         if key in self._prompt_graphs:
@@ -577,7 +579,8 @@ class Engine:
     def prepare_prompt(self, n_tokens: int, n_seqs: int = 1, n_wanted: int = 1) -> None:
         """Captures, now, the graph that prompt steps of this size replay (a server does it for the sizes it
         expects, a benchmark before its clock starts).  Needs one eager prompt step to have run before."""
-        if not (self.use_graphs and self.prompt_graphs and self.tap is None) or n_tokens > MAX_PROMPT_GRAPH_ROWS:
+        if (not (self.use_graphs and self.prompt_graphs and self.tap is None) or n_tokens > MAX_PROMPT_GRAPH_ROWS
+                or max(n_seqs, n_wanted) > DECODE_BUCKETS[-1]):
             return
         if self._prompt_lists is None:
             raise StepError("prepare_prompt: run one prompt step first (it shows which tile lists the model's parts use)")

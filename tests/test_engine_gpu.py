@@ -776,6 +776,26 @@ def test_decoding_with_the_split_plan_of_a_very_long_context(H, Hkv, lens, monke
     eng.cache.check()
 
 
+@pytest.mark.parametrize("seqs,tokens,wants", [(1, 300, 300), (300, 2, 1), (1, 300, 256)])
+def test_prompt_steps_beyond_the_largest_bucket_stay_eager(model_folders, seqs, tokens, wants):
+    """More wanted places or more sequences than any captured prompt step holds: every step returns all its rows."""
+    import bitnet_c_amd as bn
+    folder = model_folders("A", torch.float32)
+    vocab = pl.read_config(folder)["vocab"]
+    eng = bn.Engine.from_folder(folder, dtype=torch.float32, max_tokens=320 * 64)
+    rnd, outs = random.Random(3), []
+    prompts = [[rnd.randrange(vocab) for _ in range(tokens)] for _ in range(seqs)]
+    for _ in range(3):
+        slots = [eng.new_sequence() for _ in range(seqs)]
+        outs.append(eng.step([bn.StepEntry(s, p, list(range(wants))) for s, p in zip(slots, prompts)]))
+        for s in slots:
+            eng.release(s)
+    eng.prepare_prompt(seqs * tokens, seqs, seqs * wants)
+    assert bool(eng._prompt_graphs) == (max(seqs, seqs * wants) <= 256)
+    for out in outs:
+        assert out.shape[0] == seqs * wants and torch.equal(out, outs[0])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["A", "B"])
 def test_prompt_steps_are_replayed_from_graphs(model_folders, name, dtype, monkeypatch):
