@@ -18,7 +18,7 @@
 //                        a function of the sizes alone, so a token's output does not depend on how the step was cut.
 //                        This "chain" form serves decode steps, key widths above LC_MAX_DIM and prompt steps of so
 //                        many sequences that it fills the chip (bn_lightning_prefers_chunks).
-//   the chunked form     other prompt steps: a workgroup owns (sequence, head, 16 value columns) and takes the tokens in
+//   the chunked form     other prompt steps: a workgroup owns (sequence, head, 16 or 32 value columns) and takes the tokens in
 //                        chunks of 64, from a float32 copy of the recurrence's q, k and v that a kernel in front makes.  With d the decay, S the state before the chunk, n its tokens:
 //                            A_ij = (q_i . k_j) d^(i-j) for j <= i,    o_i = sum_j A_ij v_j + d^(i+1) S^T q_i,
 //                            S   <- d^n S + sum_j d^(n-1-j) k_j v_j^T
@@ -469,9 +469,13 @@ static int lc_dispatch(int dtype, LaArgs& a, int n_seqs, int n_rows, const int* 
     const int rc = bn_launch_status();
     if (rc != 0) return rc;
     a.pq = p.q; a.pk = p.k; a.pv = p.v; a.T = n_rows; a.dks = p.dks; a.dvs = p.dvs;
-    // a workgroup takes 16 value columns: blocks of 32 and 64 columns (which share one Q K^T among more columns) took as
-    // long per column when they were measured, with a fourth of the workgroups
-    return a.dk <= 64 ? lc_launch<1, 1>(a, n_seqs, s) : lc_launch<2, 1>(a, n_seqs, s);
+    // Value columns of a workgroup.  A chunk of 64 tokens takes a workgroup 8.2 us with 16 columns, 10.6 with 32 and 20 with 64 (keys
+    // 128 wide; a CU holds one workgroup): 16 while every workgroup has a CU, 32 from there on (four prompts of 500 tokens, 16
+    // heads of 128: 111 us, 153 with 16 and 187 with 64; eight of 256: 114, 153, 112).  Keys up to 64 wide leave room
+    // for several workgroups a CU: 16 (58 us against 73).
+    if (a.dk <= 64) return lc_launch<1, 1>(a, n_seqs, s);
+    const bool wide = (long long)n_seqs * a.H * ((a.dv + 15) / 16) > la_compute_units();
+    return wide ? lc_launch<2, 2>(a, n_seqs, s) : lc_launch<2, 1>(a, n_seqs, s);
 }
 
 extern "C" int bn_lightning_supports(int dk, int dv) { return (dk >= 1 && dk <= LA_MAX_DIM && dv >= 1) ? 1 : 0; }
@@ -480,7 +484,7 @@ extern "C" int bn_lightning_supports(int dk, int dv) { return (dk >= 1 && dk <= 
 extern "C" int bn_lightning_chunked(int dk, int dv) { return (dk >= 1 && dk <= LC_MAX_DIM && dv >= 1) ? 1 : 0; }
 // 1 when a prompt step of n_seqs sequences should: the chain form walks a sequence token by token and has a workgroup per
 // (sequence, head, 64 columns); from two workgroups a CU on it fills the chip and is the faster one (32 prompts of 256
-// tokens, 16 heads of 128 x 128: 0.31 ms against 0.44), below that the chunks are (one prompt of 2,048: 0.26 ms against 1.58)
+// tokens, 16 heads of 128 x 128: 0.30 ms against 0.45), below that the chunks are (one prompt of 2,048: 0.26 ms against 1.58)
 extern "C" int bn_lightning_prefers_chunks(int n_seqs, int H, int dk, int dv) {
     if (!bn_lightning_chunked(dk, dv) || n_seqs <= 0 || H <= 0) return 0;
     return (long long)n_seqs * H * ((dv + LA_CB - 1) / LA_CB) < 2LL * la_compute_units() ? 1 : 0;

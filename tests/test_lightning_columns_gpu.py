@@ -1,0 +1,31 @@
+"""The chunked form of the linear attention takes 16 or 32 value columns a workgroup, by how many workgroups that makes: a
+launch of many sequences (32) gives the bits of one launch a sequence (16), outputs and states."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("H,dk,dv,lens", [(16, 128, 128, [130, 64, 1, 65]), (40, 72, 24, [63, 5, 129, 64, 200]),
+                                          (80, 66, 41, [70, 17])])
+def test_many_sequences_and_one_at_a_time(H, dk, dv, lens):
+    from bitnet_c_amd import ops
+    torch.manual_seed(dk + dv)
+    B, T = len(lens), sum(lens)
+    assert ops.lightning_chunked(dk, dv) and B * H * -(-dv // 16) > 256 >= H * -(-dv // 16)
+    x = torch.randn(T, H * (2 * dk + dv), device=DEV)
+    decay = torch.rand(H, device=DEV) * 0.2 + 0.8
+    state = torch.randn(B + 1, H * dk * dv, device=DEV)
+    alone, slots = state.clone(), torch.randperm(B).to(torch.int32)
+    tiles, row = [], 0
+    for b, n in enumerate(lens):
+        tiles.append([b, row, n, 0 if b == 1 else 40])
+        row += n
+    scan = lambda st, tl: ops.lightning_scan(x, 0, H * dk, 2 * H * dk, decay, st, slots.to(DEV), H, dk, dv,
+                                             tiles=torch.tensor(tl, dtype=torch.int32, device=DEV), chain=False)
+    together = scan(state, tiles)
+    for t in tiles:
+        rows = slice(t[1], t[1] + t[2])
+        assert torch.equal(scan(alone, [t])[rows], together[rows])
+    assert torch.isfinite(together).all() and torch.equal(state, alone)
