@@ -3,7 +3,7 @@
 // kv groups, float32 or bf16 cache, written on the vector ALUs.  Head sizes whose rows are
 // not whole 16-byte groups are staged element by element and padded with zeros in shared
 // memory to the next multiple of 8, which changes no sum.
-// It serves the float32 path, every shape the matrix-core kernels do not take, and
+// It serves every shape and option that the matrix-core kernels (attn_f32.hip for a float32 cache) do not take, in
 // both phases: a workgroup owns up to RT "rows", a row being one (query token, query
 // head) pair that shares one kv head; decode is the case of one query token per
 // sequence, where the keys of a long context are split over gridDim.z and merged by

@@ -1,7 +1,6 @@
 // C[M, N] = A[M, K] . W[N, K]^T with float32 accumulation on the vector ALUs, for any
-// M, N, K and any alignment.  This is the matrix product of the float32 path (no
-// reduced-precision matrix mode: plain fmaf) and the fallback for shapes that the bf16
-// matrix-core kernels refuse.  W is row-major [out, in] as the reference keeps it
+// M, N, K and any alignment (plain fmaf): the fallback for shapes that the matrix-core
+// kernels of either type refuse.  W is row-major [out, in] as the reference keeps it
 // (src/model.c:157-158); out[row] = sum_col W[row, col] x[col]
 // (src/quant/f32_scalar.c:4-32, src/quant/bf16_scalar.c:4-21).
 //

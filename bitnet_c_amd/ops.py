@@ -1385,8 +1385,8 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
     padding row); row b of qkv is sequence b's token; n_splits/chunk from decode_splits.  Every entry of
     block_table names a page of the pool, also those behind a sequence's last page (0 will do): the
     matrix-core kernel asks for a workgroup's first block of keys before it knows the sequence's length.
-    bf16 with head size 64 or 128 over blocked pages runs on the matrix cores, everything else on the vector ALUs,
-    which read rows and transposed values (force_vector: say so where the pages are not blocked and the head size
+    bf16 with head size 64 or 128 over blocked pages runs on the matrix cores, and so does plain float32 (f32_attention);
+    everything else on the vector ALUs, which read rows and transposed values (force_vector: say so where the pages are not blocked and the head size
     would be the other kernel's; its qt then is that of attention_row_shape without dtype).
     Decode on the matrix cores can do the work of rope_kv_write itself (bf16: can_fuse_decode; float32: f32_attention):
     fused_rotate = inv_freq [hs/2]: qkv arrives unrotated, Q and the new K are rotated inside;
