@@ -27,7 +27,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define AF_PARTS_BYTES (64ll << 20)
 
 struct AfArgs {
-    const float* q;           // [n_tokens, q_stride], head h at h * hs (already rotated)
+    const float* q;           // [n_tokens, q_stride], head h at h * hs, rotated (unless inv_freq says that the kernel does it)
     float* out;               // [n_tokens, out_stride]
     const float* k_pages;     // [n_pages, Hkv, BN_PAGE, hs]
     const float* v_pages;
