@@ -260,7 +260,8 @@ struct WkvArgs {
 // How a workgroup of the recurrence meets its sequence: the whole of it (WKV_WALK), or, where a step offers too few sequences
 // and heads to fill the chip, one piece of WKV_PIECE tokens: every piece's own sum from nothing and the product of its decays
 // (WKV_SUMS), a pass that carries the state through the pieces (wkv_carry_kernel), every piece again from its start with
-// outputs (WKV_OUTPUTS).  The recurrence is linear in S, so this is the same sum in another order of rounding.
+// outputs (WKV_OUTPUTS).  The recurrence is linear in S, so this is the same sum in another order of rounding: not for callers
+// whose float32 bits must not depend on how a sequence was cut into steps.
 #define WKV_PIECE 64
 enum { WKV_WALK = 0, WKV_SUMS = 1, WKV_OUTPUTS = 2 };
 
@@ -679,14 +680,14 @@ extern "C" int bn_wkv_step(int dtype, const void* r, int ldr, const void* k, int
 // biases.  A workgroup owns GRU_CH channels of one sequence.  Its tokens come in stages of GRU_TC: all threads load a
 // stage (the next one is asked for before the current one is walked), turn it into gate, candidate and silu(g) and
 // park those in shared memory; one thread a channel then walks the stage, S <- S + z (cand - S), and leaves S silu(g),
-// which all threads store.  The chain of a channel is the same operations in the same order whatever the step holds.
+// which all threads store.  The chain of a walked channel is the same operations in the same order whatever the step holds.
 #define GRU_CH 64
 #define GRU_TC 64
 #define GRU_THREADS 256
 #define GRU_PER_THREAD (GRU_CH * GRU_TC / GRU_THREADS)
 
-// FORM: the whole sequence, or (long steps of few sequences) one piece of GRU_TC tokens, as the wkv recurrence is cut: its own
-// chain from nothing and the product of its (1 - z) (GRU_SUMS), the carry through the pieces (mingru_carry_kernel), the chain
+// FORM: the whole sequence, or (long bf16 steps of few sequences) one piece of GRU_TC tokens, as the wkv recurrence is cut, in
+// another order of rounding: its own chain from nothing and the product of its (1 - z) (GRU_SUMS), the carry through the pieces (mingru_carry_kernel), the chain
 // again from the piece's start with outputs (GRU_OUTPUTS).  One sequence of 2,048 tokens, 2,048 channels: 235 us walked,
 // 44 in pieces.
 enum { GRU_WALK = 0, GRU_SUMS = 1, GRU_OUTPUTS = 2 };

@@ -55,6 +55,9 @@ class StepContext:
         self.slots, self.n_new, self.pos0 = list(slots), list(n_new), list(pos0)   # host copies
         self.n_rows = int(tokens.numel())
         self.n_seqs = len(self.slots)
+        # (token rows, sequences) as a captured step of this request holds them: what a part whose choice of kernel changes
+        # bits chooses by, so that the first, eager step of a request and its replays choose alike
+        self.sizes = _row_bucket(self.n_rows), max(self.n_seqs, _bucket(self.n_seqs))
         # diagnostics: a callable (point, schedule entry, ResidualStream, ctx) that blocks call at "layer_in",
         # "ffn_in" and "layer_out" (the reference's bitnet_inp / bitnet_ffn_inp / bitnet_lout dumps,
         # src/transformer/cpu.c:401, :951, :981); `entry` is the schedule entry that is running

@@ -1978,25 +1978,51 @@ def wkv_state_floats(H: int, dk: int, dv: int) -> int:
     return H * p * WKV_ROWS_PER_THREAD * dv
 
 
-# Long prompt steps of few sequences are cut into pieces that are walked side by side instead of every sequence from its
-# first token to its last: twice the arithmetic on many times the workgroups.  us walked / in pieces, wkv with 32 heads of 64
-# and the min-GRU with 2,048 channels (32 workgroups a sequence either way): one sequence of 256 tokens 89 / 65 and 34 / 21, of
-# 2,048 617 / 203 and 235 / 44; four of 512 179 / 198 and 62 / 41; eight of 512 177 / 365 and 65 / 65.  So up to
-# SCAN_PIECES_GROUPS workgroups of the plain walk.
-SCAN_PIECES_GROUPS = 96
-SCAN_PIECES_MIN_ROWS = 256
+# Long prompt steps of few sequences may be cut into pieces that are walked side by side instead of every sequence from its
+# first token to its last: twice the arithmetic on many times the workgroups, in another order of rounding.  So float32 steps
+# are never cut (a position's float32 bits do not depend on how its sequence came in), and the choice is made by the sizes of a
+# captured step (StepContext.sizes), which the first, eager step of a request and its replays share.  What pays for pieces is
+# the length of a walk, of which rows / seqs is what is known in both; what they cost grows with the whole step's state.
+# us walked / in pieces, bf16.  wkv, 32 heads of 64 x 64: one sequence of 128 tokens 52 / 60, 256 90 / 66, 2,048 625 / 195; two
+# of 256 91 / 92, 512 167 / 130, 2,048 626 / 357; four of 512 176 / 195, 2,048 651 / 689; 64 heads: one of 256 92 / 91, 512
+# 168 / 129, two of 512 177 / 220; 16 heads of 128 x 128: one of 256 94 / 106, 512 175 / 150, two of 512 183 / 250.  Min-GRU,
+# 2,048 channels: one sequence of 128 tokens 21 / 23, 256 35 / 23, 2,048 237 / 44; four of 256 36 / 32, 512 65 / 44; eight
+# of 256 36 / 46, 512 67 / 66; 4,096 channels: four of 512 67 / 65, six 74 / 89.
+SCAN_PIECES_LENGTH = 256                  # the shortest walk; half of the shortest at which twice the state pays
+SCAN_PIECES_SEQS = 32                     # a workgroup finds its piece by going through the sequences before it
+WKV_PIECES_STATE = 32 * 64 * 64           # numbers of state of a step's sequences together
+GRU_PIECES_STATE = 4 * 2048
+SCAN_PIECES_BYTES = 2 << 30               # a state a piece: a seventh of the step's own activations at 32 heads of 64, width 2,048
 WKV_PIECE = _build.header_constant("WKV_PIECE", "state_mixers.hip")
 GRU_PIECE = _build.header_constant("GRU_TC", "state_mixers.hip")
 
 
-def _scan_pieces(pieces, tl, T: int, n_seqs: int, groups: int, piece: int, floats: int, device):
-    """(pieces that the step's sequences can have together or 0, scratch of a state a piece) of a prompt step; groups: the
-    workgroups of the plain walk; floats: of a sequence's state."""
-    most = -(-T // piece) + n_seqs                       # every sequence may end in a piece that is not full
-    if pieces is None:
-        pieces = T >= SCAN_PIECES_MIN_ROWS and groups <= SCAN_PIECES_GROUPS and n_seqs <= 32 and most * floats * 4 <= 2 << 30
+def _in_pieces(dtype, sizes, state: int, unit: int, piece: int) -> bool:
+    rows, seqs = sizes
+    return (dtype == torch.bfloat16 and seqs <= SCAN_PIECES_SEQS and seqs * state <= min(rows // seqs // SCAN_PIECES_LENGTH, 2) * unit
+            and _pieces_of(rows, seqs, piece) * state * 4 <= SCAN_PIECES_BYTES)
+
+
+def wkv_in_pieces(dtype, sizes, H: int, dk: int, dv: int) -> bool:
+    """Whether wkv_scan cuts a prompt step into pieces; sizes: StepContext.sizes, (token rows, sequences)."""
+    return _in_pieces(dtype, sizes, H * dk * dv, WKV_PIECES_STATE, WKV_PIECE)
+
+
+def mingru_in_pieces(dtype, sizes, W: int) -> bool:
+    """Whether mingru_scan cuts a prompt step into pieces; sizes: StepContext.sizes."""
+    return _in_pieces(dtype, sizes, W, GRU_PIECES_STATE, GRU_PIECE)
+
+
+def _pieces_of(T: int, n_seqs: int, piece: int) -> int:
+    """What n_seqs sequences of T tokens can have together: each may end in a piece that is not full."""
+    return -(-T // piece) + n_seqs
+
+
+def _piece_states(pieces: bool, tl, T: int, n_seqs: int, piece: int, floats: int, device):
+    """(pieces of a prompt step or 0, scratch of a state of so many floats a piece)."""
     if not pieces or tl is None or not T or not n_seqs:
         return 0, None
+    most = _pieces_of(T, n_seqs, piece)
     return most, torch.empty((most, floats), dtype=torch.float32, device=device)
 
 
@@ -2047,20 +2073,20 @@ def wkv_step(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, se
 
 
 def wkv_scan(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, *, tiles=None, seq_lens=None,
-             pieces: Optional[bool] = None) -> torch.Tensor:
+             pieces: bool = False) -> torch.Tensor:
     """The wkv recurrence over every sequence of a step; float32 [T, H dv].  r, k, d: [T, H dk] (rows contiguous, any row
     stride), v: [T, H dv], in the activations' type; w0, u: float32 [H dk] (the decay's offset, the current token's
     bonus); h [T, D]: the mixer's input.  state [slots, >= wkv_state_floats(H, dk, dv) + D] float32: the heads' matrices
     in the kernel's own order, then the last h, both updated in place.  Per head, in float32:
         w_t = exp(-exp(d_t + w0));  o_t = (S + diag(u) k_t v_t^T)^T r_t;  S <- diag(w_t) S + k_t v_t^T.
     pieces (prompt form): whether every sequence is cut into pieces of WKV_PIECE tokens that are walked side by side (the
-    results differ from the plain walk's by rounding alone); None: by the step's size (_scan_pieces)."""
+    results differ from the plain walk's by rounding alone; wkv_in_pieces says when that is the faster way)."""
     require_gpu()
     T, D, stride = _wkv_args(r, k, v, d, w0, u, h, state, slot_ids, H, dk, dv, "wkv_scan")
     tl, n_tiles, sl = _seq_args(tiles, seq_lens, "wkv_scan")
     o = torch.empty((T, H * dv), dtype=torch.float32, device=h.device)
     floats = wkv_state_floats(H, dk, dv)
-    most, carry = _scan_pieces(pieces, tl, T, n_tiles, n_tiles * H, WKV_PIECE, floats, h.device)
+    most, carry = _piece_states(pieces, tl, T, n_tiles, WKV_PIECE, floats, h.device)
     fade = torch.empty((carry.shape[0], floats // dv), dtype=torch.float32, device=h.device) if most else None
     if T and n_tiles:
         _check(_fn("state_mixers", "bn_wkv_scan")(
@@ -2092,12 +2118,12 @@ def head_norm_gate(o: torch.Tensor, gate: torch.Tensor, weight: Optional[torch.T
 
 
 def mingru_scan(zxg: torch.Tensor, bias_z, bias_x, state: torch.Tensor, slot_ids, W: int, *, tiles=None,
-                seq_lens=None, pieces: Optional[bool] = None) -> torch.Tensor:
+                seq_lens=None, pieces: bool = False) -> torch.Tensor:
     """The min-GRU recurrence over every sequence of a step.  zxg [T, 3 W]: the projections of the update gate, the
     candidate and the output gate side by side, without biases (bias_z, bias_x: float32 [W] or None).  state
     [slots, >= W] float32, updated in place.  Per channel, in float32: z = sigmoid(a + bias_z); c = b + bias_x;
     cand = c + 1/2 where c >= 0, sigmoid(c) below; S <- (1 - z) S + z cand; result S * silu(g), [T, W].
-    pieces: as wkv_scan's, of GRU_PIECE tokens."""
+    pieces: as wkv_scan's, of GRU_PIECE tokens (mingru_in_pieces)."""
     require_gpu()
     _dev(zxg, "zxg", dims=2)
     T = zxg.shape[0]
@@ -2112,7 +2138,7 @@ def mingru_scan(zxg: torch.Tensor, bias_z, bias_x, state: torch.Tensor, slot_ids
     _dev(slot_ids, "slot_ids", torch.int32, 1)
     tl, n_tiles, sl = _seq_args(tiles, seq_lens, "mingru_scan")
     y = torch.empty((T, W), dtype=zxg.dtype, device=zxg.device)
-    most, carry = _scan_pieces(pieces, tl, T, n_tiles, n_tiles * -(-W // 64), GRU_PIECE, W, zxg.device)
+    most, carry = _piece_states(pieces, tl, T, n_tiles, GRU_PIECE, W, zxg.device)
     fade = torch.empty_like(carry) if most else None
     if T and n_tiles:
         _check(_fn("state_mixers", "bn_mingru_scan")(

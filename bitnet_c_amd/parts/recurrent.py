@@ -100,7 +100,8 @@ class WKV(Part):
         if ctx.is_decode and ops.wkv_step_supported(hs, hs):
             y = ops.wkv_step(r, k, v, d, self.w0, self.u, h, state, ctx.slot_ids, H, hs, hs, ctx.seq_lens, g, self.norm, self.eps)
         else:
-            o = ops.wkv_scan(r, k, v, d, self.w0, self.u, h, state, ctx.slot_ids, H, hs, hs, **_sequences(ctx))
+            o = ops.wkv_scan(r, k, v, d, self.w0, self.u, h, state, ctx.slot_ids, H, hs, hs,
+                             pieces=ops.wkv_in_pieces(h.dtype, ctx.sizes, H, hs, hs), **_sequences(ctx))
             y = ops.head_norm_gate(o, g, self.norm, H, hs, self.eps)
         return self.o(y)
 
@@ -142,7 +143,8 @@ class MinGRU(Part):
     def forward(self, h, ctx, kv, projected=None):
         """projected: the first product's result; the last product is then left to whoever gave it."""
         zxg = self.zxg(h) if projected is None else projected
-        y = ops.mingru_scan(zxg, self.bz, self.bx, kv.state, ctx.slot_ids, self.W, **_sequences(ctx))
+        y = ops.mingru_scan(zxg, self.bz, self.bx, kv.state, ctx.slot_ids, self.W,
+                            pieces=ops.mingru_in_pieces(zxg.dtype, ctx.sizes, self.W), **_sequences(ctx))
         return self.o(y) if projected is None else y
 
 
