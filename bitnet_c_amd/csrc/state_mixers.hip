@@ -585,15 +585,16 @@ extern "C" int bn_head_norm_gate(int dtype, void* y, const float* o, const void*
 
 // ---- a decode step of wkv with its norm and gate -------------------------------------------------------------------------
 // One token of every sequence: a workgroup owns a (sequence, head) whole, a thread the rows of a column that the walk gives it
-// (P neighbouring lanes a column), so the state's way in and out is one load and one store a number; the head's root mean
-// square, weight and gate follow on the sums that the lanes hold.  Bound by latency at few sequences (a trip to memory for the
-// state, three barriers): one sequence of 32 heads of 64 6.9 us, where the walk and
-// the norm's kernel took 7.8 + 5.0.
+// (P neighbouring lanes a column), so the state's way in and out is one load and one store a number; the columns' sums meet in
+// shared memory, where every wave forms the head's mean square as head_norm_gate_kernel does (the same bits as the walk and
+// that kernel: a position's output does not depend on the step it came in), and weight and gate follow.  Bound by latency at
+// few sequences (a trip to memory for the state, two barriers): one sequence of 32 heads of 64 4.8 us in a graph of such
+// launches, 6.9 in a decode step's profile, where the walk and the norm's kernel took 7.8 + 5.0.
 template <typename T>
 __global__ __launch_bounds__(1024) void wkv_step_kernel(WkvArgs a, T* __restrict__ y, const T* __restrict__ gate, int ldg,
                                                         const float* __restrict__ weight, float eps) {
     __shared__ __align__(16) float r_s[WKV_MAX_DIM], k_s[WKV_MAX_DIM], w_s[WKV_MAX_DIM];
-    __shared__ float scratch[16];
+    __shared__ float o_s[WKV_MAX_DIM];
     const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
     const int pos = a.seq_lens[seq] - 1;
     if (pos < 0) return;
@@ -636,11 +637,15 @@ __global__ __launch_bounds__(1024) void wkv_step_kernel(WkvArgs a, T* __restrict
         ww[q] = reinterpret_cast<const float4*>(w_s + p * WKV_KR)[q];
     }
     const float o = wkv_token(rr, kk, ww, vj, ub, S, P);
+    if (owns && p == 0) o_s[j] = o;
     if (owns) {
 #pragma unroll
         for (int ii = 0; ii < WKV_KR; ++ii) S_g[((size_t)ii * dv + j) * P + p] = S[ii];
     }
-    const float ss = block_sum(owns && p == 0 ? o * o : 0.f, scratch);
+    lds_barrier();
+    float ss = 0.f;
+    for (int e = tid & (BN_WAVE - 1); e < dv; e += BN_WAVE) ss = fmaf(o_s[e], o_s[e], ss);
+    ss = wave_sum(ss);
     const float f = 1.0f / sqrtf(ss / (float)dv + eps);
     if (owns && p == 0) y[((size_t)seq * a.H + head) * dv + j] = from_f32<T>(o * f * wj * bn_unary_act(gj, BN_UNARY_SILU));
 }

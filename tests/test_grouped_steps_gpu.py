@@ -69,9 +69,27 @@ def test_wkv_step(dtype, H, d, weighted):
     got = ops.wkv_step(r, k, v, dd, w0, u, h, b, slots, H, d, d, lens, g, weight, 1e-6)
     assert torch.equal(a, b)
     live = [0, 1, 3]
-    # the same sums but for the order of the squares': the factor moves by some roundings of 2^-24, a bf16 result by one of its own
+    # (the bits are equal: test_wkv_step_gives_the_bits_of_the_scan_and_the_norm)
     tol = 2.0 ** -7 if dtype == torch.bfloat16 else 1e-6
     assert torch.all((got[live] - want[live]).abs() <= tol * want[live].abs() + 1e-30)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,d", [(3, 64), (2, 24), (2, 65), (1, 128), (1, 1)])
+def test_wkv_step_gives_the_bits_of_the_scan_and_the_norm(dtype, H, d):
+    """Head widths under, at and over a wave: a decode step's output is the one that a prompt step gives the same position."""
+    from bitnet_c_amd import ops
+    B, A, D = 7, H * d, 24
+    r, k, v, dd, g = (_rand((B, A), 30 + i, dtype) for i in range(5))
+    h, w0, u, weight = _rand((B, D), 40, dtype), _rand((A,), 41) - 2.0, _rand((A,), 42), _rand((A,), 43)
+    state = torch.zeros(B, ops.wkv_state_floats(H, d, d) + D).cuda()
+    slots, lens = torch.randperm(B).to(torch.int32).cuda(), torch.full((B,), 9, dtype=torch.int32).cuda()
+    for i in range(2):
+        ops.wkv_scan(r * (i + 1), k, v, dd, w0, u, h, state, slots, H, d, d, seq_lens=lens)
+    a, b = state.clone(), state.clone()
+    want = ops.head_norm_gate(ops.wkv_scan(r, k, v, dd, w0, u, h, a, slots, H, d, d, seq_lens=lens), g, weight, H, d, 1e-6)
+    got = ops.wkv_step(r, k, v, dd, w0, u, h, b, slots, H, d, d, lens, g, weight, 1e-6)
+    assert torch.equal(got, want) and torch.equal(a, b)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

@@ -79,3 +79,15 @@ def test_eager_recorded_and_replayed(tmp_path, monkeypatch, heads, dim, width, l
     whole = _step(eng, prompts[:1])
     cuts = [2, 3, 64, lens[0] - 69] if lens[0] > 80 else [lens[0] - 2, 2] if lens[0] > 8 else [3, lens[0] - 3]
     assert torch.equal(_step(eng, prompts[:1], cuts), whole)
+
+
+@pytest.mark.parametrize("heads,dim,width", [(2, 64, 96), (3, 24, 40), (5, 65, 33)])
+@pytest.mark.parametrize("graphs", [True, False])
+def test_float32_prompts_and_single_tokens_give_the_same_bits(tmp_path, heads, dim, width, graphs):
+    import bitnet_c_amd as bn
+    folder = write_folder(tmp_path / "m", _config(heads, dim, width), 7, torch.float32)
+    eng = bn.Engine.from_folder(folder, dtype=torch.float32, max_tokens=512, use_graphs=graphs)
+    prompt = [_prompt(3, 150)]
+    whole = _step(eng, prompt)
+    for cuts in ([1] * 40 + [110], [130] + [1] * 20, [64, 1, 1, 63, 1, 20]):
+        assert torch.equal(_step(eng, prompt, cuts), whole)
