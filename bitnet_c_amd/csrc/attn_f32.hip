@@ -25,6 +25,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define AF_RUN_PAGES 4
 #define AF_PARTS_BYTES (64ll << 20)
+#define AF_GROUPS 2048
 
 struct AfArgs {
     const float* q;           // [n_tokens, q_stride], head h at h * hs, rotated (unless inv_freq says that the kernel does it)
@@ -217,38 +218,43 @@ __global__ __launch_bounds__(256, 2) void attn_f32_prompt_kernel(AfArgs a) {
             for (int j = 0; j < 4; ++j) o[16 * S::VW * h + S::VW * (4 * g + j) + i] = __fmul_rn(tot.o[h][i][j], inv);
 }
 
-// PAGES pages are a workgroup of 4 waves each: wave t of a page multiplies the keys 16 t .. 16 t + 15 with the queries, then, with the
-// page's scores exchanged through shared memory, the weights with a quarter of the value's dimensions.  Everything is asked for at
-// once, keys as they lie (their operand comes through shared memory: sixteen rows in sixteen lanes of a load would cost four times the
-// cycles).  inv_freq: the query and the new key arrive unrotated; write: the workgroup that holds the new position stores the new key
-// and value into the pages, and reads them from the token's row itself.  The order of every sum is the prompt form's (af_page).
-// What bounds it is how fast a CU can draw its keys and values (some 25 bytes a nanosecond): one sequence of 200 keys, 16 heads
-// of 128 over 4, 8.9 us and 4.1 for the fold, rotation and store inside; with a workgroup a run of four pages 18.6 in all, with a wave a
-// page of such a run 18.2 and 5.3 for the rotation in front.  Eight sequences of 64 to 1,024 keys: 11.7 and 4.1 (20 + 4 + 4.5 before).
+// A workgroup of 4 waves takes a part of a sequence's keys, one page or the pages of a run in turn: wave t of it multiplies the keys 16 t .. 16 t + 15 with the
+// queries, then, with the page's scores exchanged through shared memory, the weights with a quarter of the value's dimensions.
+// Everything of a page is asked for at once, keys as they lie (their operand comes through shared memory: sixteen rows in sixteen
+// lanes of a load would cost four times the cycles).  inv_freq: the query and the new key arrive unrotated; write: the workgroup
+// that holds the new position stores the new key and value into the pages, and reads them from the token's row itself.  The order
+// of every sum is the prompt form's (af_page).  What bounds it is how fast a CU can draw its keys and values (some 25 bytes a
+// nanosecond), and, in a table much wider than its sequences, how fast workgroups without keys end: they ask for nothing but a
+// length.  us with the fold, 16 heads of 128 over 4, rotation and store inside, in a table of its own width / of 8,192 positions /
+// of 131,072 (in brackets: with every workgroup staging its queries first, and the pages of a run in 16 waves of one workgroup):
+// one sequence of 200 keys 10.2 / 10.2 / 10.2 (10.1 / 10.2 / 30.3), 64 of 200 23.8 / 31.0 / 31.3 (22.7 / 100 / 100), 64 of 1,000
+// 62.7 / 64.9 / 65.1 (65.6 / 154 / 155), eight of 2,000 26.1 / 25.8 / 29.5 (25.6 / 33 / 98).
 template <int HS, int PAGES>
-__global__ __launch_bounds__(256 * PAGES) void attn_f32_decode_kernel(AfArgs a) {
+__global__ __launch_bounds__(256, PAGES == 1 ? 3 : 2) void attn_f32_decode_kernel(AfArgs a) {
     constexpr int NB = HS / 16, STRIDE = HS + 4, HALF = HS / 2;
     constexpr int VW = HS >= 64 ? HS / 64 : 1;    // tiles of the second product a wave: value dimensions 16 VW part + VW row + tile
     constexpr int PARTS = HS / (16 * VW);         // waves of a page that have any
-    extern __shared__ __align__(16) float af_smem[];
-    float* ks = af_smem;                          // [4 PAGES][16][STRIDE] every wave's keys; later [PAGES][16][HS + 1], the pages' sums
-    float* so = af_smem;
-    float* sx = ks + 4 * PAGES * 16 * STRIDE;     // [PAGES][4][64][4] every page's scores, as the lanes hold them
-    float* qs = sx + PAGES * 4 * 64 * 4;          // [16][STRIDE]     the queries
-    float* kn = qs + 16 * STRIDE;                 // [HS]             the new key
-    float* sm = kn + HS;                          // [PAGES][16] each
-    float* sl = sm + PAGES * 16;
+    constexpr int OWN = HS / 16;                  // the sums that a thread folds: (head, dimension) number tid + 256 o
+    __shared__ __align__(16) float ks[4 * 16 * STRIDE];      // every wave's keys; later [16][HS + 1], the page's sums
+    __shared__ __align__(16) float sx[4 * 64 * 4];           // the page's scores, as the lanes hold them
+    __shared__ __align__(16) float qs[16 * STRIDE];          // the queries
+    __shared__ __align__(16) float kn[HS];                   // the new key
+    __shared__ float sm[16], sl[16];
+    float* so = ks;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), pg = wave >> 2, t = wave & 3;
+    const int t = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int GT = a.GT, G = a.H / a.Hkv;
     const int head_tiles = (G + GT - 1) / GT;
     const int kvh = blockIdx.y / head_tiles, ht = blockIdx.y - kvh * head_tiles;
     const int tok = blockIdx.x, len = a.seq_lens[tok];
+    constexpr int part_keys = PAGES * BN_PAGE;
+    // a table is as wide as the longest sequence there can be: most workgroups of a short one have no keys
+    if (blockIdx.z > 0 && (int)blockIdx.z * part_keys >= len) return;
     const int rows = min(GT, G - ht * GT);
     const float* row = a.q + (size_t)tok * a.q_stride;
     const float* new_v = row + (size_t)(a.H + a.Hkv + kvh) * HS;
     // the queries (rows without a head as zeros) and the new key, a pair of dimensions a thread
-    for (int idx = tid; idx < 17 * HALF; idx += 256 * PAGES) {
+    for (int idx = tid; idx < 17 * HALF; idx += 256) {
         const int h = idx / HALF, i = idx - h * HALF;
         const bool is_key = h == 16;
         if (is_key && !a.write) break;
@@ -264,16 +270,17 @@ __global__ __launch_bounds__(256 * PAGES) void attn_f32_decode_kernel(AfArgs a) 
         dst[0] = x0;
         dst[HALF] = x1;
     }
-    for (int part = blockIdx.z; part < a.n_parts && (part == 0 || part * PAGES * BN_PAGE < len); part += gridDim.z) {
-        const int j0 = (part * PAGES + pg) * BN_PAGE;
-        const bool live = j0 < len;               // this wave's page holds keys
-        const int last = min(len - 1 - j0, BN_PAGE - 1);
-        const bool newest = a.write && live && len - 1 - j0 < BN_PAGE;       // the page holds the new position: its row `last`
-        f32x4 kr[NB];
-        float vf[4][4][VW], nv[VW];
-        size_t at = 0;
-        if (live) {
-            at = ((size_t)a.block_table[(size_t)tok * a.bt_stride + j0 / BN_PAGE] * a.Hkv + kvh) * BN_PAGE * HS;
+    for (int part = blockIdx.z; part < a.n_parts && (part == 0 || part * part_keys < len); part += gridDim.z) {
+        float M[OWN], L[OWN], O[OWN];             // (of more pages than one)
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) { M[o] = -INFINITY; L[o] = 0.f; O[o] = 0.f; }
+#pragma unroll 1
+        for (int j0 = part * part_keys; j0 < min((part + 1) * part_keys, len); j0 += BN_PAGE) {
+            const int last = min(len - 1 - j0, BN_PAGE - 1);
+            const bool newest = a.write && len - 1 - j0 < BN_PAGE;           // the page holds the new position: its row `last`
+            f32x4 kr[NB];
+            float vf[4][4][VW], nv[VW];
+            const size_t at = ((size_t)a.block_table[(size_t)tok * a.bt_stride + j0 / BN_PAGE] * a.Hkv + kvh) * BN_PAGE * HS;
             const f32x4* kg = reinterpret_cast<const f32x4*>(a.k_pages + at + (size_t)16 * t * HS);
 #pragma unroll
             for (int i = 0; i < NB; ++i) kr[i] = kg[lane + 64 * i];
@@ -285,108 +292,115 @@ __global__ __launch_bounds__(256 * PAGES) void attn_f32_decode_kernel(AfArgs a) 
                     for (int e = 0; e < 4; ++e) af_values<VW>(vbase + (16 * u + e) * HS, vf[u][e]);
                 if (newest) af_values<VW>(new_v + 16 * VW * t + VW * r, nv);
             }
-        }
-        __syncthreads();                          // the queries and the new key are there; the sums of the part before have been read
-        float* mine = ks + wave * 16 * STRIDE;
-        if (live) {
+            __syncthreads();                      // the queries and the new key are there; the sums of the page before have been read
+            float* mine = ks + t * 16 * STRIDE;
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
                 const int piece = lane + 64 * i, key = piece / (HS / 4), d = 4 * (piece % (HS / 4));
                 if (newest && 16 * t + key == last) kr[i] = *reinterpret_cast<const f32x4*>(kn + d);
                 *reinterpret_cast<f32x4*>(mine + key * STRIDE + d) = kr[i];
             }
-        }
-        if (newest && ht == 0 && t == 0) {        // the new position's rows of the pages, by a wave
-            float* kd = a.k_new + at + (size_t)last * HS;
-            float* vd = a.v_new + at + (size_t)last * HS;
-            for (int d = lane; d < HS; d += 64) { kd[d] = kn[d]; vd[d] = new_v[d]; }
-        }
-        __builtin_amdgcn_wave_barrier();          // a wave's own keys: its shared-memory operations run in order
-        if (live) {
-            f32x4 s = 0.f;
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const f32x4 kf = *reinterpret_cast<const f32x4*>(mine + r * STRIDE + 16 * b + 4 * g);
-                const f32x4 qf = *reinterpret_cast<const f32x4*>(qs + r * STRIDE + 16 * b + 4 * g);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[e], s, 0, 0, 0);
+            if (newest && ht == 0 && t == 0) {    // the new position's rows of the pages, by a wave
+                float* kd = a.k_new + at + (size_t)last * HS;
+                float* vd = a.v_new + at + (size_t)last * HS;
+                for (int d = lane; d < HS; d += 64) { kd[d] = kn[d]; vd[d] = new_v[d]; }
             }
-            *reinterpret_cast<f32x4*>(sx + ((pg * 4 + t) * 64 + lane) * 4) = s;
-        }
-        __syncthreads();
-        if (live && t < PARTS) {
-            f32x4 s[4];
-            float m = -INFINITY, l = 0.f;
+            __builtin_amdgcn_wave_barrier();      // a wave's own keys: its shared-memory operations run in order
+            {
+                f32x4 s = 0.f;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                s[u] = *reinterpret_cast<const f32x4*>(sx + ((pg * 4 + u) * 64 + lane) * 4);
+                for (int b = 0; b < NB; ++b) {
+                    const f32x4 kf = *reinterpret_cast<const f32x4*>(mine + r * STRIDE + 16 * b + 4 * g);
+                    const f32x4 qf = *reinterpret_cast<const f32x4*>(qs + r * STRIDE + 16 * b + 4 * g);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    s[u][e] = 16 * u + 4 * g + e > last ? -INFINITY : __fmul_rn(s[u][e], a.scale);
-                    m = fmaxf(m, s[u][e]);
+                    for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[e], s, 0, 0, 0);
                 }
+                *reinterpret_cast<f32x4*>(sx + (t * 64 + lane) * 4) = s;
             }
-            m = fmaxf(m, __shfl_xor(m, 16, BN_WAVE));
-            m = fmaxf(m, __shfl_xor(m, 32, BN_WAVE));
-            const float base = m == -INFINITY ? 0.f : m;
-            f32x4 o[VW];
+            __syncthreads();
+            if (t < PARTS) {
+                f32x4 s[4];
+                float m = -INFINITY, l = 0.f;
 #pragma unroll
-            for (int i = 0; i < VW; ++i) o[i] = 0.f;
-            if (last < BN_PAGE - 1 || newest) {   // the new value comes from the token's row; rows behind the last key count as zeros
+                for (int u = 0; u < 4; ++u) {
+                    s[u] = *reinterpret_cast<const f32x4*>(sx + (u * 64 + lane) * 4);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        s[u][e] = 16 * u + 4 * g + e > last ? -INFINITY : __fmul_rn(s[u][e], a.scale);
+                        m = fmaxf(m, s[u][e]);
+                    }
+                }
+                m = fmaxf(m, __shfl_xor(m, 16, BN_WAVE));
+                m = fmaxf(m, __shfl_xor(m, 32, BN_WAVE));
+                const float base = m == -INFINITY ? 0.f : m;
+                f32x4 o[VW];
+#pragma unroll
+                for (int i = 0; i < VW; ++i) o[i] = 0.f;
+                if (last < BN_PAGE - 1 || newest) {       // the new value comes from the token's row; rows behind the last key count as zeros
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int key = 16 * u + 4 * g + e;
+#pragma unroll
+                            for (int i = 0; i < VW; ++i) vf[u][e][i] = key > last ? 0.f : key == last && newest ? nv[i] : vf[u][e][i];
+                        }
+                }
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int key = 16 * u + 4 * g + e;
+                    for (int e = 0; e < 4; ++e) { s[u][e] = expf(__fsub_rn(s[u][e], base)); l = __fadd_rn(l, s[u][e]); }
+                l = __fadd_rn(l, __shfl_xor(l, 16, BN_WAVE));
+                l = __fadd_rn(l, __shfl_xor(l, 32, BN_WAVE));
 #pragma unroll
-                        for (int i = 0; i < VW; ++i) vf[u][e][i] = key > last ? 0.f : key == last && newest ? nv[i] : vf[u][e][i];
-                    }
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int i = 0; i < VW; ++i) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][e][i], s[u][e], o[i], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < VW; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) so[r * (HS + 1) + 16 * VW * t + VW * (4 * g + j) + i] = o[i][j];
+                if (t == 0 && g == 0) { sm[r] = m; sl[r] = l; }
             }
+            __syncthreads();
+            if (PAGES > 1)
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { s[u][e] = expf(__fsub_rn(s[u][e], base)); l = __fadd_rn(l, s[u][e]); }
-            l = __fadd_rn(l, __shfl_xor(l, 16, BN_WAVE));
-            l = __fadd_rn(l, __shfl_xor(l, 32, BN_WAVE));
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int i = 0; i < VW; ++i) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][e][i], s[u][e], o[i], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < VW; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) so[(pg * 16 + r) * (HS + 1) + 16 * VW * t + VW * (4 * g + j) + i] = o[i][j];
-            if (t == 0 && g == 0) { sm[pg * 16 + r] = m; sl[pg * 16 + r] = l; }
-        } else if (!live && t == 0 && g == 0) {
-            sm[pg * 16 + r] = -INFINITY;
-            sl[pg * 16 + r] = 0.f;
+                for (int o = 0; o < OWN; ++o) {
+                    const int idx = tid + 256 * o, h = idx / HS, d = idx - h * HS;
+                    if (h >= rows) break;
+                    const float m = sm[h];
+                    if (m == -INFINITY) continue;
+                    float m2, fa, fb;
+                    af_factors(M[o], m, m2, fa, fb);
+                    L[o] = af_fold(L[o], fa, sl[h], fb);
+                    O[o] = af_fold(O[o], fa, so[h * (HS + 1) + d], fb);
+                    M[o] = m2;
+                }
+            // (the barrier behind the next page's loads stands before its keys are stored over the sums)
         }
-        __syncthreads();
-        for (int idx = tid; idx < rows * HS; idx += 256 * PAGES) {
-            const int h = idx / HS, d = idx - h * HS;
-            float M = -INFINITY, L = 0.f, O = 0.f;
-#pragma unroll
-            for (int w = 0; w < PAGES; ++w) {
-                const float m = sm[w * 16 + h];
-                if (m == -INFINITY) continue;
-                float m2, fa, fb;
-                af_factors(M, m, m2, fa, fb);
-                L = af_fold(L, fa, sl[w * 16 + h], fb);
-                O = af_fold(O, fa, so[(w * 16 + h) * (HS + 1) + d], fb);
-                M = m2;
-            }
-            const int head = kvh * G + ht * GT + h;
+        auto put = [&](int idx, float m, float l, float x) {
+            const int h = idx / HS, d = idx - h * HS, head = kvh * G + ht * GT + h;
             if (a.n_parts == 1) {
-                a.out[(size_t)tok * a.out_stride + (size_t)head * HS + d] = __fmul_rn(O, L > 0.f ? 1.0f / L : 0.f);
+                a.out[(size_t)tok * a.out_stride + (size_t)head * HS + d] = __fmul_rn(x, l > 0.f ? 1.0f / l : 0.f);
             } else {
                 const size_t at = ((size_t)tok * a.H + head) * a.n_parts + part;
-                a.part_o[at * HS + d] = O;
-                if (d == 0) { a.part_ml[2 * at] = M; a.part_ml[2 * at + 1] = L; }
+                a.part_o[at * HS + d] = x;
+                if (d == 0) { a.part_ml[2 * at] = m; a.part_ml[2 * at + 1] = l; }
             }
+        };
+        if (PAGES == 1) {                         // a page alone: folded into nothing it is itself
+            const bool none = len <= 0;
+            for (int idx = tid; idx < rows * HS; idx += 256) {
+                const int h = idx / HS;
+                put(idx, none ? -INFINITY : sm[h], none ? 0.f : sl[h], none ? 0.f : so[h * (HS + 1) + idx - h * HS]);
+            }
+        } else {
+#pragma unroll
+            for (int o = 0; o < OWN; ++o)
+                if (tid + 256 * o < rows * HS) put(tid + 256 * o, M[o], L[o], O[o]);
         }
-        // (the barrier behind the next part's loads stands before its keys are stored over the sums)
     }
 }
 
@@ -435,21 +449,6 @@ __global__ __launch_bounds__(1024) void attn_f32_fold_kernel(AfArgs a, int hs, i
     if (group == 0 && d < hs) a.out[(size_t)tok * a.out_stride + (size_t)head * hs + d] = __fmul_rn(O, L > 0.f ? 1.0f / L : 0.f);
 }
 
-template <int HS, int PAGES>
-static int af_launch_decode(const AfArgs& a, int n_seqs, int heads, hipStream_t s) {
-    // a workgroup a part up to some 8,192 workgroups; a longer table's parts are taken in turn
-    int z = 8192 / (n_seqs * heads);
-    z = z < 1 ? 1 : z > a.n_parts ? a.n_parts : z;
-    const size_t smem = sizeof(float) * (4 * PAGES * 16 * (HS + 4) + PAGES * 4 * 64 * 4 + 16 * (HS + 4) + HS + 2 * PAGES * 16);
-    auto kernel = attn_f32_decode_kernel<HS, PAGES>;
-    if (smem > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        if (e != hipSuccess) return (int)e;
-    }
-    hipLaunchKernelGGL(kernel, dim3(n_seqs, heads, z), dim3(256 * PAGES), smem, s, a);
-    return bn_launch_status();
-}
-
 template <int HS>
 static int af_launch(const AfArgs& a, int n_tiles, hipStream_t s) {
     const int G = a.H / a.Hkv, heads = a.Hkv * ((G + a.GT - 1) / a.GT);
@@ -457,10 +456,16 @@ static int af_launch(const AfArgs& a, int n_tiles, hipStream_t s) {
         hipLaunchKernelGGL(attn_f32_prompt_kernel<HS>, dim3(n_tiles, heads), dim3(256), 0, s, a);
         return bn_launch_status();
     }
-    const int pages = a.part_pages;
-    const int rc = pages == 1 ? af_launch_decode<HS, 1>(a, n_tiles, heads, s) : af_launch_decode<HS, AF_RUN_PAGES>(a, n_tiles, heads, s);
+    // A workgroup a part up to some AF_GROUPS workgroups, of which a CU holds three of heads 128 wide; a longer table's parts are
+    // taken in turn.  us with 8,192 / 2,048 / 768, 16 heads of 128 over 4: 64 sequences of 1,000 keys 67.6 / 62.7 / 54.9, one of
+    // 8,000 beside 63 of 200 192 / 206 / 234, one of 100,000 275 / 278 / 269.
+    int z = AF_GROUPS / (n_tiles * heads);
+    z = z < 1 ? 1 : z > a.n_parts ? a.n_parts : z;
+    if (a.part_pages == 1) hipLaunchKernelGGL((attn_f32_decode_kernel<HS, 1>), dim3(n_tiles, heads, z), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((attn_f32_decode_kernel<HS, AF_RUN_PAGES>), dim3(n_tiles, heads, z), dim3(256), 0, s, a);
+    const int rc = bn_launch_status();
     if (rc || a.n_parts == 1) return rc;
-    const int per_run = AF_RUN_PAGES / pages, runs = (a.n_parts + per_run - 1) / per_run;
+    const int per_run = AF_RUN_PAGES / a.part_pages, runs = (a.n_parts + per_run - 1) / per_run;
     hipLaunchKernelGGL(attn_f32_fold_kernel, dim3(n_tiles * a.H), dim3(128 * (runs < 8 ? runs : 8)), 0, s, a, HS, per_run);
     return bn_launch_status();
 }

@@ -64,3 +64,34 @@ def test_parts_of_a_page_and_of_a_run_give_the_same_bits(H, Hkv, hs):
                                             width, seq_lens.data_ptr(), None, B, H, Hkv, hs, GT, 0.3, 4, po.data_ptr(), pm.data_ptr(),
                                             None, 0, torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and torch.equal(one, run)
+
+
+@pytest.mark.parametrize("H,Hkv,hs", [(4, 2, 16), (3, 1, 32), (2, 2, 64), (8, 2, 128), (20, 1, 64)])
+def test_a_table_much_wider_than_its_sequences(H, Hkv, hs):
+    """Most workgroups find no keys, the others take several parts, and the parts are runs of pages where pages would be too
+    many: the bits, and the stored keys and values, of a table of the sequences' own width."""
+    from bitnet_c_amd import ops
+    from bitnet_c_amd.cache import PAGE
+    torch.manual_seed(H + hs)
+    lens = [1, 64, 65, 0, 256, 257, 4 * PAGE + 63, 1000, 319]
+    B, need = len(lens), -(-max(lens) // PAGE)
+    inv_freq = 1.0 / 10000.0 ** (torch.arange(hs // 2, device=DEV, dtype=torch.float32) * 2 / hs)
+    seq_lens = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    own = torch.randperm(B * need).to(torch.int32).reshape(B, need)
+    pages = [torch.randn(B * need, Hkv, PAGE, hs, device=DEV) for _ in range(2)]
+    qkv = torch.randn(B, (H + 2 * Hkv) * hs, device=DEV)
+    part_pages, results = set(), []
+    runs = (1 << 24) // (B * H * (hs + 2)) + 1                # pages of a table whose pages' sums would take over 64 MB
+    for width in (need, 512, max(runs, 1024)):
+        table = torch.zeros((B, width), dtype=torch.int32)
+        table[:, :need] = own
+        part_pages.add(ops._fn("attn_f32", "bn_attn_f32_part_pages")(B * H, width, hs))
+        kp, vp = (t.clone() for t in pages)
+        out = torch.full((B, H * hs), 7.0, device=DEV)
+        n_splits, chunk = ops.decode_splits(B, H, Hkv, width * PAGE, torch.float32)
+        ops.attention(qkv, out, kp, vp, table.to(DEV), H, Hkv, hs, 0.3, seq_lens=seq_lens, n_splits=n_splits, chunk=chunk,
+                      v_transposed=False, blocked=False, fused_rotate=inv_freq, fused_write=True)
+        results.append((out, kp, vp))
+    assert part_pages == {1, 4}
+    for got in results[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got, results[0]))
