@@ -25,6 +25,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define AF_RUN_PAGES 4
 #define AF_PARTS_BYTES (64ll << 20)
+#define AF_SCRATCH_BYTES (128ll << 20)
 #define AF_GROUPS 2048
 
 struct AfArgs {
@@ -35,8 +36,8 @@ struct AfArgs {
     const int* block_table;   // [n_seqs, bt_stride]
     const int* seq_lens;      // decode form: keys in the cache, the new one included
     const int* tiles;         // prompt form: [n, 4] = sequence, first token row, tokens, position of the first
-    float* part_o;            // [n_tokens * H, n_parts, hs] (n_parts > 1)
-    float* part_ml;           // [n_tokens * H, n_parts, 2]
+    float* part_o;            // [rows at once * H, n_parts, hs] (n_parts > 1)
+    float* part_ml;           // [rows at once * H, n_parts, 2]
     int q_stride, out_stride, bt_stride, H, Hkv;
     int GT;                   // heads of a kv group handled together (a power of two <= 16)
     int n_parts, part_pages;  // decode form: parts that the block table can hold, and a part's pages (1 or AF_RUN_PAGES)
@@ -449,6 +450,20 @@ __global__ __launch_bounds__(1024) void attn_f32_fold_kernel(AfArgs a, int hs, i
     if (group == 0 && d < hs) a.out[(size_t)tok * a.out_stride + (size_t)head * hs + d] = __fmul_rn(O, L > 0.f ? 1.0f / L : 0.f);
 }
 
+// Rows of a decode step that are taken at a time: as many as keep the partial sums (of n_parts parts a row) under
+// AF_SCRATCH_BYTES, in turns of equal size; one row's at the least (with four heads a kv head under a hundredth of the keys and
+// values that the row's table can hold in this layer).  The turns share one buffer, so a step's scratch does not grow with its
+// rows, and a row's sums are the same in any turn.  Tables of 131,072 positions, 32 heads of 128 over 8, 64 / 256 sequences of 200
+// keys: 126 / 516 us and 106 / 122 MB; in turns of 64 MB 235 / 991 us, of 256 MB 84 / 300; 64 rows at once 42 us and 520 MB (the
+// vector kernel, whose parts are runs of 2,048 positions: 157 / 627 us and 65 / 260 MB).
+static int af_rows_at_once(int n_seqs, int H, int n_parts, int hs) {
+    if (n_parts <= 1) return n_seqs;
+    const long long most = AF_SCRATCH_BYTES / ((long long)H * n_parts * (hs + 2) * 4);
+    if (most >= n_seqs) return n_seqs;
+    const int turns = most <= 1 ? n_seqs : (int)((n_seqs + most - 1) / most);
+    return (n_seqs + turns - 1) / turns;
+}
+
 template <int HS>
 static int af_launch(const AfArgs& a, int n_tiles, hipStream_t s) {
     const int G = a.H / a.Hkv, heads = a.Hkv * ((G + a.GT - 1) / a.GT);
@@ -456,18 +471,28 @@ static int af_launch(const AfArgs& a, int n_tiles, hipStream_t s) {
         hipLaunchKernelGGL(attn_f32_prompt_kernel<HS>, dim3(n_tiles, heads), dim3(256), 0, s, a);
         return bn_launch_status();
     }
-    // A workgroup a part up to some AF_GROUPS workgroups, of which a CU holds three of heads 128 wide; a longer table's parts are
-    // taken in turn.  us with 8,192 / 2,048 / 768, 16 heads of 128 over 4: 64 sequences of 1,000 keys 67.6 / 62.7 / 54.9, one of
-    // 8,000 beside 63 of 200 192 / 206 / 234, one of 100,000 275 / 278 / 269.
-    int z = AF_GROUPS / (n_tiles * heads);
-    z = z < 1 ? 1 : z > a.n_parts ? a.n_parts : z;
-    if (a.part_pages == 1) hipLaunchKernelGGL((attn_f32_decode_kernel<HS, 1>), dim3(n_tiles, heads, z), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((attn_f32_decode_kernel<HS, AF_RUN_PAGES>), dim3(n_tiles, heads, z), dim3(256), 0, s, a);
-    const int rc = bn_launch_status();
-    if (rc || a.n_parts == 1) return rc;
+    const int at_once = af_rows_at_once(n_tiles, a.H, a.n_parts, HS);
     const int per_run = AF_RUN_PAGES / a.part_pages, runs = (a.n_parts + per_run - 1) / per_run;
-    hipLaunchKernelGGL(attn_f32_fold_kernel, dim3(n_tiles * a.H), dim3(128 * (runs < 8 ? runs : 8)), 0, s, a, HS, per_run);
-    return bn_launch_status();
+    for (int first = 0; first < n_tiles; first += at_once) {
+        const int n = n_tiles - first < at_once ? n_tiles - first : at_once;
+        AfArgs t = a;
+        t.q += (size_t)first * a.q_stride;
+        t.out += (size_t)first * a.out_stride;
+        t.block_table += (size_t)first * a.bt_stride;
+        t.seq_lens += first;
+        // A workgroup a part up to some AF_GROUPS workgroups, of which a CU holds three of heads 128 wide; a longer table's parts
+        // are taken in turn.  us with 8,192 / 2,048 / 768, 16 heads of 128 over 4: 64 sequences of 1,000 keys 67.6 / 62.7 / 54.9,
+        // one of 8,000 beside 63 of 200 192 / 206 / 234, one of 100,000 275 / 278 / 269.
+        int z = AF_GROUPS / (n * heads);
+        z = z < 1 ? 1 : z > a.n_parts ? a.n_parts : z;
+        if (a.part_pages == 1) hipLaunchKernelGGL((attn_f32_decode_kernel<HS, 1>), dim3(n, heads, z), dim3(256), 0, s, t);
+        else hipLaunchKernelGGL((attn_f32_decode_kernel<HS, AF_RUN_PAGES>), dim3(n, heads, z), dim3(256), 0, s, t);
+        if (int rc = bn_launch_status()) return rc;
+        if (a.n_parts == 1) continue;
+        hipLaunchKernelGGL(attn_f32_fold_kernel, dim3(n * a.H), dim3(128 * (runs < 8 ? runs : 8)), 0, s, t, HS, per_run);
+        if (int rc = bn_launch_status()) return rc;
+    }
+    return 0;
 }
 
 extern "C" int bn_attn_f32_supports(int hs) { return hs == 16 || hs == 32 || hs == 64 || hs == 128; }
@@ -478,8 +503,12 @@ extern "C" int bn_attn_f32_part_pages(long long rows, int bt_stride, int hs) {
     return rows * bt_stride * (hs + 2) * 4 <= AF_PARTS_BYTES ? 1 : AF_RUN_PAGES;
 }
 
+// Rows whose partial sums, of n_parts parts each, the caller gives room for.
+extern "C" int bn_attn_f32_rows(int n_seqs, int H, int n_parts, int hs) { return af_rows_at_once(n_seqs, H, n_parts, hs); }
+
 // tiles: the prompt form, tiles of up to 64 / GT tokens; null: the decode form, n_tiles sequences in parts of
-// part_pages pages (1 or a run's), with partial sums of ceil(bt_stride / part_pages) parts a row if that is more than one.  Decode form only: inv_freq
+// part_pages pages (1 or a run's), with partial sums of ceil(bt_stride / part_pages) parts a row if that is more than one, for
+// bn_attn_f32_rows rows.  Decode form only: inv_freq
 // [hs / 2], not null: q and the new key arrive unrotated; write: a row of q is [H + 2 Hkv heads], its new key and value are stored
 // into the pages at position seq_lens - 1 (a row of no keys stores nothing).
 extern "C" int bn_attn_f32(const void* q, int q_stride, void* out, int out_stride, const void* k_pages, const void* v_pages,

@@ -167,6 +167,7 @@ _SIGNATURES = {
     "attn_f32": {
         "bn_attn_f32_supports": [c_int],
         "bn_attn_f32_part_pages": [c_longlong, c_int, c_int],
+        "bn_attn_f32_rows": [c_int, c_int, c_int, c_int],
         "bn_attn_f32": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int,
                         c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     },
@@ -1477,13 +1478,14 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
                               f"{block_table.shape[1]} pages of the block table")
         if n_splits > (1024 if fold else 64):
             raise KernelError("attention: at most 64 splits (1,024 runs of a float32 cache)")
-    parts = n_splits
+    parts, rows = n_splits, T
     if f32_plain:                     # however the caller cuts them, the keys are summed page by page and run by run
         part_pages = _fn("attn_f32", "bn_attn_f32_part_pages")(T * H, block_table.shape[1], hs)
         parts = -(-block_table.shape[1] // part_pages) if decode else 1
+        rows = _fn("attn_f32", "bn_attn_f32_rows")(T, H, parts, hs)            # the kernels take a large step's rows in turns
     if parts > 1:
-        part_o = torch.empty((T * H * parts, vd), dtype=torch.float32, device=qkv.device)
-        part_ml = torch.empty((T * H * parts, 2), dtype=torch.float32, device=qkv.device)
+        part_o = torch.empty((rows * H * parts, vd), dtype=torch.float32, device=qkv.device)
+        part_ml = torch.empty((rows * H * parts, 2), dtype=torch.float32, device=qkv.device)
     po = part_o.data_ptr() if part_o is not None else None
     pm = part_ml.data_ptr() if part_ml is not None else None
     sl = seq_lens.data_ptr() if decode else None

@@ -95,3 +95,35 @@ def test_a_table_much_wider_than_its_sequences(H, Hkv, hs):
     assert part_pages == {1, 4}
     for got in results[1:]:
         assert all(torch.equal(a, b) for a, b in zip(got, results[0]))
+
+
+@pytest.mark.parametrize("H,Hkv,hs", [(8, 2, 128), (20, 1, 64)])
+@pytest.mark.parametrize("B", [9, 7])
+def test_the_scratch_of_a_step_is_bounded(H, Hkv, hs, B):
+    """Rows whose partial sums would take more than 128 MB are taken in turns over one buffer, to the same bits."""
+    from bitnet_c_amd import ops
+    from bitnet_c_amd.cache import PAGE
+    torch.manual_seed(B)
+    limit = 128 << 20
+    width = 4 * (limit // (4 * 9 * H * (hs + 2))) * 2 + 3      # nine rows' runs take over twice the limit
+    lens = [300, 1, 0, 65, 256, 257, 700, 64, 2][:B]
+    need = -(-max(lens) // PAGE)
+    table = torch.zeros((B, width), dtype=torch.int32)
+    table[:, :need] = torch.randperm(B * need).to(torch.int32).reshape(B, need)
+    kp, vp = (torch.randn(B * need, Hkv, PAGE, hs, device=DEV) for _ in range(2))
+    qkv = torch.randn(B, (H + 2 * Hkv) * hs, device=DEV)
+    seq_lens = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    results = []
+    for t in (table[:, :need].contiguous().to(DEV), table.to(DEV)):
+        a, b = kp.clone(), vp.clone()
+        out = torch.full((B, H * hs), 7.0, device=DEV)
+        n_splits, chunk = ops.decode_splits(B, H, Hkv, t.shape[1] * PAGE, torch.float32)
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        ops.attention(qkv, out, a, b, t, H, Hkv, hs, 0.3, seq_lens=seq_lens, n_splits=n_splits, chunk=chunk, v_transposed=False,
+                      blocked=False, fused_write=True)
+        assert torch.cuda.max_memory_allocated() - before <= limit + (1 << 16)
+        results.append((out, a, b))
+    assert all(torch.equal(x, y) for x, y in zip(*results))
