@@ -76,7 +76,7 @@ template <int HS> struct AfSums {                 // a lane's sums of its row (r
             for (int i = 0; i < AfShape<HS>::VW; ++i) o[h][i] = 0.f;
     }
     __device__ __forceinline__ void fold(const AfSums& p) {
-        if (p.m == -INFINITY) return;             // a part of which this row saw no key changes nothing
+        if (p.l == 0.f) return;                   // a part of which this row saw no key changes nothing (one whose scores are all NaN does)
         float m2, fa, fb;
         af_factors(m, p.m, m2, fa, fb);
         l = af_fold(l, fa, p.l, fb);
@@ -371,11 +371,11 @@ __global__ __launch_bounds__(256, PAGES == 1 ? 3 : 2) void attn_f32_decode_kerne
                 for (int o = 0; o < OWN; ++o) {
                     const int idx = tid + 256 * o, h = idx / HS, d = idx - h * HS;
                     if (h >= rows) break;
-                    const float m = sm[h];
-                    if (m == -INFINITY) continue;
+                    const float m = sm[h], l = sl[h];
+                    if (l == 0.f) continue;
                     float m2, fa, fb;
                     af_factors(M[o], m, m2, fa, fb);
-                    L[o] = af_fold(L[o], fa, sl[h], fb);
+                    L[o] = af_fold(L[o], fa, l, fb);
                     O[o] = af_fold(O[o], fa, so[h * (HS + 1) + d], fb);
                     M[o] = m2;
                 }
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(1024) void attn_f32_fold_kernel(AfArgs a, int hs, i
             }
 #pragma unroll
             for (int i = 0; i < AF_RUN_PAGES; ++i) {
-                if (i >= per_run || first + i >= parts || m[i] == -INFINITY) continue;
+                if (i >= per_run || first + i >= parts || l[i] == 0.f) continue;
                 float m2, fa, fb;
                 af_factors(RM, m[i], m2, fa, fb);
                 RL = af_fold(RL, fa, l[i], fb);
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(1024) void attn_f32_fold_kernel(AfArgs a, int hs, i
         }
         __syncthreads();
         for (int i = 0; i < min(groups, runs - r0); ++i) {
-            if (rm[i] == -INFINITY) continue;
+            if (rl[i] == 0.f) continue;
             float m2, fa, fb;
             af_factors(M, rm[i], m2, fa, fb);
             L = af_fold(L, fa, rl[i], fb);

@@ -103,3 +103,39 @@ def test_a_key_far_above_the_others_and_rows_before_it():
     exact = _exact(q[0], keys[0], values[0], H, Hkv, hs, hs ** -0.5, 0)
     # scores up to 40 |q|^2 / 8: some 400, whose rounding (2^-24 of it, times the chain) moves a weight by some 1e-3
     assert float((out.cpu().double() - exact).abs().max()) <= 400 * 2.0 ** -24 * (hs + 4) * 4
+
+
+@pytest.mark.parametrize("hs", [16, 128])
+def test_keys_that_are_not_numbers(hs):
+    """A page of keys (and a run of pages) of nothing but NaN gives NaN to every row that sees it, as one such key among others
+    does, and so does a query of NaN: no page is passed over for it."""
+    from bitnet_c_amd import ops
+    H, Hkv, n = 4, 2, 700
+    kp, vp, bt, _, _, q = _setup(H, Hkv, hs, [n], 3)
+    q = q[0].cuda()
+    q[50, :hs] = float("nan")
+    q[699, hs:2 * hs] = float("nan")
+    for first, last in ((64, 127), (256, 511), (130, 130)):
+        k = kp.clone()
+        for p in range(first // PAGE, last // PAGE + 1):
+            lo, hi = max(first - p * PAGE, 0), min(last - p * PAGE, PAGE - 1)
+            k[int(bt[0, p]), 1, lo:hi + 1] = float("nan")
+        want = torch.zeros(n, H, dtype=torch.bool)
+        want[50, 0] = want[699, 1] = True
+        want[first:, 2:] = True
+        for plain in (True, False):
+            _, _, qt = ops.attention_row_shape(H, Hkv, False, torch.float32, hs, plain)
+            tiles = torch.tensor([(0, i, min(qt, n - i), i) for i in range(0, n, qt)], dtype=torch.int32).cuda()
+            out = torch.zeros(n, H * hs).cuda()
+            ops.attention(q, out, k, vp, bt, H, Hkv, hs, hs ** -0.5, tiles=tiles, qt=qt)
+            assert torch.equal(out.view(n, H, hs).isnan().cpu(), want[:, :, None].expand(n, H, hs))
+        rows = [50, 63, 127, 128, 129, 255, 511, 600, 699]
+        sl = torch.tensor([r + 1 for r in rows] + [0], dtype=torch.int32).cuda()
+        for width in (bt.shape[1], 2 ** 24 // (10 * H * (hs + 2)) + 1):                  # parts of a page, and of a run of pages
+            table = torch.zeros((len(sl), width), dtype=torch.int32).cuda()
+            table[:, :bt.shape[1]] = bt
+            n_splits, chunk = ops.decode_splits(len(sl), H, Hkv, width * PAGE, torch.float32)
+            got = torch.zeros(len(sl), H * hs).cuda()
+            ops.attention(torch.cat([q[rows], q[50:51]]), got, k, vp, table, H, Hkv, hs, hs ** -0.5, seq_lens=sl, n_splits=n_splits, chunk=chunk)
+            assert torch.equal(got[:-1].view(-1, H, hs).isnan().cpu(), want[rows][:, :, None].expand(len(rows), H, hs))
+            assert float(got[-1].abs().max()) == 0.0
