@@ -458,6 +458,17 @@ static int lc_launch(const LaArgs& a, int n_seqs, hipStream_t s) {
     return bn_launch_status();
 }
 
+// Value columns of a workgroup of the chunked form, the same bits either way.  A chunk of 64 tokens takes a workgroup 8.2 us with
+// 16 columns, 10.6 with 32 and 20 with 64 (keys 128 wide; a CU holds one workgroup), so the form whose rounds over the CUs take less:
+// four prompts of 500 tokens, 16 heads of 128 values 111 us with 32, 153 with 16 and 187 with 64; eight of 256 tokens, 64 heads of 16
+// values (which 32 columns do not save a workgroup) 126 with 16 and 146 with 32.  Keys up to 64 wide leave room for several
+// workgroups a CU: 16 (58 us against 73).
+extern "C" int bn_lightning_columns(int n_seqs, int H, int dk, int dv) {
+    if (dk <= 64) return 16;
+    auto rounds = [&](int cols) { return ((long long)n_seqs * H * ((dv + cols - 1) / cols) + la_compute_units() - 1) / la_compute_units(); };
+    return rounds(16) * 82 > rounds(32) * 106 ? 32 : 16;
+}
+
 static int lc_dispatch(int dtype, LaArgs& a, int n_seqs, int n_rows, const int* positions, float* prepared, hipStream_t s) {
     LcPrepArgs p;
     p.feed = a.feed; p.positions = positions;
@@ -469,13 +480,8 @@ static int lc_dispatch(int dtype, LaArgs& a, int n_seqs, int n_rows, const int* 
     const int rc = bn_launch_status();
     if (rc != 0) return rc;
     a.pq = p.q; a.pk = p.k; a.pv = p.v; a.T = n_rows; a.dks = p.dks; a.dvs = p.dvs;
-    // Value columns of a workgroup.  A chunk of 64 tokens takes a workgroup 8.2 us with 16 columns, 10.6 with 32 and 20 with 64 (keys
-    // 128 wide; a CU holds one workgroup): 16 while every workgroup has a CU, 32 from there on (four prompts of 500 tokens, 16
-    // heads of 128: 111 us, 153 with 16 and 187 with 64; eight of 256: 114, 153, 112).  Keys up to 64 wide leave room
-    // for several workgroups a CU: 16 (58 us against 73).
     if (a.dk <= 64) return lc_launch<1, 1>(a, n_seqs, s);
-    const bool wide = (long long)n_seqs * a.H * ((a.dv + 15) / 16) > la_compute_units();
-    return wide ? lc_launch<2, 2>(a, n_seqs, s) : lc_launch<2, 1>(a, n_seqs, s);
+    return bn_lightning_columns(n_seqs, a.H, a.dk, a.dv) == 32 ? lc_launch<2, 2>(a, n_seqs, s) : lc_launch<2, 1>(a, n_seqs, s);
 }
 
 extern "C" int bn_lightning_supports(int dk, int dv) { return (dk >= 1 && dk <= LA_MAX_DIM && dv >= 1) ? 1 : 0; }

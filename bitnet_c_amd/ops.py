@@ -119,6 +119,7 @@ _SIGNATURES = {
         "bn_lightning_supports": [c_int, c_int],
         "bn_lightning_chunked": [c_int, c_int],
         "bn_lightning_prefers_chunks": [c_int, c_int, c_int, c_int],
+        "bn_lightning_columns": [c_int, c_int, c_int, c_int],
         "bn_lightning_scan": [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p,
                               c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p,
                               c_float, c_void_p],

@@ -29,3 +29,13 @@ def test_many_sequences_and_one_at_a_time(H, dk, dv, lens):
         rows = slice(t[1], t[1] + t[2])
         assert torch.equal(scan(alone, [t])[rows], together[rows])
     assert torch.isfinite(together).all() and torch.equal(state, alone)
+
+
+def test_which_launches_take_32_columns():
+    """Those whose rounds over the 256 CUs are then the shorter ones; never where 32 columns save no workgroup."""
+    from bitnet_c_amd import ops
+    columns = ops._fn("lightning", "bn_lightning_columns")
+    assert columns(4, 16, 128, 128) == 32 and columns(1, 32, 128, 128) == 16 and columns(2, 32, 128, 128) == 32
+    assert columns(2, 16, 128, 128) == 16 and columns(5, 40, 72, 24) == 32 and columns(2, 65, 128, 48) == 16
+    assert all(columns(n, h, 128, dv) == 16 for n in (1, 8, 31) for h in (16, 64) for dv in (1, 16))
+    assert columns(31, 64, 64, 128) == 16
