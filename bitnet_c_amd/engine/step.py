@@ -122,6 +122,13 @@ def _query_tiles(n_new, pos0, qt: int) -> List[tuple]:
     return ops.pair_tiles(rows)
 
 
+def _most_tiles(rows: int, seqs: int, qt: int) -> int:
+    """Tiles of up to qt rows that `rows` new tokens of `seqs` sequences can need: every sequence may end in a tile that is not
+    full, and all tokens but a sequence's first may fill others (one tile a sequence where qt holds them all: a list that ended in
+    a spare one would have kernels launch, and choose their form by, a sequence that is never there)."""
+    return seqs + (rows - 1) // qt
+
+
 def _by_length(lens) -> List[int]:
     """The rows ordered by length, longest first (ties by row)."""
     return sorted(range(len(lens)), key=lambda i: (-lens[i], i))
@@ -258,7 +265,7 @@ class _PromptGraph:
         self.rows, self.seqs, self.wants, self.width = rows, seqs, wants, engine.max_pages
         dev, cache = engine.device, engine.cache
         n_groups = len(cache.groups)
-        self.n_tiles = {qt: -(-rows // qt) + seqs for qt in qts}         # every sequence may end in a tile that is not full
+        self.n_tiles = {qt: _most_tiles(rows, seqs, qt) for qt in qts}
         self.n_page_tiles = -(-rows // PAGE) + 2 * seqs if page_tiles else 0
         sizes = [rows, rows, rows, seqs, wants, seqs] + [4 * self.n_tiles[qt] for qt in qts] + [4 * self.n_page_tiles]
         self.offsets = [0]

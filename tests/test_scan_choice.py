@@ -1,5 +1,5 @@
 """Which prompt steps cut their recurrences into pieces: a choice that the eager step of a request and the captured step that
-replays it make alike."""
+replays it make alike; and the lengths of a captured step's lists of tiles."""
 import random
 
 import torch
@@ -35,3 +35,16 @@ def test_which_steps_are_cut():
     assert gru((256, 1), 2048) and gru((1024, 4), 2048) and gru((4096, 8), 2048) and not gru((2048, 8), 2048) and not gru((192, 1), 64)
     assert not wkv((2048, 1), 32, dtype=torch.float32) and not gru((2048, 1), 2048, torch.float32)
     assert not wkv((1 << 24, 1), 32)                              # scratch beyond its bound
+
+
+def test_a_captured_step_has_room_for_every_list_of_tiles():
+    from bitnet_c_amd import ops
+    from bitnet_c_amd.engine.step import _bucket, _most_tiles, _query_tiles, _row_bucket
+    rng = random.Random(6)
+    shapes = [[n] for n in (1, 2, 15, 16, 17, 63, 64, 65, 256, 8192)] + [[1] * 256, [1] * 12 + [4], [17] * 15 + [1], [65, 1, 63], [64] * 8]
+    shapes += [[rng.randint(1, 300) for _ in range(rng.randint(1, 20))] for _ in range(200)]
+    for n_new in shapes:
+        rows, seqs = _row_bucket(sum(n_new)), _bucket(len(n_new))
+        for qt in (1, 4, 16, 32, 48, 64, 128, ops.SEQUENCE_TILE):
+            assert len(_query_tiles(n_new, [5] * len(n_new), qt)) <= _most_tiles(rows, seqs, qt)
+        assert _most_tiles(rows, seqs, ops.SEQUENCE_TILE) == seqs            # no tile that no sequence can have
