@@ -763,12 +763,12 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ x, const TD* __res
     for (int i = threadIdx.x; i < dim; i += blockDim.x) o[i] = from_f32<T>(row[i] * f * w[i]);
 }
 
-// dtype: the type of out (and of delta when parts_f32 is 0); parts_f32: delta is n_parts float32 slabs [n_parts][n_rows][dim]
 // The same with the row in registers, eight numbers a thread and group (dim a multiple of 8, at most G groups a thread, everything
 // 16-byte aligned): everything that does not depend on a sum is asked for at once, so a decode step's row costs one trip to memory and
 // two sums over the workgroup.  dim 2,048, four rows: 4.5 us (5.9
 // with a number a thread and the row in shared memory between the passes).
-template <typename T> struct __align__(sizeof(T) * 8) Eight { T e[8]; };
+template <typename T> struct __align__(16) Eight { T e[8]; };        // no more than the launcher looks at
+static_assert(alignof(Eight<float>) == 16 && alignof(Eight<bf16>) == 16 && sizeof(Eight<float>) == 32, "two 16-byte accesses, or one");
 
 template <typename T, typename TD, int G>
 __global__ __launch_bounds__(256) void add_normed_rmsnorm_wide_kernel(float* __restrict__ x, const TD* __restrict__ delta, int n_parts,
@@ -847,6 +847,7 @@ static bool launch_add_normed_wide(float* x, const TD* delta, int n_parts, const
     return true;
 }
 
+// dtype: the type of out (and of delta when parts_f32 is 0); parts_f32: delta is n_parts float32 slabs [n_parts][n_rows][dim]
 extern "C" int bn_add_normed_rmsnorm(int dtype, void* x, const void* delta, int n_parts, int parts_f32, const float* wb,
                                      float eps_b, const float* w, void* out, int n_rows, int dim, float eps, hipStream_t s) {
     if (n_rows <= 0 || dim <= 0 || dim > 16384 || n_parts < 1 || !x || !delta || !wb || (w && !out))

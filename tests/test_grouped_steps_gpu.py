@@ -147,3 +147,27 @@ def test_row_norm_gate_widths(dtype, W):
     got = ops.row_norm_gate(o, gate, weight, 1e-6)
     tol = (2.0 ** -8 if dtype == torch.bfloat16 else 0.0) + 2.0 ** -24 * (W ** 0.5 + 16)
     assert float((got.double() - want).abs().max()) <= tol * float(want.abs().max())
+
+
+@pytest.mark.parametrize("shift", [4, 1])
+def test_add_normed_rmsnorm_at_any_address(shift):
+    """Rows and weights at addresses that are multiples of 16 and not of 32 bytes, and of 4 (which the wide kernel leaves to the
+    other): what rows at the start of an allocation give."""
+    from bitnet_c_amd import ops
+    T, dim = 3, 2048
+
+    def moved(t):
+        buf = torch.empty(t.numel() + 8, dtype=t.dtype, device="cuda")
+        v = buf[shift:shift + t.numel()].view(t.shape)
+        v.copy_(t)
+        assert v.data_ptr() % 32 == shift * t.element_size() % 32
+        return v
+
+    x, wb, w, delta = _rand((T, dim), 1), _rand((dim,), 2), _rand((dim,), 3), _rand((T, dim), 4)
+    a, b = x.clone(), moved(x)
+    out = ops.add_normed_rmsnorm(a, delta, wb, 1e-6, weight=w, eps=1e-5, out_dtype=torch.float32)
+    got = ops.add_normed_rmsnorm(b, moved(delta), moved(wb), 1e-6, weight=moved(w), eps=1e-5, out_dtype=torch.float32)
+    if shift == 4:
+        assert torch.equal(a, b) and torch.equal(out, got)
+    tol = 2.0 ** -24 * (dim ** 0.5 + 16)
+    assert float((a - b).abs().max()) <= 2 * tol * float(a.abs().max()) and float((out - got).abs().max()) <= 2 * tol * float(out.abs().max())
