@@ -11,8 +11,8 @@
 //
 // gemm_f32_stream_kernel, up to 64 rows: bound by the bytes of W.  A workgroup of 8 waves owns up to 16 columns and all of
 // K; a wave takes every eighth chunk, asks for its whole 8 KB of W (and the rows' 128 columns of A) at once and leaves
-// 16 x 16 sums in shared memory; then a thread an output adds them up in order.  us at one row, cold weights, and at 6.5
-// TB/s: 11,264 x 2,048 22 (14), 2,048 x 5,632 20 (7), 32,000 x 2,048 53 (40), 28,672 x 4,096 96 (72); the vector kernel that
+// 16 x 16 sums in shared memory; then a thread an output adds them up in order.  us at one row, 1.5 GB of weights in turn, and at
+// 6.5 TB/s: 11,264 x 2,048 24 (14), 2,048 x 5,632 19.5 (7), 32,000 x 2,048 52 (40), 28,672 x 4,096 103 (72); the vector kernel that
 // walked K in one chain (gemm_tiled.hip) took 325 on the average of a layer's products, whatever the rows up to 16.
 // gemm_f32_tile_kernel, more rows: bound by the instruction (157 TFLOP/s on this chip, 32 cycles each on a SIMD).  5,136 x
 // 11,264 x 2,048 2.02 ms (117 TFLOP/s), 2,048 x 2,048 x 5,632 0.40 ms; the matrix unit is busy four fifths of a round, the
@@ -274,9 +274,9 @@ static int gf_launch_tile(const GfArgs& a, hipStream_t s) {
 
 #define GF_CUS 256
 
-// Columns a workgroup of the streaming kernel owns: 16, or fewer where the busiest CU then has at least an eighth fewer
-// (us at one row: 3,072 x 2,048 in 16 / 12 9.8 / 9.3, 6,144 x 4,096 28.2 / 24.4, 2,048 x 5,632 in 16 / 8 18.6 / 17.1; where
-// the even split gains nothing fewer columns only read the rows more often: 11,264 x 2,048 in 16 / 12 22.6 / 24.5).
+// Columns a workgroup of the streaming kernel owns: 16, or fewer where the busiest CU then has at least an eighth fewer.  us at one
+// row, 1.5 GB of weights in turn: 2,048 x 5,632 in 16 / 8 20.2 / 19.5, 6,144 x 4,096 in 16 / 12 25.0 / 24.6, 3,072 x 2,048 8.8 / 8.9;
+// where the even split gains nothing fewer columns only read the rows more often: 32,000 x 2,048 in 16 / 12 51 / 60.
 static int gf_stream_cols(int N) {
     int best = 16, cost = 1 << 30;
     for (int c : {16, 12, 8}) {
