@@ -646,33 +646,40 @@ __global__ void rmsnorm_mean_kernel(T* __restrict__ out, const T* __restrict__ a
     }
 }
 
-// The same in 16-byte groups, the rows kept in registers between the passes (dim a multiple of the group, at most G groups a
-// thread, everything 16-byte aligned).  Bound by the bytes: 2,048 rows of 2,048, two bf16 branches, 25 MB: some 20 us
-// (some 125 with 2-byte accesses in two passes over memory).
+// The same with the rows in registers, eight numbers a thread and group (dim a multiple of 8, at most G groups a thread, everything
+// 16-byte aligned), weights and rows asked for together: weights asked for a number a lane at a time, 32 bytes from lane to lane,
+// cost the address unit more than the rows.  us, two bf16 branches 2,048 wide, 1 / 1,100 / 4,000 rows: 2.9 / 4.6 / 11.0 (so asked 4.3 /
+// 12.0 / 34.7; the kernel above 5.3 / 7.7 / 20).
+template <typename T> struct __align__(16) Eight { T e[8]; };        // no more than the launchers look at
+static_assert(alignof(Eight<float>) == 16 && alignof(Eight<bf16>) == 16 && sizeof(Eight<float>) == 32, "two 16-byte accesses, or one");
+
 template <typename T, int G>
 __global__ __launch_bounds__(256) void rmsnorm_mean_wide_kernel(T* __restrict__ out, const T* __restrict__ a, const T* __restrict__ b,
                                                                 const float* __restrict__ wa, const float* __restrict__ wb, int dim, float eps) {
-    constexpr int EPV = 16 / (int)sizeof(T);
-    struct __align__(16) Group { T e[EPV]; };
     __shared__ float scratch[16];
-    const size_t r = blockIdx.x;
-    const int groups = dim / EPV;
-    Group ga[G], gb[G];
+    const size_t row = (size_t)blockIdx.x * dim;
+    const int groups = dim / 8;
+    Eight<T> ga[G], gb[G];
+    Eight<float> va[G], vb[G];
     float sa = 0.f, sb = 0.f;
 #pragma unroll
     for (int q = 0; q < G; ++q) {
-        const int at = min((int)threadIdx.x + 256 * q, groups - 1) * EPV;
-        ga[q] = *reinterpret_cast<const Group*>(a + r * dim + at);
-        if (b) gb[q] = *reinterpret_cast<const Group*>(b + r * dim + at);
+        const int at = min((int)threadIdx.x + 256 * q, groups - 1) * 8;
+        ga[q] = *reinterpret_cast<const Eight<T>*>(a + row + at);
+        va[q] = *reinterpret_cast<const Eight<float>*>(wa + at);
+        if (b) {
+            gb[q] = *reinterpret_cast<const Eight<T>*>(b + row + at);
+            vb[q] = *reinterpret_cast<const Eight<float>*>(wb + at);
+        }
     }
 #pragma unroll
     for (int q = 0; q < G; ++q) {
         if ((int)threadIdx.x + 256 * q >= groups) continue;
 #pragma unroll
-        for (int e = 0; e < EPV; ++e) {
-            const float va = to_f32(ga[q].e[e]), vb = b ? to_f32(gb[q].e[e]) : 0.f;
-            sa = fmaf(va, va, sa);
-            sb = fmaf(vb, vb, sb);
+        for (int e = 0; e < 8; ++e) {
+            const float x = to_f32(ga[q].e[e]), y = b ? to_f32(gb[q].e[e]) : 0.f;
+            sa = fmaf(x, x, sa);
+            sb = fmaf(y, y, sb);
         }
     }
     sa = block_sum(sa, scratch);
@@ -680,24 +687,24 @@ __global__ __launch_bounds__(256) void rmsnorm_mean_wide_kernel(T* __restrict__ 
     const float fa = 1.0f / sqrtf(sa / (float)dim + eps), fb = 1.0f / sqrtf(sb / (float)dim + eps), share = b ? 0.5f : 1.0f;
 #pragma unroll
     for (int q = 0; q < G; ++q) {
-        const int at = ((int)threadIdx.x + 256 * q) * EPV;
+        const int at = ((int)threadIdx.x + 256 * q) * 8;
         if (at >= dim) continue;
-        Group o;
+        Eight<T> o;
 #pragma unroll
-        for (int e = 0; e < EPV; ++e) {
-            float v = to_f32(ga[q].e[e]) * fa * wa[at + e];
-            if (b) v += to_f32(gb[q].e[e]) * fb * wb[at + e];
+        for (int e = 0; e < 8; ++e) {
+            float v = to_f32(ga[q].e[e]) * fa * va[q].e[e];
+            if (b) v += to_f32(gb[q].e[e]) * fb * vb[q].e[e];
             o.e[e] = from_f32<T>(v * share);
         }
-        *reinterpret_cast<Group*>(out + r * dim + at) = o;
+        *reinterpret_cast<Eight<T>*>(out + row + at) = o;
     }
 }
 
 template <typename T>
 static bool launch_rmsnorm_mean_wide(T* out, const T* a, const T* b, const float* wa, const float* wb, int n_rows, int dim, float eps,
                                      hipStream_t s) {
-    const int epv = 16 / (int)sizeof(T), per = (dim / epv + 255) / 256;
-    if (dim % epv || per > 4 || (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b) & 15)) return false;
+    const int per = (dim / 8 + 255) / 256;
+    if (dim % 8 || per > 4 || (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b | (uintptr_t)wa | (uintptr_t)wb) & 15)) return false;
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(n_rows), dim3(256), 0, s, out, a, b, wa, wb, dim, eps); };
     if (per == 1) go(rmsnorm_mean_wide_kernel<T, 1>);
     else if (per == 2) go(rmsnorm_mean_wide_kernel<T, 2>);
@@ -767,9 +774,6 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ x, const TD* __res
 // 16-byte aligned): everything that does not depend on a sum is asked for at once, so a decode step's row costs one trip to memory and
 // two sums over the workgroup.  dim 2,048, four rows: 4.5 us (5.9
 // with a number a thread and the row in shared memory between the passes).
-template <typename T> struct __align__(16) Eight { T e[8]; };        // no more than the launcher looks at
-static_assert(alignof(Eight<float>) == 16 && alignof(Eight<bf16>) == 16 && sizeof(Eight<float>) == 32, "two 16-byte accesses, or one");
-
 template <typename T, typename TD, int G>
 __global__ __launch_bounds__(256) void add_normed_rmsnorm_wide_kernel(float* __restrict__ x, const TD* __restrict__ delta, int n_parts,
                                                                       size_t part_stride, const float* __restrict__ wb, float eps_b,

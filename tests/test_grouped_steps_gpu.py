@@ -107,6 +107,22 @@ def test_rmsnorm_mean(dtype, dim, two):
     assert float((got.double() - want).abs().max()) <= tol * float(want.abs().max())
 
 
+@pytest.mark.parametrize("shift", [4, 1])
+def test_rmsnorm_mean_weights_at_any_address(shift):
+    """Weights at addresses that are multiples of 16 bytes (the wide kernel's) and of 4 (the other's)."""
+    from bitnet_c_amd import ops
+    dim = 2048
+    a, b, wa, wb = _rand((3, dim), 1), _rand((3, dim), 2), _rand((dim,), 3), _rand((dim,), 4)
+    want = ops.rmsnorm_mean(a, wa, b, wb, 1e-5)
+    moved = []
+    for w in (wa, wb):
+        v = torch.empty(dim + 8, device="cuda")[shift:shift + dim]
+        moved.append(v.copy_(w))
+    got = ops.rmsnorm_mean(a, moved[0], b, moved[1], 1e-5)
+    assert torch.equal(got, want) or shift == 1
+    assert float((got - want).abs().max()) <= 2.0 ** -23 * (dim ** 0.5 + 8) * float(want.abs().max())
+
+
 # widths: one group of eight, a workgroup's 256 groups and one past them, the most that registers hold (8,192) and beyond, not a
 # multiple of eight
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
