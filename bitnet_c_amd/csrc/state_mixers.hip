@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void token_shift_stream_kernel(TO* __restrict_
 }
 
 // The mixes of a bf16 or float32 input in 16-byte groups of h (D a multiple of 8, everything 16-byte aligned); the state is read
-// only.  Four rows a workgroup in long steps, so that a mix's weights are read once for them.  2,048
+// only.  Four rows a workgroup in large steps, so that a mix's weights are read once for them.  2,048
 // rows x 2,048 columns, five bf16 mixes: 50 MB, 12.7 us (285 with an element a thread and 2-byte stores); one row 3.3 us in a graph of such
 // launches (4.4), 6.3 in a decode step's profile.
 template <typename T, int TS_ROWS>
@@ -185,7 +185,10 @@ template <typename T>
 static void launch_token_shift_wide(T* out, const T* h, const float* mu, const float* state, size_t st, const int* positions,
                                     const int* seq_index, const int* slot_ids, int n_tokens, int D, int n_mix, hipStream_t s) {
     const unsigned y = (unsigned)(D * (int)sizeof(T) / 16 + 255) / 256;
-    if (n_tokens >= 1024)                                         // four workgroups of one row a CU: the rows' weights count
+    // Four rows of a workgroup share a mix's weights, which pays once the rows no longer fit what is on its way at a time: us with four /
+    // one, bf16, 1,024 x 1,024 6.9 / 5.6, 1,500 x 2,048 11.4 / 11.0, 4,000 x 768 11.1 / 12.4, 2,048 x 2,048 12.7 / 13.2, 4,000 x 4,096 36 /
+    // 38; float32 1,024 x 1,024 7.1 / 6.4, 1,024 x 2,048 11.5 / 12.1.
+    if ((long long)n_tokens * D * (int)sizeof(T) >= 6000000)
         hipLaunchKernelGGL((token_shift_wide_kernel<T, 4>), dim3((n_tokens + 3) / 4, y), dim3(256), 0, s, out, h, mu, state, st, positions,
                            seq_index, slot_ids, n_tokens, D, n_mix);
     else
@@ -202,7 +205,9 @@ extern "C" int bn_token_shift(int in_dtype, int dtype, void* out, const void* h,
     if ((dtype != BN_DT_F32 && dtype != BN_DT_BF16) || (in_dtype != dtype && in_dtype != BN_DT_F32)) return BN_ERR_DTYPE;
     const dim3 grid(n_tokens), block(256);
     const size_t st = (size_t)state_stride;
-    if (in_dtype == dtype && !seq_lens && D % 8 == 0 && st % 4 == 0 &&
+    // (narrower rows leave most threads of a workgroup of groups idle: us at 64 rows in bf16, wide / not, 256 columns 3.1 / 2.7, 512
+    // 3.1 / 3.4; at 1,100 rows of 64 6.6 / 3.1)
+    if (in_dtype == dtype && !seq_lens && D >= 512 && D % 8 == 0 && st % 4 == 0 &&
         !(((uintptr_t)out | (uintptr_t)h | (uintptr_t)mu | (uintptr_t)state) & 15)) {
         if (dtype == BN_DT_F32)
             launch_token_shift_wide((float*)out, (const float*)h, mu, state, st, positions, seq_index, slot_ids, n_tokens, D, n_mix, s);

@@ -86,3 +86,10 @@ def test_token_shift_wide(dtype, T, D):
     a = ops.token_shift(h, mu, plain, positions.cuda(), seq.cuda(), slots)
     b = ops.token_shift(h, mu, odd, positions.cuda(), seq.cuda(), slots)
     assert torch.equal(a, b)
+
+
+# widths around the narrowest that the wide form takes, and steps around the smallest whose workgroups take four rows
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,D", [(5, 504), (5, 512), (1, 520), (731, 4096), (733, 4096), (367, 4096), (5901, 512)])
+def test_token_shift_forms(dtype, T, D):
+    test_token_shift_wide(dtype, T, D)
