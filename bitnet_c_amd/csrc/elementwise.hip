@@ -653,6 +653,11 @@ __global__ void rmsnorm_mean_kernel(T* __restrict__ out, const T* __restrict__ a
 template <typename T> struct __align__(16) Eight { T e[8]; };        // no more than the launchers look at
 static_assert(alignof(Eight<float>) == 16 && alignof(Eight<bf16>) == 16 && sizeof(Eight<float>) == 32, "two 16-byte accesses, or one");
 
+// The narrowest row of the wide kernels, here and below: under it most of their threads have no number, while a number a thread is
+// one pass over the row as well.  us at 1,100 rows, two bf16 branches, wide / not: 256 numbers 3.8 / 3.8, 128 4.0 / 3.65, 512 3.9 / 4.4;
+// add_normed_rmsnorm in bf16 256 4.2 / 4.0, 512 4.3 / 4.6.
+#define WIDE_ROW 512
+
 template <typename T, int G>
 __global__ __launch_bounds__(256) void rmsnorm_mean_wide_kernel(T* __restrict__ out, const T* __restrict__ a, const T* __restrict__ b,
                                                                 const float* __restrict__ wa, const float* __restrict__ wb, int dim, float eps) {
@@ -704,7 +709,7 @@ template <typename T>
 static bool launch_rmsnorm_mean_wide(T* out, const T* a, const T* b, const float* wa, const float* wb, int n_rows, int dim, float eps,
                                      hipStream_t s) {
     const int per = (dim / 8 + 255) / 256;
-    if (dim % 8 || per > 4 || (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b | (uintptr_t)wa | (uintptr_t)wb) & 15)) return false;
+    if (dim % 8 || dim < WIDE_ROW || per > 4 || (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b | (uintptr_t)wa | (uintptr_t)wb) & 15)) return false;
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(n_rows), dim3(256), 0, s, out, a, b, wa, wb, dim, eps); };
     if (per == 1) go(rmsnorm_mean_wide_kernel<T, 1>);
     else if (per == 2) go(rmsnorm_mean_wide_kernel<T, 2>);
@@ -841,7 +846,7 @@ template <typename T, typename TD>
 static bool launch_add_normed_wide(float* x, const TD* delta, int n_parts, const float* wb, float eps_b, const float* w, T* out,
                                    int n_rows, int dim, float eps, hipStream_t s) {
     const int per = (dim / 8 + 255) / 256;
-    if (dim % 8 || per > 4 || (((uintptr_t)x | (uintptr_t)delta | (uintptr_t)wb | (uintptr_t)w | (uintptr_t)out) & 15)) return false;
+    if (dim % 8 || dim < WIDE_ROW || per > 4 || (((uintptr_t)x | (uintptr_t)delta | (uintptr_t)wb | (uintptr_t)w | (uintptr_t)out) & 15)) return false;
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(n_rows), dim3(256), 0, s, x, delta, n_parts, (size_t)n_rows * dim, wb, eps_b, w, out, dim, eps);
     };

@@ -187,3 +187,13 @@ def test_add_normed_rmsnorm_at_any_address(shift):
         assert torch.equal(a, b) and torch.equal(out, got)
     tol = 2.0 ** -24 * (dim ** 0.5 + 16)
     assert float((a - b).abs().max()) <= 2 * tol * float(a.abs().max()) and float((out - got).abs().max()) <= 2 * tol * float(out.abs().max())
+
+
+# the widths below and at which the wide kernels begin
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim", [504, 512, 1016, 1024])
+def test_row_kernels_where_the_wide_ones_begin(dtype, dim):
+    test_rmsnorm_mean(dtype, dim, True)
+    test_add_normed_rmsnorm_widths(dtype, dim, 0, "norm")
+    test_add_normed_rmsnorm_widths(dtype, dim, 3, "rows")
+    test_row_norm_gate_widths(dtype, dim)
