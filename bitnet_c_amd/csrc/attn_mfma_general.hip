@@ -103,8 +103,11 @@ __device__ __forceinline__ void ag_store4(bf16* op, const bf16* gp, float x0, fl
 // straight from the pages is sixteen rows in each sixteen lanes, 64 cycles an instruction instead of 16: a block took 4 x 16 x 64
 // cycles a workgroup, whatever ran beside it), now the instructions of a wave's softmax, so a block that is seen whole is not masked,
 // sums are rescaled only when a maximum has moved, and two waves a SIMD are asked for where the registers reach, which keeps the sums
-// out of the accumulation registers (the vector unit has to copy them).  2,048 tokens, 16 heads 128 wide: with 4 kv heads 228 -> 74 us,
-// with 16 of them 229 -> 115; 64 wide, 32 heads on 8: 227 -> 72; 256 wide: 397 -> 189; 128 tokens behind 2,000: 118 -> 62.
+// out of the accumulation registers (the vector unit has to copy them).  Workgroups that follow each other are heads of one tile: since
+// they go to the XCDs in turn, the tiles of a head (whose keys and values are the same) meet in few of the eight L2s, where tile
+// after tile of a head is read by every one of them (16 prompts of 100 tokens, 16 heads on 16: 25 us tile by tile, 13.3 now).  us at
+// 2,048 tokens, 16 heads 128 wide with 4 kv heads 228 -> 64, with 16 of them 228 -> 85; 64 wide, 32 heads on 8: 227 -> 55; 16 tokens
+// behind 4,000: 219 -> 107.
 template <int DC, int DT, int WAVES>     // hs = 32 DC, vd = 16 DT, heads of a workgroup
 __global__ __launch_bounds__(WAVES * BN_WAVE, DC + DT <= (WAVES > 1 ? 16 : 14) ? 2 : 1) void attn_general_prompt_kernel(GenArgs a) {
     constexpr int HS = 32 * DC, VD = 16 * DT, THREADS = WAVES * BN_WAVE;
@@ -112,9 +115,9 @@ __global__ __launch_bounds__(WAVES * BN_WAVE, DC + DT <= (WAVES > 1 ? 16 : 14) ?
     constexpr int KN = (KEYS + THREADS - 1) / THREADS, VN = (VALUES + THREADS - 1) / THREADS;       // a thread's share of them
     constexpr int BUFFERS = WAVES > 1 ? 2 : 1;
     __shared__ __align__(16) u32x4 staged[BUFFERS][KEYS + VALUES];
-    const int* tl = a.tiles + 4 * blockIdx.x;
+    const int* tl = a.tiles + 4 * blockIdx.y;
     const int seq = tl[0], row0 = tl[1], n = min(tl[2], 16), pos0 = tl[3];
-    const int head = blockIdx.y * WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int head = blockIdx.x * WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (n <= 0 || pos0 < 0) return;                      // the whole workgroup
     const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
     const int kvh = head / (a.H / a.Hkv);
@@ -509,13 +512,13 @@ extern "C" int bn_attn_general_supports(int hs, int vd) {
 }
 
 // Heads of a workgroup: as many as share a kv head, up to four, since they share the staged block: 2,048 tokens, 16 heads on 4 take
-// 74 us with four, 83 with two, 109 with one.
+// 74 us with four, 83 with two, 109 with one (tile by tile).
 static int ag_waves(int group) { return group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1; }
 
 template <int DC>
 static int ag_launch_dt(const GenArgs& a, int vd, int n_tiles, hipStream_t s) {
     const int waves = ag_waves(a.H / a.Hkv);
-    const dim3 grid(n_tiles, a.H / waves), block(waves * BN_WAVE);
+    const dim3 grid(a.H / waves, n_tiles), block(waves * BN_WAVE);
 #define AG_CASE(DT)                                                                                   \
     if (waves == 4) hipLaunchKernelGGL((attn_general_prompt_kernel<DC, DT, 4>), grid, block, 0, s, a);       \
     else if (waves == 2) hipLaunchKernelGGL((attn_general_prompt_kernel<DC, DT, 2>), grid, block, 0, s, a);  \
@@ -530,6 +533,19 @@ static int ag_launch_dt(const GenArgs& a, int vd, int n_tiles, hipStream_t s) {
         case 16: AG_CASE(16);
     }
 #undef AG_CASE
+    return BN_ERR_ARG;
+}
+
+static int ag_launch(const GenArgs& a, int hs, int vd, int n_tiles, hipStream_t s) {
+    switch (hs / 32) {
+        case 1: return ag_launch_dt<1>(a, vd, n_tiles, s);
+        case 2: return ag_launch_dt<2>(a, vd, n_tiles, s);
+        case 3: return ag_launch_dt<3>(a, vd, n_tiles, s);
+        case 4: return ag_launch_dt<4>(a, vd, n_tiles, s);
+        case 5: return ag_launch_dt<5>(a, vd, n_tiles, s);
+        case 6: return ag_launch_dt<6>(a, vd, n_tiles, s);
+        case 8: return ag_launch_dt<8>(a, vd, n_tiles, s);
+    }
     return BN_ERR_ARG;
 }
 
@@ -549,16 +565,11 @@ extern "C" int bn_attn_general_prompt(const void* q, int q_stride, void* out, in
     a.block_table = block_table; a.tiles = tiles; a.dist_a = dist_a; a.dist_b = dist_b;
     a.q_stride = q_stride; a.out_stride = out_stride; a.bt_stride = bt_stride; a.H = H; a.Hkv = Hkv;
     a.scale = scale; a.sink = sink ? 1 : 0; a.sink_values = sink ? sink_values : nullptr; a.window = window;
-    switch (hs / 32) {
-        case 1: return ag_launch_dt<1>(a, vd, n_tiles, s);
-        case 2: return ag_launch_dt<2>(a, vd, n_tiles, s);
-        case 3: return ag_launch_dt<3>(a, vd, n_tiles, s);
-        case 4: return ag_launch_dt<4>(a, vd, n_tiles, s);
-        case 5: return ag_launch_dt<5>(a, vd, n_tiles, s);
-        case 6: return ag_launch_dt<6>(a, vd, n_tiles, s);
-        case 8: return ag_launch_dt<8>(a, vd, n_tiles, s);
+    for (int first = 0; first < n_tiles; first += 65535) {       // a launch's second dimension
+        a.tiles = tiles + 4 * (size_t)first;
+        if (int rc = ag_launch(a, hs, vd, n_tiles - first < 65535 ? n_tiles - first : 65535, s)) return rc;
     }
-    return BN_ERR_ARG;
+    return 0;
 }
 
 template <int DC>

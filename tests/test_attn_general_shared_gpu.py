@@ -55,3 +55,23 @@ def test_heads_that_share_a_block_and_heads_on_their_own_give_the_same_bits(hs, 
     # the weights are rounded to bf16 in numerator and denominator (at most 2^-8 of |v| in all, |v| < 5) and the result once more
     # (2^-9 of itself)
     assert float((outs[0].float().reshape(want.shape) - want).abs().max()) <= 5 * 2.0 ** -8 + 5 * 2.0 ** -9
+
+
+def test_more_tiles_than_a_launch_has_room_for():
+    """A list of over 65,535 tiles, most of no rows (as a list may end in them), with rows in front of and behind that place."""
+    from bitnet_c_amd import ops
+    from bitnet_c_amd.cache import PAGE
+    torch.manual_seed(2)
+    H, G, hs, n, qt = 2, 1, 32, 70, ops.GENERAL_PROMPT_TILE
+    q, k, v = (torch.randn(n, h, hs).to(torch.bfloat16) for h in (H, G, G))
+    table = list(range(-(-n // PAGE)))
+    tiles = torch.tensor([[0, i, min(qt, n - i), i] for i in range(0, n, qt)], dtype=torch.int32)
+    outs = []
+    for places in (range(len(tiles)), [0, 65534, 65535, 65536, 70000]):
+        many = torch.zeros(max(places) + 1, 4, dtype=torch.int32)
+        many[list(places)] = tiles
+        out = torch.full((n, H * hs), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops.attention_general_prompt(q.reshape(n, -1).to(DEV), out, _pages(k, table, PAGE, False), _pages(v, table, PAGE, True),
+                                     torch.tensor([table], dtype=torch.int32, device=DEV), H, G, hs, hs, 0.2, many.to(DEV))
+        outs.append(out)
+    assert torch.equal(*outs) and float((outs[0].float().cpu().view(n, H, hs) - _expected(q, k, v, 0, 0.2, 0, 0)).abs().max()) < 0.05
