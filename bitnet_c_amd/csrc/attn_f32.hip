@@ -249,27 +249,36 @@ __global__ __launch_bounds__(256, PAGES == 1 ? 3 : 2) void attn_f32_decode_kerne
     const int kvh = blockIdx.y / head_tiles, ht = blockIdx.y - kvh * head_tiles;
     const int tok = blockIdx.x, len = a.seq_lens[tok];
     constexpr int part_keys = PAGES * BN_PAGE;
-    // a table is as wide as the longest sequence there can be: most workgroups of a short one have no keys
-    if (blockIdx.z > 0 && (int)blockIdx.z * part_keys >= len) return;
     const int rows = min(GT, G - ht * GT);
     const float* row = a.q + (size_t)tok * a.q_stride;
     const float* new_v = row + (size_t)(a.H + a.Hkv + kvh) * HS;
     // the queries (rows without a head as zeros) and the new key, a pair of dimensions a thread
-    for (int idx = tid; idx < 17 * HALF; idx += 256) {
-        const int h = idx / HALF, i = idx - h * HALF;
-        const bool is_key = h == 16;
-        if (is_key && !a.write) break;
-        const float* src = row + (size_t)(is_key ? a.H + kvh : kvh * G + ht * GT + min(h, rows - 1)) * HS + i;
-        float x0 = src[0], x1 = src[HALF];
+    constexpr int PAIRS = (17 * HALF + 255) / 256;
+    float x0[PAIRS], x1[PAIRS];
+#pragma unroll
+    for (int p = 0; p < PAIRS; ++p) {
+        const int idx = min(tid + 256 * p, 17 * HALF - 1), h = idx / HALF, i = idx - h * HALF;
+        const float* src = row + (size_t)(h == 16 && a.write ? a.H + kvh : kvh * G + ht * GT + min(h, rows - 1)) * HS + i;
+        x0[p] = src[0];
+        x1[p] = src[HALF];
+    }
+    // A table is as wide as the longest sequence there can be: most workgroups of a short one have no keys.  The loads above stay in
+    // front of this, on their way while the length is waited for.
+    asm volatile("" ::: "memory");
+    if (blockIdx.z > 0 && (int)blockIdx.z * part_keys >= len) return;
+#pragma unroll
+    for (int p = 0; p < PAIRS; ++p) {
+        const int idx = tid + 256 * p, h = idx / HALF, i = idx - h * HALF;
+        if (idx >= 17 * HALF || (h == 16 && !a.write)) break;
         if (a.inv_freq) {
             float sn, c;
             sincosf((float)(len - 1) * a.inv_freq[i], &sn, &c);
-            bn_rotate_pair(x0, x1, c, sn);
+            bn_rotate_pair(x0[p], x1[p], c, sn);
         }
-        if (!is_key && h >= rows) x0 = x1 = 0.f;
-        float* dst = is_key ? kn + i : qs + h * STRIDE + i;
-        dst[0] = x0;
-        dst[HALF] = x1;
+        if (h < 16 && h >= rows) x0[p] = x1[p] = 0.f;
+        float* dst = h == 16 ? kn + i : qs + h * STRIDE + i;
+        dst[0] = x0[p];
+        dst[HALF] = x1[p];
     }
     for (int part = blockIdx.z; part < a.n_parts && (part == 0 || part * part_keys < len); part += gridDim.z) {
         float M[OWN], L[OWN], O[OWN];             // (of more pages than one)
