@@ -115,11 +115,11 @@ __global__ __launch_bounds__(NWV * 64) void splitk_gemm_kernel(const bf16* __res
         const int kl = TILED ? k0 : k0 + g * 8;
         if (col && k0 + SG_STEP <= k_end) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) dst[j] = *reinterpret_cast<const uint4*>(p + j * JS);
+            for (int j = 0; j < 8; ++j) dst[j] = bn_load_once(p + j * JS);
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j)
-                dst[j] = (col && kl + j * 32 < k_end) ? *reinterpret_cast<const uint4*>(p + j * JS) : make_uint4(0, 0, 0, 0);
+                dst[j] = (col && kl + j * 32 < k_end) ? bn_load_once(p + j * JS) : make_uint4(0, 0, 0, 0);
         }
     };
     auto store_x = [&](int buf) {
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(NWV * 64) void splitk_gemm_kernel(const bf16* __res
         const int JS = TILED ? TS : 32;
         const bf16* p = TILED ? wrow + (size_t)(k0 >> 5) * TS + lane_at_w : wrow + k0 + g * 8;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dst[j] = *reinterpret_cast<const uint4*>(p + j * JS);
+        for (int j = 0; j < 8; ++j) dst[j] = bn_load_once(p + j * JS);
     };
     auto store_x_all = [&](const uint4* src, int buf) {
         unsigned char* b = xs + (size_t)buf * ROWS * SG_XROW;
