@@ -92,6 +92,13 @@ template <int HS> struct AfSums {                 // a lane's sums of its row (r
 
 // One page of keys from nothing.  k(t, b): the lane's 16 bytes of key 16 t + lane % 16, dimensions 16 b + 4 g ..; v(t, e, h):
 // its VW values of key 16 t + 4 g + e; last: the last key of the page that the lane's row sees (63: all, < 0: none).
+template <int O> __device__ __forceinline__ float af_pair_max(float v) {
+    return bn_pair_far<O>(v, [](float a, float b) { return fmaxf(a, b); });
+}
+template <int O> __device__ __forceinline__ float af_pair_sum(float v) {
+    return bn_pair_far<O>(v, [](float a, float b) { return __fadd_rn(a, b); });
+}
+
 template <int HS, typename KF, typename VF>
 __device__ __forceinline__ void af_page(const f32x4 (&q)[HS / 16], float scale, int last, bool masked, KF k, VF v, AfSums<HS>& p) {
     using S = AfShape<HS>;
@@ -115,16 +122,16 @@ __device__ __forceinline__ void af_page(const f32x4 (&q)[HS / 16], float scale, 
             s[t][e] = masked && 16 * t + 4 * g + e > last ? -INFINITY : __fmul_rn(s[t][e], scale);
             m = fmaxf(m, s[t][e]);
         }
-    m = fmaxf(m, __shfl_xor(m, 16, BN_WAVE));
-    m = fmaxf(m, __shfl_xor(m, 32, BN_WAVE));
+    m = af_pair_max<16>(m);
+    m = af_pair_max<32>(m);
     const float base = m == -INFINITY ? 0.f : m;  // a row that sees no key of the page: every exponential is 0
     float l = 0.f;
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) { s[t][e] = expf(__fsub_rn(s[t][e], base)); l = __fadd_rn(l, s[t][e]); }
-    l = __fadd_rn(l, __shfl_xor(l, 16, BN_WAVE));
-    l = __fadd_rn(l, __shfl_xor(l, 32, BN_WAVE));
+    l = af_pair_sum<16>(l);
+    l = af_pair_sum<32>(l);
     p.clear();
     p.m = m; p.l = l;
 #pragma unroll
@@ -340,8 +347,8 @@ __global__ __launch_bounds__(256, PAGES == 1 ? 3 : 2) void attn_f32_decode_kerne
                         m = fmaxf(m, s[u][e]);
                     }
                 }
-                m = fmaxf(m, __shfl_xor(m, 16, BN_WAVE));
-                m = fmaxf(m, __shfl_xor(m, 32, BN_WAVE));
+                m = af_pair_max<16>(m);
+                m = af_pair_max<32>(m);
                 const float base = m == -INFINITY ? 0.f : m;
                 f32x4 o[VW];
 #pragma unroll
@@ -360,8 +367,8 @@ __global__ __launch_bounds__(256, PAGES == 1 ? 3 : 2) void attn_f32_decode_kerne
                 for (int u = 0; u < 4; ++u)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) { s[u][e] = expf(__fsub_rn(s[u][e], base)); l = __fadd_rn(l, s[u][e]); }
-                l = __fadd_rn(l, __shfl_xor(l, 16, BN_WAVE));
-                l = __fadd_rn(l, __shfl_xor(l, 32, BN_WAVE));
+                l = af_pair_sum<16>(l);
+                l = af_pair_sum<32>(l);
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
 #pragma unroll

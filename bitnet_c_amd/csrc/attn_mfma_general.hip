@@ -401,8 +401,8 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
             s[e] = v;
             mx = fmaxf(mx, v);
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, BN_WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, BN_WAVE));
+        const auto larger = [](float x, float y) { return fmaxf(x, y); };
+        mx = bn_pair_far<32>(bn_pair_far<16>(mx, larger), larger);
         const float m_new = fmaxf(m, mx);
         float alpha = 1.f;
         if (m_new == -INFINITY) {

@@ -96,27 +96,64 @@ __device__ __forceinline__ uint4 bn_load_once(const void* p) {
     return __builtin_bit_cast(uint4, __builtin_nontemporal_load(static_cast<const bn_u32x4*>(p)));
 }
 
+// Reductions over a wave as a butterfly: every lane adds the lane 32, 16, 8, 4, 2 and 1 away, in that order.  The two long
+// steps swap halves and rows (v_permlane32_swap, v_permlane16_swap), the short ones are data-parallel-primitive moves inside
+// a row of 16; through shared memory's crossbar (__shfl_xor) every step waits some 120 cycles for the one before it, which is
+// a third of a microsecond a sum in kernels that take three (with
+// block_sum's barriers, decode steps of Llama and Fazopel at 2,048 columns take 2 and 1 % less).  The same pairs are added either way: the same bits.  All 64
+// lanes take part.
+template <int CTRL> __device__ __forceinline__ float bn_dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+#define BN_DPP_XOR1 0xB1              // quad_perm [1, 0, 3, 2]
+#define BN_DPP_XOR2 0x4E              // quad_perm [2, 3, 0, 1]
+#define BN_DPP_XOR3 0x1B              // quad_perm [3, 2, 1, 0]
+#define BN_DPP_XOR7 0x141             // row_half_mirror
+#define BN_DPP_XOR8 0x128             // row_ror:8
+// the value of the lane O away (O a power of two below 16)
+template <int O> __device__ __forceinline__ float bn_lane_xor(float v) {
+    static_assert(O == 1 || O == 2 || O == 4 || O == 8, "inside a row of 16 lanes");
+    if constexpr (O == 1) return bn_dpp<BN_DPP_XOR1>(v);
+    if constexpr (O == 2) return bn_dpp<BN_DPP_XOR2>(v);
+    if constexpr (O == 4) return bn_dpp<BN_DPP_XOR3>(bn_dpp<BN_DPP_XOR7>(v));
+    return bn_dpp<BN_DPP_XOR8>(v);
+}
+// op(v of this lane, v of the lane 32 or 16 away) for an op that does not care which is which
+template <int O, typename F> __device__ __forceinline__ float bn_pair_far(float v, F op) {
+    static_assert(O == 16 || O == 32, "across rows of 16 lanes");
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto r = O == 32 ? __builtin_amdgcn_permlane32_swap(b, b, false, false) : __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    return op(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+template <typename F> __device__ __forceinline__ float bn_wave_reduce(float v, F op) {
+    v = bn_pair_far<32>(v, op);
+    v = bn_pair_far<16>(v, op);
+    v = op(v, bn_lane_xor<8>(v));
+    v = op(v, bn_lane_xor<4>(v));
+    v = op(v, bn_lane_xor<2>(v));
+    return op(v, bn_lane_xor<1>(v));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, BN_WAVE);
-    return v;
+    return bn_wave_reduce(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, BN_WAVE));
-    return v;
+    return bn_wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
+
+// A barrier that orders shared memory alone: loads and stores of global memory stay in flight across it (__syncthreads waits
+// for a row's stores to be acknowledged, a trip to memory).
+__device__ __forceinline__ void bn_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Sum over a block of up to 1024 threads; every thread gets the result.
 // `scratch` holds at least 16 floats of shared memory.  The order of the additions is
-// fixed by the block size alone.
+// fixed by the block size alone.  Orders shared memory among the threads, not global memory.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
     const int lane = threadIdx.x & (BN_WAVE - 1), w = threadIdx.x / BN_WAVE;
     const int nw = (blockDim.x + BN_WAVE - 1) / BN_WAVE;
     v = wave_sum(v);
-    __syncthreads();
+    bn_lds_barrier();
     if (lane == 0) scratch[w] = v;
-    __syncthreads();
+    bn_lds_barrier();
     float t = 0.f;
     for (int i = 0; i < nw; ++i) t += scratch[i];
     return t;
@@ -125,9 +162,9 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
     const int lane = threadIdx.x & (BN_WAVE - 1), w = threadIdx.x / BN_WAVE;
     const int nw = (blockDim.x + BN_WAVE - 1) / BN_WAVE;
     v = wave_max(v);
-    __syncthreads();
+    bn_lds_barrier();
     if (lane == 0) scratch[w] = v;
-    __syncthreads();
+    bn_lds_barrier();
     float t = scratch[0];
     for (int i = 1; i < nw; ++i) t = fmaxf(t, scratch[i]);
     return t;

@@ -150,7 +150,7 @@ __device__ __forceinline__ void skinny_gemm_body(const bf16* __restrict__ X, con
         const int nn = (l & 15) < CW ? n0 + (l & 15) : N;          // a column past the workgroup's own is nobody's
         if (GLU8) {
             // columns 0..7 of the tile are gates, 8..15 the ups of the same result columns
-            const float up = __shfl_xor(v, 8, BN_WAVE);
+            const float up = bn_lane_xor<8>(v);
             if ((l & 8) == 0 && m < M && nn < N)
                 Y[(size_t)m * ldy + (n0 >> 1) + (l & 7)] = from_f32<TO>(bn_gate_act(v, act) * up);
         } else if (m < M && nn < N) {
@@ -311,7 +311,7 @@ void skinny_gemm_fused_kernel(const bf16* __restrict__ X, const bf16* __restrict
         const bool mine = (l & 15) < tile_cols && nn < N;                 // a column this workgroup owns
         if (PRE) v *= scale_s[m];
         if (GLU8) {
-            const float up = __shfl_xor(v, 8, BN_WAVE);
+            const float up = bn_lane_xor<8>(v);
             if ((l & 8) == 0 && m < M && nn < N)                          // GLU8: tile_cols is 16
                 Y[(size_t)m * ldy + (n0 >> 1) + (l & 7)] = __float2bfloat16(bn_gate_act(v, act) * up);
         } else if (RES) {
@@ -322,8 +322,10 @@ void skinny_gemm_fused_kernel(const bf16* __restrict__ X, const bf16* __restrict
                 f.resid_bf16[(size_t)m * f.ld_rb + nn] = __float2bfloat16(xn * f.next_weight[nn]);
             }
             float sq = xn * xn;                                   // the tile's columns of row m: lanes 16 (l / 16) + 0..15
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) sq += __shfl_xor(sq, o, BN_WAVE);
+            sq += bn_lane_xor<1>(sq);
+            sq += bn_lane_xor<2>(sq);
+            sq += bn_lane_xor<4>(sq);
+            sq += bn_lane_xor<8>(sq);
             if ((l & 15) == 0 && m < M) f.slots_out[(size_t)m * gridDim.x + blockIdx.x] = sq;
         } else if (m < M && mine) {
             Y[(size_t)m * ldy + nn] = __float2bfloat16(v);

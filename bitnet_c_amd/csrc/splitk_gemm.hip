@@ -269,7 +269,7 @@ __global__ __launch_bounds__(NWV * 64) void splitk_gemm_kernel(const bf16* __res
             for (int r = 0; r < 4; ++r) {
                 const int m = mt * 16 + 4 * g + r;
                 const float v = acc[mt][r] * ((nrm.slots && m < M) ? scale_s[m] : 1.0f);
-                const float up = __shfl_xor(v, 8, BN_WAVE);
+                const float up = bn_lane_xor<8>(v);
                 if ((i & 8) == 0 && m < M && n0 + i < N)
                     Y[(size_t)m * ldy + (n0 >> 1) + i] = __float2bfloat16(bn_gate_act(v, act) * up);
             }
