@@ -96,12 +96,18 @@ __device__ __forceinline__ uint4 bn_load_once(const void* p) {
     return __builtin_bit_cast(uint4, __builtin_nontemporal_load(static_cast<const bn_u32x4*>(p)));
 }
 
+// A buffer of `bytes` bytes for loads with one 32-bit offset a lane and one in a scalar register: no 64-bit addresses in
+// vector registers, and nothing past the buffer's end is read.
+#define BN_BUFFER_NT 2                // the loads' cache policy: non-temporal
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t bn_buffer(const void* p, unsigned bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
+}
+
 // Reductions over a wave as a butterfly: every lane adds the lane 32, 16, 8, 4, 2 and 1 away, in that order.  The two long
 // steps swap halves and rows (v_permlane32_swap, v_permlane16_swap), the short ones are data-parallel-primitive moves inside
-// a row of 16; through shared memory's crossbar (__shfl_xor) every step waits some 120 cycles for the one before it, which is
-// a third of a microsecond a sum in kernels that take three (with
-// block_sum's barriers, decode steps of Llama and Fazopel at 2,048 columns take 2 and 1 % less).  The same pairs are added either way: the same bits.  All 64
-// lanes take part.
+// a row of 16; through shared memory's crossbar (__shfl_xor) every step waits some 120 cycles for the one before it, a third
+// of a microsecond a sum in kernels that take three (whole calls of Llama, Fazopel and Sunusun at 2,048 columns take 1 to 4 %
+// less, block_sum's barriers included).  The same pairs are added either way: the same bits.  All 64 lanes take part.
 template <int CTRL> __device__ __forceinline__ float bn_dpp(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }

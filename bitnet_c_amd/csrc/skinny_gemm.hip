@@ -30,6 +30,7 @@
 //
 // Needs K % 8 == 0 and 16-byte aligned rows; other shapes go to the tiled kernel.
 #include "common.h"
+#include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -39,6 +40,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
 
 #define SK_XROW 528           // bytes between rows of a wave's staged X chunk (512 + 16: conflict-free 16-byte reads)
+
+#define SK_STREAM_WAVES 8     // waves of a workgroup over a streamed copy of whole chunks
 
 #define SK_ACT_UNARY 16       // act: this plus one of BN_UNARY_*: an activation of one argument on every result
 
@@ -333,6 +336,267 @@ void skinny_gemm_fused_kernel(const bf16* __restrict__ X, const bf16* __restrict
     }
 }
 
+// ---------------------------------------------------------------------------------------
+// The products of up to 16 rows over a streamed copy whose K is whole chunks (K % 256 == 0), which is every decode product of
+// ordinary widths.  Bound by the bytes of W, and at widths of 2,048 by what happens once a launch: the same sums in the same
+// order as the kernels above (wave w takes chunks w, w + 8, ..; the waves' sums are added in wave order: the same bits), in
+// straight-line code.  Nothing is predicated (a lane without a row or a column reads its neighbour's and drops what it forms;
+// a load under a branch makes the compiler wait for every load in flight), the number of activation loads is a template
+// argument, a wave has two chunks of weights in flight (16 KB; one where K <= 2,048 gives it no second, so that three
+// workgroups fit on a CU), and what the epilogue needs of memory is asked for before the weights.
+//   us with cold weights in a graph of such launches, 1 / 8 rows, the kernels above -> these: 2,048 columns of the stream
+//   QKV 5.7 / 6.2 -> 4.1 / 4.5, output 5.1 / 5.3 -> 3.7 / 4.0, gate/up (5,632) 12.3 / 13.1 -> 9.9 / 11.0, down 8.1 / 8.9 ->
+//   6.5 / 7.3; 8B QKV 12.2 / 13.4 -> 10.3 / 11.5, output 9.4 / 10.0 -> 7.7 / 8.3, gate/up 43.9 / 44.9 -> 38.5 / 40.4, down
+//   24.0 / 24.7 -> 21.1 / 22.0 (a plain read of the same bytes with a dependent launch: 4.0, 3.1, 8.3, 5.2; 8.9, 6.5, 35.8,
+//   18.4).  At 9 to 16 rows the activations' registers leave room for one workgroup of two chunks a wave on a CU (8B QKV 15.5
+//   -> 14.1, gate/up 48.0 -> 43.7).
+template <int XR, bool ONE>
+struct SkStream {
+    // XR: activation loads a lane and chunk, for up to 2 XR rows; ONE: a wave has one chunk at most
+    __amdgpu_buffer_rsrc_t wb, xb;
+    unsigned tile, w_at;
+    unsigned x_at[XR];
+    unsigned char *park_at, *read_at;
+    bf16x8 x[XR];
+    f32x4 acc;
+
+    // (the scheduling barriers keep the loads of a chunk where they are written: moved up over the products before them they
+    // need registers that are not there)
+    __device__ __forceinline__ void load_x(int c) {
+#pragma unroll
+        for (int r = 0; r < XR; ++r) x[r] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(xb, x_at[r], c * (SK_CHUNK * 2), 0));
+    }
+    __device__ __forceinline__ void load_w(bf16x8 (&w)[8], int c) {
+        unsigned at = (unsigned)c * 8 * tile;
+#pragma unroll
+        for (int j = 0; j < 8; ++j, at += tile)
+            w[j] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wb, w_at, at, BN_BUFFER_NT));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // the chunk's activations into the wave's own region of shared memory (a wave's operations on it run in order)
+    __device__ __forceinline__ void park() {
+#pragma unroll
+        for (int r = 0; r < XR; ++r) *reinterpret_cast<bf16x8*>(park_at + 2 * r * SK_XROW) = x[r];
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __device__ __forceinline__ void multiply(const bf16x8 (&w)[8]) {
+#pragma unroll
+        for (int h = 0; h < 8; h += 4) {
+            bf16x8 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const bf16x8*>(read_at + (h + j) * 64);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[j], w[h + j], acc, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    // this wave's share of X . W^T for row of tiles bx; `between` runs once the first weights have been asked for
+    template <typename F>
+    __device__ __forceinline__ void run(const bf16* X, const bf16* W, int M, int n_chunks, int ldx, int k_tiles, int rows, int bx,
+                                        unsigned char* xs, int lane, int wave, F between) {
+        const int i = lane & 15, g = lane >> 4;
+        tile = rows * (BN_STREAM_TILE_COLS * 2);
+        wb = bn_buffer(reinterpret_cast<const char*>(W) + (size_t)bx * k_tiles * tile, k_tiles * tile);
+        xb = bn_buffer(X, ((M - 1) * ldx + n_chunks * SK_CHUNK) * 2);
+        w_at = (g * rows + min(i, rows - 1)) * 16;
+#pragma unroll
+        for (int r = 0; r < XR; ++r) x_at[r] = (min(2 * r + (lane >> 5), M - 1) * ldx + (lane & 31) * 8) * 2;
+        xs += (size_t)wave * 2 * XR * SK_XROW;
+        park_at = xs + (lane >> 5) * SK_XROW + (lane & 31) * 16;
+        read_at = xs + min(i, M - 1) * SK_XROW + g * 16;
+        acc = (f32x4){0.f, 0.f, 0.f, 0.f};
+        const int n = (n_chunks - wave + SK_STREAM_WAVES - 1) / SK_STREAM_WAVES;       // chunks of this wave
+        if (ONE || n <= 1) {
+            if (n == 1) {
+                bf16x8 w[8];
+                load_x(wave);
+                load_w(w, wave);
+                between();
+                park();
+                multiply(w);
+            } else {
+                between();
+            }
+            return;
+        }
+        constexpr int D = SK_STREAM_WAVES;
+        int c = wave, left = n;
+        bf16x8 a[8], b[8];
+        load_x(c);
+        load_w(a, c);
+        load_w(b, c + D);
+        between();
+#pragma unroll 1
+        for (; left > 3; left -= 2, c += 2 * D) {
+            park();
+            load_x(c + D);
+            multiply(a);
+            load_w(a, c + 2 * D);
+            park();
+            load_x(c + 2 * D);
+            multiply(b);
+            load_w(b, c + 3 * D);
+        }
+        park();
+        load_x(c + D);
+        multiply(a);
+        if (left == 2) {
+            park();
+            multiply(b);
+            return;
+        }
+        load_w(a, c + 2 * D);
+        park();
+        load_x(c + 2 * D);
+        multiply(b);
+        park();
+        multiply(a);
+    }
+};
+
+// the waves' sums -> shared memory; then waves 0..3: thread (l, r = wave) holds row 4 (l / 16) + r, column l % 16 of the product
+__device__ __forceinline__ float sk_stream_total(float* red, const f32x4& acc, int lane, int wave) {
+    *reinterpret_cast<f32x4*>(red + (wave * 64 + lane) * 4) = acc;
+    bn_lds_barrier();
+    float v = 0.f;
+    if (wave < 4) {
+#pragma unroll
+        for (int w = 0; w < SK_STREAM_WAVES; ++w) v += red[(w * 64 + lane) * 4 + wave];
+    }
+    return v;
+}
+
+#define SK_STREAM_RED (SK_STREAM_WAVES * 256 + 16)       // floats: the waves' sums, the norm's row factors
+
+template <int XR, bool ONE, typename TO, bool UNARY>
+__device__ __forceinline__ void sk_stream_plain(const bf16* X, const bf16* W, TO* Y, int M, int N, int n_chunks, int ldx, int k_tiles,
+                                                int ldy, int rows, int act, int bx) {
+    extern __shared__ __align__(16) float red[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    SkStream<XR, ONE> s;
+    s.run(X, W, M, n_chunks, ldx, k_tiles, rows, bx, reinterpret_cast<unsigned char*>(red + SK_STREAM_RED), lane, wave, [] {});
+    const float v = sk_stream_total(red, s.acc, lane, wave);
+    if (wave >= 4) return;
+    const int m = 4 * (lane >> 4) + wave, n = bx * rows + (lane & 15);
+    if (m < M && (lane & 15) < rows && n < N) Y[(size_t)m * ldy + n] = from_f32<TO>(sk_result<UNARY>(v, act));
+}
+
+template <int XR, bool ONE, typename TO, bool UNARY>
+__global__ __launch_bounds__(64 * SK_STREAM_WAVES, (ONE && XR <= 4) ? 6 : XR == 8 ? 2 : 4)
+void skinny_stream_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, TO* __restrict__ Y, int M, int N, int n_chunks, int ldx,
+                          int k_tiles, int ldy, int rows, int act) {
+    sk_stream_plain<XR, ONE, TO, UNARY>(X, W, Y, M, N, n_chunks, ldx, k_tiles, ldy, rows, act, blockIdx.x);
+}
+
+template <int XR, bool ONE>
+__global__ __launch_bounds__(64 * SK_STREAM_WAVES, (ONE && XR <= 4) ? 6 : XR == 8 ? 2 : 4)
+void skinny_stream_group_kernel(SkinnyGroup p, int M, int n_chunks, int k_tiles) {
+    int j = 0;
+    while (j + 1 < p.count && (int)blockIdx.x >= p.first[j + 1]) ++j;
+    sk_stream_plain<XR, ONE, bf16, true>(p.x[j], p.w[j], p.y[j], M, p.n[j], n_chunks, p.ldx[j], k_tiles, p.n[j], p.rows[j], p.act[j],
+                                         (int)blockIdx.x - p.first[j]);
+}
+
+// the forms of skinny_gemm_fused_kernel: a gated unit behind a norm, a product behind a norm, a product into the stream
+#define SK_FUSED_GLU 0
+#define SK_FUSED_PRE 1
+#define SK_FUSED_RES 2
+template <int XR, bool ONE, int FORM, int SL>
+__global__ __launch_bounds__(64 * SK_STREAM_WAVES, (ONE && XR <= 4) ? 6 : XR == 8 ? 2 : 4)
+void skinny_stream_fused_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, bf16* __restrict__ Y, int M, int N, int n_chunks,
+                                int ldx, int k_tiles, int ldy, int rows, int act, SkinnyFused f) {
+    constexpr bool PRE = FORM != SK_FUSED_RES;
+    constexpr int H = XR <= 4 ? 1 : 2;                // rows of the norm that a wave adds up: wave, and wave + 8
+    extern __shared__ __align__(16) float red[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float* scale_s = red + SK_STREAM_WAVES * 256;
+    const int n0 = blockIdx.x * rows, at = lane & 15;
+    const int m = 4 * (lane >> 4) + (wave & 3), n = n0 + at;
+    float sv[H][SL];
+    if (PRE) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            const unsigned row = (unsigned)min(wave + SK_STREAM_WAVES * h, M - 1) * f.n_slots;
+#pragma unroll
+            for (int j = 0; j < SL; ++j) sv[h][j] = f.slots_in[row + min(lane + 64 * j, f.n_slots - 1)];
+        }
+    }
+    float old = 0.f, next_w = 0.f;
+    if (!PRE) {
+        const int nc = min(n, N - 1);
+        old = f.resid[(size_t)min(m, M - 1) * f.ld_resid + nc];
+        next_w = f.next_weight[nc];
+    }
+    SkStream<XR, ONE> s;
+    s.run(X, W, M, n_chunks, ldx, k_tiles, rows, blockIdx.x, reinterpret_cast<unsigned char*>(red + SK_STREAM_RED), lane, wave, [&] {
+        if (PRE) {
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                float v = 0.f;
+#pragma unroll
+                for (int j = 0; j < SL; ++j) v += lane + 64 * j < f.n_slots ? sv[h][j] : 0.f;
+                v = 1.0f / sqrtf(wave_sum(v) * f.inv_width + f.eps);
+                if (lane == 0) scale_s[wave + SK_STREAM_WAVES * h] = v;
+            }
+        }
+    });
+    float v = sk_stream_total(red, s.acc, lane, wave);
+    if (wave >= 4) return;
+    const bool mine = m < M && at < rows && n < N;
+    if (PRE) v *= scale_s[m];                         // rows past M: whatever lies there, not stored
+    if (FORM == SK_FUSED_GLU) {
+        const float up = bn_lane_xor<8>(v);           // columns 0..7 of the tile are gates, 8..15 the ups of the same results
+        if (mine && (lane & 8) == 0) Y[(size_t)m * ldy + (n0 >> 1) + (lane & 7)] = __float2bfloat16(bn_gate_act(v, act) * up);
+    } else if (FORM == SK_FUSED_PRE) {
+        if (mine) Y[(size_t)m * ldy + n] = __float2bfloat16(v);
+    } else {
+        float xn = 0.f;
+        if (mine) {
+            xn = old + v;
+            f.resid[(size_t)m * f.ld_resid + n] = xn;
+            f.resid_bf16[(size_t)m * f.ld_rb + n] = __float2bfloat16(xn * next_w);
+        }
+        float sq = xn * xn;                           // the tile's columns of row m: lanes 16 (l / 16) + 0..15
+        sq += bn_lane_xor<1>(sq);
+        sq += bn_lane_xor<2>(sq);
+        sq += bn_lane_xor<4>(sq);
+        sq += bn_lane_xor<8>(sq);
+        if (at == 0 && m < M) f.slots_out[(size_t)m * gridDim.x + blockIdx.x] = sq;
+    }
+}
+
+// whole chunks only; offsets inside a row of tiles and inside the activations are 32 bits wide
+static bool sk_stream_ok(int M, int K, int ldx) {
+    return M <= 16 && K % SK_CHUNK == 0 && K <= 1 << 24 && (long long)M * ldx <= 1 << 29;
+}
+
+// go(XR, ONE) as integral constants for M rows and K columns
+template <typename F> static int sk_stream_pick(int M, int K, F go) {
+    using std::integral_constant;
+    const bool one = K <= SK_CHUNK * SK_STREAM_WAVES;
+#define SK_PICK(XR_) return one ? go(integral_constant<int, XR_>(), integral_constant<bool, true>()) \
+                                : go(integral_constant<int, XR_>(), integral_constant<bool, false>())
+    if (M <= 2) SK_PICK(1);
+    if (M <= 4) SK_PICK(2);
+    if (M <= 8) SK_PICK(4);
+    SK_PICK(8);
+#undef SK_PICK
+}
+
+template <typename KERNEL, typename... ARGS>
+static int sk_stream_launch(KERNEL kernel, int xr, unsigned groups, hipStream_t s, ARGS... args) {
+    const size_t smem = SK_STREAM_RED * sizeof(float) + (size_t)SK_STREAM_WAVES * 2 * xr * SK_XROW;
+    if (smem > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return (int)e;
+    }
+    hipLaunchKernelGGL(kernel, dim3(groups), dim3(64 * SK_STREAM_WAVES), smem, s, args...);
+    return bn_launch_status();
+}
+
 extern "C" int bn_skinny_gemm_supports(int M, int N, int K, int ldx, int ldw);
 static bool sk_tiled_ok(int K, int ldw) { return ldw == (K + BN_STREAM_TILE_COLS - 1) / BN_STREAM_TILE_COLS; }
 
@@ -408,6 +672,20 @@ extern "C" int bn_skinny_gemm_fused(const void* X, const void* W, void* Y, int M
     f.slots_in = slots_in; f.n_slots = n_slots; f.inv_width = pre ? 1.0f / (float)stream_width : 0.f; f.eps = eps;
     f.resid = resid; f.resid_bf16 = (bf16*)resid_bf16; f.next_weight = next_weight; f.slots_out = slots_out;
     f.ld_resid = ld_resid; f.ld_rb = ld_rb;
+    const bool few = n_slots <= 256;                  // four slot loads per row and lane are enough
+    if (glu8 && !pre) return BN_ERR_ARG;
+    if (tiled && sk_stream_ok(M, K, ldx) && !(pre && res))
+        return sk_stream_pick(M, K, [&](auto xr, auto one) {
+            constexpr int XR = decltype(xr)::value;
+            constexpr bool ONE = decltype(one)::value;
+            auto go = [&](auto kernel) {
+                return sk_stream_launch(kernel, XR, (unsigned)((N + tile_rows - 1) / tile_rows), s, (const bf16*)X, (const bf16*)W, (bf16*)Y,
+                                        M, N, K / SK_CHUNK, ldx, ldw, ldy, tile_rows, act, f);
+            };
+            if (glu8) return few ? go(skinny_stream_fused_kernel<XR, ONE, SK_FUSED_GLU, 4>) : go(skinny_stream_fused_kernel<XR, ONE, SK_FUSED_GLU, 8>);
+            if (pre) return few ? go(skinny_stream_fused_kernel<XR, ONE, SK_FUSED_PRE, 4>) : go(skinny_stream_fused_kernel<XR, ONE, SK_FUSED_PRE, 8>);
+            return go(skinny_stream_fused_kernel<XR, ONE, SK_FUSED_RES, 1>);
+        });
     const size_t smem = (size_t)(8 * 256 + 16) * sizeof(float) + (size_t)8 * M * SK_XROW;
     const int tile_cols = tiled ? tile_rows : (glu8 ? 16 : sk_fused_tile_cols(N));
     const dim3 grid((N + tile_cols - 1) / tile_cols), block(8 * 64);
@@ -421,8 +699,6 @@ extern "C" int bn_skinny_gemm_fused(const void* X, const void* W, void* Y, int M
                            tile_cols, act, f);
         return bn_launch_status();
     };
-    const bool few = n_slots <= 256;                  // four slot loads per row and lane are enough
-    if (glu8 && !pre) return BN_ERR_ARG;
 #define SK_FUSED(T)                                                                                                      \
     do {                                                                                                                 \
         if (glu8) return few ? go(skinny_gemm_fused_kernel<true, true, false, 4, T>)                                     \
@@ -505,6 +781,19 @@ extern "C" int bn_skinny_gemm(int out_dtype, const void* X, const void* W, void*
     if (((uintptr_t)X | (uintptr_t)W) & 15) return BN_ERR_ARG;
     if (tiled) {
         if (dual || M > 16 || !sk_tiled_ok(K, ldw) || tile_rows < 1 || tile_rows > BN_STREAM_TILE_ROWS) return BN_ERR_ARG;
+        if (sk_stream_ok(M, K, ldx) && (out_dtype == BN_DT_BF16 || out_dtype == BN_DT_F32))
+            return sk_stream_pick(M, K, [&](auto xr, auto one) {
+                constexpr int XR = decltype(xr)::value;
+                constexpr bool ONE = decltype(one)::value;
+                const unsigned groups = (unsigned)((N + tile_rows - 1) / tile_rows);
+                auto go = [&](auto kernel, auto* y) {
+                    return sk_stream_launch(kernel, XR, groups, s, (const bf16*)X, (const bf16*)W, y, M, N, K / SK_CHUNK, ldx, ldw, ldy,
+                                            tile_rows, act);
+                };
+                if (unary) return go(skinny_stream_kernel<XR, ONE, bf16, true>, (bf16*)Y);
+                if (out_dtype == BN_DT_BF16) return go(skinny_stream_kernel<XR, ONE, bf16, false>, (bf16*)Y);
+                return go(skinny_stream_kernel<XR, ONE, float, false>, (float*)Y);
+            });
         int n_waves = 8;                           // as the row-major form with staged activations
         const int k_chunks = (K + SK_CHUNK - 1) / SK_CHUNK;
         while (n_waves > 1 && n_waves / 2 >= k_chunks) n_waves >>= 1;
@@ -556,6 +845,7 @@ extern "C" int bn_skinny_group(int count, const void* const* X, const void* cons
     SkinnyGroup p;
     p.count = count;
     int groups = 0;
+    bool whole = true;
     for (int j = 0; j < count; ++j) {
         if (!bn_skinny_gemm_supports(M, N[j], K, ldx[j], 8) || ldx[j] < K || tile_rows[j] < 1 || tile_rows[j] > BN_STREAM_TILE_ROWS ||
             unary[j] < -1 || unary[j] >= BN_UNARY_KINDS || (((uintptr_t)X[j] | (uintptr_t)W[j]) & 15) || !Y[j])
@@ -564,7 +854,13 @@ extern "C" int bn_skinny_group(int count, const void* const* X, const void* cons
         p.n[j] = N[j]; p.ldx[j] = ldx[j]; p.rows[j] = tile_rows[j]; p.act[j] = unary[j] < 0 ? 0 : SK_ACT_UNARY + unary[j];
         p.first[j] = groups;
         groups += (N[j] + tile_rows[j] - 1) / tile_rows[j];
+        whole = whole && sk_stream_ok(M, K, ldx[j]);
     }
+    if (whole)
+        return sk_stream_pick(M, K, [&](auto xr, auto one) {
+            return sk_stream_launch(skinny_stream_group_kernel<decltype(xr)::value, decltype(one)::value>, decltype(xr)::value,
+                                    (unsigned)groups, s, p, M, K / SK_CHUNK, k_tiles);
+        });
     int n_waves = 8;
     const int k_chunks = (K + SK_CHUNK - 1) / SK_CHUNK;
     while (n_waves > 1 && n_waves / 2 >= k_chunks) n_waves >>= 1;
