@@ -27,9 +27,12 @@
 // where that spreads the tiles more evenly over the CUs); its 32 R elements are stored so that the eight of lane
 // r + 16 g (r < R) are the elements 8 (R g + r) .. 8 (R g + r) + 7; tiles in the order [ceil(N / R)][ceil(K / 32)], rows
 // past N and columns past K zero.  One load of a wave reads one tile as 64 R consecutive bytes (the lanes r >= R idle).
+// A float32 matrix (gemm_f32.hip) is kept the same way in tiles of R rows x 16 columns, four columns to a lane's 16 bytes:
+// the elements 4 (R g + r) .. 4 (R g + r) + 3 of a tile are columns 4 g .. 4 g + 3 of its row r.
 // The Python side reads these lines too.
 #define BN_STREAM_TILE_ROWS 16        // the most rows of a tile
 #define BN_STREAM_TILE_COLS 32
+#define BN_STREAM_TILE_COLS_F32 16
 
 // Cache pages in the matrix-core attention kernels' own order ("blocked"; bf16, head sizes that are multiples of 32).  A
 // page still holds BN_PAGE positions of hs elements for every kv head, keys and values each, but inside a (page, kv head)

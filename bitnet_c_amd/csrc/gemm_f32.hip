@@ -9,16 +9,18 @@
 // added in order.  The cut is what lets a product of few rows spread one output's K over the waves of a workgroup (and it
 // keeps the rounding error at that of a sum of 128 and of K / 128 terms).
 //
-// gemm_f32_stream_kernel, up to 64 rows: bound by the bytes of W.  A workgroup of 8 waves owns up to 16 columns and all of
-// K; a wave takes every eighth chunk, asks for its whole 8 KB of W (and the rows' 128 columns of A) at once and leaves
-// 16 x 16 sums in shared memory; then a thread an output adds them up in order.  us at one row, 1.5 GB of weights in turn, and at
-// 6.5 TB/s: 11,264 x 2,048 24 (14), 2,048 x 5,632 19.5 (7), 32,000 x 2,048 52 (40), 28,672 x 4,096 103 (72); the vector kernel that
-// walked K in one chain (gemm_tiled.hip) took 325 on the average of a layer's products, whatever the rows up to 16.
+// gemm_f32_streamed_kernel, up to 16 rows over a streamed copy of W: see there.
+// gemm_f32_stream_kernel, up to 64 rows over W itself: bound by the bytes of W.  A workgroup of 8 waves owns up to 16 columns
+// and all of K; a wave takes every eighth chunk, asks for its whole 8 KB of W (and the rows' 128 columns of A) at once and
+// leaves 16 x 16 sums in shared memory; then a thread an output adds them up in order.  us at one row, 1.5 GB of weights in
+// turn, and at 6.5 TB/s: 11,264 x 2,048 24 (14), 2,048 x 5,632 19.5 (7), 32,000 x 2,048 52 (40), 28,672 x 4,096 103 (72); the
+// vector kernel that walked K in one chain (gemm_tiled.hip) took 325 on the average of a layer's products, whatever the rows
+// up to 16.  Its loads of W are plain: two of them take the halves of a line, and non-temporal ones were slower (11,264 x 2,048
+// at 8 rows 25 -> 26 us, 32,000 x 2,048 59 -> 65).
 // gemm_f32_tile_kernel, more rows: bound by the instruction (157 TFLOP/s on this chip, 32 cycles each on a SIMD).  5,136 x
 // 11,264 x 2,048 2.02 ms (117 TFLOP/s), 2,048 x 2,048 x 5,632 0.40 ms; the matrix unit is busy four fifths of a round, the
 // rest is the last round's empty CUs.  The vector kernel did 27 TFLOP/s.
 #include "common.h"
-#include <type_traits>
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -47,14 +49,8 @@ __device__ __forceinline__ f32x4 gf_load(const float* p, bool ok) {
     return v;
 }
 
-__device__ __forceinline__ f32x4 gf_load_once(const float* p, bool ok) {
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (ok) v = __builtin_bit_cast(f32x4, bn_load_once(p));
-    return v;
-}
-
 // MT row tiles of 16 share a wave's registers of W
-template <int MT, bool ONCE>
+template <int MT>
 __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArgs a) {
     constexpr int ROUND = GF_SUMS_KB / MT;                       // chunks whose sums shared memory holds at a time
     constexpr int THREADS = 64 * GF_WAVES;
@@ -80,19 +76,17 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
         const int c1 = min(n_chunks, c0 + ROUND);
         auto chunk = [&](int c, auto whole) {
             const int k0 = c * GF_CHUNK;
-            auto fetch = [&](const float* p, f32x4 (&v)[GF_BLOCKS], auto once) {
+            auto fetch = [&](const float* p, f32x4 (&v)[GF_BLOCKS]) {
 #pragma unroll
-                for (int j = 0; j < GF_BLOCKS; ++j) {
-                    const bool ok = decltype(whole)::value || k0 + 16 * j + 4 * g < a.K;
-                    v[j] = decltype(once)::value ? gf_load_once(p + k0 + 16 * j, ok) : gf_load(p + k0 + 16 * j, ok);
-                }
+                for (int j = 0; j < GF_BLOCKS; ++j)
+                    v[j] = gf_load(p + k0 + 16 * j, decltype(whole)::value || k0 + 16 * j + 4 * g < a.K);
             };
             f32x4 wv[GF_BLOCKS];
-            fetch(wp, wv, std::integral_constant<bool, ONCE>());
+            fetch(wp, wv);
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
                 f32x4 xv[GF_BLOCKS], acc = {0.f, 0.f, 0.f, 0.f};
-                fetch(xp[t], xv, gf_false());
+                fetch(xp[t], xv);
 #pragma unroll
                 for (int j = 0; j < GF_BLOCKS; ++j)
 #pragma unroll
@@ -128,6 +122,126 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
     for (int idx = tid; idx < MT * 128; idx += THREADS) {
         const int m = idx >> 3, n = idx & 7;
         if (m < a.M) a.y[(size_t)m * a.ldy + n0 / 2 + n] = bn_gate_act(sums[m * 16 + n], a.act) * sums[m * 16 + 8 + n];
+    }
+}
+
+// ---------------------------------------------------------------------------------------
+// The product of up to 16 rows over a streamed copy of W (common.h) whose K is whole chunks.  Bound by the bytes of W: over
+// the row-major matrix a load takes 64 bytes of each of 16 rows, half of a cache line, and waits under a test; here it takes
+// a tile, 1 KB in a run, non-temporally, in straight-line code with two chunks (16 KB) a wave in flight, and the activations
+// go through the wave's own shared memory, so that one row costs one load a chunk instead of eight.  The same sums in the
+// same order as the kernels around it (a chunk by itself, the chunks in order): the same bits.  XR: activation loads a lane
+// and chunk, for up to 2 XR rows.
+//   us at 1 / 8 rows with cold weights in a graph of such launches, row-major -> streamed: 3,072 x 2,048 8.4 / 10.1 -> 7.2 /
+//   7.6, 2,048 x 2,048 7.9 / 8.0 -> 6.0 / 6.8, 11,264 x 2,048 23.2 / 26.5 -> 17.6 / 18.7, 2,048 x 5,632 19.3 / 19.7 -> 11.6 /
+//   13.1, 32,000 x 2,048 55.6 / 66.4 -> 43.2 / 44.4, 28,672 x 4,096 96 / 117 -> 76.5 / 75.5, 4,096 x 14,336 57 / 63 -> 41 / 42.
+//   (16 instructions of 32 cycles stand for 4 KB of eight columns: up to 2,048 columns the matrix unit has half the time.)
+#define GF_XROW (GF_CHUNK * 4 + 16)  // bytes between the rows of a wave's staged activations
+
+template <int XR>
+__global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_streamed_kernel(GfArgs a, int k_tiles) {
+    constexpr int ROWS = 2 * XR;
+    extern __shared__ __align__(16) unsigned char smem[];
+    float* sums = reinterpret_cast<float*>(smem + GF_WAVES * ROWS * GF_XROW);        // [chunk][row][column]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const unsigned tile = a.cols * (BN_STREAM_TILE_COLS_F32 * 4);
+    const auto wb = bn_buffer(reinterpret_cast<const char*>(a.w) + (size_t)blockIdx.x * k_tiles * tile, k_tiles * tile);
+    const auto xb = bn_buffer(a.x, ((a.M - 1) * a.ldx + a.K) * 4);
+    const unsigned w_at = (g * a.cols + min(r, a.cols - 1)) * 16;
+    unsigned x_at[XR];
+#pragma unroll
+    for (int i = 0; i < XR; ++i) x_at[i] = (min(2 * i + (lane >> 5), a.M - 1) * a.ldx + (lane & 31) * 4) * 4;
+    unsigned char* xs = smem + wave * ROWS * GF_XROW;
+    unsigned char* park_at = xs + (lane >> 5) * GF_XROW + (lane & 31) * 16;
+    const unsigned char* read_at = xs + min(r, a.M - 1) * GF_XROW + g * 16;
+    f32x4 x[XR];
+    auto load_x = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < XR; ++i) x[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xb, x_at[i], c * (GF_CHUNK * 4), 0));
+    };
+    auto load_w = [&](f32x4 (&w)[GF_BLOCKS], int c) {
+        unsigned at = (unsigned)c * GF_BLOCKS * tile;
+#pragma unroll
+        for (int j = 0; j < GF_BLOCKS; ++j, at += tile)
+            w[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(wb, w_at, at, BN_BUFFER_NT));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto park = [&]() {
+#pragma unroll
+        for (int i = 0; i < XR; ++i) *reinterpret_cast<f32x4*>(park_at + 2 * i * GF_XROW) = x[i];
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](const f32x4 (&w)[GF_BLOCKS], int c) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int h = 0; h < GF_BLOCKS; h += 4) {
+            f32x4 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const f32x4*>(read_at + (h + j) * 64);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[h + j][e], v[j][e], acc, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (r < ROWS) *reinterpret_cast<f32x4*>(sums + ((size_t)c * ROWS + r) * 16 + 4 * g) = acc;   // columns 4 g .. 4 g + 3 of row r
+        __builtin_amdgcn_wave_barrier();
+    };
+    const int n_chunks = a.K / GF_CHUNK;
+    const int n = (n_chunks - wave + GF_WAVES - 1) / GF_WAVES;               // chunks of this wave: wave, wave + 8, ..
+    constexpr int D = GF_WAVES;
+    if (n == 1) {
+        f32x4 w[GF_BLOCKS];
+        load_x(wave);
+        load_w(w, wave);
+        park();
+        multiply(w, wave);
+    } else if (n > 1) {
+        int c = wave, left = n;
+        f32x4 p[GF_BLOCKS], q[GF_BLOCKS];
+        load_x(c);
+        load_w(p, c);
+        load_w(q, c + D);
+#pragma unroll 1
+        for (; left > 3; left -= 2, c += 2 * D) {
+            park();
+            load_x(c + D);
+            multiply(p, c);
+            load_w(p, c + 2 * D);
+            park();
+            load_x(c + 2 * D);
+            multiply(q, c + D);
+            load_w(q, c + 3 * D);
+        }
+        park();
+        load_x(c + D);
+        multiply(p, c);
+        if (left == 2) {
+            park();
+            multiply(q, c + D);
+        } else {
+            load_w(p, c + 2 * D);
+            park();
+            load_x(c + 2 * D);
+            multiply(q, c + D);
+            park();
+            multiply(p, c + 2 * D);
+        }
+    }
+    bn_lds_barrier();
+    if (tid >= ROWS * 16) return;
+    float tot = 0.f;
+#pragma unroll 8
+    for (int c = 0; c < n_chunks; ++c) tot += sums[(size_t)c * (ROWS * 16) + tid];
+    const int m = tid >> 4, col = tid & 15, n0 = blockIdx.x * a.cols;
+    if (a.glu) {                                                             // columns 0..7 of the tile are gates, 8..15 their ups
+        const float up = bn_lane_xor<8>(tot);
+        if (m < a.M && col < 8) a.y[(size_t)m * a.ldy + n0 / 2 + col] = bn_gate_act(tot, a.act) * up;
+    } else if (m < a.M && col < a.cols && n0 + col < a.N) {
+        a.y[(size_t)m * a.ldy + n0 + col] = tot;
     }
 }
 
@@ -268,16 +382,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(GfArgs a, int m_t
     }
 }
 
-// Matrices of less than 1 MB are read as any other operand: a model of such matrices stays in the L2s from step to step (a
-// decode step of a model of 64 columns 1.17 ms, 1.23 with non-temporal loads).
-#define GF_ONCE_BYTES (1 << 20)
-
 template <int MT>
 static int gf_launch_stream(const GfArgs& a, hipStream_t s) {
-    const bool once = (long long)a.N * a.K * 4 >= GF_ONCE_BYTES;
-    const dim3 grid((a.N + a.cols - 1) / a.cols), block(64 * GF_WAVES);
-    if (once) hipLaunchKernelGGL((gemm_f32_stream_kernel<MT, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((gemm_f32_stream_kernel<MT, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((gemm_f32_stream_kernel<MT>), dim3((a.N + a.cols - 1) / a.cols), dim3(64 * GF_WAVES), 0, s, a);
     return bn_launch_status();
 }
 
@@ -348,4 +455,44 @@ extern "C" int bn_gemm_f32(const void* x, const void* w, void* y, int M, int N, 
         case 5: return gf_launch_tile<32, 64>(a, s);
     }
     return BN_ERR_ARG;
+}
+
+// Columns a workgroup of the streaming kernels owns: the rows per tile that a streamed copy of W is best made with.
+extern "C" int bn_gemm_f32_stream_cols(int N) { return N < 1 ? 0 : gf_stream_cols(N); }
+
+#define GF_STREAMED_SMEM (150 * 1024)
+static int gf_streamed_xr(int M) { return M <= 2 ? 1 : M <= 4 ? 2 : M <= 8 ? 4 : 8; }
+static size_t gf_streamed_smem(int M, int K) {                               // the staged activations, a sum a chunk, row and column
+    const size_t rows = 2 * gf_streamed_xr(M);
+    return GF_WAVES * rows * GF_XROW + (size_t)(K / GF_CHUNK) * rows * 64;
+}
+
+// 1 if the kernel over a streamed copy takes the product: up to 16 rows, whole chunks whose sums fit into shared memory
+// (every K up to 10,496, and three times that at 8 rows), rows of activations that are whole 16-byte groups.
+extern "C" int bn_gemm_f32_streamed_supports(int M, int N, int K, int ldx, int tile_rows, const void* x) {
+    return M >= 1 && M <= 16 && N >= 1 && K >= GF_CHUNK && K % GF_CHUNK == 0 && gf_streamed_smem(M, K) <= GF_STREAMED_SMEM && ldx >= K &&
+           ldx % 4 == 0 && ldx <= 1 << 22 && tile_rows >= 1 && tile_rows <= BN_STREAM_TILE_ROWS && ((uintptr_t)x & 15) == 0;
+}
+
+// As bn_gemm_f32 over W's streamed copy (common.h) with that many rows a tile (16 with glu).
+extern "C" int bn_gemm_f32_streamed(const void* x, const void* tiles, void* y, int M, int N, int K, int ldx, int tile_rows, int ldy,
+                                    int glu, int act, hipStream_t s) {
+    if (!bn_gemm_f32_streamed_supports(M, N, K, ldx, tile_rows, x) || !tiles || !y || ((uintptr_t)tiles & 15)) return BN_ERR_ARG;
+    if (ldy < (glu ? N / 2 : N) || (glu && (N % 16 || tile_rows != 16)) || act < 0 || act >= BN_ACT_KINDS) return BN_ERR_ARG;
+    GfArgs a = {(const float*)x, (const float*)tiles, (float*)y, M, N, K, ldx, 0, ldy, tile_rows, glu ? 1 : 0, act};
+    auto go = [&](auto kernel) {
+        const size_t smem = gf_streamed_smem(M, K);
+        if (smem > 64 * 1024) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            if (e != hipSuccess) return (int)e;
+        }
+        hipLaunchKernelGGL(kernel, dim3((N + tile_rows - 1) / tile_rows), dim3(64 * GF_WAVES), smem, s, a, K / BN_STREAM_TILE_COLS_F32);
+        return bn_launch_status();
+    };
+    switch (gf_streamed_xr(M)) {
+        case 1: return go(gemm_f32_streamed_kernel<1>);
+        case 2: return go(gemm_f32_streamed_kernel<2>);
+        case 4: return go(gemm_f32_streamed_kernel<4>);
+        default: return go(gemm_f32_streamed_kernel<8>);
+    }
 }

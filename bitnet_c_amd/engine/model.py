@@ -96,7 +96,7 @@ class DecoderModel:
 
     def streamed_bytes(self) -> int:
         """Bytes that the streamed copies of all weight matrices take (taken or not)."""
-        if self.dtype != torch.bfloat16 or self.device.type != "cuda":
+        if self.device.type != "cuda":
             return 0
         return sum(l.stream_bytes() for l in self.linears())
 
@@ -107,7 +107,7 @@ class DecoderModel:
         and no other of its size or larger is tried, and so is a copy that the device has no room for.  Returns the bytes that the copies
         take."""
         matrices = self.linears()
-        applies = self.dtype == torch.bfloat16 and self.device.type == "cuda"
+        applies = self.device.type == "cuda"
         sizes = [l.stream_bytes() if applies else 0 for l in matrices]
         used, too_large = 0, None                # too_large: the size of a copy that found no place (smaller ones still may)
         for i in sorted(range(len(matrices)), key=lambda i: -sizes[i]):      # a stable order: equal sizes in model order

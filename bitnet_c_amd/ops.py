@@ -175,6 +175,9 @@ _SIGNATURES = {
     "gemm_f32": {
         "bn_gemm_f32_supports": [c_int, c_int, c_int, c_void_p],
         "bn_gemm_f32": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+        "bn_gemm_f32_stream_cols": [c_int],
+        "bn_gemm_f32_streamed_supports": [c_int, c_int, c_int, c_int, c_int, c_void_p],
+        "bn_gemm_f32_streamed": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     },
     "gemm_tiled": {
         "bn_gemm_tiled": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
@@ -460,11 +463,12 @@ def _tiled(x, w, out_dtype):
     return y
 
 
-def _f32_product(x, w, glu: bool = False, activation: str = "silu", form: int = 0):
+def _f32_product(x, w, glu: bool = False, activation: str = "silu", form: int = 0, streamed: Optional["StreamedWeight"] = None):
     """x . w^T in float32 on the float32 matrix instruction (gemm_f32.hip), or with glu act(gate) * up for w = gate and up
     rows interleaved in blocks of 8; None for weights that the kernels do not take (rows that are not whole 16-byte groups).
     Whether they do depends on the weights alone, and every form of the kernels has one order of summation, so a row's bits do
-    not depend on the step it comes in.  form: 0, by the sizes; the others are bn_gemm_f32's, for tests."""
+    not depend on the step it comes in.  form: 0, by the sizes; the others are bn_gemm_f32's, for tests.  streamed: w's
+    streamed copy, which products of up to 16 rows read instead (the same bits)."""
     M, K = x.shape
     N, ldw = w.shape[0], _rows(w, "w")
     if not _fn("gemm_f32", "bn_gemm_f32_supports")(N, K, ldw, w.data_ptr()):
@@ -474,6 +478,12 @@ def _f32_product(x, w, glu: bool = False, activation: str = "silu", form: int = 
         x = x.clone(memory_format=torch.contiguous_format)
         ldx = K
     y = torch.empty((M, N // 2 if glu else N), dtype=torch.float32, device=x.device)
+    if (streamed is not None and form == 0 and (not glu or streamed.tile_rows == STREAM_TILE_ROWS)
+            and _fn("gemm_f32", "bn_gemm_f32_streamed_supports")(M, N, K, ldx, streamed.tile_rows, x.data_ptr())):
+        tiles, _, rows = _weight_arg(w, streamed, "float32 product")
+        _check(_fn("gemm_f32", "bn_gemm_f32_streamed")(x.data_ptr(), tiles, y.data_ptr(), M, N, K, ldx, rows, y.shape[1], int(glu),
+                                                       _act(activation), _stream()), "gemm_f32(streamed)")
+        return y
     _check(_fn("gemm_f32", "bn_gemm_f32")(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, ldx, ldw, y.shape[1], int(glu),
                                           _act(activation), int(form), _stream()), "gemm_f32")
     return y
@@ -523,6 +533,15 @@ def skinny_supported(M: int, N: int, K: int, ldx: int, ldw: int) -> bool:
 # --------------------------------------------------------------------------------------
 STREAM_TILE_ROWS = _build.header_constant("BN_STREAM_TILE_ROWS")
 STREAM_TILE_COLS = _build.header_constant("BN_STREAM_TILE_COLS")
+STREAM_TILE_COLS_F32 = _build.header_constant("BN_STREAM_TILE_COLS_F32")
+
+
+F32_STREAM_CHUNK = _build.header_constant("GF_CHUNK", "gemm_f32.hip")      # float32 copies: K is whole chunks of this
+
+
+def stream_tile_cols(dtype) -> int:
+    """Columns of a tile of a streamed copy: 64 bytes of a row."""
+    return STREAM_TILE_COLS_F32 if dtype == torch.float32 else STREAM_TILE_COLS
 
 
 @dataclass
@@ -533,7 +552,8 @@ class StreamedWeight:
     A second copy beside the row-major matrix, which the products of many rows (the library's) and everything else keep
     reading: the kernels of up to 128 rows take it through their `streamed` argument and give the same result bit for
     bit, 5 to 15 % sooner.  The kernel of up to 16 rows gives a workgroup one row of tiles, so fewer than 16 rows a tile
-    are chosen where that spreads the tiles more evenly over the CUs (stream_tile_rows)."""
+    are chosen where that spreads the tiles more evenly over the CUs (stream_tile_rows).
+    A float32 matrix is kept in tiles of 16 columns (four to a lane's 16 bytes), for the float32 product of up to 16 rows."""
     tiles: torch.Tensor
     N: int
     K: int
@@ -547,20 +567,22 @@ class StreamedWeight:
         return self.tiles.numel() * self.tiles.element_size()
 
 
-def stream_tile_rows(N: int) -> int:
+def stream_tile_rows(N: int, dtype=torch.bfloat16) -> int:
     """The rows per tile with which a matrix of N rows is best streamed: the columns that the fused product of up to 16
     rows gives a workgroup over the row-major matrix (16, or fewer when that leaves the busiest CU at least 15 % fewer
-    columns: 12 for 6,144 rows on 256 CUs, 10 for 5,120)."""
+    columns: 12 for 6,144 rows on 256 CUs, 10 for 5,120); in float32 the columns that its streaming kernel gives one."""
+    if dtype == torch.float32:
+        return int(_fn("gemm_f32", "bn_gemm_f32_stream_cols")(int(N)))
     return int(_fn("skinny_gemm", "bn_skinny_gemm_fused_tile_cols")(int(N)))
 
 
 def stream_copy(w: torch.Tensor, tile_rows: Optional[int] = None) -> StreamedWeight:
-    """The streamed copy of w [N, K] (bf16, on the device; made there).  tile_rows None: stream_tile_rows(N); a matrix
-    with gate and up rows interleaved in blocks of 8 needs 16."""
+    """The streamed copy of w [N, K] (bf16 or float32, on the device; made there).  tile_rows None: stream_tile_rows(N); a
+    matrix with gate and up rows interleaved in blocks of 8 needs 16."""
     require_gpu()
-    _dev(w, "w", torch.bfloat16, 2)
+    _dev(w, "w", torch.float32 if w.dtype == torch.float32 else torch.bfloat16, 2)
     N, K = w.shape
-    R, C = (stream_tile_rows(N) if tile_rows is None else int(tile_rows)), STREAM_TILE_COLS
+    R, C = (stream_tile_rows(N, w.dtype) if tile_rows is None else int(tile_rows)), stream_tile_cols(w.dtype)
     if not 1 <= R <= STREAM_TILE_ROWS:
         raise KernelError(f"stream_copy: a tile has 1 to {STREAM_TILE_ROWS} rows, not {R}")
     nt, kt = (N + R - 1) // R, (K + C - 1) // C
@@ -568,16 +590,16 @@ def stream_copy(w: torch.Tensor, tile_rows: Optional[int] = None) -> StreamedWei
         padded = torch.zeros((nt * R, kt * C), dtype=w.dtype, device=w.device)
         padded[:N, :K] = w
         w = padded
-    # [nt, r, kt, g, 8] -> [nt, kt, g, r, 8]: lane r + 16 g of tile (nt, kt)
-    tiles = w.view(nt, R, kt, C // 8, 8).permute(0, 2, 3, 1, 4).contiguous().view(nt, kt, R * C)
+    # [nt, r, kt, g, C / 4] -> [nt, kt, g, r, C / 4]: lane r + 16 g of tile (nt, kt), 16 bytes
+    tiles = w.view(nt, R, kt, 4, C // 4).permute(0, 2, 3, 1, 4).contiguous().view(nt, kt, R * C)
     return StreamedWeight(tiles, N, K, R)
 
 
 def unstream(sw: StreamedWeight) -> torch.Tensor:
     """The row-major matrix [N, K] that a streamed copy holds."""
-    R, C = sw.tile_rows, STREAM_TILE_COLS
+    R, C = sw.tile_rows, stream_tile_cols(sw.tiles.dtype)
     nt, kt = sw.tiles.shape[:2]
-    return sw.tiles.view(nt, kt, C // 8, R, 8).permute(0, 3, 1, 2, 4).reshape(nt * R, kt * C)[:sw.N, :sw.K].contiguous()
+    return sw.tiles.view(nt, kt, 4, R, C // 4).permute(0, 3, 1, 2, 4).reshape(nt * R, kt * C)[:sw.N, :sw.K].contiguous()
 
 
 def _weight_arg(w: torch.Tensor, streamed: Optional[StreamedWeight], what: str, need_rows: int = 0):
@@ -591,9 +613,9 @@ def _weight_arg(w: torch.Tensor, streamed: Optional[StreamedWeight], what: str, 
     t = streamed.tiles
     R = streamed.tile_rows
     if (not isinstance(streamed, StreamedWeight) or (streamed.N, streamed.K) != tuple(w.shape) or t.device != w.device
-            or t.dtype != torch.bfloat16 or not t.is_contiguous() or t.dim() != 3 or not 1 <= R <= STREAM_TILE_ROWS
-            or tuple(t.shape) != ((streamed.N + R - 1) // R, (streamed.K + STREAM_TILE_COLS - 1) // STREAM_TILE_COLS,
-                                  R * STREAM_TILE_COLS)):
+            or t.dtype != w.dtype or not t.is_contiguous() or t.dim() != 3 or not 1 <= R <= STREAM_TILE_ROWS
+            or tuple(t.shape) != ((streamed.N + R - 1) // R, (streamed.K + stream_tile_cols(t.dtype) - 1) // stream_tile_cols(t.dtype),
+                                  R * stream_tile_cols(t.dtype))):
         raise KernelError(f"{what}: the streamed copy does not belong to w {tuple(w.shape)}")
     return t.data_ptr(), t.shape[1], R
 
@@ -632,7 +654,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, *, allow_library: O
     if x.dtype == torch.float32:
         if out_dtype != torch.float32:
             raise KernelError("linear: float32 inputs give float32 outputs")
-        y = _f32_product(x, w)
+        y = _f32_product(x, w, streamed=streamed)
         return y if y is not None else _tiled(x, w, torch.float32)
     if x.dtype != torch.bfloat16:
         raise KernelError(f"linear: unsupported dtype {x.dtype}")
@@ -789,7 +811,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, interleaved: bool = 
         return torch.empty((0, F), dtype=x.dtype, device=x.device)
     ldx, ldw = _rows(x, "x"), _rows(w_gate_up, "w_gate_up")
     if x.dtype == torch.float32 and interleaved:
-        y = _f32_product(x, w_gate_up, True, activation)
+        y = _f32_product(x, w_gate_up, True, activation, streamed=streamed)
         if y is not None:
             return y
     aligned = x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0

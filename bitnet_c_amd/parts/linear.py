@@ -28,13 +28,16 @@ class Linear:
     def stream_bytes(self) -> int:
         """Bytes that keep_streamed() would add (0 where the kernels that read a streamed copy do not apply)."""
         w = self.weight
-        if w is None or w.dtype != torch.bfloat16 or w.dim() != 2 or not w.is_cuda or w.shape[1] % 8:
+        if w is None or w.dim() != 2 or not w.is_cuda or w.dtype not in (torch.bfloat16, torch.float32):
             return 0
-        R, C = self.stream_tile_rows or ops.stream_tile_rows(w.shape[0]), ops.STREAM_TILE_COLS
-        return -(-w.shape[0] // R) * R * -(-w.shape[1] // C) * C * 2
+        if w.shape[1] % (8 if w.dtype == torch.bfloat16 else ops.F32_STREAM_CHUNK):
+            return 0
+        R, C = self.stream_tile_rows or ops.stream_tile_rows(w.shape[0], w.dtype), ops.stream_tile_cols(w.dtype)
+        return -(-w.shape[0] // R) * R * -(-w.shape[1] // C) * C * w.element_size()
 
     def keep_streamed(self, keep: bool = True) -> None:
-        """Makes (or drops) the streamed copy of the weight, which every product of up to 128 rows then reads."""
+        """Makes (or drops) the streamed copy of the weight, which every product of up to 128 rows (in float32, of up to 16) then
+        reads."""
         self.streamed = ops.stream_copy(self.weight, self.stream_tile_rows) if keep and self.stream_bytes() else None
 
     def __call__(self, x, out_dtype=None, rows: slice | None = None) -> torch.Tensor:

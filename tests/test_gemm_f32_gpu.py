@@ -97,3 +97,30 @@ def test_infinities_and_nan_stay_in_their_rows_and_columns():
         assert not fine[3].any() and not fine[4].any() and not fine[:, 5].any()
         fine[3], fine[4], fine[:, 5] = True, True, True
         assert fine.all()
+
+
+# rows: the edges of 2, 4, 8 and 16; K: one chunk of 128, fewer chunks than waves, a chunk a wave, one wave with two, two and
+# three a wave, five and six a wave; columns: one, no multiple of the tile's rows
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("N,K,R", [(1, 128, 16), (33, 896, 8), (40, 1024, 12), (16, 1152, 16), (30, 2048, 16), (17, 3072, 10), (24, 5632, 8)])
+def test_streamed_copies_give_the_same_bits(M, N, K, R):
+    ops = _ops()
+    x, w = _data(M, N, K, 7 * M + N)
+    xd, wd = x.cuda(), w.cuda()
+    sw = ops.stream_copy(wd, R)
+    assert torch.equal(ops.unstream(sw), wd)
+    assert torch.equal(ops.linear(xd, wd, streamed=sw), ops.linear(xd, wd))
+    wide = torch.full((M, K + 12), float("nan"), device="cuda")
+    wide[:, :K] = xd
+    assert torch.equal(ops.linear(wide[:, :K], wd, streamed=sw), ops.linear(xd, wd))
+    if R == 16 and N % 16 == 0:
+        assert torch.equal(ops.linear_swiglu(xd, wd, True, streamed=sw), ops.linear_swiglu(xd, wd, True))
+
+
+def test_streamed_copies_whose_sums_do_not_fit_are_not_read():
+    """At 9 to 16 rows shared memory holds the sums of 82 chunks: a longer K is read from the row-major matrix."""
+    ops = _ops()
+    x, w = _data(16, 16, 14336, 3)
+    xd, wd = x.cuda(), w.cuda()
+    for m in (8, 16):
+        assert torch.equal(ops.linear(xd[:m].contiguous(), wd, streamed=ops.stream_copy(wd)), ops.linear(xd[:m].contiguous(), wd)), m
