@@ -22,6 +22,26 @@ __global__ void embed_gather_kernel(float* __restrict__ x, const T* __restrict__
     for (int i = threadIdx.x; i < dim; i += blockDim.x) row[i] = to_f32(src[i]) * scale;
 }
 
+// The integers of a captured decode step one token on: fields of `rows` numbers each, in the order tokens, positions, sequence
+// index, lengths, wanted rows, order by length, slot ids, and behind them the longest length (engine/step.py).  The first n
+// rows are sequences: their tokens come from `tokens`, positions and lengths grow by one.  A launch in place of a copy from
+// pinned memory, an event and a copy of the tokens: 10 us less host work a step and one launch less on the device.
+__global__ __launch_bounds__(256) void step_advance_kernel(int* __restrict__ step, int rows, const int* __restrict__ tokens, int n) {
+    const int i = threadIdx.x;
+    if (i < n) {
+        step[i] = tokens[i];
+        step[rows + i] += 1;
+        step[3 * rows + i] += 1;
+    }
+    if (i == 0) step[7 * rows] += 1;
+}
+
+extern "C" int bn_step_advance(int* step, int rows, const int* tokens, int n, hipStream_t s) {
+    if (!step || !tokens || n < 1 || n > rows || rows > 256) return BN_ERR_ARG;
+    hipLaunchKernelGGL(step_advance_kernel, dim3(1), dim3(256), 0, s, step, rows, tokens, n);
+    return bn_launch_status();
+}
+
 // logits = cap * tanh(logits / cap), in place (src/transformer/logits.c:325-333)
 __global__ void softcap_kernel(float* __restrict__ x, size_t n, float cap, float inv) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -16,6 +16,7 @@ from __future__ import annotations
 from dataclasses import dataclass
 from typing import Dict, List, Sequence
 
+import numpy as np
 import torch
 
 from .. import ops
@@ -150,6 +151,24 @@ def _bucket(n: int) -> int:
     return DECODE_BUCKETS[-1]
 
 
+def _token_array(tokens):
+    """A list of plain integers as an array, or None for anything else (which is walked number by number)."""
+    if type(tokens) is not list:
+        return None
+    try:
+        a = np.array(tokens)
+    except (ValueError, OverflowError, TypeError):
+        return None
+    return a if a.ndim == 1 and a.dtype.kind == "i" else None
+
+
+def _tokens_inside(tokens, vocab: int) -> bool:
+    """Whether the tokens are known to lie in [0, vocab) without a look at each of them (a prompt of some thousand tokens
+    costs the host half a millisecond that way)."""
+    a = _token_array(tokens)
+    return a is not None and a.size > 0 and int(a.min()) >= 0 and int(a.max()) < vocab
+
+
 class _DecodeGraph:
     """A captured decode step for up to `rows` sequences.  The block tables are as wide as the engine's longest
     sequence and the split plan of attention follows the longest sequence of each replay through a device-side
@@ -157,7 +176,8 @@ class _DecodeGraph:
     capture because a sequence has grown.  The step's integers live in pinned buffers that are refilled
     before every replay; a row of the block tables is rewritten only when its sequence's pages have changed."""
 
-    N_FIELDS = 7            # tokens, positions, sequence index, lengths, wanted rows, order by length, slot ids
+    N_FIELDS = 7            # tokens, positions, sequence index, lengths, wanted rows, order by length, slot ids; the longest
+    #                         length behind them (ops.step_advance knows this order)
 
     def __init__(self, engine: "Engine", rows: int):
         self.rows, self.width = rows, engine.max_pages
@@ -173,6 +193,7 @@ class _DecodeGraph:
         self.dev_tables = torch.zeros(self.host_tables.shape, dtype=torch.int32, device=dev)
         self.row_keys = [None] * rows                         # (slot, version of its pages) that a table row holds
         self.tables_dirty = True
+        self.on_device = None                                 # (slots, lengths) that the device's integers describe
         self.copied = torch.cuda.Event()
         self.copied.record()
         f = [self.dev[k * rows:(k + 1) * rows] for k in range(self.N_FIELDS)]
@@ -232,6 +253,22 @@ class _DecodeGraph:
             self.dev_tables.copy_(self.host_tables, non_blocking=True)
             self.tables_dirty = False
         self.copied.record()
+
+    def advance(self, slots, lens_after, device_tokens, engine) -> bool:
+        """The step's integers where they follow from the last step's on this graph: the same sequences, one token longer
+        each, on the pages that the tables hold, with their tokens on the device.  One small kernel then stands for the
+        copy from pinned memory, its event and the copy of the tokens (and the order by length stays as it is); the host
+        waits for nothing.  False: fill and upload."""
+        if self.on_device is None or self.tables_dirty or not device_tokens.is_contiguous():
+            return False
+        last_slots, last_lens = self.on_device
+        if slots != last_slots or any(a != b + 1 for a, b in zip(lens_after, last_lens)):
+            return False
+        version, keys = engine.cache.slot_version, self.row_keys
+        if any(keys[r] != (s, version(s)) for r, s in enumerate(slots)):
+            return False
+        ops.step_advance(self.dev, self.rows, device_tokens)
+        return True
 
     def run(self):
         self.graph.replay()
@@ -315,7 +352,7 @@ class _PromptGraph:
         h[o[2]:o[3]] = 0
         r = 0
         for b, (n, p0) in enumerate(zip(n_new, pos0)):
-            h[o[1] + r:o[1] + r + n] = range(p0, p0 + n)
+            h[o[1] + r:o[1] + r + n] = np.arange(p0, p0 + n, dtype=np.int32)
             h[o[2] + r:o[2] + r + n] = b
             r += n
         h[o[3]:o[4]] = 0
@@ -467,9 +504,10 @@ class Engine:
             n = len(e.tokens)
             if n == 0:
                 raise StepError(f"slot {e.slot}: no tokens in this step")
-            for t in e.tokens:
-                if not (0 <= int(t) < self.vocab_size):
-                    raise StepError(f"slot {e.slot}: token {t} is outside [0, {self.vocab_size})")
+            if n < 32 or not _tokens_inside(e.tokens, self.vocab_size):
+                for t in e.tokens:
+                    if not (0 <= int(t) < self.vocab_size):
+                        raise StepError(f"slot {e.slot}: token {t} is outside [0, {self.vocab_size})")
             if have + n > self.max_seq_len:
                 raise StepError(f"slot {e.slot}: {have} + {n} tokens exceed the sequence limit {self.max_seq_len}")
             for w in e.want:
@@ -609,7 +647,11 @@ class Engine:
 
     def _step_prompt_graph(self, entries, slots, n_new, pos0):
         g = self._prompt_graph_for(self._prompt_key(entries, n_new))
-        tokens = [int(t) for e in entries for t in e.tokens]
+        arrays = [_token_array(e.tokens) for e in entries]
+        if any(a is None for a in arrays):
+            tokens = [int(t) for e in entries for t in e.tokens]
+        else:
+            tokens = np.concatenate(arrays)
         want, row = [], 0
         for e, n in zip(entries, n_new):
             want += [row + int(w) for w in e.want]
@@ -640,10 +682,13 @@ class Engine:
         B = len(entries)
         lens_after = [p + 1 for p in pos0]
         g = self._graph_for(_bucket(B))
-        g.fill(slots, [int(e.tokens[0]) for e in entries], lens_after, self)
-        g.upload()
-        if device_tokens is not None:
-            g.tokens[:B].copy_(device_tokens)            # behind the upload, before the replay
+        if device_tokens is None or not g.advance(slots, lens_after, device_tokens, self):
+            g.on_device = None
+            g.fill(slots, [int(e.tokens[0]) for e in entries], lens_after, self)
+            g.upload()
+            if device_tokens is not None:
+                g.tokens[:B].copy_(device_tokens)        # behind the upload, before the replay
+        g.on_device = list(slots), lens_after
         logits = g.run()
         rows = [i for i, e in enumerate(entries) for _ in e.want]
         if rows == list(range(B)):

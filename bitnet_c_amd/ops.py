@@ -29,6 +29,7 @@ class KernelError(RuntimeError):
 
 _SIGNATURES = {
     "elementwise": {
+        "bn_step_advance": [c_void_p, c_int, c_void_p, c_int, c_void_p],
         "bn_embed_gather": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_void_p],
         "bn_softcap": [c_void_p, c_longlong, c_float, c_void_p],
         "bn_gather_rows": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
@@ -302,6 +303,17 @@ def _act(name: str) -> int:
 # --------------------------------------------------------------------------------------
 # row-wise kernels
 # --------------------------------------------------------------------------------------
+
+def step_advance(step: torch.Tensor, rows: int, tokens: torch.Tensor) -> None:
+    """The integers of a captured decode step of up to `rows` sequences (engine/step.py: seven fields of `rows` int32, then
+    the longest length) one token on: the sequences' new tokens (int32, on the device), positions and lengths one more."""
+    require_gpu()
+    _dev(step, "step", torch.int32, 1)
+    _dev(tokens, "tokens", torch.int32, 1)
+    if not step.is_contiguous() or step.numel() < 7 * rows + 1 or not tokens.is_contiguous():
+        raise KernelError(f"step_advance: {step.numel()} integers do not hold the fields of {rows} rows")
+    _check(_fn("elementwise", "bn_step_advance")(step.data_ptr(), int(rows), tokens.data_ptr(), tokens.numel(), _stream()), "step_advance")
+
 
 def embed_gather(table: torch.Tensor, tokens: torch.Tensor, scale: float = 1.0) -> torch.Tensor:
     """float32 rows of the embedding table for int32 token ids, times `scale` (an architecture's embedding
