@@ -106,6 +106,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t bn_buffer(const void* p, unsig
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
 }
 
+// A load of 16 bytes a lane from a buffer straight into shared memory: lane l's bytes go to lds + 16 l (lds the same in every
+// lane).  The wave's count of outstanding loads covers it.
+__device__ __forceinline__ void bn_load_to_lds(__amdgpu_buffer_rsrc_t b, void* lds, unsigned lane_offset, unsigned offset) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (__attribute__((address_space(3))) void*)lds, 16, lane_offset, offset, 0, 0);
+}
+
 // Reductions over a wave as a butterfly: every lane adds the lane 32, 16, 8, 4, 2 and 1 away, in that order.  The two long
 // steps swap halves and rows (v_permlane32_swap, v_permlane16_swap), the short ones are data-parallel-primitive moves inside
 // a row of 16; through shared memory's crossbar (__shfl_xor) every step waits some 120 cycles for the one before it, a third

@@ -17,9 +17,10 @@
 // vector kernel that walked K in one chain (gemm_tiled.hip) took 325 on the average of a layer's products, whatever the rows
 // up to 16.  Its loads of W are plain: two of them take the halves of a line, and non-temporal ones were slower (11,264 x 2,048
 // at 8 rows 25 -> 26 us, 32,000 x 2,048 59 -> 65).
-// gemm_f32_tile_kernel, more rows: bound by the instruction (157 TFLOP/s on this chip, 32 cycles each on a SIMD).  5,136 x
-// 11,264 x 2,048 2.02 ms (117 TFLOP/s), 2,048 x 2,048 x 5,632 0.40 ms; the matrix unit is busy four fifths of a round, the
-// rest is the last round's empty CUs.  The vector kernel did 27 TFLOP/s.
+// gemm_f32_dma_kernel, more rows, K of whole steps of 32: bound by the instruction (157 TFLOP/s on this chip, 32 cycles each on
+// a SIMD).  5,136 x 11,264 x 2,048 1.72 ms (138 TFLOP/s), 5,136 x 2,048 x 5,632 0.91 ms (131), 5,136 x 2,048 x 2,048 0.35 ms (124;
+// the last round's empty CUs).
+// gemm_f32_tile_kernel, other K: the same products staged through registers (117, 109 and 106 TFLOP/s there).
 #include "common.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -382,6 +383,150 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(GfArgs a, int m_t
     }
 }
 
+// Tiles for K of whole steps (K % 32 == 0).  Float32 matrix instructions and vector instructions share the SIMD's
+// multipliers, so what the loop above spends on staging (addresses, tests, registers on their way to shared memory: one vector
+// instruction for every matrix instruction) it takes from the products.  Here memory goes straight into shared memory
+// (buffer loads with an LDS destination: a lane's offset is a constant, the step's lies in a scalar register), rows past the
+// matrix lie past the buffer's end, and a chunk's first product starts from a constant zero.  A staged row is 128 bytes, chunk
+// c of 16 bytes of row r at c ^ (r / 2 % 8), which keeps the sixteen lanes that shared memory serves together on different banks.
+// NB buffers, NB - 1 steps ahead: two where a CU holds several workgroups, four where a launch gives it one or two, whose
+// steps would each wait for memory.
+template <int BM, int BN, int NB>
+__global__ __launch_bounds__(256, 2) void gemm_f32_dma_kernel(GfArgs a, int m_tiles, int n_tiles) {
+    constexpr int MT = BM / 32, NT = BN / 32;                    // 16 x 16 tiles of a wave
+    constexpr int XI = BM / 32, WI = BN / 32;                    // staging loads of a wave and step, 8 rows each
+    // buffers of their own names: the compiler then knows which loads a read of shared memory has to wait for
+    __shared__ __align__(1024) unsigned char b0[(BM + BN) * 128], b1[(BM + BN) * 128];
+    __shared__ __align__(1024) unsigned char b2[NB == 4 ? (BM + BN) * 128 : 16], b3[NB == 4 ? (BM + BN) * 128 : 16];
+    static_assert(NB == 2 || NB == 4, "a chunk is four steps");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    int id = blockIdx.x;                                         // as in gemm_f32_tile_kernel
+    const int total = m_tiles * n_tiles;
+    {
+        const int per = total / 8, rest = total % 8, xcd = id % 8, at = id / 8;
+        id = xcd * per + min(xcd, rest) + at;
+    }
+    const int band = id / (8 * n_tiles), in_band = id - band * 8 * n_tiles;
+    const int band_rows = min(8, m_tiles - band * 8);
+    const int m0 = (band * 8 + in_band % band_rows) * BM, n0 = (in_band / band_rows) * BN;
+    const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
+
+    f32x4 acc[NT][MT], tot[NT][MT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) tot[i][j] = 0.f;
+
+    const auto xb = bn_buffer(a.x + (size_t)m0 * a.ldx, ((min(BM, a.M - m0) - 1) * a.ldx + a.K) * 4);
+    const auto wb = bn_buffer(a.w + (size_t)n0 * a.ldw, ((min(BN, a.N - n0) - 1) * a.ldw + a.K) * 4);
+    // load i of a wave: rows 32 i + 8 wave .. + 7, a lane the 16 bytes at slot lane % 8 of row lane / 8
+    const int sr = 8 * wave + (lane >> 3), sc = ((lane & 7) ^ ((sr >> 1) & 7)) * 16;
+    unsigned xo[XI], wo[WI];
+#pragma unroll
+    for (int i = 0; i < XI; ++i) xo[i] = (sr + 32 * i) * a.ldx * 4 + sc;
+#pragma unroll
+    for (int i = 0; i < WI; ++i) wo[i] = (sr + 32 * i) * a.ldw * 4 + sc;
+    auto stage = [&](unsigned char* to, int s) {                 // A's rows, then W's
+#pragma unroll
+        for (int i = 0; i < XI; ++i) bn_load_to_lds(xb, to + (32 * i + 8 * wave) * 128, xo[i], s * (GF_BK * 4));
+#pragma unroll
+        for (int i = 0; i < WI; ++i) bn_load_to_lds(wb, to + (BM + 32 * i + 8 * wave) * 128, wo[i], s * (GF_BK * 4));
+    };
+    // block b of a row: chunk 4 b + g, at (4 b + g) ^ (row / 2 % 8) (a tile's rows begin at multiples of 16)
+    const int at0 = r * 128 + ((g ^ (r >> 1)) << 4), at1 = r * 128 + (((4 + g) ^ (r >> 1)) << 4);
+    f32x4 wv[2][NT], xv[2][MT];
+    auto read = [&](const unsigned char* from, int b) {
+        const int at = b ? at1 : at0;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) wv[b][i] = *reinterpret_cast<const f32x4*>(from + (BM + wn + 16 * i) * 128 + at);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) xv[b][j] = *reinterpret_cast<const f32x4*>(from + (wm + 16 * j) * 128 + at);
+    };
+    auto multiply = [&](int b, auto first) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int j = 0; j < MT; ++j) {
+                    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[b][i][e], xv[b][j][e], decltype(first)::value && e == 0 ? zero : acc[i][j], 0, 0, 0);
+                }
+    };
+    const int steps = a.K / GF_BK;
+    // A step asks for the rows of NB - 1 steps on, into the buffer that the step before it has left, and multiplies its own;
+    // past its barrier the next step's rows are there.  (The last steps ask for the last rows again, into buffers that nobody
+    // reads any more.)
+    constexpr int AHEAD = (NB - 2) * (XI + WI);                  // loads that may still be on their way behind a step
+    auto arrived = [&]() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(AHEAD) : "memory"); };
+    auto step = [&](const unsigned char* now, unsigned char* next, int s, auto first) {
+        stage(next, min(s + NB - 1, steps - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        read(now, 0);
+        read(now, 1);
+        multiply(0, first);
+        multiply(1, gf_false());
+        arrived();
+    };
+    auto fold = [&]() {
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) tot[i][j] += acc[i][j];
+    };
+    // step k of a chunk, k = 0..3
+    auto step0 = [&](int s) { step(b0, NB == 2 ? b1 : b3, s, gf_true()); };
+    auto step1 = [&](int s) { step(b1, b0, s, gf_false()); };
+    auto step2 = [&](int s) { step(NB == 2 ? b0 : b2, b1, s, gf_false()); };
+    auto step3 = [&](int s) { step(NB == 2 ? b1 : b3, NB == 2 ? b0 : b2, s, gf_false()); };
+    stage(b0, 0);
+    if (NB == 4) {
+        stage(b1, min(1, steps - 1));
+        stage(b2, min(2, steps - 1));
+    }
+    arrived();
+    int s = 0;
+#pragma unroll 1
+    for (; s + 4 <= steps; s += 4) {
+        step0(s);
+        step1(s + 1);
+        step2(s + 2);
+        step3(s + 3);
+        fold();
+    }
+    if (s < steps) {
+        step0(s);
+        if (s + 1 < steps) step1(s + 1);
+        if (s + 2 < steps) step2(s + 2);
+        fold();
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // nothing is on its way into shared memory when the wave ends
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        const int n = n0 + wn + 16 * i + 4 * g;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const int m = m0 + wm + 16 * j + r;
+            if (a.glu) {                                         // lanes with g < 2 hold gates, the lane 32 further their ups
+                f32x4 up;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) up[e] = __shfl_xor(tot[i][j][e], 32, BN_WAVE);
+                if (g < 2 && m < a.M && n < a.N) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        a.y[(size_t)m * a.ldy + (n0 + wn + 16 * i) / 2 + 4 * g + e] = bn_gate_act(tot[i][j][e], a.act) * up[e];
+                }
+            } else if (m < a.M) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < a.N) a.y[(size_t)m * a.ldy + n + e] = tot[i][j][e];
+            }
+        }
+    }
+}
+
 template <int MT>
 static int gf_launch_stream(const GfArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((gemm_f32_stream_kernel<MT>), dim3((a.N + a.cols - 1) / a.cols), dim3(64 * GF_WAVES), 0, s, a);
@@ -392,6 +537,14 @@ template <int BM, int BN>
 static int gf_launch_tile(const GfArgs& a, hipStream_t s) {
     const int mt = (a.M + BM - 1) / BM, nt = (a.N + BN - 1) / BN;
     hipLaunchKernelGGL((gemm_f32_tile_kernel<BM, BN>), dim3(mt * nt), dim3(256), 0, s, a, mt, nt);
+    return bn_launch_status();
+}
+
+template <int BM, int BN, int NB>
+static int gf_launch_dma(const GfArgs& a, hipStream_t s) {
+    const int mt = (a.M + BM - 1) / BM, nt = (a.N + BN - 1) / BN;
+    if (a.K % GF_BK) return BN_ERR_ARG;
+    hipLaunchKernelGGL((gemm_f32_dma_kernel<BM, BN, NB>), dim3(mt * nt), dim3(256), 0, s, a, mt, nt);
     return bn_launch_status();
 }
 
@@ -409,17 +562,22 @@ static int gf_stream_cols(int N) {
     return best;
 }
 
-// The tile kernel's form with the least time for the busiest CU, which is the longer of one tile's own chain of steps and of
-// all its tiles' instructions.  ns a step of 32 columns of K, measured at 2,048 columns with one tile a CU and with many: 128 x
-// 128 2,400 and 2,090 a tile, 64 x 128 1,360 and 1,060, 64 x 64 790 and 520, 32 x 64 520 and 290.
-static int gf_tile_form(int M, int N) {
-    static const int bm[4] = {128, 64, 64, 32}, bn[4] = {128, 128, 64, 64}, alone[4] = {2400, 1360, 790, 520}, many[4] = {2090, 1060, 520, 290};
+// The tile kernels' form with the least time for the busiest CU.  Whole steps (K % 32 == 0): a launch's first tile on a CU costs
+// more than the ones beside it, ns a step of 32 columns of K with n tiles a CU 200 + 478 n of 64 x 64, 150 + 255 n of 32 x 64, 130
+// + 130 n of 32 x 32 (fitted at 2,048 columns, n = 1 to 222, within 5 %).  us at 199 rows, these three: 3,072 x 2,048 45 / 41 / 33,
+// 2,048 x 5,632 109 / 64 / 58, 11,264 x 2,048 110 / 91 / 93; at 5,136 rows 11,264 x 2,048 1,722 / 1,811 / 1,860; the kernel that
+// stages through registers took 54, 82, 126 and 2,025.  Other K, that kernel: the longer of one tile's own chain of steps and of
+// all its tiles' instructions, 128 x 128 2,400 and 2,090 a tile, 64 x 128 1,360 and 1,060, 64 x 64 790 and 520, 32 x 64 520 and 290.
+static int gf_tile_form(int M, int N, int K) {
+    static const int bm[7] = {128, 64, 64, 32, 64, 32, 32}, bn[7] = {128, 128, 64, 64, 64, 64, 32};
+    static const int alone[4] = {2400, 1360, 790, 520}, many[7] = {2090, 1060, 520, 290, 478, 255, 130}, first[3] = {200, 150, 130};
+    const bool whole = K % GF_BK == 0;
     int best = 0;
     long long cost = -1;
-    for (int i = 0; i < 4; ++i) {
+    for (int i = whole ? 4 : 0; i < (whole ? 7 : 4); ++i) {
         const long long tiles = (long long)((M + bm[i] - 1) / bm[i]) * ((N + bn[i] - 1) / bn[i]);
         const long long per_cu = (tiles + GF_CUS - 1) / GF_CUS, t = per_cu * many[i];
-        const long long c = t > alone[i] ? t : alone[i];
+        const long long c = whole ? t + first[i - 4] : t > alone[i] ? t : alone[i];
         if (cost < 0 || c < cost) { best = i; cost = c; }
     }
     return 2 + best;
@@ -431,10 +589,13 @@ extern "C" int bn_gemm_f32_supports(int N, int K, int ldw, const void* w) {
     return N > 0 && K > 0 && K % 4 == 0 && ldw % 4 == 0 && ldw >= K && ldw <= (1 << 22) && ((uintptr_t)w & 15) == 0;
 }
 
-// form 0: by the sizes; 1: streaming; 2 .. 5: tiles of 128 x 128, 64 x 128, 64 x 64, 32 x 64 (every form gives the same bits).
-// Streaming up to 16 rows; up to 64 while the rows' 16-row tiles times the column tiles of a CU stay few, since every
-// workgroup of it reads all rows (us at 64 rows, streaming against tiles: 2,048 x 5,632 54 / 82, 4,096 x 14,336 139 / 202,
-// 11,264 x 2,048 60 / 54, 28,672 x 4,096 255 / 164; at 20 rows 6,144 x 4,096 43 / 61, 32,000 x 2,048 86 / 54).
+// form 0: by the sizes; 1: streaming; 2 .. 5: tiles of 128 x 128, 64 x 128, 64 x 64, 32 x 64; 6 .. 8, for whole steps: tiles of
+// 64 x 64, 32 x 64, 32 x 32 straight into shared memory (every form gives the same bits).
+// Streaming up to 16 rows.  Whole steps: up to 32 while a CU has one tile of 16 columns, since every workgroup of it reads all
+// rows (us at 17 / 32 rows, streaming against tiles of 32 x 32: 2,048 x 2,048 13.6 / 14.9 against 17, 2,048 x 5,632 28 / 33 against
+// 38, 4,096 x 14,336 83 / 93 against 106, 11,264 x 2,048 34 / 40 against 26 / 29; at 33 rows 2,048 x 2,048 19.8 against 17.5).  Other K:
+// up to 64 while the rows' 16-row tiles times the column tiles of a CU stay few (at 64 rows, against tiles through registers,
+// 2,048 x 5,632 54 / 82, 11,264 x 2,048 60 / 54, 28,672 x 4,096 255 / 164; at 20 rows 6,144 x 4,096 43 / 61, 32,000 x 2,048 86 / 54).
 extern "C" int bn_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K, int ldx, int ldw, int ldy, int glu, int act,
                            int form, hipStream_t s) {
     if (M <= 0 || !bn_gemm_f32_supports(N, K, ldw, w) || ldx % 4 || ldx < K || ldx > (1 << 22) || ((uintptr_t)x & 15)) return BN_ERR_ARG;
@@ -442,8 +603,10 @@ extern "C" int bn_gemm_f32(const void* x, const void* w, void* y, int M, int N, 
     if ((long long)((M + 31) / 32) * ((N + 63) / 64) > 0x7fffffffLL) return BN_ERR_ARG;
     GfArgs a = {(const float*)x, (const float*)w, (float*)y, M, N, K, ldx, ldw, ldy, 16, glu ? 1 : 0, act};
     const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-    if (form == 0)
-        form = M <= 16 || (M <= 64 && (long long)mt * N <= 6LL * 16 * GF_CUS) ? 1 : gf_tile_form(M, N);
+    if (form == 0) {
+        const bool streams = K % GF_BK == 0 ? M <= 32 && N <= 16 * GF_CUS : M <= 64 && (long long)mt * N <= 6LL * 16 * GF_CUS;
+        form = M <= 16 || streams ? 1 : gf_tile_form(M, N, K);
+    }
     switch (form) {
         case 1:
             if (M > 64) return BN_ERR_ARG;
@@ -453,6 +616,9 @@ extern "C" int bn_gemm_f32(const void* x, const void* w, void* y, int M, int N, 
         case 3: return gf_launch_tile<64, 128>(a, s);
         case 4: return gf_launch_tile<64, 64>(a, s);
         case 5: return gf_launch_tile<32, 64>(a, s);
+        case 6: return gf_launch_dma<64, 64, 2>(a, s);
+        case 7: return gf_launch_dma<32, 64, 4>(a, s);
+        case 8: return gf_launch_dma<32, 32, 4>(a, s);
     }
     return BN_ERR_ARG;
 }

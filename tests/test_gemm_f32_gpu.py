@@ -99,6 +99,35 @@ def test_infinities_and_nan_stay_in_their_rows_and_columns():
         assert fine.all()
 
 
+# the forms that stage straight into shared memory (K of whole steps of 32): rows and columns at the edges of tiles of 32 and
+# 64, one row and one column; K: one step, two, three and four (a chunk), chunks with one, two and three steps behind them,
+# fewer and more steps than the four buffers; rows that lie further apart than they are long, NaN between and behind them
+@pytest.mark.parametrize("M,N", [(1, 1), (31, 33), (32, 64), (64, 16), (65, 130), (129, 48), (300, 257)])
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 192, 224, 256, 1056, 2048])
+def test_forms_straight_into_shared_memory(M, N, K):
+    ops = _ops()
+    x, w = _data(M, N, K, M + 3 * N + K)
+    wide, tall = torch.full((M + 1, K + 8), float("nan"), device="cuda"), torch.full((N + 1, K + 4), float("nan"), device="cuda")
+    wide[:M, :K], tall[:N, :K] = x.cuda(), w.cuda()
+    xd, wd = wide[:M, :K], tall[:N, :K]
+    want = ops._f32_product(xd, wd, form=4)
+    assert torch.all((want.cpu().double() - x.double() @ w.double().t()).abs() <= _bound(x, w))
+    for form in (6, 7, 8, 0):
+        assert torch.equal(ops._f32_product(xd, wd, form=form), want), form
+    if N % 16 == 0:
+        glu = ops._f32_product(xd, wd, True, "silu", form=4)
+        for form in (6, 7, 8):
+            assert torch.equal(ops._f32_product(xd, wd, True, "silu", form=form), glu), form
+
+
+def test_forms_of_whole_steps_refuse_other_widths():
+    ops = _ops()
+    x, w = _data(40, 40, 100, 1)
+    for form in (6, 7, 8):
+        with pytest.raises(ops.KernelError):
+            ops._f32_product(x.cuda(), w.cuda(), form=form)
+
+
 # rows: the edges of 2, 4, 8 and 16; K: one chunk of 128, fewer chunks than waves, a chunk a wave, one wave with two, two and
 # three a wave, five and six a wave; columns: one, no multiple of the tile's rows
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 9, 16])
