@@ -90,6 +90,8 @@ struct MfmaArgs {
     const int* max_len;
 };
 
+// sixteen bytes that the launch reads once: a decode step's cached keys and values
+__device__ __forceinline__ bf16x8 ld16_once(const bf16* p) { return __builtin_bit_cast(bf16x8, bn_load_once(p)); }
 __device__ __forceinline__ bf16x8 ld16(const bf16* p) {
     return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
 }
@@ -184,11 +186,11 @@ __device__ __forceinline__ void load_block(const bf16* __restrict__ kbase, const
                                            bf16x8 (&ka)[HS / 32][2], bf16x8 (&va)[HS / 16], int lane) {
 #pragma unroll
     for (int c = 0; c < HS / 32; ++c) {
-        ka[c][0] = ld16(kbase + (2 * c) * 512 + lane * 8);
-        ka[c][1] = ld16(kbase + (2 * c + 1) * 512 + lane * 8);
+        ka[c][0] = ld16_once(kbase + (2 * c) * 512 + lane * 8);
+        ka[c][1] = ld16_once(kbase + (2 * c + 1) * 512 + lane * 8);
     }
 #pragma unroll
-    for (int t = 0; t < HS / 16; ++t) va[t] = ld16(vbase + t * 512 + lane * 8);
+    for (int t = 0; t < HS / 16; ++t) va[t] = ld16_once(vbase + t * 512 + lane * 8);
 }
 
 template <int HS, int NT, bool need_mask>

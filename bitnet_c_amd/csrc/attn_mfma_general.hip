@@ -54,6 +54,8 @@ struct GenArgs {
     int keep_first;           // with a window: the first keep_first positions stay visible however far back they are
 };
 
+// sixteen bytes that the launch reads once: a decode step's cached keys and values
+__device__ __forceinline__ bf16x8 ag_ld16_once(const bf16* p) { return __builtin_bit_cast(bf16x8, bn_load_once(p)); }
 __device__ __forceinline__ bf16x8 ag_ld16(const bf16* p) {
     return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
 }
@@ -369,7 +371,7 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
         const int page = a.block_table[(size_t)seq * a.bt_stride + kb / BN_PAGE];
         const bf16* kbase = a.k_pages + (((size_t)page * a.Hkv + kvh) * BN_PAGE + kb % BN_PAGE + krow) * HS + 8 * g;
 #pragma unroll
-        for (int c = 0; c < DC; ++c) { kn0[c] = ag_ld16(kbase + 32 * c); kn1[c] = ag_ld16(kbase + 4 * HS + 32 * c); }
+        for (int c = 0; c < DC; ++c) { kn0[c] = ag_ld16_once(kbase + 32 * c); kn1[c] = ag_ld16_once(kbase + 4 * HS + 32 * c); }
     };
     const int first_block = k_lo & ~31, last_block = ((k_hi - 1) / 32) * 32;
     auto leap = [&](int kb) { return kb >= keep && kb < first_block ? first_block : kb; };
@@ -389,7 +391,7 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
         }
         bf16x8 va[DT];
 #pragma unroll
-        for (int t = 0; t < DT; ++t) va[t] = ag_ld16(vbase + (size_t)t * 16 * BN_PAGE);
+        for (int t = 0; t < DT; ++t) va[t] = ag_ld16_once(vbase + (size_t)t * 16 * BN_PAGE);
         float s[8];
         ag_scores(s, st0, st1, scale2, bias, ba, bb, qpos, kb + 8 * g);
         float mx = -INFINITY;
