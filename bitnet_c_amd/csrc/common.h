@@ -155,6 +155,13 @@ __device__ __forceinline__ float wave_max(float v) {
     return bn_wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
+// A thread's sum of squares over its groups of four numbers of a row (k: the group's number): one chain, every rounding written
+// out, so that kernels which norm the same row form the same bits.
+template <typename V> __device__ __forceinline__ float bn_add_squares(float ss, const V& v, int k) {
+    ss = k == 0 ? __builtin_fmaf(v.x, v.x, __fmul_rn(v.y, v.y)) : __builtin_fmaf(v.y, v.y, __builtin_fmaf(v.x, v.x, ss));
+    return __builtin_fmaf(v.w, v.w, __builtin_fmaf(v.z, v.z, ss));
+}
+
 // A barrier that orders shared memory alone: loads and stores of global memory stay in flight across it (__syncthreads waits
 // for a row's stores to be acknowledged, a trip to memory).
 __device__ __forceinline__ void bn_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }

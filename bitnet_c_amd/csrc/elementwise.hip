@@ -135,7 +135,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_row_kernel(float* __restrict_
         const int i = (k * 256 + threadIdx.x) * 4;
         if (i < dim) {
             if (write_back) *reinterpret_cast<float4*>(xr + i) = v[k];
-            ss += v[k].x * v[k].x; ss += v[k].y * v[k].y; ss += v[k].z * v[k].z; ss += v[k].w * v[k].w;
+            ss = bn_add_squares(ss, v[k], k);
         }
     }
     ss = block_sum(ss, scratch);

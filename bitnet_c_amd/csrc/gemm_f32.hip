@@ -22,6 +22,7 @@
 // the last round's empty CUs).
 // gemm_f32_tile_kernel, other K: the same products staged through registers (117, 109 and 106 TFLOP/s there).
 #include "common.h"
+#include <type_traits>
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -39,6 +40,9 @@ struct GfArgs {
     int cols;                        // columns a workgroup of the streaming kernel owns (<= 16)
     int glu;                         // rows of W are gate and up rows in turns of 8; y[M, N / 2] = act(gate) * up
     int act;
+    int add;                         // y += the product (kernels of up to 16 rows, no glu)
+    const float* norm_w;             // rows of x are normed on their way in: x * scale * norm_w; null: as they are
+    float eps;
 };
 
 struct gf_true { static constexpr bool value = true; };
@@ -50,12 +54,67 @@ __device__ __forceinline__ f32x4 gf_load(const float* p, bool ok) {
     return v;
 }
 
-// MT row tiles of 16 share a wave's registers of W
-template <int MT>
+// A norm in front of a product of few rows: every workgroup sums the squares of the rows itself, while its first weights are on
+// their way, instead of a kernel of its own that the product would wait for (4.4 us a launch; the rows come from the L2).  The
+// sums, their order and the factor are add_rmsnorm_row_kernel's (elementwise.hip): 256 threads take a row in groups of four, a
+// wave's sums are added as a butterfly, the four waves' in order; here the halves of the workgroup take every other row.
+// NR: rows a half takes; NV: groups a thread and row.  parts: [2 NR][4], a wave's sum of a row.
+//   us in a decode step of Llama, 2,048 columns, one row: norm 4.4 + 11,264 x 2,048 16.4 -> 16.7, norm 4.4 + 3,072 x 2,048 6.9 -> 6.9;
+//   whole calls, prompt of 199 and 16 steps 14.3 -> 13.7 ms, eight prompts and 8 steps 55.3 -> 54.8.  Up to 8 rows: beyond that a
+//   workgroup reads more of the rows than of its weights, and the rows' registers are not there (GF_NORM_LOADS).
+__device__ __forceinline__ float gf_norm_scale(const GfArgs& a, const float* parts, int row) {
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ss += parts[row * 4 + i];
+    return 1.0f / sqrtf(ss / (float)a.K + a.eps);
+}
+template <int NR, int NV> struct GfNorm {
+    f32x4 v[NR][NV], w[NV];
+    __device__ __forceinline__ void load(const GfArgs& a, int tid) {
+        const int t = tid & 255, half = __builtin_amdgcn_readfirstlane(tid >> 8);
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+#pragma unroll
+            for (int k = 0; k < NV; ++k)
+                v[i][k] = *reinterpret_cast<const f32x4*>(a.x + (size_t)min(half + 2 * i, a.M - 1) * a.ldx + min((k * 256 + t) * 4, a.K - 4));
+#pragma unroll
+        for (int k = 0; k < NV; ++k) w[k] = *reinterpret_cast<const f32x4*>(a.norm_w + min((k * 256 + t) * 4, a.K - 4));
+    }
+    __device__ __forceinline__ void sum(const GfArgs& a, int tid, float* parts) {
+        const int t = tid & 255, half = __builtin_amdgcn_readfirstlane(tid >> 8), wave = (tid >> 6) & 3;
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            float ss = 0.f;
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                const float s = bn_add_squares(ss, v[i][k], k);
+                if ((k * 256 + t) * 4 < a.K) ss = s;
+            }
+            ss = wave_sum(ss);
+            if ((tid & 63) == 0) parts[(half + 2 * i) * 4 + wave] = ss;
+        }
+    }
+    // the normed rows to shared memory, row_bytes apart (behind a barrier after sum)
+    __device__ __forceinline__ void store(const GfArgs& a, int tid, const float* parts, unsigned char* rows, int row_bytes) {
+        const int t = tid & 255, half = __builtin_amdgcn_readfirstlane(tid >> 8);
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const float scale = gf_norm_scale(a, parts, half + 2 * i);
+#pragma unroll
+            for (int k = 0; k < NV; ++k)
+                if ((k * 256 + t) * 4 < a.K) *reinterpret_cast<f32x4*>(rows + (half + 2 * i) * row_bytes + (k * 256 + t) * 16) = v[i][k] * scale * w[k];
+        }
+    }
+};
+#define GF_NORM_LOADS 10             // (NR + 1) * NV at the most: what registers hold beside the first weights in flight
+
+// MT row tiles of 16 share a wave's registers of W.  NR, NV: as GfNorm's; NR 0: no norm.
+template <int MT, int NR = 0, int NV = 1>
 __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArgs a) {
     constexpr int ROUND = GF_SUMS_KB / MT;                       // chunks whose sums shared memory holds at a time
     constexpr int THREADS = 64 * GF_WAVES;
     __shared__ float sums[ROUND * MT * 256];                     // [chunk][row tile][row][column]
+    float scale = 1.f;                                           // of row r
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
@@ -69,9 +128,21 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
     const int n_chunks = (a.K + GF_CHUNK - 1) / GF_CHUNK;
     // the outputs that this thread adds up
     constexpr int OWN = (MT * 256 + THREADS - 1) / THREADS;
-    float tot[OWN];
+    float tot[OWN], old[OWN];
 #pragma unroll
-    for (int o = 0; o < OWN; ++o) tot[o] = 0.f;
+    for (int o = 0; o < OWN; ++o) tot[o] = old[o] = 0.f;
+    if (a.add && MT == 1 && tid < 256) {                         // asked for before the weights
+        const int m = tid >> 4, n = n0 + (tid & 15);
+        if (m < a.M && n < a.N) old[0] = a.y[(size_t)m * a.ldy + n];
+    }
+    if constexpr (NR > 0) {
+        GfNorm<NR, NV> norm;
+        norm.load(a, tid);
+        norm.sum(a, tid, sums);                                  // where the chunks' sums come later
+        bn_lds_barrier();
+        scale = gf_norm_scale(a, sums, min(r, a.M - 1));
+        bn_lds_barrier();
+    }
 
     for (int c0 = 0; c0 < n_chunks; c0 += ROUND) {
         const int c1 = min(n_chunks, c0 + ROUND);
@@ -88,6 +159,12 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
             for (int t = 0; t < MT; ++t) {
                 f32x4 xv[GF_BLOCKS], acc = {0.f, 0.f, 0.f, 0.f};
                 fetch(xp[t], xv);
+                if constexpr (NR > 0) {
+                    f32x4 nw[GF_BLOCKS];
+                    fetch(a.norm_w + 4 * g, nw);
+#pragma unroll
+                    for (int j = 0; j < GF_BLOCKS; ++j) xv[j] = xv[j] * scale * nw[j];
+                }
 #pragma unroll
                 for (int j = 0; j < GF_BLOCKS; ++j)
 #pragma unroll
@@ -116,7 +193,7 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
         if (idx >= MT * 256) continue;
         const int m = idx >> 4, c = idx & 15;
         if (a.glu) sums[idx] = tot[o];
-        else if (m < a.M && c < a.cols && n0 + c < a.N) a.y[(size_t)m * a.ldy + n0 + c] = tot[o];
+        else if (m < a.M && c < a.cols && n0 + c < a.N) a.y[(size_t)m * a.ldy + n0 + c] = a.add ? old[o] + tot[o] : tot[o];
     }
     if (!a.glu) return;
     __syncthreads();
@@ -139,11 +216,15 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
 //   (16 instructions of 32 cycles stand for 4 KB of eight columns: up to 2,048 columns the matrix unit has half the time.)
 #define GF_XROW (GF_CHUNK * 4 + 16)  // bytes between the rows of a wave's staged activations
 
-template <int XR>
+// NV > 0: behind a norm (GfNorm<XR, NV>; every wave has a chunk).  The normed rows are staged once, all of them, by the threads
+// that summed their squares, and the waves read their chunks from there.
+template <int XR, int NV = 0>
 __global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_streamed_kernel(GfArgs a, int k_tiles) {
     constexpr int ROWS = 2 * XR;
+    constexpr bool NORM = NV > 0;
     extern __shared__ __align__(16) unsigned char smem[];
-    float* sums = reinterpret_cast<float*>(smem + GF_WAVES * ROWS * GF_XROW);        // [chunk][row][column]
+    const int row_bytes = NORM ? a.K * 4 + 16 : GF_XROW;
+    float* sums = reinterpret_cast<float*>(smem + (NORM ? 1 : GF_WAVES) * ROWS * row_bytes);     // [chunk][row][column]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
@@ -154,11 +235,12 @@ __global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_strea
     unsigned x_at[XR];
 #pragma unroll
     for (int i = 0; i < XR; ++i) x_at[i] = (min(2 * i + (lane >> 5), a.M - 1) * a.ldx + (lane & 31) * 4) * 4;
-    unsigned char* xs = smem + wave * ROWS * GF_XROW;
+    unsigned char* xs = smem + (NORM ? 0 : wave * ROWS * GF_XROW);
     unsigned char* park_at = xs + (lane >> 5) * GF_XROW + (lane & 31) * 16;
-    const unsigned char* read_at = xs + min(r, a.M - 1) * GF_XROW + g * 16;
+    const unsigned char* read_at = xs + min(r, a.M - 1) * row_bytes + g * 16;
     f32x4 x[XR];
     auto load_x = [&](int c) {
+        if (NORM) return;
 #pragma unroll
         for (int i = 0; i < XR; ++i) x[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xb, x_at[i], c * (GF_CHUNK * 4), 0));
     };
@@ -170,18 +252,20 @@ __global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_strea
         __builtin_amdgcn_sched_barrier(0);
     };
     auto park = [&]() {
+        if (NORM) return;
 #pragma unroll
         for (int i = 0; i < XR; ++i) *reinterpret_cast<f32x4*>(park_at + 2 * i * GF_XROW) = x[i];
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_sched_barrier(0);
     };
     auto multiply = [&](const f32x4 (&w)[GF_BLOCKS], int c) {
+        const unsigned char* from = read_at + (NORM ? c * (GF_CHUNK * 4) : 0);
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int h = 0; h < GF_BLOCKS; h += 4) {
             f32x4 v[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const f32x4*>(read_at + (h + j) * 64);
+            for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const f32x4*>(from + (h + j) * 64);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -194,10 +278,25 @@ __global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_strea
     const int n_chunks = a.K / GF_CHUNK;
     const int n = (n_chunks - wave + GF_WAVES - 1) / GF_WAVES;               // chunks of this wave: wave, wave + 8, ..
     constexpr int D = GF_WAVES;
+    // what the results are added to: an empty buffer, of which a load gives zero and reads nothing, where they are not
+    const int om = tid >> 4, on = blockIdx.x * a.cols + (tid & 15);
+    const auto yb = bn_buffer(a.y, a.add ? ((a.M - 1) * a.ldy + a.N) * 4 : 0);
+    const float old = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(yb, (min(om, a.M - 1) * a.ldy + min(on, a.N - 1)) * 4, 0, 0));
+    GfNorm<XR, NORM ? NV : 1> norm;
+    if (NORM) norm.load(a, tid);
+    auto stage = [&] {                                                       // once a wave, behind its first loads of W
+        if (!NORM) return;
+        norm.sum(a, tid, sums);                                              // where the chunks' sums come later
+        bn_lds_barrier();
+        norm.store(a, tid, sums, smem, row_bytes);
+        bn_lds_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
     if (n == 1) {
         f32x4 w[GF_BLOCKS];
         load_x(wave);
         load_w(w, wave);
+        stage();
         park();
         multiply(w, wave);
     } else if (n > 1) {
@@ -205,6 +304,7 @@ __global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_strea
         f32x4 p[GF_BLOCKS], q[GF_BLOCKS];
         load_x(c);
         load_w(p, c);
+        stage();                                                             // (the rows' registers are the second chunk's)
         load_w(q, c + D);
 #pragma unroll 1
         for (; left > 3; left -= 2, c += 2 * D) {
@@ -242,7 +342,7 @@ __global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_strea
         const float up = bn_lane_xor<8>(tot);
         if (m < a.M && col < 8) a.y[(size_t)m * a.ldy + n0 / 2 + col] = bn_gate_act(tot, a.act) * up;
     } else if (m < a.M && col < a.cols && n0 + col < a.N) {
-        a.y[(size_t)m * a.ldy + n0 + col] = tot;
+        a.y[(size_t)m * a.ldy + n0 + col] = a.add ? old + tot : tot;
     }
 }
 
@@ -527,9 +627,26 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_dma_kernel(GfArgs a, int m_ti
     }
 }
 
-template <int MT>
+// go(NR, NV) as integral constants for a norm of M rows of K numbers
+static int gf_norm_rows(int M) { return M <= 2 ? 1 : M <= 4 ? 2 : 4; }
+static bool gf_norm_ok(int M, int K, const float* norm_w) {
+    return M >= 1 && M <= 8 && K >= 4 && K % 4 == 0 && K <= 4096 && ((K <= 2048 ? 2 : 4) * (gf_norm_rows(M) + 1)) <= GF_NORM_LOADS &&
+           ((uintptr_t)norm_w & 15) == 0;
+}
+template <typename F> static int gf_norm_pick(int M, int K, F go) {
+    using std::integral_constant;
+    const int nr = gf_norm_rows(M);
+#define GF_PICK(NR_, NV_) return go(integral_constant<int, NR_>(), integral_constant<int, NV_>())
+    if (nr == 1 && K > 2048) GF_PICK(1, 4);
+    if (nr == 1) GF_PICK(1, 2);
+    if (nr == 2) GF_PICK(2, 2);
+    GF_PICK(4, 2);
+#undef GF_PICK
+}
+
+template <int MT, int NR = 0, int NV = 1>
 static int gf_launch_stream(const GfArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL((gemm_f32_stream_kernel<MT>), dim3((a.N + a.cols - 1) / a.cols), dim3(64 * GF_WAVES), 0, s, a);
+    hipLaunchKernelGGL((gemm_f32_stream_kernel<MT, NR, NV>), dim3((a.N + a.cols - 1) / a.cols), dim3(64 * GF_WAVES), 0, s, a);
     return bn_launch_status();
 }
 
@@ -596,12 +713,20 @@ extern "C" int bn_gemm_f32_supports(int N, int K, int ldw, const void* w) {
 // 38, 4,096 x 14,336 83 / 93 against 106, 11,264 x 2,048 34 / 40 against 26 / 29; at 33 rows 2,048 x 2,048 19.8 against 17.5).  Other K:
 // up to 64 while the rows' 16-row tiles times the column tiles of a CU stay few (at 64 rows, against tiles through registers,
 // 2,048 x 5,632 54 / 82, 11,264 x 2,048 60 / 54, 28,672 x 4,096 255 / 164; at 20 rows 6,144 x 4,096 43 / 61, 32,000 x 2,048 86 / 54).
+//
+// norm_w (form 0): the rows of x are normed on their way in, bn_gemm_f32_norm_supports says of which sizes.  add (form 0, up to 16
+// rows, no glu): y += the product.
 extern "C" int bn_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K, int ldx, int ldw, int ldy, int glu, int act,
-                           int form, hipStream_t s) {
+                           int form, const float* norm_w, float eps, int add, hipStream_t s) {
     if (M <= 0 || !bn_gemm_f32_supports(N, K, ldw, w) || ldx % 4 || ldx < K || ldx > (1 << 22) || ((uintptr_t)x & 15)) return BN_ERR_ARG;
     if (ldy < (glu ? N / 2 : N) || (glu && N % 16) || act < 0 || act >= BN_ACT_KINDS) return BN_ERR_ARG;
     if ((long long)((M + 31) / 32) * ((N + 63) / 64) > 0x7fffffffLL) return BN_ERR_ARG;
-    GfArgs a = {(const float*)x, (const float*)w, (float*)y, M, N, K, ldx, ldw, ldy, 16, glu ? 1 : 0, act};
+    if (((norm_w || add) && form) || (norm_w && !gf_norm_ok(M, K, norm_w)) || (add && (glu || M > 16))) return BN_ERR_ARG;
+    GfArgs a = {(const float*)x, (const float*)w, (float*)y, M, N, K, ldx, ldw, ldy, 16, glu ? 1 : 0, act, add ? 1 : 0, norm_w, eps};
+    if (norm_w) {
+        a.cols = glu ? 16 : gf_stream_cols(N);
+        return gf_norm_pick(M, K, [&](auto nr, auto nv) { return gf_launch_stream<1, decltype(nr)::value, decltype(nv)::value>(a, s); });
+    }
     const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
     if (form == 0) {
         const bool streams = K % GF_BK == 0 ? M <= 32 && N <= 16 * GF_CUS : M <= 64 && (long long)mt * N <= 6LL * 16 * GF_CUS;
@@ -628,26 +753,30 @@ extern "C" int bn_gemm_f32_stream_cols(int N) { return N < 1 ? 0 : gf_stream_col
 
 #define GF_STREAMED_SMEM (150 * 1024)
 static int gf_streamed_xr(int M) { return M <= 2 ? 1 : M <= 4 ? 2 : M <= 8 ? 4 : 8; }
-static size_t gf_streamed_smem(int M, int K) {                               // the staged activations, a sum a chunk, row and column
+static size_t gf_streamed_smem(int M, int K, bool norm) {                    // the staged activations, a sum a chunk, row and column
     const size_t rows = 2 * gf_streamed_xr(M);
-    return GF_WAVES * rows * GF_XROW + (size_t)(K / GF_CHUNK) * rows * 64;
+    return (norm ? rows * (K * 4 + 16) : GF_WAVES * rows * GF_XROW) + (size_t)(K / GF_CHUNK) * rows * 64;
 }
+
+// 1 if the products of up to 16 rows take a norm of such rows with them
+extern "C" int bn_gemm_f32_norm_supports(int M, int K) { return gf_norm_ok(M, K, nullptr); }
 
 // 1 if the kernel over a streamed copy takes the product: up to 16 rows, whole chunks whose sums fit into shared memory
 // (every K up to 10,496, and three times that at 8 rows), rows of activations that are whole 16-byte groups.
 extern "C" int bn_gemm_f32_streamed_supports(int M, int N, int K, int ldx, int tile_rows, const void* x) {
-    return M >= 1 && M <= 16 && N >= 1 && K >= GF_CHUNK && K % GF_CHUNK == 0 && gf_streamed_smem(M, K) <= GF_STREAMED_SMEM && ldx >= K &&
+    return M >= 1 && M <= 16 && N >= 1 && K >= GF_CHUNK && K % GF_CHUNK == 0 && gf_streamed_smem(M, K, false) <= GF_STREAMED_SMEM && ldx >= K &&
            ldx % 4 == 0 && ldx <= 1 << 22 && tile_rows >= 1 && tile_rows <= BN_STREAM_TILE_ROWS && ((uintptr_t)x & 15) == 0;
 }
 
 // As bn_gemm_f32 over W's streamed copy (common.h) with that many rows a tile (16 with glu).
 extern "C" int bn_gemm_f32_streamed(const void* x, const void* tiles, void* y, int M, int N, int K, int ldx, int tile_rows, int ldy,
-                                    int glu, int act, hipStream_t s) {
+                                    int glu, int act, const float* norm_w, float eps, int add, hipStream_t s) {
     if (!bn_gemm_f32_streamed_supports(M, N, K, ldx, tile_rows, x) || !tiles || !y || ((uintptr_t)tiles & 15)) return BN_ERR_ARG;
     if (ldy < (glu ? N / 2 : N) || (glu && (N % 16 || tile_rows != 16)) || act < 0 || act >= BN_ACT_KINDS) return BN_ERR_ARG;
-    GfArgs a = {(const float*)x, (const float*)tiles, (float*)y, M, N, K, ldx, 0, ldy, tile_rows, glu ? 1 : 0, act};
+    if ((norm_w && (!gf_norm_ok(M, K, norm_w) || K < GF_WAVES * GF_CHUNK)) || (add && (glu || (long long)M * ldy > 1 << 29))) return BN_ERR_ARG;
+    GfArgs a = {(const float*)x, (const float*)tiles, (float*)y, M, N, K, ldx, 0, ldy, tile_rows, glu ? 1 : 0, act, add ? 1 : 0, norm_w, eps};
     auto go = [&](auto kernel) {
-        const size_t smem = gf_streamed_smem(M, K);
+        const size_t smem = gf_streamed_smem(M, K, norm_w != nullptr);
         if (smem > 64 * 1024) {
             const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
             if (e != hipSuccess) return (int)e;
@@ -655,6 +784,8 @@ extern "C" int bn_gemm_f32_streamed(const void* x, const void* tiles, void* y, i
         hipLaunchKernelGGL(kernel, dim3((N + tile_rows - 1) / tile_rows), dim3(64 * GF_WAVES), smem, s, a, K / BN_STREAM_TILE_COLS_F32);
         return bn_launch_status();
     };
+    if (norm_w)
+        return gf_norm_pick(M, K, [&](auto nr, auto nv) { return go(gemm_f32_streamed_kernel<decltype(nr)::value, decltype(nv)::value>); });
     switch (gf_streamed_xr(M)) {
         case 1: return go(gemm_f32_streamed_kernel<1>);
         case 2: return go(gemm_f32_streamed_kernel<2>);

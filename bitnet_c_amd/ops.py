@@ -175,10 +175,13 @@ _SIGNATURES = {
     },
     "gemm_f32": {
         "bn_gemm_f32_supports": [c_int, c_int, c_int, c_void_p],
-        "bn_gemm_f32": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+        "bn_gemm_f32": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_float,
+                        c_int, c_void_p],
+        "bn_gemm_f32_norm_supports": [c_int, c_int],
         "bn_gemm_f32_stream_cols": [c_int],
         "bn_gemm_f32_streamed_supports": [c_int, c_int, c_int, c_int, c_int, c_void_p],
-        "bn_gemm_f32_streamed": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+        "bn_gemm_f32_streamed": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_float,
+                                 c_int, c_void_p],
     },
     "gemm_tiled": {
         "bn_gemm_tiled": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
@@ -475,30 +478,40 @@ def _tiled(x, w, out_dtype):
     return y
 
 
-def _f32_product(x, w, glu: bool = False, activation: str = "silu", form: int = 0, streamed: Optional["StreamedWeight"] = None):
+def _f32_product(x, w, glu: bool = False, activation: str = "silu", form: int = 0, streamed: Optional["StreamedWeight"] = None,
+                 norm: Optional["StreamNorm"] = None, into: Optional[torch.Tensor] = None):
     """x . w^T in float32 on the float32 matrix instruction (gemm_f32.hip), or with glu act(gate) * up for w = gate and up
     rows interleaved in blocks of 8; None for weights that the kernels do not take (rows that are not whole 16-byte groups).
     Whether they do depends on the weights alone, and every form of the kernels has one order of summation, so a row's bits do
     not depend on the step it comes in.  form: 0, by the sizes; the others are bn_gemm_f32's, for tests.  streamed: w's
-    streamed copy, which products of up to 16 rows read instead (the same bits)."""
+    streamed copy, which products of up to 16 rows read instead (the same bits).  norm: x is its stream, whose rows are normed
+    on their way in (sizes that can_norm_rows takes); into: a contiguous float32 tensor that the product (of up to 16 rows) is
+    added to, and the result."""
     M, K = x.shape
     N, ldw = w.shape[0], _rows(w, "w")
-    if not _fn("gemm_f32", "bn_gemm_f32_supports")(N, K, ldw, w.data_ptr()):
+    if not f32_product_takes(w):
         return None
     ldx = _rows(x, "x")
     if ldx % 4 or ldx > 1 << 22 or x.data_ptr() % 16:
         x = x.clone(memory_format=torch.contiguous_format)
         ldx = K
-    y = torch.empty((M, N // 2 if glu else N), dtype=torch.float32, device=x.device)
+    y = into if into is not None else torch.empty((M, N // 2 if glu else N), dtype=torch.float32, device=x.device)
+    nw, eps = (norm.weight.data_ptr(), norm.eps) if norm is not None else (None, 0.0)
     if (streamed is not None and form == 0 and (not glu or streamed.tile_rows == STREAM_TILE_ROWS)
-            and _fn("gemm_f32", "bn_gemm_f32_streamed_supports")(M, N, K, ldx, streamed.tile_rows, x.data_ptr())):
+            and (norm is None or K >= F32_STREAM_NORM_MIN_K) and _fn("gemm_f32", "bn_gemm_f32_streamed_supports")(M, N, K, ldx, streamed.tile_rows, x.data_ptr())):
         tiles, _, rows = _weight_arg(w, streamed, "float32 product")
         _check(_fn("gemm_f32", "bn_gemm_f32_streamed")(x.data_ptr(), tiles, y.data_ptr(), M, N, K, ldx, rows, y.shape[1], int(glu),
-                                                       _act(activation), _stream()), "gemm_f32(streamed)")
+                                                       _act(activation), nw, eps, int(into is not None), _stream()),
+               "gemm_f32(streamed)")
         return y
     _check(_fn("gemm_f32", "bn_gemm_f32")(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, ldx, ldw, y.shape[1], int(glu),
-                                          _act(activation), int(form), _stream()), "gemm_f32")
+                                          _act(activation), int(form), nw, eps, int(into is not None), _stream()), "gemm_f32")
     return y
+
+
+def f32_product_takes(w: torch.Tensor) -> bool:
+    """Whether the float32 matrix instruction's kernels take weights w [N, K] (rows of whole 16-byte groups)."""
+    return bool(_fn("gemm_f32", "bn_gemm_f32_supports")(w.shape[0], w.shape[1], _rows(w, "w"), w.data_ptr()))
 
 
 def gemm_mfma(x: torch.Tensor, w: torch.Tensor, out_dtype=None, glu8: bool = False, activation: str = "silu",
@@ -544,6 +557,7 @@ def skinny_supported(M: int, N: int, K: int, ldx: int, ldw: int) -> bool:
 # the streamed copy of a weight matrix
 # --------------------------------------------------------------------------------------
 STREAM_TILE_ROWS = _build.header_constant("BN_STREAM_TILE_ROWS")
+F32_STREAM_NORM_MIN_K = _build.header_constant("GF_CHUNK", "gemm_f32.hip") * _build.header_constant("GF_WAVES", "gemm_f32.hip")
 STREAM_TILE_COLS = _build.header_constant("BN_STREAM_TILE_COLS")
 STREAM_TILE_COLS_F32 = _build.header_constant("BN_STREAM_TILE_COLS_F32")
 
@@ -939,6 +953,54 @@ class DeferredNorm:
         return add_rmsnorm(self.stream, None, self.weight, self.eps, out_dtype or self.scaled.dtype, rows)
 
 
+@dataclass
+class StreamNorm(DeferredNorm):
+    """An RMSNorm of rows that already lie in the residual stream, left to a product of few rows that norms them on their way
+    into its kernel, as add_rmsnorm would (the same bits).  The stream must not change before that product has been launched."""
+
+    @property
+    def shape(self):
+        return self.stream.shape
+
+    @property
+    def dtype(self):
+        return torch.float32
+
+    @property
+    def device(self):
+        return self.stream.device
+
+    def materialize(self, out_dtype=None, rows=None) -> torch.Tensor:
+        return add_rmsnorm(self.stream, None, self.weight, self.eps, out_dtype or self.dtype, rows)
+
+
+def stream_norm(stream: torch.Tensor, weight: torch.Tensor, eps: float) -> StreamNorm:
+    return StreamNorm(None, None, stream, weight, float(eps))
+
+
+def can_norm_rows(M: int, K: int, dtype) -> bool:
+    """Whether the float32 products of M rows of K numbers norm their rows themselves."""
+    return (FUSE_NORMS and dtype == torch.float32 and torch.cuda.is_available()
+            and bool(_fn("gemm_f32", "bn_gemm_f32_norm_supports")(M, K)))
+
+
+def takes_stream_norm(pre: DeferredNorm, w: torch.Tensor) -> bool:
+    """Whether a product with w norms the rows of pre's stream itself."""
+    return (isinstance(pre, StreamNorm) and w.dtype == torch.float32 and w.shape[1] == pre.stream.shape[1]
+            and can_norm_rows(*pre.stream.shape, w.dtype) and pre.stream.is_contiguous() and pre.stream.data_ptr() % 16 == 0
+            and pre.weight.is_contiguous() and pre.weight.data_ptr() % 16 == 0 and pre.weight.numel() == w.shape[1]
+            and pre.weight.dtype == torch.float32 and f32_product_takes(w))
+
+
+def linear_stream_norm(pre: StreamNorm, w: torch.Tensor, streamed: Optional[StreamedWeight] = None, glu: bool = False,
+                       activation: str = "silu") -> torch.Tensor:
+    """linear(rmsnorm(stream), w), or with glu linear_swiglu for gate and up interleaved in blocks of 8, in one float32 kernel;
+    for what takes_stream_norm says."""
+    if not takes_stream_norm(pre, w):
+        raise KernelError(f"linear_stream_norm: rows {tuple(pre.shape)}, w {tuple(w.shape)} cannot be fused")
+    return _f32_product(pre.stream, w, glu, activation, streamed=streamed, norm=pre)
+
+
 DEFER_ROWS = (17, 128)    # row counts at which a norm is left to its consumer through sum_deferred (below: the fused products)
 
 
@@ -1076,14 +1138,21 @@ def linear_into_stream(x: torch.Tensor, w: torch.Tensor, stream: torch.Tensor, w
                        eps: float, streamed: Optional[StreamedWeight] = None) -> DeferredNorm:
     """stream += linear(x, w) (float32 stream [M, N], in place), and what the next norm (weights
     `weight`, `eps`) needs: the bf16 copy of the new stream times the weights and the rows' sums of
-    squares in parts.  Returns that norm, deferred."""
+    squares in parts.  Returns that norm, deferred.  float32: the new rows in the stream are all that the norm needs."""
     require_gpu()
-    _dev(x, "x", torch.bfloat16, 2)
-    _dev(w, "w", torch.bfloat16, 2)
+    _dev(x, "x", dims=2)
+    _dev(w, "w", x.dtype, 2)
     _dev(stream, "stream", torch.float32, 2)
     _dev(weight, "weight", torch.float32, 1)
     M, K = x.shape
     N = w.shape[0]
+    if x.dtype == torch.float32:
+        if (w.shape[1] != K or tuple(stream.shape) != (M, N) or not stream.is_contiguous() or weight.numel() != N
+                or not can_norm_rows(M, N, x.dtype) or _f32_product(x, w, streamed=streamed, into=stream) is None):
+            raise KernelError(f"linear_into_stream: x {tuple(x.shape)}, w {tuple(w.shape)}, stream {tuple(stream.shape)}, "
+                              f"weight {tuple(weight.shape)} do not agree or cannot be fused")
+        return stream_norm(stream, weight, eps)
+    _dev(x, "x", torch.bfloat16, 2)
     if w.shape[1] != K or tuple(stream.shape) != (M, N) or weight.numel() != N or not weight.is_contiguous():
         raise KernelError(f"linear_into_stream: x {tuple(x.shape)}, w {tuple(w.shape)}, stream {tuple(stream.shape)}, "
                           f"weight {tuple(weight.shape)} do not agree")

@@ -352,6 +352,8 @@ class ResidualStream:
                 deferred = ops.sum_deferred(self.x, self.pending, norm.weight, norm.eps)
                 self.pending = None
                 return deferred
+            if self.pending is None and out_dtype == torch.float32 and self.x.is_contiguous() and ops.can_norm_rows(*self.x.shape, out_dtype):
+                return ops.stream_norm(self.x, norm.weight, norm.eps)        # nothing to add: the consumer norms the rows
         delta = self._pending_tensor()
         if delta is not None and not isinstance(delta, torch.Tensor) and not getattr(norm, "takes_partial_sums", False):
             self.flush()                         # partial sums, and a norm that only knows tensors: add them up first

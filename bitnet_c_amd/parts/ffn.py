@@ -121,6 +121,9 @@ class SwiGLU(Part):
         if isinstance(h, ops.DeferredNorm):
             w = self.gate_up.weight
             M = h.shape[0]
+            if not self.has_bias and self.interleaved and ops.takes_stream_norm(h, w):
+                act = ops.linear_stream_norm(h, w, self.gate_up.streamed, True, self.activation)
+                return self.down.lazy(act) if lazy_ok else self.down(act)
             if (not self.has_bias and self.interleaved and w.dtype == torch.bfloat16
                     and (ops.can_fuse_norm(M, self.F, self.hidden, w.dtype)
                          or (M > ops.FUSED_ROWS and ops.LIBRARY_PRODUCTS and w.data_ptr() % 16 == 0))):

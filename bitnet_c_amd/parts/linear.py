@@ -49,6 +49,8 @@ class Linear:
             if (self.bias is None and out_dtype in (None, torch.bfloat16) and w.dtype == torch.bfloat16
                     and ops.can_fuse_norm(M, N, K, w.dtype) and w.data_ptr() % 16 == 0):
                 return ops.linear_prenorm(x, w, streamed)
+            if self.bias is None and out_dtype in (None, torch.float32) and ops.takes_stream_norm(x, w):
+                return ops.linear_stream_norm(x, w, streamed)
             x = x.materialize()
         y = ops.linear(x, w, out_dtype, streamed=streamed)
         if self.bias is not None:
@@ -56,8 +58,8 @@ class Linear:
         return y
 
     def lazy(self, x: torch.Tensor):
-        """The product in the form in which it reaches a residual stream cheapest (bf16, no bias): a LazyDelta at
-        decode sizes, where it can add itself to the stream; partial sums over ranges of K (ops.PartialSums), which the
+        """The product in the form in which it reaches a residual stream cheapest (no bias): a LazyDelta at
+        decode sizes, where it can add itself to the stream; in bf16 partial sums over ranges of K (ops.PartialSums), which the
         kernel of the next norm adds up, where ops.can_split_sums says so; else its result."""
         from .base import LazyDelta
         M, (N, K) = x.shape[0], self.weight.shape
@@ -67,6 +69,9 @@ class Linear:
             return LazyDelta(x, self)
         if plain and ops.can_split_sums(M, N, K, x.dtype) and x.stride(1) == 1 and x.stride(0) % 8 == 0:
             return ops.linear_partial_sums(x, self.weight, self.streamed)
+        if (self.bias is None and x.dim() == 2 and x.dtype == self.weight.dtype == torch.float32 and M > 0
+                and ops.can_norm_rows(M, N, x.dtype) and ops.f32_product_takes(self.weight)):
+            return LazyDelta(x, self)
         return self(x)
 
     def into_stream(self, x: torch.Tensor, stream: torch.Tensor, norm_weight: torch.Tensor, eps: float):

@@ -153,3 +153,35 @@ def test_streamed_copies_whose_sums_do_not_fit_are_not_read():
     xd, wd = x.cuda(), w.cuda()
     for m in (8, 16):
         assert torch.equal(ops.linear(xd[:m].contiguous(), wd, streamed=ops.stream_copy(wd)), ops.linear(xd[:m].contiguous(), wd)), m
+
+
+# a norm taken into the product behind it, and a product added into the stream, against the kernels of their own: the same bits.
+# rows: the edges of 1, 2, 4 and 8; K: less than a thread's group of four, a chunk's remainder, fewer chunks than waves (the
+# row-major kernel), one to four a wave, the widest at 2 rows and at 8; infinite and NaN rows stay their own
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("N,K,R", [(16, 4, 16), (36, 172, 16), (40, 896, 12), (28, 1024, 16), (24, 1152, 8), (16, 2048, 16), (32, 4096, 16)])
+def test_products_with_a_norm_and_into_the_stream(M, N, K, R):
+    ops = _ops()
+    x, w = _data(M, N, K, 5 * M + N)
+    xd, wd = x.cuda(), w.cuda()
+    nw = torch.linspace(0.5, 1.5, K, device="cuda")
+    if M > 3:
+        xd[1, K // 2], xd[2, 0] = float("inf"), float("nan")
+    copies = [None] + ([ops.stream_copy(wd, R)] if K % ops.F32_STREAM_CHUNK == 0 else [])
+    xd = xd * torch.logspace(-1, 1, K, device="cuda") if K > 4 else xd
+    if ops.can_norm_rows(M, K, torch.float32):
+        h = ops.add_rmsnorm(xd.clone(), None, nw, 1e-5, torch.float32)
+        for sw in copies:
+            pre = ops.stream_norm(xd, nw, 1e-5)
+            assert torch.equal(ops.linear_stream_norm(pre, wd, sw).nan_to_num(7.0), ops.linear(h, wd).nan_to_num(7.0)), sw is None
+            if N % 16 == 0 and R == 16:
+                assert torch.equal(ops.linear_stream_norm(pre, wd, sw, True).nan_to_num(7.0),
+                                   ops.linear_swiglu(h, wd, True).nan_to_num(7.0)), sw is None
+    else:
+        assert K == 4096 and M > 2
+    stream = torch.randn(M, N, device="cuda")
+    for sw in copies:
+        got = stream.clone()
+        out = ops.linear_into_stream(xd, wd, got, torch.ones(N, device="cuda"), 1e-5, sw)
+        assert out.stream is got
+        assert torch.equal(got.nan_to_num(7.0), (stream + ops.linear(xd, wd)).nan_to_num(7.0)), sw is None
