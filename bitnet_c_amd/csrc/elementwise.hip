@@ -2,6 +2,7 @@
 // RMSNorm, SwiGLU, bias add, row gather.  The residual stream is float32; `T` is the
 // activation type (float or bf16) that the matrix products read and write.
 #include "common.h"
+#include <type_traits>
 
 // x[t, :] = float(E[token[t], :]) * scale.  A token outside [0, vocab) gives a zero row, as the
 // reference's embedding does (src/model_embed.c:6-28, test/test_safety.c:278-315); the
@@ -678,18 +679,21 @@ static_assert(alignof(Eight<float>) == 16 && alignof(Eight<bf16>) == 16 && sizeo
 // add_normed_rmsnorm in bf16 256 4.2 / 4.0, 512 4.3 / 4.6.
 #define WIDE_ROW 512
 
-template <typename T, int G>
-__global__ __launch_bounds__(256) void rmsnorm_mean_wide_kernel(T* __restrict__ out, const T* __restrict__ a, const T* __restrict__ b,
-                                                                const float* __restrict__ wa, const float* __restrict__ wb, int dim, float eps) {
+// ADD: out is float32 and the mean, rounded to T, is added to it (a residual stream whose next norm is its reader's).
+template <typename T, int G, bool ADD>
+__global__ __launch_bounds__(256) void rmsnorm_mean_wide_kernel(std::conditional_t<ADD, float, T>* __restrict__ out, const T* __restrict__ a,
+                                                                const T* __restrict__ b, const float* __restrict__ wa,
+                                                                const float* __restrict__ wb, int dim, float eps) {
     __shared__ float scratch[16];
     const size_t row = (size_t)blockIdx.x * dim;
     const int groups = dim / 8;
     Eight<T> ga[G], gb[G];
-    Eight<float> va[G], vb[G];
+    Eight<float> va[G], vb[G], old[G];
     float sa = 0.f, sb = 0.f;
 #pragma unroll
     for (int q = 0; q < G; ++q) {
         const int at = min((int)threadIdx.x + 256 * q, groups - 1) * 8;
+        if constexpr (ADD) old[q] = *reinterpret_cast<const Eight<float>*>(out + row + at);
         ga[q] = *reinterpret_cast<const Eight<T>*>(a + row + at);
         va[q] = *reinterpret_cast<const Eight<float>*>(wa + at);
         if (b) {
@@ -721,19 +725,25 @@ __global__ __launch_bounds__(256) void rmsnorm_mean_wide_kernel(T* __restrict__ 
             if (b) v += to_f32(gb[q].e[e]) * fb * vb[q].e[e];
             o.e[e] = from_f32<T>(v * share);
         }
-        *reinterpret_cast<Eight<T>*>(out + row + at) = o;
+        if constexpr (ADD) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) old[q].e[e] += to_f32(o.e[e]);
+            *reinterpret_cast<Eight<float>*>(out + row + at) = old[q];
+        } else {
+            *reinterpret_cast<Eight<T>*>(out + row + at) = o;
+        }
     }
 }
 
-template <typename T>
-static bool launch_rmsnorm_mean_wide(T* out, const T* a, const T* b, const float* wa, const float* wb, int n_rows, int dim, float eps,
+template <typename T, bool ADD = false>
+static bool launch_rmsnorm_mean_wide(std::conditional_t<ADD, float, T>* out, const T* a, const T* b, const float* wa, const float* wb, int n_rows, int dim, float eps,
                                      hipStream_t s) {
     const int per = (dim / 8 + 255) / 256;
     if (dim % 8 || dim < WIDE_ROW || per > 4 || (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b | (uintptr_t)wa | (uintptr_t)wb) & 15)) return false;
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(n_rows), dim3(256), 0, s, out, a, b, wa, wb, dim, eps); };
-    if (per == 1) go(rmsnorm_mean_wide_kernel<T, 1>);
-    else if (per == 2) go(rmsnorm_mean_wide_kernel<T, 2>);
-    else go(rmsnorm_mean_wide_kernel<T, 4>);
+    if (per == 1) go(rmsnorm_mean_wide_kernel<T, 1, ADD>);
+    else if (per == 2) go(rmsnorm_mean_wide_kernel<T, 2, ADD>);
+    else go(rmsnorm_mean_wide_kernel<T, 4, ADD>);
     return true;
 }
 
@@ -753,6 +763,17 @@ extern "C" int bn_rmsnorm_mean(int dtype, void* out, const void* a, const void* 
     else
         return BN_ERR_DTYPE;
     return bn_launch_status();
+}
+
+// x [n_rows, dim] (float32) += the same, rounded to dtype first: rows of WIDE_ROW to 8,192 numbers, a multiple of 8, everything
+// 16-byte aligned.
+extern "C" int bn_rmsnorm_mean_add(int dtype, float* x, const void* a, const void* b, const float* wa, const float* wb, int n_rows, int dim,
+                                   float eps, hipStream_t s) {
+    if (n_rows <= 0 || dim <= 0 || !x || !a || !wa || (b && !wb)) return BN_ERR_ARG;
+    if (dtype != BN_DT_F32 && dtype != BN_DT_BF16) return BN_ERR_DTYPE;
+    const bool done = dtype == BN_DT_F32 ? launch_rmsnorm_mean_wide<float, true>(x, (const float*)a, (const float*)b, wa, wb, n_rows, dim, eps, s)
+                                         : launch_rmsnorm_mean_wide<bf16, true>(x, (const bf16*)a, (const bf16*)b, wa, wb, n_rows, dim, eps, s);
+    return done ? bn_launch_status() : BN_ERR_ARG;
 }
 
 // A part's output that has a norm of its own before it joins the stream, and the norm of the next part, in one pass over

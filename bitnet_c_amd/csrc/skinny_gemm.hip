@@ -41,6 +41,8 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast
 
 #define SK_XROW 528           // bytes between rows of a wave's staged X chunk (512 + 16: conflict-free 16-byte reads)
 
+#define SK_ROWS_MAX 8         // rows that a product forms itself: more cost a workgroup more than its weights do
+
 #define SK_STREAM_WAVES 8     // waves of a workgroup over a streamed copy of whole chunks
 
 #define SK_ACT_UNARY 16       // act: this plus one of BN_UNARY_*: an activation of one argument on every result
@@ -350,9 +352,12 @@ void skinny_gemm_fused_kernel(const bf16* __restrict__ X, const bf16* __restrict
 //   24.0 / 24.7 -> 21.1 / 22.0 (a plain read of the same bytes with a dependent launch: 4.0, 3.1, 8.3, 5.2; 8.9, 6.5, 35.8,
 //   18.4).  At 9 to 16 rows the activations' registers leave room for one workgroup of two chunks a wave on a CU (8B QKV 15.5
 //   -> 14.1, gate/up 48.0 -> 43.7).
-template <int XR, bool ONE>
+#define SK_STAGED_ROW(k) ((k) * 2 + 16)      // bytes between staged rows of k numbers
+
+template <int XR, bool ONE, bool STAGED = false>
 struct SkStream {
-    // XR: activation loads a lane and chunk, for up to 2 XR rows; ONE: a wave has one chunk at most
+    // XR: activation loads a lane and chunk, for up to 2 XR rows; ONE: a wave has one chunk at most; STAGED (with ONE): the rows
+    // lie in shared memory, SK_STAGED_ROW(K) bytes apart, when run's `between` returns
     __amdgpu_buffer_rsrc_t wb, xb;
     unsigned tile, w_at;
     unsigned x_at[XR];
@@ -363,6 +368,7 @@ struct SkStream {
     // (the scheduling barriers keep the loads of a chunk where they are written: moved up over the products before them they
     // need registers that are not there)
     __device__ __forceinline__ void load_x(int c) {
+        if (STAGED) return;
 #pragma unroll
         for (int r = 0; r < XR; ++r) x[r] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(xb, x_at[r], c * (SK_CHUNK * 2), 0));
     }
@@ -375,6 +381,7 @@ struct SkStream {
     }
     // the chunk's activations into the wave's own region of shared memory (a wave's operations on it run in order)
     __device__ __forceinline__ void park() {
+        if (STAGED) return;
 #pragma unroll
         for (int r = 0; r < XR; ++r) *reinterpret_cast<bf16x8*>(park_at + 2 * r * SK_XROW) = x[r];
         __builtin_amdgcn_wave_barrier();
@@ -407,6 +414,7 @@ struct SkStream {
         xs += (size_t)wave * 2 * XR * SK_XROW;
         park_at = xs + (lane >> 5) * SK_XROW + (lane & 31) * 16;
         read_at = xs + min(i, M - 1) * SK_XROW + g * 16;
+        if (STAGED) read_at = xs - (size_t)wave * 2 * XR * SK_XROW + min(i, M - 1) * SK_STAGED_ROW(n_chunks * SK_CHUNK) + wave * (SK_CHUNK * 2) + g * 16;
         acc = (f32x4){0.f, 0.f, 0.f, 0.f};
         const int n = (n_chunks - wave + SK_STREAM_WAVES - 1) / SK_STREAM_WAVES;       // chunks of this wave
         if (ONE || n <= 1) {
@@ -504,11 +512,12 @@ void skinny_stream_group_kernel(SkinnyGroup p, int M, int n_chunks, int k_tiles)
 #define SK_FUSED_GLU 0
 #define SK_FUSED_PRE 1
 #define SK_FUSED_RES 2
+#define SK_FUSED_ADD 3               // into the stream as a bf16 output would be added: rounded first, and nothing left for a norm
 template <int XR, bool ONE, int FORM, int SL>
 __global__ __launch_bounds__(64 * SK_STREAM_WAVES, (ONE && XR <= 4) ? 6 : XR == 8 ? 2 : 4)
 void skinny_stream_fused_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, bf16* __restrict__ Y, int M, int N, int n_chunks,
                                 int ldx, int k_tiles, int ldy, int rows, int act, SkinnyFused f) {
-    constexpr bool PRE = FORM != SK_FUSED_RES;
+    constexpr bool PRE = FORM == SK_FUSED_GLU || FORM == SK_FUSED_PRE;
     constexpr int H = XR <= 4 ? 1 : 2;                // rows of the norm that a wave adds up: wave, and wave + 8
     extern __shared__ __align__(16) float red[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -528,7 +537,7 @@ void skinny_stream_fused_kernel(const bf16* __restrict__ X, const bf16* __restri
     if (!PRE) {
         const int nc = min(n, N - 1);
         old = f.resid[(size_t)min(m, M - 1) * f.ld_resid + nc];
-        next_w = f.next_weight[nc];
+        if (FORM == SK_FUSED_RES) next_w = f.next_weight[nc];
     }
     SkStream<XR, ONE> s;
     s.run(X, W, M, n_chunks, ldx, k_tiles, rows, blockIdx.x, reinterpret_cast<unsigned char*>(red + SK_STREAM_RED), lane, wave, [&] {
@@ -552,6 +561,8 @@ void skinny_stream_fused_kernel(const bf16* __restrict__ X, const bf16* __restri
         if (mine && (lane & 8) == 0) Y[(size_t)m * ldy + (n0 >> 1) + (lane & 7)] = __float2bfloat16(bn_gate_act(v, act) * up);
     } else if (FORM == SK_FUSED_PRE) {
         if (mine) Y[(size_t)m * ldy + n] = __float2bfloat16(v);
+    } else if (FORM == SK_FUSED_ADD) {
+        if (mine) f.resid[(size_t)m * f.ld_resid + n] = old + to_f32(__float2bfloat16(v));
     } else {
         float xn = 0.f;
         if (mine) {
@@ -566,6 +577,106 @@ void skinny_stream_fused_kernel(const bf16* __restrict__ X, const bf16* __restri
         sq += bn_lane_xor<8>(sq);
         if (at == 0 && m < M) f.slots_out[(size_t)m * gridDim.x + blockIdx.x] = sq;
     }
+}
+
+// A product whose rows the residual stream still has to give: every workgroup forms them itself while its weights are on their
+// way, instead of a kernel of one workgroup a row that the product would wait for (3.4 us a launch; the rows come from the L2).
+// The operations and their order are those of the kernels in whose place this runs (elementwise.hip), so are the bits; here
+// the halves of the workgroup take every other row, eight numbers a thread.
+#define SK_ROWS_NORM 0               // x w / rms(x): add_rmsnorm_row_kernel
+#define SK_ROWS_SUM 1                // x + w d / rms(d), the new stream: add_normed_rmsnorm_wide_kernel
+struct SkinnyRows {
+    const float* x;                  // [M, K] the stream
+    const bf16* delta;               // [M, K] SUM
+    const float* w;                  // [K]
+    float* x_new;                    // [M, K] SUM: where the first workgroup writes the new stream (the others may still read x)
+    int K;
+    float eps;
+};
+
+template <int NR, int MODE> struct SkRowStage {
+    float4 x[NR][2], w[2];
+    uint4 d[NR];
+    int t, half;
+    __device__ __forceinline__ int at(int k) const { return MODE == SK_ROWS_NORM ? (k * 256 + t) * 4 : t * 8 + k * 4; }
+    __device__ __forceinline__ void load(const SkinnyRows& p, int M) {
+        t = threadIdx.x & 255;
+        half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const size_t row = (size_t)min(half + 2 * i, M - 1) * p.K;
+            if (MODE == SK_ROWS_SUM) d[i] = *reinterpret_cast<const uint4*>(p.delta + row + min(t * 8, p.K - 8));
+#pragma unroll
+            for (int k = 0; k < 2; ++k) x[i][k] = *reinterpret_cast<const float4*>(p.x + row + min(at(k), p.K - 4));
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) w[k] = *reinterpret_cast<const float4*>(p.w + min(at(k), p.K - 4));
+    }
+    // parts: [2 NR][4] floats; rows: the staged rows.  Two barriers; behind the second the rows are there.
+    __device__ __forceinline__ void stage(const SkinnyRows& p, int M, float* parts, unsigned char* rows) {
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            float ss = 0.f;
+            if (MODE == SK_ROWS_NORM) {
+#pragma unroll
+                for (int k = 0; k < 2; ++k) ss = at(k) < p.K ? bn_add_squares(ss, x[i][k], k) : ss;
+            } else {
+                const uint32_t two[4] = {d[i].x, d[i].y, d[i].z, d[i].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float lo = bf16lo_to_f32(two[e]), hi = bf16hi_to_f32(two[e]);
+                    ss = __builtin_fmaf(hi, hi, __builtin_fmaf(lo, lo, ss));
+                }
+                if (at(0) >= p.K) ss = 0.f;
+            }
+            ss = wave_sum(ss);
+            if ((threadIdx.x & 63) == 0) parts[(half + 2 * i) * 4 + ((threadIdx.x >> 6) & 3)] = ss;
+        }
+        bn_lds_barrier();
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int row = half + 2 * i;
+            float ss = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) ss += parts[row * 4 + j];
+            const float f = 1.0f / sqrtf(ss / (float)p.K + p.eps);
+            const uint32_t two[4] = {d[i].x, d[i].y, d[i].z, d[i].w};
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                if (at(k) >= p.K) continue;
+                float4 v;
+                if (MODE == SK_ROWS_NORM) {
+                    v = make_float4(x[i][k].x * f * w[k].x, x[i][k].y * f * w[k].y, x[i][k].z * f * w[k].z, x[i][k].w * f * w[k].w);
+                } else {
+                    v.x = __builtin_fmaf(bf16lo_to_f32(two[2 * k]) * f, w[k].x, x[i][k].x);
+                    v.y = __builtin_fmaf(bf16hi_to_f32(two[2 * k]) * f, w[k].y, x[i][k].y);
+                    v.z = __builtin_fmaf(bf16lo_to_f32(two[2 * k + 1]) * f, w[k].z, x[i][k].z);
+                    v.w = __builtin_fmaf(bf16hi_to_f32(two[2 * k + 1]) * f, w[k].w, x[i][k].w);
+                    if (blockIdx.x == 0 && row < M) *reinterpret_cast<float4*>(p.x_new + (size_t)row * p.K + at(k)) = v;
+                }
+                bf16 o[4] = {from_f32<bf16>(v.x), from_f32<bf16>(v.y), from_f32<bf16>(v.z), from_f32<bf16>(v.w)};
+                *reinterpret_cast<uint2*>(rows + row * SK_STAGED_ROW(p.K) + at(k) * 2) = *reinterpret_cast<const uint2*>(o);
+            }
+        }
+        bn_lds_barrier();
+    }
+};
+
+template <int XR, int MODE, bool UNARY>
+__global__ __launch_bounds__(64 * SK_STREAM_WAVES, 4)
+void skinny_stream_rows_kernel(SkinnyRows p, const bf16* __restrict__ W, bf16* __restrict__ Y, int M, int N, int n_chunks, int k_tiles,
+                               int rows, int act) {
+    extern __shared__ __align__(16) float red[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned char* staged = reinterpret_cast<unsigned char*>(red + SK_STREAM_RED);
+    SkRowStage<XR, MODE> st;
+    st.load(p, M);
+    SkStream<XR, true, true> s;
+    s.run(nullptr, W, M, n_chunks, 0, k_tiles, rows, blockIdx.x, staged, lane, wave, [&] { st.stage(p, M, red, staged); });
+    const float v = sk_stream_total(red, s.acc, lane, wave);
+    if (wave >= 4) return;
+    const int m = 4 * (lane >> 4) + wave, n = blockIdx.x * rows + (lane & 15);
+    if (m < M && (lane & 15) < rows && n < N) Y[(size_t)m * N + n] = __float2bfloat16(sk_result<UNARY>(v, act));
 }
 
 // whole chunks only; offsets inside a row of tiles and inside the activations are 32 bits wide
@@ -598,6 +709,51 @@ static int sk_stream_launch(KERNEL kernel, int xr, unsigned groups, hipStream_t 
 }
 
 extern "C" int bn_skinny_gemm_supports(int M, int N, int K, int ldx, int ldw);
+
+// 1 if bn_skinny_rows takes M rows of K numbers: whole chunks, one a wave at the most, and from 512 numbers on (narrower rows are
+// normed by other kernels, in other orders).
+extern "C" int bn_skinny_rows_supports(int M, int K) {
+    return M >= 1 && M <= SK_ROWS_MAX && K % SK_CHUNK == 0 && K >= 2 * SK_CHUNK && K <= SK_CHUNK * SK_STREAM_WAVES;
+}
+
+// Y[M, N] (bf16, contiguous) = act(rows . W^T) over W's streamed copy (k_tiles tiles along K, tile_rows rows a tile) for rows
+// that are formed on the way: delta null, the rows of x normed with weights w; else x + w delta / rms(delta), which x_new gets too
+// (other memory than x).  All contiguous and 16-byte aligned.  act: 0, BN_ACT_RELU2, or SK_ACT_UNARY plus one of BN_UNARY_*.
+extern "C" int bn_skinny_rows(const float* x, const void* delta, const float* w, float eps, float* x_new, const void* tiles, void* Y, int M,
+                              int N, int K, int k_tiles, int tile_rows, int act, hipStream_t s) {
+    if (!bn_skinny_rows_supports(M, K) || N < 1 || k_tiles != K / BN_STREAM_TILE_COLS || tile_rows < 1 || tile_rows > BN_STREAM_TILE_ROWS ||
+        !x || !w || !tiles || !Y || !delta != !x_new || x == x_new) return BN_ERR_ARG;
+    if (((uintptr_t)x | (uintptr_t)delta | (uintptr_t)w | (uintptr_t)x_new | (uintptr_t)tiles) & 15) return BN_ERR_ARG;
+    if (act != 0 && act != BN_ACT_RELU2 && (act < SK_ACT_UNARY || act >= SK_ACT_UNARY + BN_UNARY_KINDS)) return BN_ERR_ARG;
+    const SkinnyRows p = {x, (const bf16*)delta, w, x_new, K, eps};
+    return sk_stream_pick(M, K, [&](auto xr, auto) {
+        constexpr int XR = decltype(xr)::value < 4 ? decltype(xr)::value : 4;
+        auto go = [&](auto kernel) {
+            const size_t smem = SK_STREAM_RED * sizeof(float) + (size_t)2 * XR * SK_STAGED_ROW(K);
+            hipLaunchKernelGGL(kernel, dim3((N + tile_rows - 1) / tile_rows), dim3(64 * SK_STREAM_WAVES), smem, s, p, (const bf16*)tiles,
+                               (bf16*)Y, M, N, K / SK_CHUNK, k_tiles, tile_rows, act);
+            return bn_launch_status();
+        };
+        if (delta) return act >= SK_ACT_UNARY ? go(skinny_stream_rows_kernel<XR, SK_ROWS_SUM, true>) : go(skinny_stream_rows_kernel<XR, SK_ROWS_SUM, false>);
+        return act >= SK_ACT_UNARY ? go(skinny_stream_rows_kernel<XR, SK_ROWS_NORM, true>) : go(skinny_stream_rows_kernel<XR, SK_ROWS_NORM, false>);
+    });
+}
+
+// resid [M, N] (float32, row stride ld_resid) += X . W^T over W's streamed copy, every result rounded to bf16 first; whole chunks.
+extern "C" int bn_skinny_add(const void* X, const void* tiles, int M, int N, int K, int ldx, int k_tiles, int tile_rows, float* resid,
+                             int ld_resid, hipStream_t s) {
+    if (!bn_skinny_gemm_supports(M, N, K, ldx, 8) || ldx < K || !sk_stream_ok(M, K, ldx) || k_tiles != K / BN_STREAM_TILE_COLS ||
+        tile_rows < 1 || tile_rows > BN_STREAM_TILE_ROWS || !resid || ld_resid < N || (((uintptr_t)X | (uintptr_t)tiles) & 15))
+        return BN_ERR_ARG;
+    SkinnyFused f = {};
+    f.resid = resid; f.ld_resid = ld_resid;
+    return sk_stream_pick(M, K, [&](auto xr, auto one) {
+        constexpr int XR = decltype(xr)::value;
+        return sk_stream_launch(skinny_stream_fused_kernel<XR, decltype(one)::value, SK_FUSED_ADD, 1>, XR, (unsigned)((N + tile_rows - 1) / tile_rows),
+                                s, (const bf16*)X, (const bf16*)tiles, (bf16*)nullptr, M, N, K / SK_CHUNK, ldx, k_tiles, 0, tile_rows, 0, f);
+    });
+}
+
 static bool sk_tiled_ok(int K, int ldw) { return ldw == (K + BN_STREAM_TILE_COLS - 1) / BN_STREAM_TILE_COLS; }
 
 static int sk_compute_units() {

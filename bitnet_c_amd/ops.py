@@ -52,6 +52,7 @@ _SIGNATURES = {
         "bn_unary_act_apply": [c_int, c_void_p, c_void_p, c_longlong, c_int, c_void_p],
         "bn_scale": [c_void_p, c_longlong, c_float, c_void_p],
         "bn_rmsnorm_mean": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
+        "bn_rmsnorm_mean_add": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
         "bn_add_normed_rmsnorm": [c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, c_float, c_void_p, c_void_p, c_int, c_int,
                                   c_float, c_void_p],
     },
@@ -198,6 +199,10 @@ _SIGNATURES = {
         "bn_skinny_gemm_supports": [c_int, c_int, c_int, c_int, c_int],
         "bn_skinny_gemm": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                            c_int, c_int, c_int, c_void_p],
+        "bn_skinny_rows_supports": [c_int, c_int],
+        "bn_skinny_rows": [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
+                           c_int, c_void_p],
+        "bn_skinny_add": [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p],
         "bn_skinny_gemm_fused_tile_cols": [c_int],
         "bn_skinny_gemm_fused_tiles": [c_int, c_int],
         "bn_skinny_group": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
@@ -546,6 +551,7 @@ def gemm_mfma_supported(M: int, N: int, K: int, ldx: int, ldw: int) -> bool:
     return M >= 1 and N >= 1 and K >= 8 and K % 8 == 0 and ldx % 8 == 0 and ldw % 8 == 0 and ldx >= K and ldw >= K
 
 
+SK_CHUNK = _build.header_constant("SK_CHUNK", "skinny_gemm.hip")      # columns of K that a wave of the streaming kernels takes at a time
 SKINNY_ROWS = 16      # bf16 products with more rows than this go to the library
 
 
@@ -957,6 +963,7 @@ class DeferredNorm:
 class StreamNorm(DeferredNorm):
     """An RMSNorm of rows that already lie in the residual stream, left to a product of few rows that norms them on their way
     into its kernel, as add_rmsnorm would (the same bits).  The stream must not change before that product has been launched."""
+    out_dtype: torch.dtype = torch.float32
 
     @property
     def shape(self):
@@ -964,7 +971,7 @@ class StreamNorm(DeferredNorm):
 
     @property
     def dtype(self):
-        return torch.float32
+        return self.out_dtype
 
     @property
     def device(self):
@@ -974,31 +981,93 @@ class StreamNorm(DeferredNorm):
         return add_rmsnorm(self.stream, None, self.weight, self.eps, out_dtype or self.dtype, rows)
 
 
-def stream_norm(stream: torch.Tensor, weight: torch.Tensor, eps: float) -> StreamNorm:
-    return StreamNorm(None, None, stream, weight, float(eps))
+@dataclass
+class StreamSum(StreamNorm):
+    """The residual stream itself once a held-back output (`delta`, bf16) has joined it under a norm of its own (weight, eps),
+    left to a product of few rows that forms the rows on their way into its kernel, as add_normed_rmsnorm would (the same
+    bits).  The new stream is written to memory of its own, since other workgroups may still read the old one, and `owner`
+    (whatever has it as its x) is told.  One reader, at once: until then the stream lacks the output."""
+    delta: torch.Tensor = None
+    owner: object = None
+
+    def materialize(self, out_dtype=None, rows=None) -> torch.Tensor:
+        if rows is not None or out_dtype not in (None, self.dtype):
+            raise KernelError("StreamSum: all rows, in the activations' type")
+        return add_normed_rmsnorm(self.stream, self.delta, self.weight, self.eps, out_dtype=self.dtype, rows_out=True)
+
+
+def stream_norm(stream: torch.Tensor, weight: torch.Tensor, eps: float, dtype=torch.float32) -> StreamNorm:
+    return StreamNorm(None, None, stream, weight, float(eps), dtype)
+
+
+def stream_sum(owner, delta: torch.Tensor, weight: torch.Tensor, eps: float) -> StreamSum:
+    return StreamSum(None, None, owner.x, weight, float(eps), delta.dtype, delta, owner)
 
 
 def can_norm_rows(M: int, K: int, dtype) -> bool:
-    """Whether the float32 products of M rows of K numbers norm their rows themselves."""
-    return (FUSE_NORMS and dtype == torch.float32 and torch.cuda.is_available()
-            and bool(_fn("gemm_f32", "bn_gemm_f32_norm_supports")(M, K)))
+    """Whether products of M rows of K numbers (over streamed copies, in bf16) form their rows from the stream themselves."""
+    if not FUSE_NORMS or dtype not in _DT or not torch.cuda.is_available():
+        return False
+    if dtype == torch.float32:
+        return bool(_fn("gemm_f32", "bn_gemm_f32_norm_supports")(M, K))
+    return bool(_fn("skinny_gemm", "bn_skinny_rows_supports")(M, K))
 
 
-def takes_stream_norm(pre: DeferredNorm, w: torch.Tensor) -> bool:
-    """Whether a product with w norms the rows of pre's stream itself."""
-    return (isinstance(pre, StreamNorm) and w.dtype == torch.float32 and w.shape[1] == pre.stream.shape[1]
-            and can_norm_rows(*pre.stream.shape, w.dtype) and pre.stream.is_contiguous() and pre.stream.data_ptr() % 16 == 0
-            and pre.weight.is_contiguous() and pre.weight.data_ptr() % 16 == 0 and pre.weight.numel() == w.shape[1]
-            and pre.weight.dtype == torch.float32 and f32_product_takes(w))
+def _plain_f32(t, n: int) -> bool:
+    return t.dtype == torch.float32 and t.numel() == n and t.is_contiguous() and t.data_ptr() % 16 == 0
+
+
+def takes_stream_norm(pre: DeferredNorm, w: torch.Tensor, streamed: Optional[StreamedWeight] = None) -> bool:
+    """Whether a product with w (streamed: its streamed copy) forms the rows of a StreamNorm or a StreamSum itself."""
+    if not isinstance(pre, StreamNorm) or w.dtype != pre.dtype or w.dim() != 2:
+        return False
+    M, K = pre.stream.shape
+    if w.shape[1] != K or not can_norm_rows(M, K, w.dtype) or not _plain_f32(pre.stream, M * K) or not _plain_f32(pre.weight, K):
+        return False
+    if isinstance(pre, StreamSum) and not (w.dtype == torch.bfloat16 and tuple(pre.delta.shape) == (M, K)
+                                           and pre.delta.is_contiguous() and pre.delta.data_ptr() % 16 == 0):
+        return False
+    return streamed is not None if w.dtype == torch.bfloat16 else f32_product_takes(w)
 
 
 def linear_stream_norm(pre: StreamNorm, w: torch.Tensor, streamed: Optional[StreamedWeight] = None, glu: bool = False,
-                       activation: str = "silu") -> torch.Tensor:
-    """linear(rmsnorm(stream), w), or with glu linear_swiglu for gate and up interleaved in blocks of 8, in one float32 kernel;
-    for what takes_stream_norm says."""
-    if not takes_stream_norm(pre, w):
+                       activation: Optional[str] = None) -> torch.Tensor:
+    """linear(rows, w) for the rows of a StreamNorm or a StreamSum, in one kernel: activation(linear) (one of
+    UNARY_ACTIVATIONS, bf16), or with glu linear_swiglu for gate and up interleaved in blocks of 8 (float32); for what
+    takes_stream_norm says."""
+    if not takes_stream_norm(pre, w, streamed) or (glu and w.dtype != torch.float32) or (activation and not glu and w.dtype != torch.bfloat16):
         raise KernelError(f"linear_stream_norm: rows {tuple(pre.shape)}, w {tuple(w.shape)} cannot be fused")
-    return _f32_product(pre.stream, w, glu, activation, streamed=streamed, norm=pre)
+    if w.dtype == torch.float32:
+        return _f32_product(pre.stream, w, glu, activation or "silu", streamed=streamed, norm=pre)
+    require_gpu()
+    M, K = pre.stream.shape
+    y = torch.empty((M, w.shape[0]), dtype=torch.bfloat16, device=w.device)
+    tiles, k_tiles, rows = _weight_arg(w, streamed, "linear_stream_norm")
+    act = 0 if activation is None else _act("relu2") if activation == "relu2" else _ACT_UNARY + UNARY_ACTIVATIONS[activation]
+    summed = isinstance(pre, StreamSum)
+    new = torch.empty_like(pre.stream) if summed else None
+    _check(_fn("skinny_gemm", "bn_skinny_rows")(pre.stream.data_ptr(), pre.delta.data_ptr() if summed else None, pre.weight.data_ptr(),
+                                                float(pre.eps), new.data_ptr() if summed else None, tiles, y.data_ptr(), M, w.shape[0],
+                                                K, k_tiles, rows, act, _stream()), "skinny_rows")
+    if summed:
+        pre.owner.x = new
+    return y
+
+
+def linear_add(x: torch.Tensor, w: torch.Tensor, streamed: Optional[StreamedWeight], stream: torch.Tensor) -> bool:
+    """stream (float32 [M, N], in place) += linear(x, w) as add_rmsnorm would add the bf16 result, in the product's kernel;
+    False, and nothing done, where that kernel does not take it (more than 16 rows, no streamed copy, no whole chunks)."""
+    M, K = x.shape
+    N = w.shape[0]
+    if (not FUSE_NORMS or streamed is None or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not 1 <= M <= SKINNY_ROWS
+            or K % SK_CHUNK or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or tuple(stream.shape) != (M, N)
+            or stream.dtype != torch.float32 or not stream.is_contiguous() or not skinny_supported(M, N, K, _rows(x, "x"), 8)):
+        return False
+    require_gpu()
+    tiles, k_tiles, rows = _weight_arg(w, streamed, "linear_add")
+    _check(_fn("skinny_gemm", "bn_skinny_add")(x.data_ptr(), tiles, M, N, K, _rows(x, "x"), k_tiles, rows, stream.data_ptr(), N,
+                                               _stream()), "skinny_add")
+    return True
 
 
 DEFER_ROWS = (17, 128)    # row counts at which a norm is left to its consumer through sum_deferred (below: the fused products)
@@ -1978,9 +2047,19 @@ def sigmoid_gate_(y: torch.Tensor, gate: torch.Tensor) -> None:
                                                 y.shape[0], y.shape[1], _stream()), "sigmoid_gate")
 
 
+WIDE_ROW = _build.header_constant("WIDE_ROW", "elementwise.hip")      # the narrowest row of the kernels that take eight numbers a thread
+
+
+def can_mean_into(*tensors) -> bool:
+    """Whether rmsnorm_mean adds to a stream: rows of whole groups of eight, WIDE_ROW to 8,192 wide, everything 16-byte aligned."""
+    D = tensors[0].shape[-1]
+    return FUSE_NORMS and D % 8 == 0 and WIDE_ROW <= D <= 8192 and all(t.data_ptr() % 16 == 0 and t.is_contiguous() for t in tensors)
+
+
 def rmsnorm_mean(a: torch.Tensor, wa: torch.Tensor, b: Optional[torch.Tensor], wb: Optional[torch.Tensor],
-                 eps: float) -> torch.Tensor:
-    """The mean of two branches [T, D], each under an RMSNorm of its own (float32 weights [D]); b None: a alone."""
+                 eps: float, into: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The mean of two branches [T, D], each under an RMSNorm of its own (float32 weights [D]); b None: a alone.  into: a
+    contiguous float32 [T, D] to which the mean, rounded to the branches' type, is added in the same kernel (can_mean_into)."""
     require_gpu()
     _dev(a, "a", dims=2)
     _dev(wa, "wa", torch.float32, 1)
@@ -1992,6 +2071,16 @@ def rmsnorm_mean(a: torch.Tensor, wa: torch.Tensor, b: Optional[torch.Tensor], w
         _dev(wb, "wb", torch.float32, 1)
         if b.shape != a.shape or not b.is_contiguous() or wb.numel() != D or not wb.is_contiguous():
             raise KernelError("rmsnorm_mean: the branches must be alike")
+    if into is not None:
+        _dev(into, "into", torch.float32, 2)
+        if into.shape != a.shape or not into.is_contiguous():
+            raise KernelError("rmsnorm_mean: into is contiguous and as large as a branch")
+        if T:
+            _check(_fn("elementwise", "bn_rmsnorm_mean_add")(_code(a.dtype), into.data_ptr(), a.data_ptr(),
+                                                             b.data_ptr() if b is not None else None, wa.data_ptr(),
+                                                             wb.data_ptr() if b is not None else None, T, D, float(eps), _stream()),
+                   "rmsnorm_mean(add)")
+        return into
     out = torch.empty_like(a)
     if T:
         _check(_fn("elementwise", "bn_rmsnorm_mean")(_code(a.dtype), out.data_ptr(), a.data_ptr(),

@@ -57,6 +57,7 @@ class Attention(Part):
         return getattr(self.position, "prompt_capturable", False)
 
     takes_deferred_norm = True      # forward accepts an ops.DeferredNorm for h
+    takes_stream_sum = True         # and an ops.StreamSum
     gives_lazy_delta = True         # forward(..., lazy_ok=True) may return a LazyDelta
 
     def __init__(self, hidden: int, n_heads: int, n_kv_heads: int, head_dim: int, scale: float,
@@ -212,8 +213,8 @@ class Attention(Part):
         distance bias, sink and output gate (prompt steps on the matrix cores where the sizes allow, else the vector kernel); the
         output projection."""
         H, Hkv, hs, vd = self.H, self.Hkv, self.hs, self.vd
-        if isinstance(h, ops.DeferredNorm):
-            h = h.materialize()
+        if isinstance(h, ops.DeferredNorm) and not (isinstance(h, ops.StreamNorm) and projected is None and (kv.writes or self.out_gate)):
+            h = h.materialize()               # (a StreamNorm is the first product's alone)
         width = H * hs + Hkv * (hs if self.value_is_key else hs + vd) + (H * vd if self.out_gate else 0)
         if projected is not None:             # the first product's result; the last is left to whoever gave it
             qkv = projected

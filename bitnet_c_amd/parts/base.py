@@ -192,6 +192,14 @@ class LazyDelta:
         return self.linear(self.act)
 
 
+class AddingDelta(LazyDelta):
+    """A part's output that is still to be formed: compute() gives it, add(x) adds it, rounded as it would be, to the stream x
+    [T, D] in the kernel that forms it, and says whether it did (False: nothing has been done)."""
+
+    def __init__(self, compute, add):
+        self.compute, self.add = compute, add
+
+
 class NormedDelta:
     """A part's output that goes through an RMSNorm of its own before it joins the stream (a block with output norms):
     `delta` [T, D] in the activations' type, or ops.PartialSums (float32 slabs that are added first), and the norm.  The
@@ -333,8 +341,18 @@ class ResidualStream:
                 # no norm in front of the next part: the held-back output's norm, the sum, and the new rows handed on
                 from .. import ops
                 p, self.pending = self.pending, None
+                if (getattr(consumer, "takes_stream_sum", False) and isinstance(p.delta, torch.Tensor)
+                        and p.delta.dtype == out_dtype == torch.bfloat16 and ops.can_norm_rows(*self.x.shape, out_dtype)):
+                    return ops.stream_sum(self, p.delta, p.norm.weight, p.norm.eps)      # few rows: the consumer forms them
                 return ops.add_normed_rmsnorm(self.x, p.delta, p.norm.weight, p.norm.eps, out_dtype=out_dtype, rows_out=True)
             self.flush()
+        if isinstance(self.pending, AddingDelta):
+            from .. import ops
+            if (rows is None and getattr(consumer, "takes_deferred_norm", False) and getattr(norm, "deferrable", False)
+                    and self.x.is_contiguous() and ops.can_norm_rows(*self.x.shape, out_dtype) and self.pending.add(self.x)):
+                self.pending = None
+                return ops.stream_norm(self.x, norm.weight, norm.eps, out_dtype)
+            self._pending_tensor()
         if (rows is None and isinstance(self.pending, LazyDelta) and getattr(consumer, "takes_deferred_norm", False)
                 and getattr(norm, "deferrable", False)):
             deferred = self.pending.linear.into_stream(self.pending.act, self.x, norm.weight, norm.eps)

@@ -20,6 +20,7 @@ class DenseFFN(Part):
     gelu, 0.5 z (1 + erf(z / sqrt 2)); the others as the gated unit's)."""
     prompt_capturable = True    # a prompt step is read from the context's device tensors alone
     takes_deferred_norm = True      # forward accepts an ops.DeferredNorm for h (the first product applies the norm)
+    takes_stream_sum = True         # and an ops.StreamSum
     gives_lazy_delta = True         # forward(..., lazy_ok=True) may return a LazyDelta
 
     def __init__(self, hidden: int, intermediate: int, activation: str = "gelu_erf"):
@@ -39,11 +40,7 @@ class DenseFFN(Part):
         return [self.up, self.down]
 
     def forward(self, h, ctx, lazy_ok: bool = False):
-        if isinstance(h, ops.DeferredNorm):
-            a = self.up(h)
-            ops.unary_act(a, self.activation, out=a)
-        else:
-            a = ops.linear_unary(h, self.up.weight, self.activation, self.up.streamed)
+        a = self.up.unary(h, self.activation)
         return self.down.lazy(a) if lazy_ok else self.down(a)
 
 
@@ -121,7 +118,10 @@ class SwiGLU(Part):
         if isinstance(h, ops.DeferredNorm):
             w = self.gate_up.weight
             M = h.shape[0]
-            if not self.has_bias and self.interleaved and ops.takes_stream_norm(h, w):
+            if isinstance(h, ops.StreamNorm) and not (w.dtype == torch.float32 and not self.has_bias and self.interleaved
+                                                      and ops.takes_stream_norm(h, w)):
+                return self.forward(h.materialize(), ctx, lazy_ok)
+            if isinstance(h, ops.StreamNorm):
                 act = ops.linear_stream_norm(h, w, self.gate_up.streamed, True, self.activation)
                 return self.down.lazy(act) if lazy_ok else self.down(act)
             if (not self.has_bias and self.interleaved and w.dtype == torch.bfloat16

@@ -40,17 +40,29 @@ class Linear:
         reads."""
         self.streamed = ops.stream_copy(self.weight, self.stream_tile_rows) if keep and self.stream_bytes() else None
 
+    def unary(self, x, activation: str) -> torch.Tensor:
+        """activation(self(x)) (one of ops.UNARY_ACTIVATIONS; no bias), in the product's kernel where there is one."""
+        if isinstance(x, ops.StreamNorm):
+            if self.weight.dtype == torch.bfloat16 and ops.takes_stream_norm(x, self.weight, self.streamed):
+                return ops.linear_stream_norm(x, self.weight, self.streamed, activation=activation)
+            x = x.materialize()
+        if isinstance(x, ops.DeferredNorm):
+            a = self(x)
+            return ops.unary_act(a, activation, out=a)
+        return ops.linear_unary(x, self.weight, activation, self.streamed)
+
     def __call__(self, x, out_dtype=None, rows: slice | None = None) -> torch.Tensor:
         """x: activations, or an ops.DeferredNorm whose norm this product applies itself when it can."""
         w = self.weight if rows is None else self.weight[rows]
         streamed = self.streamed if rows is None else None
         if isinstance(x, ops.DeferredNorm):
             M, (N, K) = x.shape[0], w.shape
-            if (self.bias is None and out_dtype in (None, torch.bfloat16) and w.dtype == torch.bfloat16
+            if isinstance(x, ops.StreamNorm):
+                if self.bias is None and out_dtype in (None, w.dtype) and ops.takes_stream_norm(x, w, streamed):
+                    return ops.linear_stream_norm(x, w, streamed)
+            elif (self.bias is None and out_dtype in (None, torch.bfloat16) and w.dtype == torch.bfloat16
                     and ops.can_fuse_norm(M, N, K, w.dtype) and w.data_ptr() % 16 == 0):
                 return ops.linear_prenorm(x, w, streamed)
-            if self.bias is None and out_dtype in (None, torch.float32) and ops.takes_stream_norm(x, w):
-                return ops.linear_stream_norm(x, w, streamed)
             x = x.materialize()
         y = ops.linear(x, w, out_dtype, streamed=streamed)
         if self.bias is not None:

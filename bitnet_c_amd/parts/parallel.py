@@ -14,12 +14,14 @@ import dataclasses
 import torch
 
 from .. import ops
-from .base import MIXERS, CacheNeed, ParamSpec, Part, PartSpec, StateNeed
+from .base import MIXERS, AddingDelta, CacheNeed, ParamSpec, Part, PartSpec, StateNeed
 from .linear import upload
 
 
 @MIXERS.register("parallel")
 class ParallelMixer(Part):
+    gives_lazy_delta = True         # forward(..., lazy_ok=True) may return a LazyDelta
+
     def __init__(self, hidden: int, left: PartSpec, right: PartSpec, eps: float):
         self.hidden, self.eps = int(hidden), float(eps)
         self.left, self.right = MIXERS.build(left), MIXERS.build(right)
@@ -63,7 +65,7 @@ class ParallelMixer(Part):
                               device_addressed=a.state.device_addressed and b.state.device_addressed)
         return CacheNeed(kv=a.kv or b.kv, state=state)
 
-    def forward(self, h, ctx, kv):
+    def forward(self, h, ctx, kv, lazy_ok: bool = False):
         kv_a = kv_b = kv
         if self.state_split is not None:
             kv_a = dataclasses.replace(kv, state=kv.state[:, :self.state_split])
@@ -77,4 +79,13 @@ class ParallelMixer(Part):
         else:
             a = self.left.forward(h, ctx, kv_a)
             b = self.right.forward(h, ctx, kv_b)
-        return ops.rmsnorm_mean(a, self.w_left, b, self.w_right, self.eps)
+        args = (a, self.w_left, b, self.w_right)
+        if not lazy_ok or not ops.can_mean_into(*args):
+            return ops.rmsnorm_mean(*args, self.eps)
+
+        def add(x):
+            if x.data_ptr() % 16:
+                return False
+            ops.rmsnorm_mean(*args, self.eps, into=x)
+            return True
+        return AddingDelta(lambda: ops.rmsnorm_mean(*args, self.eps), add)

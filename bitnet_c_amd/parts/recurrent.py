@@ -32,7 +32,7 @@ from __future__ import annotations
 import torch
 
 from .. import ops
-from .base import MIXERS, CacheNeed, ParamSpec, Part, StateNeed
+from .base import MIXERS, AddingDelta, CacheNeed, ParamSpec, Part, StateNeed
 from .linear import Linear, upload
 from .position import rope_frequencies
 
@@ -48,6 +48,7 @@ def _sequences(ctx):
 @MIXERS.register("wkv")
 class WKV(Part):
     prompt_capturable = True    # a prompt step is read from the context's device tensors alone
+    gives_lazy_delta = True         # forward(..., lazy_ok=True) may return a LazyDelta
 
     MIXES = ("r", "k", "v", "g", "w")
 
@@ -90,7 +91,7 @@ class WKV(Part):
         # per head a [head_dim, head_dim] matrix (in the kernel's own order and rounding of its rows), then the last input row
         return CacheNeed(state=StateNeed((self.state_floats + self.hidden,), torch.float32, device_addressed=True))
 
-    def forward(self, h, ctx, kv):
+    def forward(self, h, ctx, kv, lazy_ok: bool = False):
         H, hs = self.H, self.hs
         state = kv.state
         mixes = ops.token_shift(h, self.mu, state[:, self.state_floats:], ctx.positions, ctx.seq_index, ctx.slot_ids)
@@ -103,7 +104,9 @@ class WKV(Part):
             o = ops.wkv_scan(r, k, v, d, self.w0, self.u, h, state, ctx.slot_ids, H, hs, hs,
                              pieces=ops.wkv_in_pieces(h.dtype, ctx.sizes, H, hs, hs), **_sequences(ctx))
             y = ops.head_norm_gate(o, g, self.norm, H, hs, self.eps)
-        return self.o(y)
+        if not lazy_ok:
+            return self.o(y)
+        return AddingDelta(lambda: self.o(y), lambda x: ops.linear_add(y, self.o.weight, self.o.streamed, x))
 
 
 @MIXERS.register("mingru")
@@ -150,6 +153,7 @@ class MinGRU(Part):
 
 class DecayedSums(Part):
     """What linear attention with a constant decay per head shares: the four projections stacked, the decays, the state."""
+    takes_stream_sum = True         # forward accepts an ops.StreamSum for h (the first product alone reads it)
     prompt_capturable = True    # a prompt step is read from the context's device tensors alone
     what = "decayed sums"
 
