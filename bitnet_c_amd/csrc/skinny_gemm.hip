@@ -41,8 +41,6 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast
 
 #define SK_XROW 528           // bytes between rows of a wave's staged X chunk (512 + 16: conflict-free 16-byte reads)
 
-#define SK_ROWS_MAX 8         // rows that a product forms itself: more cost a workgroup more than its weights do
-
 #define SK_STREAM_WAVES 8     // waves of a workgroup over a streamed copy of whole chunks
 
 #define SK_ACT_UNARY 16       // act: this plus one of BN_UNARY_*: an activation of one argument on every result
@@ -585,20 +583,31 @@ void skinny_stream_fused_kernel(const bf16* __restrict__ X, const bf16* __restri
 // the halves of the workgroup take every other row, eight numbers a thread.
 #define SK_ROWS_NORM 0               // x w / rms(x): add_rmsnorm_row_kernel
 #define SK_ROWS_SUM 1                // x + w d / rms(d), the new stream: add_normed_rmsnorm_wide_kernel
+#define SK_ROWS_SHIFT 2              // h + (h' - h) mu for h the normed row and h' the one before it: that, then token_shift_wide_kernel
+#define SK_ROWS_GATE 3               // x w act(gate) / rms(x): row_norm_gate_wide_kernel (lightning.hip)
 struct SkinnyRows {
-    const float* x;                  // [M, K] the stream
-    const bf16* delta;               // [M, K] SUM
+    const float* x;                  // [M, K] the stream (GATE: any rows)
+    const bf16* delta;               // [M, K] SUM; GATE: the gates, rows ld_gate apart
+    int ld_gate, gate_act;           // GATE: BN_UNARY_*
     const float* w;                  // [K]
     float* x_new;                    // [M, K] SUM: where the first workgroup writes the new stream (the others may still read x)
     int K;
     float eps;
+    // SHIFT, row m one token of a sequence of its own: the mixes' weights (of this product), the sequences' state rows, whose
+    // first K numbers are h', the tokens' positions (0: h' is zeros; below: a row that is nobody's), and [M, K] for h
+    const float* mu;
+    const float* state;
+    long long state_stride;
+    const int* positions;
+    const int* slot_ids;
+    bf16* h;
 };
 
 template <int NR, int MODE> struct SkRowStage {
-    float4 x[NR][2], w[2];
+    float4 x[NR][2], w[2], before[NR][2], mu[2];
     uint4 d[NR];
-    int t, half;
-    __device__ __forceinline__ int at(int k) const { return MODE == SK_ROWS_NORM ? (k * 256 + t) * 4 : t * 8 + k * 4; }
+    int t, half, pos[NR];
+    __device__ __forceinline__ int at(int k) const { return MODE == SK_ROWS_SUM || MODE == SK_ROWS_GATE ? t * 8 + k * 4 : (k * 256 + t) * 4; }
     __device__ __forceinline__ void load(const SkinnyRows& p, int M) {
         t = threadIdx.x & 255;
         half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
@@ -606,18 +615,39 @@ template <int NR, int MODE> struct SkRowStage {
         for (int i = 0; i < NR; ++i) {
             const size_t row = (size_t)min(half + 2 * i, M - 1) * p.K;
             if (MODE == SK_ROWS_SUM) d[i] = *reinterpret_cast<const uint4*>(p.delta + row + min(t * 8, p.K - 8));
+            if (MODE == SK_ROWS_GATE)
+                d[i] = *reinterpret_cast<const uint4*>(p.delta + (size_t)min(half + 2 * i, M - 1) * p.ld_gate + min(t * 8, p.K - 8));
 #pragma unroll
             for (int k = 0; k < 2; ++k) x[i][k] = *reinterpret_cast<const float4*>(p.x + row + min(at(k), p.K - 4));
         }
 #pragma unroll
         for (int k = 0; k < 2; ++k) w[k] = *reinterpret_cast<const float4*>(p.w + min(at(k), p.K - 4));
+        if (MODE == SK_ROWS_SHIFT) {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const int row = min(half + 2 * i, M - 1);
+                pos[i] = p.positions[row];
+                const float* from = p.state + (size_t)p.slot_ids[row] * p.state_stride;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) before[i][k] = *reinterpret_cast<const float4*>(from + min(at(k), p.K - 4));
+            }
+#pragma unroll
+            for (int k = 0; k < 2; ++k) mu[k] = *reinterpret_cast<const float4*>(p.mu + min(at(k), p.K - 4));
+        }
     }
     // parts: [2 NR][4] floats; rows: the staged rows.  Two barriers; behind the second the rows are there.
     __device__ __forceinline__ void stage(const SkinnyRows& p, int M, float* parts, unsigned char* rows) {
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
             float ss = 0.f;
-            if (MODE == SK_ROWS_NORM) {
+            if (MODE == SK_ROWS_GATE) {
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    ss = __builtin_fmaf(x[i][k].y, x[i][k].y, __builtin_fmaf(x[i][k].x, x[i][k].x, ss));
+                    ss = __builtin_fmaf(x[i][k].w, x[i][k].w, __builtin_fmaf(x[i][k].z, x[i][k].z, ss));
+                }
+                if (at(0) >= p.K) ss = 0.f;
+            } else if (MODE != SK_ROWS_SUM) {
 #pragma unroll
                 for (int k = 0; k < 2; ++k) ss = at(k) < p.K ? bn_add_squares(ss, x[i][k], k) : ss;
             } else {
@@ -645,8 +675,14 @@ template <int NR, int MODE> struct SkRowStage {
             for (int k = 0; k < 2; ++k) {
                 if (at(k) >= p.K) continue;
                 float4 v;
-                if (MODE == SK_ROWS_NORM) {
+                if (MODE != SK_ROWS_SUM) {
                     v = make_float4(x[i][k].x * f * w[k].x, x[i][k].y * f * w[k].y, x[i][k].z * f * w[k].z, x[i][k].w * f * w[k].w);
+                    if (MODE == SK_ROWS_GATE) {
+                        v.x *= bn_unary_act(bf16lo_to_f32(two[2 * k]), p.gate_act);
+                        v.y *= bn_unary_act(bf16hi_to_f32(two[2 * k]), p.gate_act);
+                        v.z *= bn_unary_act(bf16lo_to_f32(two[2 * k + 1]), p.gate_act);
+                        v.w *= bn_unary_act(bf16hi_to_f32(two[2 * k + 1]), p.gate_act);
+                    }
                 } else {
                     v.x = __builtin_fmaf(bf16lo_to_f32(two[2 * k]) * f, w[k].x, x[i][k].x);
                     v.y = __builtin_fmaf(bf16hi_to_f32(two[2 * k]) * f, w[k].y, x[i][k].y);
@@ -655,6 +691,15 @@ template <int NR, int MODE> struct SkRowStage {
                     if (blockIdx.x == 0 && row < M) *reinterpret_cast<float4*>(p.x_new + (size_t)row * p.K + at(k)) = v;
                 }
                 bf16 o[4] = {from_f32<bf16>(v.x), from_f32<bf16>(v.y), from_f32<bf16>(v.z), from_f32<bf16>(v.w)};
+                if (MODE == SK_ROWS_SHIFT) {
+                    if (blockIdx.x == 0 && row < M) *reinterpret_cast<uint2*>(p.h + (size_t)row * p.K + at(k)) = *reinterpret_cast<const uint2*>(o);
+                    const float b4[4] = {before[i][k].x, before[i][k].y, before[i][k].z, before[i][k].w}, m4[4] = {mu[k].x, mu[k].y, mu[k].z, mu[k].w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float c = to_f32(o[e]), gap = (pos[i] > 0 ? b4[e] : 0.f) - c;
+                        o[e] = from_f32<bf16>(pos[i] >= 0 ? fmaf(gap, m4[e], c) : 0.f);
+                    }
+                }
                 *reinterpret_cast<uint2*>(rows + row * SK_STAGED_ROW(p.K) + at(k) * 2) = *reinterpret_cast<const uint2*>(o);
             }
         }
@@ -677,6 +722,27 @@ void skinny_stream_rows_kernel(SkinnyRows p, const bf16* __restrict__ W, bf16* _
     if (wave >= 4) return;
     const int m = 4 * (lane >> 4) + wave, n = blockIdx.x * rows + (lane & 15);
     if (m < M && (lane & 15) < rows && n < N) Y[(size_t)m * N + n] = __float2bfloat16(sk_result<UNARY>(v, act));
+}
+
+// Several such products of the same rows in one launch; SHIFT: product j's mixes have the weights mu + j K.
+template <int XR, int MODE>
+__global__ __launch_bounds__(64 * SK_STREAM_WAVES, 4)
+void skinny_stream_rows_group_kernel(SkinnyGroup g, SkinnyRows p, int M, int n_chunks, int k_tiles) {
+    extern __shared__ __align__(16) float red[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned char* staged = reinterpret_cast<unsigned char*>(red + SK_STREAM_RED);
+    int j = 0;
+    while (j + 1 < g.count && (int)blockIdx.x >= g.first[j + 1]) ++j;
+    if (MODE == SK_ROWS_SHIFT) p.mu += (size_t)j * p.K;
+    const int rows = g.rows[j], bx = (int)blockIdx.x - g.first[j];
+    SkRowStage<XR, MODE> st;
+    st.load(p, M);
+    SkStream<XR, true, true> s;
+    s.run(nullptr, g.w[j], M, n_chunks, 0, k_tiles, rows, bx, staged, lane, wave, [&] { st.stage(p, M, red, staged); });
+    const float v = sk_stream_total(red, s.acc, lane, wave);
+    if (wave >= 4) return;
+    const int m = 4 * (lane >> 4) + wave, n = bx * rows + (lane & 15);
+    if (m < M && (lane & 15) < rows && n < g.n[j]) g.y[j][(size_t)m * g.n[j] + n] = __float2bfloat16(sk_result<true>(v, g.act[j]));
 }
 
 // whole chunks only; offsets inside a row of tiles and inside the activations are 32 bits wide
@@ -710,10 +776,14 @@ static int sk_stream_launch(KERNEL kernel, int xr, unsigned groups, hipStream_t 
 
 extern "C" int bn_skinny_gemm_supports(int M, int N, int K, int ldx, int ldw);
 
-// 1 if bn_skinny_rows takes M rows of K numbers: whole chunks, one a wave at the most, and from 512 numbers on (narrower rows are
-// normed by other kernels, in other orders).
-extern "C" int bn_skinny_rows_supports(int M, int K) {
-    return M >= 1 && M <= SK_ROWS_MAX && K % SK_CHUNK == 0 && K >= 2 * SK_CHUNK && K <= SK_CHUNK * SK_STREAM_WAVES;
+// 1 if products form M rows of K numbers themselves (mode: SK_ROWS_*): whole chunks, one a wave at the most, and from 512 numbers on,
+// gated ones from 1,024 (narrower rows are normed by other kernels, in other orders).  Up to the rows where that is the faster way: us
+// at 1 / 2 / 4 / 8 rows of 2,048 numbers, two kernels -> one: normed rows x 8,192 9.7 / 10.1 / 10.1 / 10.6 -> 7.6 / 7.5 / 8.0 / 9.5; the new
+// stream's x 8,192 9.3 / 9.4 / 9.9 / 10.2 -> 7.4 / 7.5 / 8.6 / 10.9; gated x 2,048 7.0 / 7.1 / 7.1 / 7.9 -> 5.0 / 5.0 / 7.4 / 11.4; five mixes x 4 x
+// 2,048 and 64, three kernels -> one, 13.6 / 13.9 / 14.2 / 15.5 -> 11.1 / 11.0 / 13.6 / 19.6.
+extern "C" int bn_skinny_rows_supports(int M, int K, int mode) {
+    const int most = mode == SK_ROWS_NORM ? 8 : mode == SK_ROWS_SUM || mode == SK_ROWS_SHIFT ? 4 : mode == SK_ROWS_GATE ? 2 : 0;
+    return M >= 1 && M <= most && K % SK_CHUNK == 0 && K >= (mode == SK_ROWS_GATE ? 4 : 2) * SK_CHUNK && K <= SK_CHUNK * SK_STREAM_WAVES;
 }
 
 // Y[M, N] (bf16, contiguous) = act(rows . W^T) over W's streamed copy (k_tiles tiles along K, tile_rows rows a tile) for rows
@@ -721,22 +791,38 @@ extern "C" int bn_skinny_rows_supports(int M, int K) {
 // (other memory than x).  All contiguous and 16-byte aligned.  act: 0, BN_ACT_RELU2, or SK_ACT_UNARY plus one of BN_UNARY_*.
 extern "C" int bn_skinny_rows(const float* x, const void* delta, const float* w, float eps, float* x_new, const void* tiles, void* Y, int M,
                               int N, int K, int k_tiles, int tile_rows, int act, hipStream_t s) {
-    if (!bn_skinny_rows_supports(M, K) || N < 1 || k_tiles != K / BN_STREAM_TILE_COLS || tile_rows < 1 || tile_rows > BN_STREAM_TILE_ROWS ||
+    if (!bn_skinny_rows_supports(M, K, delta ? SK_ROWS_SUM : SK_ROWS_NORM) || N < 1 || k_tiles != K / BN_STREAM_TILE_COLS || tile_rows < 1 || tile_rows > BN_STREAM_TILE_ROWS ||
         !x || !w || !tiles || !Y || !delta != !x_new || x == x_new) return BN_ERR_ARG;
     if (((uintptr_t)x | (uintptr_t)delta | (uintptr_t)w | (uintptr_t)x_new | (uintptr_t)tiles) & 15) return BN_ERR_ARG;
     if (act != 0 && act != BN_ACT_RELU2 && (act < SK_ACT_UNARY || act >= SK_ACT_UNARY + BN_UNARY_KINDS)) return BN_ERR_ARG;
-    const SkinnyRows p = {x, (const bf16*)delta, w, x_new, K, eps};
+    SkinnyRows p = {};
+    p.x = x; p.delta = (const bf16*)delta; p.w = w; p.x_new = x_new; p.K = K; p.eps = eps;
     return sk_stream_pick(M, K, [&](auto xr, auto) {
-        constexpr int XR = decltype(xr)::value < 4 ? decltype(xr)::value : 4;
+        constexpr int XR = decltype(xr)::value < 4 ? decltype(xr)::value : 4, FEW = XR < 2 ? XR : 2;
         auto go = [&](auto kernel) {
             const size_t smem = SK_STREAM_RED * sizeof(float) + (size_t)2 * XR * SK_STAGED_ROW(K);
             hipLaunchKernelGGL(kernel, dim3((N + tile_rows - 1) / tile_rows), dim3(64 * SK_STREAM_WAVES), smem, s, p, (const bf16*)tiles,
                                (bf16*)Y, M, N, K / SK_CHUNK, k_tiles, tile_rows, act);
             return bn_launch_status();
         };
-        if (delta) return act >= SK_ACT_UNARY ? go(skinny_stream_rows_kernel<XR, SK_ROWS_SUM, true>) : go(skinny_stream_rows_kernel<XR, SK_ROWS_SUM, false>);
+        if (delta) return act >= SK_ACT_UNARY ? go(skinny_stream_rows_kernel<FEW, SK_ROWS_SUM, true>) : go(skinny_stream_rows_kernel<FEW, SK_ROWS_SUM, false>);
         return act >= SK_ACT_UNARY ? go(skinny_stream_rows_kernel<XR, SK_ROWS_NORM, true>) : go(skinny_stream_rows_kernel<XR, SK_ROWS_NORM, false>);
     });
+}
+
+// Y[M, N] (bf16, contiguous) = rows . W^T, the rows x w act(gate) / rms(x): x [M, K] float32 contiguous, gate bf16 with row stride
+// ld_gate, act one of BN_UNARY_*; W's streamed copy as above.
+extern "C" int bn_skinny_gated_rows(const float* x, const void* gate, int ld_gate, int act, const float* w, float eps, const void* tiles, void* Y,
+                                    int M, int N, int K, int k_tiles, int tile_rows, hipStream_t s) {
+    if (!bn_skinny_rows_supports(M, K, SK_ROWS_GATE) || N < 1 || k_tiles != K / BN_STREAM_TILE_COLS || tile_rows < 1 || tile_rows > BN_STREAM_TILE_ROWS ||
+        !x || !gate || !w || !tiles || !Y || ld_gate < K || ld_gate % 8 || act < 0 || act >= BN_UNARY_KINDS) return BN_ERR_ARG;
+    if (((uintptr_t)x | (uintptr_t)gate | (uintptr_t)w | (uintptr_t)tiles) & 15) return BN_ERR_ARG;
+    SkinnyRows p = {};
+    p.x = x; p.delta = (const bf16*)gate; p.ld_gate = ld_gate; p.gate_act = act; p.w = w; p.K = K; p.eps = eps;
+    const size_t smem = SK_STREAM_RED * sizeof(float) + (size_t)2 * SK_STAGED_ROW(K);
+    hipLaunchKernelGGL((skinny_stream_rows_kernel<1, SK_ROWS_GATE, false>), dim3((N + tile_rows - 1) / tile_rows), dim3(64 * SK_STREAM_WAVES),
+                       smem, s, p, (const bf16*)tiles, (bf16*)Y, M, N, K / SK_CHUNK, k_tiles, tile_rows, 0);
+    return bn_launch_status();
 }
 
 // resid [M, N] (float32, row stride ld_resid) += X . W^T over W's streamed copy, every result rounded to bf16 first; whole chunks.
@@ -1028,4 +1114,39 @@ extern "C" int bn_skinny_group(int count, const void* const* X, const void* cons
     }
     hipLaunchKernelGGL(skinny_group_kernel, dim3(groups), dim3(n_waves * 64), smem, s, p, M, K, k_tiles);
     return bn_launch_status();
+}
+
+// The same for products of rows that are formed on the way (bn_skinny_rows' norm of the rows of x [M, K] with weights w).  mu null:
+// of these rows; else of their mixes with the rows before them, product j's with weights mu + j K (SkinnyRows), and h [M, K] (bf16)
+// gets the normed rows.  All contiguous and 16-byte aligned, state_stride a multiple of 4.
+extern "C" int bn_skinny_rows_group(const float* x, const float* w, float eps, const float* mu, const float* state, long long state_stride,
+                                    const int* positions, const int* slot_ids, void* h, int count, const void* const* W, void* const* Y,
+                                    const int* N, const int* tile_rows, const int* unary, int M, int K, int k_tiles, hipStream_t s) {
+    if (count < 1 || count > SK_GROUP || !bn_skinny_rows_supports(M, K, mu ? SK_ROWS_SHIFT : SK_ROWS_NORM) || k_tiles != K / BN_STREAM_TILE_COLS || !x || !w) return BN_ERR_ARG;
+    if (mu && (!state || !positions || !slot_ids || !h || state_stride < K || state_stride % 4)) return BN_ERR_ARG;
+    if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)mu | (uintptr_t)(mu ? state : nullptr) | (uintptr_t)(mu ? h : nullptr)) & 15) return BN_ERR_ARG;
+    SkinnyGroup g = {};
+    g.count = count;
+    int groups = 0;
+    for (int j = 0; j < count; ++j) {
+        if (N[j] < 1 || tile_rows[j] < 1 || tile_rows[j] > BN_STREAM_TILE_ROWS || unary[j] < -1 || unary[j] >= BN_UNARY_KINDS || !W[j] ||
+            ((uintptr_t)W[j] & 15) || !Y[j])
+            return BN_ERR_ARG;
+        g.w[j] = (const bf16*)W[j]; g.y[j] = (bf16*)Y[j];
+        g.n[j] = N[j]; g.rows[j] = tile_rows[j]; g.act[j] = unary[j] < 0 ? 0 : SK_ACT_UNARY + unary[j];
+        g.first[j] = groups;
+        groups += (N[j] + tile_rows[j] - 1) / tile_rows[j];
+    }
+    SkinnyRows p = {};
+    p.x = x; p.w = w; p.K = K; p.eps = eps;
+    p.mu = mu; p.state = state; p.state_stride = state_stride; p.positions = positions; p.slot_ids = slot_ids; p.h = (bf16*)h;
+    return sk_stream_pick(M, K, [&](auto xr, auto) {
+        constexpr int XR = decltype(xr)::value < 4 ? decltype(xr)::value : 4, FEW = XR < 2 ? XR : 2;
+        auto go = [&](auto kernel) {
+            const size_t smem = SK_STREAM_RED * sizeof(float) + (size_t)2 * XR * SK_STAGED_ROW(K);
+            hipLaunchKernelGGL(kernel, dim3(groups), dim3(64 * SK_STREAM_WAVES), smem, s, g, p, M, K / SK_CHUNK, k_tiles);
+            return bn_launch_status();
+        };
+        return mu ? go(skinny_stream_rows_group_kernel<FEW, SK_ROWS_SHIFT>) : go(skinny_stream_rows_group_kernel<XR, SK_ROWS_NORM>);
+    });
 }

@@ -199,9 +199,13 @@ _SIGNATURES = {
         "bn_skinny_gemm_supports": [c_int, c_int, c_int, c_int, c_int],
         "bn_skinny_gemm": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                            c_int, c_int, c_int, c_void_p],
-        "bn_skinny_rows_supports": [c_int, c_int],
+        "bn_skinny_rows_supports": [c_int, c_int, c_int],
         "bn_skinny_rows": [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                            c_int, c_void_p],
+        "bn_skinny_rows_group": [c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p, c_int,
+                                 c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
+        "bn_skinny_gated_rows": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                 c_int, c_void_p],
         "bn_skinny_add": [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p],
         "bn_skinny_gemm_fused_tile_cols": [c_int],
         "bn_skinny_gemm_fused_tiles": [c_int, c_int],
@@ -1004,13 +1008,17 @@ def stream_sum(owner, delta: torch.Tensor, weight: torch.Tensor, eps: float) -> 
     return StreamSum(None, None, owner.x, weight, float(eps), delta.dtype, delta, owner)
 
 
-def can_norm_rows(M: int, K: int, dtype) -> bool:
-    """Whether products of M rows of K numbers (over streamed copies, in bf16) form their rows from the stream themselves."""
+ROWS_NORM, ROWS_SUM, ROWS_SHIFT, ROWS_GATE = (_build.header_constant("SK_ROWS_" + n, "skinny_gemm.hip") for n in ("NORM", "SUM", "SHIFT", "GATE"))
+
+
+def can_norm_rows(M: int, K: int, dtype, form: int = ROWS_NORM) -> bool:
+    """Whether products of M rows of K numbers (over streamed copies, in bf16) form their rows themselves: normed (form ROWS_NORM),
+    in bf16 also a StreamSum's (ROWS_SUM), mixes with the rows before them (ROWS_SHIFT), normed and gated ones (ROWS_GATE)."""
     if not FUSE_NORMS or dtype not in _DT or not torch.cuda.is_available():
         return False
     if dtype == torch.float32:
-        return bool(_fn("gemm_f32", "bn_gemm_f32_norm_supports")(M, K))
-    return bool(_fn("skinny_gemm", "bn_skinny_rows_supports")(M, K))
+        return form == ROWS_NORM and bool(_fn("gemm_f32", "bn_gemm_f32_norm_supports")(M, K))
+    return bool(_fn("skinny_gemm", "bn_skinny_rows_supports")(M, K, form))
 
 
 def _plain_f32(t, n: int) -> bool:
@@ -1022,7 +1030,7 @@ def takes_stream_norm(pre: DeferredNorm, w: torch.Tensor, streamed: Optional[Str
     if not isinstance(pre, StreamNorm) or w.dtype != pre.dtype or w.dim() != 2:
         return False
     M, K = pre.stream.shape
-    if w.shape[1] != K or not can_norm_rows(M, K, w.dtype) or not _plain_f32(pre.stream, M * K) or not _plain_f32(pre.weight, K):
+    if w.shape[1] != K or not can_norm_rows(M, K, w.dtype, ROWS_SUM if isinstance(pre, StreamSum) else ROWS_NORM) or not _plain_f32(pre.stream, M * K) or not _plain_f32(pre.weight, K):
         return False
     if isinstance(pre, StreamSum) and not (w.dtype == torch.bfloat16 and tuple(pre.delta.shape) == (M, K)
                                            and pre.delta.is_contiguous() and pre.delta.data_ptr() % 16 == 0):
@@ -1052,6 +1060,65 @@ def linear_stream_norm(pre: StreamNorm, w: torch.Tensor, streamed: Optional[Stre
     if summed:
         pre.owner.x = new
     return y
+
+
+def can_group_stream_norm(M: int, K: int, linears, shift: bool = False) -> bool:
+    """Whether linear_group_stream_norm takes M rows and these parts.linear.Linear (without biases) of K columns."""
+    return (len(linears) <= GROUP_PRODUCTS and can_norm_rows(M, K, torch.bfloat16, ROWS_SHIFT if shift else ROWS_NORM)
+            and all(l.bias is None and l.weight.dtype == torch.bfloat16 and l.weight.shape[1] == K and l.streamed is not None for l in linears))
+
+
+def linear_group_stream_norm(pre: StreamNorm, items, shift=None) -> list:
+    """[linear(rows, w) or activation(linear(rows, w))] for items (w, streamed copy, activation or None) that read the rows of one
+    StreamNorm, in one launch, for what can_group_stream_norm says.  shift = (mu [items, K], state, positions, slot_ids): a
+    decode step's token_shift in front of them; item j reads mix j, and the normed rows are the list's last entry."""
+    require_gpu()
+    items = list(items)
+    M, K = pre.stream.shape
+    n = len(items)
+    if (isinstance(pre, StreamSum) or not 1 <= n <= GROUP_PRODUCTS
+            or not can_norm_rows(M, K, torch.bfloat16, ROWS_NORM if shift is None else ROWS_SHIFT)
+            or not all(takes_stream_norm(pre, w, sw) for w, sw, _ in items)):
+        raise KernelError(f"linear_group_stream_norm: rows {tuple(pre.shape)} and {n} products cannot be fused")
+    more = [None, None, 0, None, None, None]
+    h = None
+    if shift is not None:
+        mu, state, positions, slot_ids = shift
+        stride = _state_rows(state, K, "linear_group_stream_norm")
+        for t, nm in ((positions, "positions"), (slot_ids, "slot_ids")):
+            _dev(t, nm, torch.int32, 1)
+            if t.numel() != M or not t.is_contiguous():
+                raise KernelError(f"linear_group_stream_norm: {nm} has one entry per row")
+        if not _plain_f32(mu, n * K) or stride % 4 or state.data_ptr() % 16:
+            raise KernelError("linear_group_stream_norm: mu float32 contiguous [products, K], state rows 16-byte aligned")
+        h = torch.empty((M, K), dtype=torch.bfloat16, device=mu.device)
+        more = [mu.data_ptr(), state.data_ptr(), stride, positions.data_ptr(), slot_ids.data_ptr(), h.data_ptr()]
+    ys = [torch.empty((M, w.shape[0]), dtype=torch.bfloat16, device=w.device) for w, _, _ in items]
+    args = [_weight_arg(w, sw, "linear_group_stream_norm") for w, sw, _ in items]
+    ptr, num = c_void_p * n, c_int * n
+    _check(_fn("skinny_gemm", "bn_skinny_rows_group")(
+        pre.stream.data_ptr(), pre.weight.data_ptr(), float(pre.eps), *more, n, ptr(*[a[0] for a in args]), ptr(*[y.data_ptr() for y in ys]),
+        num(*[w.shape[0] for w, _, _ in items]), num(*[a[2] for a in args]),
+        num(*[-1 if act is None else UNARY_ACTIVATIONS[act] for _, _, act in items]), M, K, args[0][1], _stream()), "skinny_rows_group")
+    return ys + ([h] if h is not None else [])
+
+
+def linear_row_norm_gate(o: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, eps: float, activation: str, w: torch.Tensor,
+                         streamed: Optional[StreamedWeight] = None) -> torch.Tensor:
+    """linear(row_norm_gate(o, gate, weight, eps, activation), w): one kernel for bf16 steps of few rows over a streamed copy (the
+    same bits), else the two."""
+    M, K = o.shape
+    if (FUSE_NORMS and streamed is not None and gate.dtype == w.dtype == torch.bfloat16 and w.shape[1] == K and gate.shape == o.shape
+            and can_norm_rows(M, K, w.dtype, ROWS_GATE) and activation in UNARY_ACTIVATIONS and _plain_f32(o, M * K)
+            and _plain_f32(weight, K) and gate.stride(1) == 1 and _rows(gate, "gate") % 8 == 0 and gate.data_ptr() % 16 == 0):
+        require_gpu()
+        y = torch.empty((M, w.shape[0]), dtype=torch.bfloat16, device=w.device)
+        tiles, k_tiles, rows = _weight_arg(w, streamed, "linear_row_norm_gate")
+        _check(_fn("skinny_gemm", "bn_skinny_gated_rows")(o.data_ptr(), gate.data_ptr(), _rows(gate, "gate"), UNARY_ACTIVATIONS[activation],
+                                                          weight.data_ptr(), float(eps), tiles, y.data_ptr(), M, w.shape[0], K, k_tiles,
+                                                          rows, _stream()), "skinny_gated_rows")
+        return y
+    return linear(row_norm_gate(o, gate, weight, eps, activation), w, streamed=streamed)
 
 
 def linear_add(x: torch.Tensor, w: torch.Tensor, streamed: Optional[StreamedWeight], stream: torch.Tensor) -> bool:

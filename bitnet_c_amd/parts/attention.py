@@ -213,7 +213,7 @@ class Attention(Part):
         distance bias, sink and output gate (prompt steps on the matrix cores where the sizes allow, else the vector kernel); the
         output projection."""
         H, Hkv, hs, vd = self.H, self.Hkv, self.hs, self.vd
-        if isinstance(h, ops.DeferredNorm) and not (isinstance(h, ops.StreamNorm) and projected is None and (kv.writes or self.out_gate)):
+        if projected is None and isinstance(h, ops.DeferredNorm) and not (isinstance(h, ops.StreamNorm) and (kv.writes or self.out_gate)):
             h = h.materialize()               # (a StreamNorm is the first product's alone)
         width = H * hs + Hkv * (hs if self.value_is_key else hs + vd) + (H * vd if self.out_gate else 0)
         if projected is not None:             # the first product's result; the last is left to whoever gave it

@@ -191,6 +191,11 @@ class LazyDelta:
     def compute(self) -> torch.Tensor:
         return self.linear(self.act)
 
+    def add(self, x: torch.Tensor) -> bool:
+        """Adds compute() to x [T, D] in the product's kernel, rounded as it would be; False: nothing has been done."""
+        from .. import ops
+        return self.linear.bias is None and ops.linear_add(self.act, self.linear.weight, self.linear.streamed, x)
+
 
 class AddingDelta(LazyDelta):
     """A part's output that is still to be formed: compute() gives it, add(x) adds it, rounded as it would be, to the stream x
@@ -342,16 +347,21 @@ class ResidualStream:
                 from .. import ops
                 p, self.pending = self.pending, None
                 if (getattr(consumer, "takes_stream_sum", False) and isinstance(p.delta, torch.Tensor)
-                        and p.delta.dtype == out_dtype == torch.bfloat16 and ops.can_norm_rows(*self.x.shape, out_dtype)):
+                        and p.delta.dtype == out_dtype == torch.bfloat16 and ops.can_norm_rows(*self.x.shape, out_dtype, ops.ROWS_SUM)):
                     return ops.stream_sum(self, p.delta, p.norm.weight, p.norm.eps)      # few rows: the consumer forms them
                 return ops.add_normed_rmsnorm(self.x, p.delta, p.norm.weight, p.norm.eps, out_dtype=out_dtype, rows_out=True)
             self.flush()
-        if isinstance(self.pending, AddingDelta):
+        if rows is None and (isinstance(self.pending, LazyDelta) or self.pending is None) and getattr(norm, "deferrable", False):
             from .. import ops
-            if (rows is None and getattr(consumer, "takes_deferred_norm", False) and getattr(norm, "deferrable", False)
-                    and self.x.is_contiguous() and ops.can_norm_rows(*self.x.shape, out_dtype) and self.pending.add(self.x)):
+            # few rows: the output adds itself to the stream, rounded as it would be, and the consumer forms the normed rows
+            asks = getattr(consumer, "wants_stream_norm", None)
+            wants = asks(ctx, self.x.shape[0]) if asks is not None and ctx is not None else (
+                isinstance(self.pending, AddingDelta) and getattr(consumer, "takes_deferred_norm", False))
+            if (wants and out_dtype == torch.bfloat16 and self.x.is_contiguous() and ops.can_norm_rows(*self.x.shape, out_dtype)
+                    and (self.pending is None or self.pending.add(self.x))):
                 self.pending = None
                 return ops.stream_norm(self.x, norm.weight, norm.eps, out_dtype)
+        if isinstance(self.pending, AddingDelta):
             self._pending_tensor()
         if (rows is None and isinstance(self.pending, LazyDelta) and getattr(consumer, "takes_deferred_norm", False)
                 and getattr(norm, "deferrable", False)):

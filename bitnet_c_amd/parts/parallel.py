@@ -65,15 +65,26 @@ class ParallelMixer(Part):
                               device_addressed=a.state.device_addressed and b.state.device_addressed)
         return CacheNeed(kv=a.kv or b.kv, state=state)
 
+    def wants_stream_norm(self, ctx, rows: int) -> bool:
+        """Whether forward is better given its rows undone (an ops.StreamNorm)."""
+        ends = [getattr(m, "ends", None) for m in (self.left, self.right)]
+        return all(ends) and ops.can_group_stream_norm(rows, self.hidden, [first for first, _ in ends])
+
     def forward(self, h, ctx, kv, lazy_ok: bool = False):
         kv_a = kv_b = kv
         if self.state_split is not None:
             kv_a = dataclasses.replace(kv, state=kv.state[:, :self.state_split])
             kv_b = dataclasses.replace(kv, state=kv.state[:, self.state_split:])
         ends = [getattr(m, "ends", None) for m in (self.left, self.right)]
-        if all(ends) and kv.writes and isinstance(h, torch.Tensor):
+        undone = isinstance(h, ops.StreamNorm)
+        if undone and not (all(ends) and kv.writes):
+            h, undone = h.materialize(), False
+        if undone:                               # the rows are formed in the first products' kernel
+            pa, pb = ops.linear_group_stream_norm(h, [(first.weight, first.streamed, None) for first, _ in ends])
+        elif all(ends) and kv.writes and isinstance(h, torch.Tensor):
             # both read h, and neither's last product waits for the other: two launches instead of four where steps are short
             pa, pb = ops.linear_group([(h, first.weight, first.streamed, None) for first, _ in ends])
+        if undone or (all(ends) and kv.writes and isinstance(h, torch.Tensor)):
             ya, yb = self.left.forward(h, ctx, kv_a, projected=pa), self.right.forward(h, ctx, kv_b, projected=pb)
             a, b = ops.linear_group([(y, last.weight, last.streamed, None) for y, (_, last) in zip((ya, yb), ends)])
         else:

@@ -87,6 +87,15 @@ class WKV(Part):
     def linears(self):
         return [self.r, self.k, self.v, self.g, self.w1, self.w2, self.o]
 
+    def _first(self):
+        return [self.r, self.k, self.v, self.g, self.w1]
+
+    def wants_stream_norm(self, ctx, rows: int) -> bool:
+        """Whether forward is better given its rows undone (an ops.StreamNorm): decode steps whose products form them; the row
+        of the token before lies behind the heads' matrices, which has to leave it 16-byte aligned."""
+        return bool(ctx.is_decode and self.state_floats % 4 == 0 and self.hidden % 4 == 0
+                    and ops.can_group_stream_norm(rows, self.hidden, self._first(), shift=True))
+
     def cache_need(self) -> CacheNeed:
         # per head a [head_dim, head_dim] matrix (in the kernel's own order and rounding of its rows), then the last input row
         return CacheNeed(state=StateNeed((self.state_floats + self.hidden,), torch.float32, device_addressed=True))
@@ -94,9 +103,15 @@ class WKV(Part):
     def forward(self, h, ctx, kv, lazy_ok: bool = False):
         H, hs = self.H, self.hs
         state = kv.state
-        mixes = ops.token_shift(h, self.mu, state[:, self.state_floats:], ctx.positions, ctx.seq_index, ctx.slot_ids)
-        r, k, v, g, low = ops.linear_group([(x, l.weight, l.streamed, None) for x, l in zip(mixes, (self.r, self.k, self.v, self.g))]
-                                           + [(mixes[4], self.w1.weight, self.w1.streamed, "tanh")])
+        last = state[:, self.state_floats:]               # the rows of the tokens before
+        if isinstance(h, ops.StreamNorm):                 # a decode step of few rows: norm and mixes are formed in the products' kernel
+            r, k, v, g, low, h = ops.linear_group_stream_norm(h, [(l.weight, l.streamed, "tanh" if l is self.w1 else None)
+                                                                  for l in self._first()],
+                                                              (self.mu, last, ctx.positions, ctx.slot_ids))
+        else:
+            mixes = ops.token_shift(h, self.mu, last, ctx.positions, ctx.seq_index, ctx.slot_ids)
+            r, k, v, g, low = ops.linear_group([(x, l.weight, l.streamed, "tanh" if l is self.w1 else None)
+                                                for x, l in zip(mixes, self._first())])
         d = self.w2(low)
         if ctx.is_decode and ops.wkv_step_supported(hs, hs):
             y = ops.wkv_step(r, k, v, d, self.w0, self.u, h, state, ctx.slot_ids, H, hs, hs, ctx.seq_lens, g, self.norm, self.eps)
@@ -224,8 +239,7 @@ class Lightning(DecayedSums):
         x = self.qkvg(h)
         o = ops.lightning_scan(x, 0, self.k_col, self.v_col, self.decay, kv.state, ctx.slot_ids, self.H, self.hs, self.vd,
                                **_sequences(ctx))
-        y = ops.row_norm_gate(o, x[:, self.g_col:], self.norm, self.eps, self.gate_activation)
-        return self.o(y)
+        return ops.linear_row_norm_gate(o, x[:, self.g_col:], self.norm, self.eps, self.gate_activation, self.o.weight, self.o.streamed)
 
 
 @MIXERS.register("retention")

@@ -42,6 +42,9 @@ def test_products_form_their_rows(M, N, K, R):
         assert ops.takes_stream_norm(pre, w, sw) and not ops.takes_stream_norm(pre, w, None)
         want = ops.linear(h, w, streamed=sw) if act is None else ops.linear_unary(h, w, act, sw)
         assert _same(ops.linear_stream_norm(pre, w, sw, activation=act), want), act
+    if not ops.can_norm_rows(M, K, torch.bfloat16, ops.ROWS_SUM):
+        assert M > 4
+        return
     new = x.clone()
     h = ops.add_normed_rmsnorm(new, d, nw, 1e-6, out_dtype=torch.bfloat16, rows_out=True)
     for act in (None, "relu2", "gelu_erf"):
@@ -52,6 +55,47 @@ def test_products_form_their_rows(M, N, K, R):
         assert _same(got, want) and _same(owner.x, new) and _same(old, x) and owner.x is not old, act
     owner = types.SimpleNamespace(x=x.clone())
     assert _same(ops.stream_sum(owner, d, nw, 1e-6).materialize(), h) and _same(owner.x, new)
+
+
+# several products of the same rows, as they are or mixed with the rows before them (a token without one, a row that is nobody's)
+@pytest.mark.parametrize("M", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("K", [512, 768, 2048])
+def test_groups_form_their_rows(M, K):
+    ops = _ops()
+    x, _, nw, g = _rows(M, K, M + K)
+    items = []
+    for N, R, act in ((33, 16, None), (40, 8, "tanh"), (1, 12, None)):
+        w = torch.randn(N, K, generator=g).bfloat16().cuda()
+        items.append((w, ops.stream_copy(w, R), act))
+    h = ops.add_rmsnorm(x.clone(), None, nw, 1e-5, torch.bfloat16)
+    pre = ops.stream_norm(x, nw, 1e-5, torch.bfloat16)
+    for got, want in zip(ops.linear_group_stream_norm(pre, items), ops.linear_group([(h, *i) for i in items])):
+        assert _same(got, want)
+    if not ops.can_norm_rows(M, K, torch.bfloat16, ops.ROWS_SHIFT):
+        assert M > 4
+        return
+    mu = torch.rand(len(items), K, generator=g).cuda()
+    state = torch.randn(M + 2, K + 12, generator=g).cuda()[:, 8:]
+    slots = torch.arange(M + 1, 1, -1, dtype=torch.int32).cuda()
+    positions = torch.tensor([(5, 0, -1)[m % 3] for m in range(M)], dtype=torch.int32).cuda()
+    mixes = ops.token_shift(h, mu, state, positions, torch.arange(M, dtype=torch.int32).cuda(), slots)
+    got = ops.linear_group_stream_norm(pre, items, (mu, state, positions, slots))
+    assert _same(got[-1], h)
+    for a, b in zip(got, ops.linear_group([(m, *i) for m, i in zip(mixes, items)])):
+        assert _same(a, b)
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("N,K,R", [(33, 1024, 8), (24, 1792, 16), (40, 2048, 12), (16, 768, 16)])
+def test_products_norm_and_gate_their_rows(M, N, K, R):
+    ops = _ops()
+    o, _, nw, g = _rows(M, K, M + N + K)
+    wide = torch.randn(M, K + 16, generator=g).bfloat16().cuda()
+    w = torch.randn(N, K, generator=g).bfloat16().cuda()
+    for gate in (wide[:, :K], wide[:, 8:K + 8], wide[:, 1:K + 1]):
+        for act in ("sigmoid", "silu"):
+            want = ops.linear(ops.row_norm_gate(o, gate, nw, 1e-6, act), w)
+            assert _same(ops.linear_row_norm_gate(o, gate, nw, 1e-6, act, w, ops.stream_copy(w, R)), want), act
 
 
 def test_other_sizes_keep_their_kernels():
