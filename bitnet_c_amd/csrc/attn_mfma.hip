@@ -709,12 +709,12 @@ __device__ __forceinline__ void rotate8(uint4& lo, uint4& hi, const float* __res
     }
 }
 
-template <int HS>
-__global__ __launch_bounds__(256) void attn_mfma_decode_kernel(MfmaArgs a) {
+template <int HS, int NW>
+__global__ __launch_bounds__(64 * NW) void attn_mfma_decode_kernel(MfmaArgs a) {
     constexpr int DC = HS / 32, DT = HS / 16, HALF = HS / 2;
-    __shared__ float m_s[4][16], l_s[4][16];
-    __shared__ float o_s[4][HS][17];                    // [wave][dim][col], padded
+    __shared__ float m_s[NW][16], l_s[NW][16];
     __shared__ float cos_s[HALF], sin_s[HALF];
+    extern __shared__ float o_s[];                      // [wave][dim][GT + 1]: the heads' columns, padded
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, g = lane >> 4;
     const int G = a.H / a.Hkv, GT = a.GT;
@@ -770,7 +770,7 @@ __global__ __launch_bounds__(256) void attn_mfma_decode_kernel(MfmaArgs a) {
     // (With a window, or a table that ends before the block, the loads go to the table's first page and are dropped:
     // loads under a branch would make everything behind it wait for all of them.)
     const int kb_first = split * chunk + 32 * __builtin_amdgcn_readfirstlane(wave);
-    const bool ahead = a.window == 0 && kb_first / BN_PAGE < a.bt_stride;
+    const bool ahead = a.window == 0 && kb_first / BN_PAGE < a.bt_stride && 32 * wave < chunk;
     bf16x8 ka0[DC][2];
     bf16x8 va0[DT];
     const int page0 = uniform_load(a.block_table, (size_t)seq * a.bt_stride + (ahead ? kb_first / BN_PAGE : 0));
@@ -875,9 +875,9 @@ __global__ __launch_bounds__(256) void attn_mfma_decode_kernel(MfmaArgs a) {
                 attend_loaded_m<HS, 1, true>(ka0, va0, kb, q, acc, m, l, qpos, lo, k_hi, scale2, lane);
             else
                 attend_loaded_m<HS, 1, false>(ka0, va0, kb, q, acc, m, l, qpos, lo, k_hi, scale2, lane);
-            kb += 128;
+            kb += 32 * NW;
         }
-        for (; kb < k_hi; kb += 128) {
+        for (; kb < k_hi; kb += 32 * NW) {
             // the page index is the same for the whole wave: read through the scalar unit, so that it
             // does not queue behind the vector loads
             const int page = uniform_load(a.block_table, bt_row + __builtin_amdgcn_readfirstlane(kb / BN_PAGE));
@@ -888,24 +888,29 @@ __global__ __launch_bounds__(256) void attn_mfma_decode_kernel(MfmaArgs a) {
             attend_block<HS, 1>(kbase, vbase, kb, q, acc, m, l, qpos, lo, k_hi, need_mask, scale2, lane);
         }
     }
-    // merge the four waves: every wave's (m, l, O^T) through shared memory, in wave order
+    // merge the waves: every wave's (m, l, O^T) through shared memory, in wave order
     if (g == 0) { m_s[wave][n] = m[0]; l_s[wave][n] = l[0]; }
+    const int os = GT + 1;
+    if (n < GT) {
 #pragma unroll
-    for (int t = 0; t < DT; ++t)
+        for (int t = 0; t < DT; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o_s[wave][t * 16 + 4 * g + r][n] = acc[0][t][r];
+            for (int r = 0; r < 4; ++r) o_s[(wave * HS + t * 16 + 4 * g + r) * os + n] = acc[0][t][r];
+    }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < HS * GT; idx += 256) {
+    for (int idx = threadIdx.x; idx < HS * GT; idx += 64 * NW) {
         const int col = idx / HS, dim = idx - col * HS;      // consecutive threads: consecutive dims
         const int hg2 = ht * GT + col;
         if (hg2 >= G) continue;
-        float M = fmaxf(fmaxf(m_s[0][col], m_s[1][col]), fmaxf(m_s[2][col], m_s[3][col]));
+        float M = m_s[0][col];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) M = fmaxf(M, m_s[w][col]);
         float num = 0.f, den = 0.f;
         if (M != -INFINITY) {
 #pragma unroll
-            for (int w = 0; w < 4; ++w) {
+            for (int w = 0; w < NW; ++w) {
                 const float e = exp2f(m_s[w][col] - M);
-                num = fmaf(e, o_s[w][dim][col], num);
+                num = fmaf(e, o_s[(w * HS + dim) * os + col], num);
                 den = fmaf(e, l_s[w][col], den);
             }
         }
@@ -1040,9 +1045,24 @@ static int attn_mfma_launch(const void* q, int q_stride, void* out, int out_stri
     }
     if (n_tiles > 65535) return BN_ERR_ARG;                 // sequences are the grid's y
     const dim3 grid(Hkv * n_head_tiles, n_tiles, n_splits);
-    if (hs == 64) hipLaunchKernelGGL(attn_mfma_decode_kernel<64>, grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(attn_mfma_decode_kernel<128>, grid, dim3(256), 0, s, a);
-    int rc = bn_launch_status();
+    auto go = [&](auto kernel, int nw) {
+        const size_t smem = (size_t)nw * hs * (GT + 1) * sizeof(float);
+        if (smem > 48 * 1024) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
+            if (e != hipSuccess) return (int)e;
+        }
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * nw), smem, s, a);
+        return bn_launch_status();
+    };
+    // Sequences of five to nine pages whole, a workgroup a CU at the most: eight waves, which take a second block of 32 keys where
+    // four take a third to a fifth.  us, 8B heads, four waves / eight: one sequence of 250 keys 7.0 / 6.8, 380 8.6 / 8.0, 510 10.0 / 9.0,
+    // 16 of 250 8.3 / 8.7, 380 10.1 / 9.5, 570 13.6 / 12.1; shorter ones leave the waves without keys (16 of 125 6.8 / 8.1).  Cut
+    // and merged by a kernel of its own 510 keys take 9.4, 16 times 14.0; 700 are better cut (10.2 against 11.1).  A table that is
+    // wider says nothing of its sequences, and 16 waves spill their registers (14.6 at 600 keys).
+    const bool wide = n_splits == 1 && window == 0 && bt_stride > 4 && bt_stride <= BN_UNSPLIT_PAGES &&
+                      (long long)n_tiles * wgs_per_seq <= compute_units();
+    const int rc = wide ? (hs == 64 ? go(attn_mfma_decode_kernel<64, 8>, 8) : go(attn_mfma_decode_kernel<128, 8>, 8))
+                        : (hs == 64 ? go(attn_mfma_decode_kernel<64, 4>, 4) : go(attn_mfma_decode_kernel<128, 4>, 4));
     if (rc != 0 || n_splits == 1) return rc;
     hipLaunchKernelGGL(attn_mfma_combine_kernel, dim3(n_tokens * H), dim3(64), 0, s, (bf16*)out, out_stride, part_o,
                        part_ml, H, hs, n_splits);

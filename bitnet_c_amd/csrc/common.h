@@ -10,6 +10,8 @@
 // Decode attention splits a sequence's keys over workgroups in runs of at least this many pages: shorter
 // runs cost more in merging than they gain in parallelism (measured at batch 1, 8 and 64 of an 8B shape).
 #define BN_SPLIT_MIN_PAGES 2
+// Sequences of up to this many pages are not cut for the matrix-core decode kernel (attn_mfma.hip: measured on both sides).
+#define BN_UNSPLIT_PAGES 9
 // A float32 cache's keys are summed by attn_rows.hip (what attn_f32.hip, with runs of its own, does not take) in runs of this
 // many positions (whole pages, counted from position 0), each run by
 // itself and the runs folded in order: a decode step then spreads a long sequence's runs over workgroups and still forms

@@ -322,6 +322,29 @@ def test_decode_attention_applies_a_deferred_norm_s_factor(H, Hkv, hs, n_splits)
         ops.attention(raw.cuda(), out, k_pages, v_pages, bt.cuda(), H, Hkv, hs, hs ** -0.5, seq_lens=d_lens, row_scale=pre)
 
 
+# sequences that are not cut, by the width of the table: four and eight waves, tables at the edges of the choice; lengths: one key,
+# a block's and a page's edges, waves without keys
+@pytest.mark.parametrize("H,Hkv,hs", [(8, 2, 128), (6, 6, 64), (16, 1, 128)])
+@pytest.mark.parametrize("W", [1, 4, 5, 9, 10])
+def test_whole_sequences_of_decode_attention(H, Hkv, hs, W):
+    ops = _ops()
+    dtype = torch.bfloat16
+    lens = [l for l in (1, 32, 33, 64, 65, 129, 257, 64 * W - 31, 64 * W) if 0 < l <= 64 * W]
+    ks = [_rand((l, Hkv, hs), dtype, 10 + i) for i, l in enumerate(lens)]
+    vs = [_rand((l, Hkv, hs), dtype, 40 + i) for i, l in enumerate(lens)]
+    kp, vp, bt = _paged(ks, vs, dtype, sum((l + 63) // 64 for l in lens) + 2, 90)
+    assert bt.shape[1] == W
+    q = _rand((len(lens), H * hs), dtype, 91)
+    out = torch.full((len(lens), H * hs), float("nan"), dtype=dtype).cuda()
+    ops.attention(q.cuda(), out, kp.cuda(), vp.cuda(), bt.cuda(), H, Hkv, hs, hs ** -0.5, seq_lens=torch.tensor(lens, dtype=torch.int32).cuda())
+    for b, (k, v) in enumerate(zip(ks, vs)):
+        k, v = (t.float().repeat_interleave(H // Hkv, dim=1).transpose(0, 1).contiguous() for t in (k, v))
+        s = torch.matmul(k, q[b].float().view(H, hs, 1)).squeeze(-1) * hs ** -0.5
+        want = torch.matmul(torch.softmax(s, dim=-1).unsqueeze(1), v).reshape(-1)
+        # a weight's and the result's rounding to bf16 (2^-9 each, the weights' sum in float32)
+        assert float((out[b].float().cpu() - want).norm()) <= 2.0 ** -7 * float(want.norm()) + 1e-6, (b, lens[b])
+
+
 def test_partial_sums_refuse_what_they_cannot_take():
     ops = _ops()
     assert ops.can_split_sums(64, 64, 128, torch.bfloat16) and ops.can_split_sums(128, 64, 512, torch.bfloat16)
