@@ -261,6 +261,9 @@ struct WkvArgs {
     int n_tiles;              // (the piece forms)
     float* carry;             // [pieces, H dkp dv]: a piece's own sum, then what the piece starts from
     float* fade;              // [pieces, H dkp]: the product of a piece's decays
+    const bf16* low;          // (the step in bf16) [T, ldlow], w2 [H * dk, rank]: d is low . w2^T, formed here (d null)
+    const bf16* w2;
+    int ldlow, rank;
 };
 
 // How a workgroup of the recurrence meets its sequence: the whole of it (WKV_WALK), or, where a step offers too few sequences
@@ -596,11 +599,14 @@ extern "C" int bn_head_norm_gate(int dtype, void* y, const float* o, const void*
 // that kernel: a position's output does not depend on the step it came in), and weight and gate follow.  Bound by latency at
 // few sequences (a trip to memory for the state, two barriers): one sequence of 32 heads of 64 4.8 us in a graph of such
 // launches, 6.9 in a decode step's profile, where the walk and the norm's kernel took 7.8 + 5.0.
-template <typename T>
+// NJ > 0: the decay's last product (low . w2^T, up to 32 NJ columns) is formed here as well, 16 channels a wave on the matrix cores
+// in the order of skinny_gemm's kernel (the same bits), instead of in a launch of its own that reads 8 KB a head (3.8 us; this
+// kernel 5.0 -> 5.8 with one sequence of 32 heads of 64).
+template <typename T, int NJ>
 __global__ __launch_bounds__(1024) void wkv_step_kernel(WkvArgs a, T* __restrict__ y, const T* __restrict__ gate, int ldg,
                                                         const float* __restrict__ weight, float eps) {
     __shared__ __align__(16) float r_s[WKV_MAX_DIM], k_s[WKV_MAX_DIM], w_s[WKV_MAX_DIM];
-    __shared__ float o_s[WKV_MAX_DIM];
+    __shared__ float o_s[WKV_MAX_DIM], d_s[WKV_MAX_DIM];
     const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
     const int pos = a.seq_lens[seq] - 1;
     if (pos < 0) return;
@@ -614,13 +620,35 @@ __global__ __launch_bounds__(1024) void wkv_step_kernel(WkvArgs a, T* __restrict
         S[ii] = S_g[((size_t)ii * dv + jc) * P + p];
         ub[ii] = a.u[(size_t)head * dk + min(p * WKV_KR + ii, dk - 1)];
     }
+    if constexpr (NJ > 0) {
+        typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+        typedef __attribute__((ext_vector_type(4))) float f32x4;
+        const int lane = tid & (BN_WAVE - 1), n_waves = blockDim.x / BN_WAVE, i = lane & 15, g = lane >> 4;
+        for (int tile = __builtin_amdgcn_readfirstlane(tid / BN_WAVE); 16 * tile < dk; tile += n_waves) {
+            const bf16* wr = a.w2 + ((size_t)head * dk + 16 * tile + i) * a.rank + 8 * g;
+            const bf16* xr = a.low + (size_t)seq * a.ldlow + 8 * g;
+            bf16x8 x[NJ], w[NJ];
+#pragma unroll
+            for (int q = 0; q < NJ; ++q) {                // past the last 32 columns: those again, not multiplied
+                const int c = min(32 * q, a.rank - 32);
+                x[q] = *reinterpret_cast<const bf16x8*>(xr + c);
+                w[q] = *reinterpret_cast<const bf16x8*>(wr + c);
+            }
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < NJ; ++q)
+                if (32 * q < a.rank) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[q], w[q], acc, 0, 0, 0);
+            if (g == 0) d_s[16 * tile + i] = to_f32(from_f32<bf16>(acc[0]));
+        }
+        lds_barrier();
+    }
     const float vj = to_f32(reinterpret_cast<const T*>(a.v)[(size_t)seq * a.ldv + (size_t)head * dv + jc]);
     const float gj = to_f32(gate[(size_t)seq * ldg + (size_t)head * dv + jc]), wj = weight ? weight[(size_t)head * dv + jc] : 1.0f;
     for (int i = tid; i < dkp; i += blockDim.x) {
         const size_t c = (size_t)head * dk + min(i, dk - 1);
         const float r = to_f32(reinterpret_cast<const T*>(a.r)[(size_t)seq * a.ldr + c]);
         const float k = to_f32(reinterpret_cast<const T*>(a.k)[(size_t)seq * a.ldk + c]);
-        const float d = to_f32(reinterpret_cast<const T*>(a.d)[(size_t)seq * a.ldd + c]) + a.w0[c];
+        const float d = (NJ > 0 ? d_s[min(i, dk - 1)] : to_f32(reinterpret_cast<const T*>(a.d)[(size_t)seq * a.ldd + c])) + a.w0[c];
         r_s[i] = i < dk ? r : 0.f;
         k_s[i] = i < dk ? k : 0.f;
         w_s[i] = i < dk ? expf(-expf(d)) : 0.f;
@@ -662,28 +690,39 @@ extern "C" int bn_wkv_step_supports(int dk, int dv) {
     return wkv_shape(dk, dv, 1, P, CB, TC, wk, th) && P * dv <= 1024 ? 1 : 0;
 }
 
+// 1 if the step forms d itself from low [n, rank] and w2 [H dk, rank] (bf16, rows of 16-byte groups at 16-byte addresses)
+extern "C" int bn_wkv_step_takes_low(int dk, int dv, int rank) {
+    return bn_wkv_step_supports(dk, dv) && dk % 16 == 0 && rank >= 32 && rank <= 256 && rank % 32 == 0;
+}
+
+// d null: low [n_seqs, rank] (row stride ldlow) and w2 [H dk, rank] (contiguous) in its place, bf16
 extern "C" int bn_wkv_step(int dtype, const void* r, int ldr, const void* k, int ldk, const void* v, int ldv, const void* d, int ldd,
-                           const float* w0, const float* u, const void* h, float* state, long long state_stride,
+                           const void* low, int ldlow, const void* w2, int rank, const float* w0, const float* u, const void* h, float* state, long long state_stride,
                            const int* seq_lens, const int* slot_ids, int n_seqs, int H, int dk, int dv, int D, void* y,
                            const void* gate, int ldg, const float* weight, float eps, hipStream_t s) {
     WkvArgs a = {};
     int threads;
     if (n_seqs <= 0 || H <= 0 || D <= 0 || !bn_wkv_step_supports(dk, dv) || !wkv_shape(dk, dv, 1, a.P, a.CB, a.TC, a.walkers, threads))
         return BN_ERR_ARG;
-    if (!r || !k || !v || !d || !w0 || !u || !h || !state || !slot_ids || !seq_lens || !y || !gate || ldg < H * dv) return BN_ERR_ARG;
+    if (!r || !k || !v || !d != (low && w2) || !w0 || !u || !h || !state || !slot_ids || !seq_lens || !y || !gate || ldg < H * dv) return BN_ERR_ARG;
+    if (!d && (dtype != BN_DT_BF16 || !bn_wkv_step_takes_low(dk, dv, rank) || ldlow < rank || ldlow % 8 || (((uintptr_t)low | (uintptr_t)w2) & 15)))
+        return BN_ERR_ARG;
     if (state_stride < (long long)H * a.P * WKV_KR * dv + D) return BN_ERR_ARG;
     a.r = r; a.k = k; a.v = v; a.d = d; a.ldr = ldr; a.ldk = ldk; a.ldv = ldv; a.ldd = ldd;
     a.w0 = w0; a.u = u; a.h = h; a.state = state; a.state_stride = (size_t)state_stride;
     a.seq_lens = seq_lens; a.slot_ids = slot_ids;
     a.H = H; a.dk = dk; a.dv = dv; a.D = D;
+    a.low = (const bf16*)low; a.w2 = (const bf16*)w2; a.ldlow = ldlow; a.rank = rank;
     const dim3 grid(n_seqs, H), block((a.P * dv + BN_WAVE - 1) / BN_WAVE * BN_WAVE);
-    if (dtype == BN_DT_F32)
-        hipLaunchKernelGGL(wkv_step_kernel<float>, grid, block, 0, s, a, (float*)y, (const float*)gate, ldg, weight, eps);
-    else if (dtype == BN_DT_BF16)
-        hipLaunchKernelGGL(wkv_step_kernel<bf16>, grid, block, 0, s, a, (bf16*)y, (const bf16*)gate, ldg, weight, eps);
-    else
-        return BN_ERR_DTYPE;
-    return bn_launch_status();
+    auto go = [&](auto kernel, auto* out) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, a, out, (decltype(out))gate, ldg, weight, eps);
+        return bn_launch_status();
+    };
+    if (dtype == BN_DT_F32) return go(wkv_step_kernel<float, 0>, (float*)y);
+    if (dtype != BN_DT_BF16) return BN_ERR_DTYPE;
+    if (d) return go(wkv_step_kernel<bf16, 0>, (bf16*)y);
+    if (rank <= 64) return go(wkv_step_kernel<bf16, 2>, (bf16*)y);
+    return rank <= 128 ? go(wkv_step_kernel<bf16, 4>, (bf16*)y) : go(wkv_step_kernel<bf16, 8>, (bf16*)y);
 }
 
 // ---- min-GRU ------------------------------------------------------------------------------------------------------

@@ -137,7 +137,8 @@ _SIGNATURES = {
                         c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int,
                         c_int, c_int, c_void_p, c_void_p, c_void_p],
         "bn_wkv_step_supports": [c_int, c_int],
-        "bn_wkv_step": [c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
+        "bn_wkv_step_takes_low": [c_int, c_int, c_int],
+        "bn_wkv_step": [c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                         c_void_p, c_longlong, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int,
                         c_void_p, c_float, c_void_p],
         "bn_head_norm_gate": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_float, c_void_p],
@@ -2295,7 +2296,7 @@ def _wkv_args(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, w
     T, D = h.shape
     if not wkv_supported(dk, dv):
         raise KernelError(f"{what}: head sizes up to {WKV_MAX_DIM}, got {dk} x {dv}")
-    for t, nm, n in ((r, "r", H * dk), (k, "k", H * dk), (v, "v", H * dv), (d, "d", H * dk)):
+    for t, nm, n in ((r, "r", H * dk), (k, "k", H * dk), (v, "v", H * dv)) + (((d, "d", H * dk),) if d is not None else ()):
         _dev(t, nm, h.dtype, 2)
         if t.shape != (T, n):
             raise KernelError(f"{what}: {nm} must be [{T}, {n}], got {tuple(t.shape)}")
@@ -2313,13 +2314,23 @@ def wkv_step_supported(dk: int, dv: int) -> bool:
     return bool(_fn("state_mixers", "bn_wkv_step_supports")(int(dk), int(dv)))
 
 
+def wkv_step_takes_low(low: torch.Tensor, w2: torch.Tensor, dk: int, dv: int) -> bool:
+    """Whether wkv_step forms linear(low, w2) itself (bf16, rows of whole 16-byte groups, up to 256 columns in groups of 32)."""
+    return (FUSE_NORMS and low.dtype == w2.dtype == torch.bfloat16 and low.dim() == 2 and low.stride(1) == 1 and w2.is_contiguous()
+            and _rows(low, "low") % 8 == 0 and (low.data_ptr() | w2.data_ptr()) % 16 == 0
+            and bool(_fn("state_mixers", "bn_wkv_step_takes_low")(int(dk), int(dv), w2.shape[1])))
+
+
 def wkv_step(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, seq_lens, gate: torch.Tensor,
-             weight: Optional[torch.Tensor], eps: float) -> torch.Tensor:
-    """head_norm_gate(wkv_scan(...)) of a decode step in one kernel: [T, H dv] in h's type."""
+             weight: Optional[torch.Tensor], eps: float, low: Optional[torch.Tensor] = None, w2: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """head_norm_gate(wkv_scan(...)) of a decode step in one kernel: [T, H dv] in h's type.  d None: linear(low, w2) in its place
+    (wkv_step_takes_low), formed in the same kernel."""
     require_gpu()
     T, D, stride = _wkv_args(r, k, v, d, w0, u, h, state, slot_ids, H, dk, dv, "wkv_step")
     _, n_seqs, sl = _seq_args(None, seq_lens, "wkv_step")
     _dev(gate, "gate", h.dtype, 2)
+    if d is None and (tuple(w2.shape) != (H * dk, low.shape[1]) or low.shape[0] != T or not wkv_step_takes_low(low, w2, dk, dv)):
+        raise KernelError(f"wkv_step: low {tuple(low.shape)}, w2 {tuple(w2.shape)}")
     if not wkv_step_supported(dk, dv) or n_seqs != T or tuple(gate.shape) != (T, H * dv):
         raise KernelError(f"wkv_step: {n_seqs} sequences, h {tuple(h.shape)}, gate {tuple(gate.shape)}, heads of {dk} x {dv}")
     if weight is not None:
@@ -2329,9 +2340,11 @@ def wkv_step(r, k, v, d, w0, u, h, state, slot_ids, H: int, dk: int, dv: int, se
     y = torch.empty((T, H * dv), dtype=h.dtype, device=h.device)
     if T:
         _check(_fn("state_mixers", "bn_wkv_step")(
-            _code(h.dtype), r.data_ptr(), _rows(r, "r"), k.data_ptr(), _rows(k, "k"), v.data_ptr(), _rows(v, "v"), d.data_ptr(),
-            _rows(d, "d"), w0.data_ptr(), u.data_ptr(), h.data_ptr(), state.data_ptr(), stride, sl, slot_ids.data_ptr(), T, H, dk, dv,
-            D, y.data_ptr(), gate.data_ptr(), _rows(gate, "gate"), weight.data_ptr() if weight is not None else None, float(eps),
+            _code(h.dtype), r.data_ptr(), _rows(r, "r"), k.data_ptr(), _rows(k, "k"), v.data_ptr(), _rows(v, "v"),
+            d.data_ptr() if d is not None else None, _rows(d, "d") if d is not None else 0,
+            low.data_ptr() if d is None else None, _rows(low, "low") if d is None else 0, w2.data_ptr() if d is None else None,
+            w2.shape[1] if d is None else 0, w0.data_ptr(), u.data_ptr(), h.data_ptr(), state.data_ptr(), stride, sl, slot_ids.data_ptr(),
+            T, H, dk, dv, D, y.data_ptr(), gate.data_ptr(), _rows(gate, "gate"), weight.data_ptr() if weight is not None else None, float(eps),
             _stream()), "wkv_step")
     return y
 

@@ -112,9 +112,13 @@ class WKV(Part):
             mixes = ops.token_shift(h, self.mu, last, ctx.positions, ctx.seq_index, ctx.slot_ids)
             r, k, v, g, low = ops.linear_group([(x, l.weight, l.streamed, "tanh" if l is self.w1 else None)
                                                 for x, l in zip(mixes, self._first())])
-        d = self.w2(low)
-        if ctx.is_decode and ops.wkv_step_supported(hs, hs):
-            y = ops.wkv_step(r, k, v, d, self.w0, self.u, h, state, ctx.slot_ids, H, hs, hs, ctx.seq_lens, g, self.norm, self.eps)
+        step = ctx.is_decode and ops.wkv_step_supported(hs, hs)
+        # (more rows than the streaming product takes: its bits are the library's product's)
+        inside = step and low.shape[0] <= ops.SKINNY_ROWS and ops.wkv_step_takes_low(low, self.w2.weight, hs, hs)
+        d = None if inside else self.w2(low)
+        if step:
+            y = ops.wkv_step(r, k, v, d, self.w0, self.u, h, state, ctx.slot_ids, H, hs, hs, ctx.seq_lens, g, self.norm, self.eps,
+                             *((low, self.w2.weight) if inside else ()))
         else:
             o = ops.wkv_scan(r, k, v, d, self.w0, self.u, h, state, ctx.slot_ids, H, hs, hs,
                              pieces=ops.wkv_in_pieces(h.dtype, ctx.sizes, H, hs, hs), **_sequences(ctx))

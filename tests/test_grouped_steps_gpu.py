@@ -197,3 +197,27 @@ def test_row_kernels_where_the_wide_ones_begin(dtype, dim):
     test_add_normed_rmsnorm_widths(dtype, dim, 0, "norm")
     test_add_normed_rmsnorm_widths(dtype, dim, 3, "rows")
     test_row_norm_gate_widths(dtype, dim)
+
+
+# the decay's last product inside the step: the same bits as the streaming product's in front of it.  head sizes: one tile of
+# channels, two tiles for four waves, more tiles than waves; ranks: one block of 32, as many as a form holds and one fewer
+@pytest.mark.parametrize("B", [1, 3, 16])
+@pytest.mark.parametrize("H,d,rank", [(2, 16, 32), (3, 32, 64), (4, 64, 64), (2, 64, 96), (1, 96, 128), (2, 128, 224), (1, 64, 256)])
+def test_wkv_step_with_the_decay_s_product(B, H, d, rank):
+    from bitnet_c_amd import ops
+    g = torch.Generator().manual_seed(B + H + d + rank)
+    D = 64
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=g).bfloat16().cuda()
+    r, k, v, gate, h = rand(B, H * d), rand(B, H * d), rand(B, H * d), rand(B, H * d), rand(B, D)
+    low, w2 = rand(B, rank + 8)[:, 8:], rand(H * d, rank) * 0.1
+    w0, u = torch.rand(H * d, generator=g).cuda() - 3.0, torch.rand(H * d, generator=g).cuda()
+    state = torch.randn(B + 2, ops.wkv_state_floats(H, d, d) + D, generator=g).cuda()
+    slots, lens = torch.arange(B, 0, -1, dtype=torch.int32).cuda(), torch.tensor([5 - 5 * (i == 1) for i in range(B)], dtype=torch.int32).cuda()
+    assert ops.wkv_step_takes_low(low, w2, d, d) and not ops.wkv_step_takes_low(low[:, :rank - 8], w2[:, :rank - 8].contiguous(), d, d)
+    a, b = state.clone(), state.clone()
+    want = ops.wkv_step(r, k, v, ops.linear(low, w2), w0, u, h, a, slots, H, d, d, lens, gate, None, 1e-6)
+    got = ops.wkv_step(r, k, v, None, w0, u, h, b, slots, H, d, d, lens, gate, None, 1e-6, low, w2)
+    live = lens > 0
+    assert torch.equal(got[live], want[live]) and torch.equal(a, b)
