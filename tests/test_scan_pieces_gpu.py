@@ -93,3 +93,23 @@ def test_token_shift_wide(dtype, T, D):
 @pytest.mark.parametrize("T,D", [(5, 504), (5, 512), (1, 520), (731, 4096), (733, 4096), (367, 4096), (5901, 512)])
 def test_token_shift_forms(dtype, T, D):
     test_token_shift_wide(dtype, T, D)
+
+
+# one token of every sequence: the same bits as the walk of a step that holds that token alone; channels under, at and over a
+# workgroup's 64, sequences at their first token and a padding row
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("W,bias", [(1, True), (64, False), (65, True), (2048, True)])
+def test_mingru_decode_step(dtype, W, bias):
+    from bitnet_c_amd import ops
+    g = torch.Generator().manual_seed(W)
+    B = 5
+    zxg = torch.randn(B, 3 * W + 8, generator=g).to(dtype).cuda()[:, :3 * W]
+    bz, bx = (torch.randn(W, generator=g).cuda() if bias else None for _ in range(2))
+    state = torch.randn(B + 1, W + 4, generator=g).cuda()
+    slots, lens = torch.tensor([3, 0, 5, 1, 4], dtype=torch.int32).cuda(), torch.tensor([1, 9, 0, 2, 70], dtype=torch.int32).cuda()
+    a, b = state.clone(), state.clone()
+    got = ops.mingru_scan(zxg, bz, bx, a, slots, W, seq_lens=lens)
+    tiles = torch.tensor([[i, i, 1, int(lens[i]) - 1] for i in (0, 1, 3, 4)], dtype=torch.int32).cuda()
+    want = ops.mingru_scan(zxg, bz, bx, b, slots, W, tiles=tiles)
+    live = [0, 1, 3, 4]
+    assert torch.equal(got[live], want[live]) and torch.equal(a, b)
