@@ -177,6 +177,65 @@ __global__ __launch_bounds__(LA_THREADS) void lightning_scan_kernel(LaArgs a) {
     }
 }
 
+// The walk's decode step without a rotation: one token of every sequence, its projections and the state asked for together (the walk
+// asks for the projections under a branch, behind the state, and waits for both there), barriers that leave the stores in flight.
+// The same operations in the same order: the same bits.  us in a decode step, four sequences of 16 heads of 128 x 128, 6.7 -> 5.8.
+template <typename T, int RPT>
+__global__ __launch_bounds__(LA_THREADS) void lightning_step_kernel(LaArgs a) {
+    constexpr int DKP = RPT * LA_RG;
+    static_assert(DKP <= LA_THREADS, "a key row a thread");
+    __shared__ __align__(16) float q_s[DKP], k_s[DKP];
+    __shared__ float v_s[LA_CB], p_s[LA_RG * LA_CB];
+    const int seq = blockIdx.x, pos = a.seq_lens[seq] - 1;
+    if (pos < 0) return;
+    const int tid = threadIdx.x, col = tid % LA_CB, rg = tid / LA_CB;
+    const int head = blockIdx.y, c0 = blockIdx.z * LA_CB, c = c0 + col, r0 = rg * RPT;
+    const bool has = c < a.dv;
+    const int cc = min(c, a.dv - 1);                     // loads in straight line: without a column or a row, a neighbour's
+    const T* row = reinterpret_cast<const T*>(a.x) + (size_t)seq * a.ld;
+    const float qr = to_f32(row[a.q_col + (size_t)head * a.dk + min(tid, a.dk - 1)]);
+    const float kr = to_f32(row[a.k_col + (size_t)head * a.dk + min(tid, a.dk - 1)]);
+    const float vr = to_f32(row[a.v_col + (size_t)head * a.dv + cc]);
+    const float decay = a.decay[head];
+    float* sp = a.state + (size_t)a.slot_ids[seq] * a.state_stride + (size_t)head * a.dk * a.dv + cc;
+    float S[RPT];
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) S[i] = sp[(size_t)min(r0 + i, a.dk - 1) * a.dv];
+    if (tid < DKP) {
+        q_s[tid] = tid < a.dk ? la_act(qr, a.feed.silu) : 0.f;
+        k_s[tid] = tid < a.dk ? la_act(kr, a.feed.silu) * a.feed.k_scale : 0.f;
+    }
+    if (tid < LA_CB) v_s[tid] = has ? la_act(vr, a.feed.silu) : 0.f;
+    bn_lds_barrier();
+#pragma unroll
+    for (int i = 0; i < RPT; ++i)
+        if (!has || r0 + i >= a.dk || pos == 0) S[i] = 0.f;
+    const float vt = v_s[col];
+    const float4* k4 = reinterpret_cast<const float4*>(k_s + r0);
+    const float4* q4 = reinterpret_cast<const float4*>(q_s + r0);
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < RPT / 4; ++i) {
+        const float4 kk = k4[i], qq = q4[i];
+        const float kv[4] = {kk.x, kk.y, kk.z, kk.w}, qv[4] = {qq.x, qq.y, qq.z, qq.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            S[4 * i + e] = fmaf(decay, S[4 * i + e], kv[e] * vt);
+            acc[e] = fmaf(S[4 * i + e], qv[e], acc[e]);
+        }
+    }
+    p_s[rg * LA_CB + col] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    if (has) {
+#pragma unroll
+        for (int i = 0; i < RPT; ++i)
+            if (r0 + i < a.dk) sp[(size_t)(r0 + i) * a.dv] = S[i];
+    }
+    bn_lds_barrier();
+    if (tid < LA_CB && has)
+        a.o[(size_t)seq * a.H * a.dv + (size_t)head * a.dv + c] =
+            (p_s[tid] + p_s[LA_CB + tid]) + (p_s[2 * LA_CB + tid] + p_s[3 * LA_CB + tid]);
+}
+
 // ---- the chunked form -------------------------------------------------------------------------------------------------
 #define LC_C 64               // tokens of a chunk
 #define LC_MAX_DIM 128        // largest key width of the chunked form
@@ -522,6 +581,17 @@ extern "C" int bn_lightning_scan(int dtype, const void* x, int ld, int q_col, in
     const int rpt = dk <= 32 ? 8 : dk <= 64 ? 16 : dk <= 128 ? 32 : 64;
     const size_t smem = (size_t)LA_TC * (2 * rpt * LA_RG + LA_CB + LA_RG * LA_CB) * sizeof(float);
     const dim3 grid(n_seqs, H, (dv + LA_CB - 1) / LA_CB), block(LA_THREADS);
+    if (!tiles && a.feed.rope_dims == 0) {
+#define LA_STEP(RPT_)                                                                                                 \
+    if (dtype == BN_DT_F32) hipLaunchKernelGGL((lightning_step_kernel<float, RPT_>), grid, block, 0, s, a);           \
+    else hipLaunchKernelGGL((lightning_step_kernel<bf16, RPT_>), grid, block, 0, s, a)
+        if (rpt == 8) { LA_STEP(8); }
+        else if (rpt == 16) { LA_STEP(16); }
+        else if (rpt == 32) { LA_STEP(32); }
+        else { LA_STEP(64); }
+#undef LA_STEP
+        return bn_launch_status();
+    }
 #define LA_GO(RPT_)                                                                                         \
     if (dtype == BN_DT_F32) hipLaunchKernelGGL((lightning_scan_kernel<float, RPT_>), grid, block, smem, s, a); \
     else hipLaunchKernelGGL((lightning_scan_kernel<bf16, RPT_>), grid, block, smem, s, a)

@@ -39,3 +39,25 @@ def test_which_launches_take_32_columns():
     assert columns(2, 16, 128, 128) == 16 and columns(5, 40, 72, 24) == 32 and columns(2, 65, 128, 48) == 16
     assert all(columns(n, h, 128, dv) == 16 for n in (1, 8, 31) for h in (16, 64) for dv in (1, 16))
     assert columns(31, 64, 64, 128) == 16
+
+
+# one token of every sequence: the same bits as the walk of a step that holds that token alone.  key widths: one row, the edges of
+# the forms' rows; value columns under, at and over a workgroup's 64; sequences at their first token and a padding row
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dk,dv", [(1, 64), (32, 33), (33, 128), (64, 65), (100, 70), (128, 128), (129, 64), (256, 100)])
+@pytest.mark.parametrize("silu", [True, False])
+def test_decode_step_gives_the_bits_of_the_walk(dtype, dk, dv, silu):
+    from bitnet_c_amd import ops
+    H, B = 3, 5
+    g = torch.Generator().manual_seed(dk + dv)
+    x = torch.randn(B, H * (2 * dk + dv) + 3, generator=g).to(dtype).cuda()
+    decay = torch.rand(H, generator=g).cuda()
+    state = torch.randn(B + 1, H * dk * dv, generator=g).cuda()
+    slots, lens = torch.tensor([3, 0, 5, 1, 4], dtype=torch.int32).cuda(), torch.tensor([1, 9, 0, 2, 70], dtype=torch.int32).cuda()
+    tiles = torch.tensor([[i, i, 1, int(lens[i]) - 1] for i in (0, 1, 3, 4)], dtype=torch.int32).cuda()
+    kw = dict(silu=silu, k_scale=1.0 if silu else 0.25)
+    a, b = state.clone(), state.clone()
+    got = ops.lightning_scan(x, 0, H * dk, 2 * H * dk, decay, a, slots, H, dk, dv, seq_lens=lens, **kw)
+    want = ops.lightning_scan(x, 0, H * dk, 2 * H * dk, decay, b, slots, H, dk, dv, tiles=tiles, chain=True, **kw)
+    live = [0, 1, 3, 4]
+    assert torch.equal(got[live], want[live]) and torch.equal(a, b)
