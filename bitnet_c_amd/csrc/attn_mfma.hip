@@ -709,13 +709,24 @@ __device__ __forceinline__ void rotate8(uint4& lo, uint4& hi, const float* __res
     }
 }
 
-template <int HS, int NW>
-__global__ __launch_bounds__(64 * NW) void attn_mfma_decode_kernel(MfmaArgs a) {
+// a - b with its own rounding, whatever a was formed by
+__device__ __forceinline__ float minus_rounded(float a, float b) {
+#pragma clang fp contract(off)
+    return a - b;
+}
+
+#define AD_WHOLE_PAGES 16             // widest block table of the WHOLE form (attn_mfma_launch)
+
+// WHOLE: a workgroup of eight waves takes both splits of a launch of two for its sequence and kv head, four waves a split, and
+// merges them itself, as attn_mfma_combine_kernel would: the same sums in the same order, so that no bit depends on the form.
+template <int HS, bool WHOLE>
+__global__ __launch_bounds__(WHOLE ? 512 : 256) void attn_mfma_decode_kernel(MfmaArgs a) {
     constexpr int DC = HS / 32, DT = HS / 16, HALF = HS / 2;
-    __shared__ float m_s[NW][16], l_s[NW][16];
+    constexpr int SPLITS = WHOLE ? 2 : 1, THREADS = 256 * SPLITS;
+    __shared__ float m_s[4 * SPLITS][16], l_s[4 * SPLITS][16];
     __shared__ float cos_s[HALF], sin_s[HALF];
-    extern __shared__ float o_s[];                      // [wave][dim][GT + 1]: the heads' columns, padded
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    extern __shared__ float o_s[];                      // [split, wave of it][dim][GT + 1]: the heads' columns, padded
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
     const int n = lane & 15, g = lane >> 4;
     const int G = a.H / a.Hkv, GT = a.GT;
     const int n_head_tiles = (G + GT - 1) / GT;
@@ -724,7 +735,7 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_decode_kernel(MfmaArgs a) {
     // batch that is a multiple of 8, a sequence's heads all landed on one XCD)
     const int kvh = blockIdx.x / n_head_tiles, ht = blockIdx.x - kvh * n_head_tiles;
     int seq = blockIdx.y;
-    const int split = blockIdx.z;
+    const int split = WHOLE ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : blockIdx.z;      // of these waves
     if (a.by_length) {
         int r = seq;
         if (a.order_period > 0) {
@@ -770,7 +781,7 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_decode_kernel(MfmaArgs a) {
     // (With a window, or a table that ends before the block, the loads go to the table's first page and are dropped:
     // loads under a branch would make everything behind it wait for all of them.)
     const int kb_first = split * chunk + 32 * __builtin_amdgcn_readfirstlane(wave);
-    const bool ahead = a.window == 0 && kb_first / BN_PAGE < a.bt_stride && 32 * wave < chunk;
+    const bool ahead = a.window == 0 && kb_first / BN_PAGE < a.bt_stride;
     bf16x8 ka0[DC][2];
     bf16x8 va0[DT];
     const int page0 = uniform_load(a.block_table, (size_t)seq * a.bt_stride + (ahead ? kb_first / BN_PAGE : 0));
@@ -781,7 +792,7 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_decode_kernel(MfmaArgs a) {
     const bool ok = q_lane && L > 0;
     const int lo_key = a.window > 0 ? max(0, L - a.window) : 0;
     const int k_lo = max(lo_key, split * chunk), k_hi = min(L, (split + 1) * chunk);       // [k_lo, k_hi)
-    if (a.n_splits > 1 && k_lo >= k_hi) {
+    if (!WHOLE && a.n_splits > 1 && k_lo >= k_hi) {
         // A split without keys (a sequence shorter than the launch's longest, a padding row): it leaves "nothing seen"
         // for the merge, which then does not read its sums, and is gone before it asks for anything else.
         if (threadIdx.x < GT && ht * GT + threadIdx.x < G) {
@@ -810,7 +821,7 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_decode_kernel(MfmaArgs a) {
     }
     // the new token's key and value go into the cache before anyone reads them: the workgroup
     // that owns the new position does it (there is one per kv head: write_kv needs n_head_tiles == 1)
-    if (a.write_kv && L > 0 && L - 1 >= k_lo && L - 1 < k_hi) {
+    if (a.write_kv && L > 0 && (WHOLE || (L - 1 >= k_lo && L - 1 < k_hi))) {
         const int pos = L - 1;
         // through the scalar unit (the length is the same in every lane), so that it does not queue behind the block
         // that is on its way
@@ -856,13 +867,14 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_decode_kernel(MfmaArgs a) {
     int qpos[1] = {ok ? L - 1 : -1};
     int lo[1] = {lo_key};
 
+    const float scale2 = a.scale * LOG2E;
+    const size_t bt_row = (size_t)seq * a.bt_stride;
+    const int os = GT + 1;
     f32x4 acc[1][DT];
     float m[1] = {-INFINITY}, l[1] = {0.f};
 #pragma unroll
     for (int t = 0; t < DT; ++t) acc[0][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    const float scale2 = a.scale * LOG2E;
     if (k_lo < k_hi) {
-        const size_t bt_row = (size_t)seq * a.bt_stride;
         // (Keeping the next block's operands in a second set of registers while the current block is multiplied was
         // measured and gained nothing: the CU's other waves already cover a wave's wait for its loads.)
         // The waves take the blocks of 32 keys in turn, so that neighbouring waves ask for the two halves of a page at
@@ -875,9 +887,9 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_decode_kernel(MfmaArgs a) {
                 attend_loaded_m<HS, 1, true>(ka0, va0, kb, q, acc, m, l, qpos, lo, k_hi, scale2, lane);
             else
                 attend_loaded_m<HS, 1, false>(ka0, va0, kb, q, acc, m, l, qpos, lo, k_hi, scale2, lane);
-            kb += 32 * NW;
+            kb += 128;
         }
-        for (; kb < k_hi; kb += 32 * NW) {
+        for (; kb < k_hi; kb += 128) {
             // the page index is the same for the whole wave: read through the scalar unit, so that it
             // does not queue behind the vector loads
             const int page = uniform_load(a.block_table, bt_row + __builtin_amdgcn_readfirstlane(kb / BN_PAGE));
@@ -888,39 +900,69 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_decode_kernel(MfmaArgs a) {
             attend_block<HS, 1>(kbase, vbase, kb, q, acc, m, l, qpos, lo, k_hi, need_mask, scale2, lane);
         }
     }
-    // merge the waves: every wave's (m, l, O^T) through shared memory, in wave order
-    if (g == 0) { m_s[wave][n] = m[0]; l_s[wave][n] = l[0]; }
-    const int os = GT + 1;
+    // every wave's (m, l, O^T) into shared memory
+    const int at = (WHOLE ? 4 * split : 0) + wave;
+    if (g == 0) { m_s[at][n] = m[0]; l_s[at][n] = l[0]; }
     if (n < GT) {
 #pragma unroll
         for (int t = 0; t < DT; ++t)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o_s[(wave * HS + t * 16 + 4 * g + r) * os + n] = acc[0][t][r];
+            for (int r = 0; r < 4; ++r) o_s[(at * HS + t * 16 + 4 * g + r) * os + n] = acc[0][t][r];
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < HS * GT; idx += 64 * NW) {
+    for (int idx = threadIdx.x; idx < HS * GT; idx += THREADS) {
         const int col = idx / HS, dim = idx - col * HS;      // consecutive threads: consecutive dims
         const int hg2 = ht * GT + col;
         if (hg2 >= G) continue;
-        float M = m_s[0][col];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) M = fmaxf(M, m_s[w][col]);
-        float num = 0.f, den = 0.f;
-        if (M != -INFINITY) {
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                const float e = exp2f(m_s[w][col] - M);
-                num = fmaf(e, o_s[(w * HS + dim) * os + col], num);
-                den = fmaf(e, l_s[w][col], den);
-            }
-        }
         const int hd = kvh * G + hg2;
-        if (a.n_splits == 1) {
-            a.out[(size_t)seq * a.out_stride + (size_t)hd * HS + dim] = __float2bfloat16(den > 0.f ? num / den : 0.f);
+        // a split's four waves, in wave order
+        auto merge = [&](int u, float& M, float& num, float& den) {
+            const int at = 4 * u;
+            M = fmaxf(fmaxf(m_s[at][col], m_s[at + 1][col]), fmaxf(m_s[at + 2][col], m_s[at + 3][col]));
+            num = den = 0.f;
+            if (M != -INFINITY) {
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const float e = exp2f(m_s[at + w][col] - M);
+                    num = fmaf(e, o_s[((at + w) * HS + dim) * os + col], num);
+                    den = fmaf(e, l_s[at + w][col], den);
+                }
+            }
+        };
+        bf16* out = a.out + (size_t)seq * a.out_stride + (size_t)hd * HS + dim;
+        if constexpr (WHOLE) {                               // then the splits, in split order
+            float ms[SPLITS], num[SPLITS], den[SPLITS], top = -INFINITY;
+#pragma unroll
+            for (int u = 0; u < SPLITS; ++u) {
+                float M;
+                merge(u, M, num[u], den[u]);
+                ms[u] = M == -INFINITY ? -INFINITY : M * LN2;
+                top = fmaxf(top, ms[u]);
+            }
+            float w[SPLITS], o = 0.f, z = 0.f;
+            int n_live = 0;
+#pragma unroll
+            for (int u = 0; u < SPLITS; ++u) {
+                w[u] = (top == -INFINITY || ms[u] == -INFINITY) ? 0.f : expf(minus_rounded(ms[u], top));
+                if (w[u] != 0.f) n_live = u + 1;
+            }
+#pragma unroll
+            for (int u = 0; u < SPLITS; ++u) {
+                if (u >= n_live) break;
+                z = fmaf(w[u], den[u], z);
+                o = fmaf(w[u], w[u] != 0.f ? num[u] : 0.f, o);
+            }
+            *out = __float2bfloat16(o * (z > 0.f ? 1.0f / z : 0.f));
         } else {
-            const size_t prow = ((size_t)seq * a.H + hd) * a.n_splits + split;
-            a.part_o[prow * HS + dim] = num;
-            if (dim == 0) { a.part_ml[prow * 2] = (M == -INFINITY) ? -INFINITY : M * LN2; a.part_ml[prow * 2 + 1] = den; }
+            float M, num, den;
+            merge(0, M, num, den);
+            if (a.n_splits == 1) {
+                *out = __float2bfloat16(den > 0.f ? num / den : 0.f);
+            } else {
+                const size_t prow = ((size_t)seq * a.H + hd) * a.n_splits + split;
+                a.part_o[prow * HS + dim] = num;
+                if (dim == 0) { a.part_ml[prow * 2] = (M == -INFINITY) ? -INFINITY : M * LN2; a.part_ml[prow * 2 + 1] = den; }
+            }
         }
     }
 }
@@ -1044,25 +1086,26 @@ static int attn_mfma_launch(const void* q, int q_stride, void* out, int out_stri
         return hs == 64 ? go(attn_mfma_prompt_kernel<64, 4, 2>, 0) : go(attn_mfma_prompt_kernel<128, 2, 2>, 1);
     }
     if (n_tiles > 65535) return BN_ERR_ARG;                 // sequences are the grid's y
-    const dim3 grid(Hkv * n_head_tiles, n_tiles, n_splits);
-    auto go = [&](auto kernel, int nw) {
-        const size_t smem = (size_t)nw * hs * (GT + 1) * sizeof(float);
-        if (smem > 48 * 1024) {
+    // Two splits and no more workgroups than CUs: both in one workgroup, without a launch for the merge (WHOLE).  us, merged by a
+    // kernel -> whole: 8B heads, one sequence of 253 keys 9.0 -> 6.2, three of 317 10.2 -> 7.6, 16 of 381 12.2 -> 9.3, of 573 14.3 ->
+    // 11.9, of 1,021 19.0 -> 17.5, 31 of 573 19.7 -> 16.2; 16 heads over one row, 128 of 573 17.7 -> 14.4.  Up to 16 pages: with sequences
+    // of unequal lengths (16 to 64 a page) and half as many workgroups as CUs 16 pages 16.1 -> 15.8, 20 pages 17.4 -> 17.8, 24 pages 18.9
+    // -> 20.1 (a long sequence has one CU, not two).  Three and four splits a workgroup, two after two: 8 pages 9.3 -> 10.2, 9 pages
+    // 10.4 -> 10.8, not taken.
+    const bool whole = n_splits == 2 && window == 0 && bt_stride <= AD_WHOLE_PAGES && (long long)n_tiles * wgs_per_seq <= compute_units();
+    auto go = [&](auto kernel, int which) {
+        const size_t smem = (size_t)(whole ? 8 : 4) * hs * (GT + 1) * sizeof(float);
+        static bool raised[4] = {false, false, false, false};
+        if (smem > 48 * 1024 && !raised[which]) {
             const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
             if (e != hipSuccess) return (int)e;
+            raised[which] = true;
         }
-        hipLaunchKernelGGL(kernel, grid, dim3(64 * nw), smem, s, a);
+        hipLaunchKernelGGL(kernel, dim3(Hkv * n_head_tiles, n_tiles, whole ? 1 : n_splits), dim3(whole ? 512 : 256), smem, s, a);
         return bn_launch_status();
     };
-    // Sequences of five to nine pages whole, a workgroup a CU at the most: eight waves, which take a second block of 32 keys where
-    // four take a third to a fifth.  us, 8B heads, four waves / eight: one sequence of 250 keys 7.0 / 6.8, 380 8.6 / 8.0, 510 10.0 / 9.0,
-    // 16 of 250 8.3 / 8.7, 380 10.1 / 9.5, 570 13.6 / 12.1; shorter ones leave the waves without keys (16 of 125 6.8 / 8.1).  Cut
-    // and merged by a kernel of its own 510 keys take 9.4, 16 times 14.0; 700 are better cut (10.2 against 11.1).  A table that is
-    // wider says nothing of its sequences, and 16 waves spill their registers (14.6 at 600 keys).
-    const bool wide = n_splits == 1 && window == 0 && bt_stride > 4 && bt_stride <= BN_UNSPLIT_PAGES &&
-                      (long long)n_tiles * wgs_per_seq <= compute_units();
-    const int rc = wide ? (hs == 64 ? go(attn_mfma_decode_kernel<64, 8>, 8) : go(attn_mfma_decode_kernel<128, 8>, 8))
-                        : (hs == 64 ? go(attn_mfma_decode_kernel<64, 4>, 4) : go(attn_mfma_decode_kernel<128, 4>, 4));
+    if (whole) return hs == 64 ? go(attn_mfma_decode_kernel<64, true>, 0) : go(attn_mfma_decode_kernel<128, true>, 1);
+    const int rc = hs == 64 ? go(attn_mfma_decode_kernel<64, false>, 2) : go(attn_mfma_decode_kernel<128, false>, 3);
     if (rc != 0 || n_splits == 1) return rc;
     hipLaunchKernelGGL(attn_mfma_combine_kernel, dim3(n_tokens * H), dim3(64), 0, s, (bf16*)out, out_stride, part_o,
                        part_ml, H, hs, n_splits);

@@ -10,8 +10,6 @@
 // Decode attention splits a sequence's keys over workgroups in runs of at least this many pages: shorter
 // runs cost more in merging than they gain in parallelism (measured at batch 1, 8 and 64 of an 8B shape).
 #define BN_SPLIT_MIN_PAGES 2
-// Sequences of up to this many pages are not cut for the matrix-core decode kernel (attn_mfma.hip: measured on both sides).
-#define BN_UNSPLIT_PAGES 9
 // A float32 cache's keys are summed by attn_rows.hip (what attn_f32.hip, with runs of its own, does not take) in runs of this
 // many positions (whole pages, counted from position 0), each run by
 // itself and the runs folded in order: a decode step then spreads a long sequence's runs over workgroups and still forms
@@ -195,7 +193,8 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
 }
 
 // Keys per split of a decode step whose longest sequence holds max_len keys, cut into n_splits runs of whole
-// pages (the same rule as ops.decode_splits): the kernels use it when the length arrives in device memory.
+// pages: the kernels use it when the length arrives in device memory.  (ops.decode_splits, which makes a plan for a length
+// that the host knows, cuts an even number of pages in the same runs while two pages a split are left; an odd one in longer runs.)
 __host__ __device__ __forceinline__ int bn_split_chunk(int max_len, int n_splits) {
     const int pages = max_len > 0 ? (max_len + BN_PAGE - 1) / BN_PAGE : 1;
     int per = (pages + n_splits - 1) / n_splits;

@@ -19,7 +19,6 @@ from .csrc import build as _build
 
 PAGE = _build.header_constant("BN_PAGE")                         # tokens per cache page: defined once, in csrc/common.h
 F32_FOLD_KEYS = _build.header_constant("BN_F32_FOLD_KEYS")       # a float32 cache's keys are summed in runs of this many
-UNSPLIT_PAGES = _build.header_constant("BN_UNSPLIT_PAGES")       # sequences that decode attention on the matrix cores does not cut
 SPLIT_MIN_PAGES = _build.header_constant("BN_SPLIT_MIN_PAGES")   # shortest run of pages that decode attention splits off
 _DT = {torch.float32: 0, torch.bfloat16: 1}
 
@@ -1541,7 +1540,7 @@ DECODE_TARGET_WGS = int(os.environ.get("BITNET_DECODE_WGS", "256"))
 VECTOR_DECODE_TARGET_WGS = int(os.environ.get("BITNET_VECTOR_DECODE_WGS", "1024"))     # see decode_splits
 
 
-def decode_splits(n_seqs: int, H: int, Hkv: int, max_len: int, dtype=None, target_wgs: int = 0, unsplit_pages: int = 0):
+def decode_splits(n_seqs: int, H: int, Hkv: int, max_len: int, dtype=None, target_wgs: int = 0):
     """(n_splits, chunk): how the keys of a decode step are cut so that the launch fills the
     chip.  A function of the batch's shape and of max_len alone.  A float32 cache is cut in runs of F32_FOLD_KEYS
     positions whatever the batch: both forms of the float32 kernel sum a query's keys run by run and fold the runs in
@@ -1557,8 +1556,7 @@ def decode_splits(n_seqs: int, H: int, Hkv: int, max_len: int, dtype=None, targe
     # target_wgs: another aim than DECODE_TARGET_WGS (the vector kernel's workgroups are small, several fit on a CU and
     # hide each other's waits: VECTOR_DECODE_TARGET_WGS)
     target = target_wgs or DECODE_TARGET_WGS
-    # unsplit_pages: sequences of up to that many pages stay whole (UNSPLIT_PAGES for the matrix-core kernel)
-    want = 1 if pages <= unsplit_pages else max(1, min(pages // SPLIT_MIN_PAGES, 64, (target + wgs - 1) // wgs))
+    want = max(1, min(pages // SPLIT_MIN_PAGES, 64, (target + wgs - 1) // wgs))
     chunk = ((pages + want - 1) // want) * PAGE
     n_splits = (pages * PAGE + chunk - 1) // chunk
     return n_splits, chunk

@@ -322,8 +322,7 @@ class Attention(Part):
             if self.window:
                 n_splits, chunk = 1, 0
             else:
-                n_splits, chunk = ops.decode_splits(ctx.n_rows, H, Hkv, kv.max_len, h.dtype,
-                                                    unsplit_pages=ops.UNSPLIT_PAGES if blocked else 0)
+                n_splits, chunk = ops.decode_splits(ctx.n_rows, H, Hkv, kv.max_len, h.dtype)
             ops.attention(qkv, out, kv.k_pages, kv.v_pages, kv.block_table, H, Hkv, hs, self.scale,
                           window=self.window, seq_lens=ctx.seq_lens, n_splits=n_splits, chunk=chunk,
                           fused_rotate=inv_freq, fused_write=kv.writes, by_length=ctx.by_length,
@@ -335,8 +334,7 @@ class Attention(Part):
             if self.window:                   # a window is short; its keys are not split
                 n_splits, chunk = 1, 0
             else:
-                n_splits, chunk = ops.decode_splits(ctx.n_rows, H, Hkv, kv.max_len, h.dtype,
-                                                    unsplit_pages=ops.UNSPLIT_PAGES if blocked else 0)
+                n_splits, chunk = ops.decode_splits(ctx.n_rows, H, Hkv, kv.max_len, h.dtype)
             ops.attention(qkv, out, kv.k_pages, kv.v_pages, kv.block_table, H, Hkv, hs, self.scale,
                           window=self.window, seq_lens=ctx.seq_lens, n_splits=n_splits, chunk=chunk,
                           by_length=ctx.by_length, max_len_dev=ctx.max_len_dev if n_splits > 1 else None,

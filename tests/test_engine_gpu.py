@@ -907,6 +907,24 @@ def test_a_graph_row_that_changes_its_owner_holds_nothing_of_the_former_one(mode
     eng.cache.check()
 
 
+@pytest.mark.parametrize("n", [250, 372, 500])
+def test_eager_steps_of_few_pages_sum_as_replays_of_a_wide_table_do(model_folders, n):
+    """Sequences of four, six and eight pages: the plan of an eager step, made for their own length, and that of a captured step,
+    made for the longest sequence that the engine allows and cut by the length on the device, are runs of two pages alike, and a
+    launch that merges them inside its workgroups adds them as the merge kernel does.  The same bits."""
+    import bitnet_c_amd as bn
+    folder = model_folders("E", torch.bfloat16)
+    outs = []
+    for graphs in (True, False):
+        eng = bn.Engine.from_folder(folder, dtype=torch.bfloat16, max_tokens=2048, use_graphs=graphs)
+        assert eng.max_pages == 32
+        s = eng.new_sequence()
+        eng.step([bn.StepEntry(s, [(7 * i) % 300 for i in range(n)], [])])
+        outs.append(torch.cat([eng.step([bn.StepEntry(s, [(5 * i) % 300], [0])]) for i in range(6)]))
+        assert bool(eng._graphs) == graphs
+    assert torch.equal(*outs)
+
+
 def test_decode_steps_of_many_sequences_are_replayed_from_graphs(model_folders):
     """300 sequences decode together: more than the largest captured step holds (256 rows), so the step is replayed in
     two pieces (256 rows and 48 rows for the other 44); then 70 of them go on (a captured step of 96 rows).  float32:

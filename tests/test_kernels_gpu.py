@@ -322,8 +322,7 @@ def test_decode_attention_applies_a_deferred_norm_s_factor(H, Hkv, hs, n_splits)
         ops.attention(raw.cuda(), out, k_pages, v_pages, bt.cuda(), H, Hkv, hs, hs ** -0.5, seq_lens=d_lens, row_scale=pre)
 
 
-# sequences that are not cut, by the width of the table: four and eight waves, tables at the edges of the choice; lengths: one key,
-# a block's and a page's edges, waves without keys
+# sequences that are not cut, by the width of the table; lengths: one key, a block's and a page's edges, waves without keys
 @pytest.mark.parametrize("H,Hkv,hs", [(8, 2, 128), (6, 6, 64), (16, 1, 128)])
 @pytest.mark.parametrize("W", [1, 4, 5, 9, 10])
 def test_whole_sequences_of_decode_attention(H, Hkv, hs, W):
@@ -343,6 +342,62 @@ def test_whole_sequences_of_decode_attention(H, Hkv, hs, W):
         want = torch.matmul(torch.softmax(s, dim=-1).unsqueeze(1), v).reshape(-1)
         # a weight's and the result's rounding to bf16 (2^-9 each, the weights' sum in float32)
         assert float((out[b].float().cpu() - want).norm()) <= 2.0 ** -7 * float(want.norm()) + 1e-6, (b, lens[b])
+
+
+# launches of two splits: one workgroup takes both and merges them, or, with a wider table, a kernel of its own does; the same bits, with
+# the rotation and the store that every decode step takes.  The new token lies in each wave's first block of each split, at their
+# edges and behind them; splits without keys, a row that is nobody's; tables at the edges of the choice
+@pytest.mark.parametrize("H,Hkv,hs", [(8, 2, 128), (6, 6, 64), (16, 1, 128), (5, 1, 64)])
+@pytest.mark.parametrize("W", [4, 5, 9, 16])
+def test_two_splits_merged_by_their_workgroup(H, Hkv, hs, W):
+    ops = _ops()
+    dtype = torch.bfloat16
+    before = [p for p in (0, 31, 32, 64, 96, 127, 128, 159, 160, 191, 192, 223, 224, 255, 256, 300, 575, 639, 64 * W - 1) if p < 64 * W]
+    B = len(before) + 1
+    ks = [_rand((p + 1, Hkv, hs), dtype, 10 + i) for i, p in enumerate(before)]
+    vs = [_rand((p + 1, Hkv, hs), dtype, 60 + i) for i, p in enumerate(before)]
+    kp, vp, bt = _paged([k[:-1] if len(k) > 1 else k for k in ks], [v[:-1] if len(v) > 1 else v for v in vs], dtype,
+                        sum((p + 64) // 64 for p in before) + 2, 90)
+    tables = torch.zeros((B, W), dtype=torch.int32)
+    tables[:B - 1, :bt.shape[1]] = bt
+    used = set(bt.flatten().tolist())
+    free = iter([p for p in range(kp.shape[0] + B) if p not in used])      # a new token that opens a page gets one of its own
+    for b, p in enumerate(before):
+        if p % 64 == 0 and p > 0:
+            tables[b, p // 64] = next(free)
+    grow = lambda t: torch.cat([t, torch.full((B,) + t.shape[1:], float("nan"), dtype=dtype)])
+    kp, vp = grow(kp), grow(vp)
+    qkv = _rand((B, (H + 2 * Hkv) * hs), dtype, 91)
+    for b in range(B - 1):                                # the last key of a sequence is the one of the new row, not rotated yet
+        ks[b][-1], vs[b][-1] = qkv[b, H * hs:(H + Hkv) * hs].view(Hkv, hs), qkv[b, (H + Hkv) * hs:].view(Hkv, hs)
+    inv = pl.rope_inv_freq(hs, 10000.0)
+    lens = torch.tensor([p + 1 for p in before] + [0], dtype=torch.int32).cuda()
+    outs = []
+    for width, dev in ((W, True), (W, False), (W + 16, True)):
+        table = torch.zeros((B, width), dtype=torch.int32)
+        table[:, :W] = tables
+        k_pages, v_pages = kp.clone().cuda(), vp.clone().cuda()
+        out = torch.full((B, H * hs), float("nan"), dtype=dtype).cuda()
+        ops.attention(qkv.cuda(), out, k_pages, v_pages, table.cuda(), H, Hkv, hs, hs ** -0.5, seq_lens=lens, n_splits=2,
+                      chunk=ops.split_chunk(64 * W, 2), fused_rotate=inv.cuda(), fused_write=True,
+                      max_len_dev=torch.tensor([64 * W], dtype=torch.int32).cuda() if dev else None)
+        outs.append((out.cpu(), k_pages.cpu(), v_pages.cpu()))
+    for other in outs[1:]:
+        for a, b in zip(outs[0], other):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    got = outs[0][0].float()
+    assert not bool(got[-1].any())
+    for b, p in enumerate(before):
+        pos = torch.tensor([p])
+        q = pl.apply_rope(qkv[b:b + 1, :H * hs].float().view(1, H, hs), pos, inv).to(dtype).float()[0]
+        k, v = ks[b].float(), vs[b].float()
+        k[-1] = pl.apply_rope(k[-1:], pos, inv).to(dtype).float()[0]
+        k, v = (t.repeat_interleave(H // Hkv, dim=1).transpose(0, 1).contiguous() for t in (k, v))
+        s = torch.matmul(k, q.view(H, hs, 1)).squeeze(-1) * hs ** -0.5
+        want = torch.matmul(torch.softmax(s, dim=-1).unsqueeze(1), v).reshape(-1)
+        # a weight's and the result's rounding to bf16 (2^-9 each) and a rotated number's that falls to the other side (2^-8 of
+        # one of hs numbers of q and k)
+        assert float((got[b] - want).norm()) <= 2.0 ** -7 * float(want.norm()) + 1e-6, (b, p)
 
 
 def test_partial_sums_refuse_what_they_cannot_take():
