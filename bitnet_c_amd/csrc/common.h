@@ -90,10 +90,13 @@ __device__ __forceinline__ void bn_rotate_pair(float& x0, float& x1, float c, fl
 __device__ __forceinline__ float bf16lo_to_f32(uint32_t two) { return __uint_as_float(two << 16); }
 __device__ __forceinline__ float bf16hi_to_f32(uint32_t two) { return __uint_as_float(two & 0xffff0000u); }
 
-// Sixteen bytes that a launch reads once (a weight matrix that streams past, a cached key or value of a decode step), as a
+// Sixteen bytes that a launch reads once (a streamed copy of weights, the blocked keys and values of a decode step), as a
 // non-temporal load: the line takes no other line's place in the L2 for long.  A plain read of cold memory by 256 to 1,792
 // workgroups, us without and with it: 8 MB 3.45 / 3.12, 32 MB 6.7 / 6.4, 48 MB 9.3 / 8.8, 112 MB 19.5 / 18.4, 224 MB
-// 38.0 / 35.8; no slower where the bytes lie in a cache from the launch before.
+// 38.0 / 35.8; no slower where the bytes lie in a cache from the launch before.  Where one load of a wave takes half a line of each
+// of 16 rows and another one the other half (row-major weights) plain loads are faster, since the line is asked for twice: us at
+// one row, with it / plain, 2,048 x 2,048 5.4 / 4.7, 2,048 x 5,632 10.9 / 9.8, 28,672 x 4,096 45.8 / 41.6, 4,096 x 14,336 26.9 / 25.2
+// (4,096 x 4,096 9.3 / 9.4), partial sums of 32 rows 2,048 x 2,048 8.7 / 7.7, 4,096 x 14,336 29.5 / 27.2.
 typedef __attribute__((ext_vector_type(4))) uint32_t bn_u32x4;
 __device__ __forceinline__ uint4 bn_load_once(const void* p) {
     return __builtin_bit_cast(uint4, __builtin_nontemporal_load(static_cast<const bn_u32x4*>(p)));

@@ -98,8 +98,8 @@ __device__ __forceinline__ void skinny_gemm_body(const bf16* __restrict__ X, con
                 wv[j] = (i < CW && kc + j * 32 < K) ? bn_load_once(wrow + (size_t)((kc >> 5) + j) * TS + lane_at)
                                                     : make_uint4(0, 0, 0, 0);
             else
-                wv[j] = (k < K) ? bn_load_once(wrow + k) : make_uint4(0, 0, 0, 0);
-            if (DUAL) uv[j] = (k < K) ? bn_load_once(urow + k) : make_uint4(0, 0, 0, 0);
+                wv[j] = (k < K) ? *reinterpret_cast<const uint4*>(wrow + k) : make_uint4(0, 0, 0, 0);
+            if (DUAL) uv[j] = (k < K) ? *reinterpret_cast<const uint4*>(urow + k) : make_uint4(0, 0, 0, 0);
         }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
@@ -253,7 +253,7 @@ void skinny_gemm_fused_kernel(const bf16* __restrict__ X, const bf16* __restrict
                 wv[j] = (col && kc + j * 32 < K) ? bn_load_once(wrow + (size_t)((kc >> 5) + j) * TS + lane_at)
                                                  : make_uint4(0, 0, 0, 0);
             else
-                wv[j] = (col && k < K) ? bn_load_once(wrow + k) : make_uint4(0, 0, 0, 0);
+                wv[j] = (col && k < K) ? *reinterpret_cast<const uint4*>(wrow + k) : make_uint4(0, 0, 0, 0);
         }
     };
     auto multiply = [&](const uint4* wv, const uint4* xd) {

@@ -96,6 +96,8 @@ __global__ __launch_bounds__(NWV * 64) void splitk_gemm_kernel(const bf16* __res
     for (int a = 0; a < MT; ++a) acc[a] = (f32x4){0.f, 0.f, 0.f, 0.f};
     uint4 wa[8], wb[8], xd[XL];
 
+    // a streamed copy's bytes are read once, whole lines at a time; a row of W half a line at a time (bn_load_once)
+    auto weight = [](const bf16* p) { return TILED ? bn_load_once(p) : *reinterpret_cast<const uint4*>(p); };
     // K is a multiple of 8 and so are k_begin and every k below: a 16-byte load at k < k_end stays inside the row.
     // A step that lies wholly inside [k_begin, k_end) needs no test per load.
     auto load_x = [&](int k0) {
@@ -115,11 +117,11 @@ __global__ __launch_bounds__(NWV * 64) void splitk_gemm_kernel(const bf16* __res
         const int kl = TILED ? k0 : k0 + g * 8;
         if (col && k0 + SG_STEP <= k_end) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) dst[j] = bn_load_once(p + j * JS);
+            for (int j = 0; j < 8; ++j) dst[j] = weight(p + j * JS);
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j)
-                dst[j] = (col && kl + j * 32 < k_end) ? bn_load_once(p + j * JS) : make_uint4(0, 0, 0, 0);
+                dst[j] = (col && kl + j * 32 < k_end) ? weight(p + j * JS) : make_uint4(0, 0, 0, 0);
         }
     };
     auto store_x = [&](int buf) {
@@ -171,7 +173,7 @@ __global__ __launch_bounds__(NWV * 64) void splitk_gemm_kernel(const bf16* __res
         const int JS = TILED ? TS : 32;
         const bf16* p = TILED ? wrow + (size_t)(k0 >> 5) * TS + lane_at_w : wrow + k0 + g * 8;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dst[j] = bn_load_once(p + j * JS);
+        for (int j = 0; j < 8; ++j) dst[j] = weight(p + j * JS);
     };
     auto store_x_all = [&](const uint4* src, int buf) {
         unsigned char* b = xs + (size_t)buf * ROWS * SG_XROW;
