@@ -54,10 +54,13 @@ struct GenArgs {
     int keep_first;           // with a window: the first keep_first positions stay visible however far back they are
 };
 
-// sixteen bytes that the launch reads once: a decode step's cached keys and values
-__device__ __forceinline__ bf16x8 ag_ld16_once(const bf16* p) { return __builtin_bit_cast(bf16x8, bn_load_once(p)); }
 __device__ __forceinline__ bf16x8 ag_ld16(const bf16* p) {
     return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
+}
+// a decode step's cached keys and values; ONCE: non-temporally
+template <bool ONCE> __device__ __forceinline__ bf16x8 ag_ld16_cached(const bf16* p) {
+    if constexpr (ONCE) return __builtin_bit_cast(bf16x8, bn_load_once(p));
+    else return ag_ld16(p);
 }
 
 // the largest of a value over the lanes 16, 32 and 48 away (the four lane groups of a column): two half-wave swaps between registers
@@ -313,7 +316,16 @@ struct GenDecodeArgs {
     float scale;
 };
 
-template <int DC, int DT>     // hs = 32 DC, vd = 16 DT
+// Keys and values that one wave reads each are read non-temporally (ONCE) while a launch's tables hold no more than this many MB of
+// them: a load takes half a line, of a key the next load the other half and of a value the next block's, and what the L2
+// does not hold in between is fetched twice.  us over memory that no cache holds, plain / non-temporal: one sequence of 2,000 at 16
+// heads over 4 (4 MB) 10.8 / 10.3, four of 2,000 (16 MB) 11.6 / 11.3, 16 of 300 over 8 (20 MB) 13.7 / 13.7, 16 of 1,000 over 4 (33 MB)
+// 14.4 / 14.6, 16 of 2,000 (66 MB) 21.1 / 22.6, 16 of 1,000 over 16 (131 MB) 33.8 / 38.4; of 300 keys alone 11.3 / 11.6.  Where
+// several waves read them: 64 heads over one, one of 500 10.3 / 11.1, 16 of 2,000 20.9 / 21.7.  (Both loops in one kernel, chosen by
+// the length on the device: 0.4 us slower than either.)
+#define AG_ONCE_MB 24
+
+template <int DC, int DT, bool ONCE>     // hs = 32 DC, vd = 16 DT
 __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeArgs a) {
     constexpr int HS = 32 * DC, VD = 16 * DT;
     const int seq = blockIdx.x, split = blockIdx.z;
@@ -371,7 +383,7 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
         const int page = a.block_table[(size_t)seq * a.bt_stride + kb / BN_PAGE];
         const bf16* kbase = a.k_pages + (((size_t)page * a.Hkv + kvh) * BN_PAGE + kb % BN_PAGE + krow) * HS + 8 * g;
 #pragma unroll
-        for (int c = 0; c < DC; ++c) { kn0[c] = ag_ld16_once(kbase + 32 * c); kn1[c] = ag_ld16_once(kbase + 4 * HS + 32 * c); }
+        for (int c = 0; c < DC; ++c) { kn0[c] = ag_ld16_cached<ONCE>(kbase + 32 * c); kn1[c] = ag_ld16_cached<ONCE>(kbase + 4 * HS + 32 * c); }
     };
     const int first_block = k_lo & ~31, last_block = ((k_hi - 1) / 32) * 32;
     auto leap = [&](int kb) { return kb >= keep && kb < first_block ? first_block : kb; };
@@ -391,7 +403,7 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
         }
         bf16x8 va[DT];
 #pragma unroll
-        for (int t = 0; t < DT; ++t) va[t] = ag_ld16_once(vbase + (size_t)t * 16 * BN_PAGE);
+        for (int t = 0; t < DT; ++t) va[t] = ag_ld16_cached<ONCE>(vbase + (size_t)t * 16 * BN_PAGE);
         float s[8];
         ag_scores(s, st0, st1, scale2, bias, ba, bb, qpos, kb + 8 * g);
         float mx = -INFINITY;
@@ -575,8 +587,11 @@ extern "C" int bn_attn_general_prompt(const void* q, int q_stride, void* out, in
 }
 
 template <int DC>
-static int ag_launch_decode_dt(const GenDecodeArgs& a, int vd, dim3 grid, hipStream_t s) {
-#define AG_CASE(DT) hipLaunchKernelGGL((attn_general_decode_kernel<DC, DT>), grid, dim3(BN_WAVE), 0, s, a); return bn_launch_status()
+static int ag_launch_decode_dt(const GenDecodeArgs& a, int vd, bool once, dim3 grid, hipStream_t s) {
+#define AG_CASE(DT)                                                                                                       \
+    if (once) hipLaunchKernelGGL((attn_general_decode_kernel<DC, DT, true>), grid, dim3(BN_WAVE), 0, s, a);               \
+    else hipLaunchKernelGGL((attn_general_decode_kernel<DC, DT, false>), grid, dim3(BN_WAVE), 0, s, a);                   \
+    return bn_launch_status()
     switch (vd / 16) {
         case 2: AG_CASE(2);
         case 4: AG_CASE(4);
@@ -613,15 +628,17 @@ extern "C" int bn_attn_general_decode(const void* q, int q_stride, void* out, in
     a.q_stride = q_stride; a.out_stride = out_stride; a.bt_stride = bt_stride; a.H = H; a.Hkv = Hkv; a.n_splits = n_splits;
     a.chunk = chunk; a.window = window; a.sink = sink ? 1 : 0; a.sink_values = sink ? sink_values : nullptr; a.scale = scale;
     const dim3 grid(n_seqs, Hkv * head_tiles, n_splits);
+    const long long held = (long long)bt_stride * BN_PAGE, seen = (long long)window + keep_first;     // keys a sequence at the most
+    const bool once = head_tiles == 1 && (window > 0 && seen < held ? seen : held) * n_seqs * Hkv * (hs + vd) * 2 <= (long long)AG_ONCE_MB << 20;
     int rc = BN_ERR_ARG;
     switch (hs / 32) {
-        case 1: rc = ag_launch_decode_dt<1>(a, vd, grid, s); break;
-        case 2: rc = ag_launch_decode_dt<2>(a, vd, grid, s); break;
-        case 3: rc = ag_launch_decode_dt<3>(a, vd, grid, s); break;
-        case 4: rc = ag_launch_decode_dt<4>(a, vd, grid, s); break;
-        case 5: rc = ag_launch_decode_dt<5>(a, vd, grid, s); break;
-        case 6: rc = ag_launch_decode_dt<6>(a, vd, grid, s); break;
-        case 8: rc = ag_launch_decode_dt<8>(a, vd, grid, s); break;
+        case 1: rc = ag_launch_decode_dt<1>(a, vd, once, grid, s); break;
+        case 2: rc = ag_launch_decode_dt<2>(a, vd, once, grid, s); break;
+        case 3: rc = ag_launch_decode_dt<3>(a, vd, once, grid, s); break;
+        case 4: rc = ag_launch_decode_dt<4>(a, vd, once, grid, s); break;
+        case 5: rc = ag_launch_decode_dt<5>(a, vd, once, grid, s); break;
+        case 6: rc = ag_launch_decode_dt<6>(a, vd, once, grid, s); break;
+        case 8: rc = ag_launch_decode_dt<8>(a, vd, once, grid, s); break;
     }
     if (rc != 0 || n_splits == 1) return rc;
     hipLaunchKernelGGL(attn_general_combine_kernel, dim3(n_seqs * H), dim3(BN_WAVE), 0, s, (bf16*)out, out_stride, part_o, part_ml,

@@ -293,6 +293,28 @@ def test_decode_on_the_matrix_cores_a_batch_with_a_padding_row_and_the_length_on
         assert float(out[2].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("H,G,hs,vd", [(4, 2, 128, 128), (16, 1, 64, 64), (17, 1, 192, 128)])
+def test_decode_reads_keys_alike_whatever_the_launch_could_hold(H, G, hs, vd):
+    """A launch over few keys reads them another way than one over many, by what its table can hold: the same bits."""
+    from bitnet_c_amd import ops
+    from bitnet_c_amd.cache import PAGE
+    g = torch.Generator().manual_seed(H)
+    lens, W = [1, 31, 33, 64, 200, 300, 0], 5
+    B = len(lens)
+    kp = torch.randn(B * W, G, PAGE, hs, generator=g).bfloat16().to(DEV)
+    vp = torch.randn(B * W, G, vd, PAGE, generator=g).bfloat16().to(DEV)
+    q = torch.randn(B, H * hs, generator=g).bfloat16().to(DEV)
+    outs = []
+    for width in (W, 400):
+        assert (width == 400) == (B * G * width * PAGE * (hs + vd) * 2 > 24 << 20)
+        table = torch.zeros(B, width, dtype=torch.int32)
+        table[:, :W] = torch.arange(B * W).view(B, W)
+        out = torch.full((B, H * vd), 5.0, dtype=torch.bfloat16, device=DEV)
+        ops.attention_general_decode(q, out, kp, vp, table.to(DEV), i32(lens), H, G, hs, vd, hs ** -0.5)
+        outs.append(out)
+    assert torch.equal(*outs) and not bool(outs[0][-1].any())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,I,O,T", [(3, 16, 32, 5), (5, 12, 24, 40), (4, 64, 128, 16), (2, 128, 32, 100), (1, 20, 30, 1)])
 def test_a_product_per_head(dtype, H, I, O, T):
