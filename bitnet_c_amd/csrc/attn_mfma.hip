@@ -31,6 +31,7 @@
 #include "common.h"
 #include "attn_mfma.h"
 #include <mutex>
+#include <type_traits>
 
 #define PROMPT_BUFFERS 3      // staged key blocks of the prompt form in shared memory
 
@@ -90,10 +91,13 @@ struct MfmaArgs {
     const int* max_len;
 };
 
-// sixteen bytes that the launch reads once: a decode step's cached keys and values
-__device__ __forceinline__ bf16x8 ld16_once(const bf16* p) { return __builtin_bit_cast(bf16x8, bn_load_once(p)); }
 __device__ __forceinline__ bf16x8 ld16(const bf16* p) {
     return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
+}
+// a decode step's cached keys and values; ONCE: non-temporally
+template <bool ONCE> __device__ __forceinline__ bf16x8 ld16_cached(const bf16* p) {
+    if constexpr (ONCE) return __builtin_bit_cast(bf16x8, bn_load_once(p));
+    else return ld16(p);
 }
 // Combining a value with the ones 16 and 32 lanes away (the four lane groups of a column) without
 // going through shared memory: gfx950 swaps 16- and 32-lane halves between two registers.
@@ -181,16 +185,16 @@ __device__ __forceinline__ int v_swizzle(int row) {
 // this code out, and changes made for the staged form must not move it.
 // The operands of a block of 32 keys from blocked pages: tile row i of key tile 0 is the block's key 8 (i / 4) + i % 4,
 // tile 1 four further; lane i + 16 g of value tile t holds dimension 16 t + i of the block's keys 8 g .. 8 g + 7.
-template <int HS>
+template <int HS, bool ONCE>
 __device__ __forceinline__ void load_block(const bf16* __restrict__ kbase, const bf16* __restrict__ vbase,
                                            bf16x8 (&ka)[HS / 32][2], bf16x8 (&va)[HS / 16], int lane) {
 #pragma unroll
     for (int c = 0; c < HS / 32; ++c) {
-        ka[c][0] = ld16_once(kbase + (2 * c) * 512 + lane * 8);
-        ka[c][1] = ld16_once(kbase + (2 * c + 1) * 512 + lane * 8);
+        ka[c][0] = ld16_cached<ONCE>(kbase + (2 * c) * 512 + lane * 8);
+        ka[c][1] = ld16_cached<ONCE>(kbase + (2 * c + 1) * 512 + lane * 8);
     }
 #pragma unroll
-    for (int t = 0; t < HS / 16; ++t) va[t] = ld16_once(vbase + t * 512 + lane * 8);
+    for (int t = 0; t < HS / 16; ++t) va[t] = ld16_cached<ONCE>(vbase + t * 512 + lane * 8);
 }
 
 template <int HS, int NT, bool need_mask>
@@ -417,7 +421,7 @@ __device__ __forceinline__ void block_weights_values_m(const f32x4 (&st)[NT][2],
 
 // The masked form (a block on the causal diagonal, at a window's edge or at the end of the keys) and
 // the plain one are separate instantiations: almost every block is plain, and it carries no mask code.
-template <int HS, int NT>
+template <int HS, int NT, bool ONCE>
 __device__ __forceinline__ void attend_block(const bf16* __restrict__ kbase, const bf16* __restrict__ vbase,
                                              int kb, const bf16x8 (&q)[NT][HS / 32], f32x4 (&acc)[NT][HS / 16],
                                              float (&m)[NT], float (&l)[NT], const int (&qpos)[NT],
@@ -425,7 +429,7 @@ __device__ __forceinline__ void attend_block(const bf16* __restrict__ kbase, con
                                              int lane) {
     bf16x8 ka[HS / 32][2];
     bf16x8 va[HS / 16];
-    load_block<HS>(kbase, vbase, ka, va, lane);
+    load_block<HS, ONCE>(kbase, vbase, ka, va, lane);
     if (need_mask)
         attend_loaded_m<HS, NT, true>(ka, va, kb, q, acc, m, l, qpos, lo, key_hi, scale2, lane);
     else
@@ -719,7 +723,7 @@ __device__ __forceinline__ float minus_rounded(float a, float b) {
 
 // WHOLE: a workgroup of eight waves takes both splits of a launch of two for its sequence and kv head, four waves a split, and
 // merges them itself, as attn_mfma_combine_kernel would: the same sums in the same order, so that no bit depends on the form.
-template <int HS, bool WHOLE>
+template <int HS, bool WHOLE, bool ONCE>
 __global__ __launch_bounds__(WHOLE ? 512 : 256) void attn_mfma_decode_kernel(MfmaArgs a) {
     constexpr int DC = HS / 32, DT = HS / 16, HALF = HS / 2;
     constexpr int SPLITS = WHOLE ? 2 : 1, THREADS = 256 * SPLITS;
@@ -788,7 +792,7 @@ __global__ __launch_bounds__(WHOLE ? 512 : 256) void attn_mfma_decode_kernel(Mfm
     const size_t at0 = (((size_t)page0 * a.Hkv + kvh) * BN_PAGE + kb_first % BN_PAGE) * HS;
     const bf16* kbase0 = a.k_pages + at0;
     const bf16* vbase0 = a.vt_pages + at0;
-    load_block<HS>(kbase0, vbase0, ka0, va0, lane);
+    load_block<HS, ONCE>(kbase0, vbase0, ka0, va0, lane);
     const bool ok = q_lane && L > 0;
     const int lo_key = a.window > 0 ? max(0, L - a.window) : 0;
     const int k_lo = max(lo_key, split * chunk), k_hi = min(L, (split + 1) * chunk);       // [k_lo, k_hi)
@@ -882,7 +886,7 @@ __global__ __launch_bounds__(WHOLE ? 512 : 256) void attn_mfma_decode_kernel(Mfm
         // the sequences of a large batch: the order by length with unsplit sequences keeps the CUs busiest).
         int kb = (k_lo / 32) * 32 + 32 * wave;
         if (ahead && kb == kb_first && kb < k_hi) {        // the block that was asked for at the start
-            if (a.write_kv && L - 1 >= kb && L - 1 < kb + 32) load_block<HS>(kbase0, vbase0, ka0, va0, lane);
+            if (a.write_kv && L - 1 >= kb && L - 1 < kb + 32) load_block<HS, ONCE>(kbase0, vbase0, ka0, va0, lane);
             if ((kb + 32 > k_hi) || (kb < k_lo))
                 attend_loaded_m<HS, 1, true>(ka0, va0, kb, q, acc, m, l, qpos, lo, k_hi, scale2, lane);
             else
@@ -897,7 +901,7 @@ __global__ __launch_bounds__(WHOLE ? 512 : 256) void attn_mfma_decode_kernel(Mfm
             const bf16* kbase = a.k_pages + (((size_t)page * a.Hkv + kvh) * BN_PAGE + koff) * HS;
             const bf16* vbase = a.vt_pages + (((size_t)page * a.Hkv + kvh) * BN_PAGE + koff) * HS;
             const bool need_mask = (kb + 32 > k_hi) || (kb < k_lo);
-            attend_block<HS, 1>(kbase, vbase, kb, q, acc, m, l, qpos, lo, k_hi, need_mask, scale2, lane);
+            attend_block<HS, 1, ONCE>(kbase, vbase, kb, q, acc, m, l, qpos, lo, k_hi, need_mask, scale2, lane);
         }
     }
     // every wave's (m, l, O^T) into shared memory
@@ -1095,7 +1099,7 @@ static int attn_mfma_launch(const void* q, int q_stride, void* out, int out_stri
     const bool whole = n_splits == 2 && window == 0 && bt_stride <= AD_WHOLE_PAGES && (long long)n_tiles * wgs_per_seq <= compute_units();
     auto go = [&](auto kernel, int which) {
         const size_t smem = (size_t)(whole ? 8 : 4) * hs * (GT + 1) * sizeof(float);
-        static bool raised[4] = {false, false, false, false};
+        static bool raised[8] = {false, false, false, false, false, false, false, false};
         if (smem > 48 * 1024 && !raised[which]) {
             const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
             if (e != hipSuccess) return (int)e;
@@ -1104,8 +1108,17 @@ static int attn_mfma_launch(const void* q, int q_stride, void* out, int out_stri
         hipLaunchKernelGGL(kernel, dim3(Hkv * n_head_tiles, n_tiles, whole ? 1 : n_splits), dim3(whole ? 512 : 256), smem, s, a);
         return bn_launch_status();
     };
-    if (whole) return hs == 64 ? go(attn_mfma_decode_kernel<64, true>, 0) : go(attn_mfma_decode_kernel<128, true>, 1);
-    const int rc = hs == 64 ? go(attn_mfma_decode_kernel<64, false>, 2) : go(attn_mfma_decode_kernel<128, false>, 3);
+    // Keys that many workgroups read (of more than 64 heads over one kv head) are read plainly, others non-temporally.  us, plain /
+    // non-temporal, over memory that no cache holds: 8B heads, one sequence of 2,000 10.6 / 9.7, 16 of 2,000 32.2 / 28.4; 32 heads over one
+    // (two workgroups) one of 2,000 12.0 / 11.4, 64 over one 16 of 500 13.6 / 12.9, of 2,000 19.8 / 20.1; 128 over one one of 500 10.6 /
+    // 11.6, 16 of 2,000 29.0 / 31.7.
+    auto pick = [&](auto w, auto once) {
+        constexpr bool W = decltype(w)::value, O = decltype(once)::value;
+        return hs == 64 ? go(attn_mfma_decode_kernel<64, W, O>, 2 * W + 4 * O) : go(attn_mfma_decode_kernel<128, W, O>, 1 + 2 * W + 4 * O);
+    };
+    const bool once = n_head_tiles <= 4;
+    if (whole) return once ? pick(std::true_type(), std::true_type()) : pick(std::true_type(), std::false_type());
+    const int rc = once ? pick(std::false_type(), std::true_type()) : pick(std::false_type(), std::false_type());
     if (rc != 0 || n_splits == 1) return rc;
     hipLaunchKernelGGL(attn_mfma_combine_kernel, dim3(n_tokens * H), dim3(64), 0, s, (bf16*)out, out_stride, part_o,
                        part_ml, H, hs, n_splits);

@@ -400,6 +400,33 @@ def test_two_splits_merged_by_their_workgroup(H, Hkv, hs, W):
         assert float((got[b] - want).norm()) <= 2.0 ** -7 * float(want.norm()) + 1e-6, (b, p)
 
 
+# many heads over one kv head: four workgroups and five read the same keys, in another way than one does; every tile of 16 heads
+# gives the bits of a launch of its own
+@pytest.mark.parametrize("hs", [64, 128])
+@pytest.mark.parametrize("H", [64, 80, 72])
+@pytest.mark.parametrize("n_splits", [1, 2, 4])
+def test_heads_of_many_workgroups_over_one_key(H, hs, n_splits):
+    ops = _ops()
+    lens = [1, 33, 64, 300, 500]
+    kp, vp, bt = _paged([_rand((l, 1, hs), torch.bfloat16, 10 + l) for l in lens], [_rand((l, 1, hs), torch.bfloat16, 40 + l) for l in lens],
+                        torch.bfloat16, sum((l + 63) // 64 for l in lens) + 2, 90)
+    q = _rand((len(lens), H, hs), torch.bfloat16, 91).cuda()
+    dev = [t.cuda() for t in (kp, vp, bt, torch.tensor(lens, dtype=torch.int32))]
+
+    def run(heads):
+        out = torch.full((len(lens), heads.shape[1] * hs), float("nan"), dtype=torch.bfloat16, device="cuda")
+        ops.attention(heads.reshape(len(lens), -1).contiguous(), out, *dev[:3], heads.shape[1], 1, hs, hs ** -0.5, seq_lens=dev[3],
+                      n_splits=n_splits, chunk=ops.split_chunk(512, n_splits) if n_splits > 1 else 0)
+        return out
+    whole = run(q)
+    for t in range(0, H, 16):
+        few = q[:, t:t + 16]
+        if few.shape[1] < 16:                                # a tile that is not full: 16 heads, the last of them others
+            few = torch.cat([few, q[:, :16 - few.shape[1]]], dim=1)
+        n = min(16, H - t) * hs
+        assert torch.equal(whole[:, t * hs:t * hs + n], run(few)[:, :n])
+
+
 def test_partial_sums_refuse_what_they_cannot_take():
     ops = _ops()
     assert ops.can_split_sums(64, 64, 128, torch.bfloat16) and ops.can_split_sums(128, 64, 512, torch.bfloat16)
