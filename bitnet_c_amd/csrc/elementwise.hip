@@ -800,7 +800,7 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ x, const TD* __res
     const float fb = 1.0f / sqrtf(ss / (float)dim + eps_b);
     float sx = 0.f;
     for (int i = threadIdx.x; i < dim; i += blockDim.x) {
-        const float v = xr[i] + row[i] * fb * wb[i];
+        const float v = fmaf(row[i] * fb, wb[i], xr[i]);
         xr[i] = v;
         row[i] = v;
         sx = fmaf(v, v, sx);
@@ -860,7 +860,7 @@ __global__ __launch_bounds__(256) void add_normed_rmsnorm_wide_kernel(float* __r
         Eight<float> xo;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            v[q][e] = v[q][e] + d[q][e] * fb * gb[q][e];
+            v[q][e] = fmaf(d[q][e] * fb, gb[q][e], v[q][e]);      // written out: SkRowStage (skinny_gemm.hip) forms the same bits
             xo.e[e] = v[q][e];
             sx = fmaf(v[q][e], v[q][e], sx);
         }
