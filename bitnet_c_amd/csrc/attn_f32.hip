@@ -90,8 +90,7 @@ template <int HS> struct AfSums {                 // a lane's sums of its row (r
     }
 };
 
-// One page of keys from nothing.  k(t, b): the lane's 16 bytes of key 16 t + lane % 16, dimensions 16 b + 4 g ..; v(t, e, h):
-// its VW values of key 16 t + 4 g + e; last: the last key of the page that the lane's row sees (63: all, < 0: none).
+// the larger of, and the sum with, the value of the lane 16 or 32 away
 template <int O> __device__ __forceinline__ float af_pair_max(float v) {
     return bn_pair_far<O>(v, [](float a, float b) { return fmaxf(a, b); });
 }
@@ -99,6 +98,8 @@ template <int O> __device__ __forceinline__ float af_pair_sum(float v) {
     return bn_pair_far<O>(v, [](float a, float b) { return __fadd_rn(a, b); });
 }
 
+// One page of keys from nothing.  k(t, b): the lane's 16 bytes of key 16 t + lane % 16, dimensions 16 b + 4 g ..; v(t, e, h):
+// its VW values of key 16 t + 4 g + e; last: the last key of the page that the lane's row sees (63: all, < 0: none).
 template <int HS, typename KF, typename VF>
 __device__ __forceinline__ void af_page(const f32x4 (&q)[HS / 16], float scale, int last, bool masked, KF k, VF v, AfSums<HS>& p) {
     using S = AfShape<HS>;
