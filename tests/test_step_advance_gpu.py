@@ -6,11 +6,15 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_advanced_steps_are_uploaded_steps(model_folders, dtype):
+def test_advanced_steps_are_uploaded_steps(model_folders, dtype, monkeypatch):
     """Tokens from the device, many steps on end: over a page's edge, on a graph wider than the batch, in changed order, after
-    another prompt step, after a step with tokens from the host, in a slot that is used again with the same length."""
+    another prompt step, after a step with tokens from the host, in a slot that is used again with the same length.  Which steps
+    advance is asserted: those on the same graph, of the same sequences in the same order, one token longer on the same pages."""
     import bitnet_c_amd as bn
-    outs, advanced = [], 0
+    from bitnet_c_amd import ops
+    outs, advanced, now = [], [], [None]
+    advance = ops.step_advance
+    monkeypatch.setattr(ops, "step_advance", lambda *args: (advanced.append(now[0]), advance(*args))[1])
     for on_device in (False, True):
         eng = bn.Engine.from_folder(model_folders("B", dtype), dtype=dtype, max_tokens=4096)
         slots = [eng.new_sequence() for _ in range(3)]
@@ -18,6 +22,7 @@ def test_advanced_steps_are_uploaded_steps(model_folders, dtype):
         got = []
 
         def run(sl, k):
+            now[0] = k
             toks = [(11 * k + 5 * i) % 389 for i in range(len(sl))]
             if on_device:
                 dev = torch.tensor(toks, dtype=torch.int32, device="cuda")
@@ -45,6 +50,8 @@ def test_advanced_steps_are_uploaded_steps(model_folders, dtype):
         outs.append(got)
     for i, (a, b) in enumerate(zip(*outs)):
         assert torch.equal(a, b), i
+    # not: 0, 10, 11, 12, 15 (another step before them), 2 and 4 (a new page), 16 (the slot's new pages)
+    assert advanced == [1, 3, 5, 6, 7, 8, 9, 13, 14, 17, 18]
 
 
 def test_step_advance_touches_the_sequences_alone():
