@@ -762,7 +762,7 @@ static size_t gf_streamed_smem(int M, int K, bool norm) {                    // 
 extern "C" int bn_gemm_f32_norm_supports(int M, int K) { return gf_norm_ok(M, K, nullptr); }
 
 // 1 if the kernel over a streamed copy takes the product: up to 16 rows, whole chunks whose sums fit into shared memory
-// (every K up to 10,496, and three times that at 8 rows), rows of activations that are whole 16-byte groups.
+// (every K up to 10,752 at 9 to 16 rows, 29,952 at 5 to 8), rows of activations that are whole 16-byte groups.
 extern "C" int bn_gemm_f32_streamed_supports(int M, int N, int K, int ldx, int tile_rows, const void* x) {
     return M >= 1 && M <= 16 && N >= 1 && K >= GF_CHUNK && K % GF_CHUNK == 0 && gf_streamed_smem(M, K, false) <= GF_STREAMED_SMEM && ldx >= K &&
            ldx % 4 == 0 && ldx <= 1 << 22 && tile_rows >= 1 && tile_rows <= BN_STREAM_TILE_ROWS && ((uintptr_t)x & 15) == 0;

@@ -147,12 +147,18 @@ def test_streamed_copies_give_the_same_bits(M, N, K, R):
 
 
 def test_streamed_copies_whose_sums_do_not_fit_are_not_read():
-    """At 9 to 16 rows shared memory holds the sums of 82 chunks: a longer K is read from the row-major matrix."""
+    """Shared memory holds the sums of 84 chunks at 9 to 16 rows and of 234 at 5 to 8: a longer K is read from the row-major
+    matrix."""
     ops = _ops()
-    x, w = _data(16, 16, 14336, 3)
-    xd, wd = x.cuda(), w.cuda()
-    for m in (8, 16):
-        assert torch.equal(ops.linear(xd[:m].contiguous(), wd, streamed=ops.stream_copy(wd)), ops.linear(xd[:m].contiguous(), wd)), m
+    takes = ops._fn("gemm_f32", "bn_gemm_f32_streamed_supports")
+    for m, most in ((9, 84), (16, 84), (5, 234), (8, 234)):
+        assert takes(m, 16, 128 * most, 128 * most, 16, None) == 1 and takes(m, 16, 128 * (most + 1), 128 * (most + 1), 16, None) == 0
+    for K in (84 * 128, 85 * 128, 14336):
+        x, w = _data(16, 16, K, 3)
+        xd, wd = x.cuda(), w.cuda()
+        sw = ops.stream_copy(wd)
+        for m in (8, 16):
+            assert torch.equal(ops.linear(xd[:m].contiguous(), wd, streamed=sw), ops.linear(xd[:m].contiguous(), wd)), (K, m)
 
 
 # a norm taken into the product behind it, and a product added into the stream, against the kernels of their own: the same bits.
