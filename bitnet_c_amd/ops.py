@@ -1039,6 +1039,21 @@ def takes_stream_norm(pre: DeferredNorm, w: torch.Tensor, streamed: Optional[Str
     return streamed is not None if w.dtype == torch.bfloat16 else f32_product_takes(w)
 
 
+# float32 rows of this many numbers up to F32_STREAM_NORM_MIN_K are better normed by a kernel of their own where the matrix has a
+# streamed copy, which the product behind a norm reads from there on only (a chunk a wave).  us, norm and streamed product / in one
+# over the row-major matrix, N = 4 K gated at 1 / 8 rows: 384 columns 5.0 / 5.2, 5.5 / 5.9, 512 5.2 / 5.5, 5.6 / 6.3, 768 6.3 / 7.3, 6.6 /
+# 8.1, 896 6.9 / 7.7, 7.1 / 8.6; N = K: 384 4.8 / 3.6, 5.1 / 4.4, 512 4.9 / 4.6, 5.2 / 5.5, 768 5.5 / 5.5, 5.9 / 6.4; from 1,024 on 7.3 / 5.7 and
+# 5.8 / 4.4.
+F32_NORM_APART_K = 512
+
+
+def wants_stream_norm(pre: DeferredNorm, w: torch.Tensor, streamed: Optional[StreamedWeight] = None) -> bool:
+    """takes_stream_norm, where that is the faster way."""
+    if w.dtype == torch.float32 and streamed is not None and F32_NORM_APART_K <= w.shape[1] < F32_STREAM_NORM_MIN_K:
+        return False
+    return takes_stream_norm(pre, w, streamed)
+
+
 def linear_stream_norm(pre: StreamNorm, w: torch.Tensor, streamed: Optional[StreamedWeight] = None, glu: bool = False,
                        activation: Optional[str] = None) -> torch.Tensor:
     """linear(rows, w) for the rows of a StreamNorm or a StreamSum, in one kernel: activation(linear) (one of

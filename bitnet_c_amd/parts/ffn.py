@@ -119,7 +119,7 @@ class SwiGLU(Part):
             w = self.gate_up.weight
             M = h.shape[0]
             if isinstance(h, ops.StreamNorm) and not (w.dtype == torch.float32 and not self.has_bias and self.interleaved
-                                                      and ops.takes_stream_norm(h, w)):
+                                                      and ops.wants_stream_norm(h, w, self.gate_up.streamed)):
                 return self.forward(h.materialize(), ctx, lazy_ok)
             if isinstance(h, ops.StreamNorm):
                 act = ops.linear_stream_norm(h, w, self.gate_up.streamed, True, self.activation)

@@ -58,7 +58,7 @@ class Linear:
         if isinstance(x, ops.DeferredNorm):
             M, (N, K) = x.shape[0], w.shape
             if isinstance(x, ops.StreamNorm):
-                if self.bias is None and out_dtype in (None, w.dtype) and ops.takes_stream_norm(x, w, streamed):
+                if self.bias is None and out_dtype in (None, w.dtype) and ops.wants_stream_norm(x, w, streamed):
                     return ops.linear_stream_norm(x, w, streamed)
             elif (self.bias is None and out_dtype in (None, torch.bfloat16) and w.dtype == torch.bfloat16
                     and ops.can_fuse_norm(M, N, K, w.dtype) and w.data_ptr() % 16 == 0):

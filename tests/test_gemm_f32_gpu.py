@@ -191,3 +191,22 @@ def test_products_with_a_norm_and_into_the_stream(M, N, K, R):
         out = ops.linear_into_stream(xd, wd, got, torch.ones(N, device="cuda"), 1e-5, sw)
         assert out.stream is got
         assert torch.equal(got.nan_to_num(7.0), (stream + ops.linear(xd, wd)).nan_to_num(7.0)), sw is None
+
+
+# where a norm stays a kernel of its own because the product reads a streamed copy then; the same bits on every route
+@pytest.mark.parametrize("K", [384, 512, 896, 1024])
+def test_norms_of_narrow_rows_stay_in_front_of_streamed_products(K, monkeypatch):
+    ops = _ops()
+    from bitnet_c_amd.parts.linear import Linear
+    x, w = _data(3, 32, K, K)
+    lin = Linear()
+    lin.load(w, None, torch.device("cuda"), torch.float32)
+    nw, calls = torch.linspace(0.5, 1.5, K, device="cuda"), []
+    inside = ops.linear_stream_norm
+    monkeypatch.setattr(ops, "linear_stream_norm", lambda *a, **k: (calls.append(1), inside(*a, **k))[1])
+    want = ops.linear(ops.add_rmsnorm(x.cuda(), None, nw, 1e-5, torch.float32), w.cuda())
+    for keep in (False, True):
+        lin.keep_streamed(keep)
+        calls.clear()
+        assert torch.equal(lin(ops.stream_norm(x.cuda(), nw, 1e-5)), want)
+        assert len(calls) == (0 if keep and 512 <= K < 1024 else 1)
