@@ -781,6 +781,9 @@ extern "C" int bn_skinny_gemm_supports(int M, int N, int K, int ldx, int ldw);
 // at 1 / 2 / 4 / 8 rows of 2,048 numbers, two kernels -> one: normed rows x 8,192 9.7 / 10.1 / 10.1 / 10.6 -> 7.6 / 7.5 / 8.0 / 9.5; the new
 // stream's x 8,192 9.3 / 9.4 / 9.9 / 10.2 -> 7.4 / 7.5 / 8.6 / 10.9; gated x 2,048 7.0 / 7.1 / 7.1 / 7.9 -> 5.0 / 5.0 / 7.4 / 11.4; five mixes x 4 x
 // 2,048 and 64, three kernels -> one, 13.6 / 13.9 / 14.2 / 15.5 -> 11.1 / 11.0 / 13.6 / 19.6.
+// Narrower rows gain more (a workgroup forms less and the launches cost the same): of 512 numbers, normed x 2,048 at 1 / 4 / 8 rows 4.6 /
+// 4.8 / 4.9 -> 2.9 / 3.8 / 4.5, the new stream's at 1 / 4 4.5 / 4.8 -> 3.0 / 3.8, five mixes 7.6 / 8.3 -> 4.2 / 5.3; of 1,024, gated at 1 / 2
+// 5.8 / 5.9 -> 4.1 / 4.2.
 extern "C" int bn_skinny_rows_supports(int M, int K, int mode) {
     const int most = mode == SK_ROWS_NORM ? 8 : mode == SK_ROWS_SUM || mode == SK_ROWS_SHIFT ? 4 : mode == SK_ROWS_GATE ? 2 : 0;
     return M >= 1 && M <= most && K % SK_CHUNK == 0 && K >= (mode == SK_ROWS_GATE ? 4 : 2) * SK_CHUNK && K <= SK_CHUNK * SK_STREAM_WAVES;
