@@ -21,8 +21,9 @@
 // Prompt form: a workgroup of 4 waves owns 64*NT columns = consecutive query tokens x GT heads;
 // the keys and values it walks are staged through shared memory once for all four waves.
 // Decode form: the 16 columns are the heads of one kv group for the sequence's one new token;
-// the 4 waves take 32-key blocks in turn and merge through shared memory; long contexts are
-// also split over gridDim.z and merged by attn_mfma_combine_kernel in a fixed order.  What a decode workgroup needs
+// 4 waves take 32-key blocks in turn and merge through shared memory; long contexts are
+// also split over gridDim.z and merged by attn_mfma_combine_kernel in a fixed order (two splits: one workgroup
+// of 8 waves where that is the faster way, the same sums in the same order).  What a decode workgroup needs
 // before its first block (the query, the frequencies, the new key and value, the length, the first block itself) is
 // asked for at once, in straight-line code, with the length and the page numbers through the scalar unit: the first
 // block of keys is on its way before the length is known (see the kernel), so that a short launch is two trips to
