@@ -69,6 +69,55 @@ __device__ __forceinline__ int gm_swizzle(int row) {
     return ((-(row >> 2)) & 3) | (((row >> 1) & 1) << 2);
 }
 
+// A 16 x 16 tile of the result: lane (i, g) holds columns 4 g .. 4 g + 3, counted from n, of row m.  vec: rows of Y are aligned so that
+// the four go out as one word.
+template <bool GLU8, typename TO>
+__device__ __forceinline__ void gm_store(TO* __restrict__ Y, f32x4 v, int m, int n, int M, int N, int ldy, int vec, int act, int g, const GmGroups& grp) {
+    auto store4 = [&](TO* dst, int valid) {
+        if (vec && valid >= 4) {
+            if (sizeof(TO) == 4) {
+                *reinterpret_cast<f32x4*>(dst) = v;
+            } else {
+                uint2 p;
+                p.x = (uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[0])) |
+                      ((uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[1])) << 16);
+                p.y = (uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[2])) |
+                      ((uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[3])) << 16);
+                *reinterpret_cast<uint2*>(dst) = p;
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (r < valid) dst[r] = from_f32<TO>(v[r]);
+        }
+    };
+    if (GLU8) {
+        // rows 16t..16t+7 of W are gates, 16t+8..16t+15 the ups of the same result columns:
+        // lanes with g >= 2 hold the ups of what lanes g - 2 hold the gates of
+        f32x4 up;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(v[r], 32, BN_WAVE);
+        if (g < 2 && m < M) {
+            const int f = (n >> 1) + 4 * g;           // result column of v[0]
+#pragma unroll
+            // silu(g) * u with the hardware's exp2 and reciprocal (an ulp each, far below the result's
+            // rounding): expf and a division cost 25 vector instructions a value, a tenth of this kernel's time
+            for (int r = 0; r < 4; ++r)
+                v[r] = (act == BN_ACT_SILU ? v[r] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * v[r]))
+                                           : bn_gate_act(v[r], act)) * up[r];
+            store4(Y + (size_t)m * ldy + f, (N >> 1) - f);
+        }
+    } else if (m < M) {
+        if (grp.unary >= 0) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = bn_unary_act(v[r], grp.unary);
+        }
+        if (grp.row_scale) v *= grp.row_scale[m];
+        const size_t mo = grp.row_map ? (size_t)grp.row_map[m] : (size_t)m;
+        store4(Y + mo * ldy + n + 4 * g, N - n - 4 * g);
+    }
+}
+
 template <int BN, bool GLU8, typename TO>
 __global__ __launch_bounds__(GM_THREADS) void gemm_mfma_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W,
                                                                TO* __restrict__ Y, int M, int N, int K, int ldx, int ldw,
@@ -233,60 +282,217 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_mfma_kernel(const bf16* __res
         }
     }
 
-    // acc[a][b]: lane (i, g) holds columns n = 4g..4g+3 of row m = i of the result tile (a, b); vec: rows of Y
-    // are aligned so that the four go out as one word
-    auto store4 = [&](TO* dst, f32x4 v, int valid) {
-        if (vec && valid >= 4) {
-            if (sizeof(TO) == 4) {
-                *reinterpret_cast<f32x4*>(dst) = v;
-            } else {
-                uint2 p;
-                p.x = (uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[0])) |
-                      ((uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[1])) << 16);
-                p.y = (uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[2])) |
-                      ((uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[3])) << 16);
-                *reinterpret_cast<uint2*>(dst) = p;
-            }
-        } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (r < valid) dst[r] = from_f32<TO>(v[r]);
+    for (int a = 0; a < NT; ++a)
+#pragma unroll
+        for (int b = 0; b < MT; ++b) gm_store<GLU8>(Y, acc[a][b], m0 + wm + b * 16 + i, n0 + wn + a * 16, M, N, ldy, vec, act, g, grp);
+}
+
+// ---------------------------------------------------------------------------------------
+// The same product where K is whole steps of 64 (every ordinary width).  What bounds it is the matrix cores' power: at 8,192 rows the
+// chip runs this kernel a fifth faster over zeros than over numbers, and so it does the library's.
+//
+// Eight waves (2 x 4), two on every SIMD, in two groups: waves 0 .. 3 own the upper half of the tile's rows of X, waves 4 .. 7 the lower
+// one, half a turn behind (one barrier more in front of their loop, one less behind it).  A step is two turns of a group: it reads
+// operands from shared memory while the other group multiplies, then multiplies while the other reads, a barrier between; so the
+// matrix cores of a SIMD have one wave's products at a time and never wait for shared memory.  The tile's rows of X are taken in two
+// parts (first and second half of each group's), W's in two as well: turn I reads X's first part and both of W's and multiplies
+// these, turn II reads X's second part in their place and multiplies it with W's parts that are still in registers.
+//
+// Loads go from memory straight into shared memory (16 bytes a lane; the swizzle of gm_swizzle lies in the address that a lane asks
+// for), into buffers of their own names for every part of the even and the odd steps, so that the compiler knows which loads a read of
+// shared memory waits for.  A part's buffer is asked for again, for the step after the next, as soon as both groups have read it, a
+// step and a half before it is needed: X's first part and W's two in turn II of the step that read them, X's second part in turn I of
+// the next.  The waits are counts of a wave's own later loads; the barrier behind them makes them everybody's.
+//   us, registers and one barrier a step (above) -> this, 256 x 256: 4,096 x 4,096 at 4,096 rows 139 -> 101, 28,672 x 4,096 at 2,048 /
+//   8,192 rows 479 / 1,892 -> 378 / 1,357, 4,096 x 14,336 at 8,192 870 -> 643 (1.50 PFLOP/s; the library 607).  Four waves of 128 x 128
+//   over a ring of four stages of 32 took 1,569 at 28,672 x 4,096 x 8,192, the 32x32x16 instruction 1,459.
+//
+// splits > 1: K is cut into that many ranges of steps_per steps, Y holds a slab of float32 sums for each.
+// Workgroups: XCD x takes a run of the tiles, a run is walked in bands of GM_BAND row tiles, the band's rows fastest, so that the
+// workgroups which an XCD runs at a time share rows of X and of W in its L2.
+#define GM_BAND 4
+// EPI: what becomes of the sums.  Each has kernels of its own: a choice between them at run time makes the epilogue too long for the
+// instruction cache (28,672 x 4,096 with its gated unit at 2,048 rows 366 us, with every activation in one kernel 395).
+#define GM_STORE 0                    // stored (TO)
+#define GM_SILU 1                     // silu(gate) * up
+#define GM_GATED 2                    // act(gate) * up, the other activations
+#define GM_GROUPED 3                  // the grouped form's
+template <int BM, int BN, int EPI, typename TO>
+__global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, TO* __restrict__ Y, int M,
+                                                            int N, int K, int ldx, int ldw, int ldy, int tiles_m, int tiles_n, int splits,
+                                                            int steps_per, int act, GmGroups grp) {
+    constexpr int WM = BM / 2, WN = BN / 4;              // a wave's part of the tile, taken in quarters of (16 MH) x (16 NH)
+    constexpr int MH = WM / 32, NH = WN / 32;
+    constexpr int XL = (BM / 2 + 63) / 64, WL = BN / 128;        // loads of a wave for a part: 8 rows each
+    constexpr int XP = BM / 2 % 64 / 8;                  // waves that take the last of X's (0: all)
+    static_assert(BM % 64 == 0 && BN % 128 == 0, "whole 16 x 16 tiles in a quarter");
+    __shared__ __align__(1024) unsigned char xa0[BM / 2 * 128], xa1[BM / 2 * 128], xb0[BM / 2 * 128], xb1[BM / 2 * 128];
+    __shared__ __align__(1024) unsigned char wa0[BN / 2 * 128], wa1[BN / 2 * 128], wb0[BN / 2 * 128], wb1[BN / 2 * 128];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = lane & 15, g = lane >> 4;
+    const int wr = wave >> 2, wc = wave & 3;
+
+    const int mn = tiles_m * tiles_n, total = mn * splits;
+    const int xcd = blockIdx.x % GM_XCDS, local = blockIdx.x / GM_XCDS;
+    int id = xcd * (total / GM_XCDS) + min(xcd, total % GM_XCDS) + local;
+    const int sp = id / mn;
+    id -= sp * mn;
+    const int band = id / (GM_BAND * tiles_n), in = id - band * GM_BAND * tiles_n, high = min(GM_BAND, tiles_m - band * GM_BAND);
+    const int tm = band * GM_BAND + in % high, n0 = in / high * BN;
+    int m0 = tm * BM;
+    if (EPI == GM_GROUPED) {                             // the tile's rows end where its matrix's rows end
+        if (tm >= grp.n_tiles[0]) return;
+        const int* tl = grp.tiles + 3 * tm;
+        W += (size_t)tl[0] * grp.w_stride;
+        m0 = tl[1];
+        M = tl[1] + tl[2];
+    }
+    const int k0 = sp * steps_per, steps = min(steps_per, K / GM_BK - k0);
+    const int rows = min(BM, M - m0), cols = min(BN, N - n0);
+    const __amdgpu_buffer_rsrc_t xbuf = bn_buffer(X + (size_t)m0 * ldx, ((rows - 1) * ldx + K) * 2);
+    const __amdgpu_buffer_rsrc_t wbuf = bn_buffer(W + (size_t)n0 * ldw, ((cols - 1) * ldw + K) * 2);
+    // load j of part p: rows 64 j + 8 wave + lane / 8 of the part, which holds WM / 2 rows of each group (WN / 2 of each column of waves);
+    // rows past the end are the last one again
+    unsigned xo[2][XL], wo[2][WL];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+#pragma unroll
+        for (int j = 0; j < XL; ++j) {
+            const int r = 64 * j + 8 * wave + (lane >> 3), R = r / (WM / 2) * WM + p * (WM / 2) + r % (WM / 2);
+            xo[p][j] = min(R, rows - 1) * ldx * 2 + (((lane & 7) ^ gm_swizzle(r & 15)) << 4);
         }
-    };
 #pragma unroll
-    for (int a = 0; a < NT; ++a) {
-        const int n = n0 + wn + a * 16 + 4 * g;
-#pragma unroll
-        for (int b = 0; b < MT; ++b) {
-            const int m = m0 + wm + b * 16 + i;
-            f32x4 v = acc[a][b];
-            if (GLU8) {
-                // rows 16t..16t+7 of W are gates, 16t+8..16t+15 the ups of the same result columns:
-                // lanes with g >= 2 hold the ups of what lanes g - 2 hold the gates of
-                f32x4 up;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(v[r], 32, BN_WAVE);
-                if (g < 2 && m < M) {
-                    const int f = ((n0 + wn + a * 16) >> 1) + 4 * g;      // result column of v[0]
-#pragma unroll
-                    // silu(g) * u with the hardware's exp2 and reciprocal (an ulp each, far below the result's
-                    // rounding): expf and a division cost 25 vector instructions a value, a tenth of this kernel's time
-                    for (int r = 0; r < 4; ++r)
-                        v[r] = (act == BN_ACT_SILU ? v[r] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * v[r]))
-                                                   : bn_gate_act(v[r], act)) * up[r];
-                    store4(Y + (size_t)m * ldy + f, v, (N >> 1) - f);
-                }
-            } else if (m < M) {
-                if (grp.unary >= 0) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = bn_unary_act(v[r], grp.unary);
-                }
-                if (grp.row_scale) v *= grp.row_scale[m];
-                const size_t mo = grp.row_map ? (size_t)grp.row_map[m] : (size_t)m;
-                store4(Y + mo * ldy + n, v, N - n);
-            }
+        for (int j = 0; j < WL; ++j) {
+            const int r = 64 * j + 8 * wave + (lane >> 3), R = r / (WN / 2) * WN + p * (WN / 2) + r % (WN / 2);
+            wo[p][j] = min(R, cols - 1) * ldw * 2 + (((lane & 7) ^ gm_swizzle(r & 15)) << 4);
         }
     }
+    // a step past the last is the last one again: read by nobody
+    auto load_x = [&](unsigned char* to, int p, int s) {
+#pragma unroll
+        for (int j = 0; j < XL; ++j)
+            if (XP == 0 || j < XL - 1 || wave < XP) bn_load_to_lds(xbuf, to + (8 * j + wave) * 1024, xo[p][j], (k0 + min(s, steps - 1)) * (GM_BK * 2));
+    };
+    auto load_w = [&](unsigned char* to, int p, int s) {
+#pragma unroll
+        for (int j = 0; j < WL; ++j) bn_load_to_lds(wbuf, to + (8 * j + wave) * 1024, wo[p][j], (k0 + min(s, steps - 1)) * (GM_BK * 2));
+    };
+    const int c0 = (g ^ gm_swizzle(i)) << 4, c1 = ((4 + g) ^ gm_swizzle(i)) << 4;
+    bf16x8 xf[MH][2], w0[NH][2], w1[NH][2];
+    auto read_x = [&](const unsigned char* from) {
+        const unsigned char* b = from + (wr * (WM / 2) + i) * 128;
+#pragma unroll
+        for (int a = 0; a < MH; ++a) {
+            xf[a][0] = *reinterpret_cast<const bf16x8*>(b + a * 2048 + c0);
+            xf[a][1] = *reinterpret_cast<const bf16x8*>(b + a * 2048 + c1);
+        }
+    };
+    auto read_w = [&](const unsigned char* from, bf16x8 (&w)[NH][2]) {
+        const unsigned char* b = from + (wc * (WN / 2) + i) * 128;
+#pragma unroll
+        for (int a = 0; a < NH; ++a) {
+            w[a][0] = *reinterpret_cast<const bf16x8*>(b + a * 2048 + c0);
+            w[a][1] = *reinterpret_cast<const bf16x8*>(b + a * 2048 + c1);
+        }
+    };
+    f32x4 acc[2][2][NH][MH];                             // [part of X][part of W]
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+#pragma unroll
+            for (int a = 0; a < NH; ++a)
+#pragma unroll
+                for (int b = 0; b < MH; ++b) acc[u][v][a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](f32x4 (&c)[NH][MH], const bf16x8 (&w)[NH][2]) {
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int a = 0; a < NH; ++a)
+#pragma unroll
+                for (int b = 0; b < MH; ++b) c[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[a][kk], xf[b][kk], c[a][b], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+    };
+    // What the next turn reads has arrived when no more of this wave's loads are on their way than it has asked for since: in either
+    // turn X's two parts and W's two.  This turn's operands are in registers as well: their buffers may be asked for again.
+    auto arrived = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        if (XP == 0 || wave < XP) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * XL + 2 * WL) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * XL - 2 + 2 * WL) : "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto turn = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto step = [&](int s, unsigned char* x0, unsigned char* x1, unsigned char* v0, unsigned char* v1, unsigned char* other_x1) {
+        read_x(x0); read_w(v0, w0); read_w(v1, w1); load_x(other_x1, 1, s + 1);
+        arrived(); multiply(acc[0][0], w0); multiply(acc[0][1], w1); turn();
+        read_x(x1); load_x(x0, 0, s + 2); load_w(v0, 0, s + 2); load_w(v1, 1, s + 2);
+        arrived(); multiply(acc[1][1], w1); multiply(acc[1][0], w0); turn();
+    };
+    load_x(xa0, 0, 0); load_w(wa0, 0, 0); load_w(wa1, 1, 0); load_x(xa1, 1, 0);
+    load_x(xb0, 0, 1); load_w(wb0, 0, 1); load_w(wb1, 1, 1);
+    arrived();
+    if (wr == 1) turn();
+    int s = 0;
+    for (; s + 1 < steps; s += 2) {
+        step(s, xa0, xa1, wa0, wa1, xb1);
+        step(s + 1, xb0, xb1, wb0, wb1, xa1);
+    }
+    if (s < steps) step(s, xa0, xa1, wa0, wa1, xb1);
+    if (wr == 0) turn();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // nothing is on its way into shared memory when the wave ends
+
+    // lane (i, g) of a 16 x 16 tile holds columns 4 g .. 4 g + 3 of row i; rows of Y are whole groups of four (the host has seen to it)
+    auto store = [&](TO* dst, const f32x4& v) {
+        if (sizeof(TO) == 4) {
+            *reinterpret_cast<f32x4*>(dst) = v;
+        } else {
+            uint2 p;
+            p.x = (uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[0])) | ((uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[1])) << 16);
+            p.y = (uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[2])) | ((uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(v[3])) << 16);
+            *reinterpret_cast<uint2*>(dst) = p;
+        }
+    };
+    if (EPI == GM_STORE) Y += (size_t)sp * M * ldy;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+#pragma unroll
+            for (int a = 0; a < NH; ++a)
+#pragma unroll
+                for (int b = 0; b < MH; ++b) {
+                    const int m = m0 + wr * WM + u * (WM / 2) + b * 16 + i, n = n0 + wc * WN + v * (WN / 2) + a * 16;
+                    f32x4 c = acc[u][v][a][b];
+                    if (EPI == GM_SILU || EPI == GM_GATED) {
+                        // rows n .. n + 7 of W are gates, n + 8 .. n + 15 the ups of the same columns: the lanes with g >= 2 hold the ups
+                        // of what the lanes with g - 2 hold the gates of.  silu with the hardware's exp2 and reciprocal (an ulp each)
+                        f32x4 up;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(c[r], 32, BN_WAVE);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            c[r] = (EPI == GM_SILU ? c[r] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * c[r])) : bn_gate_act(c[r], act)) * up[r];
+                        if (g < 2 && m < M && n < N) store(Y + (size_t)m * ldy + (n >> 1) + 4 * g, c);
+                    } else if (m < M && n + 4 * g < N) {
+                        size_t mo = m;
+                        if (EPI == GM_GROUPED) {
+                            if (grp.unary >= 0) {
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) c[r] = bn_unary_act(c[r], grp.unary);
+                            }
+                            if (grp.row_scale) c *= grp.row_scale[m];
+                            if (grp.row_map) mo = grp.row_map[m];
+                        }
+                        store(Y + mo * ldy + n + 4 * g, c);
+                    }
+                }
 }
 
 static GmGroups gm_no_groups() {
@@ -328,6 +534,77 @@ static int gm_compute_units() {
     return cus;
 }
 
+// Tiles of the form above and what a step of 64 takes, us: a tile alone on its CU, and two where shared memory leaves room for two (0:
+// it does not).  Fitted to 2,600 measurements of 14 matrices at 129 to 8,192 rows, which it meets within 8 % (rms): a round costs
+// GM_ROUND more (the first loads, the stores), and a step of a round that fills no CU would take GM_IDLE of it (power, memory).
+struct GmTile { int bm, bn; double one, two; };
+static const GmTile gm_tiles[] = {{256, 256, 1.46, 0.}, {192, 256, 1.17, 0.}, {128, 256, 0.92, 0.}, {256, 128, 0.91, 0.}, {192, 128, 0.74, 1.38}, {128, 128, 0.61, 1.06}};
+#define GM_TILES 6
+#define GM_ROUND 7.3
+#define GM_IDLE 0.68
+#define GM_MAX_SPLITS 6
+
+static double gm_cost(const GmTile& t, long long tiles, int steps, int cus) {
+    auto round = [&](double step, double fill) { return GM_ROUND + steps * step * (GM_IDLE + (1. - GM_IDLE) * fill); };
+    if (t.two > 0.) {                                    // two a CU run on without rounds
+        if (tiles <= cus) return round(t.one, (double)tiles / cus);
+        if (tiles <= 2 * cus) return round(t.two, tiles / (2. * cus));
+        return 2 * GM_ROUND + steps * t.two * tiles / (2. * cus);
+    }
+    return tiles / cus * round(t.one, 1.) + (tiles % cus ? round(t.one, (double)(tiles % cus) / cus) : 0.);
+}
+
+// The tile and the ranges of K (up to max_splits) that take the least time for M rows, N rows of W and K columns; slabs are written and
+// read again at 5 TB/s, and more than two of them cost a launch.  bm: the only height to look at, or 0.
+static void gm_plan(int M, int N, int K, int bm, int max_splits, int* tile, int* splits) {
+    const int cus = gm_compute_units(), steps = K / GM_BK;
+    double best = -1.;
+    for (int i = 0; i < GM_TILES; ++i) {
+        const GmTile& t = gm_tiles[i];
+        if (bm && t.bm != bm) continue;
+        const long long tiles = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        for (int s = 1; s <= max_splits; ++s) {
+            const int per = (steps + s - 1) / s;
+            if ((steps + per - 1) / per != s) continue;
+            const double cost = gm_cost(t, tiles * s, per, cus) + (s > 1 ? s * 8e-6 * M * N / 5. + (s > 2 ? 4. : 0.) : 0.);
+            if (best < 0. || cost < best) { best = cost; *tile = i; *splits = s; }
+        }
+    }
+}
+
+// whole steps, 32-bit offsets inside a tile, results in whole groups of four
+static bool gm_turns_takes(int N, int K, int ldx, int ldw, int ldy, const void* Y, int size) {
+    return K % GM_BK == 0 && ldx <= 1 << 22 && ldw <= 1 << 22 && N % 4 == 0 && ldy % 4 == 0 && (uintptr_t)Y % (4 * size) == 0;
+}
+
+template <int BM, int BN, int EPI, typename TO>
+static int gm_turns_launch(const void* X, const void* W, void* Y, int M, int N, int K, int ldx, int ldw, int ldy, int splits, int act, hipStream_t s,
+                           const GmGroups& grp, int max_tiles) {
+    const int tiles_m = EPI == GM_GROUPED ? max_tiles : (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    const long long grid = (long long)tiles_m * tiles_n * splits;
+    if (grid > 0x7fffffffLL) return BN_ERR_ARG;
+    hipLaunchKernelGGL((gemm_turns_kernel<BM, BN, EPI, TO>), dim3((unsigned)grid), dim3(512), 0, s, (const bf16*)X, (const bf16*)W, (TO*)Y, M, N, K,
+                       ldx, ldw, ldy, tiles_m, tiles_n, splits, (K / GM_BK + splits - 1) / splits, act, grp);
+    return bn_launch_status();
+}
+
+template <int EPI, typename TO>
+static int gm_turns(int tile, const void* X, const void* W, void* Y, int M, int N, int K, int ldx, int ldw, int ldy, int splits, int act,
+                    hipStream_t s, const GmGroups& grp, int max_tiles = 0) {
+#define GM_TILE(I, BM_, BN_) \
+    if (tile == I) return gm_turns_launch<BM_, BN_, EPI, TO>(X, W, Y, M, N, K, ldx, ldw, ldy, splits, act, s, grp, max_tiles)
+    GM_TILE(0, 256, 256);
+    GM_TILE(3, 256, 128);
+    if constexpr (EPI != GM_GROUPED) {                   // grouped tiles are 256 rows
+        GM_TILE(1, 192, 256);
+        GM_TILE(2, 128, 256);
+        GM_TILE(4, 192, 128);
+        GM_TILE(5, 128, 128);
+    }
+#undef GM_TILE
+    return BN_ERR_ARG;
+}
+
 static int gm_pick_bn(int M, int N, int cus) {
     const int widths[3] = {256, 192, 128};
     const int weight[3] = {100, 104, 112};            // cost of a result column, relative
@@ -360,11 +637,20 @@ extern "C" int bn_gemm_mfma(int out_dtype, const void* X, const void* W, void* Y
         if (N % 8) return BN_ERR_ARG;
         N *= 2;                                       // rows of W
     }
+    const bool f32 = out_dtype == BN_DT_F32;
+    if (width != 192 && !(glu8 && f32) && gm_turns_takes(N, K, ldx, ldw, ldy, Y, f32 ? 4 : 2)) {
+        int tile = width == 256 ? 0 : 3, splits = 1;
+        if (!width) gm_plan(M, N, K, 0, 1, &tile, &splits);
+        const GmGroups none = gm_no_groups();
+        if (glu8 && act == BN_ACT_SILU) return gm_turns<GM_SILU, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, act, s, none);
+        if (glu8) return gm_turns<GM_GATED, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, act, s, none);
+        return f32 ? gm_turns<GM_STORE, float>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, 0, s, none)
+                   : gm_turns<GM_STORE, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, 0, s, none);
+    }
     // The tile width: the one with the least work on the busiest CU (rounds of workgroups over the
     // CUs times the width), a wider tile counting a little less than its width because it reads
     // less of X per result.
     const int bn = width ? width : gm_pick_bn(M, N, gm_compute_units());
-    const bool f32 = out_dtype == BN_DT_F32;
 #define GM_GO(BN_, GLU_)                                                                          \
     return f32 ? gm_launch<BN_, GLU_, float>(X, W, Y, M, N, K, ldx, ldw, ldy, act, s)             \
                : gm_launch<BN_, GLU_, bf16>(X, W, Y, M, N, K, ldx, ldw, ldy, act, s)
@@ -379,6 +665,23 @@ extern "C" int bn_gemm_mfma(int out_dtype, const void* X, const void* W, void* Y
 #undef GM_GO
 }
 
+// Ranges of K into which bn_gemm_mfma_slabs cuts a product (1 to GM_MAX_SPLITS).
+extern "C" int bn_gemm_mfma_splits(int M, int N, int K) {
+    if (M < 1 || N < 1 || K < GM_BK || K % GM_BK) return 0;
+    int tile = 0, splits = 1;
+    gm_plan(M, N, K, 0, GM_MAX_SPLITS, &tile, &splits);
+    return splits;
+}
+
+// Y [splits, M, N] (float32, contiguous): the sums of X . W^T over bn_gemm_mfma_splits(M, N, K) ranges of K; whole steps of K.
+extern "C" int bn_gemm_mfma_slabs(const void* X, const void* W, float* Y, int M, int N, int K, int ldx, int ldw, int splits, hipStream_t s) {
+    if (!bn_gemm_mfma_supports(M, N, K, ldx, ldw) || !gm_turns_takes(N, K, ldx, ldw, N, Y, 4) || (((uintptr_t)X | (uintptr_t)W) & 15)) return BN_ERR_ARG;
+    int tile = 0, plan = 1;
+    gm_plan(M, N, K, 0, GM_MAX_SPLITS, &tile, &plan);
+    if (plan != splits) return BN_ERR_ARG;
+    return gm_turns<GM_STORE, float>(tile, X, W, Y, M, N, K, ldx, ldw, N, splits, 0, s, gm_no_groups());
+}
+
 // The grouped form: X [rows, K] ordered by matrix, W [matrices][N, K] (w_stride elements apart), tiles [max_tiles][3] and
 // n_tiles [1] in device memory (tiles of at most 256 rows), Y row row_map[m] (or m) = unary(X[m] . W[matrix]^T) * row_scale[m].
 // rows: all rows of X (sizes the tile width).  out_dtype: type of Y.
@@ -391,13 +694,19 @@ extern "C" int bn_gemm_mfma_grouped(int out_dtype, const void* X, const void* W,
     GmGroups g;
     g.tiles = tiles; g.n_tiles = n_tiles; g.row_map = row_map; g.row_scale = row_scale; g.w_stride = w_stride;
     g.unary = unary < 0 ? -1 : unary;
-    const int bn = gm_pick_bn(rows, N, gm_compute_units());
     const bool f32 = out_dtype == BN_DT_F32;
-#define GM_GROUPED(BN_)                                                                                         \
+    if (gm_turns_takes(N, K, ldx, ldw, ldy, Y, f32 ? 4 : 2)) {
+        int tile = 0, splits = 1;
+        gm_plan(rows, N, K, GM_BM, 1, &tile, &splits);
+        return f32 ? gm_turns<GM_GROUPED, float>(tile, X, W, Y, rows, N, K, ldx, ldw, ldy, 1, 0, s, g, max_tiles)
+                   : gm_turns<GM_GROUPED, bf16>(tile, X, W, Y, rows, N, K, ldx, ldw, ldy, 1, 0, s, g, max_tiles);
+    }
+    const int bn = gm_pick_bn(rows, N, gm_compute_units());
+#define GM_GO_GROUPED(BN_)                                                                                         \
     return f32 ? gm_launch<BN_, false, float>(X, W, Y, rows, N, K, ldx, ldw, ldy, 0, s, g, max_tiles)          \
                : gm_launch<BN_, false, bf16>(X, W, Y, rows, N, K, ldx, ldw, ldy, 0, s, g, max_tiles)
-    if (bn == 256) { GM_GROUPED(256); }
-    if (bn == 192) { GM_GROUPED(192); }
-    GM_GROUPED(128);
-#undef GM_GROUPED
+    if (bn == 256) { GM_GO_GROUPED(256); }
+    if (bn == 192) { GM_GO_GROUPED(192); }
+    GM_GO_GROUPED(128);
+#undef GM_GO_GROUPED
 }

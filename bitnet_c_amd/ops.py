@@ -193,6 +193,8 @@ _SIGNATURES = {
         "bn_gemm_mfma_supports": [c_int, c_int, c_int, c_int, c_int],
         "bn_gemm_mfma": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                          c_int, c_void_p],
+        "bn_gemm_mfma_splits": [c_int, c_int, c_int],
+        "bn_gemm_mfma_slabs": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
         "bn_gemm_mfma_grouped": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_longlong,
                                  c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     },
@@ -556,6 +558,42 @@ def gemm_mfma_supported(M: int, N: int, K: int, ldx: int, ldw: int) -> bool:
     return M >= 1 and N >= 1 and K >= 8 and K % 8 == 0 and ldx % 8 == 0 and ldw % 8 == 0 and ldx >= K and ldw >= K
 
 
+GEMM_STEP = _build.header_constant("GM_BK", "gemm_mfma.hip")      # K in whole steps of this: the prompt product's faster form
+# Prompt products that are this library's own beside the library's: from this many rows on (fewer: the kernels of a decode step) ...
+PROMPT_ROWS = 129
+# ... a part's last product, as slabs over ranges of K where its tiles would leave half of the CUs without work and K is long enough for
+# the slabs' way through memory not to count.  us with the kernels of the next norm, the library's product -> slabs: 4,096 x 14,336 at 129 /
+# 256 / 576 / 1,024 / 2,048 rows 67 -> 46, 69 -> 57, 121 -> 79, 141 -> 118, 227 -> 195 (2,560: 252 -> 275); 5,120 x 13,824 at 512 / 1,536 (1,792)
+# 122 -> 84, 206 -> 181 (232 -> 255); 8,192 x 28,672 at 256 / 1,024 (1,280) 328 -> 157, 394 -> 361 (469 -> 507); 4,096 x 11,008 at 640 / 2,048
+# (2,560) 96 -> 87, 176 -> 160 (201 -> 220); 2,048 x 8,192 at 384 / 1,280 (2,048) 31 -> 29, 60 -> 54 (75 -> 78); 2,048 x 5,632 at 512 / 1,024
+# 26 -> 28, 40 -> 38: not worth it, 4,096 x 4,096 at 256 / 1,024 25 -> 29, 46 -> 52.
+SPLIT_ROWS_MIN_K = 8192
+
+
+def can_split_rows(M: int, N: int, K: int, dtype) -> bool:
+    """Whether a product of a prompt's rows whose result goes to the residual stream is left as slabs of sums (linear_split_rows)."""
+    if not (SPLIT_SUMS and dtype == torch.bfloat16 and M >= PROMPT_ROWS and K >= SPLIT_ROWS_MIN_K and K % GEMM_STEP == 0 and N % 4 == 0):
+        return False
+    tiles = -(-M // 256) * -(-N // 256)
+    return tiles * 2 <= _compute_units() and (K > SPLIT_ROWS_MIN_K or tiles * 16 <= 3 * _compute_units())
+
+
+def linear_split_rows(x: torch.Tensor, w: torch.Tensor) -> "PartialSums":
+    """x [M, K] . w[N, K]^T as float32 sums over ranges of K (bf16, K whole steps of GEMM_STEP), for the kernel of the next norm."""
+    require_gpu()
+    _dev(x, "x", torch.bfloat16, 2)
+    _dev(w, "w", torch.bfloat16, 2)
+    M, K = x.shape
+    N = w.shape[0]
+    if w.shape[1] != K or M < 1 or K % GEMM_STEP or N % 4 or (x.data_ptr() | w.data_ptr()) % 16:
+        raise KernelError(f"linear_split_rows: x {tuple(x.shape)} and w {tuple(w.shape)} do not agree, or K is not whole steps of {GEMM_STEP}")
+    S = _fn("gemm_mfma", "bn_gemm_mfma_splits")(M, N, K)
+    slabs = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
+    _check(_fn("gemm_mfma", "bn_gemm_mfma_slabs")(x.data_ptr(), w.data_ptr(), slabs.data_ptr(), M, N, K, _rows(x, "x"), _rows(w, "w"), S,
+                                                  _stream()), "gemm_mfma(slabs)")
+    return PartialSums(slabs)
+
+
 SK_CHUNK = _build.header_constant("SK_CHUNK", "skinny_gemm.hip")      # columns of K that a wave of the streaming kernels takes at a time
 SKINNY_ROWS = 16      # bf16 products with more rows than this go to the library
 
@@ -856,6 +894,14 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, interleaved: bool = 
         y = _staged_swiglu(x, w_gate_up, None, activation, streamed)
         if y is not None:
             return y
+    # A prompt's rows: this library's product with the gated unit in its epilogue.  us, the library's product and the unit's kernel -> this:
+    # 28,672 x 4,096 at 129 / 512 / 1,024 / 2,048 / 4,096 / 8,192 rows 75 -> 64, 107 -> 96, 204 -> 188, 376 -> 366, 730 -> 703, 1,404 -> 1,375;
+    # 27,648 x 5,120 at 512 / 2,048 / 8,192 150 -> 124, 507 -> 466, 1,950 -> 1,632; 57,344 x 8,192 at 512 / 640 / 4,096 374 -> 352, 541 -> 560,
+    # 2,632 -> 2,614; 16,384 x 3,072 at 512 / 4,096 60 -> 51, 323 -> 315; 11,264 x 2,048 at 129 / 512 / 2,048 / 8,192 31 -> 24, 37 -> 33, 98 -> 84,
+    # 411 -> 311; 5,632 x 1,024 at 512 / 2,048 18 -> 14, 43 -> 26.
+    if (x.dtype == torch.bfloat16 and interleaved and aligned and M >= PROMPT_ROWS and K % GEMM_STEP == 0
+            and gemm_mfma_supported(M, 2 * F, K, ldx, ldw)):
+        return gemm_mfma(x, w_gate_up, x.dtype, glu8=True, activation=activation)
     if (x.dtype == torch.bfloat16 and (M <= SKINNY_ROWS or (M <= 64 and not allow_library))
             and aligned and skinny_supported(M, F, K, ldx, ldw)):
         y = torch.empty((M, F), dtype=x.dtype, device=x.device)

@@ -81,6 +81,8 @@ class Linear:
             return LazyDelta(x, self)
         if plain and ops.can_split_sums(M, N, K, x.dtype) and x.stride(1) == 1 and x.stride(0) % 8 == 0:
             return ops.linear_partial_sums(x, self.weight, self.streamed)
+        if plain and ops.can_split_rows(M, N, K, x.dtype) and x.stride(1) == 1 and x.stride(0) % 8 == 0:
+            return ops.linear_split_rows(x, self.weight)
         if (self.bias is None and x.dim() == 2 and x.dtype == self.weight.dtype == torch.float32 and M > 0
                 and ops.can_norm_rows(M, N, x.dtype) and ops.f32_product_takes(self.weight)):
             return LazyDelta(x, self)

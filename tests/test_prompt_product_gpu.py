@@ -1,0 +1,91 @@
+"""The prompt product whose two groups of waves take turns at the matrix cores: whole results, gated units and slabs over ranges of K, at
+sizes that fill no tile and at which every tile is the one that is chosen."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _ops():
+    from bitnet_c_amd import ops
+    return ops
+
+
+def _data(M, N, K, pad=0):
+    g = torch.Generator(device="cuda").manual_seed(M * 31 + N * 7 + K)
+    x = torch.randn(M, K + pad, generator=g, device="cuda").to(torch.bfloat16)[:, :K]
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    return x, w, x.double() @ w.double().t()
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+# one step, two, an odd and an even number of them; rows and columns: one past a tile, one short of it, sixteen and four past
+SHAPES = [(1, 16, 64), (129, 208, 64), (129, 1040, 4096), (193, 4112, 192), (300, 528, 128), (511, 8208, 1088), (700, 8208, 448),
+          (1000, 12304, 320), (1025, 16400, 128), (385, 16400, 192), (570, 11216, 2048), (257, 4112, 64)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_products_and_gated_units(M, N, K):
+    ops = _ops()
+    x, w, ref = _data(M, N, K, 24)                   # rows that lie further apart than they are long
+    assert _rel(ops.gemm_mfma(x, w, torch.float32), ref) < 1e-5          # bf16 products are exact in float32: the sums' roundings
+    assert _rel(ops.gemm_mfma(x, w), ref) < 2.0 ** -8                    # one rounding to bf16
+    if N % 4 == 0:                                   # columns that end inside a tile of 16
+        assert _rel(ops.gemm_mfma(x, w[:N - 12], torch.float32), ref[:, :N - 12]) < 1e-5
+    v = ref.view(M, N // 16, 2, 8)
+    for act, fn in (("silu", torch.nn.functional.silu), ("relu2", lambda t: t.clamp(min=0) ** 2),
+                    ("gelu_tanh", lambda t: torch.nn.functional.gelu(t, approximate="tanh"))):
+        want = (fn(v[:, :, 0]) * v[:, :, 1]).reshape(M, N // 2)
+        got = ops.gemm_mfma(x, w, glu8=True, activation=act)
+        assert _rel(got, want) < 2.0 ** -8, act      # the unit is formed in float32 and rounded once
+        if M >= ops.PROMPT_ROWS:
+            assert torch.equal(ops.linear_swiglu(x, w, True, activation=act), got), act
+
+
+# slabs: two to six ranges of K, the last one shorter; every range summed alone
+@pytest.mark.parametrize("M,N,K", [(129, 264, 8256), (200, 4096, 8192), (257, 4104, 14336), (513, 1032, 4160), (1500, 2056, 8192),
+                                   (513, 4104, 14336), (900, 4100, 9024), (300, 520, 64), (130, 136, 8896)])
+def test_slabs(M, N, K):
+    ops = _ops()
+    x, w, ref = _data(M, N, K)
+    parts = ops.linear_split_rows(x, w)
+    S = parts.slabs.shape[0]
+    steps = -(-(K // 64) // S) * 64
+    assert 1 <= S <= 6 and (S - 1) * steps < K and _rel(parts.slabs.double().sum(0), ref) < 1e-5
+    for s in range(S):
+        a, b = s * steps, min(K, (s + 1) * steps)
+        assert _rel(parts.slabs[s], x[:, a:b].double() @ w[:, a:b].double().t()) < 1e-5, s
+    # into the stream, and normed
+    stream = torch.linspace(-1, 1, M * N, device="cuda").view(M, N).contiguous()
+    weight = torch.linspace(0.5, 1.5, N, device="cuda")
+    want = stream.double() + ref
+    h = ops.add_rmsnorm(stream, parts, weight, 1e-5, torch.bfloat16)
+    assert _rel(stream, want) < 1e-5
+    assert _rel(h, want / torch.sqrt((want * want).mean(1, keepdim=True) + 1e-5) * weight) < 2.0 ** -8
+
+
+def test_numbers_that_are_none():
+    """A row of X or of W that holds NaN or an infinity reaches its own results alone."""
+    ops = _ops()
+    M, N, K = 260, 528, 192
+    x, w, ref = _data(M, N, K)
+    x, w = x.clone(), w.clone()
+    x[255, 3], x[256, 191], w[17, 64] = float("nan"), float("inf"), float("nan")
+    y = ops.gemm_mfma(x, w, torch.float32)
+    bad = torch.zeros(M, N, dtype=torch.bool, device="cuda")
+    bad[255], bad[256], bad[:, 17] = True, True, True
+    assert not bool(y[bad].isfinite().any()) and _rel(y[~bad], ref[~bad]) < 1e-5
+
+
+def test_what_the_rules_say():
+    ops = _ops()
+    bf = torch.bfloat16
+    assert ops.can_split_rows(129, 4096, 14336, bf) and ops.can_split_rows(2048, 4096, 14336, bf)
+    assert not ops.can_split_rows(128, 4096, 14336, bf) and not ops.can_split_rows(2049, 4096, 14336, bf)
+    assert not ops.can_split_rows(548, 4096, 4096, bf) and not ops.can_split_rows(548, 4096, 14336 + 32, bf)
+    assert not ops.can_split_rows(548, 4096, 14336, torch.float32)
+    with pytest.raises(ops.KernelError):
+        ops.linear_split_rows(torch.zeros(130, 96, dtype=bf, device="cuda"), torch.zeros(64, 96, dtype=bf, device="cuda"))
