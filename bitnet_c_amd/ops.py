@@ -412,8 +412,11 @@ def add_rmsnorm(x: torch.Tensor, delta, weight: torch.Tensor, eps: float, out_dt
     out = torch.empty((n, D), dtype=out_dtype, device=x.device)
     if n == 0:
         return out
-    if parts is not None and rows is None and D % 4 == 0 and parts.slabs.shape[0] > 2 and T <= 65535:
-        # many slabs: the sum over the whole chip first, then the norm (one workgroup a row would pull all of its slabs alone)
+    if (parts is not None and rows is None and D % 4 == 0 and parts.slabs.shape[0] > 2 and T <= 65535
+            and (T < PROMPT_ROWS or (T < 512 and parts.slabs.shape[0] * D > ROW_SLABS))):
+        # many slabs: the sum over the whole chip first, then the norm (one workgroup a row would pull all of its slabs alone; a prompt's
+        # rows fill the chip by themselves unless their slabs are long: us, two kernels -> one, 4,096 wide, four slabs at 129 / 512 /
+        # 1,024 rows 6.9 -> 5.9, 12.7 -> 11.6, 21.6 -> 17.7; 8,192 wide, three at 256 12.1 -> 11.7, four 13.8 -> 15.9, at 512 21.7 -> 19.7)
         ssq = torch.empty((T, _fn("elementwise", "bn_add_rmsnorm_parts_pieces")(D)), dtype=torch.float32, device=x.device)
         _check(_fn("elementwise", "bn_add_rmsnorm_parts_wide")(_code(out_dtype), x.data_ptr(), parts.slabs.data_ptr(),
                                                                parts.slabs.shape[0], T, weight.data_ptr(), out.data_ptr(),
@@ -568,6 +571,7 @@ PROMPT_ROWS = 129
 # (2,560) 96 -> 87, 176 -> 160 (201 -> 220); 2,048 x 8,192 at 384 / 1,280 (2,048) 31 -> 29, 60 -> 54 (75 -> 78); 2,048 x 5,632 at 512 / 1,024
 # 26 -> 28, 40 -> 38: not worth it, 4,096 x 4,096 at 256 / 1,024 25 -> 29, 46 -> 52.
 SPLIT_ROWS_MIN_K = 8192
+ROW_SLABS = 24576         # numbers of a row's slabs together that one workgroup of a prompt step adds up
 
 
 def can_split_rows(M: int, N: int, K: int, dtype) -> bool:
