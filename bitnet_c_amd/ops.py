@@ -2311,9 +2311,11 @@ def wkv_state_floats(H: int, dk: int, dv: int) -> int:
 # are never cut (a position's float32 bits do not depend on how its sequence came in), and the choice is made by the sizes of a
 # captured step (StepContext.sizes), which the first, eager step of a request and its replays share.  What pays for pieces is
 # the length of a walk, of which rows / seqs is what is known in both; what they cost grows with the whole step's state.
-# us walked / in pieces, bf16.  wkv, 32 heads of 64 x 64: one sequence of 128 tokens 52 / 60, 256 90 / 66, 2,048 625 / 195; two
-# of 256 91 / 92, 512 167 / 130, 2,048 626 / 357; four of 512 176 / 195, 2,048 651 / 689; 64 heads: one of 256 92 / 91, 512
-# 168 / 129, two of 512 177 / 220; 16 heads of 128 x 128: one of 256 94 / 106, 512 175 / 150, two of 512 183 / 250.  Min-GRU,
+# us walked / in pieces, bf16.  wkv a token at a time, 32 heads of 64 x 64: one sequence of 128 tokens 52 / 60, 256 90 / 66, 2,048 625 / 195;
+# two of 256 91 / 92, 512 167 / 130, 2,048 626 / 357; four of 512 176 / 195, 2,048 651 / 689.  Sixteen tokens at a time (heads of 33 to 128):
+# one sequence of 128 21 / 24, 256 39 / 25, 2,048 289 / 64; two of 256 42 / 34, 512 75 / 47, 2,048 290 / 106; four of 512 77 / 61, 1,024 149 / 99,
+# 2,048 294 / 183; 64 heads: two of 512 83 / 66, 2,048 315 / 193, four of 512 88 / 105, 2,048 318 / 369; 16 heads of 128 x 128: one of 256 73 / 40, two
+# of 2,048 564 / 162, four of 2,048 565 / 297: pieces up to four times the state from 1,024 tokens on.  Min-GRU,
 # 2,048 channels: one sequence of 128 tokens 21 / 23, 256 35 / 23, 2,048 237 / 44; four of 256 36 / 32, 512 65 / 44; eight
 # of 256 36 / 46, 512 67 / 66; 4,096 channels: four of 512 67 / 65, six 74 / 89.
 SCAN_PIECES_LENGTH = 256                  # the shortest walk; half of the shortest at which twice the state pays
@@ -2325,15 +2327,16 @@ WKV_PIECE = _build.header_constant("WKV_PIECE", "state_mixers.hip")
 GRU_PIECE = _build.header_constant("GRU_TC", "state_mixers.hip")
 
 
-def _in_pieces(dtype, sizes, state: int, unit: int, piece: int) -> bool:
+def _in_pieces(dtype, sizes, state: int, unit: int, piece: int, most: int = 2) -> bool:
     rows, seqs = sizes
-    return (dtype == torch.bfloat16 and seqs <= SCAN_PIECES_SEQS and seqs * state <= min(rows // seqs // SCAN_PIECES_LENGTH, 2) * unit
+    return (dtype == torch.bfloat16 and seqs <= SCAN_PIECES_SEQS and seqs * state <= min(rows // seqs // SCAN_PIECES_LENGTH, most) * unit
             and _pieces_of(rows, seqs, piece) * state * 4 <= SCAN_PIECES_BYTES)
 
 
 def wkv_in_pieces(dtype, sizes, H: int, dk: int, dv: int) -> bool:
     """Whether wkv_scan cuts a prompt step into pieces; sizes: StepContext.sizes, (token rows, sequences)."""
-    return _in_pieces(dtype, sizes, H * dk * dv, WKV_PIECES_STATE, WKV_PIECE)
+    blocks = 32 < dk <= 128 and dk % 4 == 0 and dv <= (64 if dk <= 64 else 128) and sizes[0] // sizes[1] >= 4 * SCAN_PIECES_LENGTH     # walked sixteen tokens at a time
+    return _in_pieces(dtype, sizes, H * dk * dv, WKV_PIECES_STATE, WKV_PIECE, 4 if blocks else 2)
 
 
 def mingru_in_pieces(dtype, sizes, W: int) -> bool:
