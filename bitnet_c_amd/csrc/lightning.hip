@@ -543,6 +543,385 @@ static int lc_dispatch(int dtype, LaArgs& a, int n_seqs, int n_rows, const int* 
     return bn_lightning_columns(n_seqs, a.H, a.dk, a.dv) == 32 ? lc_launch<2, 2>(a, n_seqs, s) : lc_launch<2, 1>(a, n_seqs, s);
 }
 
+// ---- blocks of 64 tokens, bf16 ----------------------------------------------------------------------------------------
+// The chunked form's sums (with the same powers of the decay) of a bf16 step without a rotation, cut differently: a workgroup owns (sequence or block of
+// 64 tokens, head, 64 NCT value columns), its waves 16 NCT columns each, whole: a wave's columns of S stay in registers, tile by tile in the order in
+// which a product leaves them, which is also the order in which Q S reads its right operand; v's columns are no one else's and come straight from memory,
+// silu taken on the way; q and k are staged with theirs once, and the scores A, ten tiles on and under the diagonal, are dealt to the waves
+// once for all the columns.
+//   LB_WALK     a sequence from block to block: S <- d^n S + the block's own sum
+//   LB_SUMS     every block's own sum from nothing, side by side; lightning_carry_kernel then leaves in its place what the block starts from
+//   LB_OUTPUTS  every block's outputs from there
+// The three give the bits of the walk: both form a block's sum from zero and add the decayed state to it in one operation.  (Unlike the chunked form,
+// which adds to the decayed state; float32 steps stay there.)
+// Bound by the matrix cores' float32 rate where a launch fills the chip (256 instructions of 32 cycles a wave for a block's sum, 416 for its outputs, at
+// 128 x 128 with 32 columns a wave; two workgroups a CU hide the staging), by a block's latency (12 us) in short walks.  us with the launches, chunked form with its
+// copy of q, k and v -> the faster of the two cuts, 16 heads of 128 x 128: one sequence of 64 tokens 18.8 -> 17.0, 256 43 -> 27, 2,048 262 -> 70; four of
+// 128 40 -> 30, 500 106 -> 68, of 1,100, 300, 600 and 333 205 -> 84, 2,048 420 -> 208; sixteen of 64 68 -> 28, 512 433 -> 153; 32 heads of 64 x 64: one of
+// 2,048 187 -> 53, sixteen of 512 303 -> 94; the chain 31 of 256 tokens 294 -> 158 and 174 -> 95.
+#define LB_C 64               // tokens of a block
+enum { LB_WALK = 0, LB_SUMS = 1, LB_OUTPUTS = 2 };
+
+struct LbArgs {
+    LaArgs a;
+    int n_tiles;              // (the block forms)
+    float* carry;             // [blocks][H][dv / (64 NCT)]: S's tiles of a workgroup, wave by wave, column tile, row tile, lane, four numbers
+};
+
+// block number `at` of the step's sequences cut into blocks, numbered through sequence after sequence; n = 0 behind the last one
+__device__ __forceinline__ LaRange lb_range(const int* tiles, int n_tiles, int at) {
+    LaRange r = {0, 0, 0, -1};
+    for (int i = 0; i < n_tiles; ++i) {
+        const int n = tiles[4 * i + 2], count = (max(n, 0) + LB_C - 1) / LB_C;
+        if (at < count) {
+            r = la_range(tiles, nullptr, i);
+            r.row0 += at * LB_C;
+            r.n = min(LB_C, n - at * LB_C);
+            return r;
+        }
+        at -= count;
+    }
+    return r;
+}
+
+// Read before the next branch: this compiler (ROCm 7.2) leaves out the wait between a matrix product and a read of its result that lies behind a branch.
+__device__ __forceinline__ void lb_settle(f32x4& x) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float v = x[e];
+        asm("" : "+v"(v));
+        x[e] = v;
+    }
+}
+
+// z / (1 + exp(-z)) for a z of eight bits: z times the upper sixteen bits of log2 e is exact, the rest of the exponent a factor near 1, the reciprocal
+// refined once.  Ten instructions for some 35 of the library's exponential and quotient, which were half of a block's time.
+__device__ __forceinline__ float lb_act(bf16 x, int silu) {
+    const float z = to_f32(x);
+    if (!silu) return z;
+    const float c = __builtin_amdgcn_fmed3f(z, -87.f, 87.f);
+    const float p = __builtin_amdgcn_exp2f(c * -1.44268799f);             // 0x3fb8aa00
+    const float d = 1.f + fmaf(p, c * -4.8884952e-6f, p);
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-d, r, 1.f), r, r);
+    return z * r;
+}
+
+// RT: row tiles of 16 key rows (the key width rounded up to 64 or 128); NCT: column tiles of 16 of a wave
+template <int RT, int NCT, int FORM>
+__global__ __launch_bounds__(LA_THREADS, 2) void lightning_block_kernel(LbArgs b) {
+    constexpr int DKP = 16 * RT, LDQ = DKP + 4, CB = 64 * NCT, NQ = LB_C * (DKP / 8) / LA_THREADS;
+    const LaArgs& a = b.a;
+    extern __shared__ __align__(16) float la_smem[];
+    float* K_s = la_smem;                                 // [LB_C][LDQ], rows from the block's tokens on zero
+    float* P_s = K_s + LB_C * LDQ;                        // [LC_POW]     decay^0 .. decay^LB_C
+    float* Q_s = P_s + LC_POW;                            // [LB_C][LDQ]  (not LB_SUMS)
+    float* A_s = Q_s + LB_C * LDQ;                        // [10][16][16] the tiles of the decayed scores
+    const LaRange sr = FORM == LB_WALK ? la_range(a.tiles, a.seq_lens, blockIdx.x) : lb_range(a.tiles, b.n_tiles, blockIdx.x);
+    if (sr.n <= 0 || sr.pos0 < 0) return;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / BN_WAVE), lane = tid % BN_WAVE, m = lane % 16, g = lane / 16;
+    const int head = blockIdx.y, c0 = blockIdx.z * CB + wave * 16 * NCT + m;       // the lane's first column
+    const bf16* x = reinterpret_cast<const bf16*>(a.x) + (size_t)sr.row0 * a.ld;
+    f32x4 S[NCT][RT];
+    float* sp = a.state + (size_t)a.slot_ids[sr.seq] * a.state_stride + (size_t)head * a.dk * a.dv;
+    f32x4* cp = reinterpret_cast<f32x4*>(b.carry) +
+                ((((size_t)blockIdx.x * a.H + head) * gridDim.z + blockIdx.z) * 4 + wave) * (NCT * RT * BN_WAVE) + lane;
+    if (FORM == LB_OUTPUTS) {
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+            for (int t = 0; t < RT; ++t) S[ct][t] = cp[(ct * RT + t) * BN_WAVE];
+    } else if (FORM == LB_WALK) {
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = 16 * t + 4 * g + r, c = c0 + 16 * ct;
+                    const float v = sp[(size_t)min(row, a.dk - 1) * a.dv + min(c, a.dv - 1)];
+                    S[ct][t][r] = sr.pos0 > 0 && row < a.dk && c < a.dv ? v : 0.f;
+                }
+    }
+    if (tid <= LB_C) P_s[tid] = (float)pow((double)a.decay[head], (double)tid);
+    struct __align__(16) Eight { bf16 e[8]; };
+    for (int t0 = 0; t0 < sr.n; t0 += LB_C) {
+        const int nt = min(LB_C, sr.n - t0);
+        // ---- the block's q, k and v: from places that exist, dropped behind its tokens and the head's width ----
+        Eight kq[NQ], qq[NQ];
+        bf16 vq[NCT][16];
+#pragma unroll
+        for (int it = 0; it < NQ; ++it) {
+            const int idx = tid + it * LA_THREADS, tt = idx / (DKP / 8), r = idx % (DKP / 8) * 8;
+            const bf16* row = x + (size_t)(t0 + min(tt, nt - 1)) * a.ld + (size_t)head * a.dk + (r < a.dk ? r : 0);
+            kq[it] = *reinterpret_cast<const Eight*>(row + a.k_col);
+            if (FORM != LB_SUMS) qq[it] = *reinterpret_cast<const Eight*>(row + a.q_col);
+        }
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {                // token 16 (j / 4) + 4 g + j % 4
+                const int tt = min(16 * (j / 4) + 4 * g + j % 4, nt - 1);
+                vq[ct][j] = x[(size_t)(t0 + tt) * a.ld + a.v_col + (size_t)head * a.dv + min(c0 + 16 * ct, a.dv - 1)];
+            }
+#pragma unroll
+        for (int it = 0; it < NQ; ++it) {
+            const int idx = tid + it * LA_THREADS, tt = idx / (DKP / 8), r = idx % (DKP / 8) * 8;
+            const bool live = tt < nt && r < a.dk;
+            f32x4 k4[2], q4[2];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float k = lb_act(kq[it].e[e], a.feed.silu) * a.feed.k_scale;
+                k4[e / 4][e % 4] = live ? k : 0.f;
+                if (FORM == LB_SUMS) continue;
+                const float q = lb_act(qq[it].e[e], a.feed.silu);
+                q4[e / 4][e % 4] = live ? q : 0.f;
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                *reinterpret_cast<f32x4*>(K_s + tt * LDQ + r + 4 * h) = k4[h];
+                if (FORM != LB_SUMS) *reinterpret_cast<f32x4*>(Q_s + tt * LDQ + r + 4 * h) = q4[h];
+            }
+        }
+        float v[NCT][16];
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const float z = lb_act(vq[ct][j], a.feed.silu);
+                v[ct][j] = 16 * (j / 4) + 4 * g + j % 4 < nt && c0 + 16 * ct < a.dv ? z : 0.f;
+            }
+        lc_barrier();
+        if (FORM != LB_SUMS) {
+            // ---- A = (Q K^T) with the decay, the ten tiles on and under the diagonal dealt to the waves ----
+#pragma unroll
+            for (int n = 0; n < 3; ++n) {
+                const int ti = wave + 4 * n;
+                if (ti >= 10) break;
+                const int ib = ti < 1 ? 0 : ti < 3 ? 1 : ti < 6 ? 2 : 3, jb = ti - ib * (ib + 1) / 2;
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                const float* qp = Q_s + (16 * ib + m) * LDQ + 4 * g;
+                const float* kp = K_s + (16 * jb + m) * LDQ + 4 * g;
+#pragma unroll
+                for (int u = 0; u < RT; ++u) {
+                    const f32x4 qa = *reinterpret_cast<const f32x4*>(qp + 16 * u), kb = *reinterpret_cast<const f32x4*>(kp + 16 * u);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc = LC_MFMA(qa[e], kb[e], acc);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int i = 16 * ib + 4 * g + r, j = 16 * jb + m;
+                    const float w = acc[r] * P_s[max(i - j, 0)];
+                    A_s[ti * 256 + (4 * g + r) * 16 + m] = i >= j ? w : 0.f;
+                }
+            }
+            // ---- Q S ----
+            f32x4 qs[4][NCT], av[4][NCT];
+#pragma unroll
+            for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+                for (int ct = 0; ct < NCT; ++ct) qs[ib][ct] = av[ib][ct] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                f32x4 qa[4];
+#pragma unroll
+                for (int ib = 0; ib < 4; ++ib) qa[ib] = *reinterpret_cast<const f32x4*>(Q_s + (16 * ib + m) * LDQ + 16 * t + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+                        for (int ct = 0; ct < NCT; ++ct) qs[ib][ct] = LC_MFMA(qa[ib][e], S[ct][t][e], qs[ib][ct]);
+            }
+            lc_barrier();
+            // ---- o = A V + d^(i+1) Q S; an infinity or a NaN among the values must not meet the zeros of the tokens before it ----
+            bool fine = true;
+#pragma unroll
+            for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) fine = fine && fabsf(v[ct][j]) < INFINITY;
+            const int keep = __all(fine) ? -1 : 0;
+            if (!keep) {
+#pragma unroll
+                for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+                    for (int s = 0; s < 16; ++s)
+#pragma unroll
+                        for (int ct = 0; ct < NCT; ++ct) {
+                            const float vs = __shfl(v[ct][4 * ib + s % 4], s / 4 * 16 + m);
+#pragma unroll
+                            for (int r = 0; r < 4; ++r)
+                                if (4 * g + r >= s) av[ib][ct][r] = fmaf(A_s[(ib * (ib + 1) / 2 + ib) * 256 + (4 * g + r) * 16 + s], vs, av[ib][ct][r]);
+                        }
+            }
+#pragma unroll
+            for (int jb = 0; jb < 4; ++jb) {
+                f32x4 a4[4];
+#pragma unroll
+                for (int ib = jb; ib < 4; ++ib) a4[ib] = *reinterpret_cast<const f32x4*>(A_s + (ib * (ib + 1) / 2 + jb) * 256 + m * 16 + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int ib = jb; ib < 4; ++ib)
+#pragma unroll
+                        for (int ct = 0; ct < NCT; ++ct) {
+                            const float vj = v[ct][4 * jb + e];
+                            av[ib][ct] = LC_MFMA(a4[ib][e], ib == jb ? __int_as_float(__float_as_int(vj) & keep) : vj, av[ib][ct]);
+                        }
+            }
+#pragma unroll
+            for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+                for (int ct = 0; ct < NCT; ++ct) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) av[ib][ct][r] += P_s[16 * ib + 4 * g + r + 1] * qs[ib][ct][r];
+                    lb_settle(av[ib][ct]);
+                }
+            float* o = a.o + (size_t)(sr.row0 + t0) * a.H * a.dv + (size_t)head * a.dv;
+#pragma unroll
+            for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+                for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int i = 16 * ib + 4 * g + r;
+                        if (i < nt && c0 + 16 * ct < a.dv) o[(size_t)i * a.H * a.dv + c0 + 16 * ct] = av[ib][ct][r];
+                    }
+        }
+        if (FORM != LB_OUTPUTS) {
+            // ---- the block's own sum K^T (d^(n-1-j) V) ----
+            const float whole = P_s[nt];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const float p = P_s[max(nt - 1 - (16 * (j / 4) + 4 * g + j % 4), 0)];
+#pragma unroll
+                for (int ct = 0; ct < NCT; ++ct) v[ct][j] *= p;
+            }
+#pragma unroll
+            for (int t = 0; t < RT; t += 4) {
+                f32x4 own[4][NCT];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int ct = 0; ct < NCT; ++ct) own[q][ct] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    const float* kp = K_s + (16 * (j / 4) + 4 * g + j % 4) * LDQ + 16 * t + m;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+#pragma unroll
+                        for (int ct = 0; ct < NCT; ++ct) own[q][ct] = LC_MFMA(kp[16 * q], v[ct][j], own[q][ct]);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int ct = 0; ct < NCT; ++ct) {
+                        lb_settle(own[q][ct]);
+                        if (FORM == LB_SUMS) cp[(ct * RT + t + q) * BN_WAVE] = own[q][ct];
+                        else
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) S[ct][t + q][r] = fmaf(whole, S[ct][t + q][r], own[q][ct][r]);
+                    }
+            }
+            if (FORM == LB_WALK) lc_barrier();            // every wave has read this block's q, k and scores
+        }
+    }
+    if (FORM == LB_WALK) {
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = 16 * t + 4 * g + r, c = c0 + 16 * ct;
+                    if (row < a.dk && c < a.dv) sp[(size_t)row * a.dv + c] = S[ct][t][r];
+                }
+    }
+}
+
+// A thread four rows of a column of a head's state: through the blocks of a sequence S <- d^n S + the block's sum, leaving what each block starts from in
+// its place and the last in the slot's state.  Four blocks' sums are asked for at once.
+template <int RT, int NCT>
+__global__ __launch_bounds__(256) void lightning_carry_kernel(LbArgs b, int cuts) {
+    __shared__ float d_s[2];
+    const LaArgs& a = b.a;
+    const LaRange sr = la_range(a.tiles, nullptr, blockIdx.y);
+    if (sr.n <= 0 || sr.pos0 < 0) return;
+    constexpr int WAVE = NCT * RT * BN_WAVE, CUT = 4 * WAVE;       // a wave's, a workgroup's groups of four (a multiple of 256)
+    const int e = blockIdx.x * 256 + threadIdx.x, head = e / (CUT * cuts), at = e % (CUT * cuts);
+    const int blocks = (sr.n + LB_C - 1) / LB_C;
+    if (threadIdx.x < 2) d_s[threadIdx.x] = (float)pow((double)a.decay[head], (double)(threadIdx.x ? sr.n - (blocks - 1) * LB_C : LB_C));
+    const int lane = at % BN_WAVE, row = 16 * (at / BN_WAVE % RT) + 4 * (lane / 16);
+    const int c = at / CUT * 64 * NCT + at % CUT / WAVE * 16 * NCT + at / (RT * BN_WAVE) % NCT * 16 + lane % 16;
+    float* sp = a.state + (size_t)a.slot_ids[sr.seq] * a.state_stride + (size_t)head * a.dk * a.dv;
+    f32x4 S = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        if (sr.pos0 > 0 && row + r < a.dk && c < a.dv) S[r] = sp[(size_t)(row + r) * a.dv + c];
+    int before = 0;
+    for (int i = 0; i < (int)blockIdx.y; ++i) before += (max(a.tiles[4 * i + 2], 0) + LB_C - 1) / LB_C;
+    const size_t n = (size_t)a.H * CUT * cuts;
+    f32x4* cp = reinterpret_cast<f32x4*>(b.carry) + before * n + e;
+    __syncthreads();
+    const float full = d_s[0], rest = d_s[1];
+    for (int p0 = 0; p0 < blocks; p0 += 4) {
+        f32x4 own[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) own[q] = cp[min(p0 + q, blocks - 1) * n];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (p0 + q < blocks) {
+                cp[(p0 + q) * n] = S;
+                const float d = p0 + q + 1 < blocks ? full : rest;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) S[r] = fmaf(d, S[r], own[q][r]);
+            }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        if (row + r < a.dk && c < a.dv) sp[(size_t)(row + r) * a.dv + c] = S[r];
+}
+
+template <int RT, int NCT, int FORM>
+static int lb_launch(const LbArgs& b, int groups, int cuts, hipStream_t s) {
+    constexpr size_t one = sizeof(float) * (LB_C * (16 * RT + 4)), smem = one + sizeof(float) * LC_POW + (FORM == LB_SUMS ? 0 : one + sizeof(float) * 2560);
+    static bool raised = false;              // beyond the default limit of dynamic shared memory
+    if (smem > 64 * 1024 && !raised) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(lightning_block_kernel<RT, NCT, FORM>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return (int)e;
+        raised = true;
+    }
+    hipLaunchKernelGGL((lightning_block_kernel<RT, NCT, FORM>), dim3(groups, b.a.H, cuts), dim3(LA_THREADS), smem, s, b);
+    return bn_launch_status();
+}
+
+// blocks: 0, a workgroup walks a sequence; else what the step's sequences can be cut into together (rows of carry)
+template <int RT, int NCT>
+static int lb_go(const LbArgs& b, int blocks, hipStream_t s) {
+    const int cuts = (b.a.dv + 64 * NCT - 1) / (64 * NCT);
+    if (blocks == 0) return lb_launch<RT, NCT, LB_WALK>(b, b.n_tiles, cuts, s);
+    if (int rc = lb_launch<RT, NCT, LB_SUMS>(b, blocks, cuts, s)) return rc;
+    hipLaunchKernelGGL((lightning_carry_kernel<RT, NCT>), dim3(b.a.H * cuts * NCT * RT, b.n_tiles), dim3(256), 0, s, b, cuts);
+    if (int rc = bn_launch_status()) return rc;
+    return lb_launch<RT, NCT, LB_OUTPUTS>(b, blocks, cuts, s);
+}
+
+static int lb_dispatch(const LaArgs& a, int n_seqs, int blocks, float* carry, hipStream_t s) {
+    LbArgs b;
+    b.a = a; b.n_tiles = n_seqs; b.carry = carry;
+    // 32 columns a wave read q and k once for twice the columns where that still leaves a workgroup a CU, and in no walk, whose registers they overfill
+    // (one block of 128 x 128 29.4 us with 32, 17.2 with 16; four sequences of 500 in blocks 79 and 68 with the quicker silu)
+    const bool wide = a.dv > 64 && (long long)blocks * a.H * ((a.dv + 127) / 128) >= la_compute_units();
+    if (a.dk <= 64) return wide ? lb_go<4, 2>(b, blocks, s) : lb_go<4, 1>(b, blocks, s);
+    return wide ? lb_go<8, 2>(b, blocks, s) : lb_go<8, 1>(b, blocks, s);
+}
+
+// Whether bf16 rows of this layout take the blocks: groups of eight of q and k, heads up to LC_MAX_DIM rows, no rotation.
+extern "C" int bn_lightning_blocks_take(const void* x, int ld, int q_col, int k_col, int dk, int rope_dims) {
+    return (dk >= 8 && dk <= LC_MAX_DIM && dk % 8 == 0 && rope_dims == 0 && ((ld | q_col | k_col) & 7) == 0 && ((uintptr_t)x & 15) == 0) ? 1 : 0;
+}
+
 extern "C" int bn_lightning_supports(int dk, int dv) { return (dk >= 1 && dk <= LA_MAX_DIM && dv >= 1) ? 1 : 0; }
 
 // 1 when prompt steps of these sizes can take the chunked form
@@ -560,10 +939,13 @@ extern "C" int bn_lightning_prefers_chunks(int n_seqs, int H, int dk, int dv) {
 // dvs the widths rounded up to a multiple of 4; null: the chain form also where the chunked form would run
 // silu: 1, q, k and v pass a silu, 0, they come as projected; inv_freq [rope_dims / 2] or null: the rotation of q and k, whose
 // positions the chunked form takes from positions [n_rows]; k_scale multiplies k
+// blocks: -1, or the blocks of 64 tokens of a prompt step that bn_lightning_blocks_take() takes: 0, every sequence from block to block, else what the step's
+// sequences can be cut into together, with carry's blocks H (dk rounded up to 64 or 128) (dv rounded up to 64 or multiples of 128) floats
 extern "C" int bn_lightning_scan(int dtype, const void* x, int ld, int q_col, int k_col, int v_col, const float* decay, float* o,
                                  float* state, long long state_stride, const int* tiles, int n_seqs, const int* seq_lens,
                                  const int* slot_ids, int H, int dk, int dv, int n_rows, float* prepared, int silu,
-                                 const float* inv_freq, int rope_dims, const int* positions, float k_scale, hipStream_t s) {
+                                 const float* inv_freq, int rope_dims, const int* positions, float k_scale, int blocks, float* carry,
+                                 hipStream_t s) {
     if (inv_freq ? (rope_dims < 2 || rope_dims % 2 || rope_dims > dk) : rope_dims != 0) return BN_ERR_ARG;
     if (n_seqs <= 0 || H <= 0 || !bn_lightning_supports(dk, dv) || !x || !decay || !o || !state || !slot_ids) return BN_ERR_ARG;
     if ((!tiles && !seq_lens) || state_stride < (long long)H * dk * dv || q_col < 0 || k_col < 0 || v_col < 0) return BN_ERR_ARG;
@@ -574,6 +956,12 @@ extern "C" int bn_lightning_scan(int dtype, const void* x, int ld, int q_col, in
     a.H = H; a.dk = dk; a.dv = dv;
     a.feed.silu = silu ? 1 : 0; a.feed.rope_dims = rope_dims; a.feed.inv_freq = inv_freq; a.feed.k_scale = k_scale;
     if (dtype != BN_DT_F32 && dtype != BN_DT_BF16) return BN_ERR_DTYPE;
+    if (blocks >= 0) {
+        if (!tiles || dtype != BN_DT_BF16 || !bn_lightning_blocks_take(x, ld, q_col, k_col, dk, rope_dims) || n_seqs > 65535 ||
+            (blocks > 0 && (!carry || (uintptr_t)carry % 16 != 0)))
+            return BN_ERR_ARG;
+        return lb_dispatch(a, n_seqs, blocks, carry, s);
+    }
     if (tiles && prepared && bn_lightning_chunked(dk, dv)) {
         if (n_rows <= 0 || (uintptr_t)prepared % 16 != 0 || (inv_freq && !positions)) return BN_ERR_ARG;
         return lc_dispatch(dtype, a, n_seqs, n_rows, positions, prepared, s);

@@ -124,7 +124,8 @@ _SIGNATURES = {
         "bn_lightning_columns": [c_int, c_int, c_int, c_int],
         "bn_lightning_scan": [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p,
                               c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p,
-                              c_float, c_void_p],
+                              c_float, c_int, c_void_p, c_void_p],
+        "bn_lightning_blocks_take": [c_void_p, c_int, c_int, c_int, c_int, c_int],
         "bn_row_norm_gate": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_float, c_int, c_void_p],
     },
     "state_mixers": {
@@ -2508,10 +2509,29 @@ def lightning_chunked(dk: int, dv: int) -> bool:
     return bool(_fn("lightning", "bn_lightning_chunked")(int(dk), int(dv)))
 
 
+LIGHTNING_BLOCK = _build.header_constant("LB_C", "lightning.hip")
+
+
+def lightning_in_blocks(sizes, H: int, dk: int, dv: int) -> bool:
+    """Whether a prompt step (sizes: StepContext.sizes) that could take the blocks of 64 tokens should: where the chunked form would run, and where the chain
+    would from half a block a sequence on (us, chain / blocks, 16 heads of 128 x 128: sixteen sequences of 64 tokens 66 / 28; 31 of 256 294 / 158)."""
+    rows, seqs = sizes
+    return rows // seqs >= LIGHTNING_BLOCK // 2 or bool(_fn("lightning", "bn_lightning_prefers_chunks")(seqs, H, dk, dv))
+
+
+def lightning_in_pieces(T: int, n_seqs: int, H: int, dv: int) -> bool:
+    """Whether those blocks are formed side by side, the same bits: a walk's time is its length, side by side costs three launches and the traffic of a state a
+    block.  us one after the other / side by side, 16 heads of 128 x 128: one sequence of 64 tokens 17 / 25, 65 28 / 24, 256 52 / 27; four of 256 53 / 56,
+    500 101 / 68; sixteen of 512 153 / 206; 32 heads of 64 x 64: one of 128 17.8 / 19.5, 192 25 / 19; four of 256 33 / 38, 500 63 / 51; sixteen of
+    512 94 / 140."""
+    walks = n_seqs * H * -(-dv // 64)
+    return walks < 512 and T // n_seqs > 2 * walks
+
+
 def lightning_scan(x: torch.Tensor, q_col: int, k_col: int, v_col: int, decay: torch.Tensor, state: torch.Tensor, slot_ids,
                    H: int, dk: int, dv: int, *, tiles=None, seq_lens=None, chain: Optional[bool] = None, silu: bool = True,
                    inv_freq: Optional[torch.Tensor] = None, positions: Optional[torch.Tensor] = None,
-                   k_scale: float = 1.0) -> torch.Tensor:
+                   k_scale: float = 1.0, pieces: Optional[bool] = None, sizes=None) -> torch.Tensor:
     """Linear attention with a fixed decay per head over every sequence of a step; float32 [T, H dv].  x [T, >= ...] in
     the activations' type holds the projections side by side: queries at column q_col and keys at k_col (H dk wide),
     values at v_col (H dv wide); each passes silu in float32.  decay [H] float32.  state [slots, >= H dk dv] float32, the
@@ -2522,7 +2542,9 @@ def lightning_scan(x: torch.Tensor, q_col: int, k_col: int, v_col: int, decay: t
     chunks where they can be, None whichever is the faster for this many sequences and heads.
     silu False: q, k and v enter as projected.  inv_freq [n <= dk / 2] float32 (with positions [T] int32, the rows' positions
     once more): dimension i < n of every query and key head turns with dimension i + n by position * inv_freq[i].
-    k_scale multiplies the keys."""
+    k_scale multiplies the keys.
+    bf16 rows without a rotation and in groups of eight take blocks of 64 tokens in the chunks' place (lightning_in_blocks, for the step's sizes: T and the
+    number of sequences where they are None); pieces: whether side by side (True) or one after the other (False), the same bits; None: by their number."""
     require_gpu()
     _dev(x, "x", dims=2)
     _dev(decay, "decay", torch.float32, 1)
@@ -2548,8 +2570,16 @@ def lightning_scan(x: torch.Tensor, q_col: int, k_col: int, v_col: int, decay: t
             raise KernelError(f"lightning_scan: {rope_dims} rotated dimensions of {dk}, positions {tuple(positions.shape)} for {T} rows")
     o = torch.empty((T, H * dv), dtype=torch.float32, device=x.device)
     if T and n_seqs:
-        prepared = None
-        if tiles is not None and chain is not True and lightning_chunked(dk, dv) and (
+        prepared = carry = None
+        blocks = -1
+        if (tiles is not None and chain is not True and x.dtype == torch.bfloat16
+                and _fn("lightning", "bn_lightning_blocks_take")(x.data_ptr(), ld, int(q_col), int(k_col), dk, rope_dims)
+                and (chain is False or lightning_in_blocks(sizes or (T, n_seqs), H, dk, dv))):
+            state_floats = H * (64 if dk <= 64 else 128) * (64 if dv <= 64 else -(-dv // 128) * 128)
+            most = _pieces_of(T, n_seqs, LIGHTNING_BLOCK)
+            blocks = most if (pieces if pieces is not None else lightning_in_pieces(T, n_seqs, H, dv)) and most * state_floats * 4 <= SCAN_PIECES_BYTES else 0
+            carry = torch.empty(blocks * state_floats, dtype=torch.float32, device=x.device) if blocks else None
+        elif tiles is not None and chain is not True and lightning_chunked(dk, dv) and (
                 chain is False or _fn("lightning", "bn_lightning_prefers_chunks")(n_seqs, H, dk, dv)):
             # the chunked form's own copy of the step's q, k and v: what they pass applied, float32, head by head
             prepared = torch.empty(H * T * (2 * ((dk + 3) // 4 * 4) + (dv + 3) // 4 * 4), dtype=torch.float32, device=x.device)
@@ -2558,7 +2588,8 @@ def lightning_scan(x: torch.Tensor, q_col: int, k_col: int, v_col: int, decay: t
                                                      slot_ids.data_ptr(), H, dk, dv, T,
                                                      prepared.data_ptr() if prepared is not None else None, int(bool(silu)),
                                                      inv_freq.data_ptr() if rope_dims else None, rope_dims,
-                                                     positions.data_ptr() if rope_dims else None, float(k_scale), _stream()),
+                                                     positions.data_ptr() if rope_dims else None, float(k_scale), blocks,
+                                                     carry.data_ptr() if carry is not None else None, _stream()),
                "lightning_scan")
     return o
 

@@ -242,7 +242,7 @@ class Lightning(DecayedSums):
     def forward(self, h, ctx, kv):
         x = self.qkvg(h)
         o = ops.lightning_scan(x, 0, self.k_col, self.v_col, self.decay, kv.state, ctx.slot_ids, self.H, self.hs, self.vd,
-                               **_sequences(ctx))
+                               sizes=ctx.sizes, **_sequences(ctx))
         return ops.linear_row_norm_gate(o, x[:, self.g_col:], self.norm, self.eps, self.gate_activation, self.o.weight, self.o.streamed)
 
 
@@ -270,7 +270,7 @@ class Retention(DecayedSums):
         x = self.qkvg(h)
         o = ops.lightning_scan(x, 0, self.k_col, self.v_col, self.decay, kv.state, ctx.slot_ids, self.H, self.hs, self.vd,
                                silu=False, inv_freq=self.inv_freq, positions=ctx.positions if self.rope_dims else None,
-                               k_scale=self.hs ** -0.5, **_sequences(ctx))
+                               k_scale=self.hs ** -0.5, sizes=ctx.sizes, **_sequences(ctx))
         y = ops.head_norm_gate(o, x[:, self.g_col:], None, self.H, self.vd, self.eps)
         return self.o(y)
 
