@@ -18,8 +18,9 @@
 // its values tile by tile in the lanes' order, so that the decode form loads an operand tile as 1 KB of
 // consecutive bytes and the prompt form fetches a stage as one run.
 //
-// Prompt form: a workgroup of 4 waves owns 64*NT columns = consecutive query tokens x GT heads;
-// the keys and values it walks are staged through shared memory once for all four waves.
+// Prompt form: four waves own 64*NT columns = consecutive query tokens x GT heads;
+// the keys and values they walk are staged through shared memory once for all four, or, where two groups of four take turns
+// (attn_mfma_turns_kernel, heads of 128), for all eight.
 // Decode form: the 16 columns are the heads of one kv group for the sequence's one new token;
 // 4 waves take 32-key blocks in turn and merge through shared memory; long contexts are
 // also split over gridDim.z and merged by attn_mfma_combine_kernel in a fixed order (two splits: one workgroup
@@ -461,6 +462,7 @@ __device__ __forceinline__ void block_weights_values(const f32x4 (&st)[NT][2], c
 // that a tile of late positions has to walk is NG times shorter; at the end the groups' partial
 // results (reference point, sum, accumulators) are merged through shared memory in group order.  NG is 2 for
 // launches of one round over the chip and 1 (with two workgroups a CU) for longer ones; the launch code says why.
+// (Heads of 128 take this form, with NG = 1, for many short sequences alone.)
 //
 // A causal tile's work grows with its position, and a launch is as long as its longest workgroup.  A workgroup
 // therefore takes two tiles, 2p and 2p + 1 of the list, and the host orders the list so that these are a long and
@@ -694,6 +696,403 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2, 2))
         }
     }
     __syncthreads();                                      // the staging memory is free for the next tile
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// prompt form, long walks: two groups of waves take turns
+// ---------------------------------------------------------------------------------------
+// The weights of a block of 32 keys, as in block_weights_values_m: mask, reference point, exponentials; the rescaling of what has been summed.
+template <int HS, int NT, typename READS>
+__device__ __forceinline__ void turn_weights(f32x4 (&st)[NT][2], int kb, f32x4 (&acc)[NT][HS / 16], float (&m)[NT], float (&l)[NT],
+                                             const int (&qpos)[NT], const int (&lo)[NT], int key_hi, bool need_mask, float scale2, int g, bf16x8 (&pb)[NT],
+                                             READS reads) {
+    float s[NT][8];
+    if (need_mask) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const int from = lo[nt] - kb - 8 * g, to = min(qpos[nt] + 1, key_hi) - kb - 8 * g;       // of the lane's eight keys
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                float v = st[nt][e / 4][e % 4];
+                v = e < from ? -INFINITY : v;
+                v = e >= to ? -INFINITY : v;
+                st[nt][e / 4][e % 4] = v;
+            }
+        }
+    }
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[nt][e] = st[nt][e / 4][e % 4];
+    float mx[NT];
+    bool above = false;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        mx[nt] = max3(s[nt][0], s[nt][1], s[nt][2]);
+        mx[nt] = max3(mx[nt], s[nt][3], s[nt][4]);
+        mx[nt] = max3(mx[nt], s[nt][5], s[nt][6]);
+        mx[nt] = max3(mx[nt], s[nt][7], s[nt][7]) * scale2;
+        above = above || mx[nt] > m[nt] + 8.0f;
+    }
+    if (__any(above)) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            mx[nt] = max_over_lane_groups(mx[nt]);
+            const bool moved = mx[nt] > m[nt] + 8.0f;
+            const float alpha = moved ? (m[nt] != -INFINITY ? __builtin_amdgcn_exp2f(m[nt] - mx[nt]) : 0.f) : 1.f;
+            if (moved) m[nt] = mx[nt];
+            l[nt] *= alpha;
+#pragma unroll
+            for (int t = 0; t < HS / 16; ++t) acc[nt][t] *= alpha;
+        }
+    }
+    // the next slot's reads between the exponentials: shared memory takes one in some thirty cycles from the four waves of a group
+    __builtin_amdgcn_sched_barrier(0);
+    reads();
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const float ref = m[nt] == -INFINITY ? 0.f : m[nt];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[nt][e] = __builtin_amdgcn_exp2f(fmaf(s[nt][e], scale2, -ref));
+        pb[nt] = pack8(s[nt]);
+    }
+#pragma unroll
+    for (int r = 0; r < 12; ++r) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x402, 4, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// Eight waves, two a SIMD, in two groups of four.  A group's block of 32 keys is two turns, the products (scores of its next block, weights times values of this
+// one, from registers alone) and the vector work (the next block's weights, and between its exponentials the reads of the operands after that),
+// with a barrier behind each; the groups are one turn apart, so that of the two waves of a SIMD one has the matrix cores while the other
+// has the vector unit.  (Left alone the two often want the same one, and wait for operands in front of their products.)
+// SPLIT: both groups hold a tile's query columns and share its keys, of every 64 the first group the first 32, the other the rest; at the end
+// their partial results (reference point, sum, accumulators) are merged through shared memory, each group merging one of two column tiles.  Else a
+// group holds a tile of its own and both walk all the keys that either needs, which are fetched once for both: a workgroup takes two
+// neighbouring pairs of the list that belong to one sequence, first their long tiles together, then their short ones, or, of the last of an odd
+// number of pairs, its two tiles, which are the middle ones (two pairs of a sequence follow each other in the list, see ops.pair_tiles;
+// tiles in another order are taken two by two just the same, and those of a pair of two sequences one by one).
+// A block's keys and values go from the pages straight to shared memory, in the pages' own order, which is the operands': a wave fetches pieces of
+// 1 KB, three turns or more before they are read.  Ring slot u holds block u's values and block u + 1's keys, which are used together.
+// Blocks that every column sees whole run in a loop without a comparison.
+// What bounds a step (two blocks, 8 products of 16 x 16 x 128 or so a wave and block: 34 matrix instructions of 16 cycles, some 75 vector instructions): 2,240
+// cycles of 2 x (544 + 300), since a vector instruction delays its SIMD's matrix instructions (both read the same registers' ports); the two
+// barriers take 10 % of it. 4,096 tokens of 32 heads over 8, us: 179 before, 143; 8,100 tokens 640, 510 (0.84 and 1.05 PFLOP/s).  Tried: operands read in
+// the products' turn (8,100 tokens 607, from shared memory's latency); conditions instead of numbers for a block's kind (684: they are carried in
+// vector registers); variants of a turn with and without masks (798: their accumulators are copied where they meet).
+template <int HS, int NT, bool SPLIT>
+__global__ __launch_bounds__(512, 2) void attn_mfma_turns_kernel(MfmaArgs a, int n_tiles, int paired) {
+    constexpr int DC = HS / 32, DT = HS / 16, BLOCK = 32 * HS * 2, SLOT = 2 * BLOCK;
+    constexpr int RING = SPLIT ? 4 : 5, GROUPS = SPLIT ? 2 : 1;          // slots, and the groups that have slots of their own
+    constexpr int LOADS = 2 * GROUPS;                    // of a wave for a slot
+    static_assert(BLOCK == 8 * 1024 && NT == 2, "eight pieces of keys and of values; a column tile a group to merge");
+    static_assert(4 * 64 * DT * 4 * 4 <= 2 * SLOT, "a group's accumulators of a column tile fit a slot of both groups");
+    __shared__ __align__(1024) unsigned char r0[GROUPS * SLOT], r1[GROUPS * SLOT], r2[GROUPS * SLOT], r3[GROUPS * SLOT], r4[SPLIT ? 16 : SLOT];
+    __shared__ int on_simd[4];
+    const int lane = threadIdx.x & 63;
+    int wave, grp;                                        // the wave's number in its group, and its group
+    bn_turn_roles(on_simd, wave, grp);
+    const int own = SPLIT ? grp : 0, piece = SPLIT ? wave : 4 * grp + wave;         // among those that share a slot
+    const int n = lane & 15, g = lane >> 4;
+    const int G = a.H / a.Hkv, GT = a.GT;
+    const int n_head_tiles = (G + GT - 1) / GT;
+    const int hy = a.Hkv * n_head_tiles;
+    const int number = blockIdx.x / hy, y = blockIdx.x - number * hy;
+    const int kvh = y / n_head_tiles, ht = y - kvh * n_head_tiles;
+    const float scale2 = a.scale * LOG2E;
+    // the list's entries of either group in either turn; -1: none
+    int entry[2][2] = {{-1, -1}, {-1, -1}}, first_turn = 0;
+    if (SPLIT) {
+        entry[0][0] = entry[0][1] = paired ? 2 * number : number;
+        if (paired && 2 * number + 1 < n_tiles) entry[1][0] = entry[1][1] = 2 * number + 1;
+    } else {
+        // Every other pair of a sequence is taken along, and its workgroup leaves.  A tile without a partner comes first, then the even pairs, then the odd
+        // ones (with a turn a workgroup: all of this for the first turn, then for the second): workgroups go to the shader engines in turn, and those that had
+        // only leaving ones would stay idle (8,100 tokens in the list's order: 894 us, so 510).
+        const int pairs = n_tiles / 2, slots = (n_tiles + 1) / 2, at = number % slots - n_tiles % 2, even = (pairs + 1) / 2;
+        const int j = at < 0 ? pairs : at < even ? 2 * at : 2 * (at - even) + 1;
+        first_turn = number / slots;
+        auto of = [&](int p, int seq) { return a.tiles[8 * p] == seq && a.tiles[8 * p + 4] == seq && a.tiles[8 * p + 2] > 0 && a.tiles[8 * p + 6] > 0; };
+        const int seq = j < pairs ? a.tiles[8 * j] : 0;
+        if (j < pairs && of(j, seq)) {
+            int before = 0;                               // pairs of the sequence in front of this one
+            for (int p = j - 1 - lane;; p -= 64) {
+                const unsigned long long no = ~__ballot(p >= 0 && of(max(p, 0), seq));
+                if (no) { before += __builtin_ctzll(no); break; }
+                before += 64;
+            }
+            if (before & 1) return;                       // the pair in front of it takes it along
+            const bool two = j + 1 < pairs && of(j + 1, seq);
+            entry[0][0] = 2 * j;
+            entry[0][1] = two ? 2 * j + 2 : 2 * j + 1;
+            if (two) { entry[1][0] = 2 * j + 1; entry[1][1] = 2 * j + 3; }
+        } else {
+            entry[0][0] = 2 * j;
+            if (2 * j + 1 < n_tiles) entry[1][0] = 2 * j + 1;
+        }
+    }
+  for (int turn = first_turn; turn <= (paired ? 1 : first_turn); ++turn) {
+    const int e0 = turn ? entry[1][0] : entry[0][0], e1 = turn ? entry[1][1] : entry[0][1];
+    if (e0 < 0) break;
+    const int* t0 = a.tiles + 4 * e0;
+    const int* t1 = a.tiles + 4 * max(e1, 0);
+    const int n0 = max(t0[2], 0), n1 = e1 < 0 ? 0 : max(t1[2], 0), pos_0 = t0[3], pos_1 = t1[3];
+    if (n0 + n1 == 0) continue;                           // empty tiles (a list padded to a fixed length): the whole workgroup skips them
+    const int seq = t0[0], tok0 = grp ? t1[1] : t0[1], n_tok = grp ? n1 : n0, pos0 = grp ? pos_1 : pos_0;
+    // the positions that the workgroup's tiles begin and end at
+    const int pos_first = n0 == 0 ? pos_1 : n1 == 0 ? pos_0 : min(pos_0, pos_1);
+    const int pos_last = max(n0 ? pos_0 + n0 - 1 : 0, n1 ? pos_1 + n1 - 1 : 0);
+
+    bf16x8 q[NT][DC];
+    int qpos[NT], lo[NT];
+    int w_hi = -1, w_lo = 0x7fffffff, all_hi = 0x7fffffff, all_lo = 0;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int c = (wave * NT + nt) * 16 + n;
+        const int ti = c / GT, hg = ht * GT + (c - ti * GT);
+        const bool ok = ti < n_tok && hg < G;
+        qpos[nt] = ok ? pos0 + ti : -1;
+        lo[nt] = (ok && a.window > 0) ? max(0, qpos[nt] + 1 - a.window) : 0;
+#pragma unroll
+        for (int c2 = 0; c2 < DC; ++c2) {
+            uint4 z = make_uint4(0, 0, 0, 0);
+            if (ok) z = *reinterpret_cast<const uint4*>(a.q + (size_t)(tok0 + ti) * a.q_stride + (size_t)(kvh * G + hg) * HS + c2 * 32 + g * 8);
+            q[nt][c2] = __builtin_bit_cast(bf16x8, z);
+        }
+        if (ok) { w_hi = max(w_hi, qpos[nt]); w_lo = min(w_lo, lo[nt]); all_hi = min(all_hi, qpos[nt]); all_lo = max(all_lo, lo[nt]); }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        w_hi = max(w_hi, __shfl_xor(w_hi, o, BN_WAVE));
+        w_lo = min(w_lo, __shfl_xor(w_lo, o, BN_WAVE));
+        all_hi = min(all_hi, __shfl_xor(all_hi, o, BN_WAVE));
+        all_lo = max(all_lo, __shfl_xor(all_lo, o, BN_WAVE));
+    }
+    w_hi = __builtin_amdgcn_readfirstlane(w_hi); w_lo = __builtin_amdgcn_readfirstlane(w_lo);
+    all_hi = __builtin_amdgcn_readfirstlane(all_hi); all_lo = __builtin_amdgcn_readfirstlane(all_lo);
+    f32x4 acc[NT][DT];
+    float m[NT], l[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        m[nt] = -INFINITY; l[nt] = 0.f;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) acc[nt][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+    // The workgroup's steps: the same in every wave.  The group's block of step u starts at key first_key + STEP u.
+    constexpr int STEP = 32 * GROUPS;
+    static_assert(BN_PAGE == 64, "a page is two blocks");
+    const int g_lo = a.window > 0 ? max(0, pos_first + 1 - a.window) : 0;
+    const int step0 = g_lo / STEP, steps = pos_last / STEP - step0 + 1, last = steps - 1, first_key = step0 * STEP + 32 * own;
+    // of its blocks, the ones that some column of the wave sees (first_u .. last_u), the ones whose keys do not all exist for it (from edge_u on) and the ones
+    // that some of its columns sees only in part (from part_u on, and below whole_u); numbers, not conditions: every test is a scalar comparison
+    auto from = [&](int key) { return key < first_key ? 0 : (key - first_key) / STEP + 1; };           // the first block that starts behind a key
+    const int first_u = w_hi < 0 ? steps : from(w_lo - 32), last_u = min(last, from(w_hi) - 1);
+    const int edge_u = from(w_hi - 31), part_u = from(all_hi - 31), whole_u = from(all_lo - 1);
+    const size_t page_bytes = (size_t)a.Hkv * BN_PAGE * HS * 2, head_bytes = (size_t)kvh * BN_PAGE * HS * 2;
+    const unsigned char* k_pool = reinterpret_cast<const unsigned char*>(a.k_pages) + head_bytes;
+    const unsigned char* v_pool = reinterpret_cast<const unsigned char*>(a.vt_pages) + head_bytes;
+    const int* table = a.block_table + (size_t)seq * a.bt_stride;
+    auto page_of = [&](int u) { return uniform_load(table, (unsigned)(step0 + min(u, last)) / (BN_PAGE / STEP)); };    // a step past the last is the last again: read by nobody
+    const unsigned mine = (piece * 64 + lane) * 16;
+    auto fetch = [&](const unsigned char* page, int u, unsigned char* to) {
+        const __amdgpu_buffer_rsrc_t b = bn_buffer(page, BN_PAGE * HS * 2);
+        const unsigned half = (SPLIT ? grp : (step0 + min(u, last)) & 1) * BLOCK;
+        bn_load_to_lds(b, to + piece * 1024, mine, half);
+        if (SPLIT) bn_load_to_lds(b, to + (piece + 4) * 1024, mine, half + 4096);
+    };
+    bf16x8 kf[DC][2], vf[DT], pb[NT];
+    f32x4 st[NT][2];
+    const int at = own * SLOT + lane * 16;
+    auto read_keys = [&](const unsigned char* from, int c0, int c1) {
+#pragma unroll
+        for (int c = c0; c < c1; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) kf[c][h] = *reinterpret_cast<const bf16x8*>(from + at + BLOCK + (2 * c + h) * 1024);
+    };
+    auto read_values = [&](const unsigned char* from) {
+#pragma unroll
+        for (int t = 0; t < DT; ++t) vf[t] = *reinterpret_cast<const bf16x8*>(from + at + t * 1024);
+    };
+    auto scores = [&]() {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) st[nt][0] = st[nt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < DC; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) st[nt][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[c][h], q[nt][c], st[nt][h], 0, 0, 0);
+    };
+    auto values = [&](int u, auto edges) {
+        if (decltype(edges)::value && u >= edge_u) {      // keys that do not exist may hold anything, NaN included (0 * NaN is NaN)
+            const int left = w_hi + 1 - (first_key + STEP * u + 8 * g);        // of the lane's eight keys
+            uint32_t there[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) there[e] = left > 2 * e + 1 ? ~0u : left > 2 * e ? 0xffffu : 0u;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+                uint4 x = __builtin_bit_cast(uint4, vf[t]);
+                x.x &= there[0]; x.y &= there[1]; x.z &= there[2]; x.w &= there[3];
+                vf[t] = __builtin_bit_cast(bf16x8, x);
+            }
+        }
+        f32x4 lsum[NT];
+        const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) lsum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[nt], (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) acc[nt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], pb[nt], acc[nt][t], 0, 0, 0);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) l[nt] += lsum[nt][0];
+    };
+    auto weights = [&](int u, auto edges, auto reads) {
+        if (decltype(edges)::value && (u < first_u || u > last_u)) return;
+        turn_weights<HS, NT>(st, first_key + STEP * u, acc, m, l, qpos, lo, w_hi + 1, decltype(edges)::value && (u >= part_u || u < whole_u), scale2, g, pb, reads);
+    };
+    // a turn's end; behind the products LEFT of this wave's loads may still be on their way: the slot that is read next has arrived
+    auto end = [&](auto left) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (decltype(left)::value >= 0) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(decltype(left)::value < 0 ? 0 : decltype(left)::value) : "memory");
+        else asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    using std::integral_constant;
+    size_t v_at = page_of(0) * page_bytes;                // of the step whose values are asked for next
+    int page_k = page_of(1);                              // of the next step's keys
+    auto fill = [&](int u, unsigned char* to) {
+        const size_t k_at = page_k * page_bytes;
+        fetch(v_pool + v_at, u, to + own * SLOT);
+        fetch(k_pool + k_at, u + 1, to + own * SLOT + BLOCK);
+        v_at = k_at;
+    };
+    unsigned char* const r_last = SPLIT ? r3 : r4;
+    fetch(k_pool + v_at, 0, r_last + own * SLOT + BLOCK);
+    fill(0, r0); page_k = page_of(2);
+    fill(1, r1); page_k = page_of(3);
+    fill(2, r2); page_k = page_of(4);
+    if (!SPLIT) { fill(3, r3); page_k = page_of(5); }
+    constexpr int AHEAD = RING - 1;                       // slots that are asked for at the start, and then one a step
+    end(integral_constant<int, AHEAD * LOADS>());         // the first keys
+    if (grp == 1) end(integral_constant<int, (AHEAD - 1) * LOADS>());        // one turn behind
+    read_keys(r_last, 0, DC);
+    __builtin_amdgcn_s_setprio(1);
+    if (first_u <= 0) scores();
+    __builtin_amdgcn_s_setprio(0);
+    end(integral_constant<int, (AHEAD - 1) * LOADS>());
+    read_keys(r0, 0, DC);
+    read_values(r0);
+    weights(0, std::true_type(), [] {});
+    end(integral_constant<int, (AHEAD - 2) * LOADS>());
+    // Slot u's turns.  The vector turn reads slot u + 1 and asks for slot u + AHEAD in the place of slot u - 1, whose operands the last products of either group have
+    // used up.  Slot u + 1 has arrived: at the barrier in front of that turn a wave that shares it has asked for slots up to u + AHEAD - 1 and
+    // may still wait for AHEAD - 2 of them, whether it ends its products there or, one turn apart, its vector work.
+    auto step = [&](int u, unsigned char* free, const unsigned char* next, auto edges) {
+        __builtin_amdgcn_s_setprio(1);
+        if (!decltype(edges)::value || (u + 1 >= first_u && u < last_u)) scores();
+        if (!decltype(edges)::value || (u >= first_u && u <= last_u)) values(u, edges);
+        __builtin_amdgcn_s_setprio(0);
+        end(integral_constant<int, (AHEAD - 2) * LOADS>());
+        if (decltype(edges)::value) {
+            read_keys(next, 0, DC);
+            read_values(next);
+            fill(u + AHEAD, free);
+            weights(u + 1, edges, [] {});
+        } else {
+            read_keys(next, 0, 2);
+            fill(u + AHEAD, free);
+            weights(u + 1, edges, [&] { read_keys(next, 2, DC); read_values(next); });
+        }
+        page_k = page_of(u + AHEAD + 2);
+        end(integral_constant<int, (AHEAD - 2) * LOADS>());
+    };
+    // steps whose blocks, and the next step's, every column of the workgroup sees whole
+    const int clear = a.window > 0 ? 0 : (pos_first + 1) / STEP;
+    int u = 0;
+    if constexpr (SPLIT) {
+        for (; u + RING < clear; u += RING) {
+            step(u, r3, r1, std::false_type());
+            step(u + 1, r0, r2, std::false_type());
+            step(u + 2, r1, r3, std::false_type());
+            step(u + 3, r2, r0, std::false_type());
+        }
+        for (; u < steps; u += RING) {
+            step(u, r3, r1, std::true_type());
+            if (u + 1 >= steps) break;
+            step(u + 1, r0, r2, std::true_type());
+            if (u + 2 >= steps) break;
+            step(u + 2, r1, r3, std::true_type());
+            if (u + 3 >= steps) break;
+            step(u + 3, r2, r0, std::true_type());
+        }
+    } else {
+        for (; u + RING < clear; u += RING) {
+            step(u, r4, r1, std::false_type());
+            step(u + 1, r0, r2, std::false_type());
+            step(u + 2, r1, r3, std::false_type());
+            step(u + 3, r2, r4, std::false_type());
+            step(u + 4, r3, r0, std::false_type());
+        }
+        for (; u < steps; u += RING) {
+            step(u, r4, r1, std::true_type());
+            if (u + 1 >= steps) break;
+            step(u + 1, r0, r2, std::true_type());
+            if (u + 2 >= steps) break;
+            step(u + 2, r1, r3, std::true_type());
+            if (u + 3 >= steps) break;
+            step(u + 3, r2, r4, std::true_type());
+            if (u + 4 >= steps) break;
+            step(u + 4, r3, r0, std::true_type());
+        }
+    }
+    if (grp == 0) end(integral_constant<int, 0>());
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");       // nothing is on its way: the ring is free
+    auto store = [&](int nt, float inv, auto value) {
+        const int c = (wave * NT + nt) * 16 + n, ti = c / GT, hg = ht * GT + (c - ti * GT);
+        bf16* o = a.out + (size_t)(tok0 + ti) * a.out_stride + (size_t)(kvh * G + hg) * HS + 4 * g;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+            uint2 w;
+            w.x = pack2(value(t, 0) * inv, value(t, 1) * inv);
+            w.y = pack2(value(t, 2) * inv, value(t, 3) * inv);
+            *reinterpret_cast<uint2*>(o + t * 16) = w;
+        }
+    };
+    if constexpr (SPLIT) {                                // the first group finishes column tile 0, the other tile 1
+        float* given = reinterpret_cast<float*>(grp ? r1 : r0) + wave * DT * 4 * 64 + lane;
+        const float* got = reinterpret_cast<const float*>(grp ? r0 : r1) + wave * DT * 4 * 64 + lane;
+        float2* ml = reinterpret_cast<float2*>(r2) + wave * 64 + lane;           // [group][wave][lane]
+        auto give = [&](int nt) {
+            ml[grp * 256] = make_float2(m[nt], l[nt]);
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) given[(t * 4 + r) * 64] = acc[nt][t][r];
+        };
+        auto finish = [&](int nt) {
+            if (qpos[nt] < 0) return;
+            const float2 o2 = ml[(1 - grp) * 256];
+            const float m0 = grp ? o2.x : m[nt], m1 = grp ? m[nt] : o2.x, l0 = grp ? o2.y : l[nt], l1 = grp ? l[nt] : o2.y, M = fmaxf(m0, m1);
+            const float a0 = m0 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m0 - M), a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - M);
+            const float sum = l0 * a0 + l1 * a1;
+            store(nt, sum > 0.f ? 1.0f / sum : 0.f, [&](int t, int r) {
+                const float v = got[(t * 4 + r) * 64];
+                return (grp ? v : acc[nt][t][r]) * a0 + (grp ? acc[nt][t][r] : v) * a1;
+            });
+        };
+        if (grp == 0) give(1); else give(0);
+        lds_barrier();
+        if (grp == 0) finish(0); else finish(1);
+    } else {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+            if (qpos[nt] >= 0) store(nt, l[nt] > 0.f ? 1.0f / l[nt] : 0.f, [&](int t, int r) { return acc[nt][t][r]; });
+    }
+    lds_barrier();                                        // the ring is free for the next tile
   }
 }
 
@@ -1026,11 +1425,12 @@ static int attn_mfma_launch(const void* q, int q_stride, void* out, int out_stri
                             const int* tiles, int n_tiles, int n_tokens, int H, int Hkv, int hs, int GT,
                             int window, float scale, int n_splits, int chunk, float* part_o, float* part_ml,
                             const float* inv_freq, int rotate, int write_kv, const int* by_length,
-                            const int* max_len, const float* row_ssq, int n_pieces, int ssq_width, float ssq_eps,
+                            const int* max_len, const float* row_ssq, int n_pieces, int ssq_width, float ssq_eps, int n_seqs,
                             hipStream_t s) {
     if (!bn_attn_mfma_supports(hs) || n_tiles <= 0 || n_tokens <= 0 || H <= 0 || Hkv <= 0 || H % Hkv) return BN_ERR_ARG;
     if (row_ssq && (tiles || !rotate || n_pieces < 1 || n_pieces > 64 || ssq_width < 1)) return BN_ERR_ARG;   // decode form, rotating
     if (GT <= 0 || GT > 16 || (GT & (GT - 1)) || window < 0 || n_splits < 1 || n_splits > 64) return BN_ERR_ARG;
+    if (tiles && n_seqs < 1) return BN_ERR_ARG;
     if (n_splits > 1 && (!part_o || !part_ml || (!max_len && (chunk <= 0 || chunk % BN_PAGE)))) return BN_ERR_ARG;
     if (!tiles && (!seq_lens || bt_stride < 1)) return BN_ERR_ARG;      // the decode form reads a row's first entry unasked
     if (max_len && tiles) return BN_ERR_ARG;                               // decode form only
@@ -1056,27 +1456,14 @@ static int attn_mfma_launch(const void* q, int q_stride, void* out, int out_stri
     a.by_length = (!tiles && n_splits == 1 && (long long)n_tiles * wgs_per_seq > compute_units()) ? by_length : nullptr;
     a.order_period = compute_units() / wgs_per_seq;
     if (tiles) {
-        // a workgroup takes a pair of tiles when there are more tiles than CUs
-        const int paired = (long long)n_tiles * wgs_per_seq > compute_units() ? 1 : 0;
-        const long long wgs = (long long)(paired ? (n_tiles + 1) / 2 : n_tiles) * wgs_per_seq;
-        if (wgs > 0x7fffffff) return BN_ERR_ARG;
-        const dim3 grid((unsigned)wgs);
-        // Two groups of waves a workgroup (eight waves, one workgroup a CU) halve the chain of blocks that a tile walks,
-        // which is what a launch of one round waits for.  A launch of several rounds is faster with one group a
-        // workgroup and two workgroups a CU: they share nothing and drift apart, so that one's matrix instructions
-        // meet the other's vector work, where the two groups of one workgroup meet at a barrier in every stage and do
-        // the same thing at the same time (8 to 16 % at 8,192 tokens and for eight or 64 prompts of 128 to 2,048).
-        // It is taken from four rounds on, and from two when its rounds (of two workgroups a CU) are not much emptier
-        // than those of the wide form (6,144 tokens of one sequence are three full rounds of the wide form and one and
-        // a half of the other: 410 against 445 us).
         const long long cus = compute_units();
-        const double fill1 = (double)wgs / (double)(((wgs + 2 * cus - 1) / (2 * cus)) * 2 * cus);
-        const double fill2 = (double)wgs / (double)(((wgs + cus - 1) / cus) * cus);
-        const int ng = (wgs >= 4 * cus || (wgs >= 2 * cus && fill1 * 1.1 >= fill2)) ? 1 : 2;
-        // three staged blocks of 32 keys a group with their values: up to 96 KB, beyond the default limit of dynamic
-        // shared memory
-        const size_t smem = (size_t)PROMPT_BUFFERS * (32 * ng * hs + hs * 32 * ng) * 2;
-        auto go = [&](auto kernel, int which) {
+        // A workgroup takes a pair of tiles, a long and a short one, when there are more of them than CUs.
+        const int paired = (long long)n_tiles * wgs_per_seq > cus ? 1 : 0;
+        const long long pairs = (n_tiles + 1) / 2, wgs = (paired ? pairs : n_tiles) * wgs_per_seq;
+        if (2 * wgs > 0x7fffffff) return BN_ERR_ARG;
+        auto go = [&](auto kernel, int which, int ng) {
+            // three staged blocks of 32 keys a group with their values: up to 96 KB, beyond the default limit of dynamic shared memory
+            const size_t smem = (size_t)PROMPT_BUFFERS * (32 * ng * hs + hs * 32 * ng) * 2;
             static bool raised[4] = {false, false, false, false};
             if (!raised[which]) {
                 const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -1084,11 +1471,46 @@ static int attn_mfma_launch(const void* q, int q_stride, void* out, int out_stri
                 if (e != hipSuccess) return (int)e;
                 raised[which] = true;
             }
-            hipLaunchKernelGGL(kernel, grid, dim3(256 * ng), smem, s, a, n_tiles, paired);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256 * ng), smem, s, a, n_tiles, paired);
             return bn_launch_status();
         };
-        if (ng == 1) return hs == 64 ? go(attn_mfma_prompt_kernel<64, 4, 1>, 2) : go(attn_mfma_prompt_kernel<128, 2, 1>, 3);
-        return hs == 64 ? go(attn_mfma_prompt_kernel<64, 4, 2>, 0) : go(attn_mfma_prompt_kernel<128, 2, 2>, 1);
+        if (hs == 64) {
+            // Two groups of waves a workgroup (eight waves, one workgroup a CU) halve the chain of blocks that a tile walks,
+            // which is what a launch of one round waits for.  A launch of several rounds is faster with one group a
+            // workgroup and two workgroups a CU: they share nothing and drift apart, so that one's matrix instructions
+            // meet the other's vector work, where the two groups of one workgroup meet at a barrier in every stage and do
+            // the same thing at the same time (8 to 16 % at 8,192 tokens and for eight or 64 prompts of 128 to 2,048).
+            // It is taken from four rounds on, and from two when its rounds (of two workgroups a CU) are not much emptier
+            // than those of the wide form (6,144 tokens of one sequence are three full rounds of the wide form and one and
+            // a half of the other: 410 against 445 us).
+            const double fill1 = (double)wgs / (double)(((wgs + 2 * cus - 1) / (2 * cus)) * 2 * cus);
+            const double fill2 = (double)wgs / (double)(((wgs + cus - 1) / cus) * cus);
+            return (wgs >= 4 * cus || (wgs >= 2 * cus && fill1 * 1.1 >= fill2)) ? go(attn_mfma_prompt_kernel<64, 4, 1>, 1, 1)
+                                                                                : go(attn_mfma_prompt_kernel<64, 4, 2>, 0, 2);
+        }
+        // Heads of 128: groups that take turns over split keys (short chains) or with a tile each (a CU's keys are fetched once for two), or workgroups of one
+        // group that share nothing, two a CU (one's start hides behind the other's work).  us, one group / split / a tile each (before: the faster or
+        // the slower of one group and of two that walk in step, by the rule above), 32 heads over 8: one prompt of 300 15.3 / 14.4 / 16.9
+        // (15.3), 1,024 36 / 25 / 37 (30), 2,048 71 / 48 / 64 (59), 3,000 124 / 112 / 97 (146), 4,096 163 / 147 / 130 (166), 5,000 351 / 249 / 291 (329),
+        // 8,100 602 / 512 / 465 (615); 64 new tokens behind 4,000 115 / 60 / 108 (83); four of 70 to 500 26 / 24 / 23 (26), eight of 300
+        // 30 / 41 / 30 (44), of 128 to 2,048 191 / 184 / 169 (192), 16 of 1,024 220 / 243 / 195 (220), of 150 25 / 38 / 28 (38), 32 of 128 24 / 39 / 29 (25), of 512
+        // 143 / 192 / 148 (145), 64 of 16 to 512 155 / 223 / 166 (156); a window of 700 over 2,000 56 / 42 / 37 (49).
+        auto turns = [&](auto kernel, long long n, int two) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(512), 0, s, a, n_tiles, two);
+            return bn_launch_status();
+        };
+        // (a tile each: half of the workgroups find that another has taken their pair along)
+        const int paired2 = pairs * wgs_per_seq > cus ? 1 : 0;
+        auto split = [&] { return turns(attn_mfma_turns_kernel<128, 2, true>, wgs, paired); };
+        auto each = [&] { return turns(attn_mfma_turns_kernel<128, 2, false>, pairs * (paired2 ? 1 : 2) * wgs_per_seq, paired2); };
+        if (!paired) return split();                      // the chip is not full: as many, short chains as there can be
+        if (n_tokens < 640LL * n_seqs)                    // short sequences (by their new tokens): two workgroups a CU once there are that many
+            return wgs >= 2 * cus ? go(attn_mfma_prompt_kernel<128, 2, 1>, 3, 1) : each();
+        // Rounds over the CUs, whole ones where they are few; a split workgroup's is half as long, and costs an eighth more.  Tiles that all fit at once
+        // are as long as the last of them, twice the average where every token sees all before it.
+        auto rounds = [&](long long n) { const double r = (double)n / (double)cus; return r <= 2.0 ? std::ceil(r) : r + 0.35; };
+        const long long quads = (pairs + 1) / 2 * wgs_per_seq;
+        return rounds(paired2 ? quads : 2 * quads) * (window > 0 && !paired2 ? 0.5 : 1.0) <= rounds(wgs) * 0.56 ? each() : split();
     }
     if (n_tiles > 65535) return BN_ERR_ARG;                 // sequences are the grid's y
     // Two splits and no more workgroups than CUs: both in one workgroup, without a launch for the merge (WHOLE).  us, merged by a
@@ -1131,10 +1553,10 @@ extern "C" int bn_attn_mfma(const void* q, int q_stride, void* out, int out_stri
                             const int* tiles, int n_tiles, int n_tokens, int H, int Hkv, int hs, int GT,
                             int window, float scale, int n_splits, int chunk, float* part_o, float* part_ml,
                             const float* inv_freq, int rotate, int write_kv, const int* by_length,
-                            const int* max_len, hipStream_t s) {
+                            const int* max_len, int n_seqs, hipStream_t s) {
     return attn_mfma_launch(q, q_stride, out, out_stride, k_pages, vt_pages, block_table, bt_stride, seq_lens, tiles, n_tiles,
                             n_tokens, H, Hkv, hs, GT, window, scale, n_splits, chunk, part_o, part_ml, inv_freq, rotate,
-                            write_kv, by_length, max_len, nullptr, 0, 0, 0.f, s);
+                            write_kv, by_length, max_len, nullptr, 0, 0, 0.f, n_seqs, s);
 }
 
 // The decode form (tiles none, rotate on) over rows whose RMSNorm was left undone: q, the new key and the new value of
@@ -1148,7 +1570,7 @@ extern "C" int bn_attn_mfma_scaled(const void* q, int q_stride, void* out, int o
     if (!row_ssq) return BN_ERR_ARG;
     return attn_mfma_launch(q, q_stride, out, out_stride, k_pages, vt_pages, block_table, bt_stride, seq_lens, nullptr, n_seqs,
                             n_seqs, H, Hkv, hs, GT, window, scale, n_splits, chunk, part_o, part_ml, inv_freq, 1, write_kv,
-                            by_length, max_len, row_ssq, n_pieces, ssq_width, ssq_eps, s);
+                            by_length, max_len, row_ssq, n_pieces, ssq_width, ssq_eps, n_seqs, s);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1197,5 +1619,5 @@ extern "C" int bn_attn_mfma_decode_static(const void* q, int q_stride, void* out
     }
     return bn_attn_mfma(q, q_stride, out, out_stride, k_pages, vt_pages, block_table, bt_stride, seq_lens, nullptr,
                         n_seqs, n_seqs, H, Hkv, hs, GT, window, scale, n_splits, chunk, part_o, part_ml, inv_freq, rotate,
-                        write_kv, by_length, nullptr, s);
+                        write_kv, by_length, nullptr, n_seqs, s);
 }

@@ -167,7 +167,7 @@ _SIGNATURES = {
                                 c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
         "bn_attn_mfma": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                          c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p,
-                         c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p],
+                         c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p],
     },
     "attn_f32": {
         "bn_attn_f32_supports": [c_int],
@@ -1833,7 +1833,7 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
             float(scale), int(n_splits), int(chunk), po, pm,
             fused_rotate.data_ptr() if fused_rotate is not None else None, int(fused_rotate is not None),
             int(bool(fused_write)), by_length.data_ptr() if by_length is not None else None,
-            max_len_dev.data_ptr() if max_len_dev is not None else None, _stream()),
+            max_len_dev.data_ptr() if max_len_dev is not None else None, block_table.shape[0], _stream()),
             "attention(mfma)")
         return
     if f32_plain:
