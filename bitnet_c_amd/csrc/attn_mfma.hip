@@ -791,10 +791,9 @@ __global__ __launch_bounds__(512, 2) void attn_mfma_turns_kernel(MfmaArgs a, int
     static_assert(BLOCK == 8 * 1024 && NT == 2, "eight pieces of keys and of values; a column tile a group to merge");
     static_assert(4 * 64 * DT * 4 * 4 <= 2 * SLOT, "a group's accumulators of a column tile fit a slot of both groups");
     __shared__ __align__(1024) unsigned char r0[GROUPS * SLOT], r1[GROUPS * SLOT], r2[GROUPS * SLOT], r3[GROUPS * SLOT], r4[SPLIT ? 16 : SLOT];
-    __shared__ int on_simd[4];
     const int lane = threadIdx.x & 63;
-    int wave, grp;                                        // the wave's number in its group, and its group
-    bn_turn_roles(on_simd, wave, grp);
+    // a wave's number in its group, and its group: waves w and w + 4 share a SIMD (groups by the SIMD that a wave finds itself on measured the same or 1 to 2 % slower)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     const int own = SPLIT ? grp : 0, piece = SPLIT ? wave : 4 * grp + wave;         // among those that share a slot
     const int n = lane & 15, g = lane >> 4;
     const int G = a.H / a.Hkv, GT = a.GT;

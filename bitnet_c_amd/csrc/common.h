@@ -115,24 +115,6 @@ __device__ __forceinline__ void bn_load_to_lds(__amdgpu_buffer_rsrc_t b, void* l
     __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (__attribute__((address_space(3))) void*)lds, 16, lane_offset, offset, 0, 0);
 }
 
-// The roles of eight waves of which two share a SIMD, in two groups that take turns: the two of a SIMD are in different groups.  A workgroup on an empty CU gets waves w and
-// w + 4 on one SIMD, one that follows another as its waves end may get any two, so the waves count themselves: the SIMD's number is the
-// wave's number in its group, the order of arrival there its group (waves w and w + 4 should a SIMD have got more than two).  on_simd: four
-// numbers of shared memory.  All 512 threads.
-__device__ __forceinline__ void bn_turn_roles(int* on_simd, int& wave, int& group) {
-    const int simd = __builtin_amdgcn_s_getreg((2 - 1) << 11 | 4 << 6 | 4);         // HW_ID, bits 4 and 5
-    if (threadIdx.x < 4) on_simd[threadIdx.x] = 0;
-    __syncthreads();
-    int before = 0;
-    if ((threadIdx.x & 63) == 0) before = atomicAdd(&on_simd[simd], 1);
-    before = __builtin_amdgcn_readfirstlane(before);
-    __syncthreads();
-    const bool two = on_simd[0] == 2 && on_simd[1] == 2 && on_simd[2] == 2 && on_simd[3] == 2;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    wave = __builtin_amdgcn_readfirstlane(two ? simd : w & 3);
-    group = __builtin_amdgcn_readfirstlane(two ? before : w >> 2);
-}
-
 // Reductions over a wave as a butterfly: every lane adds the lane 32, 16, 8, 4, 2 and 1 away, in that order.  The two long
 // steps swap halves and rows (v_permlane32_swap, v_permlane16_swap), the short ones are data-parallel-primitive moves inside
 // a row of 16; through shared memory's crossbar (__shfl_xor) every step waits some 120 cycles for the one before it, a third
