@@ -20,8 +20,7 @@ CASES = [
 
 
 @pytest.mark.parametrize("H,Hkv,before,new,window", CASES)
-@pytest.mark.parametrize("order", ["paired", "ascending", "shuffled", "padded"])
-def test_turns(H, Hkv, before, new, window, order):
+def test_turns(H, Hkv, before, new, window):
     hs, dtype = 128, torch.bfloat16
     ops, qkv, kp, vp, bt, ref, scale = _attn_case(dtype, H, Hkv, hs, before, new, window, 77)
     _, _, qt = ops.attention_row_shape(H, Hkv, False, dtype, hs)
@@ -29,10 +28,9 @@ def test_turns(H, Hkv, before, new, window, order):
     for s, (p0, n) in enumerate(zip(before, new)):
         tiles += [(s, r + i, min(qt, n - i), p0 + i) for i in range(0, n, qt)]
         r += n
-    if order == "shuffled":
-        random.Random(1).shuffle(tiles)
-    elif order != "ascending":
-        tiles = ops.pair_tiles(tiles) + [(0, 0, 0, 0)] * (5 if order == "padded" else 0)
-    out = torch.full((r, H * hs), float("nan"), dtype=dtype).cuda()
-    ops.attention(qkv, out, kp, vp, bt, H, Hkv, hs, scale, window=window, tiles=torch.tensor(tiles, dtype=torch.int32).cuda(), qt=qt)
-    assert mfma_close(out.float(), ref)
+    paired, shuffled = ops.pair_tiles(tiles), list(tiles)
+    random.Random(1).shuffle(shuffled)
+    for order in (paired, tiles, shuffled, paired + [(0, 0, 0, 0)] * 5):
+        out = torch.full((r, H * hs), float("nan"), dtype=dtype).cuda()
+        ops.attention(qkv, out, kp, vp, bt, H, Hkv, hs, scale, window=window, tiles=torch.tensor(order, dtype=torch.int32).cuda(), qt=qt)
+        assert mfma_close(out.float(), ref)
