@@ -51,6 +51,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 __device__ __forceinline__ bf16x8 gm_as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
 
+#define GM_MAX_ITEMS 6
+
 struct GmGroups {
     const int* tiles;         // [n][3]: matrix of the stack, first row of X, rows (<= GM_BM); null: one product over all rows
     const int* n_tiles;       // [1]: tiles in the list
@@ -58,6 +60,9 @@ struct GmGroups {
     const float* row_scale;   // [rows of X]: a factor on row m's result; null: none
     long long w_stride;       // elements from one matrix of the stack to the next
     int unary;                // BN_UNARY_* applied to the result before anything else; < 0: none
+    const bf16* x[GM_MAX_ITEMS];            // (GM_ITEMS: X, W and Y of each product)
+    const bf16* w[GM_MAX_ITEMS];
+    bf16* y[GM_MAX_ITEMS];
 };
 
 // Shared memory serves a 16-byte read in four turns of 16 lanes; in the operand layout
@@ -318,6 +323,7 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_mfma_kernel(const bf16* __res
 #define GM_SILU 1                     // silu(gate) * up
 #define GM_GATED 2                    // act(gate) * up, the other activations
 #define GM_GROUPED 3                  // the grouped form's
+#define GM_ITEMS 4                    // stored, of several products of the same sizes (in the ranges' place)
 template <int BM, int BN, int EPI, typename TO>
 __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, TO* __restrict__ Y, int M,
                                                             int N, int K, int ldx, int ldw, int ldy, int tiles_m, int tiles_n, int splits,
@@ -348,7 +354,8 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
         m0 = tl[1];
         M = tl[1] + tl[2];
     }
-    const int k0 = sp * steps_per, steps = min(steps_per, K / GM_BK - k0);
+    if constexpr (EPI == GM_ITEMS) { X = grp.x[sp]; W = grp.w[sp]; Y = grp.y[sp]; }
+    const int k0 = EPI == GM_ITEMS ? 0 : sp * steps_per, steps = EPI == GM_ITEMS ? K / GM_BK : min(steps_per, K / GM_BK - k0);
     const int rows = min(BM, M - m0), cols = min(BN, N - n0);
     const __amdgpu_buffer_rsrc_t xbuf = bn_buffer(X + (size_t)m0 * ldx, ((rows - 1) * ldx + K) * 2);
     const __amdgpu_buffer_rsrc_t wbuf = bn_buffer(W + (size_t)n0 * ldw, ((cols - 1) * ldw + K) * 2);
@@ -497,7 +504,8 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
 
 static GmGroups gm_no_groups() {
     GmGroups g;
-    g.tiles = nullptr; g.n_tiles = nullptr; g.row_map = nullptr; g.row_scale = nullptr; g.w_stride = 0; g.unary = -1;
+    g = {};
+    g.unary = -1;
     return g;
 }
 
@@ -556,13 +564,13 @@ static double gm_cost(const GmTile& t, long long tiles, int steps, int cus) {
 
 // The tile and the ranges of K (up to max_splits) that take the least time for M rows, N rows of W and K columns; slabs are written and
 // read again at 5 TB/s, and more than two of them cost a launch.  bm: the only height to look at, or 0.
-static void gm_plan(int M, int N, int K, int bm, int max_splits, int* tile, int* splits) {
+static void gm_plan(int M, int N, int K, int bm, int max_splits, int* tile, int* splits, int items = 1) {
     const int cus = gm_compute_units(), steps = K / GM_BK;
     double best = -1.;
     for (int i = 0; i < GM_TILES; ++i) {
         const GmTile& t = gm_tiles[i];
         if (bm && t.bm != bm) continue;
-        const long long tiles = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        const long long tiles = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * items;
         for (int s = 1; s <= max_splits; ++s) {
             const int per = (steps + s - 1) / s;
             if ((steps + per - 1) / per != s) continue;
@@ -680,6 +688,22 @@ extern "C" int bn_gemm_mfma_slabs(const void* X, const void* W, float* Y, int M,
     gm_plan(M, N, K, 0, GM_MAX_SPLITS, &tile, &plan);
     if (plan != splits) return BN_ERR_ARG;
     return gm_turns<GM_STORE, float>(tile, X, W, Y, M, N, K, ldx, ldw, N, splits, 0, s, gm_no_groups());
+}
+
+// y[i] [M, N] (bf16, contiguous) = x[i] . w[i]^T for n products of the same sizes, in one launch: rows of x[i] ldx apart, w[i] contiguous.
+// A product of 2,048 x 2,048 over 2,048 rows is 128 tiles of 256 x 128 on 256 CUs and 23 us, as long as the other half stands idle; four
+// of them side by side are two whole rounds of 256 x 256 tiles' work, 57 us instead of 93 (1.2 PFLOP/s).  The item takes the place of the
+// range of K, so that the kernels' loops are the same; the tile is the one that suits all items' tiles together.
+extern "C" int bn_gemm_mfma_items(int n, const void* const* x, const void* const* w, void* const* y, int M, int N, int K, int ldx, hipStream_t s) {
+    if (n < 1 || n > GM_MAX_ITEMS || !bn_gemm_mfma_supports(M, N, K, ldx, K)) return BN_ERR_ARG;
+    GmGroups g = gm_no_groups();
+    for (int i = 0; i < n; ++i) {
+        if (!x[i] || !w[i] || !y[i] || (((uintptr_t)x[i] | (uintptr_t)w[i]) & 15) || !gm_turns_takes(N, K, ldx, K, N, y[i], 2)) return BN_ERR_ARG;
+        g.x[i] = (const bf16*)x[i]; g.w[i] = (const bf16*)w[i]; g.y[i] = (bf16*)y[i];
+    }
+    int tile = 0, splits = 1;
+    gm_plan(M, N, K, 0, 1, &tile, &splits, n);
+    return gm_turns<GM_ITEMS, bf16>(tile, nullptr, nullptr, nullptr, M, N, K, ldx, K, N, n, 0, s, g);
 }
 
 // The grouped form: X [rows, K] ordered by matrix, W [matrices][N, K] (w_stride elements apart), tiles [max_tiles][3] and

@@ -194,6 +194,7 @@ _SIGNATURES = {
         "bn_gemm_mfma_supports": [c_int, c_int, c_int, c_int, c_int],
         "bn_gemm_mfma": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                          c_int, c_void_p],
+        "bn_gemm_mfma_items": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
         "bn_gemm_mfma_splits": [c_int, c_int, c_int],
         "bn_gemm_mfma_slabs": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
         "bn_gemm_mfma_grouped": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_longlong,
@@ -583,6 +584,42 @@ def can_split_rows(M: int, N: int, K: int, dtype) -> bool:
     return tiles * 2 <= _compute_units() and (K > SPLIT_ROWS_MIN_K or tiles * 16 <= 3 * _compute_units())
 
 
+# ... products of the same sizes that do not depend on each other (linear_group), in one launch: alone each leaves CUs without work or ends
+# in a round that few of them share.  us one after the other (the library) -> together, 4 products of 2,048 x 2,048 at 129 / 512 / 2,048 /
+# 4,096 (8,192) rows 38 -> 23, 46 -> 26, 93 -> 57, 147 -> 125 (222 -> 257); 1,024 x 1,024 21 -> 13, 34 -> 14, 43 -> 23, 55 -> 35 (8,192: 87 ->
+# 68); 4,096 x 4,096 at 129 / 512 / 2,048 / 3,072 (4,096) 66 -> 39, 108 -> 69, 253 -> 218, 345 -> 329 (396 -> 430); 2,560 x 2,560 at 4,096 220 ->
+# 199.  So up to three quarters as many tiles of 256 x 256 a product as there are CUs.  Two products gain less, and nothing where few rows
+# make the tiles small in number (2,048 x 2,048 at 256 / 512 / 1,024 rows 20 -> 21, 23 -> 23, 32 -> 26; 4,096 x 4,096 at 256 / 2,048 / 3,072
+# 37 -> 39, 125 -> 106, 171 -> 176): from 1,024 rows to half as many tiles as CUs.
+GEMM_ITEMS = _build.header_constant("GM_MAX_ITEMS", "gemm_mfma.hip")
+
+
+def group_rows(n: int, M: int, N: int, K: int) -> bool:
+    """Whether n bf16 products x [M, K] . w[N, K]^T run faster in one launch (gemm_items)."""
+    if not (2 <= n <= GEMM_ITEMS and M >= (PROMPT_ROWS if n > 2 else 1024) and K % GEMM_STEP == 0 and K and N % 4 == 0):
+        return False
+    tiles = -(-M // 256) * -(-N // 256)
+    return tiles * 4 <= (3 if n > 2 else 2) * _compute_units()
+
+
+def gemm_items(xs, ws) -> list:
+    """[x . w^T] for up to GEMM_ITEMS pairs of the same sizes (bf16, K whole steps of GEMM_STEP, rows of the xs equally far apart,
+    contiguous ws), in one launch."""
+    require_gpu()
+    M, K = xs[0].shape
+    N, n, ld = ws[0].shape[0], len(xs), _rows(xs[0], "x")
+    for x, w in zip(xs, ws):
+        _dev(x, "x", torch.bfloat16, 2)
+        _dev(w, "w", torch.bfloat16, 2)
+        if tuple(x.shape) != (M, K) or tuple(w.shape) != (N, K) or _rows(x, "x") != ld or not w.is_contiguous():
+            raise KernelError(f"gemm_items: x {tuple(x.shape)} and w {tuple(w.shape)} among x {(M, K)} and w {(N, K)}")
+    ys = [torch.empty((M, N), dtype=torch.bfloat16, device=xs[0].device) for _ in xs]
+    ptr = c_void_p * n
+    _check(_fn("gemm_mfma", "bn_gemm_mfma_items")(n, ptr(*[x.data_ptr() for x in xs]), ptr(*[w.data_ptr() for w in ws]),
+                                                  ptr(*[y.data_ptr() for y in ys]), M, N, K, ld, _stream()), "gemm_mfma(items)")
+    return ys
+
+
 def linear_split_rows(x: torch.Tensor, w: torch.Tensor) -> "PartialSums":
     """x [M, K] . w[N, K]^T as float32 sums over ranges of K (bf16, K whole steps of GEMM_STEP), for the kernel of the next norm."""
     require_gpu()
@@ -786,7 +823,7 @@ GROUP_PRODUCTS = _build.header_constant("SK_GROUP", "skinny_gemm.hip")
 def linear_group(items) -> list:
     """[linear(x, w) or activation(linear(x, w))] for items (x, w, streamed copy of w or None, activation or None) whose
     products do not depend on each other: one launch for bf16 steps of up to 16 rows over streamed copies of matrices with
-    equally many columns, else one after the other."""
+    equally many columns, one for those of a prompt's products that group_rows says it of, else one after the other."""
     items = list(items)
     M, K = items[0][0].shape
     if (len(items) > 1 and len(items) <= GROUP_PRODUCTS and 1 <= M <= SKINNY_ROWS
@@ -801,7 +838,20 @@ def linear_group(items) -> list:
             num(*[w.shape[0] for _, w, _, _ in items]), num(*[_rows(x, "x") for x, _, _, _ in items]), num(*[a[2] for a in args]),
             num(*[-1 if act is None else UNARY_ACTIVATIONS[act] for _, _, _, act in items]), M, K, args[0][1], _stream()), "skinny_group")
         return ys
-    return [linear(x, w, streamed=sw) if act is None else linear_unary(x, w, act, sw) for x, w, sw, act in items]
+    ys = [None] * len(items)
+    if M >= PROMPT_ROWS:
+        same: dict = {}                                   # the products of one size
+        for i, (x, w, _, act) in enumerate(items):
+            if (act is None and x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and x.dim() == w.dim() == 2 and w.shape[1] == x.shape[1]
+                    and x.stride(1) == 1 and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0 and x.stride(0) <= 1 << 22
+                    and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+                same.setdefault((x.shape[0], x.stride(0), tuple(w.shape)), []).append(i)
+        for (rows, _, (N, k)), group in same.items():
+            if group_rows(len(group), rows, N, k):
+                for i, y in zip(group, gemm_items([items[i][0] for i in group], [items[i][1] for i in group])):
+                    ys[i] = y
+    return [y if y is not None else linear(x, w, streamed=sw) if act is None else linear_unary(x, w, act, sw)
+            for y, (x, w, sw, act) in zip(ys, items)]
 
 
 def interleave_gate_up(w_gate: torch.Tensor, w_up: torch.Tensor) -> torch.Tensor:

@@ -67,6 +67,27 @@ def test_slabs(M, N, K):
     assert _rel(h, want / torch.sqrt((want * want).mean(1, keepdim=True) + 1e-5) * weight) < 2.0 ** -8
 
 
+# products in one launch: sizes at which each tile is chosen, with rows and columns that fill none, and a group beside others
+@pytest.mark.parametrize("n,M,N,K", [(3, 129, 260, 64), (6, 130, 2052, 192), (2, 1025, 2048, 128), (4, 1000, 1028, 576), (5, 2049, 1540, 64),
+                                     (4, 4099, 2564, 128)])
+def test_products_side_by_side(n, M, N, K):
+    ops = _ops()
+    assert ops.group_rows(n, M, N, K)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    xs = torch.randn(n, M, K + 8, generator=g, device="cuda").to(torch.bfloat16)[:, :, :K]        # rows further apart than they are long
+    ws = [(torch.randn(N, K, generator=g, device="cuda") * 0.05).to(torch.bfloat16) for _ in range(n)]
+    other = (xs[0], ws[0][:16].contiguous(), None, "tanh"), (xs[1], ws[1][:N - 4], None, None)
+    items = [(x, w, None, None) for x, w in zip(xs, ws)]
+    got = ops.linear_group([items[0], other[0], *items[1:], other[1]])
+    beside = [got.pop(1), got.pop()]
+    for (x, w, _, _), y, alone in zip(items, got, ops.gemm_items(list(xs), ws)):
+        assert torch.equal(y, alone) and _rel(y, x.double() @ w.double().t()) < 2.0 ** -8
+    assert _rel(beside[0], torch.tanh(xs[0].double() @ ws[0][:16].double().t())) < 2.0 ** -7
+    assert torch.equal(beside[1], ops.linear(xs[1], ws[1][:N - 4]))
+    with pytest.raises(ops.KernelError):
+        ops.gemm_items([xs[0], xs[1, 1:]], ws[:2])
+
+
 def test_numbers_that_are_none():
     """A row of X or of W that holds NaN or an infinity reaches its own results alone."""
     ops = _ops()
@@ -87,5 +108,8 @@ def test_what_the_rules_say():
     assert not ops.can_split_rows(128, 4096, 14336, bf) and not ops.can_split_rows(2049, 4096, 14336, bf)
     assert not ops.can_split_rows(548, 4096, 4096, bf) and not ops.can_split_rows(548, 4096, 14336 + 32, bf)
     assert not ops.can_split_rows(548, 4096, 14336, torch.float32)
+    assert ops.group_rows(4, 129, 2048, 2048) and ops.group_rows(2, 1024, 2048, 2048) and not ops.group_rows(2, 1023, 2048, 2048)
+    assert not ops.group_rows(4, 128, 2048, 2048) and not ops.group_rows(4, 8192, 2048, 2048) and not ops.group_rows(7, 512, 512, 512)
+    assert not ops.group_rows(4, 512, 2048, 2080) and not ops.group_rows(4, 512, 2046, 2048) and not ops.group_rows(1, 2048, 512, 512)
     with pytest.raises(ops.KernelError):
         ops.linear_split_rows(torch.zeros(130, 96, dtype=bf, device="cuda"), torch.zeros(64, 96, dtype=bf, device="cuda"))
