@@ -325,6 +325,7 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_mfma_kernel(const bf16* __res
 #define GM_GROUPED 3                  // the grouped form's
 #define GM_ITEMS 4                    // stored, of several products of the same sizes (in the ranges' place)
 #define GM_GELU_ERF 5                 // gelu(sum), the exact one
+#define GM_RELU2 6                    // max(sum, 0)^2
 
 // z (1 + erf(z / sqrt 2)) / 2 in 17 instructions (erff's alone are 40, with a branch): with x = |z| / sqrt 2 and t = 1 / (1 + 0.46 x),
 // erfc(x) / 2 = t 2^(p(t) - x^2 / ln 2), p the polynomial of degree 7 that interpolates log2(exp(x^2) erfc(x) / (2 t)) at the Chebyshev
@@ -486,7 +487,7 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
         }
     };
     if (EPI == GM_STORE) Y += (size_t)sp * M * ldy;
-    if constexpr (sizeof(TO) == 2 && (EPI == GM_STORE || EPI == GM_ITEMS || EPI == GM_GELU_ERF)) {
+    if constexpr (sizeof(TO) == 2 && EPI != GM_SILU && EPI != GM_GATED && EPI != GM_GROUPED) {
         // bf16 rows go out through shared memory, which nobody reads any more: a wave's part of the tile is written to a buffer of its
         // own, the 16-byte chunks of a row swizzled, and read back row by row, so that a store writes whole rows of 128 bytes and not 32
         // bytes of sixteen (8,192 x 2,048 at 2,048 / 8,192 rows 65.8 -> 52.6, 244 -> 207 us: rows of Y a power of two apart share a
@@ -509,6 +510,9 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
                         if (EPI == GM_GELU_ERF) {
 #pragma unroll
                             for (int r = 0; r < 4; ++r) c[r] = gm_gelu_erf(c[r]);
+                        } else if (EPI == GM_RELU2) {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) c[r] = bn_unary_act(c[r], BN_UNARY_RELU2);
                         }
                         store(reinterpret_cast<TO*>(at(u * HALF + b * 16 + i, (v * (WN / 2) + a * 16 >> 3) + (g >> 1)) + 8 * (g & 1)), c);
                     }
@@ -751,12 +755,14 @@ extern "C" int bn_gemm_mfma_slabs(const void* X, const void* W, float* Y, int M,
     return gm_turns<GM_STORE, float>(tile, X, W, Y, M, N, K, ldx, ldw, N, splits, 0, s, gm_no_groups());
 }
 
-// Y [M, N] (bf16, contiguous) = gelu(X . W^T), the exact gelu on the float32 sums.
-extern "C" int bn_gemm_mfma_gelu(const void* X, const void* W, void* Y, int M, int N, int K, int ldx, int ldw, hipStream_t s) {
+// Y [M, N] (bf16, contiguous) = act(X . W^T) on the float32 sums, act the exact gelu or relu2 (BN_UNARY_*).
+extern "C" int bn_gemm_mfma_unary(const void* X, const void* W, void* Y, int M, int N, int K, int ldx, int ldw, int kind, hipStream_t s) {
     if (!bn_gemm_mfma_supports(M, N, K, ldx, ldw) || !gm_turns_takes(N, K, ldx, ldw, N, Y, 2) || (((uintptr_t)X | (uintptr_t)W) & 15)) return BN_ERR_ARG;
+    if (kind != BN_UNARY_GELU_ERF && kind != BN_UNARY_RELU2) return BN_ERR_ARG;
     int tile = 0, splits = 1;
     gm_plan(M, N, K, 0, 1, &tile, &splits);
-    return gm_turns<GM_GELU_ERF, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, N, 1, 0, s, gm_no_groups());
+    return kind == BN_UNARY_RELU2 ? gm_turns<GM_RELU2, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, N, 1, 0, s, gm_no_groups())
+                                  : gm_turns<GM_GELU_ERF, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, N, 1, 0, s, gm_no_groups());
 }
 
 // y[i] [M, N] (bf16, contiguous) = x[i] . w[i]^T for n products of the same sizes, in one launch: rows of x[i] ldx apart, w[i] contiguous.

@@ -194,7 +194,7 @@ _SIGNATURES = {
         "bn_gemm_mfma_supports": [c_int, c_int, c_int, c_int, c_int],
         "bn_gemm_mfma": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                          c_int, c_void_p],
-        "bn_gemm_mfma_gelu": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
+        "bn_gemm_mfma_unary": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
         "bn_gemm_mfma_items": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
         "bn_gemm_mfma_splits": [c_int, c_int, c_int],
         "bn_gemm_mfma_slabs": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
@@ -621,32 +621,34 @@ def gemm_items(xs, ws) -> list:
     return ys
 
 
-# ... and a feed-forward's first product with the exact gelu on its sums, from 256 rows on and where the tiles of 256 x 256 are at least the
-# square root of K (with fewer the library's products over ranges of K are faster).  us, the library's product and the activation's kernel ->
-# one kernel: 8,192 x 2,048 at 512 / 1,024 / 2,048 / 8,192 rows 29 -> 24, 45 -> 40, 72 -> 62, 263 -> 243; 4,096 x 1,024 at 512 / 2,048 /
-# 8,192 (256: 16 tiles) 16 -> 15, 32 -> 25, 91 -> 77 (13 -> 14); 2,048 x 2,048 at 1,536 / 4,096 (1,024: 32 tiles) 25 -> 24, 44 -> 39 (21 -> 22);
-# 16,384 x 4,096 at 256 / 2,048 / 8,192 (129) 50 -> 42, 221 -> 205, 855 -> 814 (37 -> 43); 4,096 x 4,096 at 1,024 / 4,096 (768: 48 tiles)
-# 43 -> 42, 114 -> 103 (36 -> 39).
-GELU_ROWS = 256
+# ... and a feed-forward's first product with the exact gelu or relu2 on its sums, from 256 rows on and where the tiles of 256 x 256 are at
+# least the square root of K (with fewer the library's products over ranges of K are faster).  us, the library's product and the activation's
+# kernel -> one kernel with gelu: 8,192 x 2,048 at 512 / 1,024 / 2,048 / 8,192 rows 29 -> 24, 45 -> 40, 72 -> 62, 263 -> 243; 4,096 x 1,024
+# at 512 / 2,048 / 8,192 (256: 16 tiles) 16 -> 15, 32 -> 25, 91 -> 77 (13 -> 14); 2,048 x 2,048 at 1,536 / 4,096 (1,024: 32 tiles) 25 -> 24,
+# 44 -> 39 (21 -> 22); 16,384 x 4,096 at 256 / 2,048 / 8,192 (129) 50 -> 42, 221 -> 205, 855 -> 814 (37 -> 43); 4,096 x 4,096 at 1,024 /
+# 4,096 (768: 48 tiles) 43 -> 42, 114 -> 103 (36 -> 39).  With relu2 8,192 x 2,048 at 512 / 2,048 / 2,560 / 8,192 28 -> 25,
+# 66 -> 57, 92 -> 80, 236 -> 210; 4,096 x 1,024 at 2,048 29 -> 21; 16,384 x 4,096 at 512 / 8,192 66 -> 63, 802 -> 755.
+UNARY_PROMPT_ROWS = 256
+UNARY_PROMPT = ("gelu_erf", "relu2")
 
 
-def gelu_in_product(M: int, N: int, K: int) -> bool:
-    """Whether gelu(x [M, K] . w[N, K]^T) of a bf16 prompt is one kernel (gemm_gelu)."""
+def unary_in_product(M: int, N: int, K: int, activation: str) -> bool:
+    """Whether activation(x [M, K] . w[N, K]^T) of a bf16 prompt is one kernel (gemm_unary)."""
     tiles = -(-M // 256) * -(-N // 256)
-    return M >= GELU_ROWS and K > 0 and K % GEMM_STEP == 0 and N % 4 == 0 and tiles * tiles >= K
+    return activation in UNARY_PROMPT and M >= UNARY_PROMPT_ROWS and K > 0 and K % GEMM_STEP == 0 and N % 4 == 0 and tiles * tiles >= K
 
 
-def gemm_gelu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """gelu(x [M, K] . w[N, K]^T), the exact gelu, on the float32 sums (bf16, K whole steps of GEMM_STEP, N a multiple of 4)."""
+def gemm_unary(x: torch.Tensor, w: torch.Tensor, activation: str) -> torch.Tensor:
+    """activation(x [M, K] . w[N, K]^T), one of UNARY_PROMPT, on the float32 sums (bf16, K whole steps of GEMM_STEP, N a multiple of 4)."""
     require_gpu()
     _dev(x, "x", torch.bfloat16, 2)
     _dev(w, "w", torch.bfloat16, 2)
     (M, K), N = x.shape, w.shape[0]
-    if w.shape[1] != K:
-        raise KernelError(f"gemm_gelu: x {tuple(x.shape)} and w {tuple(w.shape)} do not agree")
+    if w.shape[1] != K or activation not in UNARY_PROMPT:
+        raise KernelError(f"gemm_unary: x {tuple(x.shape)}, w {tuple(w.shape)}, {activation!r}")
     y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    _check(_fn("gemm_mfma", "bn_gemm_mfma_gelu")(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, _rows(x, "x"), _rows(w, "w"), _stream()),
-           "gemm_mfma(gelu)")
+    _check(_fn("gemm_mfma", "bn_gemm_mfma_unary")(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, _rows(x, "x"), _rows(w, "w"),
+                                                  UNARY_ACTIVATIONS[activation], _stream()), "gemm_mfma(unary)")
     return y
 
 
@@ -828,8 +830,8 @@ _ACT_UNARY = _build.header_constant("SK_ACT_UNARY", "skinny_gemm.hip")     # + a
 
 def linear_unary(x: torch.Tensor, w: torch.Tensor, activation: str, streamed: Optional[StreamedWeight] = None) -> torch.Tensor:
     """activation(linear(x, w)) (one of UNARY_ACTIVATIONS): a feed-forward's first product without a gate.  bf16 steps of up
-    to 16 rows form it in the product's own kernel, on the float32 sums, and so do a prompt's where it is the exact gelu and
-    gelu_in_product says so; everything else is the product, then the activation's kernel."""
+    to 16 rows form it in the product's own kernel, on the float32 sums, and so do a prompt's where
+    unary_in_product says so; everything else is the product, then the activation's kernel."""
     require_gpu()
     _dev(x, "x", dims=2)
     _dev(w, "w", x.dtype, 2)
@@ -843,10 +845,10 @@ def linear_unary(x: torch.Tensor, w: torch.Tensor, activation: str, streamed: Op
         _check(_fn("skinny_gemm", "bn_skinny_gemm")(_code(torch.bfloat16), x.data_ptr(), wp, y.data_ptr(), M, N, K, _rows(x, "x"),
                                                     wl, N, 0, 0, act, tiled, _stream()), "skinny_gemm(unary)")
         return y
-    if (x.dtype == torch.bfloat16 and activation == "gelu_erf" and w.shape[1] == K and gelu_in_product(M, N, K)
+    if (x.dtype == torch.bfloat16 and w.shape[1] == K and unary_in_product(M, N, K, activation)
             and (x.data_ptr() | w.data_ptr()) % 16 == 0 and _rows(x, "x") % 8 == 0 and _rows(w, "w") % 8 == 0
             and max(_rows(x, "x"), _rows(w, "w")) <= 1 << 22):
-        return gemm_gelu(x, w)
+        return gemm_unary(x, w, activation)
     y = linear(x, w, streamed=streamed)
     return unary_act(y, activation, out=y)
 

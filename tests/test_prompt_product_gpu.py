@@ -88,26 +88,26 @@ def test_products_side_by_side(n, M, N, K):
         ops.gemm_items([xs[0], xs[1, 1:]], ws[:2])
 
 
-# gelu on the sums: the same edges, from its least rows on; results that lie nowhere near a whole 16 bytes
+# an activation on the sums: the same edges, from its least rows on; results that lie nowhere near a whole 16 bytes
 @pytest.mark.parametrize("M,N,K", [(256, 2048, 64), (257, 4112, 64), (300, 528, 128), (511, 8204, 1088), (700, 8208, 448), (1025, 16396, 128)])
-def test_gelu_on_the_sums(M, N, K):
+@pytest.mark.parametrize("act", ["gelu_erf", "relu2"])
+def test_activations_on_the_sums(M, N, K, act):
     ops = _ops()
     x, w, ref = _data(M, N, K, 24)
-    got = ops.gemm_gelu(x, w)
-    want = torch.nn.functional.gelu(ref)
+    got = ops.gemm_unary(x, w, act)
+    want = torch.nn.functional.gelu(ref) if act == "gelu_erf" else ref.clamp(min=0) ** 2
     assert _rel(got, want) < 2.0 ** -8
     # element by element: the sums' roundings, the rounding to bf16 and 1e-4 of the value where it is as small as 1e-20 (|z| < 9.3)
     assert bool(((got.double() - want).abs() <= want.abs() * (2.0 ** -8 + 1e-4) + 1e-5).all())
-    two = ops.unary_act(ops.linear(x, w), "gelu_erf")
+    two = ops.unary_act(ops.linear(x, w), act)
     assert _rel(got, want) <= _rel(two, want)            # one rounding instead of two
-    if ops.gelu_in_product(M, N, K):
-        assert torch.equal(ops.linear_unary(x, w, "gelu_erf"), got)
-    else:
-        assert torch.equal(ops.linear_unary(x, w, "gelu_erf"), two)
+    assert torch.equal(ops.linear_unary(x, w, act), got if ops.unary_in_product(M, N, K, act) else two)
     x = x.clone()
-    x[M - 1, 5], x[M - 2, 7] = float("nan"), 1e30         # NaN stays NaN; +-1e28 or so gives itself or 0
-    got, z = ops.gemm_gelu(x, w), x[M - 2].double() @ w.double().t()
-    assert bool(got[M - 1].isnan().all()) and _rel(got[M - 2], z.clamp(min=0)) < 2.0 ** -8 and _rel(got[:M - 2], want[:M - 2]) < 2.0 ** -8
+    x[M - 1, 5], x[M - 2, 7] = float("nan"), 1e9          # NaN stays NaN (as the library's two kernels have it), a large number gives itself or 0
+    got, z = ops.gemm_unary(x, w, act), x[M - 2].double() @ w.double().t()
+    large = z.clamp(min=0) if act == "gelu_erf" else z.clamp(min=0) ** 2
+    assert torch.equal(got[M - 1].isnan(), ops.unary_act(ops.linear(x, w), act)[M - 1].isnan())
+    assert _rel(got[M - 2], large) < 2.0 ** -8 and _rel(got[:M - 2], want[:M - 2]) < 2.0 ** -8
 
 
 def test_numbers_that_are_none():
@@ -132,8 +132,9 @@ def test_what_the_rules_say():
     assert not ops.can_split_rows(548, 4096, 14336, torch.float32)
     assert ops.group_rows(4, 129, 2048, 2048) and ops.group_rows(2, 1024, 2048, 2048) and not ops.group_rows(2, 1023, 2048, 2048)
     assert not ops.group_rows(4, 128, 2048, 2048) and not ops.group_rows(4, 8192, 2048, 2048) and not ops.group_rows(7, 512, 512, 512)
-    assert ops.gelu_in_product(256, 16384, 4096) and not ops.gelu_in_product(255, 16384, 4096) and not ops.gelu_in_product(1024, 2048, 2048)
-    assert not ops.gelu_in_product(2048, 8192, 2080) and not ops.gelu_in_product(2048, 8190, 2048)
+    for act, (M, N, K) in (("gelu_erf", (256, 16384, 4096)), ("relu2", (2048, 8192, 2048))):
+        assert ops.unary_in_product(M, N, K, act) and not ops.unary_in_product(255, N, K, act) and not ops.unary_in_product(1024, 2048, 2048, act)
+        assert not ops.unary_in_product(M, N, K + 32, act) and not ops.unary_in_product(M, N - 2, K, act) and not ops.unary_in_product(M, N, K, "silu")
     assert not ops.group_rows(4, 512, 2048, 2080) and not ops.group_rows(4, 512, 2046, 2048) and not ops.group_rows(1, 2048, 512, 512)
     with pytest.raises(ops.KernelError):
         ops.linear_split_rows(torch.zeros(130, 96, dtype=bf, device="cuda"), torch.zeros(64, 96, dtype=bf, device="cuda"))
