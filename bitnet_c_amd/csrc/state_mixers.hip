@@ -840,10 +840,64 @@ __global__ __launch_bounds__(BN_WAVE) void head_norm_gate_kernel(T* __restrict__
     }
 }
 
+// The same for the rows of a bf16 prompt: a lane holds eight neighbouring numbers of a head (16-byte loads and stores), dv / 8 lanes a
+// head.  Bound by memory (5.2 TB/s at 8,192 rows of 32 heads of 64).  us, a wave a head (above: one number a lane at dv = 64, workgroups of
+// one wave) -> this at 129 / 512 / 2,048 / 8,192 rows: 32 heads of 64 3.2 -> 2.8, 6.0 -> 3.6, 18.2 -> 8.2, 62.6 -> 30.7; 16 of 128 3.1 -> 3.0, 4.8 ->
+// 3.6, 12.3 -> 8.3, 42.9 -> 30.7; 8 of 64 2.5 -> 2.8, 3.2 -> 2.9, 6.0 -> 3.6, 18.3 -> 8.0.  With fewer than HNG_MIN numbers the other is as fast
+// or faster by up to 0.6 (16 rows).
+#define HNG_WAVES 4
+#define HNG_MIN (1 << 18)
+__global__ __launch_bounds__(HNG_WAVES* BN_WAVE) void head_norm_gate_rows_kernel(bf16* __restrict__ y, const float* __restrict__ o,
+                                                                                 const bf16* __restrict__ gate, int ldg,
+                                                                                 const float* __restrict__ weight, size_t n8, int row8, int lanes,
+                                                                                 float eps) {
+    const size_t at = (size_t)blockIdx.x * (HNG_WAVES * BN_WAVE) + threadIdx.x;
+    const bool live = at < n8;                           // (dead lanes are whole heads: n8 is a multiple of lanes)
+    const size_t j = live ? at : 0;
+    const size_t t = j / row8;
+    const int c = (int)(j - t * row8) * 8;
+    float v[8], g[8];
+    const float4 a0 = reinterpret_cast<const float4*>(o)[2 * j], a1 = reinterpret_cast<const float4*>(o)[2 * j + 1];
+    const uint4 b = *reinterpret_cast<const uint4*>(gate + t * (size_t)ldg + c);
+    v[0] = a0.x; v[1] = a0.y; v[2] = a0.z; v[3] = a0.w; v[4] = a1.x; v[5] = a1.y; v[6] = a1.z; v[7] = a1.w;
+    const uint32_t w[4] = {b.x, b.y, b.z, b.w};
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        g[e] = e & 1 ? bf16hi_to_f32(w[e >> 1]) : bf16lo_to_f32(w[e >> 1]);
+        ss = fmaf(v[e], v[e], ss);
+    }
+    for (int m = 1; m < lanes; m <<= 1) ss += __shfl_xor(ss, m, BN_WAVE);
+    if (!live) return;
+    const float f = 1.0f / sqrtf(ss / (float)(8 * lanes) + eps);
+    float wt[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
+    if (weight) {
+        const float4 w0 = *reinterpret_cast<const float4*>(weight + c), w1 = *reinterpret_cast<const float4*>(weight + c + 4);
+        wt[0] = w0.x; wt[1] = w0.y; wt[2] = w0.z; wt[3] = w0.w; wt[4] = w1.x; wt[5] = w1.y; wt[6] = w1.z; wt[7] = w1.w;
+    }
+    uint32_t p[4];
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        const bf16 lo = from_f32<bf16>(v[e] * f * wt[e] * bn_unary_act(g[e], BN_UNARY_SILU));
+        const bf16 hi = from_f32<bf16>(v[e + 1] * f * wt[e + 1] * bn_unary_act(g[e + 1], BN_UNARY_SILU));
+        p[e >> 1] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
+    }
+    reinterpret_cast<uint4*>(y)[j] = make_uint4(p[0], p[1], p[2], p[3]);
+}
+
 extern "C" int bn_head_norm_gate(int dtype, void* y, const float* o, const void* gate, int ldg, const float* weight,
                                  int n_tokens, int H, int dv, float eps, hipStream_t s) {
     if (n_tokens <= 0 || H <= 0 || dv <= 0 || !y || !o || !gate || ldg < H * dv) return BN_ERR_ARG;
     const dim3 grid(n_tokens, H);
+    const int lanes = dv / 8;
+    if (dtype == BN_DT_BF16 && (long long)n_tokens * H * dv >= HNG_MIN && dv % 8 == 0 && lanes <= BN_WAVE && (lanes & (lanes - 1)) == 0 && ldg % 8 == 0 &&
+        !(((uintptr_t)y | (uintptr_t)o | (uintptr_t)gate | (uintptr_t)weight) & 15)) {
+        const size_t n8 = (size_t)n_tokens * H * lanes, wgs = (n8 + HNG_WAVES * BN_WAVE - 1) / (HNG_WAVES * BN_WAVE);
+        if (wgs > 0x7fffffff) return BN_ERR_ARG;
+        hipLaunchKernelGGL(head_norm_gate_rows_kernel, dim3((unsigned)wgs), dim3(HNG_WAVES * BN_WAVE), 0, s, (bf16*)y, o, (const bf16*)gate, ldg,
+                           weight, n8, H * lanes, lanes, eps);
+        return bn_launch_status();
+    }
     if (dtype == BN_DT_F32)
         hipLaunchKernelGGL(head_norm_gate_kernel<float>, grid, dim3(BN_WAVE), 0, s, (float*)y, o, (const float*)gate, ldg, weight, H, dv, eps);
     else if (dtype == BN_DT_BF16)

@@ -86,3 +86,26 @@ def test_numbers_that_are_none_reach_no_token_before_them(what, pieces):
         assert not bool(torch.isfinite(got[bad:, 5]).any()) and bool(torch.isfinite(got[:, :5]).all())
     else:
         assert not bool(torch.isfinite(got[bad]).any())
+
+
+# the norm and gate behind the recurrence: heads of 1 to 64 lanes, a last workgroup that is not full, gates further apart than they are
+# long, and what the form of eight numbers a lane does not take (an odd gate, other head sizes, few numbers)
+@pytest.mark.parametrize("T,H,dv,skip,pad", [(4097, 8, 8, 8, 8), (1025, 16, 16, 0, 0), (347, 24, 32, 8, 0), (131, 32, 64, 16, 8), (129, 17, 128, 0, 8),
+                                             (70, 15, 256, 8, 0), (37, 14, 512, 8, 8), (131, 32, 64, 3, 5), (300, 10, 96, 0, 0), (127, 32, 64, 0, 0)])
+def test_norm_and_gate_of_a_prompt(T, H, dv, skip, pad):
+    from bitnet_c_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(T + dv)
+    o = torch.randn(T, H * dv, generator=g, device="cuda") * torch.logspace(-6, 6, T, device="cuda")[:, None]
+    gate = torch.randn(T, skip + H * dv + pad, generator=g, device="cuda").to(torch.bfloat16)[:, skip:skip + H * dv]
+    weight = torch.rand(H * dv, generator=g, device="cuda") + 0.5
+    o[T // 2, :dv] = 0                                   # a head of zeros; a head with NaN keeps it to itself
+    o[T - 1, -1] = float("nan")
+    d = o.double().view(T, H, dv)
+    for w in (weight, None):
+        want = (d / torch.sqrt((d * d).mean(2, keepdim=True) + 1e-6)).view(T, H * dv) * torch.nn.functional.silu(gate.double())
+        want = want if w is None else want * w.double()
+        got = ops.head_norm_gate(o, gate, w, H, dv, 1e-6)
+        assert torch.equal(got.isnan(), want.isnan()) and int(got.isnan().sum()) == dv
+        got, want = got.nan_to_num(0.0).double(), want.nan_to_num(0.0)
+        assert float((got - want).norm() / want.norm()) < 2.0 ** -8          # one rounding to bf16
+        assert bool(((got - want).abs() <= want.abs() * (2.0 ** -8 + 1e-5)).all())
