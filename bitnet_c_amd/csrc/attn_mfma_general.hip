@@ -314,6 +314,15 @@ struct GenDecodeArgs {
     int q_stride, out_stride, bt_stride, H, Hkv, n_splits, chunk, window, keep_first, sink;
     const float* sink_values; // [H] float32, or null (score 0)
     float scale;
+    // (NEW: the row of q holds projections, its keys at q + H hs)
+    bf16* k_new;              // the pages again, to be written
+    bf16* v_new;
+    const float* wq;          // [hs] norms of every query and key head; null: none
+    const float* wk;
+    const float* inv_freq;    // [rope_dims / 2] rotation in split-half pairs; null: none
+    int rope_dims, temp_every;
+    int v_col;                // the first value's column of the row: behind the keys, or the keys as projected
+    float eps, temp_coef;
 };
 
 // Keys and values that one wave reads each are read non-temporally (ONCE) while a launch's tables hold no more than this many MB of
@@ -325,7 +334,15 @@ struct GenDecodeArgs {
 // the length on the device: 0.4 us slower than either.)
 #define AG_ONCE_MB 24
 
-template <int DC, int DT, bool ONCE>     // hs = 32 DC, vd = 16 DT
+// NEW: the new token's row is still as projected.  Every wave norms, rotates and scales its queries, and the waves of the run that holds
+// the new position its key, in the registers in which they are multiplied (rotations turn pairs a whole number of 32 dimensions apart, so
+// a lane holds both); these put key and value in the place of what their block's loads found there, and one of them writes the pages.
+// The arithmetic is qk_norm_store_kernel's but for the order of a norm's sum.  us, that kernel and this without NEW -> this alone (norms,
+// 64 rotated dimensions), one sequence of 300 / four of 2,000 / 64 of 2,000 keys: 16 heads of 128 over 4 13.4 -> 11.1, 16.6 -> 14.1, 54.6 ->
+// 49.9; 64 of 128 over one 13.7 -> 11.2, 16.3 -> 13.8, 48.0 -> 40.9; 16 of 256 over 2 16.8 -> 13.6, 22.5 -> 18.3, 70.6 -> 63.9; 16 of 64 over 16
+// 11.8 -> 9.4, 18.5 -> 15.1, 126 -> 119: faster everywhere.  Bound by latency: everything that waits for no length is asked for in front of
+// the length itself, and the pages are written behind the loop (asked for inside branches and written in front of it 2 us more).
+template <int DC, int DT, bool ONCE, bool NEW>     // hs = 32 DC, vd = 16 DT
 __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeArgs a) {
     constexpr int HS = 32 * DC, VD = 16 * DT;
     const int seq = blockIdx.x, split = blockIdx.z;
@@ -334,6 +351,32 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
     const int lane = threadIdx.x, i = lane & 15, g = lane >> 4;
     const bool col_ok = 16 * ht + i < G;                 // this lane's column is a head that exists
     const int head = kvh * G + min(16 * ht + i, G - 1);
+    bf16x8 qf[DC], key[DC];                              // (NEW) the new token's key, and its value's column 16 t + i
+    bf16 value[DT];
+    constexpr int HC = DC / 2 > 0 ? DC / 2 : 1;
+    float4 nq[2 * DC], nk[2 * DC], turn[2 * HC];
+    const int hc = NEW && a.inv_freq ? a.rope_dims / 64 : 0;            // chunks of 32 between the two of a pair
+    if constexpr (NEW) {                                 // all that no length is needed for, before the loads that follow from one another
+        const bf16* row = a.q + (size_t)seq * a.q_stride + 8 * g;
+        const bf16* vp = a.q + (size_t)seq * a.q_stride + a.v_col + (size_t)kvh * VD + i;
+#pragma unroll
+        for (int c = 0; c < DC; ++c) { qf[c] = ag_ld16(row + (size_t)head * HS + 32 * c); key[c] = ag_ld16(row + (size_t)(a.H + kvh) * HS + 32 * c); }
+#pragma unroll
+        for (int t = 0; t < DT; ++t) value[t] = vp[16 * t];
+        const float4 one = make_float4(1.f, 1.f, 1.f, 1.f);
+#pragma unroll
+        for (int c = 0; c < 2 * DC; ++c) { nq[c] = one; nk[c] = one; }
+        if (a.wq) {
+#pragma unroll
+            for (int c = 0; c < 2 * DC; ++c) {
+                nq[c] = *reinterpret_cast<const float4*>(a.wq + 32 * (c >> 1) + 8 * g + 4 * (c & 1));
+                nk[c] = *reinterpret_cast<const float4*>(a.wk + 32 * (c >> 1) + 8 * g + 4 * (c & 1));
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 2 * HC; ++c)
+            if (c < 2 * hc) turn[c] = *reinterpret_cast<const float4*>(a.inv_freq + 32 * (c >> 1) + 8 * g + 4 * (c & 1));
+    }
     const int len = a.seq_lens[seq], qpos = len - 1;
     int k_lo = 0, k_hi = 0, keep = 0;                    // this wave's keys: k_lo .. k_hi - 1, and 0 .. keep - 1
     if (len > 0) {
@@ -363,8 +406,7 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
         }
         return;
     }
-    bf16x8 qf[DC];
-    {
+    if constexpr (!NEW) {
         const bf16* qp = a.q + (size_t)seq * a.q_stride + (size_t)head * HS + 8 * g;
 #pragma unroll
         for (int c = 0; c < DC; ++c) qf[c] = ag_ld16(qp + 32 * c);
@@ -388,12 +430,66 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
     const int first_block = k_lo & ~31, last_block = ((k_hi - 1) / 32) * 32;
     auto leap = [&](int kb) { return kb >= keep && kb < first_block ? first_block : kb; };
     ask_keys(leap(0));
+    const int new_block = NEW && k_hi == len ? last_block : -1;
+    if constexpr (NEW) {
+        float sn[HC][8], cs[HC][8];
+#pragma unroll
+        for (int c = 0; c < HC; ++c)
+            if (c < hc) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) bn_sincos((float)qpos * reinterpret_cast<const float*>(&turn[2 * c + (e >> 2)])[e & 3], &sn[c][e], &cs[c][e]);
+            }
+        auto shape = [&](bf16x8(&f)[DC], const float4(&w)[2 * DC], float factor) {
+            float x[DC][8], ss = 0.f;
+#pragma unroll
+            for (int c = 0; c < DC; ++c)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) { x[c][e] = (float)f[c][e]; ss = fmaf(x[c][e], x[c][e], ss); }
+            if (a.wq) {
+                const auto sum = [](float u, float v) { return u + v; };
+                ss = bn_pair_far<32>(bn_pair_far<16>(ss, sum), sum);
+                const float r = 1.0f / sqrtf(ss / (float)HS + a.eps);
+#pragma unroll
+                for (int c = 0; c < DC; ++c)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x[c][e] = x[c][e] * r * reinterpret_cast<const float*>(&w[2 * c + (e >> 2)])[e & 3];
+            }
+#pragma unroll
+            for (int h = 1; h <= DC / 2; ++h)
+                if (h == hc) {
+#pragma unroll
+                    for (int c = 0; c < h; ++c)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            const float u = x[c][e], v = x[c + h][e];
+                            x[c][e] = u * cs[c][e] - v * sn[c][e];
+                            x[c + h][e] = v * cs[c][e] + u * sn[c][e];
+                        }
+                }
+#pragma unroll
+            for (int c = 0; c < DC; ++c) {
+                const f32x8 y = {x[c][0] * factor, x[c][1] * factor, x[c][2] * factor, x[c][3] * factor,
+                                 x[c][4] * factor, x[c][5] * factor, x[c][6] * factor, x[c][7] * factor};
+                f[c] = __builtin_convertvector(y, bf16x8);
+            }
+        };
+        shape(qf, nq, a.temp_every > 0 ? 1.0f + a.temp_coef * logf((float)(len / a.temp_every) + 1.0f) : 1.0f);
+        if (new_block >= 0) shape(key, nk, 1.0f);
+    }
     for (int kb = leap(0); kb < k_hi; kb = leap(kb + 32)) {
         const int page = a.block_table[(size_t)seq * a.bt_stride + kb / BN_PAGE];
         const bf16* vbase = a.v_pages + (((size_t)page * a.Hkv + kvh) * VD + i) * BN_PAGE + kb % BN_PAGE + 8 * g;
         bf16x8 k0[DC], k1[DC];
 #pragma unroll
         for (int c = 0; c < DC; ++c) { k0[c] = kn0[c]; k1[c] = kn1[c]; }
+        if (NEW && kb == new_block) {
+            const int at = qpos - kb;
+#pragma unroll
+            for (int c = 0; c < DC; ++c) {
+                if (krow == at) k0[c] = key[c];
+                if (krow + 4 == at) k1[c] = key[c];
+            }
+        }
         ask_keys(min(leap(kb + 32), last_block));
         f32x4 st0 = (f32x4){0.f, 0.f, 0.f, 0.f}, st1 = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -432,6 +528,14 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
         const bf16x8 pb = __builtin_convertvector(pv, bf16x8);
         const f32x4 lsum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
         l = fmaf(l, alpha, lsum[0]);
+        if (NEW && kb == new_block) {
+            const int at = qpos - kb - 8 * g;
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (e == at) va[t][e] = __builtin_bit_cast(__bf16, value[t]);
+        }
         // positions past the sequence's end may hold anything in V^T (0 * NaN is NaN): cleared
         if (kb + 32 > k_hi) {
 #pragma unroll
@@ -453,6 +557,19 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
         for (int t = 0; t < DT; ++t) {
             acc[t] *= alpha;
             acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[t], pb, acc[t], 0, 0, 0);
+        }
+    }
+    if (NEW && new_block >= 0 && ht == 0) {              // (behind the loop: a load would wait for the stores in front of it)
+        const int page = a.block_table[(size_t)seq * a.bt_stride + qpos / BN_PAGE];
+        if (i == 0) {
+            bf16* dst = a.k_new + (((size_t)page * a.Hkv + kvh) * BN_PAGE + qpos % BN_PAGE) * HS + 8 * g;
+#pragma unroll
+            for (int c = 0; c < DC; ++c) *reinterpret_cast<bf16x8*>(dst + 32 * c) = key[c];
+        }
+        if (g == 0) {
+            bf16* dst = a.v_new + (((size_t)page * a.Hkv + kvh) * VD + i) * BN_PAGE + qpos % BN_PAGE;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) dst[(size_t)t * 16 * BN_PAGE] = value[t];
         }
     }
     if (!col_ok) return;
@@ -589,8 +706,10 @@ extern "C" int bn_attn_general_prompt(const void* q, int q_stride, void* out, in
 template <int DC>
 static int ag_launch_decode_dt(const GenDecodeArgs& a, int vd, bool once, dim3 grid, hipStream_t s) {
 #define AG_CASE(DT)                                                                                                       \
-    if (once) hipLaunchKernelGGL((attn_general_decode_kernel<DC, DT, true>), grid, dim3(BN_WAVE), 0, s, a);               \
-    else hipLaunchKernelGGL((attn_general_decode_kernel<DC, DT, false>), grid, dim3(BN_WAVE), 0, s, a);                   \
+    if (once && a.k_new) hipLaunchKernelGGL((attn_general_decode_kernel<DC, DT, true, true>), grid, dim3(BN_WAVE), 0, s, a);   \
+    else if (once) hipLaunchKernelGGL((attn_general_decode_kernel<DC, DT, true, false>), grid, dim3(BN_WAVE), 0, s, a);        \
+    else if (a.k_new) hipLaunchKernelGGL((attn_general_decode_kernel<DC, DT, false, true>), grid, dim3(BN_WAVE), 0, s, a);     \
+    else hipLaunchKernelGGL((attn_general_decode_kernel<DC, DT, false, false>), grid, dim3(BN_WAVE), 0, s, a);                 \
     return bn_launch_status()
     switch (vd / 16) {
         case 2: AG_CASE(2);
@@ -607,11 +726,18 @@ static int ag_launch_decode_dt(const GenDecodeArgs& a, int vd, bool once, dim3 g
 // Decode form: row b of q is sequence b's new token (seq_lens[b] keys in the cache, 0 for a padding row, whose output is
 // zeros).  n_splits > 1: part_o [n_seqs H n_splits, vd] and part_ml [n_seqs H n_splits, 2] float32 work space; the keys per
 // split are `chunk` (a multiple of BN_PAGE), or follow the longest sequence's key count in *max_len.
+// fresh: q's rows are projections (queries, keys, values) that this kernel norms (wq, wk [hs] or null), rotates (inv_freq or null:
+// rope_dims a multiple of 64, split-half pairs) and scales (temp_every > 0), and whose keys and values (v_from_k: the keys as projected) it
+// writes to the pages.
 extern "C" int bn_attn_general_decode(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
                                       const void* v_pages, const int* block_table, int bt_stride, const int* seq_lens, int n_seqs,
                                       int H, int Hkv, int hs, int vd, float scale, const float* dist_a, const float* dist_b,
                                       int sink, const float* sink_values, int window, int keep_first, const void* gate, int gate_stride,
-                                      int n_splits, int chunk, float* part_o, float* part_ml, const int* max_len, hipStream_t s) {
+                                      int n_splits, int chunk, float* part_o, float* part_ml, const int* max_len, int fresh, int v_from_k, const float* wq,
+                                      const float* wk, float eps, const float* inv_freq, int rope_dims, float temp_coef, int temp_every,
+                                      hipStream_t s) {
+    if (fresh && ((((uintptr_t)wq | (uintptr_t)wk | (uintptr_t)inv_freq) & 15) || q_stride < (H + Hkv) * hs + (v_from_k ? 0 : Hkv * vd) || (v_from_k && vd != hs) || (wq == nullptr) != (wk == nullptr) ||
+                  (inv_freq && (rope_dims <= 0 || rope_dims % 64 || rope_dims > hs)))) return BN_ERR_ARG;
     if (n_seqs <= 0 || H <= 0 || Hkv <= 0 || H % Hkv || window < 0 || keep_first < 0 || n_splits < 1 || !bn_attn_general_supports(hs, vd)) return BN_ERR_ARG;
     if (!q || !out || !k_pages || !v_pages || !block_table || !seq_lens || (dist_b && !dist_a)) return BN_ERR_ARG;
     if (q_stride % 8 || out_stride % 4 || (((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages) & 15) || ((uintptr_t)out & 7))
@@ -627,6 +753,9 @@ extern "C" int bn_attn_general_decode(const void* q, int q_stride, void* out, in
     a.max_len = n_splits > 1 ? max_len : nullptr;
     a.q_stride = q_stride; a.out_stride = out_stride; a.bt_stride = bt_stride; a.H = H; a.Hkv = Hkv; a.n_splits = n_splits;
     a.chunk = chunk; a.window = window; a.sink = sink ? 1 : 0; a.sink_values = sink ? sink_values : nullptr; a.scale = scale;
+    a.k_new = fresh ? (bf16*)k_pages : nullptr; a.v_new = fresh ? (bf16*)v_pages : nullptr;
+    a.v_col = (v_from_k ? H : H + Hkv) * hs;
+    a.wq = wq; a.wk = wk; a.eps = eps; a.inv_freq = inv_freq; a.rope_dims = inv_freq ? rope_dims : 0; a.temp_coef = temp_coef; a.temp_every = temp_every;
     const dim3 grid(n_seqs, Hkv * head_tiles, n_splits);
     const long long held = (long long)bt_stride * BN_PAGE, seen = (long long)window + keep_first;     // keys a sequence at the most
     const bool once = head_tiles == 1 && (window > 0 && seen < held ? seen : held) * n_seqs * Hkv * (hs + vd) * 2 <= (long long)AG_ONCE_MB << 20;

@@ -158,6 +158,16 @@ __device__ __forceinline__ float wave_max(float v) {
     return bn_wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
+// sine and cosine of an angle of any size: the angle less the nearest multiple of 2 pi (2 pi as the sum of two floats, the
+// products exact inside the fused operations), then the hardware's functions on what is left, which lies in [-pi, pi]
+__device__ __forceinline__ void bn_sincos(float a, float* sn, float* cs) {
+    const float k = rintf(a * 0.15915494309189535f);
+    float r = fmaf(-k, 6.2831854820251465f, a);
+    r = fmaf(-k, -1.7484555e-7f, r);
+    *sn = __sinf(r);
+    *cs = __cosf(r);
+}
+
 // A thread's sum of squares over its groups of four numbers of a row (k: the group's number): one chain, every rounding written
 // out, so that kernels which norm the same row form the same bits.
 template <typename V> __device__ __forceinline__ float bn_add_squares(float ss, const V& v, int k) {

@@ -46,16 +46,6 @@ struct QkNormArgs {
     int v_from_k;             // the values are the keys as projected (vd == hs; qkv has no value columns)
 };
 
-// sine and cosine of an angle of any size: the angle less the nearest multiple of 2 pi (2 pi as the sum of two floats, the
-// products exact inside the fused operations), then the hardware's functions on what is left, which lies in [-pi, pi]
-__device__ __forceinline__ void qkn_sincos(float a, float* sn, float* cs) {
-    const float k = rintf(a * 0.15915494309189535f);
-    float r = fmaf(-k, 6.2831854820251465f, a);
-    r = fmaf(-k, -1.7484555e-7f, r);
-    *sn = __sinf(r);
-    *cs = __cosf(r);
-}
-
 // a workgroup takes QKN_WAVES heads of one row, a wave each; heads 0 .. H-1 are queries, then Hkv keys, then Hkv values.
 // With norms over the whole projections one workgroup (of up to QKN_MAX_WAVES waves) takes all heads of a row, its waves in turn: the query heads are
 // rewritten in place, so the sums of squares over the whole projections must have been formed (by all threads, in front
@@ -137,7 +127,7 @@ __global__ __launch_bounds__(QKN_MAX_WAVES * BN_WAVE) void qk_norm_store_kernel(
                     const int i = a.rope_interleaved ? (d >> 1) : (d < half ? d : d - half);
                     const bool first = a.rope_interleaved ? !(d & 1) : d < half;
                     float sn, cs;
-                    qkn_sincos((float)pos * a.inv_freq[i], &sn, &cs);
+                    bn_sincos((float)pos * a.inv_freq[i], &sn, &cs);
                     x = first ? x * cs - ps[j] * sn : x * cs + ps[j] * sn;
                 }
                 dst[d] = from_f32<T>(x * temp);

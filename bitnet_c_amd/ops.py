@@ -11,7 +11,7 @@ from __future__ import annotations
 import os
 from ctypes import c_float, c_int, c_longlong, c_void_p
 from dataclasses import dataclass
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -91,7 +91,8 @@ _SIGNATURES = {
                                    c_void_p],
         "bn_attn_general_decode": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int,
                                    c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_int,
-                                   c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
+                                   c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_int,
+                                   c_float, c_int, c_void_p],
     },
     "hyper": {
         "bn_hc_step": [c_int, c_int, c_void_p, c_longlong, c_void_p, c_longlong, c_void_p, c_int, c_longlong, c_void_p, c_void_p,
@@ -534,7 +535,7 @@ def f32_product_takes(w: torch.Tensor) -> bool:
 
 def gemm_mfma(x: torch.Tensor, w: torch.Tensor, out_dtype=None, glu8: bool = False, activation: str = "silu",
               width: int = 0) -> torch.Tensor:
-    """The library-free bf16 product for many rows: y[M, N] = x[M, K] . w[N, K]^T on the matrix cores,
+    """This library's own bf16 product for many rows: y[M, N] = x[M, K] . w[N, K]^T on the matrix cores,
     or with glu8 act(gate) * up for w = gate and up rows interleaved in blocks of 8 ([2N, K]).
     width: the tile's rows of w (256, 192 or 128); 0 lets the kernel pick by the shape."""
     require_gpu()
@@ -769,9 +770,10 @@ def _weight_arg(w: torch.Tensor, streamed: Optional[StreamedWeight], what: str, 
     return t.data_ptr(), t.shape[1], R
 
 
-# bf16 products with many rows: the library's matrix product (as the reference hands its batched
+# Plain bf16 products with many rows: the library's matrix product (as the reference hands its batched
 # products to a library, src/gpu_cuda.cu:11571) unless this is False or BITNET_NO_LIBRARY is set;
-# then this library's own matrix-core kernel (gemm_mfma) does them.
+# then this library's own matrix-core kernel (gemm_mfma) does them, which takes a prompt's gated units, slabs, groups and
+# activations (PROMPT_ROWS) either way.
 LIBRARY_PRODUCTS = os.environ.get("BITNET_NO_LIBRARY", "") in ("", "0")
 
 
@@ -783,7 +785,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, *, allow_library: O
     are not whole 16-byte groups go to the tiled kernel (plain fmaf, a fixed order of summation).
     bf16: up to 16 rows (one MFMA tile of activations) the matrix-core kernel that streams
     the weights once; above that the library's matrix product, which from 32 rows on is about
-    twice as fast as the streaming kernel, with a bf16 or a float32 result (logits).  Without the
+    twice as fast as the streaming kernel, with a bf16 or a float32 result (logits; a plain product: see linear_swiglu, linear_unary,
+    linear_group and linear_split_rows for what a prompt's rows do beside it).  Without the
     library (allow_library False; None follows LIBRARY_PRODUCTS) the streaming kernel takes up to 64
     rows and the tiled matrix-core kernel (gemm_mfma) everything above; shapes that none of them
     takes (rows that are not 16-byte aligned) go to the plain tiled kernel."""
@@ -2079,20 +2082,55 @@ def general_decode_plan(n_seqs: int, H: int, Hkv: int, max_len: int, window: int
     return n_splits, chunk, True
 
 
+class FreshRows(NamedTuple):
+    """What attention_general_decode does to the new rows in qk_norm_store's place: its arguments of these names, pairs split-half."""
+    q_weight: Optional[torch.Tensor] = None
+    k_weight: Optional[torch.Tensor] = None
+    eps: float = 0.0
+    inv_freq: Optional[torch.Tensor] = None
+    rope_dims: int = 0
+    temp_coef: float = 0.0
+    temp_every: int = 0
+    v_from_k: bool = False
+
+
+def takes_fresh_rope(hs: int, rope_dims: int) -> bool:
+    """Whether the decode kernel turns the first rope_dims dimensions of its rows itself: a pair lies whole steps of 32 apart, so that
+    one lane holds both."""
+    return 0 < rope_dims <= hs and rope_dims % 64 == 0
+
+
+def _fresh_args(f: Optional[FreshRows]) -> tuple:
+    if f is None:
+        return 0, 0, None, None, 0.0, None, 0, 0.0, 0
+    ptr = lambda t: t.data_ptr() if t is not None else None
+    return 1, int(f.v_from_k), ptr(f.q_weight), ptr(f.k_weight), float(f.eps), ptr(f.inv_freq), int(f.rope_dims), float(f.temp_coef), int(f.temp_every)
+
+
 def attention_general_decode(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                              block_table: torch.Tensor, seq_lens: torch.Tensor, H: int, Hkv: int, hs: int, v_dim: int, scale: float,
                              *, window: int = 0, n_splits: int = 1, chunk: int = 0, max_len_dev=None, distance_bias=None,
-                             sink: bool = False, keep_first: int = 0, gate=None) -> None:
+                             sink: bool = False, keep_first: int = 0, gate=None, fresh: Optional[FreshRows] = None) -> None:
     """The decode form of attention_general_prompt (bf16, the same head sizes and pages): row b of qkv is sequence b's new
     token, seq_lens [B] its keys in the cache (0: a padding row, whose output is zeros).  A wave takes the heads that share
     a kv head together, so their keys and values are read once.  n_splits > 1 cuts the keys into runs of `chunk` positions
     (a multiple of PAGE; with max_len_dev, a device int32, into runs of split_chunk(longest sequence, n_splits)), merged in
     index order; with a window the runs are counted from the page of the window's first key and need only cover
     window + PAGE positions (kept first keys are the first run's).  distance_bias, sink, keep_first: as attention()'s; gate: as
-    attention_general_prompt's."""
+    attention_general_prompt's.  fresh: qkv's rows are projections on which qk_norm_store has not run; the kernel does its work on
+    the new token of every sequence (position seq_lens - 1) and leaves qkv as it is."""
     require_gpu()
     _dev(qkv, "qkv", torch.bfloat16, 2)
     _dev(out, "out", torch.bfloat16, 2)
+    if fresh is not None:
+        for t, nm, n in ((fresh.q_weight, "q_weight", hs), (fresh.k_weight, "k_weight", hs), (fresh.inv_freq, "inv_freq", fresh.rope_dims // 2)):
+            if t is not None:
+                _dev(t, nm, torch.float32, 1)
+                if t.numel() != n or not t.is_contiguous():
+                    raise KernelError(f"attention_general_decode: {nm} must hold {n} float32 values")
+        if (qkv.shape[1] < (H + Hkv) * hs + (0 if fresh.v_from_k else Hkv * v_dim) or (fresh.v_from_k and v_dim != hs) or (fresh.q_weight is None) != (fresh.k_weight is None)
+                or (fresh.inv_freq is not None and not takes_fresh_rope(hs, fresh.rope_dims))):
+            raise KernelError(f"attention_general_decode: rows {tuple(qkv.shape)}, rotation of {fresh.rope_dims} dimensions do not fit")
     if not attention_general_supported(qkv.dtype, hs, v_dim):
         raise KernelError(f"attention_general_decode: bf16 with head sizes from {_GENERAL_SIZES}, got {hs} and {v_dim}")
     _check_pages(k_pages, v_pages, Hkv, hs, qkv.dtype, True, False, v_dim)
@@ -2128,7 +2166,8 @@ def attention_general_decode(qkv: torch.Tensor, out: torch.Tensor, k_pages: torc
         block_table.data_ptr(), block_table.shape[1], seq_lens.data_ptr(), T, H, Hkv, hs, v_dim, float(scale),
         da, db, *_sink_args(sink, H, "attention_general_decode"), int(window), int(keep_first), gp, gld, int(n_splits), int(chunk), part_o.data_ptr() if part_o is not None else None,
         part_ml.data_ptr() if part_ml is not None else None,
-        max_len_dev.data_ptr() if (max_len_dev is not None and n_splits > 1) else None, _stream()), "attention_general_decode")
+        max_len_dev.data_ptr() if (max_len_dev is not None and n_splits > 1) else None, *_fresh_args(fresh), _stream()),
+        "attention_general_decode")
 
 
 # --------------------------------------------------------------------------------------

@@ -233,25 +233,32 @@ class Attention(Part):
                 qkv = qk
             else:
                 qkv[:, :self.q_dim + self.kv_dim].copy_(qk)
-        ops.qk_norm_store(qkv, ctx.positions, H, Hkv, hs, v_dim=vd, q_weight=self.q_norm, k_weight=self.k_norm,
-                          eps=self.qk_norm_eps or 0.0, temp_coef=self.q_temp_coef, temp_every=self.q_temp_every,
-                          norm_projection=self.norm_projection, inv_freq=self.position.inv_freq,
-                          rope_dims=self.position.rope_dims, rope_interleaved=getattr(self.position, "interleaved", False),
-                          seq_index=ctx.seq_index if kv.writes else None, block_table=kv.block_table if kv.writes else None,
-                          k_pages=kv.k_pages if kv.writes else None, v_pages=kv.v_pages if kv.writes else None,
-                          v_transposed=True, v_from_k=self.value_is_key, bias=self.qk_b, head_temp=self.temp)
+        on_matrix_cores = (ops.attention_general_supported(h.dtype, hs, vd) and ops.GENERAL_PROMPT_ON_MATRIX_CORES
+                           and width % 8 == 0 and qkv.data_ptr() % 16 == 0)
+        pos, fresh = self.position, None
+        if (ctx.is_decode and on_matrix_cores and kv.writes and self.qk_b is None and self.temp is None
+                and not self.norm_projection
+                and (pos.inv_freq is None or (not getattr(pos, "interleaved", False) and ops.takes_fresh_rope(hs, pos.rope_dims)))):
+            fresh = ops.FreshRows(self.q_norm, self.k_norm, self.qk_norm_eps or 0.0, pos.inv_freq,
+                                  pos.rope_dims if pos.inv_freq is not None else 0, self.q_temp_coef, self.q_temp_every, self.value_is_key)
+        else:
+            ops.qk_norm_store(qkv, ctx.positions, H, Hkv, hs, v_dim=vd, q_weight=self.q_norm, k_weight=self.k_norm,
+                              eps=self.qk_norm_eps or 0.0, temp_coef=self.q_temp_coef, temp_every=self.q_temp_every,
+                              norm_projection=self.norm_projection, inv_freq=self.position.inv_freq,
+                              rope_dims=self.position.rope_dims, rope_interleaved=getattr(self.position, "interleaved", False),
+                              seq_index=ctx.seq_index if kv.writes else None, block_table=kv.block_table if kv.writes else None,
+                              k_pages=kv.k_pages if kv.writes else None, v_pages=kv.v_pages if kv.writes else None,
+                              v_transposed=True, v_from_k=self.value_is_key, bias=self.qk_b, head_temp=self.temp)
         out = torch.empty((h.shape[0], H * vd), dtype=h.dtype, device=h.device)
         bias = (self.dist_a, self.dist_b) if self.dist_a is not None else None
         gate = qkv[:, width - H * vd:] if self.out_gate else None
         mask = dict(window=self.window, keep_first=self.keep_first)
-        on_matrix_cores = (ops.attention_general_supported(h.dtype, hs, vd) and ops.GENERAL_PROMPT_ON_MATRIX_CORES
-                           and width % 8 == 0 and qkv.data_ptr() % 16 == 0)
         if ctx.is_decode and on_matrix_cores:
             n_splits, chunk, follows = ops.general_decode_plan(ctx.n_rows, H, Hkv, kv.max_len, self.window)
             ops.attention_general_decode(qkv, out, kv.k_pages, kv.v_pages, kv.block_table, ctx.seq_lens, H, Hkv, hs, vd, self.scale,
                                          n_splits=n_splits, chunk=chunk,
                                          max_len_dev=ctx.max_len_dev if follows and n_splits > 1 else None,
-                                         distance_bias=bias, sink=self._sink(), gate=gate, **mask)
+                                         distance_bias=bias, sink=self._sink(), gate=gate, fresh=fresh, **mask)
         elif ctx.is_decode:
             if not self.window:
                 n_splits, chunk = ops.decode_splits(ctx.n_rows, H, Hkv, kv.max_len, h.dtype, target_wgs=ops.VECTOR_DECODE_TARGET_WGS)

@@ -72,7 +72,7 @@ class Linear:
     def lazy(self, x: torch.Tensor):
         """The product in the form in which it reaches a residual stream cheapest (no bias): a LazyDelta at
         decode sizes, where it can add itself to the stream; in bf16 partial sums over ranges of K (ops.PartialSums), which the
-        kernel of the next norm adds up, where ops.can_split_sums says so; else its result."""
+        kernel of the next norm adds up, where ops.can_split_sums or, for a prompt's rows, ops.can_split_rows says so; else its result."""
         from .base import LazyDelta
         M, (N, K) = x.shape[0], self.weight.shape
         plain = (self.bias is None and x.dim() == 2 and x.dtype == torch.bfloat16 and self.weight.dtype == torch.bfloat16
