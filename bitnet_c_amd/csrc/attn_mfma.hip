@@ -1552,10 +1552,20 @@ extern "C" int bn_attn_mfma(const void* q, int q_stride, void* out, int out_stri
                             const int* tiles, int n_tiles, int n_tokens, int H, int Hkv, int hs, int GT,
                             int window, float scale, int n_splits, int chunk, float* part_o, float* part_ml,
                             const float* inv_freq, int rotate, int write_kv, const int* by_length,
-                            const int* max_len, int n_seqs, hipStream_t s) {
+                            const int* max_len, hipStream_t s) {
     return attn_mfma_launch(q, q_stride, out, out_stride, k_pages, vt_pages, block_table, bt_stride, seq_lens, tiles, n_tiles,
                             n_tokens, H, Hkv, hs, GT, window, scale, n_splits, chunk, part_o, part_ml, inv_freq, rotate,
-                            write_kv, by_length, max_len, nullptr, 0, 0, 0.f, n_seqs, s);
+                            write_kv, by_length, max_len, nullptr, 0, 0, 0.f, 1, s);
+}
+
+// the prompt form by a caller who knows how many sequences the tiles are of (above: one): the choice among its kernels asks for it
+extern "C" int bn_attn_mfma_prompt(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
+                                   const void* vt_pages, const int* block_table, int bt_stride, const int* tiles, int n_tiles,
+                                   int n_tokens, int H, int Hkv, int hs, int GT, int window, float scale, int n_seqs, hipStream_t s) {
+    if (!tiles) return BN_ERR_ARG;
+    return attn_mfma_launch(q, q_stride, out, out_stride, k_pages, vt_pages, block_table, bt_stride, nullptr, tiles, n_tiles,
+                            n_tokens, H, Hkv, hs, GT, window, scale, 1, 0, nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr,
+                            nullptr, 0, 0, 0.f, n_seqs, s);
 }
 
 // The decode form (tiles none, rotate on) over rows whose RMSNorm was left undone: q, the new key and the new value of
@@ -1618,5 +1628,5 @@ extern "C" int bn_attn_mfma_decode_static(const void* q, int q_stride, void* out
     }
     return bn_attn_mfma(q, q_stride, out, out_stride, k_pages, vt_pages, block_table, bt_stride, seq_lens, nullptr,
                         n_seqs, n_seqs, H, Hkv, hs, GT, window, scale, n_splits, chunk, part_o, part_ml, inv_freq, rotate,
-                        write_kv, by_length, nullptr, n_seqs, s);
+                        write_kv, by_length, nullptr, s);
 }

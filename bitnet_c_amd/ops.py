@@ -168,7 +168,9 @@ _SIGNATURES = {
                                 c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
         "bn_attn_mfma": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                          c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p,
-                         c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p],
+                         c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p],
+        "bn_attn_mfma_prompt": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int,
+                                c_int, c_int, c_int, c_int, c_float, c_int, c_void_p],
     },
     "attn_f32": {
         "bn_attn_f32_supports": [c_int],
@@ -1915,6 +1917,12 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
             max_len_dev.data_ptr() if max_len_dev is not None else None, row_scale.slots.data_ptr(),
             row_scale.slots.shape[1], row_scale.stream.shape[1], float(row_scale.eps), _stream()), "attention(mfma, scaled)")
         return
+    if use_mfma and not decode and n_splits == 1:
+        _check(_fn("attn_mfma", "bn_attn_mfma_prompt")(
+            qkv.data_ptr(), _rows(qkv, "qkv"), out.data_ptr(), H * hs, k_pages.data_ptr(), v_pages.data_ptr(), block_table.data_ptr(),
+            block_table.shape[1], tl, n_tiles, T, H, Hkv, hs, GT, int(window), float(scale), block_table.shape[0], _stream()),
+            "attention(mfma, prompt)")
+        return
     if use_mfma:
         _check(_fn("attn_mfma", "bn_attn_mfma")(
             qkv.data_ptr(), _rows(qkv, "qkv"), out.data_ptr(), H * hs, k_pages.data_ptr(), v_pages.data_ptr(),
@@ -1922,8 +1930,7 @@ def attention(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pag
             float(scale), int(n_splits), int(chunk), po, pm,
             fused_rotate.data_ptr() if fused_rotate is not None else None, int(fused_rotate is not None),
             int(bool(fused_write)), by_length.data_ptr() if by_length is not None else None,
-            max_len_dev.data_ptr() if max_len_dev is not None else None, block_table.shape[0], _stream()),
-            "attention(mfma)")
+            max_len_dev.data_ptr() if max_len_dev is not None else None, _stream()), "attention(mfma)")
         return
     if f32_plain:
         _check(_fn("attn_f32", "bn_attn_f32")(
