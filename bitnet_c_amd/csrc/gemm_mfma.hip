@@ -1,8 +1,9 @@
 // Prompt-phase matrix product for bf16 on the matrix cores: Y[M, N] = X[M, K] . W[N, K]^T for many
-// rows of activations, with float32 accumulation and a bf16 or float32 result.  It is the
-// library-free form of the reference's batched products (src/gpu_cuda.cu:11571 hands them to a
+// rows of activations, with float32 accumulation and a bf16 or float32 result.  It has the place of
+// the reference's batched products (src/gpu_cuda.cu:11571 hands them to a
 // library; its own tiled kernels are src/gpu_cuda.cu:4012-4170), written for 64-wide waves and
-// v_mfma_f32_16x16x32_bf16.
+// v_mfma_f32_16x16x32_bf16.  Two kernels: gemm_turns_kernel (below) where K is whole steps of 64 and rows
+// of Y whole groups of four, which is what a model's prompt has; gemm_mfma_kernel for everything else:
 //
 // A workgroup of eight waves (2 x 4, two waves on every SIMD so that one multiplies while the other
 // waits for shared memory) owns a tile of 256 rows of X by BN (256, 192 or 128) rows of W and
