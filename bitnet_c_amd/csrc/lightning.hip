@@ -595,7 +595,8 @@ __device__ __forceinline__ void lb_settle(f32x4& x) {
 }
 
 // z / (1 + exp(-z)) for a z of eight bits: z times the upper sixteen bits of log2 e is exact, the rest of the exponent a factor near 1, the reciprocal
-// refined once.  Ten instructions for some 35 of the library's exponential and quotient, which were half of a block's time.
+// refined once.  Twelve instructions for some 35 of the library's exponential and quotient, which were half of a block's time.  Below -87, where the value is
+// nearer to zero than -1.5e-36, the factor is 0: -0 for a finite z, NaN for an infinity, as the quotient gives (which is -0 from -88.8 on).
 __device__ __forceinline__ float lb_act(bf16 x, int silu) {
     const float z = to_f32(x);
     if (!silu) return z;
@@ -604,7 +605,7 @@ __device__ __forceinline__ float lb_act(bf16 x, int silu) {
     const float d = 1.f + fmaf(p, c * -4.8884952e-6f, p);
     float r = __builtin_amdgcn_rcpf(d);
     r = fmaf(fmaf(-d, r, 1.f), r, r);
-    return z * r;
+    return z * (z >= -87.f ? r : 0.f);
 }
 
 // RT: row tiles of 16 key rows (the key width rounded up to 64 or 128); NCT: column tiles of 16 of a wave

@@ -75,6 +75,26 @@ def test_numbers_that_are_none_reach_no_token_before_them(pieces):
     assert torch.equal(run(), clean)
 
 
+@pytest.mark.parametrize("pieces", [False, True])
+def test_silu_of_every_number_there_is(pieces):
+    """A token whose values are all 2^16 numbers of bf16, infinities and NaN among them, a column each; beside the walk token by token and float64."""
+    from bitnet_c_amd import ops
+    H, dk, dv = 64, 8, 1024
+    v = torch.arange(-2 ** 15, 2 ** 15, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    x = torch.cat([torch.ones(2 * H * dk, dtype=torch.bfloat16), v]).view(1, -1)
+    tiles, slots = torch.tensor([(0, 0, 1, 0)], dtype=torch.int32).cuda(), torch.zeros(1, dtype=torch.int32).cuda()
+    run = lambda **kw: ops.lightning_scan(x.cuda(), 0, H * dk, 2 * H * dk, torch.full((H,), 0.5).cuda(), torch.zeros(1, H * dk * dv).cuda(), slots, H, dk, dv,
+                                          tiles=tiles, silu=True, k_scale=0.125, **kw).cpu().view(-1).double()
+    got, chain = run(chain=False, pieces=pieces), run(chain=True)
+    one = torch.sigmoid(torch.ones((), dtype=torch.float64))
+    want = v.double() * torch.sigmoid(v.double()) * (one * one)         # k . q = 8 (silu 1)^2 / 8
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    for other in (want, chain):
+        ok = v.isfinite()
+        # a dozen roundings of factors near 1, two of exponents of up to 126; below -87 a value is given as 0
+        assert bool(((got - other).abs()[ok] <= 64 * 2.0 ** -24 * other.abs()[ok] + 1.5e-36).all())
+
+
 def test_which_steps_take_blocks():
     from bitnet_c_amd import ops
     assert ops.lightning_in_blocks((16, 1), 16, 128, 128) and ops.lightning_in_blocks((2048, 64), 16, 128, 128) and not ops.lightning_in_blocks((1984, 64), 16, 128, 128)
