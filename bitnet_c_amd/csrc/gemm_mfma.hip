@@ -360,8 +360,14 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
     const int i = lane & 15, g = lane >> 4;
     const int wr = wave >> 2, wc = wave & 3;
 
+    // The experts' list holds its tiles in front, and the runs are cut from those: cut from all that the grid is for, the last XCDs' would be empty
+    // (both products and what stands around them, us, in gemm_mfma_kernel / runs of all / of those with the width that is now taken, 16 experts of 5,632 x 2,048, two a token: 17 tokens
+    // 210 / 236 / 189, 512 239 / 290 / 220, 1,000 277 / 392 / 265, 4,096 723 / 673 / 612; 64 gated ones of 1,536 x 4,096, six a token: 64 tokens 673 / 649 /
+    // 529, 2,048 862 / 989 / 755)
+    if (EPI == GM_GROUPED) tiles_m = grp.n_tiles[0];
     const int mn = tiles_m * tiles_n, total = mn * splits;
     const int xcd = blockIdx.x % GM_XCDS, local = blockIdx.x / GM_XCDS;
+    if (EPI == GM_GROUPED && local >= total / GM_XCDS + (xcd < total % GM_XCDS)) return;
     int id = xcd * (total / GM_XCDS) + min(xcd, total % GM_XCDS) + local;
     const int sp = id / mn;
     id -= sp * mn;
@@ -369,7 +375,6 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
     const int tm = band * GM_BAND + in % high, n0 = in / high * BN;
     int m0 = tm * BM;
     if (EPI == GM_GROUPED) {                             // the tile's rows end where its matrix's rows end
-        if (tm >= grp.n_tiles[0]) return;
         const int* tl = grp.tiles + 3 * tm;
         W += (size_t)tl[0] * grp.w_stride;
         m0 = tl[1];
@@ -618,19 +623,20 @@ static const GmTile gm_tiles[] = {{256, 256, 1.46, 0.}, {192, 256, 1.17, 0.}, {1
 #define GM_IDLE 0.68
 #define GM_MAX_SPLITS 6
 
-static double gm_cost(const GmTile& t, long long tiles, int steps, int cus) {
-    auto round = [&](double step, double fill) { return GM_ROUND + steps * step * (GM_IDLE + (1. - GM_IDLE) * fill); };
+static double gm_cost(const GmTile& t, long long tiles, int steps, int cus, double start) {
+    auto round = [&](double step, double fill) { return start + steps * step * (GM_IDLE + (1. - GM_IDLE) * fill); };
     if (t.two > 0.) {                                    // two a CU run on without rounds
         if (tiles <= cus) return round(t.one, (double)tiles / cus);
         if (tiles <= 2 * cus) return round(t.two, tiles / (2. * cus));
-        return 2 * GM_ROUND + steps * t.two * tiles / (2. * cus);
+        return 2 * start + steps * t.two * tiles / (2. * cus);
     }
     return tiles / cus * round(t.one, 1.) + (tiles % cus ? round(t.one, (double)(tiles % cus) / cus) : 0.);
 }
 
 // The tile and the ranges of K (up to max_splits) that take the least time for M rows, N rows of W and K columns; slabs are written and
-// read again at 5 TB/s, and more than two of them cost a launch.  bm: the only height to look at, or 0.
-static void gm_plan(int M, int N, int K, int bm, int max_splits, int* tile, int* splits, int items = 1) {
+// read again at 5 TB/s, and more than two of them cost a launch.  bm: the only height to look at, or 0.  cold: what a round costs besides for
+// every 256 of its tiles' columns.
+static void gm_plan(int M, int N, int K, int bm, int max_splits, int* tile, int* splits, int items = 1, double cold = 0.) {
     const int cus = gm_compute_units(), steps = K / GM_BK;
     double best = -1.;
     for (int i = 0; i < GM_TILES; ++i) {
@@ -640,7 +646,7 @@ static void gm_plan(int M, int N, int K, int bm, int max_splits, int* tile, int*
         for (int s = 1; s <= max_splits; ++s) {
             const int per = (steps + s - 1) / s;
             if ((steps + per - 1) / per != s) continue;
-            const double cost = gm_cost(t, tiles * s, per, cus) + (s > 1 ? s * 8e-6 * M * N / 5. + (s > 2 ? 4. : 0.) : 0.);
+            const double cost = gm_cost(t, tiles * s, per, cus, GM_ROUND + cold * t.bn / 256) + (s > 1 ? s * 8e-6 * M * N / 5. + (s > 2 ? 4. : 0.) : 0.);
             if (best < 0. || cost < best) { best = cost; *tile = i; *splits = s; }
         }
     }
@@ -796,8 +802,14 @@ extern "C" int bn_gemm_mfma_grouped(int out_dtype, const void* X, const void* W,
     g.unary = unary < 0 ? -1 : unary;
     const bool f32 = out_dtype == BN_DT_F32;
     if (gm_turns_takes(N, K, ldx, ldw, ldy, Y, f32 ? 4 : 2)) {
+        // Tiles that hold rows, if the rows are spread evenly over the matrices (a tenth of a tile more makes no other); a tile of an expert's matrix is
+        // read from memory and by few others, so that a round starts later.  us, the width by rows / 256 tiles and a round as above -> this, 16 experts of
+        // 5,632 x 2,048, two a token: 1,000 tokens 291 -> 265, 1,600 314 -> 287, 2,048 383 -> 398; of 2 x 5,504 x 4,096 200 569 -> 493
+        // (with the number of tiles known the width is within 5 % of the better of the two everywhere, so within 16 %).
+        const int full = (rows + GM_BM - 1) / GM_BM, matrices = max_tiles - full;
+        const int live = matrices < 1 ? full : std::min(max_tiles, matrices * std::max(1, (rows / matrices - GM_BM / 10 + GM_BM - 1) / GM_BM));
         int tile = 0, splits = 1;
-        gm_plan(rows, N, K, GM_BM, 1, &tile, &splits);
+        gm_plan(live * GM_BM, N, K, GM_BM, 1, &tile, &splits, 1, 17.);
         return f32 ? gm_turns<GM_GROUPED, float>(tile, X, W, Y, rows, N, K, ldx, ldw, ldy, 1, 0, s, g, max_tiles)
                    : gm_turns<GM_GROUPED, bf16>(tile, X, W, Y, rows, N, K, ldx, ldw, ldy, 1, 0, s, g, max_tiles);
     }

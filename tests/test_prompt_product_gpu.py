@@ -110,6 +110,28 @@ def test_activations_on_the_sums(M, N, K, act):
     assert _rel(got[M - 2], large) < 2.0 ** -8 and _rel(got[:M - 2], want[:M - 2]) < 2.0 ** -8
 
 
+# experts whose lists hold more tiles than rows fill: one live tile, numbers of them that are no multiple of the XCDs, every tile live; some experts without rows
+@pytest.mark.parametrize("E,D,F,T,used", [(64, 64, 640, 17, 1), (16, 192, 1096, 40, 3), (8, 320, 576, 300, 8), (5, 128, 4168, 700, 2), (2, 576, 2056, 1024, 2)])
+def test_experts_whose_lists_are_not_full(E, D, F, T, used):
+    ops = _ops()
+    g = torch.Generator(device="cuda").manual_seed(E + D + F + T)
+    h = torch.randn(T, D, generator=g, device="cuda").to(torch.bfloat16)
+    up = (torch.randn(E, F, D, generator=g, device="cuda") / D ** 0.5).to(torch.bfloat16)
+    down = (torch.randn(E, D, F, generator=g, device="cuda") / F ** 0.5).to(torch.bfloat16)
+    names = torch.randperm(E, generator=torch.Generator().manual_seed(T))[:used].int()
+    ids = names[torch.randint(0, used, (T, 1), generator=torch.Generator().manual_seed(D))].cuda()
+    ids[:used, 0] = names.cuda()
+    wts = torch.rand(T, 1, generator=g, device="cuda") + 0.5
+    y = ops.moe_experts_grouped(h, up, down, ids, wts, "relu2", False).slabs[0]
+    for e in names.tolist():
+        rows = (ids[:, 0] == e).nonzero().view(-1)
+        mid = ((h[rows].double() @ up[e].double().t()).clamp(min=0) ** 2).to(torch.bfloat16).double()
+        want = wts[rows].double() * (mid @ down[e].double().t())
+        off = (y[rows].double() - want).norm(dim=1) / want.norm(dim=1)
+        # most rows: float32 sums; a few: a term of the middle whose float32 sum is rounded to the neighbouring bf16 number, 2^-8 of that term
+        assert float(off.median()) < 1e-6 and float(off.max()) < 2.0 ** -8
+
+
 def test_numbers_that_are_none():
     """A row of X or of W that holds NaN or an infinity reaches its own results alone."""
     ops = _ops()
