@@ -570,12 +570,14 @@ def gemm_mfma_supported(M: int, N: int, K: int, ldx: int, ldw: int) -> bool:
 GEMM_STEP = _build.header_constant("GM_BK", "gemm_mfma.hip")      # K in whole steps of this: the prompt product's faster form
 # Prompt products that are this library's own beside the library's: from this many rows on (fewer: the kernels of a decode step) ...
 PROMPT_ROWS = 129
-# ... a part's last product, as slabs over ranges of K where its tiles would leave half of the CUs without work and K is long enough for
-# the slabs' way through memory not to count.  us with the kernels of the next norm, the library's product -> slabs: 4,096 x 14,336 at 129 /
-# 256 / 576 / 1,024 / 2,048 rows 67 -> 46, 69 -> 57, 121 -> 79, 141 -> 118, 227 -> 195 (2,560: 252 -> 275); 5,120 x 13,824 at 512 / 1,536 (1,792)
-# 122 -> 84, 206 -> 181 (232 -> 255); 8,192 x 28,672 at 256 / 1,024 (1,280) 328 -> 157, 394 -> 361 (469 -> 507); 4,096 x 11,008 at 640 / 2,048
-# (2,560) 96 -> 87, 176 -> 160 (201 -> 220); 2,048 x 8,192 at 384 / 1,280 (2,048) 31 -> 29, 60 -> 54 (75 -> 78); 2,048 x 5,632 at 512 / 1,024
-# 26 -> 28, 40 -> 38: not worth it, 4,096 x 4,096 at 256 / 1,024 25 -> 29, 46 -> 52.
+# ... a part's last product, as slabs over ranges of K, where K is long enough for the slabs' way through memory not to count, its tiles leave
+# half of the CUs without work, and the kernel's plan, which weighs the rounds of tiles against the slabs' bytes, finds ranges that pay (in one
+# range the library's product is the faster one by 2 to 9 %).  us with the kernel of the next norm, the library's product -> slabs: 4,096 x 14,336 at
+# 129 / 256 / 576 / 1,024 / 2,048 rows 67 -> 46, 69 -> 57, 121 -> 79, 141 -> 118, 227 -> 195; 5,120 x 13,824 at 512 / 1,536 (1,792) 120 -> 80, 208 -> 183
+# (239 -> 245); 8,192 x 28,672 at 256 / 640 / 1,024 (1,280) 323 -> 163, 286 -> 290, 400 -> 361 (487 -> 501); 4,096 x 11,008 at 640 / 2,048 (2,560) 93 -> 81, 182 -> 156
+# (203 -> 213); 4,096 x 9,216 at 512 / 1,792 (2,048) 69 -> 52, 139 -> 127 (149 -> 156); 2,048 x 8,256 at 384 / 1,280 / 2,560 (3,072) 48 -> 29, 80 -> 60, 99 ->
+# 91 (110 -> 113); 2,048 x 8,192 at 384 / 1,280 / 2,048 / 2,560 (3,072) 37 -> 30, 68 -> 59, 81 -> 78, 94 -> 88 (106 -> 112); 5,120 x 8,192 at 1,280 (1,536) 116 -> 108
+# (130 -> 139).  Shorter K: 2,048 x 5,632 at 512 / 1,024 26 -> 28, 40 -> 38, 4,096 x 4,096 at 256 / 1,024 25 -> 29, 46 -> 52.
 SPLIT_ROWS_MIN_K = 8192
 ROW_SLABS = 24576         # numbers of a row's slabs together that one workgroup of a prompt step adds up
 
@@ -584,8 +586,7 @@ def can_split_rows(M: int, N: int, K: int, dtype) -> bool:
     """Whether a product of a prompt's rows whose result goes to the residual stream is left as slabs of sums (linear_split_rows)."""
     if not (SPLIT_SUMS and dtype == torch.bfloat16 and M >= PROMPT_ROWS and K >= SPLIT_ROWS_MIN_K and K % GEMM_STEP == 0 and N % 4 == 0):
         return False
-    tiles = -(-M // 256) * -(-N // 256)
-    return tiles * 2 <= _compute_units() and (K > SPLIT_ROWS_MIN_K or tiles * 16 <= 3 * _compute_units())
+    return -(-M // 256) * -(-N // 256) * 2 <= _compute_units() and _fn("gemm_mfma", "bn_gemm_mfma_splits")(M, N, K) > 1
 
 
 # ... products of the same sizes that do not depend on each other (linear_group), in one launch: alone each leaves CUs without work or ends

@@ -160,3 +160,14 @@ def test_what_the_rules_say():
     assert not ops.group_rows(4, 512, 2048, 2080) and not ops.group_rows(4, 512, 2046, 2048) and not ops.group_rows(1, 2048, 512, 512)
     with pytest.raises(ops.KernelError):
         ops.linear_split_rows(torch.zeros(130, 96, dtype=bf, device="cuda"), torch.zeros(64, 96, dtype=bf, device="cuda"))
+
+
+def test_slabs_are_left_where_ranges_pay():
+    """The rule goes by the plan's ranges on both sides of any K, the shortest as well."""
+    ops = _ops()
+    for K in (8192, 8256, 8704):
+        assert ops.can_split_rows(2048, 2048, K, torch.bfloat16) and ops.can_split_rows(1280, 4096, K, torch.bfloat16)
+        assert not ops.can_split_rows(4096, 2048, K, torch.bfloat16) and not ops.can_split_rows(2048, 4096, K, torch.bfloat16)
+    for M, N, K in ((2048, 2048, 8192), (3072, 2048, 8192), (3072, 2048, 8256), (4096, 2048, 10240), (2048, 4096, 9216), (2048, 4096, 10240), (1024, 8192, 9216)):
+        assert ops.can_split_rows(M, N, K, torch.bfloat16) == (ops._fn("gemm_mfma", "bn_gemm_mfma_splits")(M, N, K) > 1)
+    assert not ops.can_split_rows(2048, 2048, 8192 - 64, torch.bfloat16)
