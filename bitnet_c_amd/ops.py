@@ -2108,6 +2108,12 @@ def takes_fresh_rope(hs: int, rope_dims: int) -> bool:
     return 0 < rope_dims <= hs and rope_dims % 64 == 0
 
 
+def on_16_bytes(*tensors) -> bool:
+    """Whether what there is of the tensors begins on 16 bytes (the decode kernel reads a norm's weights and the rotation's frequencies in
+    such groups; qk_norm_store reads them number by number)."""
+    return all(t is None or t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def _fresh_args(f: Optional[FreshRows]) -> tuple:
     if f is None:
         return 0, 0, None, None, 0.0, None, 0, 0.0, 0

@@ -209,9 +209,9 @@ class Attention(Part):
         return (self.qkv, self.o) if self.general and self.qkv.bias is None and self.o.bias is None else None
 
     def _forward_general(self, h, ctx, kv, lazy_ok: bool = False, projected=None):
-        """Projections; biases, norms, rotation and temperature with the cache write (one kernel); attention with its window,
-        distance bias, sink and output gate (prompt steps on the matrix cores where the sizes allow, else the vector kernel); the
-        output projection."""
+        """Projections; biases, norms, rotation and temperature with the cache write (one kernel, or, in a bf16 decode step without a bias
+        or head temperatures, the work of the attention kernel itself: ops.FreshRows); attention with its window, distance bias, sink
+        and output gate (on the matrix cores where the sizes allow, else the vector kernel); the output projection."""
         H, Hkv, hs, vd = self.H, self.Hkv, self.hs, self.vd
         if projected is None and isinstance(h, ops.DeferredNorm) and not (isinstance(h, ops.StreamNorm) and (kv.writes or self.out_gate)):
             h = h.materialize()               # (a StreamNorm is the first product's alone)
@@ -237,7 +237,7 @@ class Attention(Part):
                            and width % 8 == 0 and qkv.data_ptr() % 16 == 0)
         pos, fresh = self.position, None
         if (ctx.is_decode and on_matrix_cores and kv.writes and self.qk_b is None and self.temp is None
-                and not self.norm_projection
+                and not self.norm_projection and ops.on_16_bytes(self.q_norm, self.k_norm, pos.inv_freq)
                 and (pos.inv_freq is None or (not getattr(pos, "interleaved", False) and ops.takes_fresh_rope(hs, pos.rope_dims)))):
             fresh = ops.FreshRows(self.q_norm, self.k_norm, self.qk_norm_eps or 0.0, pos.inv_freq,
                                   pos.rope_dims if pos.inv_freq is not None else 0, self.q_temp_coef, self.q_temp_every, self.value_is_key)

@@ -85,3 +85,34 @@ def test_what_is_refused():
                          (ops.FreshRows(q_weight=torch.ones(128, device="cuda")), 768), (ops.FreshRows(inv_freq=_freq(64), rope_dims=128), 768)):
         with pytest.raises(ops.KernelError):
             run(fresh, width)
+
+
+def test_norms_that_lie_anywhere():
+    """A layer whose norms are pieces of one tensor, on no 16 bytes, decodes as before: through qk_norm_store."""
+    from bitnet_c_amd.cache import PagedCache
+    from bitnet_c_amd.parts import MIXERS, PartSpec
+    from test_parts_gpu import _ctx
+    H, G, hs, hidden, bf = 4, 2, 64, 64, torch.bfloat16
+    gen = torch.Generator().manual_seed(3)
+    steps = [torch.randn(n, hidden, generator=gen).to(bf).cuda() for n in (70, 1, 1)]
+    results, weights = [], None
+    for shift in (0, 1):
+        att = MIXERS.build(PartSpec.of("attention", hidden=hidden, n_heads=H, n_kv_heads=G, head_dim=hs, scale=hs ** -0.5, position=PartSpec.of("none"),
+                                       qk_norm_eps=1e-6))
+        weights = weights or {k: torch.randn(v.shape, generator=gen) * 0.2 + (k in ("q_norm", "k_norm")) for k, v in att.tensors().items()}
+        norms = torch.zeros(2 * hs + 4, device="cuda")
+        tensors = dict(weights, q_norm=norms[shift:shift + hs], k_norm=norms[hs + shift:2 * hs + shift])
+        for k in ("q_norm", "k_norm"):
+            tensors[k].copy_(weights[k])
+        att.load(tensors, "cuda", bf)
+        assert att.q_norm.data_ptr() % 16 == 4 * shift
+        cache = PagedCache([att.cache_need()], [None], 64 * 8, dtype=bf, device="cuda")
+        slot, out = cache.alloc_slot(), []
+        for x in steps:
+            ctx, tables, longest = _ctx(cache, [slot], [x.shape[0]], bf)
+            out.append(att.forward(x, ctx, cache.view(0, tables, longest)))
+            cache.commit([slot], [x.shape[0]])
+        results.append(torch.cat(out))
+    a, b = (r.double() for r in results)
+    assert torch.equal(a[:70], b[:70])                    # prompts go one way
+    assert float((a - b).norm()) <= 2.0 ** -7 * float(a.norm())        # a norm's sum in another order, then two roundings to bf16
