@@ -322,11 +322,12 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_mfma_kernel(const bf16* __res
 // instruction cache (28,672 x 4,096 with its gated unit at 2,048 rows 366 us, with every activation in one kernel 395).
 #define GM_STORE 0                    // stored (TO)
 #define GM_SILU 1                     // silu(gate) * up
-#define GM_GATED 2                    // act(gate) * up, the other activations
+#define GM_GATED_GELU 2               // gelu(gate) * up, the tanh form
 #define GM_GROUPED 3                  // the grouped form's
 #define GM_ITEMS 4                    // stored, of several products of the same sizes (in the ranges' place)
 #define GM_GELU_ERF 5                 // gelu(sum), the exact one
 #define GM_RELU2 6                    // max(sum, 0)^2
+#define GM_GATED_RELU2 7              // max(gate, 0)^2 * up
 
 // z (1 + erf(z / sqrt 2)) / 2 in 17 instructions (erff's alone are 40, with a branch): with x = |z| / sqrt 2 and t = 1 / (1 + 0.46 x),
 // erfc(x) / 2 = t 2^(p(t) - x^2 / ln 2), p the polynomial of degree 7 that interpolates log2(exp(x^2) erfc(x) / (2 t)) at the Chebyshev
@@ -345,10 +346,21 @@ __device__ __forceinline__ float gm_gelu_erf(float z) {
     return z * (z < 0.f ? h : 1.0f - h);
 }
 
+// The gated units' activations, with the hardware's exp2 and reciprocal (an ulp each): z / (1 + exp(-z)), and z (1 + tanh(y)) / 2 with
+// y = sqrt(2 / pi) (z + 0.044715 z^3) as z / (1 + exp(-2 y)), which is the same and has no difference of numbers near 1 in it.  (One kernel for both and
+// relu2 with the library's functions: 16,384 x 2,048 at 129 / 2,048 / 8,192 rows with gelu 26 / 143 / 549 us, with relu2 23 / 132 / 511; the library's product
+// and the unit's kernel 26 / 118 / 479 and 25 / 117 / 462; this 25 / 109 / 422 and 25 / 106 / 407.)
+template <int EPI> __device__ __forceinline__ float gm_gate(float z) {
+    if (EPI == GM_SILU) return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * z));
+    if (EPI == GM_GATED_GELU) return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-z * fmaf(0.10294324f, z * z, 2.3022082f)));
+    const float p = fmaxf(z, 0.f);
+    return p * p;
+}
+
 template <int BM, int BN, int EPI, typename TO>
 __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, TO* __restrict__ Y, int M,
                                                             int N, int K, int ldx, int ldw, int ldy, int tiles_m, int tiles_n, int splits,
-                                                            int steps_per, int act, GmGroups grp) {
+                                                            int steps_per, GmGroups grp) {
     constexpr int WM = BM / 2, WN = BN / 4;              // a wave's part of the tile, taken in quarters of (16 MH) x (16 NH)
     constexpr int MH = WM / 32, NH = WN / 32;
     constexpr int XL = (BM / 2 + 63) / 64, WL = BN / 128;        // loads of a wave for a part: 8 rows each
@@ -493,7 +505,8 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
         }
     };
     if (EPI == GM_STORE) Y += (size_t)sp * M * ldy;
-    if constexpr (sizeof(TO) == 2 && EPI != GM_SILU && EPI != GM_GATED && EPI != GM_GROUPED) {
+    constexpr bool GATED = EPI == GM_SILU || EPI == GM_GATED_GELU || EPI == GM_GATED_RELU2;
+    if constexpr (sizeof(TO) == 2 && !GATED && EPI != GM_GROUPED) {
         // bf16 rows go out through shared memory, which nobody reads any more: a wave's part of the tile is written to a buffer of its
         // own, the 16-byte chunks of a row swizzled, and read back row by row, so that a store writes whole rows of 128 bytes and not 32
         // bytes of sixteen (8,192 x 2,048 at 2,048 / 8,192 rows 65.8 -> 52.6, 244 -> 207 us: rows of Y a power of two apart share a
@@ -548,15 +561,14 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
                 for (int b = 0; b < MH; ++b) {
                     const int m = m0 + wr * WM + u * (WM / 2) + b * 16 + i, n = n0 + wc * WN + v * (WN / 2) + a * 16;
                     f32x4 c = acc[u][v][a][b];
-                    if (EPI == GM_SILU || EPI == GM_GATED) {
+                    if (GATED) {
                         // rows n .. n + 7 of W are gates, n + 8 .. n + 15 the ups of the same columns: the lanes with g >= 2 hold the ups
-                        // of what the lanes with g - 2 hold the gates of.  silu with the hardware's exp2 and reciprocal (an ulp each)
+                        // of what the lanes with g - 2 hold the gates of
                         f32x4 up;
 #pragma unroll
                         for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(c[r], 32, BN_WAVE);
 #pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            c[r] = (EPI == GM_SILU ? c[r] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * c[r])) : bn_gate_act(c[r], act)) * up[r];
+                        for (int r = 0; r < 4; ++r) c[r] = gm_gate<EPI>(c[r]) * up[r];
                         if (g < 2 && m < M && n < N) store(Y + (size_t)m * ldy + (n >> 1) + 4 * g, c);
                     } else if (m < M && n + 4 * g < N) {
                         size_t mo = m;
@@ -658,21 +670,21 @@ static bool gm_turns_takes(int N, int K, int ldx, int ldw, int ldy, const void* 
 }
 
 template <int BM, int BN, int EPI, typename TO>
-static int gm_turns_launch(const void* X, const void* W, void* Y, int M, int N, int K, int ldx, int ldw, int ldy, int splits, int act, hipStream_t s,
+static int gm_turns_launch(const void* X, const void* W, void* Y, int M, int N, int K, int ldx, int ldw, int ldy, int splits, hipStream_t s,
                            const GmGroups& grp, int max_tiles) {
     const int tiles_m = EPI == GM_GROUPED ? max_tiles : (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     const long long grid = (long long)tiles_m * tiles_n * splits;
     if (grid > 0x7fffffffLL) return BN_ERR_ARG;
     hipLaunchKernelGGL((gemm_turns_kernel<BM, BN, EPI, TO>), dim3((unsigned)grid), dim3(512), 0, s, (const bf16*)X, (const bf16*)W, (TO*)Y, M, N, K,
-                       ldx, ldw, ldy, tiles_m, tiles_n, splits, (K / GM_BK + splits - 1) / splits, act, grp);
+                       ldx, ldw, ldy, tiles_m, tiles_n, splits, (K / GM_BK + splits - 1) / splits, grp);
     return bn_launch_status();
 }
 
 template <int EPI, typename TO>
-static int gm_turns(int tile, const void* X, const void* W, void* Y, int M, int N, int K, int ldx, int ldw, int ldy, int splits, int act,
+static int gm_turns(int tile, const void* X, const void* W, void* Y, int M, int N, int K, int ldx, int ldw, int ldy, int splits,
                     hipStream_t s, const GmGroups& grp, int max_tiles = 0) {
 #define GM_TILE(I, BM_, BN_) \
-    if (tile == I) return gm_turns_launch<BM_, BN_, EPI, TO>(X, W, Y, M, N, K, ldx, ldw, ldy, splits, act, s, grp, max_tiles)
+    if (tile == I) return gm_turns_launch<BM_, BN_, EPI, TO>(X, W, Y, M, N, K, ldx, ldw, ldy, splits, s, grp, max_tiles)
     GM_TILE(0, 256, 256);
     GM_TILE(3, 256, 128);
     if constexpr (EPI != GM_GROUPED) {                   // grouped tiles are 256 rows
@@ -722,10 +734,11 @@ extern "C" int bn_gemm_mfma(int out_dtype, const void* X, const void* W, void* Y
         int tile = width == 256 ? 0 : 3, splits = 1;
         if (!width) gm_plan(M, N, K, 0, 1, &tile, &splits);
         const GmGroups none = gm_no_groups();
-        if (glu8 && act == BN_ACT_SILU) return gm_turns<GM_SILU, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, act, s, none);
-        if (glu8) return gm_turns<GM_GATED, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, act, s, none);
-        return f32 ? gm_turns<GM_STORE, float>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, 0, s, none)
-                   : gm_turns<GM_STORE, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, 0, s, none);
+        if (glu8 && act == BN_ACT_SILU) return gm_turns<GM_SILU, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, s, none);
+        if (glu8 && act == BN_ACT_GELU_TANH) return gm_turns<GM_GATED_GELU, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, s, none);
+        if (glu8) return gm_turns<GM_GATED_RELU2, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, s, none);
+        return f32 ? gm_turns<GM_STORE, float>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, s, none)
+                   : gm_turns<GM_STORE, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, ldy, 1, s, none);
     }
     // The tile width: the one with the least work on the busiest CU (rounds of workgroups over the
     // CUs times the width), a wider tile counting a little less than its width because it reads
@@ -759,7 +772,7 @@ extern "C" int bn_gemm_mfma_slabs(const void* X, const void* W, float* Y, int M,
     int tile = 0, plan = 1;
     gm_plan(M, N, K, 0, GM_MAX_SPLITS, &tile, &plan);
     if (plan != splits) return BN_ERR_ARG;
-    return gm_turns<GM_STORE, float>(tile, X, W, Y, M, N, K, ldx, ldw, N, splits, 0, s, gm_no_groups());
+    return gm_turns<GM_STORE, float>(tile, X, W, Y, M, N, K, ldx, ldw, N, splits, s, gm_no_groups());
 }
 
 // Y [M, N] (bf16, contiguous) = act(X . W^T) on the float32 sums, act the exact gelu or relu2 (BN_UNARY_*).
@@ -768,8 +781,8 @@ extern "C" int bn_gemm_mfma_unary(const void* X, const void* W, void* Y, int M, 
     if (kind != BN_UNARY_GELU_ERF && kind != BN_UNARY_RELU2) return BN_ERR_ARG;
     int tile = 0, splits = 1;
     gm_plan(M, N, K, 0, 1, &tile, &splits);
-    return kind == BN_UNARY_RELU2 ? gm_turns<GM_RELU2, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, N, 1, 0, s, gm_no_groups())
-                                  : gm_turns<GM_GELU_ERF, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, N, 1, 0, s, gm_no_groups());
+    return kind == BN_UNARY_RELU2 ? gm_turns<GM_RELU2, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, N, 1, s, gm_no_groups())
+                                  : gm_turns<GM_GELU_ERF, bf16>(tile, X, W, Y, M, N, K, ldx, ldw, N, 1, s, gm_no_groups());
 }
 
 // y[i] [M, N] (bf16, contiguous) = x[i] . w[i]^T for n products of the same sizes, in one launch: rows of x[i] ldx apart, w[i] contiguous.
@@ -785,7 +798,7 @@ extern "C" int bn_gemm_mfma_items(int n, const void* const* x, const void* const
     }
     int tile = 0, splits = 1;
     gm_plan(M, N, K, 0, 1, &tile, &splits, n);
-    return gm_turns<GM_ITEMS, bf16>(tile, nullptr, nullptr, nullptr, M, N, K, ldx, K, N, n, 0, s, g);
+    return gm_turns<GM_ITEMS, bf16>(tile, nullptr, nullptr, nullptr, M, N, K, ldx, K, N, n, s, g);
 }
 
 // The grouped form: X [rows, K] ordered by matrix, W [matrices][N, K] (w_stride elements apart), tiles [max_tiles][3] and
@@ -810,8 +823,8 @@ extern "C" int bn_gemm_mfma_grouped(int out_dtype, const void* X, const void* W,
         const int live = matrices < 1 ? full : std::min(max_tiles, matrices * std::max(1, (rows / matrices - GM_BM / 10 + GM_BM - 1) / GM_BM));
         int tile = 0, splits = 1;
         gm_plan(live * GM_BM, N, K, GM_BM, 1, &tile, &splits, 1, 17.);
-        return f32 ? gm_turns<GM_GROUPED, float>(tile, X, W, Y, rows, N, K, ldx, ldw, ldy, 1, 0, s, g, max_tiles)
-                   : gm_turns<GM_GROUPED, bf16>(tile, X, W, Y, rows, N, K, ldx, ldw, ldy, 1, 0, s, g, max_tiles);
+        return f32 ? gm_turns<GM_GROUPED, float>(tile, X, W, Y, rows, N, K, ldx, ldw, ldy, 1, s, g, max_tiles)
+                   : gm_turns<GM_GROUPED, bf16>(tile, X, W, Y, rows, N, K, ldx, ldw, ldy, 1, s, g, max_tiles);
     }
     const int bn = gm_pick_bn(rows, N, gm_compute_units());
 #define GM_GO_GROUPED(BN_)                                                                                         \

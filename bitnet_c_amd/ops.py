@@ -996,6 +996,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, interleaved: bool = 
     # 27,648 x 5,120 at 512 / 2,048 / 8,192 150 -> 124, 507 -> 466, 1,950 -> 1,632; 57,344 x 8,192 at 320 / 512 / 640 / 4,096 304 -> 302, 410 -> 379,
     # 548 -> 529, 2,552 -> 2,514; 16,384 x 3,072 at 512 / 4,096 60 -> 51, 323 -> 315; 11,264 x 2,048 at 129 / 512 / 2,048 / 8,192 31 -> 24, 37 -> 33, 98 -> 84,
     # 411 -> 311; 5,632 x 1,024 at 512 / 2,048 18 -> 14, 43 -> 26.  Of 24 row counts from 129 to 8,192 for each of the six the least gain is 0.7 %.
+    # The other activations: 16,384 x 2,048 at 512 / 2,048 / 8,192 with gelu 42 -> 35, 118 -> 109, 479 -> 422, with relu2 40 -> 35, 117 -> 106, 462 -> 407.
     if (x.dtype == torch.bfloat16 and interleaved and aligned and M >= PROMPT_ROWS and K % GEMM_STEP == 0
             and gemm_mfma_supported(M, 2 * F, K, ldx, ldw)):
         return gemm_mfma(x, w_gate_up, x.dtype, glu8=True, activation=activation)

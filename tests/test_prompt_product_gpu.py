@@ -45,6 +45,25 @@ def test_products_and_gated_units(M, N, K):
             assert torch.equal(ops.linear_swiglu(x, w, True, activation=act), got), act
 
 
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu2"])
+def test_gates_of_every_finite_number(act):
+    """Eight gates a row that are one bf16 number each, beside ups of one: the activation of every finite number."""
+    ops = _ops()
+    v = torch.arange(2 ** 16, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    v = v[v.isfinite()].view(-1, 8).cuda()
+    x = torch.zeros(v.shape[0], 64, dtype=torch.bfloat16, device="cuda")
+    x[:, :8], x[:, 8] = v, 1.0
+    w = torch.zeros(16, 64, dtype=torch.bfloat16, device="cuda")
+    w[torch.arange(8), torch.arange(8)], w[8:, 8] = 1.0, 1.0
+    got, z = ops.linear_swiglu(x, w, True, activation=act).double(), v.double()
+    y = (2 / torch.pi) ** 0.5 * (z + 0.044715 * z ** 3)
+    want = z * torch.sigmoid(z) if act == "silu" else z * torch.sigmoid(2 * y) if act == "gelu_tanh" else z.clamp(min=0) ** 2
+    inf = want > 3.39e38                                  # beyond bf16
+    assert bool((got[inf] > 3.38e38).all())
+    # the rounding to bf16; an exponent of up to 150 is a float32 number; factors below 1.2e-38 are 0
+    assert bool(((got - want).abs()[~inf] <= want.abs()[~inf] * (2.0 ** -8 + 150 * 2.0 ** -23) + 4e-36).all())
+
+
 # slabs: two to six ranges of K, the last one shorter; every range summed alone
 @pytest.mark.parametrize("M,N,K", [(129, 264, 8256), (200, 4096, 8192), (257, 4104, 14336), (513, 1032, 4160), (1500, 2056, 8192),
                                    (513, 4104, 14336), (900, 4100, 9024), (300, 520, 64), (130, 136, 8896)])
