@@ -780,7 +780,8 @@ __device__ __forceinline__ void turn_weights(f32x4 (&st)[NT][2], int kb, f32x4 (
 // Blocks that every column sees whole run in a loop without a comparison.
 // What bounds a step (two blocks, 8 products of 16 x 16 x 128 or so a wave and block: 34 matrix instructions of 16 cycles, some 75 vector instructions): 2,240
 // cycles of 2 x (544 + 300), since a vector instruction delays its SIMD's matrix instructions (both read the same registers' ports); the two
-// barriers take 10 % of it. 4,096 tokens of 32 heads over 8, us: 179 before, 143; 8,100 tokens 640, 510 (0.84 and 1.05 PFLOP/s).  Tried: operands read in
+// barriers take 10 % of it. 4,096 tokens of 32 heads over 8, us: one group a workgroup 167, keys split 148, a tile each 133 (1.03 PFLOP/s); 8,100 tokens 607, 510,
+// 474 (1.13).  Tried, over split keys: operands read in
 // the products' turn (8,100 tokens 607, from shared memory's latency); conditions instead of numbers for a block's kind (684: they are carried in
 // vector registers); variants of a turn with and without masks (798: their accumulators are copied where they meet).
 template <int HS, int NT, bool SPLIT>
@@ -1419,6 +1420,63 @@ extern "C" int bn_attn_mfma_supports(int hs) { return (hs == BN_MFMA_HEAD_DIM_SM
 // query tokens per tile of the prompt form, for GT heads per group
 extern "C" int bn_attn_mfma_prompt_tokens(int hs, int GT) { return (hs == 64 ? 256 : 128) / GT; }
 
+// Which kernel a prompt's launch takes, by its workgroups alone (the tiles' positions are on the device).  PAIRED: a workgroup takes a pair of the list's
+// tiles, a long and a short one.
+enum { PF_TWO, PF_TWO_PAIRED, PF_ONE, PF_ONE_PAIRED, PF_SPLIT, PF_SPLIT_PAIRED, PF_EACH, PF_EACH_PAIRED };
+
+static int prompt_form(long long n_tiles, long long n_tokens, long long n_seqs, long long wgs_per_seq, int hs, int window) {
+    const long long cus = compute_units(), pairs = (n_tiles + 1) / 2;
+    const bool paired = n_tiles * wgs_per_seq > cus;     // more tiles than CUs
+    const long long wgs = (paired ? pairs : n_tiles) * wgs_per_seq;
+    // Two groups of waves a workgroup (eight waves, one workgroup a CU) halve the chain of blocks that a tile walks,
+    // which is what a launch of one round waits for.  A launch of several rounds is faster with one group a
+    // workgroup and two workgroups a CU: they share nothing and drift apart, so that one's matrix instructions
+    // meet the other's vector work, where the two groups of one workgroup meet at a barrier in every stage and do
+    // the same thing at the same time (8 to 16 % at 8,192 tokens and for eight or 64 prompts of 128 to 2,048).
+    // It is taken from four rounds on, and from two when its rounds (of two workgroups a CU) are not much emptier
+    // than those of the wide form (6,144 tokens of one sequence are three full rounds of the wide form and one and
+    // a half of the other: 410 against 445 us).
+    const double fill1 = (double)wgs / (double)(((wgs + 2 * cus - 1) / (2 * cus)) * 2 * cus);
+    const double fill2 = (double)wgs / (double)(((wgs + cus - 1) / cus) * cus);
+    const bool one = wgs >= 4 * cus || (wgs >= 2 * cus && fill1 * 1.1 >= fill2);
+    if (hs == 64) return one ? (paired ? PF_ONE_PAIRED : PF_ONE) : (paired ? PF_TWO_PAIRED : PF_TWO);
+    // Heads of 128: the two groups take turns, over split keys, where those of 64 walk in step (always as fast or faster), or have a tile each (a CU's keys are
+    // fetched once for two).  Over 617 launches (nine shapes of heads and windows; 1 to 64 sequences of 16 to 8,100 tokens, some behind earlier ones)
+    // what this rule takes is the older forms' time (one group, or two in step, by the rule above) or less but for three (by 3 to 6 %), 14 % less on average, and
+    // 3 % more than the fastest form's.  us, one group / split / a tile each (the older form), 32 heads over 8 unless it says more: one prompt of 1,024 36 / 25 /
+    // 37 (30), 2,048 71 / 48 / 64 (59), 2,500 109 / 101 / 86 (128), 4,096 167 / 148 / 133 (167), 5,000 351 / 249 / 291 (329), 8,100 607 / 510 / 474 (607); 64 new tokens behind
+    // 4,000 115 / 60 / 108 (83); two of 640, 64 heads over 8, 44 / 49 / 38 (53); sixteen of 640 104 / 125 / 114 (104); eight of 700, 40 heads over 40, 98 / 116 / 119 (98).
+    if (!paired) return PF_SPLIT;                        // the chip is not full: as many, short chains as there can be
+    const long long tokens = n_tokens / n_seqs;          // new ones of a sequence; how many there are before them is not known here
+    const long long a_seq = n_tiles / n_seqs;
+    const bool equal = n_tiles % n_seqs == 0, alone = n_tiles < 2 * n_seqs;      // alone: sequences of one tile, nothing for two groups to share
+    if (pairs * wgs_per_seq <= cus) {
+        // Fewer pairs than CUs.  Short sequences, and narrow windows, whose walks are short as well: a tile each (32 sequences of 64 tokens 19 / 22 / 18, the older form
+        // 23; one of 2,048 under a window of 512 47 / 38 / 34, 40), where the workgroups that leave do not crowd the others (the last of an odd number of pairs of
+        // every sequence: eight of 200 26 / 22 / 27, behind 2,000 134 / 81 / 125); sequences of one tile: all of them at once, two workgroups a CU (eight of
+        // 30 behind 2,000, 40 heads over 40, a pair / split / a tile each / this 124 / 78 / 119 / 74, 98)
+        const bool spread = n_seqs == 1 || (equal && (a_seq == 2 || a_seq % 4 == 0)) || (n_tiles + n_seqs) * wgs_per_seq * 2 <= 3 * cus;
+        if (tokens < 320 && alone) return PF_ONE;
+        return (tokens < 320 || (window > 0 && 3LL * window <= 2 * tokens)) && spread ? PF_EACH : PF_SPLIT_PAIRED;
+    }
+    // A workgroup with a tile a group takes two pairs of a sequence; the last of an odd number of them, and a pair of two sequences' middle tiles, one by
+    // one.  Sequences of one length: that many workgroups, in whole rounds; of several: about the pairs' half (the short ones' fill the rounds).
+    double rounds = 0.5 * (double)(pairs * wgs_per_seq) / (double)cus + 0.1;
+    if (equal) {
+        rounds = (double)((n_seqs * ((a_seq / 2 + 1) / 2) + (a_seq % 2 * n_seqs) / 2) * wgs_per_seq) / (double)cus;
+        rounds = rounds <= 4.0 ? std::ceil(rounds) : rounds + 0.35;
+    }
+    // Short sequences (by their new tokens): a tile each in one round, and of two tiles each, whose workgroups leave nobody out (16 of 200, 40 heads over 40, 52 / 69 / 55,
+    // behind 2,000 346 / 286 / 234); else two workgroups a CU (16 of 200, 32 over 8, 29 / 41 / 42)
+    if (tokens < 640) return !alone && !one && (rounds <= 1.0 || (equal && a_seq == 2)) ? PF_EACH_PAIRED : PF_ONE_PAIRED;
+    if (!one) return rounds <= 1.0 ? PF_EACH_PAIRED : PF_SPLIT_PAIRED;
+    // Beside the one group's rounds (of two workgroups a CU; a partial one is dearer than its share) one of these takes the less the longer the walk
+    double ones = (double)wgs / (double)(2 * cus);
+    if (std::fabs(ones - std::round(ones)) > 0.1) ones += 0.2;
+    const double walk = window > 0 && window < tokens ? (double)window : (double)tokens;
+    return walk >= 1000.0 && rounds * (0.74 + 200.0 / walk) <= 0.97 * ones ? PF_EACH_PAIRED : PF_ONE_PAIRED;
+}
+
 static int attn_mfma_launch(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
                             const void* vt_pages, const int* block_table, int bt_stride, const int* seq_lens,
                             const int* tiles, int n_tiles, int n_tokens, int H, int Hkv, int hs, int GT,
@@ -1455,15 +1513,15 @@ static int attn_mfma_launch(const void* q, int q_stride, void* out, int out_stri
     a.by_length = (!tiles && n_splits == 1 && (long long)n_tiles * wgs_per_seq > compute_units()) ? by_length : nullptr;
     a.order_period = compute_units() / wgs_per_seq;
     if (tiles) {
-        const long long cus = compute_units();
-        // A workgroup takes a pair of tiles, a long and a short one, when there are more of them than CUs.
-        const int paired = (long long)n_tiles * wgs_per_seq > cus ? 1 : 0;
-        const long long pairs = (n_tiles + 1) / 2, wgs = (paired ? pairs : n_tiles) * wgs_per_seq;
-        if (2 * wgs > 0x7fffffff) return BN_ERR_ARG;
+        const int form = prompt_form(n_tiles, n_tokens, n_seqs, wgs_per_seq, hs, window);
+        const long long pairs = (n_tiles + 1LL) / 2;
+        const int paired = form == PF_ONE_PAIRED || form == PF_SPLIT_PAIRED || form == PF_TWO_PAIRED || form == PF_EACH_PAIRED;
+        const long long wgs = (form == PF_EACH ? 2 * pairs : paired ? pairs : n_tiles) * wgs_per_seq;
+        if (wgs > 0x7fffffff) return BN_ERR_ARG;
         auto go = [&](auto kernel, int which, int ng) {
             // three staged blocks of 32 keys a group with their values: up to 96 KB, beyond the default limit of dynamic shared memory
             const size_t smem = (size_t)PROMPT_BUFFERS * (32 * ng * hs + hs * 32 * ng) * 2;
-            static bool raised[4] = {false, false, false, false};
+            static bool raised[3] = {false, false, false};
             if (!raised[which]) {
                 const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -1473,43 +1531,13 @@ static int attn_mfma_launch(const void* q, int q_stride, void* out, int out_stri
             hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256 * ng), smem, s, a, n_tiles, paired);
             return bn_launch_status();
         };
-        if (hs == 64) {
-            // Two groups of waves a workgroup (eight waves, one workgroup a CU) halve the chain of blocks that a tile walks,
-            // which is what a launch of one round waits for.  A launch of several rounds is faster with one group a
-            // workgroup and two workgroups a CU: they share nothing and drift apart, so that one's matrix instructions
-            // meet the other's vector work, where the two groups of one workgroup meet at a barrier in every stage and do
-            // the same thing at the same time (8 to 16 % at 8,192 tokens and for eight or 64 prompts of 128 to 2,048).
-            // It is taken from four rounds on, and from two when its rounds (of two workgroups a CU) are not much emptier
-            // than those of the wide form (6,144 tokens of one sequence are three full rounds of the wide form and one and
-            // a half of the other: 410 against 445 us).
-            const double fill1 = (double)wgs / (double)(((wgs + 2 * cus - 1) / (2 * cus)) * 2 * cus);
-            const double fill2 = (double)wgs / (double)(((wgs + cus - 1) / cus) * cus);
-            return (wgs >= 4 * cus || (wgs >= 2 * cus && fill1 * 1.1 >= fill2)) ? go(attn_mfma_prompt_kernel<64, 4, 1>, 1, 1)
-                                                                                : go(attn_mfma_prompt_kernel<64, 4, 2>, 0, 2);
-        }
-        // Heads of 128: groups that take turns over split keys (short chains) or with a tile each (a CU's keys are fetched once for two), or workgroups of one
-        // group that share nothing, two a CU (one's start hides behind the other's work).  us, one group / split / a tile each (before: the faster or
-        // the slower of one group and of two that walk in step, by the rule above), 32 heads over 8: one prompt of 300 15.3 / 14.4 / 16.9
-        // (15.3), 1,024 36 / 25 / 37 (30), 2,048 71 / 48 / 64 (59), 3,000 124 / 112 / 97 (146), 4,096 163 / 147 / 130 (166), 5,000 351 / 249 / 291 (329),
-        // 8,100 602 / 512 / 465 (615); 64 new tokens behind 4,000 115 / 60 / 108 (83); four of 70 to 500 26 / 24 / 23 (26), eight of 300
-        // 30 / 41 / 30 (44), of 128 to 2,048 191 / 184 / 169 (192), 16 of 1,024 220 / 243 / 195 (220), of 150 25 / 38 / 28 (38), 32 of 128 24 / 39 / 29 (25), of 512
-        // 143 / 192 / 148 (145), 64 of 16 to 512 155 / 223 / 166 (156); a window of 700 over 2,000 56 / 42 / 37 (49).
-        auto turns = [&](auto kernel, long long n, int two) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(512), 0, s, a, n_tiles, two);
-            return bn_launch_status();
-        };
-        // (a tile each: half of the workgroups find that another has taken their pair along)
-        const int paired2 = pairs * wgs_per_seq > cus ? 1 : 0;
-        auto split = [&] { return turns(attn_mfma_turns_kernel<128, 2, true>, wgs, paired); };
-        auto each = [&] { return turns(attn_mfma_turns_kernel<128, 2, false>, pairs * (paired2 ? 1 : 2) * wgs_per_seq, paired2); };
-        if (!paired) return split();                      // the chip is not full: as many, short chains as there can be
-        if (n_tokens < 640LL * n_seqs)                    // short sequences (by their new tokens): two workgroups a CU once there are that many
-            return wgs >= 2 * cus ? go(attn_mfma_prompt_kernel<128, 2, 1>, 3, 1) : each();
-        // Rounds over the CUs, whole ones where they are few; a split workgroup's is half as long, and costs an eighth more.  Tiles that all fit at once
-        // are as long as the last of them, twice the average where every token sees all before it.
-        auto rounds = [&](long long n) { const double r = (double)n / (double)cus; return r <= 2.0 ? std::ceil(r) : r + 0.35; };
-        const long long quads = (pairs + 1) / 2 * wgs_per_seq;
-        return rounds(paired2 ? quads : 2 * quads) * (window > 0 && !paired2 ? 0.5 : 1.0) <= rounds(wgs) * 0.56 ? each() : split();
+        if (form == PF_TWO || form == PF_TWO_PAIRED) return go(attn_mfma_prompt_kernel<64, 4, 2>, 0, 2);
+        if (form == PF_ONE || form == PF_ONE_PAIRED) return hs == 64 ? go(attn_mfma_prompt_kernel<64, 4, 1>, 1, 1) : go(attn_mfma_prompt_kernel<128, 2, 1>, 2, 1);
+        if (form == PF_SPLIT || form == PF_SPLIT_PAIRED)
+            hipLaunchKernelGGL((attn_mfma_turns_kernel<128, 2, true>), dim3((unsigned)wgs), dim3(512), 0, s, a, n_tiles, paired);
+        else                                             // (half of the workgroups find that another has taken their pair along)
+            hipLaunchKernelGGL((attn_mfma_turns_kernel<128, 2, false>), dim3((unsigned)wgs), dim3(512), 0, s, a, n_tiles, paired);
+        return bn_launch_status();
     }
     if (n_tiles > 65535) return BN_ERR_ARG;                 // sequences are the grid's y
     // Two splits and no more workgroups than CUs: both in one workgroup, without a launch for the merge (WHOLE).  us, merged by a
@@ -1566,6 +1594,12 @@ extern "C" int bn_attn_mfma_prompt(const void* q, int q_stride, void* out, int o
     return attn_mfma_launch(q, q_stride, out, out_stride, k_pages, vt_pages, block_table, bt_stride, nullptr, tiles, n_tiles,
                             n_tokens, H, Hkv, hs, GT, window, scale, 1, 0, nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr,
                             nullptr, 0, 0, 0.f, n_seqs, s);
+}
+
+// the number of that choice (PF_*)
+extern "C" int bn_attn_mfma_prompt_form(int n_tiles, int n_tokens, int n_seqs, int H, int Hkv, int hs, int GT, int window) {
+    if (!bn_attn_mfma_supports(hs) || n_tiles < 1 || n_tokens < 1 || n_seqs < 1 || H < 1 || Hkv < 1 || H % Hkv || GT < 1) return -1;
+    return prompt_form(n_tiles, n_tokens, n_seqs, (long long)Hkv * ((H / Hkv + GT - 1) / GT), hs, window);
 }
 
 // The decode form (tiles none, rotate on) over rows whose RMSNorm was left undone: q, the new key and the new value of

@@ -171,6 +171,7 @@ _SIGNATURES = {
                          c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p],
         "bn_attn_mfma_prompt": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int,
                                 c_int, c_int, c_int, c_int, c_float, c_int, c_void_p],
+        "bn_attn_mfma_prompt_form": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     },
     "attn_f32": {
         "bn_attn_f32_supports": [c_int],
