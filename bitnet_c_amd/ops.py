@@ -2654,19 +2654,36 @@ LIGHTNING_BLOCK = _build.header_constant("LB_C", "lightning.hip")
 
 
 def lightning_in_blocks(sizes, H: int, dk: int, dv: int) -> bool:
-    """Whether a prompt step (sizes: StepContext.sizes) that could take the blocks of 64 tokens should: where the chunked form would run, and where the chain
-    would from half a block a sequence on (us, chain / blocks, 16 heads of 128 x 128: sixteen sequences of 64 tokens 66 / 28; 31 of 256 294 / 158)."""
+    """Where blocks of 64 tokens come into question for a prompt step (sizes: StepContext.sizes): where the chunked form would run, and where the chain would from
+    half a block a sequence on (us, chain / blocks, 16 heads of 128 x 128: sixteen sequences of 64 tokens 66 / 28; 31 of 256 294 / 158)."""
     rows, seqs = sizes
     return rows // seqs >= LIGHTNING_BLOCK // 2 or bool(_fn("lightning", "bn_lightning_prefers_chunks")(seqs, H, dk, dv))
+
+
+def lightning_takes_blocks(sizes, H: int, dk: int, dv: int) -> bool:
+    """Whether a prompt step that could take the blocks does.  A block costs a step of 64 tokens of keys 64 or 128 wide whatever it holds, so short sequences
+    and narrow keys stay with the form they had.  us, that form / blocks.  The chunked form: one sequence of up to 16 tokens, 16 heads of 128 x 128 16.7 /
+    19.1, 8 of 64 x 128 11 / 14, 32 of 64 x 64 15 / 14; of 96, 16 heads 26 / 26, 8 17 / 20; two of 128 28 / 29, 8 of 128 x 256 28 / 32; of 300 45 / 26; eight of
+    16, 16 heads 27 / 19.  The chain: 16 of 32, 16 heads of 128 x 128 37 / 32, 64 of 32, 32 heads of 64 x 64 57 / 66, of 48 82 / 71; 64 of 64, 64 heads of
+    32 x 32 87 / 119, eight of 300 132 / 84.  (At 1,000 sizes of twelve shapes of heads no more than 9 % slower than the older form, 17 % faster on average.)"""
+    rows, seqs = sizes
+    each, walks = rows // seqs, seqs * H * -(-dv // 64)
+    if not lightning_in_blocks(sizes, H, dk, dv):
+        return False
+    if _fn("lightning", "bn_lightning_prefers_chunks")(seqs, H, dk, dv):
+        return each >= 192 or (H >= 32 and dk >= 32) or walks >= 256 or (walks >= 128 and each >= 32)
+    if dk <= 32:
+        return walks < 1024 and each >= LIGHTNING_BLOCK
+    return each >= (32 if dk > 64 and walks < 1024 else 48)
 
 
 def lightning_in_pieces(T: int, n_seqs: int, H: int, dv: int) -> bool:
     """Whether those blocks are formed side by side, the same bits: a walk's time is its length, side by side costs three launches and the traffic of a state a
     block.  us one after the other / side by side, 16 heads of 128 x 128: one sequence of 64 tokens 17 / 25, 65 28 / 24, 256 52 / 27; four of 256 53 / 56,
     500 101 / 68; sixteen of 512 153 / 206; 32 heads of 64 x 64: one of 128 17.8 / 19.5, 192 25 / 19; four of 256 33 / 38, 500 63 / 51; sixteen of
-    512 94 / 140."""
+    512 94 / 140; 8 heads of 64 x 128: one of 64 13.8 / 19.2 (one block: nothing stands beside it)."""
     walks = n_seqs * H * -(-dv // 64)
-    return walks < 512 and T // n_seqs > 2 * walks
+    return walks < 512 and T // n_seqs > max(LIGHTNING_BLOCK, 2 * walks)
 
 
 def lightning_scan(x: torch.Tensor, q_col: int, k_col: int, v_col: int, decay: torch.Tensor, state: torch.Tensor, slot_ids,
@@ -2684,7 +2701,7 @@ def lightning_scan(x: torch.Tensor, q_col: int, k_col: int, v_col: int, decay: t
     silu False: q, k and v enter as projected.  inv_freq [n <= dk / 2] float32 (with positions [T] int32, the rows' positions
     once more): dimension i < n of every query and key head turns with dimension i + n by position * inv_freq[i].
     k_scale multiplies the keys.
-    bf16 rows without a rotation and in groups of eight take blocks of 64 tokens in the chunks' place (lightning_in_blocks, for the step's sizes: T and the
+    bf16 rows without a rotation and in groups of eight take blocks of 64 tokens in the chunks' place (lightning_takes_blocks, for the step's sizes: T and the
     number of sequences where they are None); pieces: whether side by side (True) or one after the other (False), the same bits; None: by their number."""
     require_gpu()
     _dev(x, "x", dims=2)
@@ -2715,7 +2732,7 @@ def lightning_scan(x: torch.Tensor, q_col: int, k_col: int, v_col: int, decay: t
         blocks = -1
         if (tiles is not None and chain is not True and x.dtype == torch.bfloat16
                 and _fn("lightning", "bn_lightning_blocks_take")(x.data_ptr(), ld, int(q_col), int(k_col), dk, rope_dims)
-                and (chain is False or lightning_in_blocks(sizes or (T, n_seqs), H, dk, dv))):
+                and (chain is False or lightning_takes_blocks(sizes or (T, n_seqs), H, dk, dv))):
             state_floats = H * (64 if dk <= 64 else 128) * (64 if dv <= 64 else -(-dv // 128) * 128)
             most = _pieces_of(T, n_seqs, LIGHTNING_BLOCK)
             blocks = most if (pieces if pieces is not None else lightning_in_pieces(T, n_seqs, H, dv)) and most * state_floats * 4 <= SCAN_PIECES_BYTES else 0

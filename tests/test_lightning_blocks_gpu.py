@@ -100,3 +100,36 @@ def test_which_steps_take_blocks():
     assert ops.lightning_in_blocks((16, 1), 16, 128, 128) and ops.lightning_in_blocks((2048, 64), 16, 128, 128) and not ops.lightning_in_blocks((1984, 64), 16, 128, 128)
     assert ops.lightning_in_pieces(65, 1, 16, 128) and not ops.lightning_in_pieces(64, 1, 16, 128) and not ops.lightning_in_pieces(1024, 4, 16, 128)
     assert ops.lightning_in_pieces(2000, 4, 16, 128) and not ops.lightning_in_pieces(32768, 16, 16, 128)
+
+
+def test_short_sequences_and_narrow_keys_keep_their_form():
+    from bitnet_c_amd import ops
+    take, chunks = ops.lightning_takes_blocks, lambda n, *a: bool(ops._fn("lightning", "bn_lightning_prefers_chunks")(n, *a))
+    # in the chunked form's place
+    assert chunks(1, 16, 128, 128) and chunks(4, 8, 128, 256) and chunks(8, 16, 96, 96)
+    assert not take((128, 1), 16, 128, 128) and take((192, 1), 16, 128, 128) and take((16, 1), 32, 64, 64) and not take((16, 1), 32, 16, 64)
+    assert take((16, 8), 16, 96, 96) and not take((64, 4), 8, 128, 256) and take((128, 4), 8, 128, 256)
+    # in the chain's
+    assert not chunks(16, 16, 128, 128) and not chunks(64, 32, 64, 64) and not chunks(8, 64, 32, 32)
+    assert take((512, 16), 16, 128, 128) and not take((496, 16), 16, 128, 128) and take((3072, 64), 32, 64, 64) and not take((3008, 64), 32, 64, 64)
+    assert take((512, 8), 64, 32, 32) and not take((448, 8), 64, 32, 32) and not take((8192, 16), 64, 32, 32)
+    # one block has nothing beside it
+    assert not ops.lightning_in_pieces(64, 1, 8, 128) and ops.lightning_in_pieces(65, 1, 8, 128)
+
+
+@pytest.mark.parametrize("lens,H,dk,dv", [((16,), 4, 64, 64), ((33, 31), 4, 64, 64), ((40,) * 8, 64, 32, 32), ((300, 5), 4, 64, 64)])
+def test_the_form_that_is_taken(lens, H, dk, dv):
+    """Unasked, the step takes the form that the rule names, bit for bit."""
+    from bitnet_c_amd import ops
+    T, g = sum(lens), torch.Generator().manual_seed(sum(lens))
+    x, decay = torch.randn(T, H * (2 * dk + dv), generator=g).bfloat16().cuda(), torch.linspace(0.5, 0.999, H).cuda()
+    at = [sum(lens[:i]) for i in range(len(lens))]
+    tiles, slots = torch.tensor([(i, a, n, 0) for i, (a, n) in enumerate(zip(at, lens))], dtype=torch.int32).cuda(), torch.arange(len(lens), dtype=torch.int32).cuda()
+    run = lambda **kw: ops.lightning_scan(x, 0, H * dk, 2 * H * dk, decay, torch.zeros(len(lens), H * dk * dv).cuda(), slots, H, dk, dv, tiles=tiles, **kw)
+    got, sizes = run(), (T, len(lens))
+    if ops.lightning_takes_blocks(sizes, H, dk, dv):
+        assert torch.equal(got, run(chain=False))
+    elif not ops._fn("lightning", "bn_lightning_prefers_chunks")(len(lens), H, dk, dv):
+        assert torch.equal(got, run(chain=True))
+    else:                                                 # the chunked form adds up in another order than either
+        assert not torch.equal(got, run(chain=False)) and torch.allclose(got, run(chain=True), rtol=1e-3, atol=1e-4)
