@@ -596,7 +596,9 @@ def can_split_rows(M: int, N: int, K: int, dtype) -> bool:
 # 68); 4,096 x 4,096 at 129 / 512 / 2,048 / 3,072 (4,096) 66 -> 39, 108 -> 69, 253 -> 218, 345 -> 329 (396 -> 430); 2,560 x 2,560 at 4,096 220 ->
 # 199.  So up to three quarters as many tiles of 256 x 256 a product as there are CUs.  Two products gain less, and nothing where few rows
 # make the tiles small in number (2,048 x 2,048 at 256 / 512 / 1,024 rows 20 -> 21, 23 -> 23, 32 -> 26; 4,096 x 4,096 at 256 / 2,048 / 3,072
-# 37 -> 39, 125 -> 106, 171 -> 176): from 1,024 rows to half as many tiles as CUs.
+# 37 -> 39, 125 -> 106, 171 -> 176): from 1,024 rows to half as many tiles as CUs.  Two or three products of few tiles and long K are a serial chain
+# that the library cuts (two of 256 x 4,096 at 1,024 / 2,048 (4,096) rows 23 -> 36, 30 -> 37 (39 -> 39), of 512 x 4,096 at 1,024 (2,048) 30 -> 37 (39 -> 39); three of 256 x 2,048
+# at 129 17 -> 20, of 512 x 4,096 at 129 / 512 28 -> 35, 33 -> 37, of 1,024 x 8,192 at 129 50 -> 68): they stay with it by their tiles beside K.
 GEMM_ITEMS = _build.header_constant("GM_MAX_ITEMS", "gemm_mfma.hip")
 
 
@@ -605,6 +607,8 @@ def group_rows(n: int, M: int, N: int, K: int) -> bool:
     if not (2 <= n <= GEMM_ITEMS and M >= (PROMPT_ROWS if n > 2 else 1024) and K % GEMM_STEP == 0 and K and N % 4 == 0):
         return False
     tiles = -(-M // 256) * -(-N // 256)
+    if (n == 2 and tiles * 256 < K) or (n == 3 and tiles * 1024 <= K):
+        return False
     return tiles * 4 <= (3 if n > 2 else 2) * _compute_units()
 
 

@@ -190,3 +190,10 @@ def test_slabs_are_left_where_ranges_pay():
     for M, N, K in ((2048, 2048, 8192), (3072, 2048, 8192), (3072, 2048, 8256), (4096, 2048, 10240), (2048, 4096, 9216), (2048, 4096, 10240), (1024, 8192, 9216)):
         assert ops.can_split_rows(M, N, K, torch.bfloat16) == (ops._fn("gemm_mfma", "bn_gemm_mfma_splits")(M, N, K) > 1)
     assert not ops.can_split_rows(2048, 2048, 8192 - 64, torch.bfloat16)
+
+
+def test_few_tiles_of_long_rows_are_no_group():
+    ops = _ops()
+    for n, M, N, K, take in ((2, 1024, 256, 1024, True), (2, 1024, 256, 1088, False), (2, 2048, 512, 4096, True), (2, 1024, 512, 4096, False), (3, 129, 256, 960, True),
+                             (3, 129, 256, 1024, False), (3, 129, 1024, 4096, False), (3, 129, 1280, 4096, True), (4, 129, 256, 8192, True)):
+        assert ops.group_rows(n, M, N, K) == take, (n, M, N, K)
