@@ -56,8 +56,10 @@ class StepContext:
         self.slots, self.n_new, self.pos0 = list(slots), list(n_new), list(pos0)   # host copies
         self.n_rows = int(tokens.numel())
         self.n_seqs = len(self.slots)
-        # (token rows, sequences) as a captured step of this request holds them: what a part whose choice of kernel changes
-        # bits chooses by, so that the first, eager step of a request and its replays choose alike
+        # (token rows, sequences) as a captured step of this request holds them: what a recurrence chooses its form by, so that
+        # the first, eager step of a request and its replays choose alike (products that round or do not go by ops.row_bucket).
+        # In bfloat16 the order of a float32 sum may still differ between them: the library's product, the ranges of K that slabs
+        # are cut into, products in one launch, a norm over many rows and the attention's tiles go by the rows and tiles at hand
         self.sizes = _row_bucket(self.n_rows), max(self.n_seqs, _bucket(self.n_seqs))
         # diagnostics: a callable (point, schedule entry, ResidualStream, ctx) that blocks call at "layer_in",
         # "ffn_in" and "layer_out" (the reference's bitnet_inp / bitnet_ffn_inp / bitnet_lout dumps,
@@ -277,14 +279,7 @@ MAX_PROMPT_GRAPH_ROWS = 8192      # prompt steps of more tokens than this run ea
 MAX_PROMPT_GRAPHS = 12            # captured prompt steps that an engine keeps; the one unused for longest goes first
 
 
-def _row_bucket(n: int) -> int:
-    """Token rows of the captured step that serves a prompt step of n tokens: 16 and 32 (up to 16 rows the products are
-    the fused ones of a decode step, and rows cost time there), then multiples of 64 up to 512, of 128 up to 2,048, of
-    512 beyond: from 64 tokens on the padding is at most an eighth."""
-    if n <= 32:
-        return 16 if n <= 16 else 32
-    unit = 64 if n <= 512 else 128 if n <= 2048 else 512
-    return -(-n // unit) * unit
+_row_bucket = ops.row_bucket
 
 
 class _PromptGraph:

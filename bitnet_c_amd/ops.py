@@ -571,6 +571,19 @@ def gemm_mfma_supported(M: int, N: int, K: int, ldx: int, ldw: int) -> bool:
 GEMM_STEP = _build.header_constant("GM_BK", "gemm_mfma.hip")      # K in whole steps of this: the prompt product's faster form
 # Prompt products that are this library's own beside the library's: from this many rows on (fewer: the kernels of a decode step) ...
 PROMPT_ROWS = 129
+
+
+def row_bucket(n: int) -> int:
+    """Token rows of the captured step that serves a prompt step of n tokens: 16 and 32 (up to 16 rows the products are
+    the fused ones of a decode step, and rows cost time there), then multiples of 64 up to 512, of 128 up to 2,048, of
+    512 beyond: from 64 tokens on the padding is at most an eighth.  What decides which numbers of a bf16 step are rounded goes by these rows, so that
+    a request's first, eager step and its replays choose alike."""
+    if n <= 32:
+        return 16 if n <= 16 else 32
+    unit = 64 if n <= 512 else 128 if n <= 2048 else 512
+    return -(-n // unit) * unit
+
+
 # ... a part's last product, as slabs over ranges of K, where K is long enough for the slabs' way through memory not to count, its tiles leave
 # half of the CUs without work, and the kernel's plan, which weighs the rounds of tiles against the slabs' bytes, finds ranges that pay (in one
 # range the library's product is the faster one by 2 to 9 %).  us with the kernel of the next norm, the library's product -> slabs: 4,096 x 14,336 at
@@ -842,7 +855,7 @@ _ACT_UNARY = _build.header_constant("SK_ACT_UNARY", "skinny_gemm.hip")     # + a
 def linear_unary(x: torch.Tensor, w: torch.Tensor, activation: str, streamed: Optional[StreamedWeight] = None) -> torch.Tensor:
     """activation(linear(x, w)) (one of UNARY_ACTIVATIONS): a feed-forward's first product without a gate.  bf16 steps of up
     to 16 rows form it in the product's own kernel, on the float32 sums, and so do a prompt's where
-    unary_in_product says so; everything else is the product, then the activation's kernel."""
+    unary_in_product says so of their row_bucket; everything else is the product, then the activation's kernel."""
     require_gpu()
     _dev(x, "x", dims=2)
     _dev(w, "w", x.dtype, 2)
@@ -856,7 +869,7 @@ def linear_unary(x: torch.Tensor, w: torch.Tensor, activation: str, streamed: Op
         _check(_fn("skinny_gemm", "bn_skinny_gemm")(_code(torch.bfloat16), x.data_ptr(), wp, y.data_ptr(), M, N, K, _rows(x, "x"),
                                                     wl, N, 0, 0, act, tiled, _stream()), "skinny_gemm(unary)")
         return y
-    if (x.dtype == torch.bfloat16 and w.shape[1] == K and unary_in_product(M, N, K, activation)
+    if (x.dtype == torch.bfloat16 and w.shape[1] == K and unary_in_product(row_bucket(M), N, K, activation)
             and (x.data_ptr() | w.data_ptr()) % 16 == 0 and _rows(x, "x") % 8 == 0 and _rows(w, "w") % 8 == 0
             and max(_rows(x, "x"), _rows(w, "w")) <= 1 << 22):
         return gemm_unary(x, w, activation)

@@ -72,7 +72,8 @@ class Linear:
     def lazy(self, x: torch.Tensor):
         """The product in the form in which it reaches a residual stream cheapest (no bias): a LazyDelta at
         decode sizes, where it can add itself to the stream; in bf16 partial sums over ranges of K (ops.PartialSums), which the
-        kernel of the next norm adds up, where ops.can_split_sums or, for a prompt's rows, ops.can_split_rows says so; else its result."""
+        kernel of the next norm adds up, where ops.can_split_sums or, for the row_bucket of a prompt's
+        rows, ops.can_split_rows says so; else its result."""
         from .base import LazyDelta
         M, (N, K) = x.shape[0], self.weight.shape
         plain = (self.bias is None and x.dim() == 2 and x.dtype == torch.bfloat16 and self.weight.dtype == torch.bfloat16
@@ -81,7 +82,7 @@ class Linear:
             return LazyDelta(x, self)
         if plain and ops.can_split_sums(M, N, K, x.dtype) and x.stride(1) == 1 and x.stride(0) % 8 == 0:
             return ops.linear_partial_sums(x, self.weight, self.streamed)
-        if plain and ops.can_split_rows(M, N, K, x.dtype) and x.stride(1) == 1 and x.stride(0) % 8 == 0:
+        if plain and ops.can_split_rows(ops.row_bucket(M), N, K, x.dtype) and x.stride(1) == 1 and x.stride(0) % 8 == 0:
             return ops.linear_split_rows(x, self.weight)
         if (self.bias is None and x.dim() == 2 and x.dtype == self.weight.dtype == torch.float32 and M > 0
                 and ops.can_norm_rows(M, N, x.dtype) and ops.f32_product_takes(self.weight)):

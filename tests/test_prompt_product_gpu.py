@@ -197,3 +197,23 @@ def test_few_tiles_of_long_rows_are_no_group():
     for n, M, N, K, take in ((2, 1024, 256, 1024, True), (2, 1024, 256, 1088, False), (2, 2048, 512, 4096, True), (2, 1024, 512, 4096, False), (3, 129, 256, 960, True),
                              (3, 129, 256, 1024, False), (3, 129, 1024, 4096, False), (3, 129, 1280, 4096, True), (4, 129, 256, 8192, True)):
         assert ops.group_rows(n, M, N, K) == take, (n, M, N, K)
+
+
+@pytest.mark.parametrize("M", [193, 250, 256, 300, 577, 2049])
+@pytest.mark.parametrize("act", ["gelu_erf", "relu2"])
+def test_an_eager_step_rounds_where_its_replay_does(M, act):
+    """The rows of a step are those of the captured step that replays it, which is longer: an activation is taken of rounded numbers in both or in neither."""
+    ops = _ops()
+    x, w, _ = _data(ops.row_bucket(M), 8192, 1024)
+    assert ops.unary_in_product(ops.row_bucket(M), 8192, 1024, act)
+    assert torch.equal(ops.linear_unary(x[:M], w, act), ops.linear_unary(x, w, act)[:M])
+
+
+@pytest.mark.parametrize("M,N,K,split", [(2600, 2048, 8192, False), (2560, 2048, 8192, True), (2100, 3072, 8192, False), (2048, 3072, 8192, True)])
+def test_an_eager_step_leaves_slabs_where_its_replay_does(M, N, K, split):
+    from bitnet_c_amd.parts.linear import Linear
+    ops = _ops()
+    x, w, _ = _data(ops.row_bucket(M), N, K)
+    lin = Linear()
+    lin.load(w, None, "cuda", torch.bfloat16)
+    assert isinstance(lin.lazy(x[:M]), ops.PartialSums) == isinstance(lin.lazy(x), ops.PartialSums) == split
