@@ -723,21 +723,21 @@ static int ag_launch_decode_dt(const GenDecodeArgs& a, int vd, bool once, dim3 g
     return BN_ERR_ARG;
 }
 
+struct AgFresh { int v_from_k; const float* wq; const float* wk; float eps; const float* inv_freq; int rope_dims; float temp_coef; int temp_every; };
+
 // Decode form: row b of q is sequence b's new token (seq_lens[b] keys in the cache, 0 for a padding row, whose output is
 // zeros).  n_splits > 1: part_o [n_seqs H n_splits, vd] and part_ml [n_seqs H n_splits, 2] float32 work space; the keys per
 // split are `chunk` (a multiple of BN_PAGE), or follow the longest sequence's key count in *max_len.
-// fresh: q's rows are projections (queries, keys, values) that this kernel norms (wq, wk [hs] or null), rotates (inv_freq or null:
-// rope_dims a multiple of 64, split-half pairs) and scales (temp_every > 0), and whose keys and values (v_from_k: the keys as projected) it
-// writes to the pages.
-extern "C" int bn_attn_general_decode(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
-                                      const void* v_pages, const int* block_table, int bt_stride, const int* seq_lens, int n_seqs,
-                                      int H, int Hkv, int hs, int vd, float scale, const float* dist_a, const float* dist_b,
-                                      int sink, const float* sink_values, int window, int keep_first, const void* gate, int gate_stride,
-                                      int n_splits, int chunk, float* part_o, float* part_ml, const int* max_len, int fresh, int v_from_k, const float* wq,
-                                      const float* wk, float eps, const float* inv_freq, int rope_dims, float temp_coef, int temp_every,
-                                      hipStream_t s) {
-    if (fresh && ((((uintptr_t)wq | (uintptr_t)wk | (uintptr_t)inv_freq) & 15) || q_stride < (H + Hkv) * hs + (v_from_k ? 0 : Hkv * vd) || (v_from_k && vd != hs) || (wq == nullptr) != (wk == nullptr) ||
-                  (inv_freq && (rope_dims <= 0 || rope_dims % 64 || rope_dims > hs)))) return BN_ERR_ARG;
+static int ag_decode(const void* q, int q_stride, void* out, int out_stride, const void* k_pages, const void* v_pages, const int* block_table, int bt_stride,
+                     const int* seq_lens, int n_seqs, int H, int Hkv, int hs, int vd, float scale, const float* dist_a, const float* dist_b, int sink,
+                     const float* sink_values, int window, int keep_first, const void* gate, int gate_stride, int n_splits, int chunk, float* part_o,
+                     float* part_ml, const int* max_len, const AgFresh* fresh, hipStream_t s) {
+    if (fresh) {
+        const AgFresh& f = *fresh;
+        if ((((uintptr_t)f.wq | (uintptr_t)f.wk | (uintptr_t)f.inv_freq) & 15) || q_stride < (H + Hkv) * hs + (f.v_from_k ? 0 : Hkv * vd) ||
+            (f.v_from_k && vd != hs) || (f.wq == nullptr) != (f.wk == nullptr) || (f.inv_freq && (f.rope_dims <= 0 || f.rope_dims % 64 || f.rope_dims > hs)))
+            return BN_ERR_ARG;
+    }
     if (n_seqs <= 0 || H <= 0 || Hkv <= 0 || H % Hkv || window < 0 || keep_first < 0 || n_splits < 1 || !bn_attn_general_supports(hs, vd)) return BN_ERR_ARG;
     if (!q || !out || !k_pages || !v_pages || !block_table || !seq_lens || (dist_b && !dist_a)) return BN_ERR_ARG;
     if (q_stride % 8 || out_stride % 4 || (((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages) & 15) || ((uintptr_t)out & 7))
@@ -753,9 +753,11 @@ extern "C" int bn_attn_general_decode(const void* q, int q_stride, void* out, in
     a.max_len = n_splits > 1 ? max_len : nullptr;
     a.q_stride = q_stride; a.out_stride = out_stride; a.bt_stride = bt_stride; a.H = H; a.Hkv = Hkv; a.n_splits = n_splits;
     a.chunk = chunk; a.window = window; a.sink = sink ? 1 : 0; a.sink_values = sink ? sink_values : nullptr; a.scale = scale;
+    const AgFresh f = fresh ? *fresh : AgFresh{};
     a.k_new = fresh ? (bf16*)k_pages : nullptr; a.v_new = fresh ? (bf16*)v_pages : nullptr;
-    a.v_col = (v_from_k ? H : H + Hkv) * hs;
-    a.wq = wq; a.wk = wk; a.eps = eps; a.inv_freq = inv_freq; a.rope_dims = inv_freq ? rope_dims : 0; a.temp_coef = temp_coef; a.temp_every = temp_every;
+    a.v_col = (f.v_from_k ? H : H + Hkv) * hs;
+    a.wq = f.wq; a.wk = f.wk; a.eps = f.eps; a.inv_freq = f.inv_freq; a.rope_dims = f.inv_freq ? f.rope_dims : 0;
+    a.temp_coef = f.temp_coef; a.temp_every = f.temp_every;
     const dim3 grid(n_seqs, Hkv * head_tiles, n_splits);
     const long long held = (long long)bt_stride * BN_PAGE, seen = (long long)window + keep_first;     // keys a sequence at the most
     const bool once = head_tiles == 1 && (window > 0 && seen < held ? seen : held) * n_seqs * Hkv * (hs + vd) * 2 <= (long long)AG_ONCE_MB << 20;
@@ -773,4 +775,27 @@ extern "C" int bn_attn_general_decode(const void* q, int q_stride, void* out, in
     hipLaunchKernelGGL(attn_general_combine_kernel, dim3(n_seqs * H), dim3(BN_WAVE), 0, s, (bf16*)out, out_stride, part_o, part_ml,
                        H, vd, n_splits, sink ? 1 : 0, sink ? sink_values : nullptr, (const bf16*)gate, gate_stride);
     return bn_launch_status();
+}
+
+extern "C" int bn_attn_general_decode(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
+                                      const void* v_pages, const int* block_table, int bt_stride, const int* seq_lens, int n_seqs,
+                                      int H, int Hkv, int hs, int vd, float scale, const float* dist_a, const float* dist_b,
+                                      int sink, const float* sink_values, int window, int keep_first, const void* gate, int gate_stride,
+                                      int n_splits, int chunk, float* part_o, float* part_ml, const int* max_len, hipStream_t s) {
+    return ag_decode(q, q_stride, out, out_stride, k_pages, v_pages, block_table, bt_stride, seq_lens, n_seqs, H, Hkv, hs, vd, scale, dist_a, dist_b, sink, sink_values,
+                     window, keep_first, gate, gate_stride, n_splits, chunk, part_o, part_ml, max_len, nullptr, s);
+}
+
+// The same over rows of projections (queries, keys, values) that the kernel norms (wq, wk [hs] or null), rotates (inv_freq or null: rope_dims a multiple of
+// 64, split-half pairs) and scales (temp_every > 0), and whose keys and values (v_from_k: the keys as projected) it writes to the pages.
+extern "C" int bn_attn_general_decode_fresh(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
+                                            const void* v_pages, const int* block_table, int bt_stride, const int* seq_lens, int n_seqs,
+                                            int H, int Hkv, int hs, int vd, float scale, const float* dist_a, const float* dist_b,
+                                            int sink, const float* sink_values, int window, int keep_first, const void* gate, int gate_stride,
+                                            int n_splits, int chunk, float* part_o, float* part_ml, const int* max_len, int v_from_k,
+                                            const float* wq, const float* wk, float eps, const float* inv_freq, int rope_dims, float temp_coef,
+                                            int temp_every, hipStream_t s) {
+    const AgFresh f = {v_from_k, wq, wk, eps, inv_freq, rope_dims, temp_coef, temp_every};
+    return ag_decode(q, q_stride, out, out_stride, k_pages, v_pages, block_table, bt_stride, seq_lens, n_seqs, H, Hkv, hs, vd, scale, dist_a, dist_b, sink, sink_values,
+                     window, keep_first, gate, gate_stride, n_splits, chunk, part_o, part_ml, max_len, &f, s);
 }

@@ -935,34 +935,47 @@ extern "C" int bn_lightning_prefers_chunks(int n_seqs, int H, int dk, int dv) {
     return (long long)n_seqs * H * ((dv + LA_CB - 1) / LA_CB) < 2LL * la_compute_units() ? 1 : 0;
 }
 
+static int la_args(LaArgs& a, const void* x, int ld, int q_col, int k_col, int v_col, const float* decay, float* o, float* state, long long state_stride,
+                   const int* tiles, int n_seqs, const int* seq_lens, const int* slot_ids, int H, int dk, int dv, int silu, float k_scale) {
+    if (n_seqs <= 0 || H <= 0 || !bn_lightning_supports(dk, dv) || !x || !decay || !o || !state || !slot_ids) return BN_ERR_ARG;
+    if (state_stride < (long long)H * dk * dv || q_col < 0 || k_col < 0 || v_col < 0) return BN_ERR_ARG;
+    if (ld < q_col + H * dk || ld < k_col + H * dk || ld < v_col + H * dv) return BN_ERR_ARG;
+    a.x = x; a.o = o; a.decay = decay; a.state = state; a.state_stride = (size_t)state_stride; a.tiles = tiles;
+    a.seq_lens = seq_lens; a.slot_ids = slot_ids; a.ld = ld; a.q_col = q_col; a.k_col = k_col; a.v_col = v_col;
+    a.H = H; a.dk = dk; a.dv = dv;
+    a.feed.silu = silu ? 1 : 0; a.feed.rope_dims = 0; a.feed.inv_freq = nullptr; a.feed.k_scale = k_scale;
+    return 0;
+}
+
+// The recurrence of a bf16 prompt step by blocks of 64 tokens, of rows that bn_lightning_blocks_take() takes; x, state and the rest as bn_lightning_scan's.
+// blocks: 0, every sequence from block to block, else what the step's sequences can be cut into together, with carry's blocks H (dk rounded up to 64 or
+// 128) (dv rounded up to 64 or multiples of 128) floats.
+extern "C" int bn_lightning_blocks(const void* x, int ld, int q_col, int k_col, int v_col, const float* decay, float* o, float* state,
+                                   long long state_stride, const int* tiles, int n_seqs, const int* slot_ids, int H, int dk, int dv, int silu,
+                                   float k_scale, int blocks, float* carry, hipStream_t s) {
+    LaArgs a;
+    if (int rc = la_args(a, x, ld, q_col, k_col, v_col, decay, o, state, state_stride, tiles, n_seqs, nullptr, slot_ids, H, dk, dv, silu, k_scale)) return rc;
+    if (!tiles || !bn_lightning_blocks_take(x, ld, q_col, k_col, dk, 0) || n_seqs > 65535 || blocks < 0 ||
+        (blocks > 0 && (!carry || (uintptr_t)carry % 16 != 0)))
+        return BN_ERR_ARG;
+    return lb_dispatch(a, n_seqs, blocks, carry, s);
+}
+
 // x [T, ld] holds q at q_col, k at k_col (H dk wide each) and v at v_col (H dv wide); n_seqs: tiles, or rows of a decode step;
 // prepared: room for the chunked form's copy of q, k and v, n_rows H (2 dks + dvs) floats with n_rows the rows of x and dks,
 // dvs the widths rounded up to a multiple of 4; null: the chain form also where the chunked form would run
 // silu: 1, q, k and v pass a silu, 0, they come as projected; inv_freq [rope_dims / 2] or null: the rotation of q and k, whose
 // positions the chunked form takes from positions [n_rows]; k_scale multiplies k
-// blocks: -1, or the blocks of 64 tokens of a prompt step that bn_lightning_blocks_take() takes: 0, every sequence from block to block, else what the step's
-// sequences can be cut into together, with carry's blocks H (dk rounded up to 64 or 128) (dv rounded up to 64 or multiples of 128) floats
 extern "C" int bn_lightning_scan(int dtype, const void* x, int ld, int q_col, int k_col, int v_col, const float* decay, float* o,
                                  float* state, long long state_stride, const int* tiles, int n_seqs, const int* seq_lens,
                                  const int* slot_ids, int H, int dk, int dv, int n_rows, float* prepared, int silu,
-                                 const float* inv_freq, int rope_dims, const int* positions, float k_scale, int blocks, float* carry,
-                                 hipStream_t s) {
+                                 const float* inv_freq, int rope_dims, const int* positions, float k_scale, hipStream_t s) {
     if (inv_freq ? (rope_dims < 2 || rope_dims % 2 || rope_dims > dk) : rope_dims != 0) return BN_ERR_ARG;
-    if (n_seqs <= 0 || H <= 0 || !bn_lightning_supports(dk, dv) || !x || !decay || !o || !state || !slot_ids) return BN_ERR_ARG;
-    if ((!tiles && !seq_lens) || state_stride < (long long)H * dk * dv || q_col < 0 || k_col < 0 || v_col < 0) return BN_ERR_ARG;
-    if (ld < q_col + H * dk || ld < k_col + H * dk || ld < v_col + H * dv) return BN_ERR_ARG;
+    if (!tiles && !seq_lens) return BN_ERR_ARG;
     LaArgs a;
-    a.x = x; a.o = o; a.decay = decay; a.state = state; a.state_stride = (size_t)state_stride; a.tiles = tiles;
-    a.seq_lens = seq_lens; a.slot_ids = slot_ids; a.ld = ld; a.q_col = q_col; a.k_col = k_col; a.v_col = v_col;
-    a.H = H; a.dk = dk; a.dv = dv;
-    a.feed.silu = silu ? 1 : 0; a.feed.rope_dims = rope_dims; a.feed.inv_freq = inv_freq; a.feed.k_scale = k_scale;
+    if (int rc = la_args(a, x, ld, q_col, k_col, v_col, decay, o, state, state_stride, tiles, n_seqs, seq_lens, slot_ids, H, dk, dv, silu, k_scale)) return rc;
+    a.feed.rope_dims = rope_dims; a.feed.inv_freq = inv_freq;
     if (dtype != BN_DT_F32 && dtype != BN_DT_BF16) return BN_ERR_DTYPE;
-    if (blocks >= 0) {
-        if (!tiles || dtype != BN_DT_BF16 || !bn_lightning_blocks_take(x, ld, q_col, k_col, dk, rope_dims) || n_seqs > 65535 ||
-            (blocks > 0 && (!carry || (uintptr_t)carry % 16 != 0)))
-            return BN_ERR_ARG;
-        return lb_dispatch(a, n_seqs, blocks, carry, s);
-    }
     if (tiles && prepared && bn_lightning_chunked(dk, dv)) {
         if (n_rows <= 0 || (uintptr_t)prepared % 16 != 0 || (inv_freq && !positions)) return BN_ERR_ARG;
         return lc_dispatch(dtype, a, n_seqs, n_rows, positions, prepared, s);

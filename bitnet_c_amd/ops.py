@@ -91,8 +91,11 @@ _SIGNATURES = {
                                    c_void_p],
         "bn_attn_general_decode": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int,
                                    c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_int,
-                                   c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_int,
-                                   c_float, c_int, c_void_p],
+                                   c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
+        "bn_attn_general_decode_fresh": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int,
+                                         c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_int,
+                                         c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_float, c_void_p, c_int,
+                                         c_float, c_int, c_void_p],
     },
     "hyper": {
         "bn_hc_step": [c_int, c_int, c_void_p, c_longlong, c_void_p, c_longlong, c_void_p, c_int, c_longlong, c_void_p, c_void_p,
@@ -125,7 +128,9 @@ _SIGNATURES = {
         "bn_lightning_columns": [c_int, c_int, c_int, c_int],
         "bn_lightning_scan": [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p,
                               c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p,
-                              c_float, c_int, c_void_p, c_void_p],
+                              c_float, c_void_p],
+        "bn_lightning_blocks": [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_int, c_void_p,
+                                c_int, c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p],
         "bn_lightning_blocks_take": [c_void_p, c_int, c_int, c_int, c_int, c_int],
         "bn_row_norm_gate": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_float, c_int, c_void_p],
     },
@@ -2133,11 +2138,9 @@ def on_16_bytes(*tensors) -> bool:
     return all(t is None or t.data_ptr() % 16 == 0 for t in tensors)
 
 
-def _fresh_args(f: Optional[FreshRows]) -> tuple:
-    if f is None:
-        return 0, 0, None, None, 0.0, None, 0, 0.0, 0
+def _fresh_args(f: FreshRows) -> tuple:
     ptr = lambda t: t.data_ptr() if t is not None else None
-    return 1, int(f.v_from_k), ptr(f.q_weight), ptr(f.k_weight), float(f.eps), ptr(f.inv_freq), int(f.rope_dims), float(f.temp_coef), int(f.temp_every)
+    return int(f.v_from_k), ptr(f.q_weight), ptr(f.k_weight), float(f.eps), ptr(f.inv_freq), int(f.rope_dims), float(f.temp_coef), int(f.temp_every)
 
 
 def attention_general_decode(qkv: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
@@ -2194,12 +2197,13 @@ def attention_general_decode(qkv: torch.Tensor, out: torch.Tensor, k_pages: torc
         part_ml = torch.empty((T * H * n_splits, 2), dtype=torch.float32, device=qkv.device)
     if T == 0:
         return
-    _check(_fn("attn_mfma_general", "bn_attn_general_decode")(
+    _check(_fn("attn_mfma_general", "bn_attn_general_decode" if fresh is None else "bn_attn_general_decode_fresh")(
         qkv.data_ptr(), _rows(qkv, "qkv"), out.data_ptr(), H * v_dim, k_pages.data_ptr(), v_pages.data_ptr(),
         block_table.data_ptr(), block_table.shape[1], seq_lens.data_ptr(), T, H, Hkv, hs, v_dim, float(scale),
         da, db, *_sink_args(sink, H, "attention_general_decode"), int(window), int(keep_first), gp, gld, int(n_splits), int(chunk), part_o.data_ptr() if part_o is not None else None,
         part_ml.data_ptr() if part_ml is not None else None,
-        max_len_dev.data_ptr() if (max_len_dev is not None and n_splits > 1) else None, *_fresh_args(fresh), _stream()),
+        max_len_dev.data_ptr() if (max_len_dev is not None and n_splits > 1) else None,
+        *(_fresh_args(fresh) if fresh is not None else ()), _stream()),
         "attention_general_decode")
 
 
@@ -2745,8 +2749,6 @@ def lightning_scan(x: torch.Tensor, q_col: int, k_col: int, v_col: int, decay: t
             raise KernelError(f"lightning_scan: {rope_dims} rotated dimensions of {dk}, positions {tuple(positions.shape)} for {T} rows")
     o = torch.empty((T, H * dv), dtype=torch.float32, device=x.device)
     if T and n_seqs:
-        prepared = carry = None
-        blocks = -1
         if (tiles is not None and chain is not True and x.dtype == torch.bfloat16
                 and _fn("lightning", "bn_lightning_blocks_take")(x.data_ptr(), ld, int(q_col), int(k_col), dk, rope_dims)
                 and (chain is False or lightning_takes_blocks(sizes or (T, n_seqs), H, dk, dv))):
@@ -2754,7 +2756,13 @@ def lightning_scan(x: torch.Tensor, q_col: int, k_col: int, v_col: int, decay: t
             most = _pieces_of(T, n_seqs, LIGHTNING_BLOCK)
             blocks = most if (pieces if pieces is not None else lightning_in_pieces(T, n_seqs, H, dv)) and most * state_floats * 4 <= SCAN_PIECES_BYTES else 0
             carry = torch.empty(blocks * state_floats, dtype=torch.float32, device=x.device) if blocks else None
-        elif tiles is not None and chain is not True and lightning_chunked(dk, dv) and (
+            _check(_fn("lightning", "bn_lightning_blocks")(x.data_ptr(), ld, int(q_col), int(k_col), int(v_col), decay.data_ptr(), o.data_ptr(),
+                                                           state.data_ptr(), stride, tl, n_seqs, slot_ids.data_ptr(), H, dk, dv, int(bool(silu)),
+                                                           float(k_scale), blocks, carry.data_ptr() if carry is not None else None, _stream()),
+                   "lightning_blocks")
+            return o
+        prepared = None
+        if tiles is not None and chain is not True and lightning_chunked(dk, dv) and (
                 chain is False or _fn("lightning", "bn_lightning_prefers_chunks")(n_seqs, H, dk, dv)):
             # the chunked form's own copy of the step's q, k and v: what they pass applied, float32, head by head
             prepared = torch.empty(H * T * (2 * ((dk + 3) // 4 * 4) + (dv + 3) // 4 * 4), dtype=torch.float32, device=x.device)
@@ -2763,8 +2771,7 @@ def lightning_scan(x: torch.Tensor, q_col: int, k_col: int, v_col: int, decay: t
                                                      slot_ids.data_ptr(), H, dk, dv, T,
                                                      prepared.data_ptr() if prepared is not None else None, int(bool(silu)),
                                                      inv_freq.data_ptr() if rope_dims else None, rope_dims,
-                                                     positions.data_ptr() if rope_dims else None, float(k_scale), blocks,
-                                                     carry.data_ptr() if carry is not None else None, _stream()),
+                                                     positions.data_ptr() if rope_dims else None, float(k_scale), _stream()),
                "lightning_scan")
     return o
 
