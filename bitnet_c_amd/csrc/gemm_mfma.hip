@@ -329,7 +329,8 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_mfma_kernel(const bf16* __res
 #define GM_RELU2 6                    // max(sum, 0)^2
 #define GM_GATED_RELU2 7              // max(gate, 0)^2 * up
 
-// z (1 + erf(z / sqrt 2)) / 2 in 17 instructions (erff's alone are 40, with a branch): with x = |z| / sqrt 2 and t = 1 / (1 + 0.46 x),
+// z (1 + erf(z / sqrt 2)) / 2 in 17 instructions (erff's alone are 40, with a branch), by the known form erfc(x) = t exp(-x^2 + p(t)), t = 1 / (1 + c x), with a
+// polynomial of its own (below): with x = |z| / sqrt 2 and t = 1 / (1 + 0.46 x),
 // erfc(x) / 2 = t 2^(p(t) - x^2 / ln 2), p the polynomial of degree 7 that interpolates log2(exp(x^2) erfc(x) / (2 t)) at the Chebyshev
 // points of x in [0, 7] (2.6e-7 off at most).  In float32 within 8e-7 of the value above -2, within 2e-5 of it at -13, where 1 + erff is 0.
 __device__ __forceinline__ float gm_gelu_erf(float z) {

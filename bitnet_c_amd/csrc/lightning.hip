@@ -584,7 +584,9 @@ __device__ __forceinline__ LaRange lb_range(const int* tiles, int n_tiles, int a
     return r;
 }
 
-// Read before the next branch: this compiler (ROCm 7.2) leaves out the wait between a matrix product and a read of its result that lies behind a branch.
+// A product's result that is next read behind a branch is named here, in front of it: with a short branch between the two, an earlier form of these kernels
+// compiled (ROCm 7.2) to a read of the result's last register before it was written.  In the kernels as they are compiled now, on every path, at least the
+// 10 wait states that a read behind v_mfma_f32_16x16x4_f32 needs lie in between (8 behind the bf16 instruction of the other files' kernels).
 __device__ __forceinline__ void lb_settle(f32x4& x) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -736,6 +738,10 @@ __global__ __launch_bounds__(LA_THREADS, 2) void lightning_block_kernel(LbArgs b
             }
             lc_barrier();
             // ---- o = A V + d^(i+1) Q S; an infinity or a NaN among the values must not meet the zeros of the tokens before it ----
+#pragma unroll
+            for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+                for (int ct = 0; ct < NCT; ++ct) lb_settle(qs[ib][ct]);
             bool fine = true;
 #pragma unroll
             for (int ct = 0; ct < NCT; ++ct)

@@ -488,8 +488,9 @@ template <int L> __device__ __forceinline__ float wkv_partner(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), how, 0xF, 0xF, true));
 }
 
-// Matrix products' results are read before the next branch: this compiler (ROCm 7.2) leaves out the wait between a product and a read of it that
-// lies behind a branch, and the last of its registers is then read before it is written.
+// A product's result that is next read behind a branch is named here, in front of it: with a short branch between the two, an earlier form of this kernel
+// compiled (ROCm 7.2) to a read of the result's last register before it was written.  In the kernels as they are compiled now, on every path, at least the
+// 10 wait states that a read behind v_mfma_f32_16x16x4_f32 needs lie in between.
 __device__ __forceinline__ void wkv_settle(wkv_f4& x) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
