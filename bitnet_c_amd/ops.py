@@ -507,7 +507,7 @@ def _tiled(x, w, out_dtype):
 
 def _f32_product(x, w, glu: bool = False, activation: str = "silu", form: int = 0, streamed: Optional["StreamedWeight"] = None,
                  norm: Optional["StreamNorm"] = None, into: Optional[torch.Tensor] = None):
-    """x . w^T in float32 on the float32 matrix instruction (gemm_f32.hip), or with glu act(gate) * up for w = gate and up
+    """x . w^T in float32 on the matrix cores (gemm_f32.hip: every number in three bf16 parts, float32 sums), or with glu act(gate) * up for w = gate and up
     rows interleaved in blocks of 8; None for weights that the kernels do not take (rows that are not whole 16-byte groups).
     Whether they do depends on the weights alone, and every form of the kernels has one order of summation, so a row's bits do
     not depend on the step it comes in.  form: 0, by the sizes; the others are bn_gemm_f32's, for tests.  streamed: w's
@@ -537,7 +537,7 @@ def _f32_product(x, w, glu: bool = False, activation: str = "silu", form: int = 
 
 
 def f32_product_takes(w: torch.Tensor) -> bool:
-    """Whether the float32 matrix instruction's kernels take weights w [N, K] (rows of whole 16-byte groups)."""
+    """Whether gemm_f32.hip's kernels take weights w [N, K] (rows of whole 16-byte groups)."""
     return bool(_fn("gemm_f32", "bn_gemm_f32_supports")(w.shape[0], w.shape[1], _rows(w, "w"), w.data_ptr()))
 
 
@@ -807,7 +807,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, *, allow_library: O
            streamed: Optional[StreamedWeight] = None) -> torch.Tensor:
     """y[M, N] = x[M, K] . w[N, K]^T.  streamed: w's streamed copy, which the kernel of up to 16 rows reads instead.
 
-    float32: the float32 matrix instruction (gemm_f32.hip; float32 products and sums in one order whatever M is); rows that
+    float32: gemm_f32.hip (all 24 bits of the operands, float32 sums in one order whatever M is); rows that
     are not whole 16-byte groups go to the tiled kernel (plain fmaf, a fixed order of summation).
     bf16: up to 16 rows (one MFMA tile of activations) the matrix-core kernel that streams
     the weights once; above that the library's matrix product, which from 32 rows on is about

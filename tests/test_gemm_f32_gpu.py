@@ -210,3 +210,53 @@ def test_norms_of_narrow_rows_stay_in_front_of_streamed_products(K, monkeypatch)
         calls.clear()
         assert torch.equal(lin(ops.stream_norm(x.cuda(), nw, 1e-5)), want)
         assert len(calls) == (0 if keep and 512 <= K < 1024 else 1)
+
+
+# the forms beyond the tiles' first ones: rows at the edges of 32 and 64, columns one past a tile of 16, 32, 64 and 128; K: one block of 32, a
+# chunk's remainder, as many chunks as the groups and waves that take them in turns, one more, and one round of eight more
+@pytest.mark.parametrize("M,N", [(17, 1), (33, 65), (64, 129), (65, 33), (129, 300)])
+@pytest.mark.parametrize("K", [4, 32, 36, 128, 160, 256, 512, 640, 1028, 1152, 2176])
+def test_forms_that_share_out_the_chunks(M, N, K):
+    ops = _ops()
+    x, w = _data(M, N, K, M + 3 * N + K)
+    wide, tall = torch.full((M + 1, K + 8), float("nan"), device="cuda"), torch.full((N + 1, K + 4), float("nan"), device="cuda")
+    wide[:M, :K], tall[:N, :K] = x.cuda(), w.cuda()
+    xd, wd = wide[:M, :K], tall[:N, :K]
+    want = ops._f32_product(xd, wd, form=4)
+    # _bound's links: a chunk is 24 instructions here; what the three products that are left out of nine come to is one link more at the most
+    assert torch.all((want.cpu().double() - x.double() @ w.double().t()).abs() <= _bound(x, w))
+    for form in (1, 5, 9, 10) + ((6, 8, 11, 12) if K % 32 == 0 else ()):
+        if form > 1 or M <= 64:
+            assert torch.equal(ops._f32_product(xd, wd, form=form), want), form
+    if N % 16 == 0:
+        glu = ops._f32_product(xd, wd, True, "silu", form=4)
+        for form in (9, 10) + ((11, 12) if K % 32 == 0 else ()):
+            assert torch.equal(ops._f32_product(xd, wd, True, "silu", form=form), glu), form
+
+
+@pytest.mark.parametrize("M", [1, 3, 8, 16, 40])
+def test_infinite_operands_give_infinite_sums(M):
+    """An infinite number has no second part, and the nearest bf16 number of the largest float32 ones is infinite: sums with either
+    come out as the float32 operations give them, and the others keep their bits."""
+    ops = _ops()
+    x, w = _data(M, 48, 256, M)
+    w[7] = w[7].abs()
+    plain = ops._f32_product(x.cuda(), w.cuda()).cpu()
+    x[M // 2, 9], w[3, 200], w[5] = float("inf"), float("-inf"), 0.0
+    w[5, 77], x[:, 77] = 0.25, 3.4e38
+    want = x.double() @ w.double().t()
+    sw = ops.stream_copy(w.cuda())
+    runs = [ops._f32_product(x.cuda(), w.cuda(), form=f).cpu() for f in (1, 2, 4, 5, 6, 8, 9, 10, 11, 12)]
+    runs += [ops.linear(x.cuda(), w.cuda(), streamed=sw).cpu()]
+    for i, y in enumerate(runs):
+        assert torch.equal(y.isnan(), want.isnan()), i
+        big = want.float().isinf()
+        assert torch.equal(y[big & ~want.isnan()], want.float()[big & ~want.isnan()]), i
+        assert torch.all((y[:, 5] - 0.25 * 3.4e38).abs()[torch.arange(M) != M // 2] <= 0.25 * 3.4e38 * 2.0 ** -20), i
+    x2, w2 = _data(M, 48, 256, M)
+    w2[7] = w2[7].abs()
+    x2[M // 2, 9] = float("inf")
+    for f in (1, 4, 6, 9):
+        y = ops._f32_product(x2.cuda(), w2.cuda(), form=f).cpu()
+        rest = torch.arange(M) != M // 2
+        assert torch.equal(y[rest], plain[rest]) and bool(y[M // 2].isinf().all()) and float(y[M // 2, 7]) == float("inf"), f
