@@ -1371,47 +1371,54 @@ __global__ __launch_bounds__(WHOLE ? 512 : 256) void attn_mfma_decode_kernel(Mfm
     }
 }
 
-// out[row, d] = sum_s e^{m_s - m} o_s[d] / sum_s e^{m_s - m} l_s: one wave per row, the weights
-// of all splits computed at once (one lane per split), the sums in split order.
+// out[row, d] = sum_s e^{m_s - m} o_s[d] / sum_s e^{m_s - m} l_s: one wave per row, the weights of all splits computed at once
+// (one lane per split), the sums in split order.  A launch of a few hundred waves is bound by its chain of waits, not by its
+// bytes: all S >= n_splits sums are asked for beside the weights' maxima (the last split's again past the end, and what a split
+// without keys holds is dropped: two trips to memory become one), and a weight comes out of its lane with a v_readlane instead of
+// through shared memory's crossbar, whose wait in the sum of the denominators came once a split.
+//   us inside a step, before -> this: 32 rows of 32 splits 6.9 -> 4.7, 256 of 4 4.7 -> 4.2, 64 of 3 3.9 -> 3.6 (a launch that does
+//   nothing: 2.5).
+struct __attribute__((packed, aligned(4))) TwoFloats { float x, y; };      // in one load, also where the caller's room is not on 8 bytes
+template <int S, int V>
 __global__ __launch_bounds__(64) void attn_mfma_combine_kernel(bf16* __restrict__ out, int out_stride,
                                                                const float* __restrict__ part_o,
-                                                               const float* __restrict__ part_ml, int H, int hs,
-                                                               int n_splits) {
+                                                               const float* __restrict__ part_ml, int H, int n_splits) {
+    constexpr int HS = 64 * V;
     const int row = blockIdx.x, lane = threadIdx.x;
     const int tok = row / H, head = row - tok * H;
-    const float* ml = part_ml + (size_t)row * n_splits * 2;
-    float ms = -INFINITY, ls = 0.f;
-    if (lane < n_splits) { ms = ml[2 * lane]; ls = ml[2 * lane + 1]; }
-    const float M = wave_max(ms);
-    const float w = (M == -INFINITY || ms == -INFINITY) ? 0.f : expf(ms - M);
-    // splits behind the last one with keys (a table much wider than the sequences are long) add nothing: stop there
-    const unsigned long long live = __ballot(w != 0.f);
-    const int n_live = live ? 64 - __builtin_clzll(live) : 0;
-    float den = 0.f;
-    for (int s = 0; s < n_live; ++s) den = fmaf(__shfl(w, s, BN_WAVE), __shfl(ls, s, BN_WAVE), den);
-    const float inv = den > 0.f ? 1.0f / den : 0.f;
-    // dimensions lane and lane + 64 together, sixteen splits' loads in flight at once (a split without keys is not read)
-    const bool two = lane + 64 < hs;
-    float num0 = 0.f, num1 = 0.f;
-    const float* po = part_o + (size_t)row * n_splits * hs + lane;
-    for (int s0 = 0; s0 < n_live; s0 += 16) {
-        float v0[16], v1[16], wj[16];
+    const TwoFloats ml = reinterpret_cast<const TwoFloats*>(part_ml)[(size_t)row * n_splits + min(lane, n_splits - 1)];
+    const float* po = part_o + (size_t)row * n_splits * HS + V * lane;
+    float v[S][V];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            wj[j] = __shfl(w, min(s0 + j, 63), BN_WAVE);
-            const bool in = s0 + j < n_live && wj[j] != 0.f;
-            v0[j] = (in && lane < hs) ? po[(size_t)(s0 + j) * hs] : 0.f;
-            v1[j] = (in && two) ? po[(size_t)(s0 + j) * hs + 64] : 0.f;
-        }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {                                     // then the sums, in split order
-            num0 = fmaf(wj[j], v0[j], num0);
-            num1 = fmaf(wj[j], v1[j], num1);
+    for (int s = 0; s < S; ++s) {
+        const float* from = po + (size_t)min(s, n_splits - 1) * HS;
+        if constexpr (V == 2) {
+            const TwoFloats two = *reinterpret_cast<const TwoFloats*>(from);
+            v[s][0] = two.x; v[s][1] = two.y;
+        } else {
+            v[s][0] = *from;
         }
     }
-    bf16* o = out + (size_t)tok * out_stride + (size_t)head * hs;
-    if (lane < hs) o[lane] = __float2bfloat16(num0 * inv);
-    if (two) o[lane + 64] = __float2bfloat16(num1 * inv);
+    __builtin_amdgcn_sched_barrier(0);                                     // all asked for before anything is waited for
+    const float ms = lane < n_splits ? ml.x : -INFINITY;
+    const float M = wave_max(ms);
+    const float w = (M == -INFINITY || ms == -INFINITY) ? 0.f : expf(ms - M);
+    auto of = [](float x, int s) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), s)); };
+    float den = 0.f, num[V] = {};
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const float ws = of(w, s);
+        den = fmaf(ws, ws != 0.f ? of(ml.y, s) : 0.f, den);                // (no branch: a load would be moved behind it)
+#pragma unroll
+        for (int u = 0; u < V; ++u) num[u] = fmaf(ws, ws != 0.f ? v[s][u] : 0.f, num[u]);
+    }
+    const float inv = den > 0.f ? 1.0f / den : 0.f;
+    bf16* o = out + (size_t)tok * out_stride + (size_t)head * HS + V * lane;
+    bf16 r[V];
+#pragma unroll
+    for (int u = 0; u < V; ++u) r[u] = __float2bfloat16(num[u] * inv);
+    if constexpr (V == 2) *reinterpret_cast<uint32_t*>(o) = __builtin_bit_cast(uint32_t, r);
+    else *o = r[0];
 }
 
 // 1 when the matrix-core kernels take this shape
@@ -1570,9 +1577,17 @@ static int attn_mfma_launch(const void* q, int q_stride, void* out, int out_stri
     if (whole) return once ? pick(std::true_type(), std::true_type()) : pick(std::true_type(), std::false_type());
     const int rc = once ? pick(std::false_type(), std::true_type()) : pick(std::false_type(), std::false_type());
     if (rc != 0 || n_splits == 1) return rc;
-    hipLaunchKernelGGL(attn_mfma_combine_kernel, dim3(n_tokens * H), dim3(64), 0, s, (bf16*)out, out_stride, part_o,
-                       part_ml, H, hs, n_splits);
-    return bn_launch_status();
+    auto combine = [&](auto most) {
+        constexpr int S = decltype(most)::value;
+        auto kernel = hs == 64 ? attn_mfma_combine_kernel<S, 1> : attn_mfma_combine_kernel<S, 2>;
+        hipLaunchKernelGGL(kernel, dim3(n_tokens * H), dim3(64), 0, s, (bf16*)out, out_stride, part_o, part_ml, H, n_splits);
+        return bn_launch_status();
+    };
+    if (n_splits <= 4) return combine(std::integral_constant<int, 4>());
+    if (n_splits <= 8) return combine(std::integral_constant<int, 8>());
+    if (n_splits <= 16) return combine(std::integral_constant<int, 16>());
+    if (n_splits <= 32) return combine(std::integral_constant<int, 32>());
+    return combine(std::integral_constant<int, 64>());
 }
 
 extern "C" int bn_attn_mfma(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,

@@ -90,9 +90,8 @@ __device__ __forceinline__ void ag_scores(float (&s)[8], const f32x4& s0, const 
 
 // four consecutive outputs of a head and, with a gate, times the sigmoids of the four gate values beside them:
 // one 8-byte store
-__device__ __forceinline__ void ag_store4(bf16* op, const bf16* gp, float x0, float x1, float x2, float x3) {
-    if (gp) {
-        const uint2 gw = *reinterpret_cast<const uint2*>(gp);
+__device__ __forceinline__ void ag_store4(bf16* op, bool gated, uint2 gw, float x0, float x1, float x2, float x3) {
+    if (gated) {
         x0 /= 1.0f + __expf(-bf16lo_to_f32(gw.x)); x1 /= 1.0f + __expf(-bf16hi_to_f32(gw.x));
         x2 /= 1.0f + __expf(-bf16lo_to_f32(gw.y)); x3 /= 1.0f + __expf(-bf16hi_to_f32(gw.y));
     }
@@ -101,6 +100,9 @@ __device__ __forceinline__ void ag_store4(bf16* op, const bf16* gp, float x0, fl
     w.x = (uint32_t)__builtin_bit_cast(unsigned short, o0) | ((uint32_t)__builtin_bit_cast(unsigned short, o1) << 16);
     w.y = (uint32_t)__builtin_bit_cast(unsigned short, o2) | ((uint32_t)__builtin_bit_cast(unsigned short, o3) << 16);
     *reinterpret_cast<uint2*>(op) = w;
+}
+__device__ __forceinline__ void ag_store4(bf16* op, const bf16* gp, float x0, float x1, float x2, float x3) {
+    ag_store4(op, gp != nullptr, gp ? *reinterpret_cast<const uint2*>(gp) : make_uint2(0u, 0u), x0, x1, x2, x3);
 }
 
 // A workgroup is 4, 2 or 1 heads of one kv head (a wave each); they stage a block of keys and values through shared memory, the
@@ -596,41 +598,46 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
 }
 
 // out[row, d] = sum_s e^(m_s - m) o_s[d] / (sum_s e^(m_s - m) l_s [+ e^(-m) for the sink]) [sigmoid(gate)], the splits in index order;
-// one wave a (token, head) row: the splits' factors are formed a lane a split, then a lane takes four value columns at a time
-// with several splits' loads in flight (a split without keys holds zeros, and its factor is 0)
+// one wave a (token, head) row: the splits' factors are formed a lane a split, and a lane takes four value columns.  Bound by its
+// chain of waits: all S >= n_splits sums (the last split's again past the end) and the gate are asked for beside the factors' maxima,
+// and a factor comes out of its lane with a v_readlane.  A split without keys holds zeros, and its factor is 0.  (us inside a step,
+// 64 rows of 7 splits of 128 columns: 5.4 -> 4.7.)
 #define AG_MAX_SPLITS BN_WAVE
+template <int S>
 __global__ __launch_bounds__(BN_WAVE) void attn_general_combine_kernel(bf16* __restrict__ out, int out_stride,
                                                                        const float* __restrict__ part_o,
                                                                        const float* __restrict__ part_ml, int H, int vd,
                                                                        int n_splits, int sink,
                                                                        const float* __restrict__ sink_values,
                                                                        const bf16* __restrict__ gate, int gate_stride) {
-    __shared__ float factor[AG_MAX_SPLITS], share[AG_MAX_SPLITS];
     const int row = blockIdx.x, tok = row / H, head = row - tok * H, lane = threadIdx.x;
-    const float* ml = part_ml + (size_t)row * n_splits * 2;
+    const int mine_at = min(lane, n_splits - 1), d = min(4 * lane, vd - 4);              // vd <= 256: four columns a lane
+    const float* ml = part_ml + ((size_t)row * n_splits + mine_at) * 2;
+    const float own_m = ml[0], own_l = ml[1];
+    const float* op0 = part_o + (size_t)row * n_splits * vd + d;
+    float4 o[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) o[s] = *reinterpret_cast<const float4*>(op0 + (size_t)min(s, n_splits - 1) * vd);
+    const uint2 gw = gate ? *reinterpret_cast<const uint2*>(gate + (size_t)tok * gate_stride + (size_t)head * vd + d) : make_uint2(0u, 0u);
     const float sv = sink && sink_values ? sink_values[head] : 0.f;
-    const float mine = lane < n_splits ? ml[2 * lane] : -INFINITY, sum = lane < n_splits ? ml[2 * lane + 1] : 0.f;
+    __builtin_amdgcn_sched_barrier(0);                   // all asked for before anything is waited for
+    const float mine = lane < n_splits ? own_m : -INFINITY, sum = lane < n_splits ? own_l : 0.f;
     const float m = wave_max(sink ? fmaxf(sv, mine) : mine);
-    const float f = m != -INFINITY ? expf(mine - m) : 0.f;
-    factor[lane] = f;
-    share[lane] = f * sum;
-    __syncthreads();
+    const float f = m != -INFINITY ? expf(mine - m) : 0.f, share = f * sum;
+    auto of = [](float x, int s) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), s)); };
     float den = sink ? expf(sv - m) : 0.f;
-    for (int s = 0; s < n_splits; ++s) den += share[s];
-    const float inv = den > 0.f ? 1.0f / den : 0.f;
-    for (int d = 4 * lane; d < vd; d += 4 * BN_WAVE) {
-        float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
-        const float* op0 = part_o + (size_t)row * n_splits * vd + d;
-#pragma unroll 8
-        for (int s = 0; s < n_splits; ++s) {
-            const float4 o = *reinterpret_cast<const float4*>(op0 + (size_t)s * vd);
-            const float w = factor[s];
-            num.x = fmaf(w, o.x, num.x); num.y = fmaf(w, o.y, num.y); num.z = fmaf(w, o.z, num.z); num.w = fmaf(w, o.w, num.w);
-        }
-        bf16* op = out + (size_t)tok * out_stride + (size_t)head * vd + d;
-        ag_store4(op, gate ? gate + (size_t)tok * gate_stride + (size_t)head * vd + d : nullptr, num.x * inv, num.y * inv, num.z * inv,
-                  num.w * inv);
+    float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const float w = of(f, s);                        // 0 past n_splits, and so is the share
+        const bool in = s < n_splits;                    // (no branch: a load would be moved behind it)
+        den += of(share, s);
+        num.x = fmaf(w, in ? o[s].x : 0.f, num.x); num.y = fmaf(w, in ? o[s].y : 0.f, num.y);
+        num.z = fmaf(w, in ? o[s].z : 0.f, num.z); num.w = fmaf(w, in ? o[s].w : 0.f, num.w);
     }
+    if (4 * lane >= vd) return;
+    const float inv = den > 0.f ? 1.0f / den : 0.f;
+    ag_store4(out + (size_t)tok * out_stride + (size_t)head * vd + d, gate != nullptr, gw, num.x * inv, num.y * inv, num.z * inv, num.w * inv);
 }
 
 static bool ag_size(int x) { return x == 32 || x == 64 || x == 96 || x == 128 || x == 192 || x == 256; }
@@ -772,9 +779,14 @@ static int ag_decode(const void* q, int q_stride, void* out, int out_stride, con
         case 8: rc = ag_launch_decode_dt<8>(a, vd, once, grid, s); break;
     }
     if (rc != 0 || n_splits == 1) return rc;
-    hipLaunchKernelGGL(attn_general_combine_kernel, dim3(n_seqs * H), dim3(BN_WAVE), 0, s, (bf16*)out, out_stride, part_o, part_ml,
-                       H, vd, n_splits, sink ? 1 : 0, sink ? sink_values : nullptr, (const bf16*)gate, gate_stride);
-    return bn_launch_status();
+    auto combine = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(n_seqs * H), dim3(BN_WAVE), 0, s, (bf16*)out, out_stride, part_o, part_ml, H, vd, n_splits,
+                           sink ? 1 : 0, sink ? sink_values : nullptr, (const bf16*)gate, gate_stride);
+        return bn_launch_status();
+    };
+    return n_splits <= 4 ? combine(attn_general_combine_kernel<4>) : n_splits <= 8 ? combine(attn_general_combine_kernel<8>) :
+           n_splits <= 16 ? combine(attn_general_combine_kernel<16>) : n_splits <= 32 ? combine(attn_general_combine_kernel<32>) :
+           combine(attn_general_combine_kernel<AG_MAX_SPLITS>);
 }
 
 extern "C" int bn_attn_general_decode(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
