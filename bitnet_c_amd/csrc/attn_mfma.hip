@@ -1376,8 +1376,7 @@ __global__ __launch_bounds__(WHOLE ? 512 : 256) void attn_mfma_decode_kernel(Mfm
 // bytes: all S >= n_splits sums are asked for beside the weights' maxima (the last split's again past the end, and what a split
 // without keys holds is dropped: two trips to memory become one), and a weight comes out of its lane with a v_readlane instead of
 // through shared memory's crossbar, whose wait in the sum of the denominators came once a split.
-//   us inside a step, before -> this: 32 rows of 32 splits 6.9 -> 4.7, 256 of 4 4.7 -> 4.2, 64 of 3 3.9 -> 3.6 (a launch that does
-//   nothing: 2.5).
+//   us inside a step, before -> this: 32 rows of 32 splits 6.9 -> 4.7, 64 of 3 3.9 -> 3.6, 256 of 4 4.7 -> 4.7 (its sums come from memory).
 struct __attribute__((packed, aligned(4))) TwoFloats { float x, y; };      // in one load, also where the caller's room is not on 8 bytes
 template <int S, int V>
 __global__ __launch_bounds__(64) void attn_mfma_combine_kernel(bf16* __restrict__ out, int out_stride,
