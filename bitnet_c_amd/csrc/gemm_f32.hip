@@ -46,7 +46,8 @@ struct GfArgs {
     int M, N, K;                     // N: rows of W
     int ldx, ldw, ldy;
     int cols;                        // columns a workgroup of the streaming kernel owns (<= 16)
-    int glu;                         // rows of W are gate and up rows in turns of 8; y[M, N / 2] = act(gate) * up
+    int glu;                         // y[M, N / 2] = act(gate) * up: 1, rows of W are gate and up rows in turns of 8; 2, all gate rows, then all
+                                     // up rows (gemm_f32_stream_kernel alone)
     int act;
     int add;                         // y += the product (kernels of up to 16 rows, no glu)
     const float* norm_w;             // rows of x are normed on their way in: x * scale * norm_w; null: as they are
@@ -219,7 +220,8 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
     const int n0 = blockIdx.x * a.cols;
     // lanes without a column or a row read their neighbour's (no other bytes, and no load under a branch); what they form is
     // not stored
-    const float* wp = a.w + (size_t)min(n0 + min(r, a.cols - 1), a.N - 1) * a.ldw + 4 * g;
+    const int wrow = a.glu == 2 ? min(n0 / 2 + (r & 7), a.N / 2 - 1) + (r >> 3) * (a.N / 2) : min(n0 + min(r, a.cols - 1), a.N - 1);
+    const float* wp = a.w + (size_t)wrow * a.ldw + 4 * g;
     const float* xp = a.x + (size_t)min(r, a.M - 1) * a.ldx + 4 * g;
     const int n_chunks = (a.K + GF_CHUNK - 1) / GF_CHUNK;
     // the output that this thread adds up
@@ -288,7 +290,7 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
     __syncthreads();
     if (tid < 256) sums[tid] = tot;
     __syncthreads();
-    if (tid < 128 && tid / 8 < a.M)
+    if (tid < 128 && tid / 8 < a.M && n0 / 2 + tid % 8 < a.N / 2)
         a.y[(size_t)(tid / 8) * a.ldy + n0 / 2 + tid % 8] = bn_gate_act(sums[tid / 8 * 16 + tid % 8], a.act) * sums[tid / 8 * 16 + 8 + tid % 8];
 }
 
@@ -1013,10 +1015,10 @@ extern "C" int bn_gemm_f32_supports(int N, int K, int ldw, const void* w) {
 extern "C" int bn_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K, int ldx, int ldw, int ldy, int glu, int act,
                            int form, const float* norm_w, float eps, int add, hipStream_t s) {
     if (M <= 0 || !bn_gemm_f32_supports(N, K, ldw, w) || ldx % 4 || ldx < K || ldx > (1 << 22) || ((uintptr_t)x & 15)) return BN_ERR_ARG;
-    if (ldy < (glu ? N / 2 : N) || (glu && N % 16) || act < 0 || act >= BN_ACT_KINDS) return BN_ERR_ARG;
+    if (ldy < (glu ? N / 2 : N) || (glu && (glu == 2 ? N % 2 || M > 16 || form > 1 : N % 16)) || act < 0 || act >= BN_ACT_KINDS) return BN_ERR_ARG;
     if ((long long)((M + 31) / 32) * ((N + 15) / 16) > 0x7fffffffLL) return BN_ERR_ARG;
     if (((norm_w || add) && form) || (norm_w && !gf_norm_ok(M, K, norm_w)) || (add && (glu || M > 16))) return BN_ERR_ARG;
-    GfArgs a = {(const float*)x, (const float*)w, (float*)y, M, N, K, ldx, ldw, ldy, 16, glu ? 1 : 0, act, add ? 1 : 0, norm_w, eps};
+    GfArgs a = {(const float*)x, (const float*)w, (float*)y, M, N, K, ldx, ldw, ldy, 16, glu == 2 ? 2 : glu ? 1 : 0, act, add ? 1 : 0, norm_w, eps};
     if (norm_w) {
         a.cols = glu ? 16 : gf_stream_cols(N);
         return gf_norm_pick(M, K, [&](auto nr, auto nv) { return gf_launch_stream<decltype(nr)::value, decltype(nv)::value>(a, s); });

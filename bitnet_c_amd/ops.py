@@ -505,10 +505,10 @@ def _tiled(x, w, out_dtype):
     return y
 
 
-def _f32_product(x, w, glu: bool = False, activation: str = "silu", form: int = 0, streamed: Optional["StreamedWeight"] = None,
+def _f32_product(x, w, glu: int = 0, activation: str = "silu", form: int = 0, streamed: Optional["StreamedWeight"] = None,
                  norm: Optional["StreamNorm"] = None, into: Optional[torch.Tensor] = None):
     """x . w^T in float32 on the matrix cores (gemm_f32.hip: every number in three bf16 parts, float32 sums), or with glu act(gate) * up for w = gate and up
-    rows interleaved in blocks of 8; None for weights that the kernels do not take (rows that are not whole 16-byte groups).
+    rows interleaved in blocks of 8 (1, True) or all gate rows in front of all up rows (2: up to 16 rows, over w itself); None for weights that the kernels do not take (rows that are not whole 16-byte groups).
     Whether they do depends on the weights alone, and every form of the kernels has one order of summation, so a row's bits do
     not depend on the step it comes in.  form: 0, by the sizes; the others are bn_gemm_f32's, for tests.  streamed: w's
     streamed copy, which products of up to 16 rows read instead (the same bits).  norm: x is its stream, whose rows are normed
@@ -524,7 +524,7 @@ def _f32_product(x, w, glu: bool = False, activation: str = "silu", form: int = 
         ldx = K
     y = into if into is not None else torch.empty((M, N // 2 if glu else N), dtype=torch.float32, device=x.device)
     nw, eps = (norm.weight.data_ptr(), norm.eps) if norm is not None else (None, 0.0)
-    if (streamed is not None and form == 0 and (not glu or streamed.tile_rows == STREAM_TILE_ROWS)
+    if (streamed is not None and form == 0 and glu != 2 and (not glu or streamed.tile_rows == STREAM_TILE_ROWS)
             and (norm is None or K >= F32_STREAM_NORM_MIN_K) and _fn("gemm_f32", "bn_gemm_f32_streamed_supports")(M, N, K, ldx, streamed.tile_rows, x.data_ptr())):
         tiles, _, rows = _weight_arg(w, streamed, "float32 product")
         _check(_fn("gemm_f32", "bn_gemm_f32_streamed")(x.data_ptr(), tiles, y.data_ptr(), M, N, K, ldx, rows, y.shape[1], int(glu),
@@ -984,6 +984,15 @@ def _staged_swiglu(x, w_gate_up, pre, activation, streamed=None):
     return y
 
 
+def stacked_swiglu(M: int, w_gate_up: torch.Tensor, interleaved: bool, streamed: Optional[StreamedWeight] = None) -> bool:
+    """Whether float32 gate and up rows that are not interleaved (F no multiple of 8) have a product with the gated unit in it: a
+    workgroup takes eight gate rows and the up rows that belong to them from the other half of w.  Over w itself; a matrix with
+    a streamed copy is read there, and the unit is a kernel of its own.  At these sizes a launch costs what it does: of a layer of 64
+    columns with F 172 norm, product and unit 7.9 us as three kernels, 4.0 as one (a call of 16 steps over two layers 1.10 -> 1.03 ms)."""
+    return (w_gate_up.dtype == torch.float32 and not interleaved and streamed is None and 1 <= M <= SKINNY_ROWS
+            and w_gate_up.shape[0] % 2 == 0 and f32_product_takes(w_gate_up))
+
+
 def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, interleaved: bool = False, *,
                   allow_library: Optional[bool] = None, activation: str = "silu",
                   streamed: Optional[StreamedWeight] = None) -> torch.Tensor:
@@ -1009,6 +1018,8 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, interleaved: bool = 
         y = _f32_product(x, w_gate_up, True, activation, streamed=streamed)
         if y is not None:
             return y
+    if stacked_swiglu(M, w_gate_up, interleaved, streamed):
+        return _f32_product(x, w_gate_up, 2, activation)
     aligned = x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0
     if x.dtype == torch.bfloat16 and interleaved and aligned and _staged_swiglu_rows(M, allow_library, 2 * F, streamed):
         y = _staged_swiglu(x, w_gate_up, None, activation, streamed)
@@ -1221,11 +1232,11 @@ def wants_stream_norm(pre: DeferredNorm, w: torch.Tensor, streamed: Optional[Str
     return takes_stream_norm(pre, w, streamed)
 
 
-def linear_stream_norm(pre: StreamNorm, w: torch.Tensor, streamed: Optional[StreamedWeight] = None, glu: bool = False,
+def linear_stream_norm(pre: StreamNorm, w: torch.Tensor, streamed: Optional[StreamedWeight] = None, glu: int = 0,
                        activation: Optional[str] = None) -> torch.Tensor:
     """linear(rows, w) for the rows of a StreamNorm or a StreamSum, in one kernel: activation(linear) (one of
-    UNARY_ACTIVATIONS, bf16), or with glu linear_swiglu for gate and up interleaved in blocks of 8 (float32); for what
-    takes_stream_norm says."""
+    UNARY_ACTIVATIONS, bf16), or with glu linear_swiglu for gate and up interleaved in blocks of 8 (float32; glu 2: for what
+    stacked_swiglu says); for what takes_stream_norm says."""
     if not takes_stream_norm(pre, w, streamed) or (glu and w.dtype != torch.float32) or (activation and not glu and w.dtype != torch.bfloat16):
         raise KernelError(f"linear_stream_norm: rows {tuple(pre.shape)}, w {tuple(w.shape)} cannot be fused")
     if w.dtype == torch.float32:

@@ -118,11 +118,12 @@ class SwiGLU(Part):
         if isinstance(h, ops.DeferredNorm):
             w = self.gate_up.weight
             M = h.shape[0]
-            if isinstance(h, ops.StreamNorm) and not (w.dtype == torch.float32 and not self.has_bias and self.interleaved
+            stacked = ops.stacked_swiglu(M, w, self.interleaved, self.gate_up.streamed)
+            if isinstance(h, ops.StreamNorm) and not (w.dtype == torch.float32 and not self.has_bias and (self.interleaved or stacked)
                                                       and ops.wants_stream_norm(h, w, self.gate_up.streamed)):
                 return self.forward(h.materialize(), ctx, lazy_ok)
             if isinstance(h, ops.StreamNorm):
-                act = ops.linear_stream_norm(h, w, self.gate_up.streamed, True, self.activation)
+                act = ops.linear_stream_norm(h, w, self.gate_up.streamed, 2 if stacked else 1, self.activation)
                 return self.down.lazy(act) if lazy_ok else self.down(act)
             if (not self.has_bias and self.interleaved and w.dtype == torch.bfloat16
                     and (ops.can_fuse_norm(M, self.F, self.hidden, w.dtype)

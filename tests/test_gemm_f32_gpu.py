@@ -67,6 +67,28 @@ def test_gated_epilogue(M, F, K, activation):
     assert torch.equal(ops.linear_swiglu(xd, wi, True, activation=activation), want)
 
 
+# widths that are no multiple of 8: one column, a remainder of each kind, one past whole workgroups of eight
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh", "relu2"])
+@pytest.mark.parametrize("M,F,K", [(1, 1, 4), (1, 172, 64), (3, 9, 132), (8, 15, 64), (16, 44, 1156)])
+def test_gated_epilogue_of_stacked_rows(M, F, K, activation):
+    """All gate rows in front of all up rows: the bits of the product and the gated unit's kernel, with a norm of the rows too."""
+    ops = _ops()
+    x, w = _data(M, 2 * F, K, F)
+    wide = torch.full((2 * F, K + 4), float("nan"), device="cuda")
+    wide[:, :K] = w.cuda()
+    xd, wd = x.cuda(), wide[:, :K]
+    want = ops.swiglu(ops._f32_product(xd, wd), False, activation)
+    assert ops.stacked_swiglu(M, wd, False)
+    assert torch.equal(ops.linear_swiglu(xd, wd, False, activation=activation), want)
+    pre = ops.stream_norm(xd, (torch.arange(K, device="cuda") % 7).float() / 7 + 0.5, 1e-5)
+    if ops.takes_stream_norm(pre, wd):
+        want = ops.swiglu(ops.linear_stream_norm(pre, wd), False, activation)
+        assert torch.equal(ops.linear_stream_norm(pre, wd, None, 2, activation), want)
+    assert not ops.stacked_swiglu(17, wd, False) and not ops.stacked_swiglu(M, wd, True)
+    with pytest.raises(ops.KernelError):
+        ops._f32_product(torch.cat([xd] * 17), wd, 2, activation)
+
+
 def test_operands_that_are_not_aligned():
     """Activations at any address and stride give the same bits; weights whose rows are not whole 16-byte groups go to the
     tiled kernel, at every row count."""
