@@ -9,18 +9,26 @@
 // step function rejects such tokens before it launches anything.  scale is the architecture's
 // embedding multiplier (src/model_embed.c:23-27 scales by sqrt(dim) under one of its policies;
 // 1 for this architecture, which changes no bit).
+// A row of a decode step is a chain of waits (the token, its row, the store), and a workgroup that walks the row alone repeats
+// the last two: few rows are cut into slices of a number a thread (row_slices), many rows fill the chip by themselves.  us inside a
+// step, one workgroup a row -> slices: 2,048 numbers 6.0 -> 3.1, 4,096 8.9 -> 4.7, 2,048 with a sinusoid 8.4 -> 3.7.
+static unsigned row_slices(int rows, int dim) {
+    const int most = rows < 512 ? 512 / rows : 1, all = (dim + 255) / 256;
+    return (unsigned)(all < most ? all : most);
+}
 template <typename T>
 __global__ void embed_gather_kernel(float* __restrict__ x, const T* __restrict__ table,
                                     const int* __restrict__ tokens, int dim, int vocab, float scale) {
     const int t = blockIdx.x;
     const int tok = tokens[t];
     float* row = x + (size_t)t * dim;
+    const int first = blockIdx.y * blockDim.x + threadIdx.x, step = gridDim.y * blockDim.x;
     if (tok < 0 || tok >= vocab) {
-        for (int i = threadIdx.x; i < dim; i += blockDim.x) row[i] = 0.f;
+        for (int i = first; i < dim; i += step) row[i] = 0.f;
         return;
     }
     const T* src = table + (size_t)tok * dim;
-    for (int i = threadIdx.x; i < dim; i += blockDim.x) row[i] = to_f32(src[i]) * scale;
+    for (int i = first; i < dim; i += step) row[i] = to_f32(src[i]) * scale;
 }
 
 // The integers of a captured decode step one token on: fields of `rows` numbers each, in the order tokens, positions, sequence
@@ -343,7 +351,7 @@ __global__ void bias_add_kernel(T* __restrict__ y, const float* __restrict__ b, 
 template <typename T>
 static int embed_gather_t(void* x, const void* table, const int* tokens, int n_tokens, int dim,
                           int vocab, float scale, hipStream_t s) {
-    hipLaunchKernelGGL(embed_gather_kernel<T>, dim3(n_tokens), dim3(256), 0, s, (float*)x,
+    hipLaunchKernelGGL(embed_gather_kernel<T>, dim3(n_tokens, row_slices(n_tokens, dim)), dim3(256), 0, s, (float*)x,
                        (const T*)table, tokens, dim, vocab, scale);
     return bn_launch_status();
 }
@@ -531,7 +539,7 @@ __global__ void embed_gather_sinusoid_kernel(float* __restrict__ x, const T* __r
     float* row = x + (size_t)t * dim;
     const bool known = tok >= 0 && tok < vocab;
     const T* src = table + (size_t)(known ? tok : 0) * dim;
-    for (int e = threadIdx.x; e < dim; e += blockDim.x) {
+    for (int e = blockIdx.y * blockDim.x + threadIdx.x; e < dim; e += gridDim.y * blockDim.x) {
         float v = known ? to_f32(src[e]) * scale : 0.f;
         if (pos >= 0) {
             const float angle = __fmul_rn((float)pos, freq[e >> 1]);
@@ -544,11 +552,12 @@ __global__ void embed_gather_sinusoid_kernel(float* __restrict__ x, const T* __r
 extern "C" int bn_embed_gather_sinusoid(int dtype, void* x, const void* table, const int* tokens, const int* positions,
                                         const float* freq, int n_tokens, int dim, int vocab, float scale, hipStream_t s) {
     if (n_tokens <= 0 || dim <= 0 || vocab <= 0 || !positions || !freq) return BN_ERR_ARG;
+    const dim3 grid(n_tokens, row_slices(n_tokens, dim));
     if (dtype == BN_DT_F32)
-        hipLaunchKernelGGL(embed_gather_sinusoid_kernel<float>, dim3(n_tokens), dim3(256), 0, s, (float*)x, (const float*)table,
+        hipLaunchKernelGGL(embed_gather_sinusoid_kernel<float>, grid, dim3(256), 0, s, (float*)x, (const float*)table,
                            tokens, positions, freq, dim, vocab, scale);
     else if (dtype == BN_DT_BF16)
-        hipLaunchKernelGGL(embed_gather_sinusoid_kernel<bf16>, dim3(n_tokens), dim3(256), 0, s, (float*)x, (const bf16*)table,
+        hipLaunchKernelGGL(embed_gather_sinusoid_kernel<bf16>, grid, dim3(256), 0, s, (float*)x, (const bf16*)table,
                            tokens, positions, freq, dim, vocab, scale);
     else
         return BN_ERR_DTYPE;
@@ -568,7 +577,7 @@ __global__ void embed_gather_learned_kernel(float* __restrict__ x, const T* __re
     const bool known = tok >= 0 && tok < vocab, placed = pos >= 0 && pos < n_pos;
     const T* src = table + (size_t)(known ? tok : 0) * dim;
     const T* prow = pos_table + (size_t)(placed ? pos : 0) * dim;
-    for (int e = threadIdx.x; e < dim; e += blockDim.x) {
+    for (int e = blockIdx.y * blockDim.x + threadIdx.x; e < dim; e += gridDim.y * blockDim.x) {
         const float a = to_f32(src[e]), b = to_f32(prow[e]);
         row[e] = fmaf(known ? a : 0.f, scale, placed ? b : 0.f);
     }
@@ -578,11 +587,12 @@ extern "C" int bn_embed_gather_learned(int dtype, void* x, const void* table, co
                                        const void* pos_table, int n_tokens, int dim, int vocab, int n_pos, float scale,
                                        hipStream_t s) {
     if (n_tokens <= 0 || dim <= 0 || vocab <= 0 || n_pos <= 0 || !x || !table || !tokens || !positions || !pos_table) return BN_ERR_ARG;
+    const dim3 grid(n_tokens, row_slices(n_tokens, dim));
     if (dtype == BN_DT_F32)
-        hipLaunchKernelGGL(embed_gather_learned_kernel<float>, dim3(n_tokens), dim3(256), 0, s, (float*)x, (const float*)table,
+        hipLaunchKernelGGL(embed_gather_learned_kernel<float>, grid, dim3(256), 0, s, (float*)x, (const float*)table,
                            tokens, positions, (const float*)pos_table, dim, vocab, n_pos, scale);
     else if (dtype == BN_DT_BF16)
-        hipLaunchKernelGGL(embed_gather_learned_kernel<bf16>, dim3(n_tokens), dim3(256), 0, s, (float*)x, (const bf16*)table,
+        hipLaunchKernelGGL(embed_gather_learned_kernel<bf16>, grid, dim3(256), 0, s, (float*)x, (const bf16*)table,
                            tokens, positions, (const bf16*)pos_table, dim, vocab, n_pos, scale);
     else
         return BN_ERR_DTYPE;
