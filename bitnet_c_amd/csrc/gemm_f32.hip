@@ -12,7 +12,7 @@
 //
 // One order of summation, a function of K alone, whatever M, N, the kernel and its tiles are, so that a row's result does
 // not depend on what else is in the batch: K is cut in chunks of 128; a chunk is summed from nothing, its four blocks of 32 columns one
-// after the other, a block by six instructions, the smallest products first (gf_products); lane group g takes columns 4 g .. 4 g + 3 of
+// after the other, a block by six instructions, the largest product last (gf_term); lane group g takes columns 4 g .. 4 g + 3 of
 // both halves of a block.  The chunks' sums are added in order.  The cut is what lets a product of few rows spread one output's K over the
 // waves of a workgroup (and it keeps the rounding error at that of a sum of 128 and of K / 128 terms).
 //
@@ -92,9 +92,10 @@ template <bool DOT = true> __device__ __forceinline__ GfSplit gf_split(const f32
     gf_split_pair<DOT>(hi[2], hi[3], h.w, m.w, l.w);
     return GfSplit{__builtin_bit_cast(gf_b8, h), __builtin_bit_cast(gf_b8, m), __builtin_bit_cast(gf_b8, l)};
 }
-// Product t of the six, the smallest first
+// Product t of the six, the large one last (the order of the others makes no difference that can be measured: against 64 bits
+// 1.74e-7 of the result at K = 2,048 either way)
 template <int T> __device__ __forceinline__ f32x4 gf_term(const GfSplit& w, const GfSplit& x, const f32x4& acc) {
-    const gf_b8 a = T == 0 || T == 4 ? w.m : T == 2 ? w.l : w.h, b = T == 0 || T == 3 ? x.m : T == 1 ? x.l : x.h;
+    const gf_b8 a = T == 0 || T == 2 ? w.m : T == 4 ? w.l : w.h, b = T == 0 || T == 1 ? x.m : T == 3 ? x.l : x.h;
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
 }
 __device__ __forceinline__ f32x4 gf_products(const GfSplit& w, const GfSplit& x, f32x4 acc) {
