@@ -90,8 +90,9 @@ __device__ __forceinline__ void ag_scores(float (&s)[8], const f32x4& s0, const 
 
 // four consecutive outputs of a head and, with a gate, times the sigmoids of the four gate values beside them:
 // one 8-byte store
-__device__ __forceinline__ void ag_store4(bf16* op, bool gated, uint2 gw, float x0, float x1, float x2, float x3) {
-    if (gated) {
+__device__ __forceinline__ void ag_store4(bf16* op, const bf16* gp, float x0, float x1, float x2, float x3) {
+    if (gp) {
+        const uint2 gw = *reinterpret_cast<const uint2*>(gp);
         x0 /= 1.0f + __expf(-bf16lo_to_f32(gw.x)); x1 /= 1.0f + __expf(-bf16hi_to_f32(gw.x));
         x2 /= 1.0f + __expf(-bf16lo_to_f32(gw.y)); x3 /= 1.0f + __expf(-bf16hi_to_f32(gw.y));
     }
@@ -100,9 +101,6 @@ __device__ __forceinline__ void ag_store4(bf16* op, bool gated, uint2 gw, float 
     w.x = (uint32_t)__builtin_bit_cast(unsigned short, o0) | ((uint32_t)__builtin_bit_cast(unsigned short, o1) << 16);
     w.y = (uint32_t)__builtin_bit_cast(unsigned short, o2) | ((uint32_t)__builtin_bit_cast(unsigned short, o3) << 16);
     *reinterpret_cast<uint2*>(op) = w;
-}
-__device__ __forceinline__ void ag_store4(bf16* op, const bf16* gp, float x0, float x1, float x2, float x3) {
-    ag_store4(op, gp != nullptr, gp ? *reinterpret_cast<const uint2*>(gp) : make_uint2(0u, 0u), x0, x1, x2, x3);
 }
 
 // A workgroup is 4, 2 or 1 heads of one kv head (a wave each); they stage a block of keys and values through shared memory, the
@@ -323,6 +321,7 @@ struct GenDecodeArgs {
     const float* wk;
     const float* inv_freq;    // [rope_dims / 2] rotation in split-half pairs; null: none
     int rope_dims, temp_every;
+    int min_pages;            // of a run whose length follows max_len
     int v_col;                // the first value's column of the row: behind the keys, or the keys as projected
     float eps, temp_coef;
 };
@@ -335,6 +334,14 @@ struct GenDecodeArgs {
 // several waves read them: 64 heads over one, one of 500 10.3 / 11.1, 16 of 2,000 20.9 / 21.7.  (Both loops in one kernel, chosen by
 // the length on the device: 0.4 us slower than either.)
 #define AG_ONCE_MB 24
+
+// Runs of one page, while a launch leaves no more than this many rows of partial sums (sequences x heads x splits) to merge; else of
+// BN_SPLIT_MIN_PAGES.  A wave walks its run block by block and waits for the values of each, so that a page more is 1.5 us more; against
+// that stands what the merge reads.  us, runs of two pages and more -> this, keys in front: 16 heads of 128 over 4, one sequence 130 7.4 -> 6.3,
+// 300 9.9 -> 6.8, 1,000 9.2 -> 7.6, 2,000 9.8 -> 8.5, four of 300 11.1 -> 7.4, of 800 11.8 -> 8.0, of 1,500 10.5 -> 10.5, 16 of 300 11.8 -> 9.6,
+// of 1,000 (4,096 rows) 13.8 -> 14.1, 64 of 200 (4,096) 13.8 -> 13.0; 64 heads over one, 16 of 300 (5,120) 11.2 -> 9.4, four of 1,500 (6,144)
+// 9.9 -> 10.4, 16 of 1,000 (16,384) 12.8 -> 15.2, 64 of 200 (16,384) 12.9 -> 14.5; 16 of 256 over 2, four of 800 17.5 -> 10.2.
+#define AG_PAGE_RUN_ROWS 6000
 
 // NEW: the new token's row is still as projected.  Every wave norms, rotates and scales its queries, and the waves of the run that holds
 // the new position its key, in the registers in which they are multiplied (rotations turn pairs a whole number of 32 dimensions apart, so
@@ -385,7 +392,7 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
         const int lo = a.window > 0 ? max(0, len - a.window) : 0;
         if (split == 0 && a.window > 0) keep = min(a.keep_first, lo);
         if (a.n_splits > 1) {
-            const int chunk = a.max_len ? bn_split_chunk(*a.max_len, a.n_splits) : a.chunk;
+            const int chunk = a.max_len ? bn_split_chunk(*a.max_len, a.n_splits, a.min_pages) : a.chunk;
             const int base = a.window > 0 ? (lo / BN_PAGE) * BN_PAGE : 0;
             k_lo = max(lo, base + split * chunk);
             k_hi = min(len, base + (split + 1) * chunk);
@@ -598,46 +605,55 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
 }
 
 // out[row, d] = sum_s e^(m_s - m) o_s[d] / (sum_s e^(m_s - m) l_s [+ e^(-m) for the sink]) [sigmoid(gate)], the splits in index order;
-// one wave a (token, head) row: the splits' factors are formed a lane a split, and a lane takes four value columns.  Bound by its
+// one wave a (token, head) row: the splits' factors are formed a lane a split, and a lane takes V value columns.  Bound by its
 // chain of waits: all S >= n_splits sums (the last split's again past the end) and the gate are asked for beside the factors' maxima,
 // and a factor comes out of its lane with a v_readlane.  A split without keys holds zeros, and its factor is 0.  (us inside a step,
 // 64 rows of 7 splits of 128 columns: 5.4 -> 4.7.)
 #define AG_MAX_SPLITS BN_WAVE
-template <int S>
+template <int S, int V>
 __global__ __launch_bounds__(BN_WAVE) void attn_general_combine_kernel(bf16* __restrict__ out, int out_stride,
                                                                        const float* __restrict__ part_o,
                                                                        const float* __restrict__ part_ml, int H, int vd,
                                                                        int n_splits, int sink,
                                                                        const float* __restrict__ sink_values,
                                                                        const bf16* __restrict__ gate, int gate_stride) {
+    typedef __attribute__((ext_vector_type(V))) float Floats;
+    typedef __attribute__((ext_vector_type(V))) __bf16 Bf16s;
     const int row = blockIdx.x, tok = row / H, head = row - tok * H, lane = threadIdx.x;
-    const int mine_at = min(lane, n_splits - 1), d = min(4 * lane, vd - 4);              // vd <= 256: four columns a lane
+    const int mine_at = min(lane, n_splits - 1), d = min(V * lane, vd - V);              // vd <= 64 V: V columns a lane
     const float* ml = part_ml + ((size_t)row * n_splits + mine_at) * 2;
     const float own_m = ml[0], own_l = ml[1];
     const float* op0 = part_o + (size_t)row * n_splits * vd + d;
-    float4 o[S];
+    Floats o[S];
 #pragma unroll
-    for (int s = 0; s < S; ++s) o[s] = *reinterpret_cast<const float4*>(op0 + (size_t)min(s, n_splits - 1) * vd);
-    const uint2 gw = gate ? *reinterpret_cast<const uint2*>(gate + (size_t)tok * gate_stride + (size_t)head * vd + d) : make_uint2(0u, 0u);
+    for (int s = 0; s < S; ++s) o[s] = *reinterpret_cast<const Floats*>(op0 + (size_t)min(s, n_splits - 1) * vd);
+    Bf16s gates = {};
+    if (gate) gates = *reinterpret_cast<const Bf16s*>(gate + (size_t)tok * gate_stride + (size_t)head * vd + d);
     const float sv = sink && sink_values ? sink_values[head] : 0.f;
     __builtin_amdgcn_sched_barrier(0);                   // all asked for before anything is waited for
     const float mine = lane < n_splits ? own_m : -INFINITY, sum = lane < n_splits ? own_l : 0.f;
     const float m = wave_max(sink ? fmaxf(sv, mine) : mine);
     const float f = m != -INFINITY ? expf(mine - m) : 0.f, share = f * sum;
     auto of = [](float x, int s) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), s)); };
-    float den = sink ? expf(sv - m) : 0.f;
-    float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
+    float den = sink ? expf(sv - m) : 0.f, num[V] = {};
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const float w = of(f, s);                        // 0 past n_splits, and so is the share
         const bool in = s < n_splits;                    // (no branch: a load would be moved behind it)
         den += of(share, s);
-        num.x = fmaf(w, in ? o[s].x : 0.f, num.x); num.y = fmaf(w, in ? o[s].y : 0.f, num.y);
-        num.z = fmaf(w, in ? o[s].z : 0.f, num.z); num.w = fmaf(w, in ? o[s].w : 0.f, num.w);
+#pragma unroll
+        for (int u = 0; u < V; ++u) num[u] = fmaf(w, in ? o[s][u] : 0.f, num[u]);
     }
-    if (4 * lane >= vd) return;
+    if (V * lane >= vd) return;
     const float inv = den > 0.f ? 1.0f / den : 0.f;
-    ag_store4(out + (size_t)tok * out_stride + (size_t)head * vd + d, gate != nullptr, gw, num.x * inv, num.y * inv, num.z * inv, num.w * inv);
+    Bf16s r;
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        float x = num[u] * inv;
+        if (gate) x /= 1.0f + __expf(-(float)gates[u]);
+        r[u] = __builtin_bit_cast(__bf16, __float2bfloat16(x));
+    }
+    *reinterpret_cast<Bf16s*>(out + (size_t)tok * out_stride + (size_t)head * vd + d) = r;
 }
 
 static bool ag_size(int x) { return x == 32 || x == 64 || x == 96 || x == 128 || x == 192 || x == 256; }
@@ -758,6 +774,7 @@ static int ag_decode(const void* q, int q_stride, void* out, int out_stride, con
     a.q = (const bf16*)q; a.out = (bf16*)out; a.k_pages = (const bf16*)k_pages; a.v_pages = (const bf16*)v_pages;
     a.block_table = block_table; a.seq_lens = seq_lens; a.dist_a = dist_a; a.dist_b = dist_b; a.part_o = part_o; a.part_ml = part_ml;
     a.max_len = n_splits > 1 ? max_len : nullptr;
+    a.min_pages = (long long)n_seqs * H * n_splits <= AG_PAGE_RUN_ROWS ? 1 : BN_SPLIT_MIN_PAGES;
     a.q_stride = q_stride; a.out_stride = out_stride; a.bt_stride = bt_stride; a.H = H; a.Hkv = Hkv; a.n_splits = n_splits;
     a.chunk = chunk; a.window = window; a.sink = sink ? 1 : 0; a.sink_values = sink ? sink_values : nullptr; a.scale = scale;
     const AgFresh f = fresh ? *fresh : AgFresh{};
@@ -784,9 +801,17 @@ static int ag_decode(const void* q, int q_stride, void* out, int out_stride, con
                            sink ? 1 : 0, sink ? sink_values : nullptr, (const bf16*)gate, gate_stride);
         return bn_launch_status();
     };
-    return n_splits <= 4 ? combine(attn_general_combine_kernel<4>) : n_splits <= 8 ? combine(attn_general_combine_kernel<8>) :
-           n_splits <= 16 ? combine(attn_general_combine_kernel<16>) : n_splits <= 32 ? combine(attn_general_combine_kernel<32>) :
-           combine(attn_general_combine_kernel<AG_MAX_SPLITS>);
+    auto wide = [&](auto most) {
+        constexpr int S = decltype(most)::value;
+        return vd <= 64 ? combine(attn_general_combine_kernel<S, 1>) : vd <= 128 ? combine(attn_general_combine_kernel<S, 2>) :
+               combine(attn_general_combine_kernel<S, 4>);
+    };
+    if (n_splits <= 4) return wide(std::integral_constant<int, 4>());
+    if (n_splits <= 8) return wide(std::integral_constant<int, 8>());
+    if (n_splits <= 16) return wide(std::integral_constant<int, 16>());
+    if (n_splits <= 32) return wide(std::integral_constant<int, 32>());
+    if (n_splits <= 48) return wide(std::integral_constant<int, 48>());
+    return wide(std::integral_constant<int, AG_MAX_SPLITS>());
 }
 
 extern "C" int bn_attn_general_decode(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,

@@ -208,10 +208,10 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
 // Keys per split of a decode step whose longest sequence holds max_len keys, cut into n_splits runs of whole
 // pages: the kernels use it when the length arrives in device memory.  (ops.decode_splits, which makes a plan for a length
 // that the host knows, cuts an even number of pages in the same runs while two pages a split are left; an odd one in longer runs.)
-__host__ __device__ __forceinline__ int bn_split_chunk(int max_len, int n_splits) {
+__host__ __device__ __forceinline__ int bn_split_chunk(int max_len, int n_splits, int min_pages = BN_SPLIT_MIN_PAGES) {
     const int pages = max_len > 0 ? (max_len + BN_PAGE - 1) / BN_PAGE : 1;
     int per = (pages + n_splits - 1) / n_splits;
-    if (per < BN_SPLIT_MIN_PAGES) per = BN_SPLIT_MIN_PAGES;
+    if (per < min_pages) per = min_pages;
     return per * BN_PAGE;
 }
 

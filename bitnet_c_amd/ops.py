@@ -19,6 +19,7 @@ from .csrc import build as _build
 
 PAGE = _build.header_constant("BN_PAGE")                         # tokens per cache page: defined once, in csrc/common.h
 F32_FOLD_KEYS = _build.header_constant("BN_F32_FOLD_KEYS")       # a float32 cache's keys are summed in runs of this many
+GENERAL_PAGE_RUN_ROWS = _build.header_constant("AG_PAGE_RUN_ROWS", "attn_mfma_general.hip")     # partial rows up to which its runs may be single pages
 SPLIT_MIN_PAGES = _build.header_constant("BN_SPLIT_MIN_PAGES")   # shortest run of pages that decode attention splits off
 _DT = {torch.float32: 0, torch.bfloat16: 1}
 
@@ -1733,7 +1734,7 @@ DECODE_TARGET_WGS = int(os.environ.get("BITNET_DECODE_WGS", "256"))
 VECTOR_DECODE_TARGET_WGS = int(os.environ.get("BITNET_VECTOR_DECODE_WGS", "1024"))     # see decode_splits
 
 
-def decode_splits(n_seqs: int, H: int, Hkv: int, max_len: int, dtype=None, target_wgs: int = 0):
+def decode_splits(n_seqs: int, H: int, Hkv: int, max_len: int, dtype=None, target_wgs: int = 0, min_pages: int = SPLIT_MIN_PAGES):
     """(n_splits, chunk): how the keys of a decode step are cut so that the launch fills the
     chip.  A function of the batch's shape and of max_len alone.  A float32 cache is cut in runs of F32_FOLD_KEYS
     positions whatever the batch: both forms of the float32 kernel sum a query's keys run by run and fold the runs in
@@ -1749,17 +1750,17 @@ def decode_splits(n_seqs: int, H: int, Hkv: int, max_len: int, dtype=None, targe
     # target_wgs: another aim than DECODE_TARGET_WGS (the vector kernel's workgroups are small, several fit on a CU and
     # hide each other's waits: VECTOR_DECODE_TARGET_WGS)
     target = target_wgs or DECODE_TARGET_WGS
-    want = max(1, min(pages // SPLIT_MIN_PAGES, 64, (target + wgs - 1) // wgs))
+    want = max(1, min(pages // min_pages, 64, (target + wgs - 1) // wgs))
     chunk = ((pages + want - 1) // want) * PAGE
     n_splits = (pages * PAGE + chunk - 1) // chunk
     return n_splits, chunk
 
 
-def split_chunk(max_len: int, n_splits: int) -> int:
+def split_chunk(max_len: int, n_splits: int, min_pages: int = SPLIT_MIN_PAGES) -> int:
     """Keys per split when a launch of n_splits splits meets sequences of up to max_len keys (bn_split_chunk of
     csrc/common.h): what the kernels compute themselves when the length comes in device memory."""
     pages = max(1, (max_len + PAGE - 1) // PAGE)
-    return max(SPLIT_MIN_PAGES, (pages + n_splits - 1) // n_splits) * PAGE
+    return max(min_pages, (pages + n_splits - 1) // n_splits) * PAGE
 
 
 def can_fuse_decode(dtype, H: int, Hkv: int, hs: int) -> bool:
@@ -2118,11 +2119,12 @@ def general_decode_plan(n_seqs: int, H: int, Hkv: int, max_len: int, window: int
     fills the chip with its one-wave workgroups.  Without a window the plan follows max_len (the cache's bound in a
     captured step: pass max_len_dev then, and the keys per split follow the longest sequence of each replay); with a window
     it depends on the window alone, because the kernel counts the splits from the window's first page."""
-    if window:
-        n_splits, chunk = decode_splits(n_seqs, H, Hkv, window + PAGE, torch.bfloat16, target_wgs=VECTOR_DECODE_TARGET_WGS)
-        return n_splits, chunk, False
-    n_splits, chunk = decode_splits(n_seqs, H, Hkv, max_len, torch.bfloat16, target_wgs=VECTOR_DECODE_TARGET_WGS)
-    return n_splits, chunk, True
+    most = window + PAGE if window else max_len
+    for min_pages in (1, SPLIT_MIN_PAGES):       # single pages where they leave few partial rows (AG_PAGE_RUN_ROWS)
+        n_splits, chunk = decode_splits(n_seqs, H, Hkv, most, torch.bfloat16, target_wgs=VECTOR_DECODE_TARGET_WGS, min_pages=min_pages)
+        if n_seqs * H * n_splits <= GENERAL_PAGE_RUN_ROWS:
+            break
+    return n_splits, chunk, not window
 
 
 class FreshRows(NamedTuple):
@@ -2198,7 +2200,7 @@ def attention_general_decode(qkv: torch.Tensor, out: torch.Tensor, k_pages: torc
             _dev(max_len_dev, "max_len_dev", torch.int32)
             if max_len_dev.numel() != 1 or window:
                 raise KernelError("attention_general_decode: max_len_dev is one int32 and belongs to steps without a window")
-            chunk = split_chunk(block_table.shape[1] * PAGE, n_splits)
+            chunk = split_chunk(block_table.shape[1] * PAGE, n_splits, 1)
         if chunk <= 0 or chunk % PAGE or n_splits > 64:
             raise KernelError(f"attention_general_decode: chunk {chunk} must be a positive multiple of {PAGE}, at most 64 splits")
         cover = min(block_table.shape[1] * PAGE, window + PAGE) if window else block_table.shape[1] * PAGE
