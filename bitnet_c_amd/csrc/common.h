@@ -8,7 +8,8 @@
 #define BN_WAVE 64
 #define BN_PAGE 64            // tokens per cache page; the Python side reads this line (csrc/build.py: header_constant)
 // Decode attention splits a sequence's keys over workgroups in runs of at least this many pages: shorter
-// runs cost more in merging than they gain in parallelism (measured at batch 1, 8 and 64 of an 8B shape).
+// runs cost more in merging than they gain in parallelism (measured at batch 1, 8 and 64 of an 8B shape).  The general
+// kernel's waves walk a run alone: where few partial sums are left its runs are single pages (AG_PAGE_RUN_ROWS).
 #define BN_SPLIT_MIN_PAGES 2
 // A float32 cache's keys are summed by attn_rows.hip (what attn_f32.hip, with runs of its own, does not take) in runs of this
 // many positions (whole pages, counted from position 0), each run by

@@ -509,7 +509,8 @@ def _tiled(x, w, out_dtype):
 def _f32_product(x, w, glu: int = 0, activation: str = "silu", form: int = 0, streamed: Optional["StreamedWeight"] = None,
                  norm: Optional["StreamNorm"] = None, into: Optional[torch.Tensor] = None):
     """x . w^T in float32 on the matrix cores (gemm_f32.hip: every number in three bf16 parts, float32 sums), or with glu act(gate) * up for w = gate and up
-    rows interleaved in blocks of 8 (1, True) or all gate rows in front of all up rows (2: up to 16 rows, over w itself); None for weights that the kernels do not take (rows that are not whole 16-byte groups).
+    rows interleaved in blocks of 8 (1, True) or all gate rows in front of all up rows (2: up to 16 rows, over w itself); None for
+    weights that the kernels do not take (rows that are not whole 16-byte groups).
     Whether they do depends on the weights alone, and every form of the kernels has one order of summation, so a row's bits do
     not depend on the step it comes in.  form: 0, by the sizes; the others are bn_gemm_f32's, for tests.  streamed: w's
     streamed copy, which products of up to 16 rows read instead (the same bits).  norm: x is its stream, whose rows are normed
@@ -1746,7 +1747,7 @@ def decode_splits(n_seqs: int, H: int, Hkv: int, max_len: int, dtype=None, targe
     wgs = max(1, n_seqs * Hkv * ((G + GT - 1) // GT))
     pages = max(1, (max_len + PAGE - 1) // PAGE)
     # about DECODE_TARGET_WGS workgroups, but no split shorter than SPLIT_MIN_PAGES pages: below that the merging costs
-    # more than the parallelism gains (measured at batch 1, 8 and 64 of the 8B shape)
+    # more than the parallelism gains (measured at batch 1, 8 and 64 of the 8B shape); min_pages: another least, for the general kernel
     # target_wgs: another aim than DECODE_TARGET_WGS (the vector kernel's workgroups are small, several fit on a CU and
     # hide each other's waits: VECTOR_DECODE_TARGET_WGS)
     target = target_wgs or DECODE_TARGET_WGS
