@@ -754,6 +754,18 @@ def stream_tile_rows(N: int, dtype=torch.bfloat16) -> int:
     return int(_fn("skinny_gemm", "bn_skinny_gemm_fused_tile_cols")(int(N)))
 
 
+def group_tile_rows(widths) -> list:
+    """The rows per tile for bf16 matrices of these numbers of rows that one launch streams together (linear_group): the most
+    there can be where that leaves two rows of tiles for every CU, since then more of them are only more workgroups that each form or
+    load the launch's rows; matrices of few rows, and all of smaller groups, as by themselves (None: stream_tile_rows).  us, four matrices of
+    2,048 and one of 64, 8 rows a tile (1,032 workgroups, of which the CUs hold 768) -> 16: behind a norm and a token shift 1 / 2 / 4 rows 10.6 /
+    10.6 / 13.4 -> 9.5 / 9.6 / 11.0, plain 8 / 16 rows 9.4 / 11.8 -> 8.9 / 10.1; four of 1,024 6.2 -> 6.6 at 8 rows, 7.0 -> 6.6 at one."""
+    cus, most = _compute_units(), STREAM_TILE_ROWS
+    if sum(-(-int(n) // most) for n in widths) < 2 * cus:
+        return [None] * len(widths)
+    return [most if n >= cus else None for n in widths]
+
+
 def stream_copy(w: torch.Tensor, tile_rows: Optional[int] = None) -> StreamedWeight:
     """The streamed copy of w [N, K] (bf16 or float32, on the device; made there).  tile_rows None: stream_tile_rows(N); a
     matrix with gate and up rows interleaved in blocks of 8 needs 16."""

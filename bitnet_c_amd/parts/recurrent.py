@@ -79,6 +79,10 @@ class WKV(Part):
         for lin, n in ((self.r, "wr"), (self.k, "wk"), (self.v, "wv"), (self.g, "wg"), (self.w1, "w1"), (self.w2, "w2"),
                        (self.o, "wo")):
             lin.load(tensors[n], None, device, dtype)
+        if dtype == torch.bfloat16 and torch.device(device).type == "cuda":
+            first = self._first()                # a decode step streams them in one launch
+            for lin, rows in zip(first, ops.group_tile_rows([l.weight.shape[0] for l in first])):
+                lin.stream_tile_rows = rows
         self.mu = torch.stack([upload(tensors[f"mu_{s}"], device, torch.float32) for s in self.MIXES]).contiguous()
         self.w0 = upload(tensors["w0"], device, torch.float32)
         self.u = upload(tensors["u"], device, torch.float32).reshape(-1).contiguous()
