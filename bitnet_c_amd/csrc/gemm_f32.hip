@@ -1064,7 +1064,7 @@ static bool gf_streamed_parts(int M, int K, bool norm) { return (!norm || M <= 4
 extern "C" int bn_gemm_f32_norm_supports(int M, int K) { return gf_norm_ok(M, K, nullptr); }
 
 // 1 if the kernel over a streamed copy takes the product: up to 16 rows, whole chunks whose sums fit into shared memory
-// (every K up to 10,752 at 9 to 16 rows, 29,952 at 5 to 8), rows of activations that are whole 16-byte groups.
+// (every K up to 10,752 at 9 to 16 rows, 29,952 at 5 to 8, 68,352 at 3 and 4, 145,152 at 1 and 2), rows of activations that are whole 16-byte groups.
 extern "C" int bn_gemm_f32_streamed_supports(int M, int N, int K, int ldx, int tile_rows, const void* x) {
     return M >= 1 && M <= 16 && N >= 1 && K >= GF_CHUNK && K % GF_CHUNK == 0 && gf_streamed_smem(M, K, false, false) <= GF_STREAMED_SMEM && ldx >= K &&
            ldx % 4 == 0 && ldx <= 1 << 22 && tile_rows >= 1 && tile_rows <= BN_STREAM_TILE_ROWS && ((uintptr_t)x & 15) == 0;
@@ -1092,8 +1092,8 @@ extern "C" int bn_gemm_f32_streamed(const void* x, const void* tiles, void* y, i
             return parts ? go(gemm_f32_streamed_kernel<decltype(nr)::value, true, decltype(nv)::value>) : go(gemm_f32_streamed_kernel<decltype(nr)::value, false, decltype(nv)::value>);
         });
     switch (gf_streamed_xr(M)) {
-        case 1: return go(gemm_f32_streamed_kernel<1, true>);
-        case 2: return go(gemm_f32_streamed_kernel<2, true>);
+        case 1: return parts ? go(gemm_f32_streamed_kernel<1, true>) : go(gemm_f32_streamed_kernel<1, false>);
+        case 2: return parts ? go(gemm_f32_streamed_kernel<2, true>) : go(gemm_f32_streamed_kernel<2, false>);
         case 4: return parts ? go(gemm_f32_streamed_kernel<4, true>) : go(gemm_f32_streamed_kernel<4, false>);
         default: return parts ? go(gemm_f32_streamed_kernel<8, true>) : go(gemm_f32_streamed_kernel<8, false>);
     }

@@ -282,3 +282,19 @@ def test_infinite_operands_give_infinite_sums(M):
         y = ops._f32_product(x2.cuda(), w2.cuda(), form=f).cpu()
         rest = torch.arange(M) != M // 2
         assert torch.equal(y[rest], plain[rest]) and bool(y[M // 2].isinf().all()) and float(y[M // 2, 7]) == float("inf"), f
+
+
+# chunks of K on both sides of where the rows' staged parts no longer fit beside the chunks' sums (and the rows are staged as they are),
+# and of where neither fits
+@pytest.mark.parametrize("M,fits,most", [(1, 1102, 1134), (2, 1102, 1134), (3, 502, 534), (4, 502, 534), (5, 202, 234), (8, 202, 234), (9, 52, 84), (16, 52, 84)])
+def test_streamed_copies_of_rows_about_as_long_as_shared_memory_holds(M, fits, most):
+    ops = _ops()
+    takes = ops._fn("gemm_f32", "bn_gemm_f32_streamed_supports")
+    for chunks in (fits, fits + 1, most - 1, most, most + 1):
+        K = 128 * chunks
+        assert takes(M, 16, K, K, 16, None) == (chunks <= most)
+        x, w = _data(M, 16, K, chunks)
+        xd, wd = x.cuda(), w.cuda()
+        y = ops.linear(xd, wd, streamed=ops.stream_copy(wd))
+        assert torch.equal(y, ops.linear(xd, wd)), K
+        assert torch.all((y.cpu().double() - x.double() @ w.double().t()).abs() <= _bound(x, w)), K
