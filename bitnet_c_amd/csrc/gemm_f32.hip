@@ -8,7 +8,7 @@
 // on a SIMD, six of these 96.  Fewer links in a chain of sums (six of 32 products in place of 32 of four a chunk) round less: error against
 // 64 bits over the largest of a row's sums (2-norms), float32 instruction -> this: 1,000 x 2,048 x 2,048 normal numbers 2.17e-7 -> 1.73e-7,
 // 16 x 2,048 x 5,632 2.36e-7 -> 2.05e-7, all positive 7.32e-8 -> 6.84e-8, 64 x 256 x 14,336 2.81e-7 -> 2.58e-7, rows with a few columns a
-// hundred times the others 2.10e-7 -> 1.71e-7.  What is infinite or no number comes out as before: see gf_replace.
+// hundred times the others 2.10e-7 -> 1.71e-7.  What is infinite or no number: see gf_again.
 //
 // One order of summation, a function of K alone, whatever M, N, the kernel and its tiles are, so that a row's result does
 // not depend on what else is in the batch: K is cut in chunks of 128; a chunk is summed from nothing, its four blocks of 32 columns one
@@ -106,22 +106,36 @@ __device__ __forceinline__ f32x4 gf_products(const GfSplit& w, const GfSplit& x,
     acc = gf_term<4>(w, x, acc);
     return gf_term<5>(w, x, acc);
 }
-// whether all sums so far were finite, in a register of its own (zero, or no number)
-__device__ __forceinline__ void gf_watch(float& all, const f32x4& v) {
-    all += (v[0] - v[0]) + (v[1] - v[1]) + (v[2] - v[2]) + (v[3] - v[3]);
-    asm volatile("" : "+v"(all));                                // now: the sums are not kept for it
-}
+// An infinite operand's second and third part are no numbers (nor is the nearest bf16 number of one above 3.389e38 finite): results
+// that are not finite are formed again by the float32 instruction, from the operands as they are and in one order whatever the kernel: a
+// chunk of 128 columns from nothing, 16 at a time, the chunks' sums in order.
+__device__ __forceinline__ bool gf_finite(float v) { return v - v == 0.f; }
 __device__ __forceinline__ bool gf_finite(const f32x4& v) { return (v[0] - v[0]) + (v[1] - v[1]) + (v[2] - v[2]) + (v[3] - v[3]) == 0.f; }
-// An infinite operand's second and third part are no numbers (nor is the nearest bf16 number of one above 3.389e38 finite): sums that
-// are not finite are formed again by the float32 instruction (or one by one), from the operands as they are, and the others stay.
-__device__ __forceinline__ void gf_replace(f32x4& sum, const f32x4& again) {
+// w(k), x(k): a lane's four columns of the sixteen from k on, of its row
+template <typename W, typename X> __device__ __forceinline__ f32x4 gf_again(int K, W w, X x) {
+    f32x4 all = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int k0 = 0; k0 < K; k0 += GF_CHUNK) {
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int k = k0; k < min(k0 + GF_CHUNK, K); k += 16) {
+            const f32x4 wv = w(k), xv = x(k);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) sum[e] = sum[e] - sum[e] == 0.f ? sum[e] : again[e];
+            for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[e], xv[e], sum, 0, 0, 0);
+        }
+        all += sum;
+    }
+    return all;
 }
-__device__ __forceinline__ f32x4 gf_plain(const f32x4& w, const f32x4& x, f32x4 acc) {
+// of a tile of sums as the instruction leaves them (lane r + 16 g: columns 4 g .. 4 g + 3 of row r) the one of this lane's row and column
+__device__ __forceinline__ float gf_of_tile(const f32x4& tile, int row, int col) {
+    float v = 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e], x[e], acc, 0, 0, 0);
-    return acc;
+    for (int e = 0; e < 4; ++e) {
+        const float s = __shfl(tile[e], (row & 15) + 4 * (col & 12), BN_WAVE);
+        v = (col & 3) == e ? s : v;
+    }
+    return v;
 }
 
 struct gf_true { static constexpr bool value = true; };
@@ -146,13 +160,6 @@ __device__ __forceinline__ float gf_norm_scale(const GfArgs& a, const float* par
 #pragma unroll
     for (int i = 0; i < 4; ++i) ss += parts[row * 4 + i];
     return 1.0f / sqrtf(ss / (float)a.K + a.eps);
-}
-// four numbers from their parts (an infinite one's further parts are no numbers, nor are its neighbour's)
-__device__ __forceinline__ f32x4 gf_whole(const unsigned char* at) {
-    const uint2 h = *reinterpret_cast<const uint2*>(at), m = *reinterpret_cast<const uint2*>(at + 64), l = *reinterpret_cast<const uint2*>(at + 128);
-    auto one = [](float h, float m, float l) { return m == m ? h + m + l : h; };
-    return f32x4{one(bf16lo_to_f32(h.x), bf16lo_to_f32(m.x), bf16lo_to_f32(l.x)), one(bf16hi_to_f32(h.x), bf16hi_to_f32(m.x), bf16hi_to_f32(l.x)),
-                 one(bf16lo_to_f32(h.y), bf16lo_to_f32(m.y), bf16lo_to_f32(l.y)), one(bf16hi_to_f32(h.y), bf16hi_to_f32(m.y), bf16hi_to_f32(l.y))};
 }
 // Four numbers of a row of x, from column c, to shared memory: as they are, or as their parts, 32 columns' first, second and third ones
 // behind each other (64 bytes each) in the order of the matrix instruction's lanes (column 16 h + 4 g + e at 8 g + 4 h + e)
@@ -241,7 +248,6 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
 
     for (int c0 = 0; c0 < n_chunks; c0 += GF_ROUND) {
         const int c1 = min(n_chunks, c0 + GF_ROUND);
-        float all = 0.f;
         auto chunk = [&](int c, auto whole) {
             const int k0 = c * GF_CHUNK;
             auto fetch = [&](const float* p, f32x4 (&v)[GF_BLOCKS]) {
@@ -260,7 +266,6 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
             }
 #pragma unroll
             for (int j = 0; j < GF_BLOCKS; j += 2) acc = gf_products(gf_split(wv[j], wv[j + 1]), gf_split(xv[j], xv[j + 1]), acc);
-            gf_watch(all, acc);
             // lane: columns 4 g .. 4 g + 3 of row r
             *reinterpret_cast<f32x4*>(&sums[(c - c0) * 256 + 16 * r + 4 * g]) = acc;
         };
@@ -268,21 +273,19 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
             if ((c + 1) * GF_CHUNK <= a.K) chunk(c, gf_true());
             else chunk(c, gf_false());
         }
-        if (__any(all != 0.f)) {                                 // see gf_replace
-            for (int c = c0 + wave; c < c1; c += GF_WAVES) {
-                f32x4 again = {0.f, 0.f, 0.f, 0.f};
-                for (int k = c * GF_CHUNK; k < (c + 1) * GF_CHUNK; k += 16) {
-                    f32x4 v = gf_load(xp + k, k + 4 * g < a.K);
-                    if constexpr (NR > 0) v = v * scale * gf_load(a.norm_w + 4 * g + k, k + 4 * g < a.K);
-                    again = gf_plain(gf_load(wp + k, k + 4 * g < a.K), v, again);
-                }
-                gf_replace(*reinterpret_cast<f32x4*>(&sums[(c - c0) * 256 + 16 * r + 4 * g]), again);
-            }
-        }
         __syncthreads();
         if (tid < 256)
             for (int c = 0; c < c1 - c0; ++c) tot += sums[c * 256 + tid];
         if (c1 < n_chunks) __syncthreads();
+    }
+    if (tid < 256 && __builtin_expect(__any(!gf_finite(tot)), 0)) {          // see gf_again
+        const f32x4 again = gf_again(a.K, [&](int k) { return gf_load(wp + k, k + 4 * g < a.K); }, [&](int k) {
+            const f32x4 v = gf_load(xp + k, k + 4 * g < a.K);
+            if constexpr (NR > 0) return v * scale * gf_load(a.norm_w + 4 * g + k, k + 4 * g < a.K);
+            return v;
+        });
+        const float own = gf_of_tile(again, m, col);
+        tot = gf_finite(tot) ? tot : own;
     }
     if (!a.glu) {
         if (mine) a.y[(size_t)m * a.ldy + n] = a.add ? old + tot : tot;
@@ -322,7 +325,8 @@ __global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_strea
     constexpr int UNIT = HALVES ? GF_BLOCKS / 2 : GF_BLOCKS;
     extern __shared__ __align__(16) unsigned char smem[];
     const int row_bytes = gf_row_bytes(NORM ? a.K : GF_CHUNK, PARTS);
-    float* sums = reinterpret_cast<float*>(smem + (NORM ? 1 : GF_WAVES) * ROWS * row_bytes);     // [chunk][row][column]
+    float* parts = reinterpret_cast<float*>(smem + (NORM ? 1 : GF_WAVES) * ROWS * row_bytes);    // of the rows' squares
+    float* sums = parts + (NORM ? ROWS * 4 : 0);                             // [chunk][row][column]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
@@ -389,9 +393,9 @@ __global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_strea
     if (NORM) norm.load(a, tid);
     auto stage = [&] {                                                       // once a wave, behind its first loads of W
         if (!NORM) return;
-        norm.sum(a, tid, sums);                                              // where the chunks' sums come later
+        norm.sum(a, tid, parts);
         bn_lds_barrier();
-        norm.template store<PARTS>(a, tid, sums, smem, row_bytes);
+        norm.template store<PARTS>(a, tid, parts, smem, row_bytes);
         bn_lds_barrier();
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -457,26 +461,24 @@ __global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_strea
         }
     }
     bn_lds_barrier();
-    if (tid >= ROWS * 16) return;
+    if (tid >= (ROWS > 4 ? ROWS * 16 : BN_WAVE)) return;                     // (whole waves stay)
     float tot = 0.f;
 #pragma unroll 8
-    for (int c = 0; c < n_chunks; ++c) tot += sums[(size_t)c * (ROWS * 16) + tid];
+    for (int c = 0; c < n_chunks; ++c) tot += sums[(size_t)c * (ROWS * 16) + tid % (ROWS * 16)];
     const int m = tid >> 4, col = tid & 15, n0 = blockIdx.x * a.cols;
-    if (__any(tot - tot != 0.f)) {                                           // see gf_replace
-        float again = 0.f;
-        const float* from = a.w + (size_t)blockIdx.x * k_tiles * (tile / 4) + min(col, a.cols - 1) * 4;
-#pragma unroll 1
-        for (int k = 0; k < a.K; k += 4, from += a.cols * 4) {
-            const unsigned char* at = xs + min(m, a.M - 1) * row_bytes;
-            f32x4 v;
-            if constexpr (!NORM) v = *reinterpret_cast<const f32x4*>(a.x + (size_t)min(m, a.M - 1) * a.ldx + k);
-            else if constexpr (PARTS) v = gf_whole(at + gf_part_at(k));
-            else v = *reinterpret_cast<const f32x4*>(at + k * 4);
-            const f32x4 w = *reinterpret_cast<const f32x4*>(from);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) again = fmaf(w[e], v[e], again);
-        }
-        tot = tot - tot == 0.f ? tot : again;
+    if (__builtin_expect(__any(!gf_finite(tot)), 0)) {                       // see gf_again
+        int own_lane = lane;
+        asm volatile("" : "+v"(own_lane));                                   // (nothing of this is formed ahead and kept)
+        const int row = min(own_lane & 15, a.M - 1), g4 = own_lane >> 4 << 2;
+        const float* from = a.w + (size_t)blockIdx.x * k_tiles * (tile / 4) + g4 * a.cols + min(own_lane & 15, a.cols - 1) * 4;
+        const float* x_from = a.x + (size_t)row * a.ldx + g4;
+        const f32x4 again = gf_again(a.K, [&](int k) { return *reinterpret_cast<const f32x4*>(from + k / 16 * (tile / 4)); }, [&](int k) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(x_from + k);
+            if constexpr (NORM) return v * gf_norm_scale(a, parts, row) * *reinterpret_cast<const f32x4*>(a.norm_w + g4 + k);
+            return v;
+        });
+        const float own = gf_of_tile(again, m, col);
+        tot = gf_finite(tot) ? tot : own;
     }
     if (a.glu) {                                                             // columns 0..7 of the tile are gates, 8..15 their ups
         const float up = bn_lane_xor<8>(tot);
@@ -493,14 +495,6 @@ __device__ __forceinline__ int gf_run_of_xcd(int id, int total) {
     const int per = total / 8, rest = total % 8, xcd = id % 8;
     return xcd * per + min(xcd, rest) + id / 8;
 }
-// a chunk's sums by the float32 instruction, from rows of W and x
-__device__ __forceinline__ f32x4 gf_chunk_again(const float* w, const float* x, int k0, int K, int g) {
-    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int k = k0 + 4 * g; k < k0 + GF_CHUNK; k += 16) sum = gf_plain(gf_load(w + k, k < K), gf_load(x + k, k < K), sum);
-    return sum;
-}
-
 // More than 16 rows and few tiles.  A workgroup owns 16 MT rows and 16 NT columns, its waves take K's chunks in turns, as the streaming
 // kernels': no wave waits for another inside a chunk, every one brings its operands itself (memory to shared memory, two blocks of 32
 // columns on their way) and splits them between the products of the block before.  Bound by those vector instructions: 17.7 us for 128 rows
@@ -616,12 +610,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_chunks_kernel(GfArgs a, i
 #pragma unroll
         for (int i = 0; i < NT; ++i)
 #pragma unroll
-            for (int j = 0; j < MT; ++j) {
-                if (__any(!gf_finite(acc[i][j])))
-                    gf_replace(acc[i][j], gf_chunk_again(a.w + (size_t)min(n0 + 16 * i + r, a.N - 1) * a.ldw,
-                                                         a.x + (size_t)min(m0 + 16 * j + r, a.M - 1) * a.ldx, (c0 + wave) * GF_CHUNK, a.K, g));
-                *reinterpret_cast<f32x4*>(&sums[wave][(16 * j + r) * STRIDE + 16 * i + 4 * g]) = acc[i][j];
-            }
+            for (int j = 0; j < MT; ++j) *reinterpret_cast<f32x4*>(&sums[wave][(16 * j + r) * STRIDE + 16 * i + 4 * g]) = acc[i][j];
         bn_lds_barrier();
 #pragma unroll
         for (int o = 0; o < OUT; ++o) {
@@ -633,6 +622,19 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_chunks_kernel(GfArgs a, i
         bn_lds_barrier();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // nothing is on its way into shared memory when the wave ends
+#pragma unroll
+    for (int o = 0; o < OUT; ++o) {
+        if (__builtin_expect(!__any(!gf_finite(tot[o])), 1)) continue;       // see gf_again
+        const int idx = tid + o * THREADS, m = idx / COLS, n = idx % COLS, j = __builtin_amdgcn_readfirstlane(m / 16);
+        const float* xp = a.x + (size_t)min(m0 + 16 * j + r, a.M - 1) * a.ldx + 4 * g;
+#pragma unroll 1
+        for (int i = 0; i < NT; ++i) {                           // (a wave's outputs lie in one row of tiles)
+            const float* wp = a.w + (size_t)min(n0 + 16 * i + r, a.N - 1) * a.ldw + 4 * g;
+            const f32x4 again = gf_again(a.K, [&](int k) { return gf_load(wp + k, k + 4 * g < a.K); }, [&](int k) { return gf_load(xp + k, k + 4 * g < a.K); });
+            const float own = gf_of_tile(again, m, n);
+            tot[o] = n / 16 != i || gf_finite(tot[o]) ? tot[o] : own;
+        }
+    }
     if (a.glu) {
 #pragma unroll
         for (int o = 0; o < OUT; ++o) {
@@ -890,17 +892,16 @@ __global__ __launch_bounds__(256 * KG, 2) void gemm_f32_tile_kernel(GfArgs a, in
     for (int i = 0; i < NW; ++i)
 #pragma unroll
         for (int j = 0; j < MT; ++j) fine = fine && gf_finite(tot[i][j]);
-    if (__any(!fine)) {
+    if (__builtin_expect(__any(!fine), 0)) {                     // see gf_again
 #pragma unroll
         for (int i = 0; i < NW; ++i)
 #pragma unroll
             for (int j = 0; j < MT; ++j) {
-                const float* wp = a.w + (size_t)min(n0 + 16 * i + r, a.N - 1) * a.ldw;
-                const float* xp = a.x + (size_t)min(m0 + 16 * j + r, a.M - 1) * a.ldx;
-                f32x4 again = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-                for (int k0 = 0; k0 < a.K; k0 += GF_CHUNK) again += gf_chunk_again(wp, xp, k0, a.K, g);
-                gf_replace(tot[i][j], again);
+                const float* wp = a.w + (size_t)min(n0 + 16 * i + r, a.N - 1) * a.ldw + 4 * g;
+                const float* xp = a.x + (size_t)min(m0 + 16 * j + r, a.M - 1) * a.ldx + 4 * g;
+                const f32x4 again = gf_again(a.K, [&](int k) { return gf_load(wp + k, k + 4 * g < a.K); }, [&](int k) { return gf_load(xp + k, k + 4 * g < a.K); });
+#pragma unroll
+                for (int e = 0; e < 4; ++e) tot[i][j][e] = gf_finite(tot[i][j][e]) ? tot[i][j][e] : again[e];
             }
     }
 #pragma unroll
@@ -1051,10 +1052,10 @@ extern "C" int bn_gemm_f32_stream_cols(int N) { return N < 1 ? 0 : gf_stream_col
 
 #define GF_STREAMED_SMEM (150 * 1024)
 static int gf_streamed_xr(int M) { return M <= 2 ? 1 : M <= 4 ? 2 : M <= 8 ? 4 : 8; }
-// the staged activations, a sum a chunk, row and column
+// the staged activations, the parts of their squares, a sum a chunk, row and column
 static size_t gf_streamed_smem(int M, int K, bool norm, bool parts) {
     const size_t rows = 2 * gf_streamed_xr(M);
-    return (norm ? rows * gf_row_bytes(K, parts) : GF_WAVES * rows * gf_row_bytes(GF_CHUNK, parts)) + (size_t)(K / GF_CHUNK) * rows * 64;
+    return (norm ? rows * (gf_row_bytes(K, parts) + 16) : GF_WAVES * rows * gf_row_bytes(GF_CHUNK, parts)) + (size_t)(K / GF_CHUNK) * rows * 64;
 }
 // Whether staged rows lie there in parts, split once instead of once a wave: where they fit, and unless a CU then holds one workgroup
 // instead of two (eight normed rows).

@@ -298,3 +298,33 @@ def test_streamed_copies_of_rows_about_as_long_as_shared_memory_holds(M, fits, m
         y = ops.linear(xd, wd, streamed=ops.stream_copy(wd))
         assert torch.equal(y, ops.linear(xd, wd)), K
         assert torch.all((y.cpu().double() - x.double() @ w.double().t()).abs() <= _bound(x, w)), K
+
+
+# the largest numbers, whose nearest bf16 number is infinite, in finite results: rows of every kernel and form, also of normed rows, staged in
+# parts (up to 4) and as they are; fewer chunks than waves, one a wave, more
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 16, 40, 130])
+@pytest.mark.parametrize("K", [256, 1024, 2176])
+def test_results_with_the_largest_operands_do_not_depend_on_the_kernel(M, K):
+    ops = _ops()
+    x, w = _data(M, 48, K, M + K)
+    x[:, 5], x[:, 9] = 3.4e38 * x[:, 5].sign(), x[:, 9] * 2.0 ** -100
+    w[:, 5], w[7, 9] = w[:, 5] * 2.0 ** -100, -3.395e38
+    exact = x.double() @ w.double().t()
+    xd, wd = x.cuda(), w.cuda()
+    want = ops._f32_product(xd, wd, form=4)
+    assert torch.all((want.cpu().double() - exact).abs() <= _bound(x, w))
+    for form in (0, 2, 3, 5, 9, 10) + ((6, 7, 8, 11, 12) if K % 32 == 0 else ()) + ((1,) if M <= 64 else ()):
+        assert torch.equal(ops._f32_product(xd, wd, form=form), want), form
+    if M <= 16:
+        assert torch.equal(ops.linear(xd, wd, streamed=ops.stream_copy(wd)), want)
+    if ops.can_norm_rows(M, K, torch.float32):
+        nw = torch.linspace(0.5, 1.5, K)
+        nw[5] = 3.4e38
+        xd, nw = _data(M, 48, K, M)[0].sign().cuda(), nw.cuda()              # normed: times 1 / sqrt(1 + eps)
+        h = ops.add_rmsnorm(xd.clone(), None, nw, 1e-5, torch.float32)
+        assert bool((h[:, 5].abs() > 3.389e38).all())
+        wd[7, 9], wd[20, 5] = 1.0, 1.5                                       # an infinite result among the finite ones
+        want = ops.linear(h, wd)
+        assert bool(want[:, 20].isinf().all()) and int(want.isfinite().sum()) == M * 47
+        for sw in (None, ops.stream_copy(wd)):
+            assert torch.equal(ops.linear_stream_norm(ops.stream_norm(xd, nw, 1e-5), wd, sw), want), sw is None
