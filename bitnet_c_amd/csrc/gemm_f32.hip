@@ -2,13 +2,14 @@
 // matrix product of the float32 path.  W is row-major [out, in] as the reference keeps it (src/model.c:157-158); out[row] = sum_col
 // W[row, col] x[col] (src/quant/f32_scalar.c:4-32).
 //
-// A float32 number is the sum of three bf16 numbers (gf_split: 3 x 8 bits, nothing is lost above 1e-33), a product of two nine products of
+// A float32 number is the sum of three bf16 numbers (gf_split: 3 x 8 bits, nothing is lost above 7.7e-34), a product of two nine products of
 // those; six are formed, and the three left out, the second parts times the third and the third times themselves, are at most 2^-24
 // of the product, of either sign.  The float32 instruction is the slower way to the same sum by 2.7: it takes 256 cycles for 16 x 16 x 32
 // on a SIMD, six of these 96.  Fewer links in a chain of sums (six of 32 products in place of 32 of four a chunk) round less: error against
 // 64 bits over the largest of a row's sums (2-norms), float32 instruction -> this: 1,000 x 2,048 x 2,048 normal numbers 2.17e-7 -> 1.73e-7,
 // 16 x 2,048 x 5,632 2.36e-7 -> 2.05e-7, all positive 7.32e-8 -> 6.84e-8, 64 x 256 x 14,336 2.81e-7 -> 2.58e-7, rows with a few columns a
-// hundred times the others 2.10e-7 -> 1.71e-7.  What is infinite or no number: see gf_again.
+// hundred times the others 2.10e-7 -> 1.71e-7.  Smaller
+// operands, infinite ones and what is no number: see gf_again.
 //
 // One order of summation, a function of K alone, whatever M, N, the kernel and its tiles are, so that a row's result does
 // not depend on what else is in the batch: K is cut in chunks of 128; a chunk is summed from nothing, its four blocks of 32 columns one
@@ -106,11 +107,15 @@ __device__ __forceinline__ f32x4 gf_products(const GfSplit& w, const GfSplit& x,
     acc = gf_term<4>(w, x, acc);
     return gf_term<5>(w, x, acc);
 }
-// An infinite operand's second and third part are no numbers (nor is the nearest bf16 number of one above 3.389e38 finite): results
-// that are not finite are formed again by the float32 instruction, from the operands as they are and in one order whatever the kernel: a
-// chunk of 128 columns from nothing, 16 at a time, the chunks' sums in order.
-__device__ __forceinline__ bool gf_finite(float v) { return v - v == 0.f; }
-__device__ __forceinline__ bool gf_finite(const f32x4& v) { return (v[0] - v[0]) + (v[1] - v[1]) + (v[2] - v[2]) + (v[3] - v[3]) == 0.f; }
+// An infinite operand's second and third part are no numbers (nor is the nearest bf16 number of one above 3.389e38 finite), and a part
+// below 2^-133 is rounded, so that an operand below 2^-110 loses bits (2^-134 at the most, also below 2^-126: the instructions keep denormal
+// numbers).  Results that are not finite, or so small that this could be seen, are formed again by the float32 instruction, from the
+// operands as they are and in one order whatever the kernel: a chunk of 128 columns from nothing, 16 at a time, the chunks' sums in order.
+// At or above GF_SMALL what is lost is below 2^-24 of the result while the numbers that the lost bits are multiplied by sum up to less than
+// 2^50.  (Zero is kept: a row of zeros is none of these.  A sum whose operands all are below 2^-134 comes out as zero.)
+#define GF_SMALL 0x1p-60f
+__device__ __forceinline__ bool gf_stands(float v) { return (v == 0.f) | ((fabsf(v) >= GF_SMALL) & (fabsf(v) < INFINITY)); }
+__device__ __forceinline__ bool gf_stands(const f32x4& v) { return gf_stands(v[0]) & gf_stands(v[1]) & gf_stands(v[2]) & gf_stands(v[3]); }
 // w(k), x(k): a lane's four columns of the sixteen from k on, of its row
 template <typename W, typename X> __device__ __forceinline__ f32x4 gf_again(int K, W w, X x) {
     f32x4 all = {0.f, 0.f, 0.f, 0.f};
@@ -278,14 +283,14 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemm_f32_stream_kernel(GfArg
             for (int c = 0; c < c1 - c0; ++c) tot += sums[c * 256 + tid];
         if (c1 < n_chunks) __syncthreads();
     }
-    if (tid < 256 && __builtin_expect(__any(!gf_finite(tot)), 0)) {          // see gf_again
+    if (tid < 256 && __builtin_expect(__any(!gf_stands(tot)), 0)) {          // see gf_again
         const f32x4 again = gf_again(a.K, [&](int k) { return gf_load(wp + k, k + 4 * g < a.K); }, [&](int k) {
             const f32x4 v = gf_load(xp + k, k + 4 * g < a.K);
             if constexpr (NR > 0) return v * scale * gf_load(a.norm_w + 4 * g + k, k + 4 * g < a.K);
             return v;
         });
         const float own = gf_of_tile(again, m, col);
-        tot = gf_finite(tot) ? tot : own;
+        tot = gf_stands(tot) ? tot : own;
     }
     if (!a.glu) {
         if (mine) a.y[(size_t)m * a.ldy + n] = a.add ? old + tot : tot;
@@ -466,7 +471,7 @@ __global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_strea
 #pragma unroll 8
     for (int c = 0; c < n_chunks; ++c) tot += sums[(size_t)c * (ROWS * 16) + tid % (ROWS * 16)];
     const int m = tid >> 4, col = tid & 15, n0 = blockIdx.x * a.cols;
-    if (__builtin_expect(__any(!gf_finite(tot)), 0)) {                       // see gf_again
+    if (__builtin_expect(__any(!gf_stands(tot)), 0)) {                       // see gf_again
         int own_lane = lane;
         asm volatile("" : "+v"(own_lane));                                   // (nothing of this is formed ahead and kept)
         const int row = min(own_lane & 15, a.M - 1), g4 = own_lane >> 4 << 2;
@@ -478,7 +483,7 @@ __global__ __launch_bounds__(64 * GF_WAVES, XR == 8 ? 2 : 4) void gemm_f32_strea
             return v;
         });
         const float own = gf_of_tile(again, m, col);
-        tot = gf_finite(tot) ? tot : own;
+        tot = gf_stands(tot) ? tot : own;
     }
     if (a.glu) {                                                             // columns 0..7 of the tile are gates, 8..15 their ups
         const float up = bn_lane_xor<8>(tot);
@@ -624,7 +629,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_chunks_kernel(GfArgs a, i
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // nothing is on its way into shared memory when the wave ends
 #pragma unroll
     for (int o = 0; o < OUT; ++o) {
-        if (__builtin_expect(!__any(!gf_finite(tot[o])), 1)) continue;       // see gf_again
+        if (__builtin_expect(!__any(!gf_stands(tot[o])), 1)) continue;       // see gf_again
         const int idx = tid + o * THREADS, m = idx / COLS, n = idx % COLS, j = __builtin_amdgcn_readfirstlane(m / 16);
         const float* xp = a.x + (size_t)min(m0 + 16 * j + r, a.M - 1) * a.ldx + 4 * g;
 #pragma unroll 1
@@ -632,7 +637,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_chunks_kernel(GfArgs a, i
             const float* wp = a.w + (size_t)min(n0 + 16 * i + r, a.N - 1) * a.ldw + 4 * g;
             const f32x4 again = gf_again(a.K, [&](int k) { return gf_load(wp + k, k + 4 * g < a.K); }, [&](int k) { return gf_load(xp + k, k + 4 * g < a.K); });
             const float own = gf_of_tile(again, m, n);
-            tot[o] = n / 16 != i || gf_finite(tot[o]) ? tot[o] : own;
+            tot[o] = n / 16 != i || gf_stands(tot[o]) ? tot[o] : own;
         }
     }
     if (a.glu) {
@@ -891,7 +896,7 @@ __global__ __launch_bounds__(256 * KG, 2) void gemm_f32_tile_kernel(GfArgs a, in
 #pragma unroll
     for (int i = 0; i < NW; ++i)
 #pragma unroll
-        for (int j = 0; j < MT; ++j) fine = fine && gf_finite(tot[i][j]);
+        for (int j = 0; j < MT; ++j) fine = fine && gf_stands(tot[i][j]);
     if (__builtin_expect(__any(!fine), 0)) {                     // see gf_again
 #pragma unroll
         for (int i = 0; i < NW; ++i)
@@ -901,7 +906,7 @@ __global__ __launch_bounds__(256 * KG, 2) void gemm_f32_tile_kernel(GfArgs a, in
                 const float* xp = a.x + (size_t)min(m0 + 16 * j + r, a.M - 1) * a.ldx + 4 * g;
                 const f32x4 again = gf_again(a.K, [&](int k) { return gf_load(wp + k, k + 4 * g < a.K); }, [&](int k) { return gf_load(xp + k, k + 4 * g < a.K); });
 #pragma unroll
-                for (int e = 0; e < 4; ++e) tot[i][j][e] = gf_finite(tot[i][j][e]) ? tot[i][j][e] : again[e];
+                for (int e = 0; e < 4; ++e) tot[i][j][e] = gf_stands(tot[i][j][e]) ? tot[i][j][e] : again[e];
             }
     }
 #pragma unroll

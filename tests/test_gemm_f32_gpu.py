@@ -328,3 +328,34 @@ def test_results_with_the_largest_operands_do_not_depend_on_the_kernel(M, K):
         assert bool(want[:, 20].isinf().all()) and int(want.isfinite().sum()) == M * 47
         for sw in (None, ops.stream_copy(wd)):
             assert torch.equal(ops.linear_stream_norm(ops.stream_norm(xd, nw, 1e-5), wd, sw), want), sw is None
+
+
+# operands whose third, second or first bf16 part is rounded or zero (below 2^-110, 2^-118 and 2^-126), rows of them beside ordinary ones, against
+# ordinary and large weights and small weights against ordinary and large rows: float32 products and sums, which keep denormal numbers
+@pytest.mark.parametrize("M", [1, 3, 8, 16, 40, 130])
+@pytest.mark.parametrize("K", [132, 1024])
+@pytest.mark.parametrize("small,large", [(-108, 0), (-112, 0), (-116, 30), (-120, 0), (-122, 45), (-125, 0), (-132, 20), (-133, 45)])
+def test_small_operands_keep_their_bits(M, K, small, large):
+    ops = _ops()
+    x, w = _data(M, 48, K, M + K)
+    x[::2] *= 2.0 ** small
+    w[:16] *= 2.0 ** large
+    for x, w in ((x, w), (w[:M].contiguous(), torch.cat([x, x, x])[:48].contiguous())):
+        exact = x.double() @ w.double().t()
+        bound = _bound(x, w) + K * 2.0 ** -149             # every sum is rounded to a multiple of 2^-149 at the least
+        xd, wd = x.cuda(), w.cuda()
+        want = ops._f32_product(xd, wd, form=4)
+        assert torch.all((want.cpu().double() - exact).abs() <= bound)
+        for form in (0, 2, 3, 5, 9, 10) + ((6, 7, 8, 11, 12) if K % 32 == 0 else ()) + ((1,) if len(x) <= 64 else ()):
+            assert torch.equal(ops._f32_product(xd, wd, form=form), want), form
+        if len(x) <= 16 and K % 128 == 0:
+            assert torch.equal(ops.linear(xd, wd, streamed=ops.stream_copy(wd)), want)
+    if ops.can_norm_rows(M, K, torch.float32):
+        x, w = _data(M, 48, K, M)
+        nw = torch.linspace(0.5, 1.5, K) * 2.0 ** small
+        xd, wd, nw = x.cuda(), w.cuda(), nw.cuda()
+        h = ops.add_rmsnorm(xd.clone(), None, nw, 1e-5, torch.float32)
+        want = ops.linear(h, wd)
+        assert torch.all((want.cpu().double() - h.cpu().double() @ w.double().t()).abs() <= _bound(h.cpu(), w) + K * 2.0 ** -149)
+        for sw in (None, ops.stream_copy(wd)) if K % 128 == 0 else (None,):
+            assert torch.equal(ops.linear_stream_norm(ops.stream_norm(xd, nw, 1e-5), wd, sw), want), sw is None
