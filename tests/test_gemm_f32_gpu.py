@@ -1,5 +1,5 @@
-"""The float32 product on the float32 matrix instruction: every form of the kernel against 64 bits, and against each other
-bit for bit (the order of summation is a function of K alone)."""
+"""The float32 product, every number in three bf16 parts: every form of the kernel against 64 bits, and against each other bit for bit
+(the order of summation is a function of K alone).  What the parts keep of the operands is test_f32_parts_gpu.py's."""
 import pytest
 import torch
 
@@ -17,8 +17,10 @@ def _data(M, N, K, seed):
 
 
 def _bound(x, w):
-    """What float32 sums of products can be off by at the most: a chunk is a chain of 32 instructions of four products, the
-    chunks' sums a chain of K / 128; every link rounds at 2^-24 of a partial sum, which the sum of magnitudes bounds."""
+    """What float32 sums of products can be off by at the most, whatever their order in a chunk: its 128 large part products are added by
+    as many roundings, the five kinds of small ones, 2^-8 of them and less, by 640 (two and a half large ones), the chunks' sums by
+    K / 128; every one is 2^-24 of a partial sum, which the sum of magnitudes bounds, and the part products that are not formed are
+    below one more."""
     K = x.shape[1]
     links = 4 * 32 + -(-K // 128) + 4
     return links * 2.0 ** -24 * (x.abs().double() @ w.abs().double().t())
@@ -245,7 +247,6 @@ def test_forms_that_share_out_the_chunks(M, N, K):
     wide[:M, :K], tall[:N, :K] = x.cuda(), w.cuda()
     xd, wd = wide[:M, :K], tall[:N, :K]
     want = ops._f32_product(xd, wd, form=4)
-    # _bound's links: a chunk is 24 instructions here; what the three products that are left out of nine come to is one link more at the most
     assert torch.all((want.cpu().double() - x.double() @ w.double().t()).abs() <= _bound(x, w))
     for form in (1, 5, 9, 10) + ((6, 8, 11, 12) if K % 32 == 0 else ()):
         if form > 1 or M <= 64:
