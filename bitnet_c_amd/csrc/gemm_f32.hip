@@ -26,10 +26,13 @@
 // up to 16.  Its loads of W are plain: two of them take the halves of a line, and non-temporal ones were slower (11,264 x 2,048
 // at 8 rows 25 -> 26 us, 32,000 x 2,048 59 -> 65).
 // gemm_f32_chunks_kernel, more rows and few tiles; gemm_f32_tile_kernel, more: bound by the vector instructions that split the operands
-// beside the matrix instruction, at many rows by both and the clock that power leaves them.  us, float32 instruction -> this: 5,736 rows of
-// 11,264 x 2,048 1,905 -> 1,242 (213 TFLOP/s), of 2,048 x 5,632 980 -> 630, of 3,072 x 2,048 526 -> 389, of 2,048 x 2,048 370 -> 242; 1,000 rows 342 ->
-// 240, 181 -> 132, -, 70 -> 53; 199 rows 86 -> 80, 53 -> 49, 30 -> 35, 22 -> 23; 64 rows 31 -> 38, 36 -> 23, 16 -> 18, 16 -> 11; 17 rows 22 -> 22,
-// 25 -> 21, 11 -> 11, 11 -> 10.
+// beside the matrix instruction, at many rows by both and the clock that power leaves them.  us, float32 instruction -> this, 11,264 x 2,048 /
+// 2,048 x 5,632 / 3,072 x 2,048 / 2,048 x 2,048: 5,736 rows 1,905 -> 1,242 (213 TFLOP/s) / 980 -> 630 / 526 -> 389 / 370 -> 242; 512 rows 178 ->
+// 137 / 95 -> 84 / 53 -> 50 / 38 -> 35; 256 rows 98 -> 82 / 55 -> 54 / 31 -> 35 / 22 -> 24; 199 rows 84 -> 80 / 53 -> 53 / 30 -> 35 / 22 -> 24; 144 rows
+// 62 -> 77 / 52 -> 52 / 22 -> 25 / 21 -> 23; 128 rows 55 -> 53 / 37 -> 37 / 22 -> 25 / 16 -> 17; 64 rows 31 -> 38 / 36 -> 23 / 16 -> 18 / 16 -> 11; 33
+// rows 33 -> 37 / 38 -> 22 / 16 -> 17 / 16 -> 11; 17 rows 24 -> 26 / 27 -> 21 / 12 -> 10 / 11 -> 10.  So at 33 to 320 rows a layer's first products can
+// be slower (up to a quarter), and a layer of 130 to 170 rows is by a tenth: their tiles of 64 rows and more are half empty, and smaller ones
+// split their operands too often.
 #include "common.h"
 #include <type_traits>
 
@@ -986,14 +989,16 @@ static int gf_stream_cols(int N) {
 }
 
 // The form of a product of more than 16 rows with the least time for the busiest CU: ns a block of 32 columns of K with n tiles a CU, first
-// + many n (fitted at 2,048 and 5,632 columns, n = 1 to 248, within 12 %).  A launch that gives a CU one tile or two takes a tile's K
+// + many n (fitted at 1,024 to 14,336 columns, n = 1 to 248: of 415 sizes, 17 to 5,736 rows of twelve matrices, what it takes is 0.4 % behind the
+// fastest form on the mean and 6 to 13 % at 68 to 128 rows of 28,672 x 4,096, the worst).  A launch that gives a CU one tile or two takes a tile's K
 // apart over more waves, many tiles a CU take the large ones, which split and stage their operands least.  us, 128 x 128 / 64 x 128 / its K
 // in two / 64 x 64 / its K in two / 32 x 64 in four / 32 x 32 chunks / 32 x 16 chunks: 5,736 rows of 11,264 x 2,048 1,217 / 1,317 / 1,545 /
 // 1,602 / 2,006 / 2,410 / 3,745 / 4,423; 1,000 of 2,048 x 5,632 220 / 146 / 131 / 156 / 175 / 203 / 290 / 415; 199 of 3,072 x 2,048 89 / 55 / 48 /
-// 40 / 36 / 42 / 45 / 48; 128 of 2,048 x 2,048 85 / 52 / 45 / 39 / 33 / 22 / 18 / 20; 64 of 2,048 x 5,632 220 / 125 / 116 / 98 / 83 / 50 / 42 / 24.
+// 40 / 36 / 42 / 45 / 48; 128 of 2,048 x 2,048 85 / 52 / 45 / 39 / 33 / 22 / 18 / 20; 64 of 2,048 x 5,632 220 / 125 / 116 / 98 / 83 / 50 / 42 / 24; 144 of 11,264 x
+// 2,048 97 / 82 / 94 / 77 / 96 / 89 / 98 / 107.
 static int gf_tile_form(int M, int N, int K) {
     static const int form[8] = {6, 7, 8, 11, 12, 5, 9, 10}, bm[8] = {128, 64, 64, 64, 64, 32, 32, 32}, bn[8] = {128, 128, 128, 64, 64, 64, 32, 16};
-    static const int first[8] = {300, 170, 0, 200, 45, 40, 25, 30}, many[8] = {1190, 670, 770, 395, 505, 305, 238, 135};
+    static const int first[8] = {300, 170, 0, 190, 45, 10, 25, 30}, many[8] = {1190, 670, 770, 375, 505, 330, 238, 135};
     static const int other[8] = {2, 3, 3, 4, 4, 5, 9, 10};       // the forms for K that is no whole blocks
     const bool whole = K % GF_BK == 0;
     int best = 0;
