@@ -340,7 +340,11 @@ struct GenDecodeArgs {
 // that stands what the merge reads.  us, runs of two pages and more -> this, keys in front: 16 heads of 128 over 4, one sequence 130 7.4 -> 6.3,
 // 300 9.9 -> 6.8, 1,000 9.2 -> 7.6, 2,000 9.8 -> 8.5, four of 300 11.1 -> 7.4, of 800 11.8 -> 8.0, of 1,500 10.5 -> 10.5, 16 of 300 11.8 -> 9.6,
 // of 1,000 (4,096 rows) 13.8 -> 14.1, 64 of 200 (4,096) 13.8 -> 13.0; 64 heads over one, 16 of 300 (5,120) 11.2 -> 9.4, four of 1,500 (6,144)
-// 9.9 -> 10.4, 16 of 1,000 (16,384) 12.8 -> 15.2, 64 of 200 (16,384) 12.9 -> 14.5; 16 of 256 over 2, four of 800 17.5 -> 10.2.
+// 9.9 -> 10.4, 16 of 1,000 (16,384) 12.8 -> 15.2, 64 of 200 (16,384) 12.9 -> 14.5; 16 of 256 over 2, four of 800 17.5 -> 10.2. A latent cache, 16 heads over
+// one row of 192 with 128 values: one of 300 10.3 -> 6.9, of 2,000 9.6 -> 8.6, 16 of 1,000 (4,096) 11.4 -> 9.6, of 2,000 (8,192) 12.6 -> 13.8.  Inside the
+// line up to 5 % is lost where 512 workgroups of two pages become 1,024 (eight of 2,000, 16 over 4, 13.9 -> 14.6) and up to 12 % gained
+// (16 of 64 over 16, four of 1,000, 10.9 -> 10.1).  Results differ in rounding: a run's probabilities and sums are taken from its own maximum.  (Logits
+// of Sunusun and Fazopel at 2,048 columns over three draws, from 64 bits: 3.70e-3 -> 3.71e-3, 4.54e-3 -> 4.54e-3.)
 #define AG_PAGE_RUN_ROWS 6000
 
 // NEW: the new token's row is still as projected.  Every wave norms, rotates and scales its queries, and the waves of the run that holds

@@ -2140,6 +2140,21 @@ def general_decode_plan(n_seqs: int, H: int, Hkv: int, max_len: int, window: int
     return n_splits, chunk, not window
 
 
+def general_decode_runs(n_seqs: int, H: int, Hkv: int, hs: int, max_len: int, window: int = 0):
+    """The plan that a decode step takes: general_decode_plan's, but no runs of single pages where longer ones leave nothing to merge and are
+    the faster for it.  That is in launches of 256 workgroups and more, which fill the chip (us, whole -> single pages and a merge: 64 sequences of
+    100 keys, 16 heads of 128 over 4 9.1 -> 10.6, 32 of 130, 32 over 8 10.5 -> 11.9; 32 of 100, 16 over 4 8.4 -> 8.2, one of 130 7.6 -> 6.4), and for two
+    pages with narrow heads, whose page is short (one of 100, 32 of 64 over 4 5.6 -> 6.0, 64 of them 6.8 -> 8.6), or many rows to merge (32 of 100, 64
+    of 128 over one 7.0 -> 8.4; 16 of 130 7.8 -> 7.3; with heads of 256 64 of 100, 16 over 2 13.0 -> 11.8)."""
+    n_splits, chunk, follows = general_decode_plan(n_seqs, H, Hkv, max_len, window)
+    most = window + PAGE if window else max_len
+    if n_splits > 1 and decode_splits(n_seqs, H, Hkv, most, torch.bfloat16, target_wgs=VECTOR_DECODE_TARGET_WGS)[0] == 1:
+        wgs, rows = n_seqs * Hkv * (-(-(H // Hkv) // 16)), n_seqs * H * n_splits
+        if wgs >= 256 or (most <= 2 * PAGE and (hs <= 64 or (hs < 256 and rows >= 2048))):
+            return 1, 0, follows
+    return n_splits, chunk, follows
+
+
 class FreshRows(NamedTuple):
     """What attention_general_decode does to the new rows in qk_norm_store's place: its arguments of these names, pairs split-half."""
     q_weight: Optional[torch.Tensor] = None

@@ -254,7 +254,7 @@ class Attention(Part):
         gate = qkv[:, width - H * vd:] if self.out_gate else None
         mask = dict(window=self.window, keep_first=self.keep_first)
         if ctx.is_decode and on_matrix_cores:
-            n_splits, chunk, follows = ops.general_decode_plan(ctx.n_rows, H, Hkv, kv.max_len, self.window)
+            n_splits, chunk, follows = ops.general_decode_runs(ctx.n_rows, H, Hkv, hs, kv.max_len, self.window)
             ops.attention_general_decode(qkv, out, kv.k_pages, kv.v_pages, kv.block_table, ctx.seq_lens, H, Hkv, hs, vd, self.scale,
                                          n_splits=n_splits, chunk=chunk,
                                          max_len_dev=ctx.max_len_dev if follows and n_splits > 1 else None,

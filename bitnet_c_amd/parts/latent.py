@@ -170,7 +170,7 @@ class LatentAttention(Part):
         out = torch.empty((h.shape[0], H * VW), dtype=h.dtype, device=h.device)
         on_matrix_cores = ops.attention_general_supported(h.dtype, KW, VW) and ops.GENERAL_PROMPT_ON_MATRIX_CORES
         if ctx.is_decode and on_matrix_cores:
-            n_splits, chunk, _ = ops.general_decode_plan(ctx.n_rows, H, 1, kv.max_len)
+            n_splits, chunk, _ = ops.general_decode_runs(ctx.n_rows, H, 1, KW, kv.max_len)
             ops.attention_general_decode(q, out, kv.k_pages, kv.v_pages, kv.block_table, ctx.seq_lens, H, 1, KW, VW, self.scale,
                                          n_splits=n_splits, chunk=chunk, max_len_dev=ctx.max_len_dev if n_splits > 1 else None,
                                          sink=self.sink)

@@ -39,3 +39,18 @@ def test_runs_that_follow_the_longest_sequence(n_seqs, H, Hkv, n, pages):
     ops.attention_general_decode(q, follows, *args, n_splits=n, max_len_dev=longest)
     ops.attention_general_decode(q, fixed, *args, n_splits=n, chunk=64 * pages)
     assert torch.equal(follows, fixed)
+
+
+@pytest.mark.parametrize("n_seqs,H,Hkv,hs,tokens,window,whole", [
+    (64, 16, 4, 128, 100, 0, True), (63, 16, 4, 128, 100, 0, False), (32, 32, 8, 128, 130, 0, True), (31, 32, 8, 128, 130, 0, False), (32, 32, 8, 128, 200, 0, False),
+    (1, 32, 4, 64, 128, 0, True), (1, 32, 4, 64, 129, 0, False), (1, 32, 4, 96, 128, 0, False), (16, 64, 1, 128, 128, 0, True), (15, 64, 1, 128, 128, 0, False),
+    (16, 64, 1, 128, 129, 0, False), (64, 16, 2, 256, 128, 0, False), (128, 16, 2, 256, 128, 0, True), (64, 16, 4, 128, 5000, 64, True), (64, 16, 4, 128, 5000, 65, True),
+    (64, 16, 4, 128, 5000, 129, False), (1, 16, 4, 128, 64, 0, True)])
+def test_short_sequences_stay_whole(n_seqs, H, Hkv, hs, tokens, window, whole):
+    """No merge where longer runs are one: in 256 workgroups and more, and for two pages with heads of 64 or 2,048 rows of partial sums; else the plan."""
+    ops = _ops()
+    plan = ops.general_decode_plan(n_seqs, H, Hkv, tokens, window)
+    got = ops.general_decode_runs(n_seqs, H, Hkv, hs, tokens, window)
+    assert (got[0] == 1) == whole and got[2] == plan[2]
+    if not whole:
+        assert got == plan and plan[0] > 1
