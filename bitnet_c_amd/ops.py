@@ -759,7 +759,9 @@ def group_tile_rows(widths) -> list:
     there can be where that leaves two rows of tiles for every CU, since then more of them are only more workgroups that each form or
     load the launch's rows; matrices of few rows, and all of smaller groups, as by themselves (None: stream_tile_rows).  us, four matrices of
     2,048 and one of 64, 8 rows a tile (1,032 workgroups, of which the CUs hold 768) -> 16: behind a norm and a token shift 1 / 2 / 4 rows 10.6 /
-    10.6 / 13.4 -> 9.5 / 9.6 / 11.0, plain 8 / 16 rows 9.4 / 11.8 -> 8.9 / 10.1; four of 1,024 6.2 -> 6.6 at 8 rows, 7.0 -> 6.6 at one."""
+    10.6 / 13.3 -> 9.4 / 9.4 / 10.8, plain 8 / 16 rows 8.7 / 11.7 -> 8.6 / 9.8; 3,072 12.4 / 12.3 / 14.5 -> 11.9 / 11.9 / 14.0, 10.8 / 12.7 -> 11.1 / 12.2.
+    (Two rows of tiles are where it is sure; the gain ends lower.  Groups below the line, which keep theirs: 2,032 9.8 / 9.8 / 12.2 -> 9.3 / 9.4 /
+    10.7 but 8.5 to 9.2 -> 8.8 at 8 rows, 1,024 7.2 / 7.2 / 9.2 -> 6.5 / 6.6 / 7.8, 6.2 / 8.0 -> 5.9 / 6.9, 768 5.8 / 5.9 / 7.0 -> 4.8 / 4.9 / 5.6.)"""
     cus, most = _compute_units(), STREAM_TILE_ROWS
     if sum(-(-int(n) // most) for n in widths) < 2 * cus:
         return [None] * len(widths)
