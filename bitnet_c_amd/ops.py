@@ -1000,13 +1000,18 @@ def _staged_swiglu(x, w_gate_up, pre, activation, streamed=None):
     return y
 
 
-def stacked_swiglu(M: int, w_gate_up: torch.Tensor, interleaved: bool, streamed: Optional[StreamedWeight] = None) -> bool:
+def stacked_swiglu(M: int, w_gate_up: torch.Tensor, interleaved: bool, streamed: Optional[StreamedWeight] = None, normed: bool = False) -> bool:
     """Whether float32 gate and up rows that are not interleaved (F no multiple of 8) have a product with the gated unit in it: a
     workgroup takes eight gate rows and the up rows that belong to them from the other half of w.  Over w itself; a matrix with
     a streamed copy is read there, and the unit is a kernel of its own.  At these sizes a launch costs what it does: of a layer of 64
-    columns with F 172 norm, product and unit 7.9 us as three kernels, 4.0 as one (a call of 16 steps over two layers 1.10 -> 1.03 ms)."""
+    columns with F 172 norm, product and unit 7.9 us as three kernels, 4.0 as one (a call of 16 steps over two layers 1.10 -> 1.03 ms).
+    us, product and unit -> this, one row: F 172 of 64 columns 4.2 -> 2.9, 1,364 of 512 6.7 -> 4.9, 5,461 of 2,048 23.3 -> 21.5, 10,922 of 4,096 75 -> 70.
+    normed: with the rows' norm in it, which every workgroup forms: while the CUs hold all of them at once, two each, and their norms
+    are one wait (us, norm, product and unit -> all in one: F 1,364 9.0 -> 5.3, 3,412 of 1,280 15.6 -> 11.9; 5,461 26.0 -> 26.3 and, with the norm a
+    kernel of its own, 24.2, 10,922 77.9 -> 83.7 and 72.7)."""
     return (w_gate_up.dtype == torch.float32 and not interleaved and streamed is None and 1 <= M <= SKINNY_ROWS
-            and w_gate_up.shape[0] % 2 == 0 and f32_product_takes(w_gate_up))
+            and w_gate_up.shape[0] % 2 == 0 and f32_product_takes(w_gate_up)
+            and not (normed and w_gate_up.shape[0] > 2 * 16 * _compute_units()))
 
 
 def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, interleaved: bool = False, *,

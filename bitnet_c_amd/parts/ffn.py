@@ -118,7 +118,7 @@ class SwiGLU(Part):
         if isinstance(h, ops.DeferredNorm):
             w = self.gate_up.weight
             M = h.shape[0]
-            stacked = ops.stacked_swiglu(M, w, self.interleaved, self.gate_up.streamed)
+            stacked = ops.stacked_swiglu(M, w, self.interleaved, self.gate_up.streamed, normed=True)
             if isinstance(h, ops.StreamNorm) and not (w.dtype == torch.float32 and not self.has_bias and (self.interleaved or stacked)
                                                       and ops.wants_stream_norm(h, w, self.gate_up.streamed)):
                 return self.forward(h.materialize(), ctx, lazy_ok)

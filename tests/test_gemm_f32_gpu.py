@@ -360,3 +360,21 @@ def test_small_operands_keep_their_bits(M, K, small, large):
         assert torch.all((want.cpu().double() - h.cpu().double() @ w.double().t()).abs() <= _bound(h.cpu(), w) + K * 2.0 ** -149)
         for sw in (None, ops.stream_copy(wd)) if K % 128 == 0 else (None,):
             assert torch.equal(ops.linear_stream_norm(ops.stream_norm(xd, nw, 1e-5), wd, sw), want), sw is None
+
+
+@pytest.mark.parametrize("F", [4095, 4097, 5461])
+def test_wide_stacked_rows_are_normed_in_front(F, monkeypatch):
+    """A feed-forward of gate rows in front of up rows takes its norm into the product while the CUs hold all its workgroups; the bits
+    are those of the kernels of their own either way."""
+    ops = _ops()
+    from bitnet_c_amd.parts.ffn import SwiGLU
+    part = SwiGLU(64, F)
+    x, w = _data(3, 2 * F, 64, F)
+    part.load({"w_gate": w[:F], "w_up": w[F:], "w_down": w[:F].t().contiguous()}, torch.device("cuda"), torch.float32)
+    nw, calls, inside = torch.linspace(0.5, 1.5, 64, device="cuda"), [], ops.linear_stream_norm
+    monkeypatch.setattr(ops, "linear_stream_norm", lambda *a, **k: (calls.append(1), inside(*a, **k))[1])
+    got = part.forward(ops.stream_norm(x.cuda(), nw, 1e-5), None)
+    assert len(calls) == (2 * F <= 32 * ops._compute_units())
+    h = ops.add_rmsnorm(x.cuda(), None, nw, 1e-5, torch.float32)
+    want = part.down(ops.swiglu(ops._f32_product(h, w.cuda()), False, "silu"))
+    assert torch.equal(got, want)
