@@ -610,9 +610,11 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
 
 // out[row, d] = sum_s e^(m_s - m) o_s[d] / (sum_s e^(m_s - m) l_s [+ e^(-m) for the sink]) [sigmoid(gate)], the splits in index order;
 // one wave a (token, head) row: the splits' factors are formed a lane a split, and a lane takes V value columns.  Bound by its
-// chain of waits: all S >= n_splits sums (the last split's again past the end) and the gate are asked for beside the factors' maxima,
-// and a factor comes out of its lane with a v_readlane.  A split without keys holds zeros, and its factor is 0.  (us inside a step,
-// 64 rows of 7 splits of 128 columns: 5.4 -> 4.7.)
+// chain of waits: all S >= n_splits sums (those past n_splits lie past the buffer's end: zeros, and no trip to memory) and the gate are asked
+// for beside the factors' maxima, and a factor comes out of its lane with a v_readlane.  A split without keys holds zeros, and its factor is 0.
+// us inside a step, a loop over the splits -> this, 64 rows of 7 splits of 128 columns 5.4 -> 4.6; with the attention in front of it, 16 heads of
+// 256 over 2, one sequence of 33 / 49 / 56 / 64 splits 14.5 / 15.5 / 15.2 / 16.3 -> 13.0 / 13.8 / 14.1 / 14.4; past the end the last
+// split's sums again, that is 31 more trips of a row of 33 splits: 14.9 / 16.2 / 16.4 / 16.9.
 #define AG_MAX_SPLITS BN_WAVE
 template <int S, int V>
 __global__ __launch_bounds__(BN_WAVE) void attn_general_combine_kernel(bf16* __restrict__ out, int out_stride,
@@ -627,10 +629,14 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_combine_kernel(bf16* __r
     const int mine_at = min(lane, n_splits - 1), d = min(V * lane, vd - V);              // vd <= 64 V: V columns a lane
     const float* ml = part_ml + ((size_t)row * n_splits + mine_at) * 2;
     const float own_m = ml[0], own_l = ml[1];
-    const float* op0 = part_o + (size_t)row * n_splits * vd + d;
+    const auto sums = bn_buffer(part_o + (size_t)row * n_splits * vd, n_splits * vd * 4);
     Floats o[S];
 #pragma unroll
-    for (int s = 0; s < S; ++s) o[s] = *reinterpret_cast<const Floats*>(op0 + (size_t)min(s, n_splits - 1) * vd);
+    for (int s = 0; s < S; ++s) {
+        if constexpr (V == 4) o[s] = __builtin_bit_cast(Floats, __builtin_amdgcn_raw_buffer_load_b128(sums, d * 4, s * vd * 4, 0));
+        else if constexpr (V == 2) o[s] = __builtin_bit_cast(Floats, __builtin_amdgcn_raw_buffer_load_b64(sums, d * 4, s * vd * 4, 0));
+        else o[s] = __builtin_bit_cast(Floats, __builtin_amdgcn_raw_buffer_load_b32(sums, d * 4, s * vd * 4, 0));
+    }
     Bf16s gates = {};
     if (gate) gates = *reinterpret_cast<const Bf16s*>(gate + (size_t)tok * gate_stride + (size_t)head * vd + d);
     const float sv = sink && sink_values ? sink_values[head] : 0.f;
@@ -643,10 +649,9 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_combine_kernel(bf16* __r
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const float w = of(f, s);                        // 0 past n_splits, and so is the share
-        const bool in = s < n_splits;                    // (no branch: a load would be moved behind it)
         den += of(share, s);
 #pragma unroll
-        for (int u = 0; u < V; ++u) num[u] = fmaf(w, in ? o[s][u] : 0.f, num[u]);
+        for (int u = 0; u < V; ++u) num[u] = fmaf(w, o[s][u], num[u]);
     }
     if (V * lane >= vd) return;
     const float inv = den > 0.f ? 1.0f / den : 0.f;
