@@ -612,9 +612,9 @@ __global__ __launch_bounds__(BN_WAVE) void attn_general_decode_kernel(GenDecodeA
 // one wave a (token, head) row: the splits' factors are formed a lane a split, and a lane takes V value columns.  Bound by its
 // chain of waits: all S >= n_splits sums (those past n_splits lie past the buffer's end: zeros, and no trip to memory) and the gate are asked
 // for beside the factors' maxima, and a factor comes out of its lane with a v_readlane.  A split without keys holds zeros, and its factor is 0.
-// us inside a step, a loop over the splits -> this, 64 rows of 7 splits of 128 columns 5.4 -> 4.6; with the attention in front of it, 16 heads of
+// us inside a step, a loop over the splits -> this, 64 rows of 7 splits of 128 columns 5.4 -> 4.7; with the attention in front of it, 16 heads of
 // 256 over 2, one sequence of 33 / 49 / 56 / 64 splits 14.5 / 15.5 / 15.2 / 16.3 -> 13.0 / 13.8 / 14.1 / 14.4; past the end the last
-// split's sums again, that is 31 more trips of a row of 33 splits: 14.9 / 16.2 / 16.4 / 16.9.
+// split's sums again, that is 15 more trips of a row of 33 splits: 14.9 / 16.2 / 16.4 / 16.9.
 #define AG_MAX_SPLITS BN_WAVE
 template <int S, int V>
 __global__ __launch_bounds__(BN_WAVE) void attn_general_combine_kernel(bf16* __restrict__ out, int out_stride,
