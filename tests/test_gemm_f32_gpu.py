@@ -340,6 +340,7 @@ def test_small_operands_keep_their_bits(M, K, small, large):
     ops = _ops()
     x, w = _data(M, 48, K, M + K)
     x[::2] *= 2.0 ** small
+    x[1::2, ::3] *= 2.0 ** small
     w[:16] *= 2.0 ** large
     for x, w in ((x, w), (w[:M].contiguous(), torch.cat([x, x, x])[:48].contiguous())):
         exact = x.double() @ w.double().t()
@@ -349,6 +350,11 @@ def test_small_operands_keep_their_bits(M, K, small, large):
         assert torch.all((want.cpu().double() - exact).abs() <= bound)
         for form in (0, 2, 3, 5, 9, 10) + ((6, 7, 8, 11, 12) if K % 32 == 0 else ()) + ((1,) if len(x) <= 64 else ()):
             assert torch.equal(ops._f32_product(xd, wd, form=form), want), form
+        if len(w) % 16 == 0:
+            for form in (0, 2, 4, 5, 9, 10):
+                assert torch.equal(ops._f32_product(xd, wd, True, "silu", form), ops.swiglu(want, True, "silu")), form
+            if len(x) <= 16:
+                assert torch.equal(ops._f32_product(xd, wd, 2, "silu"), ops.swiglu(want, False, "silu"))
         if len(x) <= 16 and K % 128 == 0:
             assert torch.equal(ops.linear(xd, wd, streamed=ops.stream_copy(wd)), want)
     if ops.can_norm_rows(M, K, torch.float32):
